@@ -391,6 +391,30 @@ typedef struct odmkv_worklist {
                                       * items than compute units (a batch of sequences, many levels).  0: one per compute unit */
 } odmkv_worklist_t;
 
+/* Cut the work list of a store on the host: every (segment, level) run of tiles into items of about equal cost (what the
+ * kernel was measured to need per tile of each level, plus a fixed part per item).  counts: host int64 [5][nseg] tokens per
+ * level and segment; seg_tile: host int64 [5][nseg + 1]; n_cu: compute units.  target_items > 0: the coarsest cut with at
+ * most that many items; 0: a few cuts are compared by the time a longest-first assignment of their items to the compute
+ * units would take, and `choice` keeps the winner, which is cut again without a comparison until the store has grown by
+ * 5 %.  A list with more items than compute units is cut for two eight-wavefront workgroups per compute unit, as chains
+ * of a pair's levels where the runs alone are many more than those places.  chains, pairs: -1 by these rules, 0 never,
+ * 1 always; waves: 0 by the items' length and widths, or 8, 12, 16.
+ * table (host int32, `capacity` integers) receives the items, the ranges at shape->range_at and, where shape->ordered, the
+ * dispatch order at shape->order_at; too small a table gives ODMKV_ENOSPACE with shape->need set.  No counterpart in the
+ * reference. */
+typedef struct odmkv_worklist_choice {
+    double multiple;                 /* items (or workgroups) per compute unit of the winning cut */
+    int64_t total_bytes;             /* packed bytes it was chosen at */
+    int32_t valid, chained, paired;
+} odmkv_worklist_choice_t;
+typedef struct odmkv_worklist_shape {
+    uint64_t need, range_at, order_at;               /* in integers of the table */
+    int32_t n_items, ordered, n_workgroups, two_per_cu, wavefronts;
+} odmkv_worklist_shape_t;
+int odmkv_worklist_cut(const int64_t* counts, const int64_t* seg_tile, int nseg, int n_cu, int64_t target_items,
+                       int64_t min_item_bytes, int chains, int pairs, int waves, odmkv_worklist_choice_t* choice,
+                       int32_t* table, uint64_t capacity, odmkv_worklist_shape_t* shape);
+
 size_t odmkv_decode_workspace_bytes(int B, int Hq, int n_items);
 /* The key rotation (random_rotation, kvquant/tq_backend.py:25-36, as TurboQuantMSE.dequantize applies it,
  * tq_backend.py:199-203) in the form the decode kernel multiplies the query by: pi_k device fp32 row-major [128,128];

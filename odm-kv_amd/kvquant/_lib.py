@@ -44,6 +44,17 @@ class Worklist(C.Structure):
     ]
 
 
+class WorklistChoice(C.Structure):
+    """struct odmkv_worklist_choice of include/odmkv.h."""
+    _fields_ = [("multiple", C.c_double), ("total_bytes", C.c_int64), ("valid", C.c_int32), ("chained", C.c_int32), ("paired", C.c_int32)]
+
+
+class WorklistShape(C.Structure):
+    """struct odmkv_worklist_shape of include/odmkv.h."""
+    _fields_ = [("need", C.c_uint64), ("range_at", C.c_uint64), ("order_at", C.c_uint64), ("n_items", C.c_int32),
+                ("ordered", C.c_int32), ("n_workgroups", C.c_int32), ("two_per_cu", C.c_int32), ("wavefronts", C.c_int32)]
+
+
 class Step(C.Structure):
     """struct odmkv_step of include/odmkv.h."""
     _fields_ = [
@@ -99,6 +110,8 @@ def _load() -> C.CDLL:
         "odmkv_decode_attn_static": (C.c_int, [vp, i32, i32, i32, f32, C.POINTER(Packed), C.POINTER(Worklist), vp, vp, vp,
                                                C.POINTER(C.c_float), C.POINTER(C.c_float), vp, i32, vp, vp]),
         "odmkv_decode_step": (C.c_int, [C.POINTER(Step), vp, vp, vp, i64, i64, i32, vp, vp, vp]),
+        "odmkv_worklist_cut": (C.c_int, [vp, vp, i32, i32, i64, i64, i32, i32, i32, C.POINTER(WorklistChoice), vp, C.c_uint64,
+                                         C.POINTER(WorklistShape)]),
         "odmkv_exact_tail": (C.c_int, [C.POINTER(Packed), i32, vp, vp, vp]),
         "odmkv_flush_score": (C.c_int, [vp, vp, i32, i32, i32, vp, f32, f32, i32, vp, vp, vp, vp]),
         "odmkv_flush_rank": (C.c_int, [vp, vp, i32, i32, i32, vp, vp, vp]),
@@ -116,7 +129,7 @@ EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "
            "odmkv_allocate_workspace_bytes", "odmkv_allocate", "odmkv_level_counts",
            "odmkv_store_init", "odmkv_store_gather", "odmkv_quant_pack_staged", "odmkv_store_layout", "odmkv_store_bind", "odmkv_pack_workspace_bytes", "odmkv_pack_count_chunks", "odmkv_store_finish_staged", "odmkv_quant_pack", "odmkv_quantize_rows",
            "odmkv_dequantize_rows", "odmkv_lloyd_max", "odmkv_dequant", "odmkv_dequant_from", "odmkv_append_exact",
-           "odmkv_decode_workspace_bytes", "odmkv_rotation_operands", "odmkv_decode_attn", "odmkv_decode_attn_static",
+           "odmkv_worklist_cut", "odmkv_decode_workspace_bytes", "odmkv_rotation_operands", "odmkv_decode_attn", "odmkv_decode_attn_static",
            "odmkv_decode_step", "odmkv_exact_tail", "odmkv_flush_score", "odmkv_flush_rank")
 
 

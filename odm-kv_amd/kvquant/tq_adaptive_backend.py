@@ -18,6 +18,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import os
 from typing import Optional
 
 import numpy as np
@@ -51,22 +52,6 @@ def _compute_units(device) -> int:
     if key not in _CU_COUNT:
         _CU_COUNT[key] = torch.cuda.get_device_properties(device).multi_processor_count
     return _CU_COUNT[key]
-_TILE_BYTES = [TILE * 16 * w + 2 * TILE * 4 for w in WIDTHS] + [2 * TILE * HEAD_DIM * 2]
-# what one compute unit was measured to need per 64-token tile of each level (nanoseconds; 2, 3, 4, 8 bits, exact rows)
-# and per work item (microseconds: start, table, query rotation, combining the wavefronts)
-_TILE_COST = [300, 420, 450, 890, 1310]
-_ITEM_FIXED_US = 4.0           # what the cuts without chains are compared with (its choices were measured shape by shape)
-# Chains (a workgroup that walks several quantised levels of a pair, _build_items) by a rule, not by the cost model, which
-# is off by a third either way on lists of several rounds: they are taken when the quantised runs number at least 1.5 per
-# compute unit and 2.5 per pair, cut so that the workgroups number 1.5 per compute unit or, with more pairs than that,
-# one per pair beside the exact items.  Measured whole calls: 64 sequences x 2048 tokens x 8 kv-heads, four levels each:
-# 90 -> 67 us; 16 x 8192 tokens with four levels: 44 -> 36 us; 16 x 8192 tokens with two levels (c3): no gain at any cut,
-# not taken by the rule.  The link and rotation costs below only rank the workgroups for the dispatch order.
-_CHAIN_LINK_US = 1.8
-_PAIR_CHAIN_RUNS_PER_PLACE = 1.5      # two workgroups per compute unit: chains where the runs number this many per place
-_CHAIN_ROTATE_US = 1.0
-_CHAIN_RUNS_PER_CU = 1.5
-_CHAIN_RUNS_PER_PAIR = 2.5
 
 
 _U64x33 = C.c_uint64 * 33
@@ -740,233 +725,42 @@ class TurboQuantAdaptiveKVCacheState:
     # ------------------------------------------------------------------ fused attention
     def _build_items(self, target_items: Optional[int] = None, min_item_bytes: Optional[int] = None) -> None:
         """The decode work list: every (segment, level) run of tiles cut into items of about equal
-        cost, one workgroup (one compute unit) per item.
+        cost, one workgroup (one compute unit) per item (odmkv_worklist_cut).
 
-        The cost of a tile is what the kernel was measured to need for it per level (the 2-bit loop is
-        bound by instruction issue, the wider ones and the exact rows by memory), plus a fixed part per item.
-        With a target the cut is the coarsest one that does not exceed it.  Without one, a few cuts
-        are compared by the time a longest-first assignment of their items to the compute units
-        would take, and the best is kept; when it has more items than compute units, the order in which
-        the workgroups take the items (longest first) is handed to the kernel as well.  Items of sixteen
-        tiles and more on average are run by sixteen (or twelve) wavefronts, shorter ones by eight.  A list
-        with more items than compute units is cut for two eight-wavefront workgroups per compute unit
-        (`two_per_cu`), as chains of a pair's levels where the runs alone are many more than those places."""
-        import os
-        n_cu = _compute_units(self.device)
-        env_target = int(os.environ.get("ODMKV_DECODE_ITEMS", 0))
-        min_item_bytes = int(os.environ.get("ODMKV_DECODE_MIN_ITEM_BYTES", 16384)) if min_item_bytes is None else min_item_bytes
-        used = (self._counts + TILE - 1) // TILE
-        used[4] = np.diff(self._seg_tile[4])              # exact segments grow between rebuilds
-        total_bytes = sum(int(used[li].sum()) * _TILE_BYTES[li] for li in range(5))
-        total = sum(int(used[li].sum()) * _TILE_COST[li] for li in range(5))      # cost units: nanoseconds of one compute unit
-        min_item_bytes = min_item_bytes * _TILE_COST[0] // _TILE_BYTES[0]          # the same floor, as a cost
-        # the runs of tiles, segment by segment (the merge finds a segment's items next to each other), as arrays
-        run_li, run_s = np.nonzero(used.T > 0)[1], np.nonzero(used.T > 0)[0]
-        run_nt = used[run_li, run_s].astype(np.int64)
-        run_t0 = self._seg_tile[run_li, run_s].astype(np.int64)
-        run_cnt = self._counts[run_li, run_s].astype(np.int64)
-        tile_cost = np.asarray(_TILE_COST, np.float64)
-
-        def steps_of(per_item: int) -> np.ndarray:                     # tiles per item, by level
-            return np.maximum(1, np.rint(per_item / tile_cost).astype(np.int64))
-
-        def n_pieces(per_item: int) -> int:
-            step = steps_of(per_item)[run_li]
-            return int((-(-run_nt // step)).sum())
-
-        def fit(target: int) -> int:
-            # the coarsest cut with at most `target` items (a run's last piece may be short)
-            per_item = max(total // max(target, 1), min_item_bytes)
-            while n_pieces(per_item) > target and per_item < total:
-                per_item += max(per_item // 64, 1)
-            return per_item
-
-        def cut(per_item: int) -> np.ndarray:
-            # rows (segment, level, first tile, tiles, tokens in those tiles, segment's first tile, -, -)
-            step = steps_of(per_item)[run_li]
-            pieces = -(-run_nt // step)
-            run = np.repeat(np.arange(run_nt.size), pieces)
-            a0 = (np.arange(run.size) - np.repeat(np.cumsum(pieces) - pieces, pieces)) * step[run]
-            n = np.minimum(step[run], run_nt[run] - a0)
-            out = np.zeros((run.size, 8), np.int64)
-            out[:, 0], out[:, 1], out[:, 2], out[:, 3] = run_s[run], run_li[run], run_t0[run] + a0, n
-            out[:, 4], out[:, 5] = np.minimum(run_cnt[run] - a0 * TILE, n * TILE), run_t0[run]
-            return out
-
-        # -- chains: the quantised levels of a segment as ONE run of work, cut into pieces of equal cost; a piece that
-        # crosses a level boundary becomes consecutive items of one workgroup (one query rotation, one result)
-        qr = run_li < 4
-        q_s, q_li, q_nt, q_t0, q_cnt = run_s[qr], run_li[qr], run_nt[qr], run_t0[qr], run_cnt[qr]
-        q_cost = q_nt * tile_cost[q_li]
-        q_end = np.cumsum(q_cost)
-        q_start = q_end - q_cost
-        seg_cost = np.bincount(q_s, q_cost, minlength=self._nseg) if q_s.size else np.zeros(self._nseg)
-        seg_start = np.cumsum(seg_cost) - seg_cost
-        q_first = np.ones(q_s.size, bool)
-        q_first[1:] = q_s[1:] != q_s[:-1]                               # a segment's first quantised run
-
-        def chain_pieces(per_item: int) -> np.ndarray:                  # workgroups per segment
-            return np.ceil(seg_cost / max(per_item, 1)).astype(np.int64)
-
-        def cut_exact(per_item: int) -> np.ndarray:
-            keep = run_li == 4
-            step = steps_of(per_item)[4]
-            nt, t0 = run_nt[keep], run_t0[keep]
-            pieces = -(-nt // step)
-            run = np.repeat(np.arange(nt.size), pieces)
-            a0 = (np.arange(run.size) - np.repeat(np.cumsum(pieces) - pieces, pieces)) * step
-            n = np.minimum(step, nt[run] - a0)
-            out = np.zeros((run.size, 8), np.int64)
-            out[:, 0], out[:, 1], out[:, 2], out[:, 3] = run_s[keep][run], 4, t0[run] + a0, n
-            out[:, 4], out[:, 5] = np.minimum(run_cnt[keep][run] - a0 * TILE, n * TILE), t0[run]
-            return out
-
-        def cut_chained(per_item: int) -> np.ndarray:
-            # rows as in cut(), word 6 = items that follow in the same workgroup, word 7 = 1 for those items
-            k = chain_pieces(per_item)
-            nb = np.maximum(k - 1, 0)
-            b_s = np.repeat(np.arange(self._nseg), nb)                  # one row per inner piece boundary
-            b_j = np.arange(b_s.size) - np.repeat(np.cumsum(nb) - nb, nb) + 1
-            x = seg_start[b_s] + b_j * seg_cost[b_s] / k[b_s]           # where the boundary lies on the line of all runs' cost
-            run = np.minimum(np.searchsorted(q_end, x, side="right"), q_s.size - 1)
-            off = np.clip(np.rint((x - q_start[run]) / tile_cost[q_li[run]]).astype(np.int64), 0, q_nt[run])
-            at_end = off == q_nt[run]                                   # a boundary on a run's end belongs to the next run's start
-            run, off = np.where(at_end, np.minimum(run + 1, q_s.size - 1), run), np.where(at_end, 0, off)
-            # the items' starts: every run's first tile, and the boundaries inside runs
-            st_run = np.concatenate([np.arange(q_s.size), run])
-            st_off = np.concatenate([np.zeros(q_s.size, np.int64), off])
-            st_head = np.concatenate([q_first, np.ones(run.size, bool)])  # starts a workgroup's chain
-            order_ = np.lexsort((~st_head, st_off, st_run))             # duplicates: the one that starts a chain first
-            st_run, st_off, st_head = st_run[order_], st_off[order_], st_head[order_]
-            uniq = np.ones(st_run.size, bool)
-            uniq[1:] = (st_run[1:] != st_run[:-1]) | (st_off[1:] != st_off[:-1])
-            st_run, st_off, st_head = st_run[uniq], st_off[uniq], st_head[uniq]
-            nxt = np.append(st_off[1:], 0)
-            last_of_run = np.append(st_run[1:] != st_run[:-1], True)
-            n = np.where(last_of_run, q_nt[st_run], nxt) - st_off
-            out = np.zeros((st_run.size, 8), np.int64)
-            out[:, 0], out[:, 1], out[:, 2], out[:, 3] = q_s[st_run], q_li[st_run], q_t0[st_run] + st_off, n
-            out[:, 4], out[:, 5] = np.minimum(q_cnt[st_run] - st_off * TILE, n * TILE), q_t0[st_run]
-            head_idx = np.flatnonzero(st_head)
-            follow = np.diff(np.append(head_idx, st_run.size)) - 1
-            out[head_idx, 6] = follow
-            out[:, 7] = ~st_head
-            both = np.concatenate([out, cut_exact(per_item)])
-            return both[np.lexsort((both[:, 2], both[:, 1] & 7, both[:, 0]))]
-
-        def fit_chained(target: int) -> int:
-            per_item = max(total // max(target, 1), min_item_bytes)
-            n_exact = lambda p: int((-(-run_nt[run_li == 4] // steps_of(p)[4])).sum())
-            while int(chain_pieces(per_item).sum()) + n_exact(per_item) > target and per_item < total:
-                per_item += max(per_item // 64, 1)
-            return per_item
-
-        def cost(items: np.ndarray, fixed: float = _ITEM_FIXED_US) -> np.ndarray:
-            # microseconds of one workgroup, roughly: per workgroup (an item with word 7 set adds to the one before it)
-            own = items[:, 3] * tile_cost[items[:, 1] & 7] * 1e-3
-            head = items[:, 7] == 0
-            group = np.cumsum(head) - 1
-            return (fixed + np.bincount(group, own, minlength=int(head.sum()))
-                    + _CHAIN_LINK_US * items[head, 6] + np.where(items[head, 6] > 0, _CHAIN_ROTATE_US, 0.0))
-
-        def makespan(items: np.ndarray, fixed: float = _ITEM_FIXED_US) -> float:
-            import heapq
-            free = [0.0] * n_cu
-            for c in sorted(cost(items, fixed).tolist(), reverse=True):
-                heapq.heappush(free, heapq.heappop(free) + c)
-            return max(free)
-
-        chain_env = os.environ.get("ODMKV_DECODE_CHAINS")                # "0": never, "1": always (measurements)
-        pair_env = os.environ.get("ODMKV_DECODE_PAIRS")                  # the same for two workgroups per compute unit
-        may_chain = q_s.size > 0 and bool((~q_first).any()) and chain_env != "0"
-        explicit = target_items if target_items is not None else (env_target or None)
-        paired = pair_env == "1"
-        if explicit is not None:
-            items = cut_chained(fit_chained(int(explicit))) if (may_chain and chain_env == "1") else cut(fit(int(explicit)))
-        else:
-            # the comparison is repeated only when the store has grown by more than 5 % since the
-            # last one (a decode-time flush adds a fraction of a percent): until then its winner is re-cut
-            chosen = self._items_choice
-            if chosen is not None and abs(total_bytes - chosen[1]) <= 0.05 * chosen[1]:
-                items = (cut_chained(fit_chained(int(n_cu * chosen[0]))) if chosen[2] and may_chain
-                         else cut(fit(int(n_cu * chosen[0]))))
-                paired = chosen[3]
-            else:
-                best = None
-                if chain_env != "1" or not may_chain:
-                    for mult in (1.0, 1.5, 2.0, 3.0, 4.0):
-                        cand = cut(fit(int(n_cu * mult)))
-                        t = makespan(cand)
-                        if best is None or t < best[0] - 1e-9:
-                            best = (t, cand, mult, False)
-                n_pairs = int(q_first.sum())
-                n_exact = int((run_li == 4).sum())
-                if pair_env != "0" and (paired or (best is not None and len(best[1]) > n_cu)):
-                    # More items than compute units: the workgroups would run in rounds, each paying its start (work item,
-                    # rotation, table, first bytes: about 4 us) and its end (combine) with the compute unit to itself.
-                    # Two eight-wavefront workgroups per compute unit overlap one's start and end with the other's
-                    # stream (measured: a 16 x 8192-token batch 28.1 -> 25.9 us, 64 x 2048 tokens 52 -> 40 us; lists of
-                    # one item per compute unit lose 5-10 %, and keep the wide workgroups).  Cut for one round of the
-                    # 2 x n_cu places; where the runs alone are many more than that, chain a pair's levels instead.
-                    paired = True
-                    if may_chain and (chain_env == "1" or q_s.size + n_exact > _PAIR_CHAIN_RUNS_PER_PLACE * 2 * n_cu):
-                        mult = max(2.0, (n_pairs + n_exact) / n_cu)
-                        best = (0.0, cut_chained(fit_chained(int(n_cu * mult))), mult, True)
-                    else:
-                        best = (0.0, cut(fit(2 * n_cu)), 2.0, False)
-                elif may_chain and (chain_env == "1" or (q_s.size >= _CHAIN_RUNS_PER_CU * n_cu
-                                                         and q_s.size >= _CHAIN_RUNS_PER_PAIR * n_pairs)):
-                    mult = max(1.5, (n_pairs + n_exact) / n_cu)
-                    best = (0.0, cut_chained(fit_chained(int(n_cu * mult))), mult, True)
-                items = best[1]
-                self._items_choice = (best[2], total_bytes, best[3], paired)
-        arr = items.astype(np.int32).reshape(-1, 8)
-        per_seg = np.bincount(arr[:, 0], minlength=self._nseg) if len(items) else np.zeros(self._nseg, np.int64)
-        ranges = np.concatenate([[0], np.cumsum(per_seg)])          # items are generated in segment order
-        order = None
-        heads = np.flatnonzero(arr[:, 7] == 0) if len(items) else np.zeros(0, np.int64)
-        chained = len(items) > 0 and heads.size != len(items)
-        paired = paired and len(items) > 0
-        if len(items) > n_cu or chained or paired:
-            # the workgroups' first items, longest workgroup first
-            order = heads[np.argsort(-cost(items), kind="stable")].astype(np.int32)
-            if paired and order.size > n_cu:
-                # two per compute unit: the first n_cu workgroups land one per compute unit, the next n_cu beside them in
-                # the same order of compute units; taken shortest first, the shortest joins the longest (a 16 x 8192-token
-                # batch 26.0 -> 25.5 us; long and short alternating: 32 us)
-                order = np.concatenate([order[:n_cu], order[n_cu:2 * n_cu][::-1], order[2 * n_cu:]]).astype(np.int32)
-        # one upload for the item table, the ranges and the order (the parts start at multiples of 4 integers)
-        n_arr, n_rng = arr.size, (ranges.size + 3) & ~3
-        blob = np.zeros(n_arr + n_rng + (0 if order is None else order.size), np.int32)
-        blob[:n_arr] = arr.reshape(-1)
-        blob[n_arr:n_arr + ranges.size] = ranges
-        if order is not None:
-            blob[n_arr + n_rng:] = order
-        dev_blob = torch.from_numpy(blob).to(self.device)
-        self._item_order = None if order is None else dev_blob[n_arr + n_rng:]
-        self._items = (dev_blob[:n_arr].view(-1, 8), dev_blob[n_arr:n_arr + ranges.size], len(items))
+        `target_items`: the coarsest cut with at most that many items, instead of the one the library finds best."""
+        env = os.environ.get
+        if target_items is None:
+            target_items = int(env("ODMKV_DECODE_ITEMS", 0))
+        if min_item_bytes is None:
+            min_item_bytes = int(env("ODMKV_DECODE_MIN_ITEM_BYTES", 16384))
+        chains, pairs = env("ODMKV_DECODE_CHAINS"), env("ODMKV_DECODE_PAIRS")      # "0": never, "1": always (measurements)
+        mode = {"0": 0, "1": 1}
+        choice = self._items_choice
+        if choice is None:
+            choice = _lib.WorklistChoice()
+            if target_items <= 0:
+                self._items_choice = choice
+        counts, tiles = np.ascontiguousarray(self._counts), np.ascontiguousarray(self._seg_tile)
+        shape, on_gpu = _lib.WorklistShape(), self.device.type == "cuda"
+        room = 8192
+        while True:
+            # (page-locked: the upload then waits for nothing; from pageable memory it waited for the stream to run dry)
+            table = torch.empty(room, dtype=torch.int32, pin_memory=on_gpu)
+            rc = lib.odmkv_worklist_cut(counts.ctypes.data, tiles.ctypes.data, self._nseg, _compute_units(self.device),
+                                        int(target_items), int(min_item_bytes), mode.get(chains, -1), mode.get(pairs, -1),
+                                        int(env("ODMKV_DECODE_WAVES", 0)), C.byref(choice), table.data_ptr(), room, C.byref(shape))
+            if rc != -2:
+                break
+            room = int(shape.need)
+        _lib.check(rc)
+        dev_table = table[:shape.need].to(self.device, non_blocking=True)
+        self._item_order = dev_table[shape.order_at:] if shape.ordered else None
+        self._items = (dev_table[:shape.range_at].view(-1, 8), dev_table[shape.range_at:shape.range_at + self._nseg + 1], int(shape.n_items))
         w = _lib.Worklist()
         w.items, w.item_range = self._items[0].data_ptr(), self._items[1].data_ptr()
         w.dispatch_order = _lib.ptr(self._item_order)
-        w.n_items = len(items)
-        w.n_workgroups = int(heads.size) if chained else 0
-        # wavefronts per item: eight for short items (less set-up, a lighter combine); for long ones sixteen where
-        # the narrow levels carry the bytes (their loop wants four wavefronts per SIMD) and twelve where 4- and 8-bit
-        # tokens do (memory-bound: a third unit in flight per wavefront pays more than the fourth wavefront)
-        if chained:                                                     # quantised tiles per workgroup
-            qi = (arr[:, 1] & 7) < 4
-            quant = np.bincount((np.cumsum(arr[:, 7] == 0) - 1)[qi], arr[qi, 3])
-            quant = quant[quant > 0]
-        else:
-            quant = arr[arr[:, 1] < 4, 3] if len(items) else arr[:0, 3]
-        q_bytes = [int(used[li].sum()) * _TILE_BYTES[li] for li in range(4)]
-        wide = (q_bytes[2] + q_bytes[3]) >= 0.4 * max(sum(q_bytes), 1)
-        # (items of 6 to 15 tiles that are mostly 3 bits and wider: twelve as well, 2-3 % ahead of eight, measured on
-        # a 28-head, 3-bit store of 32k tokens: their loops wait on memory, and a third unit in flight pays)
-        medium = bool(quant.size) and 6 <= quant.mean() < 16 and (sum(q_bytes) - q_bytes[0]) >= 0.5 * max(sum(q_bytes), 1)
-        auto = (12 if medium else 8) if not (quant.size and quant.mean() >= 16) else (12 if wide else 16)
-        w.wavefronts = 8 if paired else (int(os.environ.get("ODMKV_DECODE_WAVES", 0)) or auto)
-        w.two_per_cu = int(paired)
+        w.n_items, w.n_workgroups = shape.n_items, shape.n_workgroups
+        w.wavefronts, w.two_per_cu = shape.wavefronts, shape.two_per_cu
         self._worklist = w
 
     def decode_attention_block(self, query: torch.Tensor, scaling: Optional[float] = None):
