@@ -175,6 +175,24 @@ typedef struct odmkv_packed {
  * (The per-level mask / nonzero of tq_adaptive_backend.py:355-361.) */
 int odmkv_level_counts(const int32_t* bits, int B, int Hkv, int T, int32_t* counts, void* stream);
 
+/* A layer's levels between the allocation and the store, in one pass over bits (device int32 [rows, T], 16-byte aligned;
+ * rows = B*Hkv): the tokens from tail_begin on are set to 16 bits (in bits too), the levels are written down as bytes
+ * (device uint8 [rows, stride], T levels followed by 16s: what the store's level map reads behind the last token), and
+ * they are counted: counts int32 [rows, odmkv_finish_levels_chunks(stride), 2, 6], device memory or page-locked host
+ * memory, holds for every chunk of 4096 tokens the tokens of [count_begin, count_end) per level as they came (evicted, 2, 3,
+ * 4, 8, 16 bits) and all tokens as they are stored; a value that is no level is counted nowhere.  (The reference counts the
+ * prefill's level shares and sets the window in tensor operations: kvquant/adaptive_backend_press.py:292-325.) */
+int odmkv_finish_levels_chunks(int64_t stride);
+int odmkv_finish_levels(int32_t* bits, int rows, int T, int count_begin, int count_end, int tail_begin,
+                        uint8_t* levels, int64_t stride, int32_t* counts, void* stream);
+
+/* The evicted (0-bit) positions of a level map (device uint8 [B*Hkv, stride], T levels per row) in the order (sequence,
+ * head, token): out device int64 [3, n], n the caller's own count of them (masked_key_indices,
+ * kvquant/tq_adaptive_backend.py:499-505).  workspace: odmkv_evicted_workspace_bytes. */
+size_t odmkv_evicted_workspace_bytes(int B, int Hkv, int T);
+int odmkv_evicted_indices(const uint8_t* levels, int B, int Hkv, int T, int64_t stride, int64_t n, int64_t* out,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 /* Host arithmetic for callers that keep a store in ONE device allocation: where its 33 buffers lie, given the
  * segments' first tiles (seg_tile: host int32 [5][nseg + 1], the last entry of a row = tiles of the level).
  * Order: seg_tile[5], seg_count[5], (knorm, vnorm)[4], kexact, vexact, pos[5], (kcodes, vcodes)[4]; offsets and
@@ -211,7 +229,8 @@ int odmkv_store_gather(const odmkv_packed_t* staging, const odmkv_packed_t* stor
  * first of them need not move the store (seg_tile: host int32 [5][B*Hkv + 1], written); the store is laid out in `arena` (offsets, sizes, marks as odmkv_store_layout gives them), prepared
  * (odmkv_store_init), described (odmkv_store_bind into `store`) and filled from the staging store
  * (odmkv_store_gather).  need_bytes receives the size of the layout; if `arena` is NULL or smaller, nothing is
- * launched and ODMKV_ENOSPACE returned: allocate and call again.  Counts that do not add up to B*Hkv*T (a value that
+ * launched and ODMKV_ENOSPACE returned: allocate and call again.  `staging` may be NULL: the store is laid out and prepared
+ * and stays empty (for callers that know the counts and quantise straight into it).  Counts that do not add up to B*Hkv*T (a value that
  * is no level) give ODMKV_EINVAL.  No counterpart in the reference. */
 int odmkv_store_finish_staged(const int32_t* chunk_counts, int n_chunks, int B, int Hkv, int T,
                               int exact_slack, int quant_headroom, int exact_dtype, void* arena, uint64_t arena_bytes,

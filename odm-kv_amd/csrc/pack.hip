@@ -1801,7 +1801,7 @@ extern "C" int odmkv_store_finish_staged(const int32_t* chunk_counts, int n_chun
                                          const odmkv_packed_t* staging, int32_t* counts, int32_t* seg_tile,
                                          uint64_t* offsets, uint64_t* sizes, uint64_t* marks,
                                          odmkv_packed_t* store, uint64_t* need_bytes, void* stream) {
-    ODMKV_CHECK_ARG(chunk_counts && staging && counts && seg_tile && offsets && sizes && marks && store && need_bytes,
+    ODMKV_CHECK_ARG(chunk_counts && counts && seg_tile && offsets && sizes && marks && store && need_bytes,
                     "store_finish_staged: null pointer");
     ODMKV_CHECK_ARG(B > 0 && Hkv > 0 && T > 0 && n_chunks > 0 && exact_slack >= 0, "store_finish_staged: bad shape");
     const int nseg = B * Hkv;
@@ -1833,7 +1833,7 @@ extern "C" int odmkv_store_finish_staged(const int32_t* chunk_counts, int n_chun
     }
     if (int rc = odmkv_store_init(arena, seg_tile, 5, nseg + 1, offsets, marks[0], marks[2], marks[3], stream)) return rc;
     if (int rc = odmkv_store_bind(arena, offsets, seg_tile, nseg, B, Hkv, exact_dtype, store)) return rc;
-    return odmkv_store_gather(staging, store, stream);
+    return staging ? odmkv_store_gather(staging, store, stream) : 0;
 }
 
 // ------------------------------------------------------------------------------------------------

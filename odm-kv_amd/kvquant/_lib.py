@@ -85,6 +85,10 @@ def _load() -> C.CDLL:
         "odmkv_allocate": (C.c_int, [vp, i32, i32, vp, i32, i32, i32, C.POINTER(C.c_int32), i32,
                                      C.POINTER(C.c_double), vp, vp, vp, vp, vp, sz, vp]),
         "odmkv_level_counts": (C.c_int, [vp, i32, i32, i32, vp, vp]),
+        "odmkv_finish_levels_chunks": (C.c_int, [i64]),
+        "odmkv_finish_levels": (C.c_int, [vp, i32, i32, i32, i32, i32, vp, i64, vp, vp]),
+        "odmkv_evicted_workspace_bytes": (sz, [i32, i32, i32]),
+        "odmkv_evicted_indices": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, vp, sz, vp]),
         "odmkv_store_init": (C.c_int, [vp, vp, i32, i32, vp, C.c_uint64, C.c_uint64, C.c_uint64, vp]),
         "odmkv_store_gather": (C.c_int, [C.POINTER(Packed), C.POINTER(Packed), vp]),
         "odmkv_quant_pack_staged": (C.c_int, [vp, vp, i32, i32, i32, i32, i64, i64, i64, vp, i32, vp, vp, vp,
@@ -127,6 +131,7 @@ lib = _load()
 EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "odmkv_score", "odmkv_score_model_dtype", "odmkv_score_expected",
            "odmkv_window_attention_workspace_bytes", "odmkv_window_attention",
            "odmkv_allocate_workspace_bytes", "odmkv_allocate", "odmkv_level_counts",
+           "odmkv_finish_levels_chunks", "odmkv_finish_levels", "odmkv_evicted_workspace_bytes", "odmkv_evicted_indices",
            "odmkv_store_init", "odmkv_store_gather", "odmkv_quant_pack_staged", "odmkv_store_layout", "odmkv_store_bind", "odmkv_pack_workspace_bytes", "odmkv_pack_count_chunks", "odmkv_store_finish_staged", "odmkv_quant_pack", "odmkv_quantize_rows",
            "odmkv_dequantize_rows", "odmkv_lloyd_max", "odmkv_dequant", "odmkv_dequant_from", "odmkv_append_exact",
            "odmkv_worklist_cut", "odmkv_decode_workspace_bytes", "odmkv_rotation_operands", "odmkv_decode_attn", "odmkv_decode_attn_static",

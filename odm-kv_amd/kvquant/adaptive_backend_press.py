@@ -148,28 +148,32 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
         self._attach(cache, layer_idx, module, state)
 
     # ------------------------------------------------------------------ cached ratios
+    def _bulk(self, T: int) -> tuple[int, int]:
+        """The prefill positions whose level shares are recorded: sinks and the protected tail left out."""
+        start = min(int(self.sink_tokens), T) if self.sink_tokens > 0 else 0
+        end = T - min(int(self.buffer_size), T) if self.buffer_size > 0 else T
+        return (start, end) if end > start else (0, T)
+
     def _record_observed_ratios(self, layer_idx: int, bits: torch.Tensor) -> None:
         """Level fractions per kv-head over the bulk of the prefill (sinks and the protected tail
         left out), taken before the window override."""
         if bits.dim() != 3 or bits.shape[-1] == 0:
             return
         B, H, T = bits.shape
-        start = min(int(self.sink_tokens), T) if self.sink_tokens > 0 else 0
-        end = T - min(int(self.buffer_size), T) if self.buffer_size > 0 else T
-        if end <= start:
-            start, end = 0, T
+        start, end = self._bulk(T)
         bulk = bits[..., start:end].reshape(B * H, end - start)
         levels = sorted(set(int(b) for b in self.bit_levels) | {16})
         lv = torch.tensor(levels, device=bits.device, dtype=bits.dtype)
-        counts = (bulk.unsqueeze(-1) == lv).sum(dim=1).cpu()                 # [B*H, K], one transfer
-        for row in range(B * H):
-            c = counts[row]
-            total = int(c.sum())
-            if total == 0:
-                continue
-            fracs = (c.float() / total).tolist()
-            self._observed_ratios[(layer_idx, row % H)] = tuple(
-                (b, f) for b, f, n in zip(levels, fracs, c.tolist()) if n > 0)
+        self._store_observed_ratios(layer_idx, H, levels, (bulk.unsqueeze(-1) == lv).sum(dim=1).cpu().numpy())
+
+    def _store_observed_ratios(self, layer_idx: int, num_heads: int, levels, counts) -> None:
+        """counts [B*H, K]: bulk tokens of every (sequence, kv-head) at each of `levels`."""
+        import numpy as np
+        totals = counts.sum(axis=1)
+        fracs = counts.astype(np.float32) / np.maximum(totals, 1).astype(np.float32)[:, None]
+        for row, (total, c, f) in enumerate(zip(totals.tolist(), counts.tolist(), fracs.tolist())):
+            if total:
+                self._observed_ratios[(layer_idx, row % num_heads)] = tuple((b, x) for b, x, n in zip(levels, f, c) if n > 0)
 
     def _allocate_bits_via_cached_ratios(self, scores, positions, num_heads, layer_idx, allowed_levels,
                                          batch_size: Optional[int] = None):
@@ -215,16 +219,38 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
     def _finalize_prefill(self, cache) -> None:
         if self.n_outlier_channels > 0:
             raise NotImplementedError("outlier-channel separation is not built (n_outlier_channels must be 0)")
+        plan = []                   # per layer: index, bits (int32), level map, counts (page-locked)
+        arrived = {}
         for layer_idx, bits in self._allocate_bits_for_prefill().items():
+            keys, _ = self._get_cache_tensors(cache, layer_idx)
+            dev = keys.device
+            bits = bits.to(dtype=torch.int32, device=dev).contiguous()
+            B, H, T = bits.shape
+            # one pass over the levels: bulk shares counted, the window (or the whole layer) set to 16, the level map
+            # written; the counts go straight to page-locked memory, and all layers share the one wait below
+            room = (T + 2 * self.buffer_size + 255) & ~255
+            levels = torch.empty((B, H, room), dtype=torch.uint8, device=dev)
+            chunks = _lib.lib.odmkv_finish_levels_chunks(room)
+            counts = torch.empty((B * H, chunks, 2, 6), dtype=torch.int32, pin_memory=True)
+            start, end = self._bulk(T)
+            tail = 0 if layer_idx < self.initial_layers_fp16 else T - min(max(self.buffer_size, 0), T)
+            with torch.cuda.device(dev):
+                _lib.check(_lib.lib.odmkv_finish_levels(bits.data_ptr(), B * H, T, start, end, tail, levels.data_ptr(), room,
+                                                        counts.data_ptr(), _lib.stream_ptr(dev)))
+                ev = arrived.setdefault(dev, torch.cuda.Event())
+                ev.record(torch.cuda.current_stream(dev))
+            plan.append((layer_idx, bits, levels, counts))
+        for layer_idx, *_ in plan:                                # (the host's part while the counts are on their way)
+            self._get_or_create_state(layer_idx, self._get_cache_tensors(cache, layer_idx)[0])
+        for ev in arrived.values():
+            ev.synchronize()
+        for layer_idx, bits, levels, counts in plan:
             keys, values = self._get_cache_tensors(cache, layer_idx)
-            self._record_observed_ratios(layer_idx, bits)
-            if layer_idx < self.initial_layers_fp16:
-                bits = torch.full_like(bits, 16)
-            elif self.buffer_size > 0:
-                bits = bits.clone()
-                bits[..., -min(self.buffer_size, bits.shape[-1]):] = 16
+            bulk, stored = counts.sum(dim=1).numpy().swapaxes(0, 1)
+            wanted = sorted(set(int(b) for b in self.bit_levels) | {16})
+            self._store_observed_ratios(layer_idx, bits.shape[1], wanted, bulk[:, [_lib.LEVEL_ORDER.index(b) for b in wanted]])
             state = self._get_or_create_state(layer_idx, keys)
-            state.prefill(keys, values, bits.to(dtype=torch.int32, device=keys.device))
+            state.prefill(keys, values, bits, _known_counts=stored, _levels=levels)
             module = self._layer_modules.get(layer_idx)
             if module is not None:
                 if self.release_dense_cache and layer_idx >= self.initial_layers_fp16:

@@ -138,11 +138,11 @@ def _dev_key(dev) -> str:
 
 def reserve_state_memory(device, n_states: int) -> None:
     """Grow the allocator's small-block pool, in one go, by what `n_states` stores will keep in it (rotations, operand
-    and centroid tables, work lists: about a third of a megabyte each).  Otherwise the pool grows by one 2 MB device
+    and centroid tables, level maps, work lists: up to three quarters of a megabyte each).  Otherwise the pool grows by one 2 MB device
     allocation every few layers of a first prefill, 0.2 ms of host time each, at whatever small request comes next:
     between the kernels of a layer's compression.  The blocks go back to the pool at once; a process that has served a
     prompt before has them anyway."""
-    hold = [torch.empty(384 << 10, dtype=torch.uint8, device=device) for _ in range(int(n_states))]
+    hold = [torch.empty(768 << 10, dtype=torch.uint8, device=device) for _ in range(int(n_states))]
     del hold
 
 
@@ -218,6 +218,20 @@ def _rotation_operands(pi_k: torch.Tensor) -> torch.Tensor:
     return hit[1]
 
 
+_DECODE_OPERANDS: dict = {}
+
+
+def _decode_operands(head_dim: int, device):
+    """(scaled centroid tables on `device`, the same on the host, reciprocal scales): the two host blocks as the library
+    takes them.  One set per (dim, device), shared by all stores (reading the tables back waits for the stream)."""
+    key = (head_dim, str(device))
+    got = _DECODE_OPERANDS.get(key)
+    if got is None:
+        table, inv = decode_tables(head_dim, device)
+        got = _DECODE_OPERANDS[key] = (table, (C.c_float * 284)(*table.cpu().tolist()), (C.c_float * 4)(*inv))
+    return got
+
+
 def _empty_positions(device) -> torch.Tensor:
     return torch.empty((0, 3), dtype=torch.long, device=device)
 
@@ -268,9 +282,7 @@ class TurboQuantAdaptiveKVCacheState:
         # the key rotation as the decode kernel's matrix operands (fp16 high + low parts in operand order)
         self._pi_k_ops = _rotation_operands(self.pi_k)
         self.codebooks = codebook_table(head_dim, self.device)
-        self._decode_cb, inv = decode_tables(head_dim, self.device)
-        self._decode_inv = (C.c_float * 4)(*inv)
-        self._decode_cb_host = (C.c_float * 284)(*self._decode_cb.cpu().tolist())
+        self._decode_cb, self._decode_cb_host, self._decode_inv = _decode_operands(head_dim, self.device)
         self._exact_torch_dtype = torch.bfloat16 if dtype == torch.bfloat16 else torch.float16
         self._reset()
 
@@ -418,14 +430,41 @@ class TurboQuantAdaptiveKVCacheState:
                 and t.stride(2) >= t.shape[-1] and t.data_ptr() % 16 == 0)
 
     # ------------------------------------------------------------------ writes
-    def prefill(self, keys: torch.Tensor, values: torch.Tensor, bits: torch.Tensor) -> None:
+    def prefill(self, keys: torch.Tensor, values: torch.Tensor, bits: torch.Tensor,
+                _known_counts: Optional[np.ndarray] = None, _levels: Optional[torch.Tensor] = None) -> None:
         self._reset()
-        self.append(keys, values, bits)
+        self.append(keys, values, bits, _known_counts=_known_counts, _levels=_levels)
+
+    def _lay_out_first_fill(self, chunk_counts, n_chunks: int, T: int, staging, tail_bytes: int, stream: int) -> np.ndarray:
+        """Size the store's segments for the level counts (host int32 [B*H, n_chunks, 6]), lay it out and prepare it, and
+        move what `staging` holds into it, in one library call; `tail_bytes` are kept free behind it in its allocation."""
+        layout, packed, counts = _Layout.blank(self._nseg), Packed(), np.zeros((self._nseg, 6), np.int32)
+        need = C.c_uint64(0)
+        for attempt in (0, 1):
+            arena = getattr(self, "_arena", None)
+            rc = lib.odmkv_store_finish_staged(
+                chunk_counts, n_chunks, self.batch_size, self.num_heads, T, int(self.exact_slack), int(self.quant_headroom),
+                _lib.BF16 if self._exact_torch_dtype == torch.bfloat16 else _lib.F16,
+                None if arena is None else arena.data_ptr(), 0 if arena is None else max(arena.numel() - tail_bytes, 0),
+                None if staging is None else C.byref(staging.packed), counts.ctypes.data, layout.tables_ptr, layout.offsets,
+                layout.sizes, layout.marks, C.byref(packed), C.byref(need), stream)
+            if rc != -2 or attempt == 1:
+                break
+            self._arena = torch.empty(int(need.value) + int(need.value) // 8 + tail_bytes, dtype=torch.uint8, device=self.device)
+            self._arena_spare = None
+        _lib.check(rc)
+        self._bufs = _Buffers(self._arena, layout.adopt(), self._exact_torch_dtype)
+        self._seg_tile = layout.tables.astype(np.int64)
+        self._packed = packed
+        return counts.astype(np.int64)
 
     def append(self, keys: torch.Tensor, values: torch.Tensor, bits: torch.Tensor,
-               _pos_offset: Optional[int] = None, _known_counts: Optional[np.ndarray] = None) -> None:
+               _pos_offset: Optional[int] = None, _known_counts: Optional[np.ndarray] = None,
+               _levels: Optional[torch.Tensor] = None) -> None:
         """_known_counts (int [B*H, 6], levels 0, 2, 3, 4, 8, 16): what odmkv_level_counts would return for `bits`,
-        when the caller knows it without looking (levels assigned by rank with fixed shares): no read-back."""
+        when the caller knows it without looking (levels assigned by rank with fixed shares, or counted already):
+        no read-back.  _levels (first fill only): uint8 [B, H, >= T], `bits` as bytes and 16 behind them, kept as the
+        store's level map."""
         self._validate_shapes(keys, values, bits)
         B, H, T, D = keys.shape
         if T == 0:
@@ -471,22 +510,7 @@ class TurboQuantAdaptiveKVCacheState:
                 self._arena = torch.empty(_ARENA_HINT[hint_key], dtype=torch.uint8, device=dev)
             arrived.synchronize()                                     # the one wait: for the counts alone
             # what remains up to the launch of the gather is one call (the GPU has the quantiser's run to wait for it)
-            new_lay, new_packed, counts32 = _Layout.blank(self._nseg), Packed(), np.zeros((self._nseg, 6), np.int32)
-            need = C.c_uint64(0)
-            for attempt in (0, 1):
-                arena = getattr(self, "_arena", None)
-                rc = lib.odmkv_store_finish_staged(
-                    box.data_ptr(), n_chunks, B, H, T, int(self.exact_slack), int(self.quant_headroom),
-                    _lib.BF16 if self._exact_torch_dtype == torch.bfloat16 else _lib.F16,
-                    None if arena is None else arena.data_ptr(), 0 if arena is None else max(arena.numel() - lm_bytes, 0),
-                    C.byref(stg.packed), counts32.ctypes.data, new_lay.tables_ptr, new_lay.offsets, new_lay.sizes,
-                    new_lay.marks, C.byref(new_packed), C.byref(need), st)
-                if rc != -2 or attempt == 1:
-                    break
-                self._arena = torch.empty(int(need.value) + int(need.value) // 8 + lm_bytes, dtype=torch.uint8, device=dev)
-                self._arena_spare = None
-            _lib.check(rc)
-            counts = counts32.astype(np.int64)
+            counts = self._lay_out_first_fill(box.data_ptr(), n_chunks, T, stg, lm_bytes, st)
         else:
             counts_dev = torch.empty(self._nseg, 6, dtype=torch.int32, device=dev)
             _lib.check(lib.odmkv_level_counts(bits.data_ptr(), B, H, T, counts_dev.data_ptr(), st))
@@ -503,13 +527,12 @@ class TurboQuantAdaptiveKVCacheState:
         if not present <= set(self.bit_levels):
             raise ValueError(f"bits use levels {sorted(present - set(self.bit_levels))} outside bit_levels={self.bit_levels}")
         new_counts = self._counts + counts[:, 1:].T
-        if stg is not None:
-            # laid out, prepared and filled by odmkv_store_finish_staged above
-            self._bufs = _Buffers(self._arena, new_lay.adopt(), self._exact_torch_dtype)
-            self._seg_tile = new_lay.tables.astype(np.int64)
-            self._packed = new_packed
-        else:
-            self._ensure_capacity(new_counts)
+        if stg is None:
+            if self._bufs is None:
+                chunk = np.ascontiguousarray(counts, np.int32)
+                self._lay_out_first_fill(chunk.ctypes.data, 1, T, None, 0, st)
+            else:
+                self._ensure_capacity(new_counts)
         if fresh:
             _ARENA_HINT[hint_key] = self._arena.numel()
         if stg is None:
@@ -521,13 +544,16 @@ class TurboQuantAdaptiveKVCacheState:
                 C.byref(self._packed), ws.data_ptr(), ws_bytes, st))
         self._counts = new_counts
         self._exact_room = None
-        if stg is not None:
+        if _levels is not None and self.seq_len == 0:
+            self._level_store, lm = _levels, None
+        elif stg is not None:
             lm = self._arena[self._arena.numel() - lm_bytes:][:B * H * T].view(B, H, T)
             lm.copy_(bits)
         else:
             lm = bits.to(torch.uint8)
         if _pos_offset is None:
-            self._extend_levels(lm, owned=True)
+            if lm is not None:
+                self._extend_levels(lm, owned=True)
             self.seq_len += T
         else:
             self._level_store[:, :, pos_offset:pos_offset + T] = lm
@@ -627,8 +653,19 @@ class TurboQuantAdaptiveKVCacheState:
         if self._level_store is None:
             return None
         if self._masked is None:
-            idx = (self._level_map == 0).nonzero(as_tuple=True)
-            self._masked = (idx if idx[0].numel() else None,)
+            # (their number is known from the counts of what is stored: nothing waits for the device)
+            B, H, T = self.batch_size, self.num_heads, self.seq_len
+            n = self._nseg * T - int(self._counts.sum())
+            if n == 0:
+                self._masked = (None,)
+            else:
+                out = torch.empty(3, n, dtype=torch.long, device=self.device)
+                ws_bytes = lib.odmkv_evicted_workspace_bytes(B, H, T)
+                ws = _lib.workspace(self.device, ws_bytes, "evicted")
+                levels = self._level_store
+                _lib.check(lib.odmkv_evicted_indices(levels.data_ptr(), B, H, T, levels.stride(1), n, out.data_ptr(),
+                                                     ws.data_ptr(), ws_bytes, _lib.stream_ptr(self.device)))
+                self._masked = (out.unbind(0),)
         return self._masked[0]
 
     def visible_mask(self) -> torch.Tensor:
