@@ -74,6 +74,17 @@ int odmkv_score_model_dtype(const void* K, const void* V, int dtype, int Hkv, in
                             int round_dtype, float* scores, void* workspace, size_t workspace_bytes,
                             void* stream);
 
+/* The mean query (kvquant/scorer.py:204-227, kvquant/attention_utils.py:57-115), around the layer's own projection:
+ * odmkv_token_mean: out [batch, cols] = mean over the tokens of x [batch, rows, cols] (`dtype`, element strides; rows of whole
+ * 16-byte pieces), summed in fp32 and rounded to dtype; workspace odmkv_token_mean_workspace_bytes.
+ * odmkv_average_rope: out fp32 [heads, 128] = c * mu + s * rotate_half(mu) with c, s the means over the positions of cosine,
+ * sine [positions, 128]; mu [heads, 128], all contiguous and of `dtype`; every product, sum and mean is rounded to dtype. */
+size_t odmkv_token_mean_workspace_bytes(int batch, int rows, int cols);
+int odmkv_token_mean(const void* x, int dtype, int batch, int rows, int cols, int64_t stride_b, int64_t stride_t,
+                     void* out, void* workspace, size_t workspace_bytes, void* stream);
+int odmkv_average_rope(const void* mu, const void* cosine, const void* sine, int dtype, int heads, int positions,
+                       float* out, void* stream);
+
 /* Expected-attention score.  Replaces ExpectedAttentionScorer.score_prefill after the query
  * statistics are known (kvquant/scorer.py:204-257):
  *

@@ -79,6 +79,9 @@ def _load() -> C.CDLL:
         "odmkv_score": (C.c_int, [vp, vp, i32, i32, i32, i64, i64, vp, i32, vp, i32, f32, vp, vp, sz, vp]),
         "odmkv_score_model_dtype": (C.c_int, [vp, vp, i32, i32, i32, i64, i64, vp, i32, vp, i32, f32, i32, vp, vp, sz, vp]),
         "odmkv_score_expected": (C.c_int, [vp, vp, i32, i32, i32, i64, i64, vp, vp, i32, i32, f32, i32, vp, vp, sz, vp]),
+        "odmkv_token_mean_workspace_bytes": (sz, [i32, i32, i32]),
+        "odmkv_token_mean": (C.c_int, [vp, i32, i32, i32, i32, i64, i64, vp, vp, sz, vp]),
+        "odmkv_average_rope": (C.c_int, [vp, vp, vp, i32, i32, i32, vp, vp]),
         "odmkv_window_attention_workspace_bytes": (sz, [i32, i32, i32, i32]),
         "odmkv_window_attention": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, i32, i32, i32, i32, f32, vp, vp, sz, vp]),
         "odmkv_allocate_workspace_bytes": (sz, [i32, i32]),
@@ -128,7 +131,7 @@ def _load() -> C.CDLL:
 
 
 lib = _load()
-EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "odmkv_score", "odmkv_score_model_dtype", "odmkv_score_expected",
+EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "odmkv_score", "odmkv_score_model_dtype", "odmkv_score_expected", "odmkv_token_mean_workspace_bytes", "odmkv_token_mean", "odmkv_average_rope",
            "odmkv_window_attention_workspace_bytes", "odmkv_window_attention",
            "odmkv_allocate_workspace_bytes", "odmkv_allocate", "odmkv_level_counts",
            "odmkv_finish_levels_chunks", "odmkv_finish_levels", "odmkv_evicted_workspace_bytes", "odmkv_evicted_indices",

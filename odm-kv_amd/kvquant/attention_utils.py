@@ -9,6 +9,8 @@ from typing import Optional
 import torch
 from torch import nn
 
+from . import _lib
+
 
 def _repeat_kv(hidden_states: torch.Tensor, n_rep: int) -> torch.Tensor:
     """[b, Hkv, t, d] -> [b, Hkv * n_rep, t, d]; query head q reads kv-head q // n_rep."""
@@ -50,6 +52,24 @@ def _get_query_states(module: nn.Module, hidden_states: torch.Tensor) -> torch.T
     return q
 
 
+def _token_mean(hidden_states: torch.Tensor) -> torch.Tensor:
+    """Mean over the tokens, summed in fp32, of the tensor's own dtype: [b, t, hidden] -> [b, 1, hidden]."""
+    b, t, hidden = hidden_states.shape
+    n = 4 if hidden_states.dtype == torch.float32 else 8
+    if (hidden_states.is_cuda and hidden_states.dtype in _lib._DT and t > 0 and hidden_states.stride(2) == 1 and hidden % n == 0
+            and hidden_states.stride(0) % n == 0 and hidden_states.stride(1) % n == 0 and hidden_states.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and hidden_states.requires_grad)):
+        dev = hidden_states.device
+        out = torch.empty(b, 1, hidden, dtype=hidden_states.dtype, device=dev)
+        ws_bytes = _lib.lib.odmkv_token_mean_workspace_bytes(b, t, hidden)
+        ws = _lib.workspace(dev, ws_bytes, "mean")
+        _lib.check(_lib.lib.odmkv_token_mean(hidden_states.data_ptr(), _lib.dtype_code(hidden_states), b, t, hidden,
+                                             hidden_states.stride(0), hidden_states.stride(1), out.data_ptr(), ws.data_ptr(),
+                                             ws_bytes, _lib.stream_ptr(dev)))
+        return out
+    return hidden_states.float().mean(dim=1, keepdim=True).to(hidden_states.dtype)
+
+
 def _mean_query_states(module: nn.Module, hidden_states: torch.Tensor) -> torch.Tensor:
     """mean over positions of ``_get_query_states`` -> [b, Hq, d].
 
@@ -59,7 +79,7 @@ def _mean_query_states(module: nn.Module, hidden_states: torch.Tensor) -> torch.
         return _get_query_states(module, hidden_states).mean(dim=2)
     b, t, hidden = hidden_states.shape
     n_heads, head_dim = _head_geometry(module, hidden)
-    mean_h = hidden_states.float().mean(dim=1, keepdim=True).to(hidden_states.dtype)
+    mean_h = _token_mean(hidden_states)
     if hasattr(module, "qkv_proj"):
         q = module.qkv_proj(mean_h)[..., : n_heads * head_dim]
     elif hasattr(module, "q_proj"):
@@ -101,6 +121,14 @@ def _apply_avg_rope(module: nn.Module, mu: torch.Tensor, cov: Optional[torch.Ten
         return mu, cov
     pos = torch.arange(q_len, q_len + n_future_positions, device=mu.device).unsqueeze(0)
     cos, sin = _aligned_rotary_outputs(rotary_emb, mu, pos)
+    if (cov is None and mu.is_cuda and mu.dtype in _lib._DT and mu.shape[-1] == _lib.HEAD_DIM and mu.is_contiguous()
+            and cos.shape == sin.shape == (1, n_future_positions, _lib.HEAD_DIM) and cos.is_contiguous() and sin.is_contiguous()
+            and not (torch.is_grad_enabled() and mu.requires_grad)):
+        out = torch.empty(mu.shape, dtype=torch.float32, device=mu.device)       # (rounded to mu's type, held wide)
+        _lib.check(_lib.lib.odmkv_average_rope(mu.data_ptr(), cos.data_ptr(), sin.data_ptr(), _lib.dtype_code(mu),
+                                               mu.numel() // _lib.HEAD_DIM, n_future_positions, out.data_ptr(),
+                                               _lib.stream_ptr(mu.device)))
+        return out, None
     c_bar, s_bar = cos[0].mean(dim=0), sin[0].mean(dim=0)
 
     def r_avg(x):
