@@ -336,6 +336,15 @@ int odmkv_dequant_from(const odmkv_packed_t* store, void* K, void* V, int dtype,
  * untouched when a segment is full; the caller sizes segments. */
 int odmkv_append_exact(const odmkv_packed_t* store, const void* k, const void* v, int64_t stride_b,
                        int64_t stride_h, int pos, void* stream);
+/* T tokens per (b, h) at positions pos, pos + 1, ...: k, v [B, Hkv, T, 128] with token strides of their own (a question of
+ * several tokens, append_all_exact with T > 1). */
+int odmkv_append_exact_rows(const odmkv_packed_t* store, const void* k, const void* v, int T, int64_t stride_b,
+                            int64_t stride_h, int64_t stride_tk, int64_t stride_tv, int pos, void* stream);
+/* Forget the newest n tokens of every exact segment (a flush stores them again at other levels). */
+int odmkv_drop_exact_tail(const odmkv_packed_t* store, int n, void* stream);
+/* Forget every token at a position >= length (truncate, kvquant/tq_adaptive_backend.py:499-541).  counts: int32
+ * [5][B*Hkv], device or page-locked host memory, receives the segments' new counts. */
+int odmkv_truncate(const odmkv_packed_t* store, int length, int32_t* counts, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Decode-time flush of the exact token buffer on the device.  Stands where the reference scores the
@@ -419,6 +428,9 @@ typedef struct odmkv_worklist {
                                       * 128 registers a wavefront and half a compute unit's LDS, so that two of them share a
                                       * compute unit and one streams while the other starts or finishes: for lists with more
                                       * items than compute units (a batch of sequences, many levels).  0: one per compute unit */
+    int32_t covers_exact;            /* 1: the exact items cover every tile the exact segments have room in (as
+                                      * odmkv_worklist_cut makes them): a decode step's new token is then stored by the workgroup
+                                      * that attends over its tile.  0: by a launch of its own */
 } odmkv_worklist_t;
 
 /* Cut the work list of a store on the host: every (segment, level) run of tiles into items of about equal cost (what the
@@ -466,7 +478,7 @@ int odmkv_decode_attn(const void* q, int q_dtype, int B, int Hq, float scaling,
  * attends over the re-materialised cache (kvquant/adaptive_backend_press.py:221-262; append_all_exact,
  * kvquant/tq_adaptive_backend.py:412-440).  What does not change from step to step sits in a block the caller fills
  * once per store and work list (the pointers in it are those of odmkv_decode_attn and must stay valid); q, out and lse
- * as in odmkv_decode_attn.  Three launches on `stream`. */
+ * as in odmkv_decode_attn.  Two launches on `stream` (three where the work list does not cover the exact segments). */
 typedef struct odmkv_step {
     const odmkv_packed_t* store;
     const odmkv_worklist_t* work;
@@ -484,7 +496,23 @@ typedef struct odmkv_step {
 int odmkv_decode_step(const odmkv_step_t* step, const void* q, const void* k_new, const void* v_new,
                       int64_t stride_b, int64_t stride_h, int pos, void* out, float* lse, void* stream);
 
-/* The same call without a workspace, for callers that cannot allocate device memory and have none
+/* A block of L query tokens per sequence that all see the whole store (the question after a prefill): q [B, Hq, L, 128] with
+ * element strides, out fp32 [B, Hq, L, 128] and lse fp32 [B, Hq, L] contiguous.  The L tokens of a kv-head's G query heads
+ * are handed over as further heads of it, 8 / G tokens per pass over the store, the passes in one launch.  step: as for
+ * odmkv_decode_step (out_dtype is not looked at); its workspace: odmkv_decode_block_workspace_bytes. */
+size_t odmkv_decode_block_workspace_bytes(int B, int Hq, int Hkv, int L, int n_items);
+int odmkv_decode_block(const odmkv_step_t* step, const void* q, int64_t stride_b, int64_t stride_h, int64_t stride_l,
+                       int L, float* out, float* lse, void* stream);
+/* The rest of such a block's attention: every token over the block's own tokens k, v [B, Hkv, L, 128] (kv_dtype) up to its
+ * position, or where mask (uint8 [B, L, L] with strides mask_sb, mask_sl; NULL: causal) is not 0, merged by log-sum-exp
+ * with the store's part (out_store, lse_store as odmkv_decode_block left them); out [B, L, Hq, 128] of q_dtype.
+ * (kvquant/attention_patch.py:38-48 runs such a call over the re-materialised cache.) */
+int odmkv_block_merge(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                      int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl, int kv_dtype,
+                      const uint8_t* mask, int64_t mask_sb, int64_t mask_sl, int B, int Hq, int Hkv, int L, float scaling,
+                      const float* out_store, const float* lse_store, void* out, void* stream);
+
+/* odmkv_decode_attn without a workspace, for callers that cannot allocate device memory and have none
  * to hand over (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  The per-item partial results live in
  * a fixed array of ODMKV_STATIC_SCRATCH_BYTES inside the library's device image (held by every GPU

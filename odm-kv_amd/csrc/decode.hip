@@ -40,6 +40,7 @@
 // All softmax state is kept in base-2 logarithms.
 #include "decode.h"
 #include <stdlib.h>
+#include <algorithm>
 
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -873,7 +874,25 @@ __device__ static inline void run_exact_level(const DecodeArgs& a, int bh, int b
             qraw[kb] = make_uint4(w[0], w[1], w[2], w[3]);
         }
     }
-    const int count = a.s.seg_count[4][bh] - (tile0 - seg_first) * TILE;     // exact segments grow between work-list rebuilds
+    int stored = a.s.seg_count[4][bh];                     // exact segments grow between work-list rebuilds
+    if (a.k_new) {
+        // A decode step's new token goes behind the stored ones: the workgroup whose tiles hold its place writes it (its
+        // later loads of the row come after the wait and the barrier); the segment's other workgroups hold none of it.  A launch of its own cost 3.1 us of GPU time and 3 us of the host's.
+        const int at = (stored >> 6) - (tile0 - seg_first), slot = stored & (TILE - 1);
+        if (at >= 0 && at < ntiles) {                      // workgroup-uniform
+            const size_t tile = (size_t)(tile0 + at);
+            if (tid < HD) {
+                const size_t src = (size_t)(bh / a.s.Hkv) * a.new_sb + (size_t)(bh % a.s.Hkv) * a.new_sh + tid;
+                a.s.kexact[tile * TILE * HD + exact_k_index(slot, tid)] = a.k_new[src];
+                a.s.vexact[tile * TILE * HD + exact_v_index(slot, tid)] = a.v_new[src];
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (tid == 0) a.s.pos[4][tile * TILE + slot] = a.new_pos;
+        }
+        stored += 1;                                       // (the segment's count itself is moved by the merge, for everybody)
+    }
+    const int count = stored - (tile0 - seg_first) * TILE;
     for (int u = wave; u < 2 * ntiles; u += NW) {
         const int nvalid = min(count - u * UNIT, UNIT);
         if (nvalid <= 0) break;
@@ -960,9 +979,10 @@ __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(Deco
     // order of their requests: asked for first, the table would hold the item back; it does not depend on the item)
     const int bh = d0.x;
     int li = d0.y, tile0 = d0.z, ntiles = d0.w, ntok = d1.x;
-    const int bq_first = (bh / a.s.Hkv) * a.Hq + (bh % a.s.Hkv) * a.G;      // first query head of the group
+    const int pass = blockIdx.y;                               // (0 but for blocks of query tokens)
+    const int bq_first = (pass * a.B + bh / a.s.Hkv) * a.Hq + (bh % a.s.Hkv) * a.G;      // first query head of the group
 
-    float* dst = a.partial + (size_t)item * GP * PSTRIDE;      // where this item's result goes
+    float* dst = a.partial + ((size_t)pass * a.n_items + item) * GP * PSTRIDE;      // where this item's result goes
 
     WaveState st;
     st.mA = -INFINITY; st.mB = -INFINITY; st.lA = 0.0f; st.lB = 0.0f;
@@ -1077,6 +1097,14 @@ __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(Deco
 #define MERGE_THREADS 512
 #define MERGE_SLICES (MERGE_THREADS / HD)
 #define MERGE_CHUNK 64            // items merged per round: one per lane of a wavefront
+#define NO_ROW (~(size_t)0)
+
+// where query head bq (head g of its group) of this launch's pass stands in out and lse
+__device__ static inline size_t out_row(const DecodeArgs& a, int bq, int bh, int g) {
+    if (a.block_len == 0) return bq;
+    const int l = (a.pass0 + (int)blockIdx.y) * a.block_per + g / a.block_g;
+    return l < a.block_len ? ((size_t)bh * a.block_g + g % a.block_g) * a.block_len + l : NO_ROW;
+}
 
 // MERGE_SPLIT: workgroups per query head (4 when there are few heads, so that the launch still covers the device;
 // 1 for large batches, where every further workgroup only repeats the reading)
@@ -1095,7 +1123,11 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
     const int slice = __builtin_amdgcn_readfirstlane(tid >> 7);
     const int b = bq / a.Hq, hq = bq % a.Hq;
     const int bh = b * a.s.Hkv + hq / a.G, g = hq % a.G;
+    const size_t row = out_row(a, bq, bh, g);              // of out and lse
+    if (row == NO_ROW) return;                             // (workgroup-uniform: padding of a block's last pass)
+    const float* partial = a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
+    if (a.k_new && g == 0 && quarter == 0 && tid == 0) a.s.seg_count[4][bh] += 1;      // the step's token is stored
     // this thread's share of the value rotation: requested first, it does not depend on the items
     const int jj = tid % QD, rs = tid / QD;
     float pv[IN];
@@ -1111,7 +1143,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
         float m_i = -INFINITY, l_i = 0.0f;
         int level = 0;
         if (lane < nc) {
-            const float* p = a.partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE;
+            const float* p = partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE;
             m_i = p[HD]; l_i = p[HD + 1];
             level = a.items[8 * (i0 + c0 + lane) + 1];
         }
@@ -1119,7 +1151,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
 #pragma unroll
         for (int k = 0; k < MERGE_CHUNK / MERGE_SLICES; ++k) {
             const int it = slice + k * MERGE_SLICES;
-            vals[k] = it < nc ? a.partial[((size_t)(i0 + c0 + it) * GP + g) * PSTRIDE + j] : 0.0f;
+            vals[k] = it < nc ? partial[((size_t)(i0 + c0 + it) * GP + g) * PSTRIDE + j] : 0.0f;
         }
         const float Mc = fmaxf(M, wave_max(m_i));
         const float f_old = M > -INFINITY ? __builtin_amdgcn_exp2f(M - Mc) : 0.0f;
@@ -1161,11 +1193,11 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
 #pragma unroll
         for (int sl = 0; sl < MERGE_SLICES; ++sl) tot += part[1][sl][dim];
         const float o32 = L > 0.0f ? tot / L : 0.0f;
-        const size_t oi = (size_t)bq * HD + dim;
+        const size_t oi = row * HD + dim;
         if (a.out_dt == ODMKV_F32) reinterpret_cast<float*>(a.out)[oi] = o32;
         else if (a.out_dt == ODMKV_F16) reinterpret_cast<uint16_t*>(a.out)[oi] = Elem<ODMKV_F16>::from_f32(o32);
         else reinterpret_cast<uint16_t*>(a.out)[oi] = Elem<ODMKV_BF16>::from_f32(o32);
-        if (a.lse && tid == 0 && quarter == 0) a.lse[bq] = L > 0.0f ? (M + __log2f(L) - P_SHIFT) * LN2 : -INFINITY;
+        if (a.lse && tid == 0 && quarter == 0) a.lse[row] = L > 0.0f ? (M + __log2f(L) - P_SHIFT) * LN2 : -INFINITY;
     }
 }
 
@@ -1186,7 +1218,9 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
     const int tid = threadIdx.x, lane = tid & 63, j = tid & (HD - 1);
     const int slice = __builtin_amdgcn_readfirstlane(tid >> 7);
     const int b = bh / a.s.Hkv, hq0 = (bh % a.s.Hkv) * a.G;
+    const float* partial = a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
+    if (a.k_new && tid == 0) a.s.seg_count[4][bh] += 1;   // the step's token is stored
     float pv[IN];
 #pragma unroll
     for (int ii = 0; ii < IN; ++ii) pv[ii] = a.pi_v[(size_t)(slice * IN + ii) * HD + j];
@@ -1200,7 +1234,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
                 float m_i = -INFINITY, l_i = 0.0f;
                 int level = 0;
                 if (lane < nc) {
-                    const float* p = a.partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE;
+                    const float* p = partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE;
                     m_i = p[HD]; l_i = p[HD + 1];
                     level = a.items[8 * (i0 + c0 + lane) + 1];
                 }
@@ -1214,7 +1248,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
                     float vals[4];
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
-                        vals[k] = it0 + k < nc ? a.partial[((size_t)(i0 + c0 + it0 + k) * GP + g) * PSTRIDE + j] : 0.0f;
+                        vals[k] = it0 + k < nc ? partial[((size_t)(i0 + c0 + it0 + k) * GP + g) * PSTRIDE + j] : 0.0f;
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         if (it0 + k < nc) {
@@ -1257,12 +1291,13 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
         for (int r = 0; r < RS; ++r) tot += part2[g][r][j];
         const float L = headL[g];
         const float o32 = L > 0.0f ? tot / L : 0.0f;
-        const size_t bq = (size_t)b * a.Hq + hq0 + g;
-        const size_t oi = bq * HD + j;
+        const size_t row = out_row(a, b * a.Hq + hq0 + g, bh, g);
+        if (row == NO_ROW) continue;
+        const size_t oi = row * HD + j;
         if (a.out_dt == ODMKV_F32) reinterpret_cast<float*>(a.out)[oi] = o32;
         else if (a.out_dt == ODMKV_F16) reinterpret_cast<uint16_t*>(a.out)[oi] = Elem<ODMKV_F16>::from_f32(o32);
         else reinterpret_cast<uint16_t*>(a.out)[oi] = Elem<ODMKV_BF16>::from_f32(o32);
-        if (a.lse && j == 0) a.lse[bq] = L > 0.0f ? (headM[g] + __log2f(L) - P_SHIFT) * LN2 : -INFINITY;
+        if (a.lse && j == 0) a.lse[row] = L > 0.0f ? (headM[g] + __log2f(L) - P_SHIFT) * LN2 : -INFINITY;
     }
 }
 
@@ -1308,8 +1343,8 @@ extern "C" size_t odmkv_decode_workspace_bytes(int B, int Hq, int n_items) {
 }
 
 template <int GP, bool ORDERED, int NW, bool G4 = false, bool CHAIN = false, bool PAIR = false>
-static int launch_main(const DecodeArgs& a, int grid, hipEvent_t e0, hipEvent_t e1, hipStream_t st) {
-    hipExtLaunchKernelGGL((decode_main_kernel<GP, ORDERED, NW, G4, CHAIN, PAIR>), dim3(grid), dim3(NW * 64), 0, st, e0, e1, 0, a);
+static int launch_main(const DecodeArgs& a, dim3 grid, hipEvent_t e0, hipEvent_t e1, hipStream_t st) {
+    hipExtLaunchKernelGGL((decode_main_kernel<GP, ORDERED, NW, G4, CHAIN, PAIR>), grid, dim3(NW * 64), 0, st, e0, e1, 0, a);
     ODMKV_CHECK_LAUNCH("decode_main_kernel");
     return 0;
 }
@@ -1319,7 +1354,8 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
                         const uint16_t* pi_k_ops, const float* pi_v, const float* codebooks,
                         const float* codebooks_host, const float* inv_scales,
                         void* out, int out_dtype, float* lse, void* workspace, size_t workspace_bytes,
-                        void* stream, int stage_mask, void* ev_start, void* ev_stop) {
+                        void* stream, int stage_mask, void* ev_start, void* ev_stop, const NewToken* token,
+                        const int* block) {
     ODMKV_CHECK_ARG(q_dtype == ODMKV_F16 || q_dtype == ODMKV_BF16 || q_dtype == ODMKV_F32, "decode_attn: bad query dtype %d", q_dtype);
     ODMKV_CHECK_ARG(out_dtype == ODMKV_F16 || out_dtype == ODMKV_BF16 || out_dtype == ODMKV_F32, "decode_attn: bad output dtype %d", out_dtype);
     ODMKV_CHECK_ARG(codebooks_host != nullptr, "decode_attn: null host copy of the centroid tables");
@@ -1343,7 +1379,8 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
     ODMKV_CHECK_ARG(store->exact_dtype == ODMKV_F16 || store->exact_dtype == ODMKV_BF16, "decode_attn: exact dtype must be fp16 or bf16");
     const int G = Hq / store->Hkv;
     ODMKV_CHECK_ARG(G <= ODMKV_MAX_GROUP, "decode_attn: GQA group %d exceeds %d", G, ODMKV_MAX_GROUP);
-    if (workspace_bytes < odmkv_decode_workspace_bytes(B, Hq, n_items)) {
+    const int passes = block ? block[0] : 1;
+    if (workspace_bytes < passes * odmkv_decode_workspace_bytes(B, Hq, n_items)) {
         odmkv_set_error("decode_attn: workspace of %zu bytes, %zu needed", workspace_bytes, odmkv_decode_workspace_bytes(B, Hq, n_items));
         return ODMKV_ENOSPACE;
     }
@@ -1357,6 +1394,9 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
     for (int k = 0; k < 28; ++k) a.cbs[k] = codebooks_host[k];
     a.partial = (float*)workspace;
     a.out = out; a.lse = lse;
+    a.k_new = token ? (const uint16_t*)token->k : nullptr; a.v_new = token ? (const uint16_t*)token->v : nullptr;
+    a.new_sb = token ? token->stride_b : 0; a.new_sh = token ? token->stride_h : 0; a.new_pos = token ? token->pos : 0;
+    a.block_len = block ? block[1] : 0; a.block_per = block ? block[2] : 0; a.block_g = block ? block[3] : 0; a.pass0 = block ? block[4] : 0;
     const int GP = group_pad(G);
     a.gp = GP;
     if (n_items > 0 && (stage_mask & 2)) {
@@ -1373,11 +1413,15 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
         static const int g4_forced = [] { const char* e = getenv("ODMKV_DECODE_G4"); return e ? atoi(e) : -1; }();
         const bool g4 = GP == 4 && nw == 16 && g4_forced != 0;
         const bool chain = work->n_workgroups > 0 && work->n_workgroups != n_items;      // workgroups that take several items
-        const int grid = chain ? work->n_workgroups : n_items;
+        const dim3 grid(chain ? work->n_workgroups : n_items, passes);
         // two eight-wavefront workgroups per compute unit (always with a dispatch order: the list has more items than
         // compute units); groups of up to four heads in the shared-lane form
         const bool pair = work->two_per_cu != 0 && (GP == 8 || g4_forced != 0);
-        if (pair && GP == 4) rc = chain ? launch_main<4, true, 8, true, true, true>(a, grid, e0, e1, st)
+        // a block of query tokens: several passes' workgroups in one launch run in rounds whatever the list, so they share
+        // compute units too (an order is not needed: the passes even the rounds out)
+        if (passes > 1 && !pair && !a.order) rc = GP == 4 ? launch_main<4, false, 8, true, false, true>(a, grid, e0, e1, st)
+                                                          : launch_main<8, false, 8, false, false, true>(a, grid, e0, e1, st);
+        else if (pair && GP == 4) rc = chain ? launch_main<4, true, 8, true, true, true>(a, grid, e0, e1, st)
                                                           : launch_main<4, true, 8, true, false, true>(a, grid, e0, e1, st);
         else if (pair) rc = chain ? launch_main<8, true, 8, false, true, true>(a, grid, e0, e1, st)
                                   : launch_main<8, true, 8, false, false, true>(a, grid, e0, e1, st);
@@ -1394,22 +1438,22 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
         if (rc) return rc;
     }
     if (stage_mask & 4) {
-        const int heads = B * Hq;
+        const int heads = B * Hq * passes;
         // from 512 query heads on, a workgroup per (sequence, kv-head) merges all heads of the group (64 x 2048 tokens, 2048
         // heads: the merge 10.8 -> 4.8 us; 512 heads: 3.5 -> 3.2 us); ODMKV_MERGE_GROUP_FROM moves the limit, for measurements
         static const int group_from = [] { const char* e = getenv("ODMKV_MERGE_GROUP_FROM"); return e ? atoi(e) : 512; }();
         if (heads >= group_from) {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_group_kernel<4>), dim3(B * store->Hkv), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_group_kernel<8>), dim3(B * store->Hkv), dim3(MERGE_THREADS), 0, st, a);
+            if (GP == 4) hipLaunchKernelGGL((decode_merge_group_kernel<4>), dim3(B * store->Hkv, passes), dim3(MERGE_THREADS), 0, st, a);
+            else hipLaunchKernelGGL((decode_merge_group_kernel<8>), dim3(B * store->Hkv, passes), dim3(MERGE_THREADS), 0, st, a);
         } else if (heads >= 256) {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 1>), dim3(heads), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_kernel<8, 1>), dim3(heads), dim3(MERGE_THREADS), 0, st, a);
+            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 1>), dim3(B * Hq, passes), dim3(MERGE_THREADS), 0, st, a);
+            else hipLaunchKernelGGL((decode_merge_kernel<8, 1>), dim3(B * Hq, passes), dim3(MERGE_THREADS), 0, st, a);
         } else if (heads >= 128) {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 2>), dim3(heads * 2), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_kernel<8, 2>), dim3(heads * 2), dim3(MERGE_THREADS), 0, st, a);
+            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 2>), dim3(B * Hq * 2, passes), dim3(MERGE_THREADS), 0, st, a);
+            else hipLaunchKernelGGL((decode_merge_kernel<8, 2>), dim3(B * Hq * 2, passes), dim3(MERGE_THREADS), 0, st, a);
         } else {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 4>), dim3(heads * 4), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_kernel<8, 4>), dim3(heads * 4), dim3(MERGE_THREADS), 0, st, a);
+            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 4>), dim3(B * Hq * 4, passes), dim3(MERGE_THREADS), 0, st, a);
+            else hipLaunchKernelGGL((decode_merge_kernel<8, 4>), dim3(B * Hq * 4, passes), dim3(MERGE_THREADS), 0, st, a);
         }
         ODMKV_CHECK_LAUNCH("decode_merge_kernel");
     }
@@ -1431,13 +1475,209 @@ extern "C" int odmkv_decode_attn(const void* q, int q_dtype, int B, int Hq, floa
 extern "C" int odmkv_decode_step(const odmkv_step_t* step, const void* q, const void* k_new, const void* v_new,
                                  int64_t stride_b, int64_t stride_h, int pos, void* out, float* lse, void* stream) {
     ODMKV_CHECK_ARG(step != nullptr, "decode_step: null step block");
+    NewToken token = {k_new, v_new, stride_b, stride_h, pos};
+    bool fused = false;
     if (k_new || v_new) {
-        ODMKV_CHECK_ARG(step->store != nullptr, "decode_step: null store");
-        if (int rc = odmkv_append_exact(step->store, k_new, v_new, stride_b, stride_h, pos, stream)) return rc;
+        ODMKV_CHECK_ARG(step->store != nullptr && step->work != nullptr, "decode_step: null store or work list");
+        fused = step->work->covers_exact && step->work->n_items > 0;
+        if (fused) {
+            ODMKV_CHECK_ARG(k_new && v_new && stride_b >= 0 && stride_h >= 0, "decode_step: null token or negative strides");
+            ODMKV_CHECK_ARG(step->store->kexact && step->store->vexact && step->store->seg_count[4] && step->store->pos[4],
+                            "decode_step: store has no exact segments");
+        } else if (int rc = odmkv_append_exact(step->store, k_new, v_new, stride_b, stride_h, pos, stream)) return rc;
     }
     return odmkv_decode_launch(q, step->q_dtype, step->B, step->Hq, step->scaling, step->store, step->work, step->pi_k_ops,
                                step->pi_v, step->codebooks, step->codebooks_host, step->inv_scales, out, step->out_dtype, lse,
-                               step->workspace, step->workspace_bytes, stream, 7, nullptr, nullptr);
+                               step->workspace, step->workspace_bytes, stream, 7, nullptr, nullptr, fused ? &token : nullptr);
+}
+
+// ------------------------------------------------------------------------------------------------
+// Blocks of query tokens: L tokens of a kv-head's G query heads as further heads of that kv-head, 8 / G tokens per pass
+// over the store, all passes in one launch
+// ------------------------------------------------------------------------------------------------
+struct BlockQueryArgs {
+    const void* q;
+    long long sB, sH, sL;               // elements
+    int B, Hkv, G, per, L, passes, pass0;
+    void* out;                          // [passes, B, Hkv, per, G, 128], zeros behind the block's last token
+};
+
+template <int BYTES>
+__global__ __launch_bounds__(256) void block_queries_kernel(BlockQueryArgs a) {
+    constexpr int PIECES = HD * BYTES / 16;                          // 16-byte pieces of a row
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    int row = i / PIECES;
+    const int piece = i % PIECES;
+    if (row >= a.passes * a.B * a.Hkv * a.per * a.G) return;
+    const int g = row % a.G, lp = row / a.G % a.per, h = row / (a.G * a.per) % a.Hkv, b = row / (a.G * a.per * a.Hkv) % a.B;
+    const int l = (a.pass0 + row / (a.G * a.per * a.Hkv * a.B)) * a.per + lp;
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (l < a.L)
+        v = *reinterpret_cast<const uint4*>((const char*)a.q + (b * a.sB + (long long)(h * a.G + g) * a.sH + l * a.sL) * BYTES + piece * 16);
+    reinterpret_cast<uint4*>(a.out)[(size_t)row * PIECES + piece] = v;
+}
+
+#define BLOCK_WORKSPACE (64u << 20)      // a longer block goes in several launches
+static int block_passes(int B, int G, int L, int n_items, int Hkv, int* per) {
+    *per = std::max(1, ODMKV_MAX_GROUP / G);
+    const int passes = (L + *per - 1) / *per;
+    const size_t one = odmkv_decode_workspace_bytes(B, Hkv * G * *per, n_items) + (size_t)B * Hkv * G * *per * HD * 4;
+    return (int)std::max<size_t>(1, std::min<size_t>((size_t)passes, BLOCK_WORKSPACE / std::max<size_t>(one, 1)));
+}
+
+extern "C" size_t odmkv_decode_block_workspace_bytes(int B, int Hq, int Hkv, int L, int n_items) {
+    if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || Hq / Hkv > ODMKV_MAX_GROUP || L <= 0 || n_items < 0) return 0;
+    int per;
+    const int n = block_passes(B, Hq / Hkv, L, n_items, Hkv, &per);
+    return n * (odmkv_decode_workspace_bytes(B, Hq * per, n_items) + align_up((size_t)B * Hq * per * HD * 4, 256));
+}
+
+extern "C" int odmkv_decode_block(const odmkv_step_t* step, const void* q, int64_t stride_b, int64_t stride_h, int64_t stride_l,
+                                  int L, float* out, float* lse, void* stream) {
+    ODMKV_CHECK_ARG(step && q && out && lse && step->store && step->work && step->workspace, "decode_block: null pointer");
+    const int B = step->B, Hq = step->Hq, Hkv = step->store->Hkv;
+    ODMKV_CHECK_ARG(B > 0 && Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && Hq / Hkv <= ODMKV_MAX_GROUP && L > 0,
+                    "decode_block: bad shape B=%d Hq=%d Hkv=%d L=%d", B, Hq, Hkv, L);
+    ODMKV_CHECK_ARG(step->q_dtype >= ODMKV_F16 && step->q_dtype <= ODMKV_F32, "decode_block: bad query dtype %d", step->q_dtype);
+    const int bytes = step->q_dtype == ODMKV_F32 ? 4 : 2, n = 16 / bytes;
+    ODMKV_CHECK_ARG(((uintptr_t)q & 15) == 0 && stride_b % n == 0 && stride_h % n == 0 && stride_l % n == 0,
+                    "decode_block: query rows must start on multiples of 16 bytes");
+    ODMKV_CHECK_ARG(step->workspace_bytes >= odmkv_decode_block_workspace_bytes(B, Hq, Hkv, L, step->work->n_items), "decode_block: workspace too small");
+    int per;
+    const int G = Hq / Hkv, at_once = block_passes(B, G, L, step->work->n_items, Hkv, &per), passes = (L + per - 1) / per;
+    const size_t partial = at_once * odmkv_decode_workspace_bytes(B, Hq * per, step->work->n_items);
+    char* queries = (char*)step->workspace + partial;
+    for (int p0 = 0; p0 < passes; p0 += at_once) {
+        const int np = std::min(at_once, passes - p0);
+        const BlockQueryArgs qa = {q, (long long)stride_b, (long long)stride_h, (long long)stride_l, B, Hkv, G, per, L, np, p0, queries};
+        const long long pieces = (long long)np * B * Hq * per * (HD * bytes / 16);
+        ODMKV_CHECK_ARG(pieces < (1ll << 31), "decode_block: too many query rows");
+        if (bytes == 4) hipLaunchKernelGGL(block_queries_kernel<4>, dim3((pieces + 255) / 256), dim3(256), 0, (hipStream_t)stream, qa);
+        else hipLaunchKernelGGL(block_queries_kernel<2>, dim3((pieces + 255) / 256), dim3(256), 0, (hipStream_t)stream, qa);
+        ODMKV_CHECK_LAUNCH("block_queries_kernel");
+        const int block[5] = {np, L, per, G, p0};
+        if (int rc = odmkv_decode_launch(queries, step->q_dtype, B, Hq * per, step->scaling, step->store, step->work, step->pi_k_ops, step->pi_v,
+                                         step->codebooks, step->codebooks_host, step->inv_scales, out, ODMKV_F32, lse, step->workspace,
+                                         partial, stream, 7, nullptr, nullptr, nullptr, block))
+            return rc;
+    }
+    return 0;
+}
+
+// The block's own tokens (each sees those up to its own position, or what the mask says), merged with the store's part by
+// log-sum-exp.  A workgroup takes one token of one kv-head's group, a wavefront a query head at a time, a lane a key
+// (64 at a time with a running maximum), then two dims.  fp32 throughout.  Bound by latency: it replaces some twenty tensor
+// operations (conversions, repeats, products, masks, exponentials) of a question of a few dozen tokens, 140 us a layer.
+struct BlockMergeArgs {
+    const void* q; const void* k; const void* v;
+    long long qB, qH, qL, kB, kH, kL, vB, vH, vL;      // elements
+    const uint8_t* mask;                               // [B or 1, L, L], non-zero = visible, or null: causal
+    long long mB, mL;
+    int Hq, G, L;
+    float scaling;
+    const float* out_s; const float* lse_s;            // [B, Hq, L, 128], [B, Hq, L]
+    void* out;                                         // [B, L, Hq, 128]
+};
+
+template <int DT>
+__device__ static inline void row8(const typename Elem<DT>::raw* p, float* x) {       // eight consecutive elements, 16-byte aligned
+    if constexpr (DT == ODMKV_F32) {
+        const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+    } else {
+        const uint4 v = *reinterpret_cast<const uint4*>(p);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = Elem<DT>::to_f32((uint16_t)(w[e >> 1] >> (16 * (e & 1))));
+    }
+}
+
+template <int QDT, int KDT>
+__global__ __launch_bounds__(256) void block_merge_kernel(BlockMergeArgs a) {
+    __shared__ __align__(16) float qs[4][HD];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int l = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    typedef typename Elem<QDT>::raw qraw;
+    typedef typename Elem<KDT>::raw kraw;
+    const kraw* kb = (const kraw*)a.k + b * a.kB + h * a.kH;
+    const kraw* vb = (const kraw*)a.v + b * a.vB + h * a.vH;
+    const uint8_t* mask = a.mask ? a.mask + b * a.mB + l * a.mL : nullptr;
+    const int last = mask ? a.L : l + 1;                                  // keys to look at
+    for (int g = wave; g < a.G; g += 4) {
+        const int hq = h * a.G + g;
+        const qraw* q = (const qraw*)a.q + b * a.qB + (long long)hq * a.qH + l * a.qL;
+        qs[wave][lane] = Elem<QDT>::to_f32(q[lane]);
+        qs[wave][lane + 64] = Elem<QDT>::to_f32(q[lane + 64]);
+        wave_lds_fence();
+        float m = -INFINITY, sum = 0.0f, o0 = 0.0f, o1 = 0.0f;
+        for (int j0 = 0; j0 < last; j0 += 64) {
+            const int j = j0 + lane;
+            float t = -INFINITY;
+            if (j < last && (!mask || mask[j])) {
+                const kraw* kr = kb + (long long)j * a.kL;
+                float d = 0.0f;
+#pragma unroll 4
+                for (int e = 0; e < HD; e += 8) {
+                    float x[8];
+                    row8<KDT>(kr + e, x);
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) d = __fmaf_rn(qs[wave][e + c], x[c], d);
+                }
+                t = d * a.scaling;
+            }
+            const float mn = fmaxf(m, wave_max(t));
+            if (mn == -INFINITY) continue;                                // nothing visible so far (wave-uniform)
+            const float f = m > -INFINITY ? __expf(m - mn) : 0.0f, p = t > -INFINITY ? __expf(t - mn) : 0.0f;
+            sum = sum * f + wave_sum(p);
+            o0 *= f; o1 *= f;
+            for (int j = j0; j < min(j0 + 64, last); ++j) {
+                const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(p), j - j0));
+                const kraw* vr = vb + (long long)j * a.vL;
+                o0 = __fmaf_rn(w, Elem<KDT>::to_f32(vr[lane]), o0);
+                o1 = __fmaf_rn(w, Elem<KDT>::to_f32(vr[lane + 64]), o1);
+            }
+            m = mn;
+        }
+        const size_t row = ((size_t)b * a.Hq + hq) * a.L + l;
+        const float ls = a.lse_s[row], ln = sum > 0.0f ? m + __logf(sum) : -INFINITY, mx = fmaxf(ls, ln);
+        const float ws = ls > -INFINITY ? __expf(ls - mx) : 0.0f, wn = ln > -INFINITY ? __expf(ln - mx) : 0.0f;
+        const float norm = 1.0f / (ws + wn), wo = sum > 0.0f ? wn / sum : 0.0f;
+        const float s0 = ws > 0.0f ? a.out_s[row * HD + lane] : 0.0f, s1 = ws > 0.0f ? a.out_s[row * HD + lane + 64] : 0.0f;
+        qraw* out = (qraw*)a.out + (((size_t)b * a.L + l) * a.Hq + hq) * HD;
+        out[lane] = Elem<QDT>::from_f32((s0 * ws + o0 * wo) * norm);
+        out[lane + 64] = Elem<QDT>::from_f32((s1 * ws + o1 * wo) * norm);
+        wave_lds_fence();                                                  // (the query row is free for the next head)
+    }
+}
+
+extern "C" int odmkv_block_merge(const void* q, int q_dtype, int64_t q_sb, int64_t q_sh, int64_t q_sl, const void* k, int64_t k_sb,
+                                 int64_t k_sh, int64_t k_sl, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_sl, int kv_dtype,
+                                 const uint8_t* mask, int64_t mask_sb, int64_t mask_sl, int B, int Hq, int Hkv, int L, float scaling,
+                                 const float* out_store, const float* lse_store, void* out, void* stream) {
+    ODMKV_CHECK_ARG(q && k && v && out_store && lse_store && out, "block_merge: null pointer");
+    ODMKV_CHECK_ARG(B > 0 && B <= 65535 && Hkv > 0 && Hkv <= 65535 && Hq > 0 && Hq % Hkv == 0 && L > 0, "block_merge: bad shape B=%d Hq=%d Hkv=%d L=%d", B, Hq, Hkv, L);
+    ODMKV_CHECK_ARG(q_dtype >= ODMKV_F16 && q_dtype <= ODMKV_F32 && kv_dtype >= ODMKV_F16 && kv_dtype <= ODMKV_F32, "block_merge: bad dtypes %d, %d", q_dtype, kv_dtype);
+    ODMKV_CHECK_ARG(((uintptr_t)k & 15) == 0 && k_sb % 8 == 0 && k_sh % 8 == 0 && k_sl % 8 == 0, "block_merge: key rows must start on multiples of 16 bytes");
+    const BlockMergeArgs a = {q, k, v, (long long)q_sb, (long long)q_sh, (long long)q_sl, (long long)k_sb, (long long)k_sh, (long long)k_sl,
+                              (long long)v_sb, (long long)v_sh, (long long)v_sl, mask, (long long)mask_sb, (long long)mask_sl,
+                              Hq, Hq / Hkv, L, scaling, out_store, lse_store, out};
+    const dim3 grid(L, Hkv, B);
+    hipStream_t st = (hipStream_t)stream;
+#define BLOCK_MERGE(Q, K) hipLaunchKernelGGL((block_merge_kernel<Q, K>), grid, dim3(256), 0, st, a)
+    switch (q_dtype * 3 + kv_dtype) {
+        case 0: BLOCK_MERGE(0, 0); break;
+        case 1: BLOCK_MERGE(0, 1); break;
+        case 2: BLOCK_MERGE(0, 2); break;
+        case 3: BLOCK_MERGE(1, 0); break;
+        case 4: BLOCK_MERGE(1, 1); break;
+        case 5: BLOCK_MERGE(1, 2); break;
+        case 6: BLOCK_MERGE(2, 0); break;
+        case 7: BLOCK_MERGE(2, 1); break;
+        default: BLOCK_MERGE(2, 2); break;
+    }
+#undef BLOCK_MERGE
+    ODMKV_CHECK_LAUNCH("block_merge_kernel");
+    return 0;
 }
 
 // ------------------------------------------------------------------------------------------------

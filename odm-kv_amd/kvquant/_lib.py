@@ -10,6 +10,11 @@ import os
 
 import torch
 
+try:
+    from . import _native        # the decode step's host path (csrc/torch_step.cpp)
+except ImportError as e:
+    raise ImportError("kvquant/_native.so is missing or does not fit this torch: build it first (python odm-kv_amd/build.py)") from e
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("ODMKV_LIB") or os.path.join(os.path.dirname(_HERE), "lib", "libodmkv.so")
 
@@ -41,6 +46,7 @@ class Worklist(C.Structure):
     _fields_ = [
         ("items", C.c_void_p), ("item_range", C.c_void_p), ("dispatch_order", C.c_void_p),
         ("n_items", C.c_int32), ("wavefronts", C.c_int32), ("n_workgroups", C.c_int32), ("two_per_cu", C.c_int32),
+        ("covers_exact", C.c_int32),
     ]
 
 
@@ -111,6 +117,9 @@ def _load() -> C.CDLL:
         "odmkv_dequant": (C.c_int, [C.POINTER(Packed), vp, vp, i32, i32, i64, i64, i64, vp, vp, vp, i32, vp]),
         "odmkv_dequant_from": (C.c_int, [C.POINTER(Packed), vp, vp, i32, i32, i32, i64, i64, i64, vp, vp, vp, i32, vp]),
         "odmkv_append_exact": (C.c_int, [C.POINTER(Packed), vp, vp, i64, i64, i32, vp]),
+        "odmkv_append_exact_rows": (C.c_int, [C.POINTER(Packed), vp, vp, i32, i64, i64, i64, i64, i32, vp]),
+        "odmkv_drop_exact_tail": (C.c_int, [C.POINTER(Packed), i32, vp]),
+        "odmkv_truncate": (C.c_int, [C.POINTER(Packed), i32, vp, vp]),
         "odmkv_decode_workspace_bytes": (sz, [i32, i32, i32]),
         "odmkv_decode_attn": (C.c_int, [vp, i32, i32, i32, f32, C.POINTER(Packed), C.POINTER(Worklist), vp, vp, vp,
                                         C.POINTER(C.c_float), C.POINTER(C.c_float), vp, i32, vp, vp, sz, vp]),
@@ -119,6 +128,10 @@ def _load() -> C.CDLL:
         "odmkv_decode_step": (C.c_int, [C.POINTER(Step), vp, vp, vp, i64, i64, i32, vp, vp, vp]),
         "odmkv_worklist_cut": (C.c_int, [vp, vp, i32, i32, i64, i64, i32, i32, i32, C.POINTER(WorklistChoice), vp, C.c_uint64,
                                          C.POINTER(WorklistShape)]),
+        "odmkv_decode_block_workspace_bytes": (sz, [i32, i32, i32, i32, i32]),
+        "odmkv_decode_block": (C.c_int, [C.POINTER(Step), vp, i64, i64, i64, i32, vp, vp, vp]),
+        "odmkv_block_merge": (C.c_int, [vp, i32, i64, i64, i64, vp, i64, i64, i64, vp, i64, i64, i64, i32, vp, i64, i64,
+                                        i32, i32, i32, i32, f32, vp, vp, vp, vp]),
         "odmkv_exact_tail": (C.c_int, [C.POINTER(Packed), i32, vp, vp, vp]),
         "odmkv_flush_score": (C.c_int, [vp, vp, i32, i32, i32, vp, f32, f32, i32, vp, vp, vp, vp]),
         "odmkv_flush_rank": (C.c_int, [vp, vp, i32, i32, i32, vp, vp, vp]),
@@ -131,14 +144,15 @@ def _load() -> C.CDLL:
 
 
 lib = _load()
+STEP_ENTRY = C.cast(lib.odmkv_decode_step, C.c_void_p).value      # what _native.Step calls
 EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "odmkv_score", "odmkv_score_model_dtype", "odmkv_score_expected", "odmkv_token_mean_workspace_bytes", "odmkv_token_mean", "odmkv_average_rope",
            "odmkv_window_attention_workspace_bytes", "odmkv_window_attention",
            "odmkv_allocate_workspace_bytes", "odmkv_allocate", "odmkv_level_counts",
            "odmkv_finish_levels_chunks", "odmkv_finish_levels", "odmkv_evicted_workspace_bytes", "odmkv_evicted_indices",
            "odmkv_store_init", "odmkv_store_gather", "odmkv_quant_pack_staged", "odmkv_store_layout", "odmkv_store_bind", "odmkv_pack_workspace_bytes", "odmkv_pack_count_chunks", "odmkv_store_finish_staged", "odmkv_quant_pack", "odmkv_quantize_rows",
-           "odmkv_dequantize_rows", "odmkv_lloyd_max", "odmkv_dequant", "odmkv_dequant_from", "odmkv_append_exact",
+           "odmkv_dequantize_rows", "odmkv_lloyd_max", "odmkv_dequant", "odmkv_dequant_from", "odmkv_append_exact", "odmkv_append_exact_rows", "odmkv_drop_exact_tail", "odmkv_truncate",
            "odmkv_worklist_cut", "odmkv_decode_workspace_bytes", "odmkv_rotation_operands", "odmkv_decode_attn", "odmkv_decode_attn_static",
-           "odmkv_decode_step", "odmkv_exact_tail", "odmkv_flush_score", "odmkv_flush_rank")
+           "odmkv_decode_step", "odmkv_decode_block_workspace_bytes", "odmkv_decode_block", "odmkv_block_merge", "odmkv_exact_tail", "odmkv_flush_score", "odmkv_flush_rank")
 
 
 def check(rc: int) -> None:

@@ -265,6 +265,20 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
 
     # ------------------------------------------------------------------ hook
     def _forward_hook(self, module: nn.Module, args, kwargs, output):
+        # the usual decode step: the attention call has stored the token natively, the buffer grows by one
+        layer_idx = getattr(module, "layer_idx", None)
+        state = self._states.get(layer_idx)
+        if state is not None and state._fast is not None and state.exact_decode_append and module.__dict__.get("_odmkv_state") is state:
+            cache, hidden_states = kwargs.get("past_key_values"), kwargs.get("hidden_states")
+            if cache is not None and hidden_states is not None and hidden_states.shape[1] == 1:
+                layers = getattr(cache, "layers", None)
+                start = self._buffer_start_seqs.get(layer_idx)
+                if (layers is not None and getattr(layers[layer_idx], "_tq_backend_state", None) is state
+                        and layers[layer_idx].keys.shape[2] == state.seq_len and (start is None or start <= state.seq_len)):
+                    count = self._buffer_counts.get(layer_idx, 0) + 1
+                    if count < self.buffer_size:
+                        self._buffer_counts[layer_idx] = count
+                        return output
         cache, hidden_states = self._hook_inputs(module, args, kwargs)
         if cache is None or hidden_states is None:
             return output

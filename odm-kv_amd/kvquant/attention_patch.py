@@ -20,6 +20,11 @@ import os
 import torch
 from transformers.modeling_utils import ALL_ATTENTION_FUNCTIONS
 
+from kvquant import _lib
+from kvquant._lib import stream_ptr
+
+# tokens of a block whose own part the library computes (every pair on the vector ALU); longer blocks are matrix products
+_NATIVE_BLOCK = 256
 _PATCH_ATTR = "_kvtoken_quant_attention_patched"
 # how many decode calls took the fused kernel / the wrapped attention function (diagnostics)
 call_counts = {"fused": 0, "dense": 0}
@@ -118,6 +123,19 @@ def _fused_block(state, query, key, value, attention_mask, scaling, k_len):
         if not _store_part_is_open(attention_mask, k_len - L):
             return None
     out_s, lse_s = state.decode_attention_block(query, scaling=scaling)          # [B, Hq, L, D], [B, Hq, L]
+    k, v = key[:, :, -L:, :], value[:, :, -L:, :]
+    mask = attention_mask
+    if (L <= _NATIVE_BLOCK and query.dtype in _lib._DT and k.dtype == v.dtype and k.dtype in _lib._DT and query.stride(3) == 1
+            and k.stride(3) == 1 and v.stride(3) == 1 and k.data_ptr() % 16 == 0 and not any(x % 8 for x in k.stride()[:3]) and (mask is None or (mask.dtype == torch.bool and mask.shape[1] == 1
+                                                           and mask.shape[0] in (1, B) and mask.stride(3) == 1 and mask.is_cuda))):
+        out = torch.empty(B, L, Hq, D, dtype=query.dtype, device=query.device)
+        tail = None if mask is None else mask[..., -L:]
+        _lib.check(_lib.lib.odmkv_block_merge(
+            query.data_ptr(), _lib.dtype_code(query), *query.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(),
+            *v.stride()[:3], _lib.dtype_code(k), _lib.ptr(tail), 0 if tail is None or tail.shape[0] == 1 else tail.stride(0),
+            0 if tail is None else tail.stride(2), B, Hq, key.shape[1], L, scaling, out_s.data_ptr(), lse_s.data_ptr(), out.data_ptr(),
+            stream_ptr(query.device)))
+        return out
     G = Hq // key.shape[1]
     k_new = key[:, :, -L:, :].float().repeat_interleave(G, dim=1)                # [B, Hq, L, D]
     v_new = value[:, :, -L:, :].float().repeat_interleave(G, dim=1)
@@ -143,6 +161,15 @@ def _attention_patch(func):
 
     @functools.wraps(func)
     def wrapper(module, query, key, value, attention_mask, dropout=0.0, **kwargs):
+        # a decode step like the layer's last one: the native block checks the call, stores the token and attends
+        state = module.__dict__.get("_odmkv_state")
+        fast = None if state is None else getattr(state, "_fast", None)
+        if fast is not None and attention_mask is None and not dropout:
+            out = fast.attend(query, key, value, kwargs, stream_ptr(state.device))
+            if out is not None:
+                object.__setattr__(module, "_odmkv_last_query", query)
+                call_counts["fused"] += 1
+                return out, None
         if query.shape[2] == key.shape[2] and not hasattr(key, "_odmkv_store_len"):      # a prefill (no cached tokens)
             module.masked_key_indices = None
             module._odmkv_state = None

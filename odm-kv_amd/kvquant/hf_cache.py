@@ -24,6 +24,10 @@ from __future__ import annotations
 import torch
 from transformers.cache_utils import DynamicLayer
 
+from kvquant._lib import _native
+
+alias = _native.alias             # stride-0 views of the last token (two views in one call)
+
 
 class PackedCacheLayer(DynamicLayer):
     def __init__(self, state, keys: torch.Tensor, values: torch.Tensor):
@@ -40,9 +44,7 @@ class PackedCacheLayer(DynamicLayer):
         self._alias(keys.shape[-2])
 
     def _alias(self, length: int) -> None:
-        k, v = self.recent
-        self.keys = k[:, :, -1:, :].expand(-1, -1, length, -1)
-        self.values = v[:, :, -1:, :].expand(-1, -1, length, -1)
+        self.keys, self.values = alias(*self.recent, length)
 
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, *args, **kwargs):
         q_len = key_states.shape[-2]

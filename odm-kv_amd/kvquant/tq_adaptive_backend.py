@@ -287,13 +287,63 @@ class TurboQuantAdaptiveKVCacheState:
         self._reset()
 
     # ------------------------------------------------------------------ storage
+    # While decode steps run through the native block (`_fast`, a _native.Step), it counts the tokens: the state's own
+    # numbers are brought up to date, and the block dropped, as soon as anything else looks at them.
+    _fast = None
+    _fast_dtypes = None           # (query, output) types the block was made for
+    _look = None                  # (block of its own for attention alone, or None; what it was made for)
+    _seq_len_ = 0
+    _counts_ = None
+    _exact_room_ = None
+
+    def _settle(self) -> None:
+        fast = self._fast
+        if fast is not None:
+            self._fast = None
+            self._seq_len_ = fast.seq_len
+            if fast.appended:
+                self._counts_[4] += fast.appended
+                self._exact_room_ -= fast.appended
+
+    @property
+    def seq_len(self) -> int:
+        fast = self._fast
+        return self._seq_len_ if fast is None else fast.seq_len
+
+    @seq_len.setter
+    def seq_len(self, n: int) -> None:
+        self._settle()
+        self._seq_len_ = int(n)
+
+    @property
+    def _counts(self):
+        """np.int64 [5, nseg]: tokens stored per level and segment."""
+        self._settle()
+        return self._counts_
+
+    @_counts.setter
+    def _counts(self, counts) -> None:
+        self._settle()
+        self._counts_ = counts
+
+    @property
+    def _exact_room(self):
+        """Tokens every exact segment can still take (None: not known)."""
+        self._settle()
+        return self._exact_room_
+
+    @_exact_room.setter
+    def _exact_room(self, room) -> None:
+        self._settle()
+        self._exact_room_ = room
+
     def _reset(self) -> None:
         self.batch_size = 0
         self.num_heads = 0
         self.seq_len = 0
         self._nseg = 0
-        self._counts = None           # np.int64 [5, nseg]   tokens stored per level and segment
-        self._exact_room = None       # tokens every exact segment can still take (None: not known)
+        self._counts = None
+        self._exact_room = None
         self._seg_tile = None         # np.int64 [5, nseg+1] first tile of each segment
         self._bufs = None
         self._level_store = None      # uint8 [B, H, capacity]: bit level of every position (grown by doubling)
@@ -301,7 +351,6 @@ class TurboQuantAdaptiveKVCacheState:
         self._items = None
         self._item_order = None
         self._worklist = None         # ctypes twin of odmkv_worklist_t over the tensors above
-        self._step = None             # decode_step's odmkv_step_t with what it was built for and what it points to
         self._items_choice = None     # (winning items-per-compute-unit multiple, packed bytes it was chosen at)
         self._packed = None
 
@@ -567,36 +616,42 @@ class TurboQuantAdaptiveKVCacheState:
         B, H, T, D = keys.shape
         if T == 0:
             return
-        if T > 1 or self._bufs is None or keys.dtype != self._exact_torch_dtype:
+        if self._bufs is None or keys.dtype != self._exact_torch_dtype:
             bits = torch.full((B, H, T), 16, dtype=torch.int32, device=self.device)
-            self.append(keys, values, bits)
+            counts = np.zeros((self._nseg, 6), np.int64)
+            counts[:, 5] = T
+            self.append(keys, values, bits, _known_counts=counts)
             return
         had = self._seg_tile
         room = self._exact_room
         new_counts = None
-        if room is None or room <= 0:
+        if room is None or room < T:
             new_counts = self._counts.copy()
-            new_counts[4] += 1
+            new_counts[4] += T
             self._ensure_capacity(new_counts)
             # tokens every exact segment can still take before a tile has to be added (the usual decode step
             # then skips the capacity arithmetic)
-            room = int((np.diff(self._seg_tile[4]) * TILE - new_counts[4]).min()) + 1
-        # the token is read where it lies (the newest row of the model's cache): no staging copies
-        k, v = keys[:, :, 0, :], values[:, :, 0, :]
-        if k.stride(2) != 1 or v.stride() != k.stride():
-            k, v = k.contiguous(), v.contiguous()
-        _lib.check(lib.odmkv_append_exact(C.byref(self._packed), k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1),
-                                          self.seq_len, _lib.stream_ptr(self.device)))
+            room = int((np.diff(self._seg_tile[4]) * TILE - new_counts[4]).min()) + T
+        # the tokens are read where they lie (the newest rows of the model's cache): no staging copies
+        if keys.stride(3) != 1 or values.stride(3) != 1 or values.stride()[:2] != keys.stride()[:2]:
+            keys, values = keys.contiguous(), values.contiguous()
+        st = _lib.stream_ptr(self.device)
+        if T == 1:
+            _lib.check(lib.odmkv_append_exact(C.byref(self._packed), keys.data_ptr(), values.data_ptr(), keys.stride(0),
+                                              keys.stride(1), self.seq_len, st))
+        else:
+            _lib.check(lib.odmkv_append_exact_rows(C.byref(self._packed), keys.data_ptr(), values.data_ptr(), T, keys.stride(0),
+                                                   keys.stride(1), keys.stride(2), values.stride(2), self.seq_len, st))
         if new_counts is None:
-            self._counts[4] += 1
+            self._counts[4] += T
         else:
             self._counts = new_counts
-        self._exact_room = room - 1
-        if self._level_store.shape[2] < self.seq_len + 1:
-            self._extend_levels(torch.full((B, H, 1), 16, dtype=torch.uint8, device=self.device))
+        self._exact_room = room - T
+        if self._level_store.shape[2] < self.seq_len + T:
+            self._extend_levels(torch.full((B, H, T), 16, dtype=torch.uint8, device=self.device))
         # otherwise nothing to write: the level store reads 16 behind seq_len (an exact token leaves
         # the evicted set as it is)
-        self.seq_len += 1
+        self.seq_len += T
         if had is not self._seg_tile:
             self._items = None
 
@@ -608,17 +663,11 @@ class TurboQuantAdaptiveKVCacheState:
         self.seq_len = seq_len
         self._masked = None
         # positions ascend inside a segment, so the survivors are a prefix of it
-        for li in range(5):
-            if self._counts[li].sum() == 0:
-                continue
-            pos = self._bufs["pos"][li].cpu().numpy()
-            for s in range(self._nseg):
-                c = int(self._counts[li, s])
-                if c:
-                    first = int(self._seg_tile[li, s]) * TILE
-                    self._counts[li, s] = int(np.searchsorted(pos[first:first + c], seq_len, side="left"))
-                    self._exact_room = None
-            self._bufs["seg_count"][li].copy_(torch.from_numpy(self._counts[li].astype(np.int32)))
+        counts = torch.empty((5, self._nseg), dtype=torch.int32, pin_memory=True)
+        _lib.check(lib.odmkv_truncate(C.byref(self._packed), seq_len, counts.data_ptr(), _lib.stream_ptr(self.device)))
+        torch.cuda.current_stream(self.device).synchronize()
+        self._counts = counts.numpy().astype(np.int64)
+        self._exact_room = None
         self._items = None
 
     # ------------------------------------------------------------------ reads
@@ -756,7 +805,7 @@ class TurboQuantAdaptiveKVCacheState:
         # drop the buffered tokens from the exact segments, then append them at their new levels
         self._counts[4] -= n_buf
         self._exact_room = None
-        self._bufs["seg_count"][4].copy_(torch.from_numpy(self._counts[4].astype(np.int32)))
+        _lib.check(lib.odmkv_drop_exact_tail(C.byref(self._packed), n_buf, _lib.stream_ptr(self.device)))
         self.append(k, v, bits, _pos_offset=start, _known_counts=known_counts)
 
     # ------------------------------------------------------------------ fused attention
@@ -797,7 +846,7 @@ class TurboQuantAdaptiveKVCacheState:
         w.items, w.item_range = self._items[0].data_ptr(), self._items[1].data_ptr()
         w.dispatch_order = _lib.ptr(self._item_order)
         w.n_items, w.n_workgroups = shape.n_items, shape.n_workgroups
-        w.wavefronts, w.two_per_cu = shape.wavefronts, shape.two_per_cu
+        w.wavefronts, w.two_per_cu, w.covers_exact = shape.wavefronts, shape.two_per_cu, 1
         self._worklist = w
 
     def decode_attention_block(self, query: torch.Tensor, scaling: Optional[float] = None):
@@ -805,8 +854,9 @@ class TurboQuantAdaptiveKVCacheState:
         prefill, a draft to verify): query [B, Hq, L, D] -> (out fp32 [B, Hq, L, D], lse fp32 [B, Hq, L]).
 
         The kernel's GQA sharing carries the block: the L tokens of a kv-head's G query heads are handed over as G * L
-        heads of that kv-head, up to 8 per call, so the packed bytes are streamed once per 8 // G tokens instead of
-        once per token (attention among the L tokens themselves is the caller's: see attention_patch)."""
+        heads of that kv-head, up to 8 per pass, so the packed bytes are streamed once per 8 // G tokens instead of
+        once per token, all passes in one launch (attention among the L tokens themselves is the caller's: see
+        attention_patch)."""
         _lib.require_gpu(query, "query")
         if query.dim() != 4:
             raise ValueError(f"query must be [B, Hq, L, D], got {tuple(query.shape)}")
@@ -817,16 +867,28 @@ class TurboQuantAdaptiveKVCacheState:
         G = Hq // H
         if G > 8:
             raise ValueError(f"GQA group {G} exceeds 8")
-        per = max(1, 8 // G)
+        if self._bufs is None:
+            raise ValueError("the store is empty")
+        if B != self.batch_size or D != self.head_dim:
+            raise ValueError(f"query {tuple(query.shape)} does not match the store (B={self.batch_size}, Hkv={H})")
+        if query.dtype not in _lib._DT:
+            query = query.float()
+        n = 4 if query.dtype == torch.float32 else 8
+        if query.stride(3) != 1 or any(x % n for x in query.stride()[:3]) or query.data_ptr() % 16:
+            query = query.contiguous()
         out = torch.empty(B, Hq, L, D, dtype=torch.float32, device=self.device)
         lse = torch.empty(B, Hq, L, dtype=torch.float32, device=self.device)
-        q5 = query.reshape(B, H, G, L, D)
-        for l0 in range(0, L, per):
-            lc = min(per, L - l0)
-            qv = q5[:, :, :, l0:l0 + lc].permute(0, 1, 3, 2, 4).reshape(B, H * lc * G, D).contiguous()
-            o, s = self.decode_attention(qv, scaling=scaling, return_lse=True)
-            out.view(B, H, G, L, D)[:, :, :, l0:l0 + lc] = o.view(B, H, lc, G, D).permute(0, 1, 3, 2, 4)
-            lse.view(B, H, G, L)[:, :, :, l0:l0 + lc] = s.view(B, H, lc, G).permute(0, 1, 3, 2)
+        if L == 0:
+            return out, lse
+        if self._items is None:
+            self._build_items()
+        ws_bytes = lib.odmkv_decode_block_workspace_bytes(B, Hq, H, L, self._items[2])
+        ws = _lib.workspace(self.device, ws_bytes, "decode_block")
+        step = _lib.Step(C.pointer(self._packed), C.pointer(self._worklist), self._pi_k_ops.data_ptr(), self.pi_v.data_ptr(),
+                         self._decode_cb.data_ptr(), self._decode_cb_host, self._decode_inv, ws.data_ptr(), ws_bytes, B, Hq,
+                         _lib.dtype_code(query), _lib.F32, 1.0 / math.sqrt(D) if scaling is None else float(scaling))
+        _lib.check(lib.odmkv_decode_block(C.byref(step), query.data_ptr(), query.stride(0), query.stride(1), query.stride(2), L,
+                                          out.data_ptr(), lse.data_ptr(), _lib.stream_ptr(self.device)))
         return out, lse
 
     def decode_attention(self, query: torch.Tensor, scaling: Optional[float] = None,
@@ -835,6 +897,13 @@ class TurboQuantAdaptiveKVCacheState:
 
         query: [B, Hq, D] or [B, Hq, 1, D] on the GPU, fp16 / bf16 / fp32 (read as it is); returns
         [B, Hq, D] of `out_dtype` (accumulated in fp32, rounded once) and, on request, lse fp32 [B, Hq]."""
+        scale = 1.0 / math.sqrt(self.head_dim) if scaling is None else float(scaling)
+        look = self._look
+        if (look is not None and not return_lse and look[1] is self._items and look[2] is self._packed and look[3] is query.dtype
+                and look[4] is out_dtype and look[5] is self._worklist):
+            out = look[0].look(query, scale, _lib.stream_ptr(self.device))
+            if out is not None:
+                return out
         _lib.require_gpu(query, "query")
         if self._bufs is None:
             raise ValueError("the store is empty")
@@ -848,7 +917,6 @@ class TurboQuantAdaptiveKVCacheState:
         if self._items is None:
             self._build_items()
         items, ranges, n_items = self._items
-        scale = 1.0 / math.sqrt(D) if scaling is None else float(scaling)
         out = torch.empty(B, Hq, D, dtype=out_dtype, device=self.device)
         lse = torch.empty(B, Hq, dtype=torch.float32, device=self.device) if return_lse else None
         ws_bytes = lib.odmkv_decode_workspace_bytes(B, Hq, n_items)
@@ -858,45 +926,52 @@ class TurboQuantAdaptiveKVCacheState:
             self._pi_k_ops.data_ptr(), self.pi_v.data_ptr(), self._decode_cb.data_ptr(),
             self._decode_cb_host, self._decode_inv, out.data_ptr(), _lib.dtype_code(out), _lib.ptr(lse), ws.data_ptr(), ws_bytes,
             _lib.stream_ptr(self.device)))
+        if not return_lse:
+            # a second call over the same work list: those that follow like it go through the native block
+            if look is not None and look[1] is self._items:
+                self._look = (self._native_step(Hq, q.dtype, out_dtype, scale, 0), self._items, self._packed, q.dtype, out_dtype, self._worklist)
+            else:
+                self._look = (None, self._items, None, None, None, None)
         return (out, lse) if return_lse else out
 
     def decode_step(self, query: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, scaling: Optional[float] = None,
                     out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
         """``append_all_exact(keys, values)`` (one new token, [B, Hkv, 1, D]) followed by ``decode_attention(query)``:
         what one layer does in one decode step under a press that buffers new tokens exact.  When the exact segments
-        have room for the token (every step but the one in 64 that opens a tile) both run in one library call whose
-        constant arguments are kept in a block per store and work list."""
-        room = self._exact_room
-        if (room is None or room <= 0 or self._bufs is None or keys.shape[2] != 1 or keys.dtype != self._exact_torch_dtype
-                or self._level_store.shape[2] < self.seq_len + 1 or not query.is_contiguous()
-                or query.dtype not in (torch.float16, torch.bfloat16, torch.float32)):
-            self.append_all_exact(keys, values)
-            return self.decode_attention(query, scaling=scaling, out_dtype=out_dtype)
-        _lib.require_gpu(query, "query")
-        self._validate_shapes(keys, values, None)
-        B, Hq = query.shape[0], query.shape[1]
-        if self._items is None:
-            self._build_items()
+        have room for the token both run in one native call whose constant arguments are kept in a block per store and
+        work list."""
         scale = 1.0 / math.sqrt(self.head_dim) if scaling is None else float(scaling)
-        stream = _lib.stream_ptr(self.device)
-        key = (Hq, query.dtype, out_dtype, scale, stream)
-        blk = self._step
-        if blk is None or blk[4] is not self._packed or blk[5] is not self._worklist or blk[0] != key:
-            if B != self.batch_size or Hq % self.num_heads != 0 or query.numel() != B * Hq * self.head_dim:
-                raise ValueError(f"query {tuple(query.shape)} does not match the store (B={self.batch_size}, Hkv={self.num_heads})")
-            ws_bytes = lib.odmkv_decode_workspace_bytes(B, Hq, self._items[2])
-            ws = _lib.workspace(self.device, ws_bytes, "decode")
-            st = _lib.Step(C.pointer(self._packed), C.pointer(self._worklist), self._pi_k_ops.data_ptr(), self.pi_v.data_ptr(),
-                           self._decode_cb.data_ptr(), self._decode_cb_host, self._decode_inv, ws.data_ptr(), ws_bytes, B, Hq,
-                           _lib.dtype_code(query), _lib._DT[out_dtype], scale)
-            blk = self._step = (key, st, C.byref(st), ws, self._packed, self._worklist)
-        k, v = keys[:, :, 0, :], values[:, :, 0, :]
-        if k.stride(2) != 1 or v.stride() != k.stride():
-            k, v = k.contiguous(), v.contiguous()
-        out = torch.empty(B, Hq, self.head_dim, dtype=out_dtype, device=self.device)
-        _lib.check(lib.odmkv_decode_step(blk[2], query.data_ptr(), k.data_ptr(), v.data_ptr(), k.stride(0), k.stride(1),
-                                         self.seq_len, out.data_ptr(), None, stream))
-        self._counts[4] += 1
-        self._exact_room = room - 1
-        self.seq_len += 1
+        fast = self._fast
+        if fast is not None and self._fast_dtypes == (query.dtype, out_dtype):
+            out = fast.step(query, keys, values, scale, _lib.stream_ptr(self.device))
+            if out is not None:
+                return out.squeeze(1)
+        self.append_all_exact(keys, values)
+        out = self.decode_attention(query, scaling=scale, out_dtype=out_dtype)
+        self._arm_step(int(query.shape[1]), query.dtype, out_dtype, scale)
         return out
+
+    def _arm_step(self, n_q: int, q_dtype: torch.dtype, out_dtype: torch.dtype, scale: float) -> None:
+        """The native block for the steps that follow like the one just made: they run as one library call until the exact
+        segments or the level map are full, or the store is touched in any other way."""
+        room = self._exact_room
+        if room is not None and self._level_store is not None:
+            room = min(room, self._level_store.shape[2] - self.seq_len)
+        if (room is None or room <= 0 or self._bufs is None or self._items is None or q_dtype not in _lib._DT
+                or out_dtype not in _lib._DT):
+            return
+        self._fast = self._native_step(n_q, q_dtype, out_dtype, scale, room)
+        self._fast_dtypes = (q_dtype, out_dtype)
+
+    def _native_step(self, n_q: int, q_dtype: torch.dtype, out_dtype: torch.dtype, scale: float, room: int):
+        stream = _lib.stream_ptr(self.device)
+        ws_bytes = lib.odmkv_decode_workspace_bytes(self.batch_size, n_q, self._items[2])
+        ws = _lib.workspace(self.device, ws_bytes, "decode")
+        cb_host, inv = self._decode_cb_host, self._decode_inv
+        index = self.device.index
+        return _lib._native.Step(
+            _lib.STEP_ENTRY, C.addressof(self._packed), C.addressof(self._worklist), self._pi_k_ops.data_ptr(), self.pi_v.data_ptr(),
+            self._decode_cb.data_ptr(), C.addressof(cb_host), C.addressof(inv), ws.data_ptr(), ws_bytes, stream, self.batch_size, n_q,
+            self.num_heads, _lib._DT[q_dtype], _lib._DT[out_dtype], torch.cuda.current_device() if index is None else index, scale,
+            bool(getattr(self, "exact_decode_append", False)), self.seq_len, room,
+            (self._packed, self._worklist, self._items, self._bufs, ws, self._pi_k_ops, self.pi_v, self._decode_cb, cb_host, inv))
