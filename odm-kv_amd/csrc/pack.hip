@@ -1840,20 +1840,15 @@ extern "C" int odmkv_store_finish_staged(const int32_t* chunk_counts, int n_chun
 // dequantise to dense tensors
 // ------------------------------------------------------------------------------------------------
 struct DequantArgs {
+    odmkv_packed_t s;
     void* K;
     void* V;
     int64_t sB, sH, sT;
-    int Hkv, nseg, T, t_min;           // positions t_min <= t < T are written
+    int nseg, T, t_min;                // positions t_min <= t < T are written
     const float* pi_k;
     const float* pi_v;
-    const float* cb;
-    const int32_t* pos;
-    const int32_t* seg_tile;
-    const int32_t* seg_count;
-    const uint8_t* kcodes;
-    const uint8_t* vcodes;
-    const float* knorm;
-    const float* vnorm;
+    const float* cb;                   // centroids of widths 2, 3, 4, 8 back to back
+    int tile_base[ODMKV_NQ + 1];       // running sum of the levels' tile counts
 };
 
 // x_hat[token][j] = |x| * sum_i c[code_i] * Pi[i][j] on the fp16 matrix cores (v_mfma_f32_16x16x32_f16): operand
@@ -1861,147 +1856,211 @@ struct DequantArgs {
 // (three products: hi*hi, lo*hi, hi*lo; the fourth is below 2^-22), accumulated in fp32.  The result differs from
 // the fp32 sum by about 1e-6 of the row's norm: less than the rounding of a 16-bit cache by two orders of magnitude.
 // Persistent workgroups of DQ_NW waves keep Pi^T in LDS in operand order (even workgroups keys, odd ones values) and
-// walk the level's tiles, a wave per tile.  A lane ends up with four consecutive outputs of one token: 8 (16) bytes
-// of a row per store.
+// walk the tiles of all levels, a wave per tile.
 #define DQ_NW 8
-template <int W, int DT>
-__global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a, int n_tiles) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    uint16_t* pih = reinterpret_cast<uint16_t*>(smem);                             // Pi^T hi, then lo, in operand order
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    uint8_t* codes = smem + QP_PI_BYTES + wave * QP_STAGE;                         // this wave's [token][dim] codes (values)
-    uint32_t* cb = reinterpret_cast<uint32_t*>(smem + QP_PI_BYTES + DQ_NW * QP_STAGE);   // [256] centroids: fp16 hi | lo << 16
-    float* norms = reinterpret_cast<float*>(cb + 256) + wave * TILE;              // [DQ_NW][64] norm of the wave's tokens
-    long long* offs = reinterpret_cast<long long*>(cb + 256 + DQ_NW * TILE) + wave * TILE;   // element offset of the row, -1: none
-    const bool is_v = (blockIdx.x & 1) != 0;
-    {
-        // lane 16q + r of block (jb, ch) holds Pi[32 ch + 8 q .. + 7][16 jb + r]
-        const float4* __restrict__ src = reinterpret_cast<const float4*>(is_v ? a.pi_v : a.pi_k);
-        constexpr int PER_THREAD = HD * HD / 4 / (DQ_NW * 64);
-        float4 p[PER_THREAD];
+#define DQ_CB_WORDS CODEBOOK_FLOATS
+#define DQ_MAX_RUNS 1024                 // (level, segment) pairs whose tile counts fit the walk table
+// LDS: Pi^T (hi, lo) | per-wave codes | centroids (fp16 hi | lo << 16) | norms | row offsets | walk table
+#define DQ_LDS (QP_PI_BYTES + DQ_NW * QP_STAGE + DQ_CB_WORDS * 4 + DQ_NW * TILE * (4 + 8) + (DQ_MAX_RUNS + 1) * 4)
+
+// Pi^T as the A operands of dq_tile, hi then lo: lane 16 q + r of block (jb, ch) holds Pi[32 ch + 8 q .. + 7][j] of the
+// output j = 32 (jb >> 1) + 8 (r >> 2) + 4 (jb & 1) + (r & 3): a lane's accumulators of two neighbouring blocks are then
+// eight consecutive outputs.
+__device__ static inline void dq_load_rotation(const float* pi, uint16_t* pih, int tid) {
+    const float4* __restrict__ src = reinterpret_cast<const float4*>(pi);
+    constexpr int PER_THREAD = HD * HD / 4 / (DQ_NW * 64);
+    float4 p[PER_THREAD];
 #pragma unroll
-        for (int k = 0; k < PER_THREAD; ++k) p[k] = src[tid + k * (DQ_NW * 64)];
+    for (int k = 0; k < PER_THREAD; ++k) p[k] = src[tid + k * (DQ_NW * 64)];
 #pragma unroll
-        for (int k = 0; k < PER_THREAD; ++k) {
-            const int c = tid + k * (DQ_NW * 64);                // four consecutive j of row i
-            const int i = c >> 5, j0 = (c & 31) * 4;
-            const int ch = i >> 5, q = (i >> 3) & 3, e = i & 7;
-            const float pv[4] = {p[k].x, p[k].y, p[k].z, p[k].w};
+    for (int k = 0; k < PER_THREAD; ++k) {
+        const int c = tid + k * (DQ_NW * 64);                // four consecutive j of row i
+        const int i = c >> 5, j0 = (c & 31) * 4;
+        const int ch = i >> 5, q = (i >> 3) & 3, e = i & 7;
+        const float pv[4] = {p[k].x, p[k].y, p[k].z, p[k].w};
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int j = j0 + t, jb = j >> 4, r = j & 15;
-                const int dst = (((jb * 4 + ch) * 64) + 16 * q + r) * 8 + e;
-                const uint16_t h = Elem<ODMKV_F16>::from_f32(pv[t]);
-                pih[dst] = h;
-                pih[HD * HD + dst] = Elem<ODMKV_F16>::from_f32(pv[t] - Elem<ODMKV_F16>::to_f32(h));
+        for (int t = 0; t < 4; ++t) {
+            const int j = j0 + t, jb = 2 * (j >> 5) + ((j >> 2) & 1), r = 4 * ((j >> 3) & 3) + (j & 3);
+            const int dst = (((jb * 4 + ch) * 64) + 16 * q + r) * 8 + e;
+            const uint16_t h = Elem<ODMKV_F16>::from_f32(pv[t]);
+            pih[dst] = h;
+            pih[HD * HD + dst] = Elem<ODMKV_F16>::from_f32(pv[t] - Elem<ODMKV_F16>::to_f32(h));
+        }
+    }
+}
+__device__ static inline uint32_t dq_centroid(float c) {
+    const uint16_t h = Elem<ODMKV_F16>::from_f32(c);
+    return (uint32_t)h | ((uint32_t)Elem<ODMKV_F16>::from_f32(c - Elem<ODMKV_F16>::to_f32(h)) << 16);
+}
+
+// One tile of 64 tokens: codes one byte each [token][dim] in LDS (rows of CODE_ROW), cb the width's centroids, offs the
+// element offset of every token's row in `out` (-1: none).
+// Every operand of Pi^T is read once for all four token blocks (64 KB of LDS reads per tile; with a read per block, 256 KB,
+// the LDS pipe and the latency of its reads set the time), whose four accumulators are chains of their own; a lane stores 16
+// bytes of a row at a time, a token's four lanes 64.  A 2-bit layer of 32k tokens and 8 heads (both tensors): 81 -> 39 us.
+template <int DT>
+__device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* codes, const uint32_t* cb, const float* norms,
+                                               const long long* offs, void* out, int lane) {
+    const int r16 = lane & 15, q = lane >> 4;
+    uint4 bh[4][4], bl[4][4];                                 // B: the centroids of the token's codes 32 ch + 8 q .. + 7
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch) {
+            const uint2 cw = *reinterpret_cast<const uint2*>(&codes[(16 * tb + r16) * CODE_ROW + 32 * ch + 8 * q]);
+            const uint32_t w2[2] = {cw.x, cw.y};
+            uint32_t t[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t[e] = cb[(w2[e >> 2] >> (8 * (e & 3))) & 0xffu];
+            bh[tb][ch] = make_uint4(__builtin_amdgcn_perm(t[1], t[0], 0x05040100u), __builtin_amdgcn_perm(t[3], t[2], 0x05040100u),
+                                    __builtin_amdgcn_perm(t[5], t[4], 0x05040100u), __builtin_amdgcn_perm(t[7], t[6], 0x05040100u));
+            bl[tb][ch] = make_uint4(__builtin_amdgcn_perm(t[1], t[0], 0x07060302u), __builtin_amdgcn_perm(t[3], t[2], 0x07060302u),
+                                    __builtin_amdgcn_perm(t[5], t[4], 0x07060302u), __builtin_amdgcn_perm(t[7], t[6], 0x07060302u));
+        }
+#pragma unroll 1
+    for (int jp = 0; jp < 4; ++jp) {                          // outputs 32 jp .. + 31
+        qf_f4 acc[2][4];
+#pragma unroll
+        for (int o2 = 0; o2 < 2; ++o2)
+#pragma unroll
+            for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = (qf_f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int o2 = 0; o2 < 2; ++o2)
+#pragma unroll
+            for (int ch = 0; ch < 4; ++ch) {
+                const uint4 ah = piA[((2 * jp + o2) * 4 + ch) * 64 + lane];
+                const uint4 al = piA[HD * HD / 8 + ((2 * jp + o2) * 4 + ch) * 64 + lane];
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = qf_mfma<ODMKV_F16>(ah, bh[tb][ch], acc[o2][tb]);
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = qf_mfma<ODMKV_F16>(al, bh[tb][ch], acc[o2][tb]);
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = qf_mfma<ODMKV_F16>(ah, bl[tb][ch], acc[o2][tb]);
+            }
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) {
+            const long long off = offs[16 * tb + r16];
+            const float nrm = norms[16 * tb + r16];
+            if (off >= 0) {                                   // outputs 32 jp + 8 q .. + 7 of the token
+                float r[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) r[e] = acc[e >> 2][tb][e & 3] * nrm;
+                store8<DT>(out, (size_t)off + 32 * jp + 8 * q, r);
             }
         }
-        for (int i = tid; i < (1 << W); i += DQ_NW * 64) {
-            const float c = a.cb[i];
-            const uint16_t h = Elem<ODMKV_F16>::from_f32(c);
-            cb[i] = (uint32_t)h | ((uint32_t)Elem<ODMKV_F16>::from_f32(c - Elem<ODMKV_F16>::to_f32(h)) << 16);
+    }
+}
+
+// the tile's codes of width W -> one byte each in LDS, [token][dim]: the matrix operand wants eight consecutive dims of a
+// token per lane, the tile keeps (4 tokens x 32 dims) of keys or (16 tokens x 8 dims) of values per lane
+template <int W>
+__device__ static __forceinline__ void dq_unpack(const uint8_t* src, bool is_v, uint8_t* codes, int lane) {
+    const int n = lane & 15, j = lane >> 4;
+    uint32_t words[4 * W];
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+        const uint4 v = *reinterpret_cast<const uint4*>(src + ((size_t)c * TILE + lane) * 16);
+        words[4 * c] = v.x; words[4 * c + 1] = v.y; words[4 * c + 2] = v.z; words[4 * c + 3] = v.w;
+    }
+    if (!is_v) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int i = 0; i < 32; i += 4) {
+                const uint32_t w4 = get_code<W>(words, 32 * b + i) | (get_code<W>(words, 32 * b + i + 1) << 8) |
+                                    (get_code<W>(words, 32 * b + i + 2) << 16) | (get_code<W>(words, 32 * b + i + 3) << 24);
+                *reinterpret_cast<uint32_t*>(&codes[key_slot(n, b) * CODE_ROW + 32 * j + i]) = w4;
+            }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    codes[(32 * k + 8 * j + e) * CODE_ROW + 16 * m + n] = (uint8_t)get_code<W>(words, 64 * k + 8 * m + e);
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t* codes = smem + QP_PI_BYTES + wave * QP_STAGE;                         // this wave's [token][dim] codes
+    uint32_t* cb = reinterpret_cast<uint32_t*>(smem + QP_PI_BYTES + DQ_NW * QP_STAGE);
+    float* norms = reinterpret_cast<float*>(cb + DQ_CB_WORDS) + wave * TILE;      // [DQ_NW][64] norm of the wave's tokens
+    long long* offs = reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + wave * TILE;   // element offset of the row, -1: none
+    int* wbase = reinterpret_cast<int*>(reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + DQ_NW * TILE);
+    const bool is_v = (blockIdx.x & 1) != 0;
+    // running count of the tiles that hold tokens over the (level, segment) pairs, so that the waves share out those alone
+    const int n_runs = ODMKV_NQ * a.nseg;
+    const bool table = n_runs <= DQ_MAX_RUNS;
+    if (table)
+        for (int e = tid; e < DQ_MAX_RUNS; e += DQ_NW * 64)
+            wbase[e + 1] = e < n_runs ? (a.s.seg_count[e / a.nseg][e % a.nseg] + TILE - 1) / TILE : 0;
+    dq_load_rotation(is_v ? a.pi_v : a.pi_k, reinterpret_cast<uint16_t*>(smem), tid);
+    for (int i = tid; i < DQ_CB_WORDS; i += DQ_NW * 64) cb[i] = dq_centroid(a.cb[i]);
+    __syncthreads();
+    if (table && wave == 0) {                                  // 16 entries per lane, a scan over the lanes' totals
+        int mine[DQ_MAX_RUNS / 64], tot = 0;
+#pragma unroll
+        for (int i = 0; i < DQ_MAX_RUNS / 64; ++i) { mine[i] = wbase[lane * (DQ_MAX_RUNS / 64) + i + 1]; tot += mine[i]; }
+        int incl = tot;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(incl, o, WAVE);
+            if (lane >= o) incl += up;
         }
+        int run = incl - tot;
+#pragma unroll
+        for (int i = 0; i < DQ_MAX_RUNS / 64; ++i) { run += mine[i]; wbase[lane * (DQ_MAX_RUNS / 64) + i + 1] = run; }
+        if (lane == 0) wbase[0] = 0;
     }
     __syncthreads();
     const uint4* piA = reinterpret_cast<const uint4*>(smem);
     void* out = is_v ? a.V : a.K;
     const int wg = blockIdx.x >> 1, n_wg = gridDim.x >> 1;
-    const int r16 = lane & 15, q = lane >> 4;
-    for (int tile = wg * DQ_NW + wave; tile < n_tiles; tile += n_wg * DQ_NW) {
-        const int bh = find_segment(a.seg_tile, a.nseg, tile);
-        const int ts = (tile - a.seg_tile[bh]) * TILE;
-        const int hi = min(a.seg_count[bh] - ts, TILE);
-        if (hi <= 0) continue;                                       // wave-uniform
+    const int total = table ? wbase[n_runs] : a.tile_base[ODMKV_NQ];
+    for (int wi = wg * DQ_NW + wave; wi < total; wi += n_wg * DQ_NW) {
+        int li, bh, tile, hi;
+        if (table) {
+            int e = 0;                                           // the largest pair with wbase[e] <= wi
+            for (int step = DQ_MAX_RUNS / 2; step >= 1; step >>= 1)
+                if (e + step < n_runs && wbase[e + step] <= wi) e += step;
+            li = e / a.nseg; bh = e - li * a.nseg;
+            const int local = wi - wbase[e];
+            tile = a.s.seg_tile[li][bh] + local;
+            hi = min(a.s.seg_count[li][bh] - local * TILE, TILE);
+        } else {
+            li = 0;
+#pragma unroll
+            for (int k = 1; k < ODMKV_NQ; ++k) li += (wi >= a.tile_base[k]);
+            tile = wi - a.tile_base[li];
+            bh = find_segment(a.s.seg_tile[li], a.nseg, tile);
+            hi = min(a.s.seg_count[li][bh] - (tile - a.s.seg_tile[li][bh]) * TILE, TILE);
+            if (hi <= 0) continue;                               // wave-uniform
+        }
         // positions ascend inside a segment: a tile whose last token lies before t_min has nothing to write
-        if (a.t_min > 0 && a.pos[(size_t)tile * TILE + hi - 1] < a.t_min) continue;
-        const size_t slot = (size_t)tile * TILE + lane;
+        const int32_t* pos = a.s.pos[li] + (size_t)tile * TILE;
+        if (a.t_min > 0 && pos[hi - 1] < a.t_min) continue;
         const bool valid = lane < hi;
         {
-            const int t = valid ? a.pos[slot] : -1;
+            const int t = valid ? pos[lane] : -1;
             const bool write = valid && t >= a.t_min && t < a.T;
-            offs[lane] = write ? (long long)((size_t)(bh / a.Hkv) * a.sB + (size_t)(bh % a.Hkv) * a.sH + (size_t)t * a.sT) : -1ll;
-            norms[lane] = valid ? (is_v ? a.vnorm[slot] : a.knorm[slot]) : 0.0f;
+            offs[lane] = write ? (long long)((size_t)(bh / a.s.Hkv) * a.sB + (size_t)(bh % a.s.Hkv) * a.sH + (size_t)t * a.sT) : -1ll;
+            norms[lane] = valid ? (is_v ? a.s.vnorm[li] : a.s.knorm[li])[(size_t)tile * TILE + lane] : 0.0f;
         }
-        // the lane's 128 codes -> one byte each in LDS, [token][dim]: the matrix operand below wants eight consecutive
-        // dims of a token per lane, the tile keeps (4 tokens x 32 dims) of keys or (16 tokens x 8 dims) of values per lane
-        {
-            const int n = lane & 15, j = lane >> 4;
-            const uint8_t* src = (is_v ? a.vcodes : a.kcodes) + (size_t)tile * (TILE * 16 * W);
-            uint32_t words[4 * W];
-#pragma unroll
-            for (int c = 0; c < W; ++c) {
-                const uint4 v = *reinterpret_cast<const uint4*>(src + ((size_t)c * TILE + lane) * 16);
-                words[4 * c] = v.x; words[4 * c + 1] = v.y; words[4 * c + 2] = v.z; words[4 * c + 3] = v.w;
-            }
-            if (!is_v) {
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-#pragma unroll
-                    for (int i = 0; i < 32; i += 4) {
-                        const uint32_t w4 = get_code<W>(words, 32 * b + i) | (get_code<W>(words, 32 * b + i + 1) << 8) |
-                                            (get_code<W>(words, 32 * b + i + 2) << 16) | (get_code<W>(words, 32 * b + i + 3) << 24);
-                        *reinterpret_cast<uint32_t*>(&codes[key_slot(n, b) * CODE_ROW + 32 * j + i]) = w4;
-                    }
-            } else {
-#pragma unroll
-                for (int k = 0; k < 2; ++k)
-#pragma unroll
-                    for (int m = 0; m < 8; ++m)
-#pragma unroll
-                        for (int e = 0; e < 8; ++e)
-                            codes[(32 * k + 8 * j + e) * CODE_ROW + 16 * m + n] = (uint8_t)get_code<W>(words, 64 * k + 8 * m + e);
-            }
+        const uint8_t* src = (is_v ? a.s.vcodes[li] : a.s.kcodes[li]) + (size_t)tile * (TILE * 16) * width_of(li);
+        switch (li) {
+            case 0: dq_unpack<2>(src, is_v, codes, lane); break;
+            case 1: dq_unpack<3>(src, is_v, codes, lane); break;
+            case 2: dq_unpack<4>(src, is_v, codes, lane); break;
+            default: dq_unpack<8>(src, is_v, codes, lane); break;
         }
         wave_lds_fence();
-#pragma unroll 1
-        for (int tb = 0; tb < 4; ++tb) {
-            // (the lane index is made opaque per round: Pi^T's 64 operand reads do not depend on the round, and hoisted
-            // out of it they would take every register there is)
-            int ln = lane;
-            asm volatile("" : "+v"(ln));
-            const int token = 16 * tb + r16;
-            const long long off = offs[token];
-            const float nrm = norms[token];
-            // operand B: the centroids of the token's codes 32 ch + 8 q .. + 7, high and low halves
-            uint4 bh4[4], bl4[4];
-#pragma unroll
-            for (int ch = 0; ch < 4; ++ch) {
-                const uint2 cw = *reinterpret_cast<const uint2*>(&codes[token * CODE_ROW + 32 * ch + 8 * q]);
-                const uint32_t w2[2] = {cw.x, cw.y};
-                uint32_t t[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) t[e] = cb[(w2[e >> 2] >> (8 * (e & 3))) & 0xffu];
-                bh4[ch] = make_uint4(__builtin_amdgcn_perm(t[1], t[0], 0x05040100u), __builtin_amdgcn_perm(t[3], t[2], 0x05040100u),
-                                     __builtin_amdgcn_perm(t[5], t[4], 0x05040100u), __builtin_amdgcn_perm(t[7], t[6], 0x05040100u));
-                bl4[ch] = make_uint4(__builtin_amdgcn_perm(t[1], t[0], 0x07060302u), __builtin_amdgcn_perm(t[3], t[2], 0x07060302u),
-                                     __builtin_amdgcn_perm(t[5], t[4], 0x07060302u), __builtin_amdgcn_perm(t[7], t[6], 0x07060302u));
-            }
-#pragma unroll
-            for (int jb = 0; jb < 8; ++jb) {
-                qf_f4 acc = (qf_f4){0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int ch = 0; ch < 4; ++ch) {
-                    const uint4 ah = piA[(jb * 4 + ch) * 64 + ln];
-                    const uint4 al = piA[HD * HD / 8 + (jb * 4 + ch) * 64 + ln];
-                    acc = qf_mfma<ODMKV_F16>(ah, bh4[ch], acc);
-                    acc = qf_mfma<ODMKV_F16>(al, bh4[ch], acc);
-                    acc = qf_mfma<ODMKV_F16>(ah, bl4[ch], acc);
-                }
-                if (off >= 0) {                                     // outputs 16 jb + 4 q .. + 3 of the token
-                    const float r[4] = {acc[0] * nrm, acc[1] * nrm, acc[2] * nrm, acc[3] * nrm};
-                    const int c4 = 16 * jb + 4 * q;
-                    if constexpr (DT == ODMKV_F32) {
-                        *reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + off + c4) = make_float4(r[0], r[1], r[2], r[3]);
-                    } else {
-                        const uint32_t lo = (uint32_t)Elem<DT>::from_f32(r[0]) | ((uint32_t)Elem<DT>::from_f32(r[1]) << 16);
-                        const uint32_t hi2 = (uint32_t)Elem<DT>::from_f32(r[2]) | ((uint32_t)Elem<DT>::from_f32(r[3]) << 16);
-                        *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(out) + off + c4) = make_uint2(lo, hi2);
-                    }
-                }
-            }
-        }
-        wave_lds_fence();                                            // offs / norms / codes free for the next tile
+        dq_tile<DT>(piA, codes, cb + codebook_offset(li), norms, offs, out, lane);
+        wave_lds_fence();                                        // offs / norms / codes free for the next tile
     }
 }
 
@@ -2030,37 +2089,25 @@ __global__ __launch_bounds__(64) void exact_scatter_kernel(odmkv_packed_t s, voi
     }
 }
 
-template <int W, int DT>
-static int launch_dequant_w(const DequantArgs& da, int n_tiles, hipStream_t st) {
-    const size_t lds = QP_PI_BYTES + (size_t)DQ_NW * QP_STAGE + 256 * sizeof(float) + DQ_NW * TILE * (sizeof(float) + sizeof(long long));
-    static bool attr_set = false;
-    if (!attr_set) {
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(dequant_kernel<W, DT>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
-    int dev = 0, cus = 256;
-    ODMKV_CHECK_HIP(hipGetDevice(&dev));
-    ODMKV_CHECK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    // one persistent workgroup per compute unit, keys on the even and values on the odd ones; never
-    // more workgroups than there are tiles for their waves
-    int pairs = cus / 2;
-    const int need = (n_tiles + DQ_NW - 1) / DQ_NW;
-    if (pairs > need) pairs = need;
-    if (pairs < 1) pairs = 1;
-    hipLaunchKernelGGL((dequant_kernel<W, DT>), dim3(2 * pairs), dim3(DQ_NW * 64), lds, st, da, n_tiles);
-    ODMKV_CHECK_LAUNCH("dequant_kernel");
-    return 0;
+static int compute_units() {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) return v;
+    return 256;
 }
 
 template <int DT>
-static int launch_dequant(const DequantArgs& da, int li, int n_tiles, hipStream_t st) {
-    switch (li) {
-        case 0: return launch_dequant_w<2, DT>(da, n_tiles, st);
-        case 1: return launch_dequant_w<3, DT>(da, n_tiles, st);
-        case 2: return launch_dequant_w<4, DT>(da, n_tiles, st);
-        default: return launch_dequant_w<8, DT>(da, n_tiles, st);
+static int launch_dequant(const DequantArgs& da, hipStream_t st) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(dequant_kernel<DT>), hipFuncAttributeMaxDynamicSharedMemorySize, DQ_LDS));
+        attr_set = true;
     }
+    // one persistent workgroup per compute unit, keys on the even and values on the odd ones; never
+    // more workgroups than there are tiles for their waves
+    const int need = (da.tile_base[ODMKV_NQ] + DQ_NW - 1) / DQ_NW, pairs = std::max(1, std::min(compute_units() / 2, need));
+    hipLaunchKernelGGL(dequant_kernel<DT>, dim3(2 * pairs), dim3(DQ_NW * 64), DQ_LDS, st, da);
+    ODMKV_CHECK_LAUNCH("dequant_kernel");
+    return 0;
 }
 
 extern "C" int odmkv_dequant(const odmkv_packed_t* store, void* K, void* V, int dtype, int T,
@@ -2083,19 +2130,15 @@ extern "C" int odmkv_dequant_from(const odmkv_packed_t* store, void* K, void* V,
                     "dequant: strides must keep rows 16-byte aligned");
     ODMKV_CHECK_ARG(((uintptr_t)K & 15) == 0 && ((uintptr_t)V & 15) == 0, "dequant: K/V must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
-    const int nseg = store->B * store->Hkv;
-    for (int li = 0; li < ODMKV_NQ; ++li) {
-        if (store->n_tiles[li] == 0) continue;
-        DequantArgs da;
-        da.K = K; da.V = V; da.sB = stride_b; da.sH = stride_h; da.sT = stride_t;
-        da.Hkv = store->Hkv; da.nseg = nseg; da.T = T; da.t_min = t_min;
-        da.pi_k = pi_k; da.pi_v = pi_v; da.cb = codebooks + codebook_offset(li);
-        da.pos = store->pos[li]; da.seg_tile = store->seg_tile[li]; da.seg_count = store->seg_count[li];
-        da.kcodes = store->kcodes[li]; da.vcodes = store->vcodes[li];
-        da.knorm = store->knorm[li]; da.vnorm = store->vnorm[li];
-        int rc = dtype == ODMKV_F16 ? launch_dequant<ODMKV_F16>(da, li, store->n_tiles[li], st)
-               : dtype == ODMKV_BF16 ? launch_dequant<ODMKV_BF16>(da, li, store->n_tiles[li], st)
-                                     : launch_dequant<ODMKV_F32>(da, li, store->n_tiles[li], st);
+    DequantArgs da;
+    da.s = *store; da.K = K; da.V = V; da.sB = stride_b; da.sH = stride_h; da.sT = stride_t;
+    da.nseg = store->B * store->Hkv; da.T = T; da.t_min = t_min;
+    da.pi_k = pi_k; da.pi_v = pi_v; da.cb = codebooks;
+    da.tile_base[0] = 0;
+    for (int li = 0; li < ODMKV_NQ; ++li) da.tile_base[li + 1] = da.tile_base[li] + store->n_tiles[li];
+    if (da.tile_base[ODMKV_NQ] > 0) {
+        const int rc = dtype == ODMKV_F16 ? launch_dequant<ODMKV_F16>(da, st)
+                     : dtype == ODMKV_BF16 ? launch_dequant<ODMKV_BF16>(da, st) : launch_dequant<ODMKV_F32>(da, st);
         if (rc) return rc;
     }
     if (include_exact && store->n_tiles[4] > 0) {
