@@ -309,6 +309,21 @@ int odmkv_quantize_rows(const void* x, int dtype, int64_t N, int64_t stride_n, i
 int odmkv_dequantize_rows(const uint8_t* codes, const float* norms, int64_t N, int bits,
                           const float* pi, const float* cb, float* out, void* stream);
 
+/* The same with the codes in the reference's container bytes (_pack_indices, kvquant/tq_backend.py:103-125: 2-bit codes four
+ * to a byte, 3- and 4-bit codes two to a byte, 8-bit codes as they are). */
+int odmkv_quantize_rows_packed(const void* x, int dtype, int64_t N, int64_t stride_n, int bits,
+                               const float* pi, const float* cb, uint8_t* indices, float* norms, void* stream);
+int odmkv_dequantize_rows_packed(const uint8_t* indices, const float* norms, int64_t N, int bits,
+                                 const float* pi, const float* cb, float* out, void* stream);
+
+/* Rows of K and V quantised and dequantised in place (float16 / bfloat16): groups x group_rows rows each, row (g, t) at
+ * element g * stride_group + t * stride_row of both (what the uniform-width press does to the model's cache,
+ * kvquant/backend_press.py:94-148).  workspace: odmkv_round_trip_workspace_bytes(groups * group_rows). */
+size_t odmkv_round_trip_workspace_bytes(int64_t n);
+int odmkv_round_trip_rows(void* K, void* V, int dtype, int64_t groups, int64_t group_rows, int64_t stride_group,
+                          int64_t stride_row, int bits_k, int bits_v, const float* pi_k, const float* pi_v,
+                          const float* cb_k, const float* cb_v, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Dequantise the store into dense [B, Hkv, T, 128] tensors of `dtype` (strides as above):
  * x_hat = (centroids[code] @ Pi) * norm, cast to dtype, written at the stored positions
  * (TurboQuantMSE.dequantize, kvquant/tq_backend.py:199-203, and the scatter of

@@ -1065,27 +1065,9 @@ __device__ static __forceinline__ void qf_code_tile(const void* base, const uint
     }
 }
 
-// Entries first .. first + n - 1 of the wave's list (n <= 64), a lane each: the value by the definition's
-// own chain, its code, and that code in place of the estimate's in the packed tile.  The tile's codes,
-// positions and norms were written by this wave: the caller has waited for those stores.
-template <int DT, bool IS_V>
-__device__ static void qf_fix_listed(const QuantArgs& a, const float* thrs, const QfWave& w, int lane, int first, int n) {
-    const bool on = lane < n;
-    const uint32_t e = w.list[first + (on ? lane : 0)];
-    const int token = e & 63, out = (e >> 6) & 127, gt = (int)(e >> 13);
-    int li = 0;
-#pragma unroll
-    for (int k = 1; k < ODMKV_NQ; ++k) li += (gt >= a.tile_base[k]);
-    const int tile = gt - a.tile_base[li];
-    const int bh = find_segment(a.s.seg_tile[li], a.nseg, tile);
-    const size_t slot = (size_t)tile * TILE + token;
-    const size_t off = (size_t)(bh / a.Hkv) * a.sB + (size_t)(bh % a.Hkv) * a.sH +
-                       (size_t)(a.s.pos[li][slot] - a.pos_offset) * a.sT;
-    // written by this wave a moment ago: read past the vector cache
-    const float den = __hip_atomic_load((IS_V ? a.s.vnorm[li] : a.s.knorm[li]) + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1e-10f;
-    RowRegs<DT> x;
-    x.load(IS_V ? a.V : a.K, off);
-    const float4* __restrict__ prow = reinterpret_cast<const float4*>((IS_V ? a.pi_v : a.pi_k) + out * HD);
+// the definition's own value: the row's quotients times Pi's row, one fused multiply-add after the other
+template <int DT>
+__device__ static __forceinline__ float qf_chain(const RowRegs<DT>& x, const float4* __restrict__ prow, float den) {
     float y = 0.0f;
     bool row_plain = !(den >= 9.094947017729282e-13f && den <= 1.152921504606847e18f);
     if constexpr (DT != ODMKV_F16) {                            // fp16 elements cannot get that small against their norm
@@ -1123,6 +1105,31 @@ __device__ static void qf_fix_listed(const QuantArgs& a, const float* thrs, cons
             for (int e4 = 0; e4 < 4; ++e4) y = __fmaf_rn(x.get(4 * c + e4) / den, pv[e4], y);
         }
     }
+    return y;
+}
+
+// Entries first .. first + n - 1 of the wave's list (n <= 64), a lane each: the value by the definition's
+// own chain, its code, and that code in place of the estimate's in the packed tile.  The tile's codes,
+// positions and norms were written by this wave: the caller has waited for those stores.
+template <int DT, bool IS_V>
+__device__ static void qf_fix_listed(const QuantArgs& a, const float* thrs, const QfWave& w, int lane, int first, int n) {
+    const bool on = lane < n;
+    const uint32_t e = w.list[first + (on ? lane : 0)];
+    const int token = e & 63, out = (e >> 6) & 127, gt = (int)(e >> 13);
+    int li = 0;
+#pragma unroll
+    for (int k = 1; k < ODMKV_NQ; ++k) li += (gt >= a.tile_base[k]);
+    const int tile = gt - a.tile_base[li];
+    const int bh = find_segment(a.s.seg_tile[li], a.nseg, tile);
+    const size_t slot = (size_t)tile * TILE + token;
+    const size_t off = (size_t)(bh / a.Hkv) * a.sB + (size_t)(bh % a.Hkv) * a.sH +
+                       (size_t)(a.s.pos[li][slot] - a.pos_offset) * a.sT;
+    // written by this wave a moment ago: read past the vector cache
+    const float den = __hip_atomic_load((IS_V ? a.s.vnorm[li] : a.s.knorm[li]) + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1e-10f;
+    RowRegs<DT> x;
+    x.load(IS_V ? a.V : a.K, off);
+    const float4* __restrict__ prow = reinterpret_cast<const float4*>((IS_V ? a.pi_v : a.pi_k) + out * HD);
+    const float y = qf_chain<DT>(x, prow, den);
     // code = number of thresholds at or below y; the entries of a pass may be of different widths
     const int W = width_of(li);
     const float* thr = thrs + thr_offset(li);
@@ -1330,6 +1337,35 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
 }
 
 template <int DT>
+__device__ static inline void qf_load_rotation(const float* pi, uint16_t* pih, int tid) {
+    // Pi -> hi + lo in the rows' 16-bit type, in the order the matrix instruction reads a 16-output x 32-step block:
+    // lane 16q + r of block (ob, ch) holds Pi[16 ob + r][32 ch + 8 q .. + 7]
+    // (all of a thread's reads are asked for at once: eight round trips to memory would cost more
+    // than the tiles of a short call)
+    const float4* __restrict__ pi4 = reinterpret_cast<const float4*>(pi);
+    constexpr int PER_THREAD = HD * HD / 4 / (QF_NW * 64);
+    float4 p[PER_THREAD];
+#pragma unroll
+    for (int k = 0; k < PER_THREAD; ++k) p[k] = pi4[tid + k * (QF_NW * 64)];
+#pragma unroll
+    for (int k = 0; k < PER_THREAD; ++k) {
+        const int c = tid + k * (QF_NW * 64);               // four consecutive j of row i
+        const int i = c >> 5, j = (c & 31) * 4;
+        const int ob = i >> 4, r = i & 15, ch = j >> 5, q = (j >> 3) & 3, e = j & 7;
+        const int dst = (((ob * 4 + ch) * 64) + 16 * q + r) * 8 + e;
+        const float pv[4] = {p[k].x, p[k].y, p[k].z, p[k].w};
+        uint16_t h[4], l[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            h[t] = Elem<DT>::from_f32(pv[t]);
+            l[t] = Elem<DT>::from_f32(pv[t] - Elem<DT>::to_f32(h[t]));
+        }
+        *reinterpret_cast<uint2*>(pih + dst) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+        *reinterpret_cast<uint2*>(pih + HD * HD + dst) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+    }
+}
+
+template <int DT>
 __global__ __launch_bounds__(QF_NW * 64) void quant_pack_f16_kernel(QuantArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     uint16_t* pih = reinterpret_cast<uint16_t*>(smem);
@@ -1354,31 +1390,7 @@ __global__ __launch_bounds__(QF_NW * 64) void quant_pack_f16_kernel(QuantArgs a)
         }
     }
     {
-        // Pi -> hi + lo in the rows' 16-bit type, in the order the matrix instruction reads a 16-output x 32-step block:
-        // lane 16q + r of block (ob, ch) holds Pi[16 ob + r][32 ch + 8 q .. + 7]
-        // (all of a thread's reads are asked for at once: eight round trips to memory would cost more
-        // than the tiles of a short call)
-        const float4* __restrict__ pi4 = reinterpret_cast<const float4*>(is_v ? a.pi_v : a.pi_k);
-        constexpr int PER_THREAD = HD * HD / 4 / (QF_NW * 64);
-        float4 p[PER_THREAD];
-#pragma unroll
-        for (int k = 0; k < PER_THREAD; ++k) p[k] = pi4[tid + k * (QF_NW * 64)];
-#pragma unroll
-        for (int k = 0; k < PER_THREAD; ++k) {
-            const int c = tid + k * (QF_NW * 64);               // four consecutive j of row i
-            const int i = c >> 5, j = (c & 31) * 4;
-            const int ob = i >> 4, r = i & 15, ch = j >> 5, q = (j >> 3) & 3, e = j & 7;
-            const int dst = (((ob * 4 + ch) * 64) + 16 * q + r) * 8 + e;
-            const float pv[4] = {p[k].x, p[k].y, p[k].z, p[k].w};
-            uint16_t h[4], l[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                h[t] = Elem<DT>::from_f32(pv[t]);
-                l[t] = Elem<DT>::from_f32(pv[t] - Elem<DT>::to_f32(h[t]));
-            }
-            *reinterpret_cast<uint2*>(pih + dst) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-            *reinterpret_cast<uint2*>(pih + HD * HD + dst) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
-        }
+        qf_load_rotation<DT>(is_v ? a.pi_v : a.pi_k, pih, tid);
         for (int i = tid; i < QP_THR_FLOATS; i += QF_NW * 64) {
             const int li = i < 3 ? 0 : i < 10 ? 1 : i < 25 ? 2 : 3;
             const int k = i - thr_offset(li);
@@ -2152,5 +2164,205 @@ extern "C" int odmkv_dequant_from(const odmkv_packed_t* store, void* K, void* V,
             hipLaunchKernelGGL((exact_scatter_kernel<ODMKV_F32>), grid, block, 0, st, *store, K, V, stride_b, stride_h, stride_t, T, bf);
         ODMKV_CHECK_LAUNCH("exact_scatter_kernel");
     }
+    return 0;
+}
+
+// ------------------------------------------------------------------------------------------------
+// rows outside the store on the matrix cores: the 16-bit quantiser's estimate with the codes as bytes or in the reference's
+// container, and the dequantiser from byte codes.  Workgroups of the even index take job 0, of the odd one job 1 (keys and
+// values of a layer in one launch), a wave a tile of 64 rows.  A row per lane without them took 150 us for 64512 rows (the
+// fused multiply-adds of the rotation on the vector ALU), here 27 us.
+// ------------------------------------------------------------------------------------------------
+struct RowsArgs { RowsJob job[2]; int n_jobs; };
+
+template <int DT, int W>
+__device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* thr, QfWave& w, uint8_t* stage, int lane, long long tile0,
+                               long long stride) {
+    const long long tiles = (j.n + TILE - 1) / TILE;
+    const int row_bytes = j.packed ? container_bytes(W) : HD;
+    constexpr int EFF = W == 3 ? 4 : W;
+    int n_listed = 0, it = 0;                                   // it: the tile's number in this wave's walk (what the list keeps)
+    if (lane == 0) w.count = 0;
+    const auto fix = [&](int first, int n) {                    // n <= 64 listed values, a lane each, by the definition
+        const bool on = lane < n;
+        const uint32_t e = w.list[first + (on ? lane : 0)];
+        const int out = (e >> 6) & 127;
+        const long long r = (tile0 + (long long)(e >> 13) * stride) * TILE + (e & 63);
+        // written by this wave a moment ago: read past the vector cache
+        const float den = __hip_atomic_load(j.norms + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1e-10f;
+        RowRegs<DT> x;
+        x.load(j.x, (size_t)row_offset(j, r));
+        const float y = qf_chain<DT>(x, reinterpret_cast<const float4*>(j.pi + out * HD), den);
+        int code = 0;
+#pragma unroll
+        for (int st = (1 << W) / 2; st >= 1; st >>= 1)
+            if (y >= thr[code + st - 1]) code += st;
+        if (!on) return;
+        if (!j.packed) { j.codes[(size_t)r * HD + out] = (uint8_t)code; return; }
+        const int bit = EFF * out;
+        uint32_t* word = reinterpret_cast<uint32_t*>(j.codes + (size_t)r * row_bytes) + (bit >> 5);
+        const uint32_t old = (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> (bit & 31)) & ((1u << W) - 1u);
+        if (old != (uint32_t)code) atomicXor(word, (old ^ (uint32_t)code) << (bit & 31));
+    };
+    for (long long tile = tile0; tile < tiles; tile += stride, ++it) {
+        const long long r = tile * TILE + lane;
+        const bool valid = r < j.n;
+        const long long off = valid ? row_offset(j, r) : 0;
+        RowRegs<DT> x;
+        if (valid) x.load(j.x, (size_t)off);
+        else x.zero();
+        float ss = 0.0f;
+#pragma unroll
+        for (int e = 0; e < HD; ++e) {
+            const float xj = x.get(e);
+            ss = __fmaf_rn(xj, xj, ss);
+        }
+        const float norm = sqrtf(ss);
+        bool odd = !(ss <= 3.4028234663852886e38f);              // as in qf_walk
+        if constexpr (DT != ODMKV_F16) {
+            uint32_t any = 0u;
+#pragma unroll
+            for (int i = 0; i < RowRegs<DT>::N; ++i) any |= x.w[i];
+            odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
+        }
+        const bool ok = !__any(odd);
+        const int n_before = n_listed;
+        int n = 0;
+        if (ok) {
+            const float den = norm + 1e-10f;
+            w.off[lane] = valid ? (unsigned long long)off : ~0ull;
+            w.rinv[lane] = 1.0f / den;
+            w.band[lane] = (valid && ss > 0.0f) ? (DT == ODMKV_F16 ? QF_BAND : QF_BAND_BF16) : -1.0f;
+            wave_lds_fence();
+            qf_code_tile<DT, W, false, false>(j.x, piA, thr, w, stage, lane, it);
+            wave_lds_fence();
+            n = w.count;
+        }
+        if (ok && n <= QF_LIST) {
+            const int rows = (int)min((long long)TILE, j.n - tile * TILE);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {                       // sixteen codes of a row per lane and turn
+                const int token = 8 * i + (lane >> 3), piece = lane & 7;
+                const uint4 v = *reinterpret_cast<const uint4*>(stage + token * CODE_ROW + 16 * piece);
+                if (token >= rows) continue;
+                uint8_t* dst = j.codes + (size_t)(tile * TILE + token) * row_bytes;
+                if (!j.packed) { *reinterpret_cast<uint4*>(dst + 16 * piece) = v; continue; }
+                const uint32_t b[4] = {v.x, v.y, v.z, v.w};     // four codes each -> EFF bits apart
+                uint32_t g[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) g[k] = (b[k] & 0xffu) | ((b[k] >> (8 - EFF)) & (0xffu << EFF)) | ((b[k] >> (16 - 2 * EFF)) & (0xffu << (2 * EFF))) | ((b[k] >> (24 - 3 * EFF)) & (0xffu << (3 * EFF)));
+                if constexpr (EFF == 2) *reinterpret_cast<uint32_t*>(dst + 4 * piece) = (g[0] & 0xffu) | ((g[1] & 0xffu) << 8) | ((g[2] & 0xffu) << 16) | (g[3] << 24);
+                else *reinterpret_cast<uint2*>(dst + 8 * piece) = make_uint2((g[0] & 0xffffu) | (g[1] << 16), (g[2] & 0xffffu) | (g[3] << 16));
+            }
+            if (valid) j.norms[r] = norm;
+            n_listed = n;
+        } else {
+            if (valid) j.norms[r] = __uint_as_float(ROWS_HANDED_OVER);       // the exact kernel behind this one does the tile
+            n_listed = n_before;
+            if (ok && lane == 0) w.count = n_before;
+        }
+        wave_lds_fence();
+        const bool more = tile + stride < tiles;
+        if (n_listed >= WAVE || (!more && n_listed > 0)) {
+            __builtin_amdgcn_s_waitcnt(0);                      // this wave's codes and norms are in memory
+            while (n_listed >= WAVE) { n_listed -= WAVE; fix(n_listed, WAVE); }
+            if (!more && n_listed > 0) { fix(0, n_listed); n_listed = 0; }
+            if (lane == 0) w.count = n_listed;
+            wave_lds_fence();
+        }
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(QF_NW * 64) void quant_rows_f16_kernel(RowsArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const RowsJob& j = a.job[a.n_jobs == 2 ? (blockIdx.x & 1) : 0];
+    float* thr = reinterpret_cast<float*>(smem + QF_PI_BYTES + QF_NW * QP_STAGE);
+    uint8_t* stage = smem + QF_PI_BYTES + wave * QP_STAGE;
+    QfWave& w = reinterpret_cast<QfWave*>(smem + QF_PI_BYTES + QF_NW * QP_STAGE + QF_THR_BYTES)[wave];
+    qf_load_rotation<DT>(j.pi, reinterpret_cast<uint16_t*>(smem), tid);
+    if (tid < (1 << j.bits) - 1) thr[tid] = decision_threshold(j.cb[tid], j.cb[tid + 1]);
+    __syncthreads();
+    const uint4* piA = reinterpret_cast<const uint4*>(smem);
+    const long long first = (long long)(blockIdx.x / a.n_jobs) * QF_NW + wave, stride = (long long)(gridDim.x / a.n_jobs) * QF_NW;
+    switch (j.bits) {
+        case 2: qr_walk<DT, 2>(j, piA, thr, w, stage, lane, first, stride); break;
+        case 3: qr_walk<DT, 3>(j, piA, thr, w, stage, lane, first, stride); break;
+        default: qr_walk<DT, 4>(j, piA, thr, w, stage, lane, first, stride); break;
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const RowsJob& j = a.job[a.n_jobs == 2 ? (blockIdx.x & 1) : 0];
+    uint8_t* codes = smem + QP_PI_BYTES + wave * QP_STAGE;
+    uint32_t* cb = reinterpret_cast<uint32_t*>(smem + QP_PI_BYTES + DQ_NW * QP_STAGE);
+    float* norms = reinterpret_cast<float*>(cb + DQ_CB_WORDS) + wave * TILE;
+    long long* offs = reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + wave * TILE;
+    dq_load_rotation(j.pi, reinterpret_cast<uint16_t*>(smem), tid);
+    for (int i = tid; i < (1 << j.bits); i += DQ_NW * 64) cb[i] = dq_centroid(j.cb[i]);
+    __syncthreads();
+    const long long tiles = (j.n + TILE - 1) / TILE, stride = (long long)(gridDim.x / a.n_jobs) * DQ_NW;
+    for (long long tile = (long long)(blockIdx.x / a.n_jobs) * DQ_NW + wave; tile < tiles; tile += stride) {
+        const long long r = tile * TILE + lane;
+        const bool valid = r < j.n;
+        offs[lane] = valid ? row_offset(j, r) : -1ll;
+        norms[lane] = valid ? j.norms[r] : 0.0f;
+        const int rows = (int)min((long long)TILE, j.n - tile * TILE);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int token = 8 * i + (lane >> 3), piece = lane & 7;
+            const uint4 v = token < rows ? *reinterpret_cast<const uint4*>(j.codes + (size_t)(tile * TILE + token) * HD + 16 * piece) : make_uint4(0u, 0u, 0u, 0u);
+            *reinterpret_cast<uint4*>(codes + token * CODE_ROW + 16 * piece) = v;
+        }
+        wave_lds_fence();
+        dq_tile<DT>(reinterpret_cast<const uint4*>(smem), codes, cb, norms, offs, j.out, lane);
+        wave_lds_fence();
+    }
+}
+
+static dim3 rows_grid(const RowsJob* jobs, int n_jobs, int waves) {
+    long long most = 0;
+    for (int i = 0; i < n_jobs; ++i) most = std::max(most, (jobs[i].n + TILE * waves - 1) / (TILE * waves));
+    return dim3((unsigned)(n_jobs * std::max<long long>(1, std::min<long long>(most, compute_units() / n_jobs))));
+}
+
+int launch_quantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
+    const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QP_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave);
+    static bool attr_set = false;
+    if (!attr_set) {
+        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_f16_kernel<ODMKV_F16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_f16_kernel<ODMKV_BF16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        attr_set = true;
+    }
+    RowsArgs a;
+    for (int i = 0; i < 2; ++i) a.job[i] = jobs[i < n_jobs ? i : 0];
+    a.n_jobs = n_jobs;
+    const dim3 grid = rows_grid(jobs, n_jobs, QF_NW);
+    if (dtype == ODMKV_F16) hipLaunchKernelGGL(quant_rows_f16_kernel<ODMKV_F16>, grid, dim3(QF_NW * 64), lds, st, a);
+    else hipLaunchKernelGGL(quant_rows_f16_kernel<ODMKV_BF16>, grid, dim3(QF_NW * 64), lds, st, a);
+    ODMKV_CHECK_LAUNCH("quant_rows_f16_kernel");
+    return 0;
+}
+
+int launch_dequantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dequant_rows_f16_kernel<ODMKV_F16>), hipFuncAttributeMaxDynamicSharedMemorySize, DQ_LDS));
+        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dequant_rows_f16_kernel<ODMKV_BF16>), hipFuncAttributeMaxDynamicSharedMemorySize, DQ_LDS));
+        attr_set = true;
+    }
+    RowsArgs a;
+    for (int i = 0; i < 2; ++i) a.job[i] = jobs[i < n_jobs ? i : 0];
+    a.n_jobs = n_jobs;
+    const dim3 grid = rows_grid(jobs, n_jobs, DQ_NW);
+    if (dtype == ODMKV_F16) hipLaunchKernelGGL(dequant_rows_f16_kernel<ODMKV_F16>, grid, dim3(DQ_NW * 64), DQ_LDS, st, a);
+    else hipLaunchKernelGGL(dequant_rows_f16_kernel<ODMKV_BF16>, grid, dim3(DQ_NW * 64), DQ_LDS, st, a);
+    ODMKV_CHECK_LAUNCH("dequant_rows_f16_kernel");
     return 0;
 }

@@ -94,3 +94,28 @@ __device__ static inline void store8(void* base, size_t elem_off, const float* v
     }
 }
 
+// ---- rows outside the packed store (rows.hip, pack.hip) -------------------------------------------
+// n rows of 128 elements: row r lies at element (r / group_rows) * s_group + (r % group_rows) * s_row of x (and of out).
+struct RowsJob {
+    const void* x;
+    long long s_group, s_row, group_rows, n;
+    int bits, packed;            // packed: codes in the reference's container bytes, else a byte each [n, 128]
+    const float* pi;
+    const float* cb;             // the width's centroids
+    uint8_t* codes;
+    float* norms;                // [n]
+    void* out;
+};
+__host__ __device__ static inline long long row_offset(const RowsJob& j, long long r) {
+    return j.group_rows >= j.n ? r * j.s_row : (r / j.group_rows) * j.s_group + (r % j.group_rows) * j.s_row;
+}
+// bytes of a row of container codes: 2 bits four to a byte, 3 and 4 bits two to a byte, 8 bits as they are
+__host__ __device__ static inline int container_bytes(int bits) { return bits == 2 ? HD / 4 : bits <= 4 ? HD / 2 : HD; }
+// a tile of 64 rows that the matrix-core quantiser leaves to the exact one carries this in place of its first norm
+#define ROWS_HANDED_OVER 0x7fc0beefu
+// the exact quantiser (rows.hip); flagged: only tiles that carry the mark
+int launch_quantize_rows_exact(const RowsJob& j, int dtype, bool flagged, hipStream_t st);
+// the matrix-core quantiser for 16-bit rows of 2, 3 and 4 bits, and the matrix-core dequantiser from byte codes into
+// 16-bit rows (pack.hip), one or two jobs a launch
+int launch_quantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st);
+int launch_dequantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st);

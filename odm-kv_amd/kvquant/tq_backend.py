@@ -200,31 +200,36 @@ class TurboQuantMSE:
         self.pi = cached_rotation(dim, self.device, seed)
         self.centroids = _load_or_compute_codebook(bits, dim, self.device, torch.float32).contiguous()
 
-    def quantize_codes(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-        """x [..., d] -> (codes uint8 [..., d] one per byte, norms fp32 [...])."""
+    def _quantize(self, x: torch.Tensor, entry, row_bytes: int) -> tuple[torch.Tensor, torch.Tensor]:
         _lib.require_gpu(x, "x")
         flat = x.reshape(-1, self.dim)
         if flat.stride(-1) != 1:
             flat = flat.contiguous()
         n = flat.shape[0]
-        codes = torch.empty(n, self.dim, dtype=torch.uint8, device=x.device)
+        codes = torch.empty(n, row_bytes, dtype=torch.uint8, device=x.device)
         norms = torch.empty(n, dtype=torch.float32, device=x.device)
-        _lib.check(lib.odmkv_quantize_rows(
+        _lib.check(entry(
             flat.data_ptr(), _lib.dtype_code(flat), n, flat.stride(0), self.bits,
             self.pi.data_ptr(), self.centroids.data_ptr(), codes.data_ptr(), norms.data_ptr(),
             _lib.stream_ptr(x.device)))
-        return codes.reshape(*x.shape), norms.reshape(x.shape[:-1])
+        return codes.reshape(*x.shape[:-1], row_bytes), norms.reshape(x.shape[:-1])
+
+    def quantize_codes(self, x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        """x [..., d] -> (codes uint8 [..., d] one per byte, norms fp32 [...])."""
+        return self._quantize(x, lib.odmkv_quantize_rows, self.dim)
 
     def quantize(self, x: torch.Tensor) -> MSEQuantized:
-        codes, norms = self.quantize_codes(x)
-        return MSEQuantized(indices=_pack_indices(codes, self.bits), norms=norms, bits=self.bits)
+        indices, norms = self._quantize(x, lib.odmkv_quantize_rows_packed, self.dim // _container(self.bits)[0])
+        return MSEQuantized(indices=indices, norms=norms, bits=self.bits)
 
     def dequantize(self, q: MSEQuantized) -> torch.Tensor:
-        codes = _unpack_indices(q.indices, q.bits, self.dim).to(torch.uint8)
-        flat = codes.reshape(-1, self.dim).contiguous()
+        row_bytes = self.dim // _container(q.bits)[0]
+        if q.bits not in SUPPORTED_WIDTHS or q.indices.shape[-1] != row_bytes:
+            raise ValueError(f"indices of shape {tuple(q.indices.shape)} do not hold {self.dim} codes of {q.bits} bits")
+        flat = q.indices.reshape(-1, row_bytes).contiguous()
         norms = q.norms.float().reshape(-1).contiguous()
         out = torch.empty(flat.shape[0], self.dim, dtype=torch.float32, device=flat.device)
-        _lib.check(lib.odmkv_dequantize_rows(
+        _lib.check(lib.odmkv_dequantize_rows_packed(
             flat.data_ptr(), norms.data_ptr(), flat.shape[0], q.bits, self.pi.data_ptr(),
             self.centroids.data_ptr(), out.data_ptr(), _lib.stream_ptr(flat.device)))
-        return out.reshape(*codes.shape)
+        return out.reshape(*q.indices.shape[:-1], self.dim)

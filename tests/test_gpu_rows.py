@@ -1,0 +1,53 @@
+"""GPU: rows outside the store.  The matrix-core quantiser gives the exact quantiser's codes (the same numbers as fp32 rows take
+the exact kernel), in bytes and in the container; the in-place round trip gives dequantize(quantize(x))."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(n, dtype, seed):
+    x = torch.randn(n, 128, generator=torch.Generator().manual_seed(seed))
+    if n > 40:
+        x[3], x[4], x[5, 7], x[6, 9] = 0.0, 1e-6, float("inf"), float("nan")
+        x[7] *= 3e3
+        x[8, 1:] = 0.0
+    return x.to(dtype).cuda()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 700, 33000])
+def test_codes_of_16_bit_rows(n, bits, dtype):
+    from kvquant.tq_backend import TurboQuantMSE, _pack_indices
+    x = _rows(n, dtype, 10 * n + bits)
+    q = TurboQuantMSE(128, bits, device="cuda", dtype=dtype, seed=7)
+    codes, norms = q.quantize_codes(x)
+    exact, exact_norms = q.quantize_codes(x.float())
+    assert torch.equal(codes, exact) and torch.equal(norms.view(torch.int32), exact_norms.view(torch.int32))
+    mq = q.quantize(x)
+    assert torch.equal(mq.indices, _pack_indices(exact, bits)) and torch.equal(mq.norms.view(torch.int32), norms.view(torch.int32))
+    strided = torch.zeros(n, 256, dtype=dtype, device="cuda")
+    strided[:, 128:] = x
+    assert torch.equal(q.quantize_codes(strided[:, 128:])[0], exact)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,H,T,lo,hi,bits", [(1, 1, 1, 0, 1, (3, 2)), (2, 3, 90, 17, 81, (2, 4)), (1, 8, 1300, 0, 1172, (3, 2)), (2, 2, 70, 0, 70, (8, 3))])
+def test_round_trip_in_place(B, H, T, lo, hi, bits, dtype):
+    from kvquant import TurboQuantBackendPress
+    g = torch.Generator().manual_seed(T)
+    k, v = (torch.randn(B, H, T, 128, generator=g).to(dtype).cuda() for _ in range(2))
+    press = TurboQuantBackendPress(key_bits=bits[0], value_bits=bits[1], value_quantizer="mse")
+    want = []
+    for x, b, seed in ((k, bits[0], 42), (v, bits[1], 2042)):
+        q = press._q(b, seed, x)
+        y = x.clone()
+        y[:, :, lo:hi] = q.dequantize(q.quantize(x[:, :, lo:hi].reshape(-1, 128))).reshape(B, H, hi - lo, 128).to(dtype)
+        want.append(y)
+    got_k, got_v = k.clone(), v.clone()
+    press._quantise_span(0, got_k, got_v, lo, hi)
+    step = 2 ** -10 if dtype == torch.float16 else 2 ** -7         # one step of the type: fp32 sums in another order
+    for got, y in zip((got_k, got_v), want):
+        assert torch.equal(got[:, :, :lo], y[:, :, :lo]) and torch.equal(got[:, :, hi:], y[:, :, hi:])
+        assert ((got.float() - y.float()).abs() <= step * y.float().abs() + 1e-5).all()
