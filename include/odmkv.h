@@ -85,6 +85,25 @@ int odmkv_token_mean(const void* x, int dtype, int batch, int rows, int cols, in
 int odmkv_average_rope(const void* mu, const void* cosine, const void* sine, int dtype, int heads, int positions,
                        float* out, void* stream);
 
+/* Mean and covariance of the queries of every head, through the averaged RoPE (kvquant/scorer.py:204-257,
+ * kvquant/attention_utils.py:57-115): q float16 / bfloat16, head h and token t at element h * stride_h + t * stride_t; cosine,
+ * sine fp32 [positions, 128] or NULL (no RoPE); mu fp32 [heads, 128], cov fp32 [heads, 128, 128]. */
+size_t odmkv_query_covariance_workspace_bytes(int heads, int tokens);
+int odmkv_query_covariance(const void* q, int dtype, int heads, int tokens, int64_t stride_h, int64_t stride_t,
+                           const float* cosine, const float* sine, int positions, float* mu, float* cov,
+                           void* workspace, size_t workspace_bytes, void* stream);
+
+/* RoPE of a window's queries: q [heads, tokens, 128] (element strides) with cosine, sine [tokens, 128] of the same type, out
+ * contiguous; every product and sum is rounded to the type. */
+int odmkv_rotate_queries(const void* q, int dtype, int heads, int tokens, int64_t stride_h, int64_t stride_t,
+                         const void* cosine, const void* sine, void* out, void* stream);
+
+/* scores fp32 [rows, cols] -> out [rows, pad + cols]: the first pad columns are the largest score, and with scale != 0
+ * everything is normalised to [0, 1] over the whole tensor (0.5 everywhere if max - min < 1e-8; kvquant/scorer.py:36-66). */
+size_t odmkv_normalize_workspace_bytes(void);
+int odmkv_normalize_scores(const float* scores, int64_t rows, int64_t cols, int pad, int scale, float* out,
+                           void* workspace, size_t workspace_bytes, void* stream);
+
 /* Expected-attention score.  Replaces ExpectedAttentionScorer.score_prefill after the query
  * statistics are known (kvquant/scorer.py:204-257):
  *

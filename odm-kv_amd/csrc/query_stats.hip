@@ -178,3 +178,341 @@ extern "C" int odmkv_average_rope(const void* mu, const void* cosine, const void
     ODMKV_CHECK_LAUNCH("average_rope_kernel");
     return 0;
 }
+
+// ------------------------------------------------------------------------------------------------
+// mean and covariance of the queries of every head, passed through the averaged RoPE:
+//   mu = sum_t q_t / n,  C = sum_t (q_t - mu) (q_t - mu)^T / n,  mu' = R mu,  C' = R C R^T,  R = diag(c) + diag(s) (half rotation)
+// The queries are taken relative to a pivot near their mean (the mean of 64 of them, the same for every workgroup of a head),
+// x = q - pivot in fp32, and x as three bf16 pieces whose sum it is: six products of pieces on the matrix cores (what they
+// leave out is below 2^-24), fp32 sums over at most 512 tokens at a time, fp64 behind that, where the rest of the mean is
+// subtracted.  (Products of the 16-bit queries as they are would be exact and a sixth of the work, but with a mean several
+// times the deviation their fp32 sums keep less of the covariance than sums of centred queries do.)
+// v_mfma_f32_32x32x16_bf16: D[32x32] += A[32x16] B[16x32], lane l supplies A[l % 32][8 (l / 32) + e] and the same of B^T:
+// both operands are the queries with the dims along the lanes and eight tokens in a lane.  A lane loads four dims
+// (4 p .. 4 p + 3, p = l % 32) of eight tokens and pairs the tokens up by byte permutes: block b = the dims 4 p + b.  Ten of the
+// sixteen 32x32 blocks (the others mirror them).
+// Floors for 32 heads of 32k tokens: 268 MB once, 129 GFLOP of bf16 products.  As tensor operations (conversion, mean,
+// subtraction, fp32 product) 1050 us, here 139 + 25 (bound by the matrix cores: 0.93 PFLOP/s).
+// ------------------------------------------------------------------------------------------------
+#define CV_WAVES 8
+#define CV_BLOCKS 10                 // (0,0) (0,1) (0,2) (0,3) (1,1) (1,2) (1,3) (2,2) (2,3) (3,3)
+#define CV_PART (CV_BLOCKS * 1024 + 2 * HD)      // blocks, sum of x, pivot
+#define CV_TOKENS 512                // tokens a wavefront sums in fp32
+#define CV_SAMPLE 64                 // tokens of the pivot
+typedef float cv_f16 __attribute__((ext_vector_type(16)));
+typedef __bf16 cv_b8 __attribute__((ext_vector_type(8)));
+
+__device__ static __forceinline__ cv_f16 cv_mfma(const uint4& a, const uint4& b, const cv_f16& c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(cv_b8, a), __builtin_bit_cast(cv_b8, b), c, 0, 0, 0);
+}
+
+struct CovArgs {
+    const uint16_t* q;                   // head h, token t at h * sH + t * sT
+    long long sH, sT;
+    int tokens, slices, per_wave;        // per_wave: a multiple of 16
+    float* part;                         // [heads, slices, CV_PART]
+    const float* cosine;                 // [positions, 128] or null: no RoPE
+    const float* sine;
+    int positions;
+    float* rope;                         // [2, 128]
+    float* mu;                           // [heads, 128]
+    float* cov;                          // [heads, 128, 128]
+};
+
+template <int DT>
+__global__ __launch_bounds__(CV_WAVES * 64) void cov_part_kernel(CovArgs a) {
+    __shared__ float red[2][CV_WAVES][1024];
+    __shared__ float sums[CV_WAVES][HD];
+    __shared__ __align__(16) float pivot[HD];
+    const int slice = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = lane & 31, half = lane >> 5;
+    const int t0 = (slice * CV_WAVES + wave) * a.per_wave, t1 = min(t0 + a.per_wave, a.tokens);
+    const uint16_t* head = a.q + (long long)h * a.sH;
+    const uint16_t* base = head + 4 * p;
+    uint2 cur[8];
+    const auto request = [&](int t) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) cur[e] = *reinterpret_cast<const uint2*>(base + (long long)min(t + 8 * half + e, a.tokens - 1) * a.sT);
+    };
+    {
+        float s = 0.0f;
+        uint16_t v[CV_SAMPLE / 4];
+#pragma unroll
+        for (int i = 0; i < CV_SAMPLE / 4; ++i)
+            v[i] = head[(long long)(((long long)(4 * i + (tid >> 7)) * a.tokens) / CV_SAMPLE) * a.sT + (tid & 127)];
+        if (t0 < t1) request(t0);
+#pragma unroll
+        for (int i = 0; i < CV_SAMPLE / 4; ++i) s += Elem<DT>::to_f32(v[i]);
+        sums[tid >> 7][tid & 127] = s;
+        __syncthreads();
+        if (tid < HD) pivot[tid] = (sums[0][tid] + sums[1][tid] + sums[2][tid] + sums[3][tid]) / (float)CV_SAMPLE;
+        __syncthreads();
+    }
+    const float4 c4 = *reinterpret_cast<const float4*>(pivot + 4 * p);
+    const float c[4] = {c4.x, c4.y, c4.z, c4.w};
+    cv_f16 acc[CV_BLOCKS];
+#pragma unroll
+    for (int b = 0; b < CV_BLOCKS; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[b][r] = 0.0f;
+    float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int t = t0; t < t1; t += 16) {
+        uint4 op[3][4];                                               // pieces of the four blocks
+        const bool ragged = t + 16 > t1;                              // the last step (wave-uniform)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            uint32_t w[3][4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float x[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const uint32_t two = b < 2 ? cur[2 * r + k].x : cur[2 * r + k].y;
+                    x[k] = Elem<DT>::to_f32((uint16_t)((b & 1) ? two >> 16 : two & 0xffffu)) - c[b];
+                    if (ragged && t + 8 * half + 2 * r + k >= t1) x[k] = 0.0f;
+                    sum[b] += x[k];
+                }
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {                         // the upper half of each as a bf16 piece; the rest stays
+                    const uint32_t u0 = __float_as_uint(x[0]), u1 = __float_as_uint(x[1]);
+                    w[i][r] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+                    x[0] -= __uint_as_float(u0 & 0xffff0000u);
+                    x[1] -= __uint_as_float(u1 & 0xffff0000u);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) op[i][b] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+        }
+        if (t + 16 < t1) request(t + 16);                             // on their way under the products
+        int k = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = i; j < 4; ++j, ++k) {                        // small pieces first
+                acc[k] = cv_mfma(op[2][i], op[0][j], acc[k]);
+                acc[k] = cv_mfma(op[0][i], op[2][j], acc[k]);
+                acc[k] = cv_mfma(op[1][i], op[1][j], acc[k]);
+                acc[k] = cv_mfma(op[1][i], op[0][j], acc[k]);
+                acc[k] = cv_mfma(op[0][i], op[1][j], acc[k]);
+                acc[k] = cv_mfma(op[0][i], op[0][j], acc[k]);
+            }
+    }
+    __syncthreads();                                                  // (the sums' space held the pivot's shares)
+    // the eight wavefronts' blocks added up, one block at a time
+    float* part = a.part + ((size_t)h * a.slices + slice) * CV_PART;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const float s = sum[b] + __shfl_xor(sum[b], 32, WAVE);
+        if (half == 0) sums[wave][4 * p + b] = s;
+    }
+#pragma unroll
+    for (int k = 0; k < CV_BLOCKS; ++k) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[k & 1][wave][r * 64 + lane] = acc[k][r];
+        __syncthreads();
+#pragma unroll
+        for (int e = tid; e < 1024; e += CV_WAVES * 64) {
+            float s = 0.0f;
+#pragma unroll
+            for (int w = 0; w < CV_WAVES; ++w) s += red[k & 1][w][e];
+            part[k * 1024 + e] = s;
+        }
+    }
+    if (tid < HD) {
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < CV_WAVES; ++w) s += sums[w][tid];
+        part[CV_BLOCKS * 1024 + tid] = s;
+        part[CV_BLOCKS * 1024 + HD + tid] = pivot[tid];
+    }
+}
+
+// means of cos and sin over the positions (a workgroup per sixteen columns)
+__global__ __launch_bounds__(MN_THREADS) void rope_mean_kernel(CovArgs a) {
+    __shared__ float red[2][16][17];
+    const int c = threadIdx.x & 15, g = threadIdx.x >> 4, col = blockIdx.x * 16 + c;
+    float sc = 0.0f, ss = 0.0f;
+#pragma unroll 8
+    for (int x = g; x < a.positions; x += 16) { sc += a.cosine[(size_t)x * HD + col]; ss += a.sine[(size_t)x * HD + col]; }
+    red[0][g][c] = sc; red[1][g][c] = ss;
+    __syncthreads();
+    if (g < 2) {
+        float t = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) t += red[g][k][c];
+        a.rope[g * HD + col] = t / (float)a.positions;
+    }
+}
+
+// element (i, j) of the sum of q q^T: which block, and where D of a 32x32 matrix instruction keeps it (lane = 32 (x / 4 % 2) + column,
+// register 4 (x / 8) + x % 4 of row x)
+__device__ static inline int cov_at(int i, int j) {
+    int bi = i & 3, bj = j & 3, x = i >> 2, y = j >> 2;
+    if (bi > bj || (bi == bj && x > y)) { const int t = bi; bi = bj; bj = t; const int u = x; x = y; y = u; }
+    const int k = bi * 4 - bi * (bi - 1) / 2 + (bj - bi);
+    return k * 1024 + (4 * (x >> 3) + (x & 3)) * 64 + 32 * ((x >> 2) & 1) + y;
+}
+
+// A workgroup: rows i and i + 64 of four i < 64 of one head
+__global__ __launch_bounds__(256) void cov_final_kernel(CovArgs a) {
+    __shared__ double mean[HD];
+    __shared__ float c[8][HD];
+    __shared__ float cs[2][HD];
+    const int h = blockIdx.y, tid = threadIdx.x;
+    const float* part = a.part + (size_t)h * a.slices * CV_PART;
+    if (tid < HD) {
+        double s = 0.0;
+        for (int k = 0; k < a.slices; ++k) s += (double)part[(size_t)k * CV_PART + CV_BLOCKS * 1024 + tid];
+        mean[tid] = s / a.tokens;                            // relative to the pivot
+        cs[0][tid] = a.cosine ? a.rope[tid] : 1.0f;
+        cs[1][tid] = a.cosine ? a.rope[HD + tid] : 0.0f;
+    }
+    __syncthreads();
+    for (int e = tid; e < 8 * HD; e += 256) {
+        const int r = e >> 7, i = blockIdx.x * 4 + (r & 3) + 64 * (r >> 2), j = e & 127, at = cov_at(i, j);
+        double s = 0.0;
+        for (int k = 0; k < a.slices; ++k) s += (double)part[(size_t)k * CV_PART + at];
+        c[r][j] = (float)(s / a.tokens - mean[i] * mean[j]);
+    }
+    __syncthreads();
+    for (int e = tid; e < 8 * HD; e += 256) {
+        const int r = e >> 7, i = blockIdx.x * 4 + (r & 3) + 64 * (r >> 2), j = e & 127;
+        const float rj = j < 64 ? -1.0f : 1.0f, ri = i < 64 ? -1.0f : 1.0f;
+        // the map on the last axis of rows i and i +- 64, then across them
+        const float own = cs[0][j] * c[r][j] + cs[1][j] * (rj * c[r][j ^ 64]);
+        const float other = cs[0][j] * c[r ^ 4][j] + cs[1][j] * (rj * c[r ^ 4][j ^ 64]);
+        a.cov[((size_t)h * HD + i) * HD + j] = cs[0][i] * own + cs[1][i] * (ri * other);
+    }
+    if (blockIdx.x == 0 && tid < HD) {
+        const float* pivot = part + CV_BLOCKS * 1024 + HD;
+        const float m = (float)(mean[tid] + pivot[tid]), o = (float)(mean[tid ^ 64] + pivot[tid ^ 64]);
+        a.mu[(size_t)h * HD + tid] = cs[0][tid] * m + cs[1][tid] * (tid < 64 ? -o : o);
+    }
+}
+
+static int cov_slices(int tokens) { return std::max(8, (tokens + CV_WAVES * CV_TOKENS - 1) / (CV_WAVES * CV_TOKENS)); }
+
+extern "C" size_t odmkv_query_covariance_workspace_bytes(int heads, int tokens) {
+    return heads > 0 && tokens > 0 ? ((size_t)heads * cov_slices(tokens) * CV_PART + 2 * HD) * sizeof(float) : 0;
+}
+
+extern "C" int odmkv_query_covariance(const void* q, int dtype, int heads, int tokens, int64_t stride_h, int64_t stride_t,
+                                      const float* cosine, const float* sine, int positions, float* mu, float* cov,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+    ODMKV_CHECK_ARG(q && mu && cov && workspace, "query_covariance: null pointer");
+    ODMKV_CHECK_ARG(dtype == ODMKV_F16 || dtype == ODMKV_BF16, "query_covariance: 16-bit queries only");
+    ODMKV_CHECK_ARG(heads > 0 && heads <= 65535 && tokens > 0, "query_covariance: bad shape heads=%d tokens=%d", heads, tokens);
+    ODMKV_CHECK_ARG((cosine == nullptr) == (sine == nullptr) && (!cosine || positions > 0), "query_covariance: bad RoPE tables");
+    ODMKV_CHECK_ARG(((uintptr_t)q & 7) == 0 && stride_h % 4 == 0 && stride_t % 4 == 0, "query_covariance: rows must start on multiples of 8 bytes");
+    ODMKV_CHECK_ARG(workspace_bytes >= odmkv_query_covariance_workspace_bytes(heads, tokens), "query_covariance: workspace too small");
+    CovArgs a;
+    a.q = (const uint16_t*)q; a.sH = stride_h; a.sT = stride_t; a.tokens = tokens;
+    a.slices = cov_slices(tokens);
+    a.per_wave = ((tokens + a.slices * CV_WAVES - 1) / (a.slices * CV_WAVES) + 15) & ~15;
+    a.part = (float*)workspace; a.rope = a.part + (size_t)heads * a.slices * CV_PART;
+    a.cosine = cosine; a.sine = sine; a.positions = positions; a.mu = mu; a.cov = cov;
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == ODMKV_F16) hipLaunchKernelGGL(cov_part_kernel<ODMKV_F16>, dim3(a.slices, heads), dim3(CV_WAVES * 64), 0, st, a);
+    else hipLaunchKernelGGL(cov_part_kernel<ODMKV_BF16>, dim3(a.slices, heads), dim3(CV_WAVES * 64), 0, st, a);
+    ODMKV_CHECK_LAUNCH("cov_part_kernel");
+    if (cosine) {
+        hipLaunchKernelGGL(rope_mean_kernel, dim3(HD / 16), dim3(MN_THREADS), 0, st, a);
+        ODMKV_CHECK_LAUNCH("rope_mean_kernel");
+    }
+    hipLaunchKernelGGL(cov_final_kernel, dim3(16, heads), dim3(256), 0, st, a);
+    ODMKV_CHECK_LAUNCH("cov_final_kernel");
+    return 0;
+}
+
+// ------------------------------------------------------------------------------------------------
+// RoPE of a window's queries: q [heads, tokens, 128] with strides -> contiguous, q * cos + rotate_half(q) * sin with every
+// product and the sum rounded to the type (one launch for six)
+// ------------------------------------------------------------------------------------------------
+struct RotateArgs { const void* q; long long sH, sT; const void* cosine; const void* sine; int heads, tokens; void* out; };
+
+template <int DT>
+__global__ __launch_bounds__(256) void rotate_queries_kernel(RotateArgs a) {
+    typedef typename Elem<DT>::raw raw;
+    auto round_dt = [](float x) { return Elem<DT>::to_f32(Elem<DT>::from_f32(x)); };
+    const int i = blockIdx.x * 256 + threadIdx.x, col = i & 127, row = i >> 7;
+    if (row >= a.heads * a.tokens) return;
+    const int t = row % a.tokens;
+    const raw* src = (const raw*)a.q + (long long)(row / a.tokens) * a.sH + (long long)t * a.sT;
+    const float x = Elem<DT>::to_f32(src[col]), o = Elem<DT>::to_f32(src[col ^ 64]);
+    const float c = Elem<DT>::to_f32(((const raw*)a.cosine)[t * HD + col]), s = Elem<DT>::to_f32(((const raw*)a.sine)[t * HD + col]);
+    ((raw*)a.out)[i] = Elem<DT>::from_f32(round_dt(x * c) + round_dt((col < 64 ? -o : o) * s));
+}
+
+extern "C" int odmkv_rotate_queries(const void* q, int dtype, int heads, int tokens, int64_t stride_h, int64_t stride_t,
+                                    const void* cosine, const void* sine, void* out, void* stream) {
+    ODMKV_CHECK_ARG(q && cosine && sine && out, "rotate_queries: null pointer");
+    ODMKV_CHECK_ARG(dtype == ODMKV_F16 || dtype == ODMKV_BF16 || dtype == ODMKV_F32, "rotate_queries: bad dtype %d", dtype);
+    ODMKV_CHECK_ARG(heads > 0 && tokens > 0 && (long long)heads * tokens < (1ll << 24), "rotate_queries: bad shape heads=%d tokens=%d", heads, tokens);
+    const RotateArgs a = {q, (long long)stride_h, (long long)stride_t, cosine, sine, heads, tokens, out};
+    const dim3 grid((heads * tokens * HD + 255) / 256), block(256);
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == ODMKV_F16) hipLaunchKernelGGL(rotate_queries_kernel<ODMKV_F16>, grid, block, 0, st, a);
+    else if (dtype == ODMKV_BF16) hipLaunchKernelGGL(rotate_queries_kernel<ODMKV_BF16>, grid, block, 0, st, a);
+    else hipLaunchKernelGGL(rotate_queries_kernel<ODMKV_F32>, grid, block, 0, st, a);
+    ODMKV_CHECK_LAUNCH("rotate_queries_kernel");
+    return 0;
+}
+
+// ------------------------------------------------------------------------------------------------
+// scores in [0, 1] over the whole layer: (x - lo) / (hi - lo), one half everywhere where hi - lo < 1e-8; pad > 0: the rows get
+// that many columns of the largest score in front (the sinks).  The decision stays on the device (as tensor operations the
+// host waited for it), two launches for six.
+// ------------------------------------------------------------------------------------------------
+#define NRM_GROUPS 256
+struct NormalizeArgs { const float* x; long long rows, cols; int pad, scale; float* part; float* out; };
+
+// torch's amin / amax: a NaN anywhere is the result
+__device__ static inline float nan_min(float a, float b) { return a != a || b != b ? NAN : fminf(a, b); }
+__device__ static inline float nan_max(float a, float b) { return a != a || b != b ? NAN : fmaxf(a, b); }
+__device__ static inline void wg_minmax(float& lo, float& hi, float (*red)[2]) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { lo = nan_min(lo, __shfl_xor(lo, o, WAVE)); hi = nan_max(hi, __shfl_xor(hi, o, WAVE)); }
+    if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6][0] = lo; red[threadIdx.x >> 6][1] = hi; }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 4; ++w) { lo = nan_min(lo, red[w][0]); hi = nan_max(hi, red[w][1]); }
+}
+
+__global__ __launch_bounds__(256) void minmax_kernel(NormalizeArgs a) {
+    __shared__ float red[4][2];
+    const long long n = a.rows * a.cols, step = (long long)gridDim.x * 256;
+    float lo = INFINITY, hi = -INFINITY;
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += step) { const float v = a.x[i]; lo = nan_min(lo, v); hi = nan_max(hi, v); }
+    wg_minmax(lo, hi, red);
+    if (threadIdx.x == 0) { a.part[2 * blockIdx.x] = lo; a.part[2 * blockIdx.x + 1] = hi; }
+}
+
+__global__ __launch_bounds__(256) void normalize_kernel(NormalizeArgs a) {
+    __shared__ float red[4][2];
+    float lo = a.part[2 * threadIdx.x], hi = a.part[2 * threadIdx.x + 1];
+    wg_minmax(lo, hi, red);
+    const float span = hi - lo;
+    const bool flat = span < 1e-8f;
+    const long long cols = a.cols + a.pad, n = a.rows * cols, step = (long long)gridDim.x * 256;
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += step) {
+        const long long r = i / cols, c = i - r * cols;
+        const float v = c < a.pad ? hi : a.x[r * a.cols + c - a.pad];
+        a.out[i] = !a.scale ? v : flat ? 0.5f : (v - lo) / span;
+    }
+}
+
+extern "C" size_t odmkv_normalize_workspace_bytes(void) { return NRM_GROUPS * 2 * sizeof(float); }
+
+extern "C" int odmkv_normalize_scores(const float* scores, int64_t rows, int64_t cols, int pad, int scale, float* out,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+    ODMKV_CHECK_ARG(scores && out && workspace, "normalize_scores: null pointer");
+    ODMKV_CHECK_ARG(rows > 0 && cols > 0 && pad >= 0, "normalize_scores: bad shape");
+    ODMKV_CHECK_ARG(workspace_bytes >= odmkv_normalize_workspace_bytes(), "normalize_scores: workspace too small");
+    const NormalizeArgs a = {scores, (long long)rows, (long long)cols, pad, scale, (float*)workspace, out};
+    hipLaunchKernelGGL(minmax_kernel, dim3(NRM_GROUPS), dim3(256), 0, (hipStream_t)stream, a);
+    const long long n = (long long)rows * (cols + pad);
+    hipLaunchKernelGGL(normalize_kernel, dim3((unsigned)std::min<long long>((n + 1023) / 1024, 1024)), dim3(256), 0, (hipStream_t)stream, a);
+    ODMKV_CHECK_LAUNCH("normalize_kernel");
+    return 0;
+}

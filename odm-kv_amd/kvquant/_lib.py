@@ -88,6 +88,11 @@ def _load() -> C.CDLL:
         "odmkv_token_mean_workspace_bytes": (sz, [i32, i32, i32]),
         "odmkv_token_mean": (C.c_int, [vp, i32, i32, i32, i32, i64, i64, vp, vp, sz, vp]),
         "odmkv_average_rope": (C.c_int, [vp, vp, vp, i32, i32, i32, vp, vp]),
+        "odmkv_query_covariance_workspace_bytes": (sz, [i32, i32]),
+        "odmkv_query_covariance": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, vp, i32, vp, vp, vp, sz, vp]),
+        "odmkv_rotate_queries": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, vp, vp, vp]),
+        "odmkv_normalize_workspace_bytes": (sz, []),
+        "odmkv_normalize_scores": (C.c_int, [vp, i64, i64, i32, i32, vp, vp, sz, vp]),
         "odmkv_window_attention_workspace_bytes": (sz, [i32, i32, i32, i32]),
         "odmkv_window_attention": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, i32, i32, i32, i32, f32, vp, vp, sz, vp]),
         "odmkv_allocate_workspace_bytes": (sz, [i32, i32]),
@@ -150,6 +155,8 @@ def _load() -> C.CDLL:
 lib = _load()
 STEP_ENTRY = C.cast(lib.odmkv_decode_step, C.c_void_p).value      # what _native.Step calls
 EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "odmkv_score", "odmkv_score_model_dtype", "odmkv_score_expected", "odmkv_token_mean_workspace_bytes", "odmkv_token_mean", "odmkv_average_rope",
+           "odmkv_query_covariance_workspace_bytes", "odmkv_query_covariance", "odmkv_rotate_queries",
+           "odmkv_normalize_workspace_bytes", "odmkv_normalize_scores",
            "odmkv_window_attention_workspace_bytes", "odmkv_window_attention",
            "odmkv_allocate_workspace_bytes", "odmkv_allocate", "odmkv_level_counts",
            "odmkv_finish_levels_chunks", "odmkv_finish_levels", "odmkv_evicted_workspace_bytes", "odmkv_evicted_indices",

@@ -29,6 +29,17 @@ from .attention_utils import (  # noqa: F401  (re-exported under the names calle
 )
 
 
+def _scale_on_device(scores: torch.Tensor, pad: int, scale: bool) -> torch.Tensor:
+    """fp32 [rows, cols] on the GPU -> [rows, pad + cols] (odmkv_normalize_scores)."""
+    rows, cols = scores.shape
+    out = torch.empty(rows, pad + cols, dtype=torch.float32, device=scores.device)
+    ws_bytes = lib.odmkv_normalize_workspace_bytes()
+    ws = _lib.workspace(scores.device, ws_bytes, "normalize")
+    _lib.check(lib.odmkv_normalize_scores(scores.data_ptr(), rows, cols, pad, int(scale), out.data_ptr(), ws.data_ptr(), ws_bytes,
+                                          _lib.stream_ptr(scores.device)))
+    return out
+
+
 def _normalize_scores(raw: torch.Tensor, *, grain: str = "layer") -> torch.Tensor:
     """Min-max normalisation: "layer" over the whole tensor, "head" per row, "global" none."""
     if raw.numel() == 0 or grain == "global":
@@ -42,6 +53,8 @@ def _normalize_scores(raw: torch.Tensor, *, grain: str = "layer") -> torch.Tenso
         if dead.any():
             out[dead] = 0.5
         return out
+    if raw.is_cuda and raw.dtype == torch.float32 and raw.is_contiguous() and not (torch.is_grad_enabled() and raw.requires_grad):
+        return _scale_on_device(raw.reshape(1, -1), 0, True).reshape(raw.shape)
     lo, hi = raw.min(), raw.max()
     if (hi - lo) < 1e-8:
         return torch.full_like(raw, 0.5)
@@ -83,6 +96,31 @@ class _NormFallback(BaseScorer):
         return self._maybe_normalize(key.norm(dim=-1) + value.norm(dim=-1))
 
 
+def _query_covariance(module: nn.Module, q: torch.Tensor, q_len: int, n_future: int):
+    """(mu [1, Hq, d], cov [1, Hq, d, d]) in fp32 of 16-bit queries [1, Hq, t, d] through the averaged RoPE, by the library;
+    None where it does not cover the call (other types, several sequences, a RoPE of another width)."""
+    if (not q.is_cuda or q.dtype not in (torch.float16, torch.bfloat16) or q.shape[0] != 1 or q.shape[3] != _lib.HEAD_DIM
+            or q.stride(3) != 1 or q.stride(1) % 4 or q.stride(2) % 4 or q.data_ptr() % 8 or (torch.is_grad_enabled() and q.requires_grad)):
+        return None
+    _, n_q, t, D = q.shape
+    cos = sin = None
+    rotary_emb = getattr(module, "rotary_emb", None)
+    if rotary_emb is not None and n_future > 0:
+        pos = torch.arange(q_len, q_len + n_future, device=q.device).unsqueeze(0)
+        cos, sin = _aligned_rotary_outputs(rotary_emb, q.new_empty(1, dtype=torch.float32), pos)
+        if cos.shape != (1, n_future, D) or sin.shape != cos.shape:
+            return None
+        cos, sin = cos.contiguous(), sin.contiguous()
+    mu = torch.empty(1, n_q, D, dtype=torch.float32, device=q.device)
+    cov = torch.empty(1, n_q, D, D, dtype=torch.float32, device=q.device)
+    ws_bytes = lib.odmkv_query_covariance_workspace_bytes(n_q, t)
+    ws = _lib.workspace(q.device, ws_bytes, "covariance")
+    _lib.check(lib.odmkv_query_covariance(
+        q.data_ptr(), _lib.dtype_code(q), n_q, t, q.stride(1), q.stride(2), _lib.ptr(cos), _lib.ptr(sin), n_future, mu.data_ptr(),
+        cov.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_ptr(q.device)))
+    return mu, cov
+
+
 class ExpectedAttentionScorer(BaseScorer):
     """Expected attention of future queries (kvquant/scorer.py:154-282 of the reference):
 
@@ -111,7 +149,11 @@ class ExpectedAttentionScorer(BaseScorer):
             return _apply_avg_rope(module, mu, None, q_len, self.n_future_positions)
         # the covariance is accumulated in fp32 whatever the model's dtype: a 16-bit result of a sum
         # over tens of thousands of positions would overflow or lose the small eigen-directions
-        q = _get_query_states(module, query_input).float()            # [b, Hq, t, d]
+        q = _get_query_states(module, query_input)                    # [b, Hq, t, d]
+        got = _query_covariance(module, q, q_len, self.n_future_positions)
+        if got is not None:
+            return got
+        q = q.float()
         mu = q.mean(dim=2)
         centered = q - mu.unsqueeze(2)
         cov = torch.matmul(centered.transpose(-1, -2), centered) / query_input.shape[1]
@@ -269,6 +311,12 @@ class WindowRiskScorer(RiskScorer):
         if rotary_emb is not None:
             pos = torch.arange(q_len - w, q_len, device=q.device).unsqueeze(0)
             cos, sin = _aligned_rotary_outputs(rotary_emb, q, pos)
+            if (q.is_cuda and q.dtype in _lib._DT and q.shape[0] == 1 and q.shape[3] == _lib.HEAD_DIM and q.stride(3) == 1
+                    and cos.shape == sin.shape == (1, w, _lib.HEAD_DIM) and cos.is_contiguous() and sin.is_contiguous()):
+                out = torch.empty(q.shape[1:], dtype=q.dtype, device=q.device)
+                _lib.check(lib.odmkv_rotate_queries(q.data_ptr(), _lib.dtype_code(q), q.shape[1], w, q.stride(1), q.stride(2),
+                                                    cos.data_ptr(), sin.data_ptr(), out.data_ptr(), _lib.stream_ptr(q.device)))
+                return out
             q = _apply_rotary_pos_emb_q(q, cos, sin)
         return q[0]
 
@@ -287,5 +335,7 @@ class WindowRiskScorer(RiskScorer):
             return self._fallback.score_prefill(keys, values, layer_idx)
         p = _launch_window_attention(keys, queries, self.n_sink, T - w, D ** -0.5)
         core = _launch_score(keys[:, self.n_sink:], values[:, self.n_sink:], None, p, H, 0, self.epsilon)
+        if self.normalize_grain in ("layer", "global"):
+            return _scale_on_device(core, self.n_sink, self.normalize_grain == "layer")
         top = core.max().reshape(1, 1).expand(H, self.n_sink)
         return self._maybe_normalize(torch.cat([top, core], dim=1))

@@ -34,3 +34,56 @@ def test_averaged_rope(heads, positions, dtype):
     # the rounding points are the same; a mean of cos or sin may land one step of the type away, elements near zero by that noise
     step = {torch.float16: 2 ** -10, torch.bfloat16: 2 ** -7, torch.float32: 2e-6}[dtype]
     assert ((got.cpu() - want.float()).abs() <= 2 * step * (want.float().abs() + 0.1)).all()
+
+
+def _rotary(x, pos):
+    a = pos.cpu()[..., None].float() * (500000.0 ** (-torch.arange(0, 128, 2).float() / 128))
+    a = torch.cat((a, a), dim=-1)
+    return a.cos().to(x), a.sin().to(x)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,t,rope", [(1, 1, False), (3, 17, True), (8, 1023, True), (32, 4097, False), (2, 40001, True)])
+def test_query_covariance(heads, t, rope, dtype):
+    from types import SimpleNamespace
+    from kvquant.attention_utils import _apply_avg_rope
+    from kvquant.scorer import _query_covariance
+    g = torch.Generator(device="cuda").manual_seed(t)
+    q = torch.randn(1, t, heads, 128, generator=g, device="cuda")
+    q = (q * torch.rand(128, generator=g, device="cuda") + 4.0 * torch.randn(128, generator=g, device="cuda")).to(dtype).transpose(1, 2)
+    module = SimpleNamespace(rotary_emb=_rotary) if rope else SimpleNamespace()
+    mu, cov = _query_covariance(module, q, 77, 64)
+    d = q.double().cpu()
+    want_mu = d.mean(dim=2)
+    c = d - want_mu.unsqueeze(2)
+    want_mu, want_cov = _apply_avg_rope(module, want_mu, c.transpose(-1, -2).contiguous() @ c / t, 77, 64)
+    assert (mu.cpu().double() - want_mu).abs().max() <= 2e-6 * want_mu.abs().max()
+    # means of up to twelve times the deviation: they must not cost the covariance anything
+    assert (cov.cpu().double() - want_cov).abs().max() <= 3e-6 * (want_cov.abs().max() + 1e-3)
+    assert torch.equal(cov, cov.transpose(-1, -2)) or rope
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,w", [(1, 1), (28, 64), (5, 33)])
+def test_window_queries_rotated(heads, w, dtype):
+    from kvquant import _lib
+    from kvquant.attention_utils import _apply_rotary_pos_emb_q
+    g = torch.Generator(device="cuda").manual_seed(w)
+    q = torch.randn(1, w, heads, 128, generator=g, device="cuda").to(dtype).transpose(1, 2)
+    cos, sin = _rotary(q, torch.arange(900, 900 + w)[None])
+    out = torch.empty(heads, w, 128, dtype=dtype, device="cuda")
+    _lib.check(_lib.lib.odmkv_rotate_queries(q.data_ptr(), _lib.dtype_code(q), heads, w, q.stride(1), q.stride(2), cos.data_ptr(),
+                                             sin.data_ptr(), out.data_ptr(), _lib.stream_ptr(q.device)))
+    assert torch.equal(out, _apply_rotary_pos_emb_q(q, cos, sin)[0])
+
+
+@pytest.mark.parametrize("rows,cols,pad", [(1, 1, 0), (3, 255, 4), (8, 32764, 4), (2, 1000, 0)])
+def test_scores_normalised_on_the_device(rows, cols, pad):
+    from kvquant.scorer import _normalize_scores, _scale_on_device
+    x = torch.randn(rows, cols, generator=torch.Generator().manual_seed(cols))
+    for y in (x, torch.full_like(x, 3.0)):
+        padded = torch.cat([y.max().expand(rows, pad), y], dim=1)
+        assert torch.equal(_scale_on_device(y.cuda(), pad, False).cpu(), padded)
+        assert torch.allclose(_scale_on_device(y.cuda(), pad, True).cpu(), _normalize_scores(padded), rtol=1e-6, atol=1e-7)
+    x[0, cols // 2] = float("nan")
+    assert _scale_on_device(x.cuda(), pad, True).isnan().all()
