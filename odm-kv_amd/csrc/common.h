@@ -75,10 +75,7 @@ template <> struct Elem<ODMKV_BF16> {
     typedef uint16_t raw;
     __device__ static inline float to_f32(uint16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
     __device__ static inline uint16_t from_f32(float f) {
-        uint32_t u = __float_as_uint(f);
-        if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);   // quiet NaN
-        u += 0x7fffu + ((u >> 16) & 1u);                                            // round to nearest even
-        return (uint16_t)(u >> 16);
+        return __builtin_bit_cast(uint16_t, (__bf16)f);      // nearest even; one instruction on gfx950 (seven in integer arithmetic)
     }
 };
 template <> struct Elem<ODMKV_F32> {

@@ -313,7 +313,8 @@ __device__ static inline void convert_q8(const RawQ8& r, int dt, float* out) {
 __device__ static inline void load_q8(const void* q, int dt, size_t elem, float* out) { convert_q8(request_q8(q, dt, elem), dt, out); }
 
 __device__ static inline uint32_t bf16_pair(float a, float b) {
-    return (uint32_t)Elem<ODMKV_BF16>::from_f32(a) | ((uint32_t)Elem<ODMKV_BF16>::from_f32(b) << 16);
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, (b2){(__bf16)a, (__bf16)b});
 }
 __device__ static inline float bf16_rest(float a) { return a - Elem<ODMKV_BF16>::to_f32(Elem<ODMKV_BF16>::from_f32(a)); }
 
@@ -847,6 +848,55 @@ __device__ static inline void load_exact_unit(ExactUnit& t, const uint16_t* base
     for (int c = 0; c < 8; ++c) t.c[c] = stream_load(reinterpret_cast<const uint4*>(src + ((size_t)c * TILE + lane) * 16));
 }
 
+// The query rows of an exact item (lane (n, j): row n, dims 32j+8kb..+7 of step kb).  Every wavefront converts them for
+// itself, four wavefronts to a SIMD, so this is a microsecond of an item's time for every 200 instructions: a query in the
+// store's own type is taken as it is (fp16; bf16 where every value keeps its bits in fp16, that is all but values below 6e-5
+// or beyond 65504).  bf16 stores of 32k tokens: 18.1 -> 15 us per layer, with the conversions below in hardware.
+template <bool BF>
+__device__ static inline void exact_query(const DecodeArgs& a, int bq_first, int lane, uint4* qraw) {
+    const int n = lane & 15, j = lane >> 4, h = n >> 1, lo = n & 1;
+    const bool on = h < a.G && (BF || !lo);
+    if (a.q_dt == (BF ? ODMKV_BF16 : ODMKV_F16)) {
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        u16x2 worst = (u16x2){0, 0};
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            qraw[kb] = make_uint4(0u, 0u, 0u, 0u);
+            if (on) qraw[kb] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(a.q) + (size_t)(bq_first + h) * HD + 32 * j + 8 * kb);
+        }
+        if constexpr (!BF) return;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            const uint32_t w[4] = {qraw[kb].x, qraw[kb].y, qraw[kb].z, qraw[kb].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e)      // magnitude bits above those of 2^-14, the least normal fp16
+                worst = __builtin_elementwise_max(worst, __builtin_bit_cast(u16x2, w[e] & 0x7fff7fffu) - (u16x2){0x3880, 0x3880});
+        }
+        const bool plain = worst.x < 0x4780 - 0x3880 && worst.y < 0x4780 - 0x3880;      // (65536 = 0x4780)
+        if (__builtin_amdgcn_ballot_w64(on && !plain) == 0) {
+            if (lo) {
+#pragma unroll
+                for (int kb = 0; kb < 4; ++kb) qraw[kb] = make_uint4(0u, 0u, 0u, 0u);
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+        if (on) {
+            float qv[8];
+            load_q8(a.q, a.q_dt, (size_t)(bq_first + h) * HD + 32 * j + 8 * kb, qv);
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                if constexpr (BF) w[e >> 1] = lo ? bf16_pair(bf16_rest(qv[e]), bf16_rest(qv[e + 1])) : bf16_pair(qv[e], qv[e + 1]);
+                else w[e >> 1] = pack_h2(qv[e], qv[e + 1]);
+            }
+        }
+        qraw[kb] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
 // BF: the store keeps bf16 rows; they meet the query (bf16 high + low piece of q16, exact) and the
 // softmax weights (bf16 high + low piece) on the bf16 matrix instructions, products exact, sums fp32.
 template <bool BF, int NW>
@@ -857,23 +907,7 @@ __device__ static inline void run_exact_level(const DecodeArgs& a, int bh, int b
     // the query itself (no rotation): row 2h = q16 of head h, row 2h+1 = zero for fp16 rows; for bf16 rows the two
     // bf16 pieces of q16 (11 significant bits in two pieces of 8: exact)
     uint4 qraw[4];
-    {
-        const int h = n >> 1, lo = n & 1;
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            uint32_t w[4] = {0u, 0u, 0u, 0u};
-            if (h < a.G && (BF || !lo)) {
-                float qv[8];
-                load_q8(a.q, a.q_dt, (size_t)(bq_first + h) * HD + 32 * j + 8 * kb, qv);
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    if constexpr (BF) w[e >> 1] = lo ? bf16_pair(bf16_rest(qv[e]), bf16_rest(qv[e + 1])) : bf16_pair(qv[e], qv[e + 1]);
-                    else w[e >> 1] = pack_h2(qv[e], qv[e + 1]);
-                }
-            }
-            qraw[kb] = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-    }
+    exact_query<BF>(a, bq_first, lane, qraw);
     int stored = a.s.seg_count[4][bh];                     // exact segments grow between work-list rebuilds
     if (a.k_new) {
         // A decode step's new token goes behind the stored ones: the workgroup whose tiles hold its place writes it (its

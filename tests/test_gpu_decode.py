@@ -519,3 +519,20 @@ def test_large_group_with_more_items_than_compute_units(G):
     st._build_items(16, 1 << 30)                      # a few long items: every wave walks several tiles
     assert st._item_order is None
     assert rel_err(st.decode_attention(q.to(DEV)).cpu(), want) < ATTN_RTOL
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-6, 2e4, 0.0])
+@pytest.mark.parametrize("store,query", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16)])
+def test_queries_of_either_half_type_over_exact_rows(store, query, scale):
+    """A query in the store's type is taken as it is where fp16 keeps its bits: values below fp16's normal range, beyond its
+    range, and zeros take the conversion (saturated, as every query is)."""
+    g = torch.Generator().manual_seed(9)
+    k, v = ((torch.randn(1, 2, 150, 128, generator=g) * s).to(store) for s in (1.0 if scale <= 1 else 1e-4, 1.0))
+    q = torch.randn(1, 8, 128, generator=g)
+    q[:, :, ::3] *= scale
+    if scale > 1:
+        q[:, :, 3] = 9e4 if query == torch.bfloat16 else 6e4
+    q = q.to(query)
+    st, ref = _pair(k, v, torch.full((1, 2, 150), 16, dtype=torch.int32), dtype=store)
+    q16 = q.float().clamp(-65504.0, 65504.0).half().float()
+    assert rel_err(st.decode_attention(q.cuda()).float().cpu(), decode_attention_state(q16, ref)) < ATTN_RTOL
