@@ -85,6 +85,29 @@ int odmkv_token_mean(const void* x, int dtype, int batch, int rows, int cols, in
 int odmkv_average_rope(const void* mu, const void* cosine, const void* sine, int dtype, int heads, int positions,
                        float* out, void* stream);
 
+/* out [batch, rows] = x [batch, cols] . weight [rows, cols]^T + bias, weight and x of `dtype` (float16 / bfloat16), summed in
+ * fp32 and rounded to dtype; out_dtype: dtype, or float32 for the rounded values widened. */
+int odmkv_project_rows(const void* weight, int64_t ld, const void* bias, const void* x, int dtype, int batch, int rows,
+                       int cols, void* out, int out_dtype, void* stream);
+
+/* A prompt's risk scores from its hidden states (kvquant/scorer.py:285-325, 385-416), all sequences of the batch in one call:
+ * token mean behind the sinks, projection, averaged RoPE, odmkv_score_model_dtype.  hidden_states [B, T, hidden], weight
+ * [Hq * 128, hidden] and bias of `dtype` (float16 / bfloat16); cosine, sine [positions, 128] of dtype, or both NULL; K, V of
+ * kv_dtype with element strides; scores fp32 [B, Hkv, T]. */
+typedef struct odmkv_prompt {
+    const void* hidden_states; int64_t h_stride_b, h_stride_t;
+    const void* weight; int64_t ld_weight;
+    const void* bias;
+    const void* cosine; const void* sine;
+    const void* K; const void* V; int64_t stride_b, stride_h, stride_t;
+    float* scores;
+    void* workspace; size_t workspace_bytes;
+    int32_t dtype, kv_dtype, B, T, hidden, Hq, Hkv, positions, n_sink, round_dtype;
+    float eps;
+} odmkv_prompt_t;
+size_t odmkv_prompt_scores_workspace_bytes(int B, int T, int hidden, int Hq, int Hkv);
+int odmkv_prompt_scores(const odmkv_prompt_t* p, void* stream);
+
 /* Mean and covariance of the queries of every head, through the averaged RoPE (kvquant/scorer.py:204-257,
  * kvquant/attention_utils.py:57-115): q float16 / bfloat16, head h and token t at element h * stride_h + t * stride_t; cosine,
  * sine fp32 [positions, 128] or NULL (no RoPE); mu fp32 [heads, 128], cov fp32 [heads, 128, 128]. */
@@ -222,6 +245,11 @@ int odmkv_finish_levels(int32_t* bits, int rows, int T, int count_begin, int cou
 size_t odmkv_evicted_workspace_bytes(int B, int Hkv, int T);
 int odmkv_evicted_indices(const uint8_t* levels, int B, int Hkv, int T, int64_t stride, int64_t n, int64_t* out,
                           void* workspace, size_t workspace_bytes, void* stream);
+/* The same for `layers` level maps one behind the other ([layers, B*Hkv, stride]) in one pass: n host int64 [layers], out the
+ * layers' [3, n] lists one behind the other. */
+size_t odmkv_evicted_layers_workspace_bytes(int layers, int B, int Hkv, int T);
+int odmkv_evicted_indices_layers(const uint8_t* levels, int layers, int B, int Hkv, int T, int64_t stride, const int64_t* n,
+                                 int64_t* out, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Host arithmetic for callers that keep a store in ONE device allocation: where its 33 buffers lie, given the
  * segments' first tiles (seg_tile: host int32 [5][nseg + 1], the last entry of a row = tiles of the level).

@@ -85,13 +85,16 @@ extern "C" int odmkv_finish_levels(int32_t* bits, int rows, int T, int count_beg
 // ------------------------------------------------------------------------------------------------
 // evicted positions, in the order (sequence, head, token), as three int64 columns
 // ------------------------------------------------------------------------------------------------
+// (all layers of a prompt in one launch of each kernel: 16 us of latency once, not per layer)
+#define EV_LAYERS 64
 struct EvictedArgs {
     const uint8_t* levels;
     long long stride;
-    int B, H, T, chunks;
-    int32_t* chunk_count;                // [rows, chunks]
-    long long* out;                      // [3, n]
-    long long n;
+    int rows, H, T, chunks;              // rows: sequences x heads of a layer
+    int32_t* chunk_count;                // [layers, rows, chunks]
+    long long* out;                      // per layer [3, n], one behind the other
+    long long n[EV_LAYERS];
+    long long at[EV_LAYERS];             // element of out where the layer's list starts
 };
 
 __device__ static inline int sum256(int v, int* red) {                // over the workgroup, in every thread
@@ -105,8 +108,9 @@ __device__ static inline int sum256(int v, int* red) {                // over th
 
 __global__ __launch_bounds__(LV_THREADS) void evicted_count_kernel(EvictedArgs a) {
     __shared__ int red[4];
-    const int row = blockIdx.y, chunk = blockIdx.x;
-    const uint8_t* src = a.levels + (size_t)row * a.stride;
+    const int chunk = blockIdx.x;
+    const size_t row = (size_t)blockIdx.z * a.rows + blockIdx.y;
+    const uint8_t* src = a.levels + row * a.stride;
     int n = 0;
 #pragma unroll
     for (int u = 0; u < LV_CHUNK / LV_THREADS; ++u) {
@@ -114,18 +118,22 @@ __global__ __launch_bounds__(LV_THREADS) void evicted_count_kernel(EvictedArgs a
         n += t < a.T && src[t] == 0;
     }
     n = sum256(n, red);
-    if (threadIdx.x == 0) a.chunk_count[(size_t)row * a.chunks + chunk] = n;
+    if (threadIdx.x == 0) a.chunk_count[row * a.chunks + chunk] = n;
 }
 
 __global__ __launch_bounds__(LV_THREADS) void evicted_list_kernel(EvictedArgs a) {
     __shared__ int red[4];
-    const int row = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = blockIdx.y, layer = blockIdx.z, chunk = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int me = row * a.chunks + chunk;
+    const long long total = a.n[layer];
+    if (total == 0) return;                                            // (workgroup-uniform)
+    const int32_t* counted = a.chunk_count + (size_t)layer * a.rows * a.chunks;
+    long long* out = a.out + a.at[layer];
     int before = 0;
-    for (int i = tid; i < me; i += LV_THREADS) before += a.chunk_count[i];
+    for (int i = tid; i < me; i += LV_THREADS) before += counted[i];
     long long at = sum256(before, red);
     const int b = row / a.H, h = row % a.H;
-    const uint8_t* src = a.levels + (size_t)row * a.stride;
+    const uint8_t* src = a.levels + ((size_t)layer * a.rows + row) * a.stride;
     for (int u = 0; u < LV_CHUNK / LV_THREADS; ++u) {
         const int t = chunk * LV_CHUNK + u * LV_THREADS + tid;
         const bool hit = t < a.T && src[t] == 0;
@@ -135,30 +143,44 @@ __global__ __launch_bounds__(LV_THREADS) void evicted_list_kernel(EvictedArgs a)
         __syncthreads();
         int off = __popcll(m & ((1ull << lane) - 1ull));
         for (int w = 0; w < wave; ++w) off += red[w];
-        if (hit && at + off < a.n) {
-            a.out[at + off] = b;
-            a.out[a.n + at + off] = h;
-            a.out[2 * a.n + at + off] = t;
+        if (hit && at + off < total) {
+            out[at + off] = b;
+            out[total + at + off] = h;
+            out[2 * total + at + off] = t;
         }
         at += red[0] + red[1] + red[2] + red[3];
     }
 }
 
-extern "C" size_t odmkv_evicted_workspace_bytes(int B, int Hkv, int T) {
-    return B > 0 && Hkv > 0 && T > 0 ? (size_t)B * Hkv * level_chunks(T) * sizeof(int32_t) : 0;
+extern "C" size_t odmkv_evicted_layers_workspace_bytes(int layers, int B, int Hkv, int T) {
+    return layers > 0 && B > 0 && Hkv > 0 && T > 0 ? (size_t)std::min(layers, EV_LAYERS) * B * Hkv * level_chunks(T) * sizeof(int32_t) : 0;
 }
+
+extern "C" int odmkv_evicted_indices_layers(const uint8_t* levels, int layers, int B, int Hkv, int T, int64_t stride, const int64_t* n,
+                                     int64_t* out, void* workspace, size_t workspace_bytes, void* stream) {
+    ODMKV_CHECK_ARG(levels && n && out && workspace, "evicted_indices: null pointer");
+    ODMKV_CHECK_ARG(layers > 0 && B > 0 && Hkv > 0 && T > 0 && (long long)B * Hkv <= 65535 && stride >= T,
+                    "evicted_indices: bad shape layers=%d B=%d Hkv=%d T=%d", layers, B, Hkv, T);
+    for (int l = 0; l < layers; ++l)
+        ODMKV_CHECK_ARG(n[l] >= 0 && n[l] <= (int64_t)B * Hkv * T, "evicted_indices: layer %d cannot hold %lld evicted tokens", l, (long long)n[l]);
+    ODMKV_CHECK_ARG(workspace_bytes >= odmkv_evicted_layers_workspace_bytes(layers, B, Hkv, T), "evicted_indices: workspace too small");
+    long long at = 0;
+    for (int l0 = 0; l0 < layers; l0 += EV_LAYERS) {
+        const int m = std::min(layers - l0, EV_LAYERS);
+        EvictedArgs a = {levels + (size_t)l0 * B * Hkv * stride, (long long)stride, B * Hkv, Hkv, T, level_chunks(T), (int32_t*)workspace, (long long*)out, {}, {}};
+        for (int l = 0; l < m; ++l) { a.n[l] = n[l0 + l]; a.at[l] = at; at += 3 * n[l0 + l]; }
+        const dim3 grid(a.chunks, a.rows, m);
+        hipLaunchKernelGGL(evicted_count_kernel, grid, dim3(LV_THREADS), 0, (hipStream_t)stream, a);
+        ODMKV_CHECK_LAUNCH("evicted_count_kernel");
+        hipLaunchKernelGGL(evicted_list_kernel, grid, dim3(LV_THREADS), 0, (hipStream_t)stream, a);
+        ODMKV_CHECK_LAUNCH("evicted_list_kernel");
+    }
+    return 0;
+}
+
+extern "C" size_t odmkv_evicted_workspace_bytes(int B, int Hkv, int T) { return odmkv_evicted_layers_workspace_bytes(1, B, Hkv, T); }
 
 extern "C" int odmkv_evicted_indices(const uint8_t* levels, int B, int Hkv, int T, int64_t stride, int64_t n, int64_t* out,
                                      void* workspace, size_t workspace_bytes, void* stream) {
-    ODMKV_CHECK_ARG(levels && out && workspace, "evicted_indices: null pointer");
-    ODMKV_CHECK_ARG(B > 0 && Hkv > 0 && T > 0 && (long long)B * Hkv <= 65535 && stride >= T && n > 0 && n <= (int64_t)B * Hkv * T,
-                    "evicted_indices: bad shape B=%d Hkv=%d T=%d n=%lld", B, Hkv, T, (long long)n);
-    ODMKV_CHECK_ARG(workspace_bytes >= odmkv_evicted_workspace_bytes(B, Hkv, T), "evicted_indices: workspace too small");
-    EvictedArgs a = {levels, (long long)stride, B, Hkv, T, level_chunks(T), (int32_t*)workspace, (long long*)out, (long long)n};
-    const dim3 grid(a.chunks, B * Hkv);
-    hipLaunchKernelGGL(evicted_count_kernel, grid, dim3(LV_THREADS), 0, (hipStream_t)stream, a);
-    ODMKV_CHECK_LAUNCH("evicted_count_kernel");
-    hipLaunchKernelGGL(evicted_list_kernel, grid, dim3(LV_THREADS), 0, (hipStream_t)stream, a);
-    ODMKV_CHECK_LAUNCH("evicted_list_kernel");
-    return 0;
+    return odmkv_evicted_indices_layers(levels, 1, B, Hkv, T, stride, &n, out, workspace, workspace_bytes, stream);
 }

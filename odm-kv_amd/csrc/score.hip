@@ -16,6 +16,7 @@ struct ScoreArgs {
     const void* V;
     int64_t sH, sT;
     int Hkv, Hq, G, Gl, T, Tc, n_sink, nchunks;   // Gl: heads the logits pass covers (0 when p is given)
+    int Hlayer;           // kv-heads of a sequence (Hkv counts those of all sequences of the call)
     float eps;
     const float* mu;      // [Hq, 128]
     const float* attn;    // [Hkv, T] or null
@@ -579,8 +580,9 @@ __global__ __launch_bounds__(64) void score_pad_kernel(ScoreArgs a) {
     const int h = blockIdx.x, i = threadIdx.x;
     const unsigned int* part = reinterpret_cast<const unsigned int*>(a.psum);
     unsigned int mx = 0u;
+    const int first = (h / a.Hlayer) * a.Hlayer * a.nchunks;          // the heads of this head's own sequence
 #pragma unroll 8
-    for (int c = i; c < a.Hkv * a.nchunks; c += WAVE) mx = max(mx, part[c]);
+    for (int c = i; c < a.Hlayer * a.nchunks; c += WAVE) mx = max(mx, part[first + c]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned int)__shfl_xor((int)mx, o, WAVE));
     if (i < a.n_sink) a.scores[(size_t)h * a.T + i] = __uint_as_float(mx);
@@ -1008,11 +1010,10 @@ extern "C" int odmkv_score(const void* K, const void* V, int dtype, int Hkv, int
                                    scores, workspace, workspace_bytes, stream);
 }
 
-extern "C" int odmkv_score_model_dtype(const void* K, const void* V, int dtype, int Hkv, int T,
-                                       int64_t stride_h, int64_t stride_t,
-                                       const float* mu, int Hq, const float* attn, int n_sink, float eps,
-                                       int round_dtype, float* scores, void* workspace, size_t workspace_bytes,
-                                       void* stream) {
+// Hkv kv-heads (of Hkv / Hlayer sequences that lie one behind the other), scored together
+static int score_heads(const void* K, const void* V, int dtype, int Hkv, int Hlayer, int T, int64_t stride_h, int64_t stride_t,
+                       const float* mu, int Hq, const float* attn, int n_sink, float eps, int round_dtype, float* scores,
+                       void* workspace, size_t workspace_bytes, void* stream) {
     ODMKV_CHECK_ARG(K && V && scores && workspace, "score: null pointer");
     ODMKV_CHECK_ARG(round_dtype == -1 || round_dtype == ODMKV_F16 || round_dtype == ODMKV_BF16,
                     "score: rounding dtype %d (-1, fp16 or bf16)", round_dtype);
@@ -1032,7 +1033,7 @@ extern "C" int odmkv_score_model_dtype(const void* K, const void* V, int dtype, 
     char* ws = (char*)workspace;
     ScoreArgs a;
     a.K = K; a.V = V; a.sH = stride_h; a.sT = stride_t;
-    a.Hkv = Hkv; a.Hq = Hq; a.G = Hq / Hkv; a.Gl = attn ? 0 : Hq / Hkv; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
+    a.Hlayer = Hlayer; a.Hkv = Hkv; a.Hq = Hq; a.G = Hq / Hkv; a.Gl = attn ? 0 : Hq / Hkv; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
     a.nchunks = n_chunks(a.Tc); a.eps = eps; a.mu = mu; a.attn = attn; a.scores = scores;
     a.cov = nullptr; a.use_vnorm = 0; a.ea_cpw = 1; a.nstat = a.nchunks; a.round_dt = round_dtype;
     a.logits = (float*)(ws + L.logits); a.kn2 = (float*)(ws + L.kn2); a.p = (float*)(ws + L.p);
@@ -1042,6 +1043,67 @@ extern "C" int odmkv_score_model_dtype(const void* K, const void* V, int dtype, 
     if (dtype == ODMKV_F16) return run_score<ODMKV_F16>(a, st);
     if (dtype == ODMKV_BF16) return run_score<ODMKV_BF16>(a, st);
     return run_score<ODMKV_F32>(a, st);
+}
+
+extern "C" int odmkv_score_model_dtype(const void* K, const void* V, int dtype, int Hkv, int T,
+                                       int64_t stride_h, int64_t stride_t,
+                                       const float* mu, int Hq, const float* attn, int n_sink, float eps,
+                                       int round_dtype, float* scores, void* workspace, size_t workspace_bytes,
+                                       void* stream) {
+    return score_heads(K, V, dtype, Hkv, Hkv, T, stride_h, stride_t, mu, Hq, attn, n_sink, eps, round_dtype, scores, workspace,
+                       workspace_bytes, stream);
+}
+
+// A prompt's risk scores from its hidden states in one call: mean over the tokens, projection, averaged RoPE, scores of all
+// sequences.  From Python these were twelve torch operations and four library calls per layer and sequence, 150 us of the
+// host's time each; here it is 20 us a layer.
+struct PromptLayout { size_t mean, mean_ws, q, mu, score, total; };
+static PromptLayout prompt_layout(int B, int T, int hidden, int Hq, int Hkv) {
+    PromptLayout L;
+    size_t off = 0;
+    auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
+    L.mean = take((size_t)B * hidden * 2);
+    L.mean_ws = take(odmkv_token_mean_workspace_bytes(B, T, hidden));
+    L.q = take((size_t)B * Hq * HD * 2);
+    L.mu = take((size_t)B * Hq * HD * 4);
+    L.score = take(odmkv_score_workspace_bytes(B * Hkv, B * Hq, T));
+    L.total = off;
+    return L;
+}
+
+extern "C" size_t odmkv_prompt_scores_workspace_bytes(int B, int T, int hidden, int Hq, int Hkv) {
+    return B > 0 && T > 0 && hidden > 0 && Hq > 0 && Hkv > 0 ? prompt_layout(B, T, hidden, Hq, Hkv).total : 0;
+}
+
+extern "C" int odmkv_prompt_scores(const odmkv_prompt_t* p, void* stream) {
+    ODMKV_CHECK_ARG(p != nullptr, "prompt_scores: null argument block");
+    ODMKV_CHECK_ARG(p->hidden_states && p->weight && p->K && p->V && p->scores && p->workspace && (p->cosine != nullptr) == (p->sine != nullptr),
+                    "prompt_scores: null pointer");
+    ODMKV_CHECK_ARG(p->dtype == ODMKV_F16 || p->dtype == ODMKV_BF16, "prompt_scores: bad dtype %d", p->dtype);
+    ODMKV_CHECK_ARG(p->B > 0 && p->T > p->n_sink && p->n_sink >= 0 && p->hidden > 0 && p->Hkv > 0 && p->Hq > 0 && p->Hq % p->Hkv == 0
+                    && (!p->cosine || p->positions > 0), "prompt_scores: bad shape");
+    ODMKV_CHECK_ARG(p->workspace_bytes >= odmkv_prompt_scores_workspace_bytes(p->B, p->T, p->hidden, p->Hq, p->Hkv), "prompt_scores: workspace too small");
+    const PromptLayout L = prompt_layout(p->B, p->T, p->hidden, p->Hq, p->Hkv);
+    char* ws = (char*)p->workspace;
+    const char* h0 = (const char*)p->hidden_states + (size_t)p->n_sink * p->h_stride_t * 2;
+    if (int rc = odmkv_token_mean(h0, p->dtype, p->B, p->T - p->n_sink, p->hidden, p->h_stride_b, p->h_stride_t, ws + L.mean,
+                                  ws + L.mean_ws, L.q - L.mean_ws, stream)) return rc;
+    float* mu = (float*)(ws + L.mu);
+    if (int rc = odmkv_project_rows(p->weight, p->ld_weight, p->bias, ws + L.mean, p->dtype, p->B, p->Hq * HD, p->hidden,
+                                    p->cosine ? (void*)(ws + L.q) : (void*)mu, p->cosine ? p->dtype : ODMKV_F32, stream)) return rc;
+    if (p->cosine)
+        if (int rc = odmkv_average_rope(ws + L.q, p->cosine, p->sine, p->dtype, p->B * p->Hq, p->positions, mu, stream)) return rc;
+    if (p->B == 1 || p->stride_b == p->Hkv * p->stride_h)
+        return score_heads(p->K, p->V, p->kv_dtype, p->B * p->Hkv, p->Hkv, p->T, p->stride_h, p->stride_t, mu, p->B * p->Hq, nullptr,
+                           p->n_sink, p->eps, p->round_dtype, p->scores, ws + L.score, p->workspace_bytes - L.score, stream);
+    const size_t elem = p->kv_dtype == ODMKV_F32 ? 4 : 2;
+    for (int b = 0; b < p->B; ++b) {
+        const size_t at = (size_t)b * p->stride_b * elem;
+        if (int rc = score_heads((const char*)p->K + at, (const char*)p->V + at, p->kv_dtype, p->Hkv, p->Hkv, p->T, p->stride_h, p->stride_t,
+                                 mu + (size_t)b * p->Hq * HD, p->Hq, nullptr, p->n_sink, p->eps, p->round_dtype,
+                                 p->scores + (size_t)b * p->Hkv * p->T, ws + L.score, p->workspace_bytes - L.score, stream)) return rc;
+    }
+    return 0;
 }
 
 template <int DT>
@@ -1116,7 +1178,7 @@ extern "C" int odmkv_score_expected(const void* K, const void* V, int dtype, int
     char* ws = (char*)workspace;
     ScoreArgs a;
     a.K = K; a.V = V; a.sH = stride_h; a.sT = stride_t;
-    a.Hkv = Hkv; a.Hq = Hq; a.G = Hq / Hkv; a.Gl = a.G; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
+    a.Hlayer = Hkv; a.Hkv = Hkv; a.Hq = Hq; a.G = Hq / Hkv; a.Gl = a.G; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
     a.nchunks = n_chunks(a.Tc); a.eps = eps; a.mu = mu; a.attn = nullptr; a.scores = scores;
     a.cov = cov; a.use_vnorm = use_vnorm ? 1 : 0; a.ea_cpw = 1; a.nstat = a.nchunks; a.round_dt = -1;
     a.logits = (float*)(ws + L.logits); a.kn2 = (float*)(ws + L.kn2); a.p = (float*)(ws + L.p);

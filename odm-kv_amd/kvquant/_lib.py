@@ -71,6 +71,16 @@ class Step(C.Structure):
     ]
 
 
+class Prompt(C.Structure):
+    """struct odmkv_prompt of include/odmkv.h."""
+    _fields_ = ([("hidden_states", C.c_void_p), ("h_stride_b", C.c_int64), ("h_stride_t", C.c_int64), ("weight", C.c_void_p),
+                 ("ld_weight", C.c_int64), ("bias", C.c_void_p), ("cosine", C.c_void_p), ("sine", C.c_void_p), ("K", C.c_void_p),
+                 ("V", C.c_void_p), ("stride_b", C.c_int64), ("stride_h", C.c_int64), ("stride_t", C.c_int64), ("scores", C.c_void_p),
+                 ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t)]
+                + [(n, C.c_int32) for n in ("dtype", "kv_dtype", "B", "T", "hidden", "Hq", "Hkv", "positions", "n_sink", "round_dtype")]
+                + [("eps", C.c_float)])
+
+
 def _load() -> C.CDLL:
     if not os.path.exists(LIB_PATH):
         raise ImportError(
@@ -88,6 +98,9 @@ def _load() -> C.CDLL:
         "odmkv_token_mean_workspace_bytes": (sz, [i32, i32, i32]),
         "odmkv_token_mean": (C.c_int, [vp, i32, i32, i32, i32, i64, i64, vp, vp, sz, vp]),
         "odmkv_average_rope": (C.c_int, [vp, vp, vp, i32, i32, i32, vp, vp]),
+        "odmkv_project_rows": (C.c_int, [vp, i64, vp, vp, i32, i32, i32, i32, vp, i32, vp]),
+        "odmkv_prompt_scores_workspace_bytes": (sz, [i32, i32, i32, i32, i32]),
+        "odmkv_prompt_scores": (C.c_int, [C.POINTER(Prompt), vp]),
         "odmkv_query_covariance_workspace_bytes": (sz, [i32, i32]),
         "odmkv_query_covariance": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, vp, i32, vp, vp, vp, sz, vp]),
         "odmkv_rotate_queries": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, vp, vp, vp]),
@@ -102,7 +115,9 @@ def _load() -> C.CDLL:
         "odmkv_finish_levels_chunks": (C.c_int, [i64]),
         "odmkv_finish_levels": (C.c_int, [vp, i32, i32, i32, i32, i32, vp, i64, vp, vp]),
         "odmkv_evicted_workspace_bytes": (sz, [i32, i32, i32]),
+        "odmkv_evicted_layers_workspace_bytes": (sz, [i32, i32, i32, i32]),
         "odmkv_evicted_indices": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, vp, sz, vp]),
+        "odmkv_evicted_indices_layers": (C.c_int, [vp, i32, i32, i32, i32, i64, vp, vp, vp, sz, vp]),
         "odmkv_store_init": (C.c_int, [vp, vp, i32, i32, vp, C.c_uint64, C.c_uint64, C.c_uint64, vp]),
         "odmkv_store_gather": (C.c_int, [C.POINTER(Packed), C.POINTER(Packed), vp]),
         "odmkv_quant_pack_staged": (C.c_int, [vp, vp, i32, i32, i32, i32, i64, i64, i64, vp, i32, vp, vp, vp,
@@ -155,11 +170,11 @@ def _load() -> C.CDLL:
 lib = _load()
 STEP_ENTRY = C.cast(lib.odmkv_decode_step, C.c_void_p).value      # what _native.Step calls
 EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "odmkv_score", "odmkv_score_model_dtype", "odmkv_score_expected", "odmkv_token_mean_workspace_bytes", "odmkv_token_mean", "odmkv_average_rope",
-           "odmkv_query_covariance_workspace_bytes", "odmkv_query_covariance", "odmkv_rotate_queries",
+           "odmkv_project_rows", "odmkv_prompt_scores_workspace_bytes", "odmkv_prompt_scores", "odmkv_query_covariance_workspace_bytes", "odmkv_query_covariance", "odmkv_rotate_queries",
            "odmkv_normalize_workspace_bytes", "odmkv_normalize_scores",
            "odmkv_window_attention_workspace_bytes", "odmkv_window_attention",
            "odmkv_allocate_workspace_bytes", "odmkv_allocate", "odmkv_level_counts",
-           "odmkv_finish_levels_chunks", "odmkv_finish_levels", "odmkv_evicted_workspace_bytes", "odmkv_evicted_indices",
+           "odmkv_finish_levels_chunks", "odmkv_finish_levels", "odmkv_evicted_workspace_bytes", "odmkv_evicted_indices", "odmkv_evicted_layers_workspace_bytes", "odmkv_evicted_indices_layers",
            "odmkv_store_init", "odmkv_store_gather", "odmkv_quant_pack_staged", "odmkv_store_layout", "odmkv_store_bind", "odmkv_pack_workspace_bytes", "odmkv_pack_count_chunks", "odmkv_store_finish_staged", "odmkv_quant_pack", "odmkv_quantize_rows",
            "odmkv_dequantize_rows", "odmkv_quantize_rows_packed", "odmkv_dequantize_rows_packed",
            "odmkv_round_trip_workspace_bytes", "odmkv_round_trip_rows", "odmkv_lloyd_max", "odmkv_dequant", "odmkv_dequant_from", "odmkv_append_exact", "odmkv_append_exact_rows", "odmkv_drop_exact_tail", "odmkv_truncate",
@@ -215,7 +230,7 @@ _ws_cache: dict[tuple, torch.Tensor] = {}
 
 def workspace(device, nbytes: int, tag: str = "") -> torch.Tensor:
     """A reusable scratch buffer per (device, stream, tag); grown, never shrunk."""
-    key = (str(device), stream_ptr(device), tag)
+    key = (device, stream_ptr(device), tag)
     buf = _ws_cache.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)

@@ -29,7 +29,7 @@ from kvquant.attention_patch import fused_decode_enabled
 from kvquant.attention_utils import _aligned_rotary_outputs, _apply_rotary_pos_emb_q, _get_query_states
 from kvquant.hf_cache import PackedCacheLayer
 from kvquant.press import TurboQuantPerTokenPress, full_attention_modules
-from kvquant.tq_adaptive_backend import TurboQuantAdaptiveKVCacheState, release_staging, reserve_state_memory
+from kvquant.tq_adaptive_backend import TurboQuantAdaptiveKVCacheState, evicted_indices, release_staging, reserve_state_memory
 
 
 def _levels_by_rank(levels, ratios, n: int):
@@ -221,36 +221,52 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
             raise NotImplementedError("outlier-channel separation is not built (n_outlier_channels must be 0)")
         plan = []                   # per layer: index, bits (int32), level map, counts (page-locked)
         arrived = {}
+        groups = []                 # layers whose bits lie one behind the other share a launch: [device, T, tail, bits of each]
+        order = []
         for layer_idx, bits in self._allocate_bits_for_prefill().items():
             keys, _ = self._get_cache_tensors(cache, layer_idx)
-            dev = keys.device
+            dev, T = keys.device, bits.shape[2]
             bits = bits.to(dtype=torch.int32, device=dev).contiguous()
-            B, H, T = bits.shape
+            tail = 0 if layer_idx < self.initial_layers_fp16 else T - min(max(self.buffer_size, 0), T)
+            last = groups[-1] if groups else None
+            if not (last and last[:3] == [dev, T, tail] and last[3][0].shape == bits.shape
+                    and bits.data_ptr() == last[3][0].data_ptr() + 4 * len(last[3]) * bits.numel()):
+                groups.append([dev, T, tail, []])
+            groups[-1][3].append(bits)
+            order.append(layer_idx)
+        evicted = []                # per group: level maps of its layers
+        for dev, T, tail, members in groups:
             # one pass over the levels: bulk shares counted, the window (or the whole layer) set to 16, the level map
             # written; the counts go straight to page-locked memory, and all layers share the one wait below
+            n, (B, H, _) = len(members), members[0].shape
             room = (T + 2 * self.buffer_size + 255) & ~255
-            levels = torch.empty((B, H, room), dtype=torch.uint8, device=dev)
+            levels = torch.empty((n, B, H, room), dtype=torch.uint8, device=dev)
             chunks = _lib.lib.odmkv_finish_levels_chunks(room)
-            counts = torch.empty((B * H, chunks, 2, 6), dtype=torch.int32, pin_memory=True)
+            counts = torch.empty((n, B * H, chunks, 2, 6), dtype=torch.int32, pin_memory=True)
             start, end = self._bulk(T)
-            tail = 0 if layer_idx < self.initial_layers_fp16 else T - min(max(self.buffer_size, 0), T)
             with torch.cuda.device(dev):
-                _lib.check(_lib.lib.odmkv_finish_levels(bits.data_ptr(), B * H, T, start, end, tail, levels.data_ptr(), room,
+                _lib.check(_lib.lib.odmkv_finish_levels(members[0].data_ptr(), n * B * H, T, start, end, tail, levels.data_ptr(), room,
                                                         counts.data_ptr(), _lib.stream_ptr(dev)))
                 ev = arrived.setdefault(dev, torch.cuda.Event())
                 ev.record(torch.cuda.current_stream(dev))
-            plan.append((layer_idx, bits, levels, counts))
+            plan.extend(zip(order[len(plan):], members, levels, counts))
+            evicted.append((levels, T))
         for layer_idx, *_ in plan:                                # (the host's part while the counts are on their way)
             self._get_or_create_state(layer_idx, self._get_cache_tensors(cache, layer_idx)[0])
         for ev in arrived.values():
             ev.synchronize()
-        for layer_idx, bits, levels, counts in plan:
+        masked, at = [], 0
+        totals = [counts.numpy().sum(axis=1).swapaxes(0, 1) for *_, counts in plan]      # (bulk, stored) of every layer
+        for levels, T in evicted:
+            masked += evicted_indices(levels, T, [int(stored[:, 0].sum()) for _, stored in totals[at:at + len(levels)]])
+            at += len(levels)
+        for (layer_idx, bits, levels, counts), (bulk, stored), gone in zip(plan, totals, masked):
             keys, values = self._get_cache_tensors(cache, layer_idx)
-            bulk, stored = counts.sum(dim=1).numpy().swapaxes(0, 1)
             wanted = sorted(set(int(b) for b in self.bit_levels) | {16})
             self._store_observed_ratios(layer_idx, bits.shape[1], wanted, bulk[:, [_lib.LEVEL_ORDER.index(b) for b in wanted]])
             state = self._get_or_create_state(layer_idx, keys)
             state.prefill(keys, values, bits, _known_counts=stored, _levels=levels)
+            state.adopt_masked(gone)
             module = self._layer_modules.get(layer_idx)
             if module is not None:
                 if self.release_dense_cache and layer_idx >= self.initial_layers_fp16:

@@ -10,6 +10,7 @@ with p the expected attention of the mean (RoPE-averaged) query, averaged over t
 """
 from __future__ import annotations
 
+import ctypes as C
 from abc import ABC, abstractmethod
 from typing import Optional
 
@@ -94,6 +95,21 @@ class _NormFallback(BaseScorer):
 
     def score_decode(self, key, value, layer_idx, *, module=None, hidden_states=None):
         return self._maybe_normalize(key.norm(dim=-1) + value.norm(dim=-1))
+
+
+def _plain_projection(module: nn.Module):
+    """(weight, bias) of a query projection that is a 16-bit nn.Linear and nothing more (no q_norm behind it, no hooks, no
+    replaced forward), or (None, None)."""
+    proj = getattr(module, "q_proj", None)
+    if (type(proj) is not nn.Linear or proj._forward_hooks or proj._forward_pre_hooks or "forward" in proj.__dict__
+            or hasattr(module, "qkv_proj") or hasattr(module, "q_norm")):
+        return None, None
+    w, b = proj.weight, proj.bias
+    if (type(w) is not nn.Parameter or w.dtype not in (torch.float16, torch.bfloat16) or not w.is_cuda or w.stride(1) != 1
+            or w.stride(0) % 8 or w.data_ptr() % 16 or (b is not None and (b.dtype != w.dtype or b.stride(0) != 1))
+            or (torch.is_grad_enabled() and w.requires_grad)):
+        return None, None
+    return w, b
 
 
 def _query_covariance(module: nn.Module, q: torch.Tensor, q_len: int, n_future: int):
@@ -260,6 +276,62 @@ class RiskScorer(ExpectedAttentionScorer):
         rd = keys.dtype if self.model_dtype_rounding and keys.dtype in (torch.float16, torch.bfloat16) else None
         scores = _launch_score(keys, values, mu[0], None, n_q, self.n_sink, self.epsilon, round_dtype=rd)
         return self._maybe_normalize(scores)
+
+    def score_prompt(self, keys, values, layer_idx, *, module, hidden_states, out=None, rope_tables=None):
+        """``score_prefill`` of all sequences of a layer, keys / values [B, H, T, d] and hidden_states [B, T, hidden], as one
+        library call: fp32 [B, H, T] (written to `out` if given), or None where the call is not one it covers (the caller
+        then goes sequence by sequence).  rope_tables: a dict in which the layers of one forward share the RoPE tables of
+        the future positions (they ask the same rotary module for the same positions)."""
+        cls = type(self)
+        if (cls.score_prefill is not RiskScorer.score_prefill or cls._query_statistics is not ExpectedAttentionScorer._query_statistics
+                or cls._maybe_normalize is not BaseScorer._maybe_normalize or self.normalize_grain != "global"
+                or not self.__dict__.keys().isdisjoint(("score_prefill", "_query_statistics", "_maybe_normalize"))):
+            return None
+        weight, bias = _plain_projection(module)
+        if weight is None or hidden_states.dim() != 3 or hidden_states.dtype != weight.dtype or not hidden_states.is_cuda:
+            return None
+        B, H, T, D = keys.shape
+        hidden = hidden_states.shape[2]
+        dt, kt = _lib._DT[weight.dtype], _lib._DT.get(keys.dtype)
+        n_q = weight.shape[0] // D
+        if (D != _lib.HEAD_DIM or kt is None or T <= self.n_sink or hidden_states.shape[:2] != (B, T) or weight.shape[1] != hidden
+                or hidden % 8 or weight.shape[0] != n_q * D or n_q % H or n_q // H > 8 or values.dtype != keys.dtype
+                or values.stride() != keys.stride() or not values.is_cuda or weight.device != keys.device != hidden_states.device
+                or not 0 <= self.n_sink <= 64):
+            return None
+        from .attention_utils import _head_geometry
+        if _head_geometry(module, hidden) != (n_q, D):
+            return None
+        ks, hs = keys.stride(), hidden_states.stride()
+        n = 4 if keys.dtype == torch.float32 else 8
+        if (ks[3] != 1 or ks[0] % n or ks[1] % n or ks[2] % n or hs[2] != 1 or hs[0] % 8 or hs[1] % 8
+                or (keys.data_ptr() | values.data_ptr() | hidden_states.data_ptr()) % 16):
+            return None
+        dev, n_future = keys.device, self.n_future_positions
+        cos = sin = None
+        rotary_emb = getattr(module, "rotary_emb", None)
+        if rotary_emb is not None and n_future > 0:
+            key = (id(rotary_emb), T, n_future, weight.dtype, dev)
+            hit = None if rope_tables is None else rope_tables.get(key)
+            if hit is None:
+                pos = torch.arange(T, T + n_future, device=dev).unsqueeze(0)
+                cos, sin = _aligned_rotary_outputs(rotary_emb, hidden_states.new_empty(1), pos)
+                if cos.shape != (1, n_future, D) or sin.shape != cos.shape:
+                    return None
+                hit = (cos.contiguous(), sin.contiguous(), rotary_emb)
+                if rope_tables is not None:
+                    rope_tables[key] = hit
+            cos, sin = hit[:2]
+        if out is None:
+            out = torch.empty(B, H, T, dtype=torch.float32, device=dev)
+        ws_bytes = lib.odmkv_prompt_scores_workspace_bytes(B, T, hidden, n_q, H)
+        ws = _lib.workspace(dev, ws_bytes, "prompt")
+        args = _lib.Prompt(
+            hidden_states.data_ptr(), hs[0], hs[1], weight.data_ptr(), weight.stride(0), _lib.ptr(bias), _lib.ptr(cos), _lib.ptr(sin),
+            keys.data_ptr(), values.data_ptr(), ks[0], ks[1], ks[2], out.data_ptr(), ws.data_ptr(), ws_bytes, dt, kt, B, T, hidden, n_q,
+            H, n_future, self.n_sink, kt if self.model_dtype_rounding and kt != _lib.F32 else -1, float(self.epsilon))
+        _lib.check(lib.odmkv_prompt_scores(C.byref(args), _lib.stream_ptr(dev)))
+        return out
 
     def score_with_attn(self, keys, values, attn_weights, *, module=None):
         H = keys.shape[0]

@@ -232,6 +232,23 @@ def _decode_operands(head_dim: int, device):
     return got
 
 
+def evicted_indices(levels: torch.Tensor, T: int, counts) -> list:
+    """(b, h, t) index tensors of the evicted positions of every layer of `levels` (uint8 [layers, B, H, >= T]), None for a
+    layer without any; counts: how many each layer has (the host knows: nothing waits for the device)."""
+    n_layers, B, H, _ = levels.shape
+    total = sum(counts)
+    if total == 0:
+        return [None] * n_layers
+    dev = levels.device
+    out = torch.empty(3 * total, dtype=torch.long, device=dev)
+    ws_bytes = lib.odmkv_evicted_layers_workspace_bytes(n_layers, B, H, T)
+    ws = _lib.workspace(dev, ws_bytes, "evicted")
+    _lib.check(lib.odmkv_evicted_indices_layers(levels.data_ptr(), n_layers, B, H, T, levels.stride(2), (C.c_int64 * n_layers)(*counts),
+                                                out.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev)))
+    parts = out.split([3 * n for n in counts])
+    return [p.view(3, n).unbind(0) if n else None for p, n in zip(parts, counts)]
+
+
 def _empty_positions(device) -> torch.Tensor:
     return torch.empty((0, 3), dtype=torch.long, device=device)
 
@@ -703,19 +720,14 @@ class TurboQuantAdaptiveKVCacheState:
             return None
         if self._masked is None:
             # (their number is known from the counts of what is stored: nothing waits for the device)
-            B, H, T = self.batch_size, self.num_heads, self.seq_len
+            T = self.seq_len
             n = self._nseg * T - int(self._counts.sum())
-            if n == 0:
-                self._masked = (None,)
-            else:
-                out = torch.empty(3, n, dtype=torch.long, device=self.device)
-                ws_bytes = lib.odmkv_evicted_workspace_bytes(B, H, T)
-                ws = _lib.workspace(self.device, ws_bytes, "evicted")
-                levels = self._level_store
-                _lib.check(lib.odmkv_evicted_indices(levels.data_ptr(), B, H, T, levels.stride(1), n, out.data_ptr(),
-                                                     ws.data_ptr(), ws_bytes, _lib.stream_ptr(self.device)))
-                self._masked = (out.unbind(0),)
+            self._masked = (evicted_indices(self._level_store.unsqueeze(0), T, [n])[0],)
         return self._masked[0]
+
+    def adopt_masked(self, indices) -> None:
+        """`masked_key_indices` of what is stored, by a caller that has listed them (with other layers') already."""
+        self._masked = (indices,)
 
     def visible_mask(self) -> torch.Tensor:
         return self._level_map != 0

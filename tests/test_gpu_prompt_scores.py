@@ -1,0 +1,59 @@
+"""GPU: a prompt's scores in one call (odmkv_prompt_scores, odmkv_project_rows) against the same stages one by one."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+from torch import nn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("batch,rows,cols", [(1, 1, 8), (2, 7, 520), (3, 128, 2048), (7, 1025, 4104)])
+def test_projected_rows(batch, rows, cols, dtype):
+    from kvquant import _lib
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    w = (torch.randn(rows, cols + 8, generator=g, device="cuda") * cols ** -0.5).to(dtype)[:, :cols]
+    x, bias = (torch.randn(n, generator=g, device="cuda").to(dtype) for n in ((batch, cols), (rows,)))
+    for b in (None, bias):
+        want = x.double() @ w.double().t().contiguous() + (0 if b is None else b.double())
+        for out_dtype in (dtype, torch.float32):
+            out = torch.empty(batch, rows, dtype=out_dtype, device="cuda")
+            _lib.check(_lib.lib.odmkv_project_rows(w.data_ptr(), w.stride(0), _lib.ptr(b), x.data_ptr(), _lib._DT[dtype], batch, rows, cols,
+                                                   out.data_ptr(), _lib.dtype_code(out), _lib.stream_ptr(out.device)))
+            step = {torch.float16: 2 ** -11, torch.bfloat16: 2 ** -8}[dtype]
+            assert ((out.double() - want).abs() <= step * want.abs() + 1e-5).all() and torch.equal(out, out.to(dtype).to(out_dtype))
+
+
+@pytest.mark.parametrize("rope", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,T,dtype,gap", [(1, 4, 4, 5, torch.float16, 0), (2, 8, 2, 300, torch.bfloat16, 0), (3, 7, 1, 777, torch.float16, 0),
+                                                  (2, 16, 2, 1030, torch.float16, 3)])
+def test_scores_of_all_sequences(B, Hq, Hkv, T, dtype, gap, rope):
+    from kvquant import RiskScorer
+    g = torch.Generator(device="cuda").manual_seed(T)
+    hidden = 256
+    module = nn.Module()
+    module.config = SimpleNamespace(num_attention_heads=Hq, head_dim=128)
+    module.q_proj = nn.Linear(hidden, Hq * 128, bias=Hq == 7, device="cuda", dtype=dtype)
+    asked = []
+    if rope:
+        def rotary(x, pos):
+            asked.append(1)
+            a = pos[..., None].float() * (500000.0 ** (-torch.arange(0, 128, 2, device="cuda").float() / 128))
+            a = torch.cat((a, a), dim=-1)
+            return a.cos().to(x.dtype), a.sin().to(x.dtype)
+        module.rotary_emb = rotary
+    h = (torch.randn(B, T, hidden, generator=g, device="cuda") + 0.3).to(dtype)
+    k, v = (torch.randn(B, Hkv + gap, T, 128, generator=g, device="cuda").to(dtype)[:, gap:] for _ in range(2))
+    scorer = RiskScorer(n_future_positions=64, n_sink=4, epsilon=1e-2)
+    scorer.normalize_grain = "global"
+    tables = {}
+    with torch.inference_mode():
+        got = [scorer.score_prompt(k, v, i, module=module, hidden_states=h, rope_tables=tables) for i in range(2)][1]
+        assert len(asked) == (1 if rope else 0)                                   # the layers of a forward share the tables
+        for b in range(B):
+            want = scorer.score_prefill(k[b], v[b], 0, module=module, hidden_states=h[b:b + 1])
+            assert (got[b] - want).norm() <= 2e-3 * want.norm()                    # (mean queries may land one step of the type apart)
+            assert torch.equal(got[b][:, :4], got[b][:, 4:].max().expand(Hkv, 4))   # the sinks take their own sequence's largest
+        module.q_norm = nn.Identity()
+        assert scorer.score_prompt(k, v, 0, module=module, hidden_states=h) is None
