@@ -19,6 +19,12 @@ struct MeanArgs {
 
 template <int DT> struct Vec16 { static constexpr int N = DT == ODMKV_F32 ? 4 : 8; };
 
+__device__ static inline uint4 stream16(const void* p) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 template <int DT>
 __device__ static inline void add16(const uint4& v, float* acc) {
     if constexpr (DT == ODMKV_F32) {
@@ -34,11 +40,13 @@ __device__ static inline void add16(const uint4& v, float* acc) {
 }
 
 // Bound by HBM: the hidden states once (268 MB for 32k tokens of 4096).  A thread owns 16 bytes of a row and walks its
-// workgroup's rows with eight requests in flight; the rows are split so that about two thousand workgroups share the
-// matrix.  The torch form (conversion to fp32, mean) moved five times the bytes: 32k x 4096 fp16 250 us, here 60 us.
+// workgroup's rows with four requests in flight.  Two workgroups per compute unit with long runs of rows each, and loads that
+// leave nothing in the caches, read at 6.4 TB/s (32k x 4096: 42 us; 131k: 159 us, where runs of 256 rows do best); two
+// thousand workgroups of 32 rows with plain loads reached 4 TB/s (66 us; 220 us).  The torch form (conversion to fp32, mean)
+// moved five times the bytes: 250 us.
 template <int DT>
 __global__ __launch_bounds__(MN_THREADS) void mean_part_kernel(MeanArgs a) {
-    constexpr int N = Vec16<DT>::N, U = 8;
+    constexpr int N = Vec16<DT>::N, U = 4;
     const int col = (blockIdx.x * MN_THREADS + threadIdx.x) * N;
     if (col >= a.cols) return;                                        // (cols is a multiple of N)
     const int r0 = blockIdx.y * a.chunk, r1 = min(r0 + a.chunk, a.rows);
@@ -52,7 +60,7 @@ __global__ __launch_bounds__(MN_THREADS) void mean_part_kernel(MeanArgs a) {
     for (; r + U <= r1; r += U) {
         uint4 v[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const uint4*>(p + u * step);
+        for (int u = 0; u < U; ++u) v[u] = stream16(p + u * step);
         p += U * step;
 #pragma unroll
         for (int u = 0; u < U; ++u) add16<DT>(v[u], acc);
@@ -86,8 +94,8 @@ __global__ __launch_bounds__(MN_THREADS) void mean_final_kernel(MeanArgs a) {
 
 static int mean_chunk(int batch, int rows, int cols, int per_thread) {
     const long long blocks = ((cols + MN_THREADS * per_thread - 1) / (MN_THREADS * per_thread)) * (long long)batch;
-    const long long chunks = std::max<long long>(1, 2048 / blocks);
-    return (int)std::max<long long>(16, (rows + chunks - 1) / chunks);
+    const long long chunks = std::max<long long>(1, 512 / blocks);
+    return (int)std::min<long long>(256, std::max<long long>(16, (rows + chunks - 1) / chunks));
 }
 
 extern "C" size_t odmkv_token_mean_workspace_bytes(int batch, int rows, int cols) {
