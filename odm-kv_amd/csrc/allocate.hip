@@ -3,13 +3,15 @@
 // then close the remaining gap by moving the lowest- (or highest-) scored tokens one level.
 //
 // The search is the fixed sequence the host formulation runs: lambda = 1, up to 8 widenings of the
-// bracket (x10 each), 64 halvings, one final assignment.  It is evaluated in 18 launches:
+// bracket (x10 each), 64 halvings, one final assignment.  It is evaluated in 19 launches:
 //   launch 0      all nine widening candidates 1, 10, .. 1e8 at once;
-//   launch 1..16  four halvings each: the 15 midpoints the next four steps can reach form a binary
+//   launch 1..17  halvings.  While the lower end is still 0, the next fifteen midpoints on the way down (hi / 2, hi / 4, ..):
+//                 budgets are usually met at a lambda some thirty halvings below 1, two launches away.  Once the lower
+//                 end has moved, four halvings each: the 15 midpoints the next four steps can reach form a binary
 //                 tree that is known in advance, so one pass over the scores evaluates them all;
-//   launch 17     the final lambda, which also records the chosen level of every token.
+//   launch 18     the final lambda, which also records the chosen level of every token.
 // The costs use lambda rounded to fp32, so once the bracket's ends are neighbouring fp32 numbers
-// (after about 32 halvings on typical scores) the rest of the search is decided by rounding alone:
+// (after 24 halvings more) the rest of the search is decided by rounding alone:
 // it is walked on the spot and the remaining halving launches return immediately.
 // Every workgroup writes its partial bit sums with plain stores and is done.  The next launch begins,
 // in every workgroup, by adding up the row's partial sums of the launch before (a few hundred
@@ -22,21 +24,26 @@
 // Arithmetic is kept exactly as the host formulation it replaces: fp32 products rounded
 // separately and then added (no fused multiply-add), lambda rounded to fp32 before use, the
 // first (lowest-width) level wins a tie, avg = fp32(sum) / fp32(n), bracket and gap in fp64.
+#include <algorithm>
 #include "common.h"
 
 #define NLV ODMKV_MAX_LEVELS
 #define STEPS 4                               // halvings per launch
 #define NCAND ((1 << STEPS) - 1)              // 15 tree nodes, numbered 1..15
 #define N_WIDEN 9
-#define N_HALVE_LAUNCH (64 / STEPS)
+#define N_HALVE 64
+#define N_HALVE_LAUNCH (N_HALVE / STEPS + 1)  // a first launch of the way down may decide a single halving
 #define N_LAUNCH (1 + N_HALVE_LAUNCH + 1)
 #define L_FINAL (N_LAUNCH - 1)
 #define SLOTS 16                              // partial sums per workgroup
 #define EV_THREADS 512
 #ifndef EV_TPT
-#define EV_TPT 2                              // tokens per thread in an evaluation
+#define EV_TPT 2                              // tokens per thread of the candidates' and the last pass
 #endif
 #define EV_TOKENS (EV_THREADS * EV_TPT)
+#define EV_WGS 512ll                          // workgroups an evaluation is cut for over all rows (256: 305 us for 4 x 262144, 1024: 280, 512: 268)
+#define EV_BIG 2                              // tokens per thread and run where there are more than one per thread
+#define EV_MAX_CHUNKS 256                     // workgroups of a row in an evaluation
 #define CAND_MAX 16                           // repair moves of at most this many tokens take the short path
 
 struct RowState {
@@ -46,20 +53,24 @@ struct RowState {
     int has_finite, has_nonfinite;
     int lo_moved, hi_within;       // the bracket ends' averages are known (lo: above budget, hi: within)
     int collapsed;                 // the remaining halvings were resolved without evaluations
+    int done;                      // halvings decided so far
     int final_hist[NLV];
 };
 
 struct AllocArgs {
     const float* scores;
     const uint8_t* sink_mask;
-    int rows, n, period, n_sink, sink_bits, K, n_chunks;
+    int rows, n, period, n_sink, sink_bits, K;
+    int n_chunks, iters;           // workgroups of a row in an evaluation, and how many runs of tokens each of them walks
+    int n_cand;                    // workgroups of a row in the candidates' pass
+    int prune;                     // no error is negative: tokens whose level the candidates' ends settle need not see the others
     float eps[NLV];
     float bitsf[NLV];
     int nominal[NLV];
     const double* target;          // device, [rows]
     uint8_t* chosen;               // [rows, n]
     unsigned int* partial;         // [2][rows, n_chunks, SLOTS]: launch L writes half L & 1
-    unsigned long long* cand;      // [rows, n_chunks, CAND_MAX]
+    unsigned long long* cand;      // [rows, n_cand, NLV, CAND_MAX]: per move of the repair
     RowState* state;               // [3][rows]: launch L >= 1 leaves the state it starts from in third L & 1 (launch 0 starts
                                    // from third 0, which the set-up kernels fill); third 2 is the final one
     int32_t* bits_out;
@@ -105,7 +116,7 @@ __global__ void alloc_init_kernel(AllocArgs a) {
         t = fmax(t, (double)a.nominal[0]);
         st.lo = 0.0; st.hi = 1.0; st.target = t; st.gap = 0.0; st.lam = 1.0;
         st.n_active = 0; st.max_finite = 0u; st.has_finite = 0; st.has_nonfinite = 0;
-        st.lo_moved = 0; st.hi_within = 0; st.collapsed = 0;
+        st.lo_moved = 0; st.hi_within = 0; st.collapsed = 0; st.done = 0;
         for (int k = 0; k < NLV; ++k) st.final_hist[k] = 0;
     }
 }
@@ -193,11 +204,13 @@ __device__ static void advance(const AllocArgs& a, RowState& st, int L, const un
         st.hi_within = !(avg_hi > st.target);
     } else if (L < L_FINAL) {
         double lo = st.lo, hi = st.hi;
-        int node = 1;
-        for (int s = 0; s < STEPS; ++s) {
+        const int steps = min(st.lo_moved ? STEPS : NCAND, N_HALVE - st.done);
+        for (int s = 0, node = 1; s < steps; ++s) {
             const double mid = (lo + hi) * 0.5;
-            const double avg = (double)((float)sums[node] / nf);
-            if (avg > st.target) { lo = mid; node = 2 * node + 1; st.lo_moved = 1; } else { hi = mid; node = 2 * node; st.hi_within = 1; }
+            const bool above = (double)((float)sums[st.lo_moved ? node : s + 1] / nf) > st.target;
+            ++st.done;
+            if (above) { lo = mid; node = 2 * node + 1; } else { hi = mid; node = 2 * node; st.hi_within = 1; }
+            if (above && !st.lo_moved) { st.lo_moved = 1; break; }                // the way down ends here
         }
         // The costs see lambda rounded to fp32.  Once fp32(lo) and fp32(hi) are neighbouring floats,
         // every later midpoint rounds to one of the two, whose averages are known (lo was evaluated
@@ -205,13 +218,12 @@ __device__ static void advance(const AllocArgs& a, RowState& st, int L, const un
         // are walked here; the launches that would have evaluated them return at once.
         const float fl = (float)lo, fh = (float)hi;
         if (st.lo_moved && st.hi_within && fl < fh && nextafterf(fl, INFINITY) == fh) {
-            for (int s = L * STEPS; s < N_HALVE_LAUNCH * STEPS; ++s) {
+            for (; st.done < N_HALVE; ++st.done) {
                 const double mid = (lo + hi) * 0.5;
                 if ((float)mid == fl) lo = mid; else hi = mid;
             }
-            st.collapsed = 1;
-            st.lam = (lo + hi) * 0.5;
         }
+        if (st.done == N_HALVE) { st.collapsed = 1; st.lam = (lo + hi) * 0.5; }
         st.lo = lo; st.hi = hi;
     } else {
         unsigned long long S = 0ull;
@@ -223,7 +235,6 @@ __device__ static void advance(const AllocArgs& a, RowState& st, int L, const un
         st.gap = (avg - st.target) * (double)st.n_active;
         return;
     }
-    if (L + 1 == L_FINAL) st.lam = (st.lo + st.hi) * 0.5;
 }
 
 // the lambda that slot c of launch L evaluates (slots a launch does not use evaluate lambda = 0 and are ignored)
@@ -234,6 +245,7 @@ __device__ static inline float candidate(const RowState& st, int L, int c) {
         return c < N_WIDEN ? (float)h : 0.0f;
     }
     if (L == L_FINAL) return (float)((st.lo + st.hi) * 0.5);
+    if (!st.lo_moved) return c >= 1 ? (float)ldexp(st.hi, -c) : 0.0f;
     return c >= 1 ? tree_candidate(st.lo, st.hi, c) : 0.0f;
 }
 
@@ -251,13 +263,15 @@ __device__ static void carry_state(const AllocArgs& a, int row, int L, RowState*
     const int tid = threadIdx.x;
     const RowState* in = a.state + (size_t)((L - 1) & 1) * a.rows + row;
     // Everything the launch needs of the last one is asked for here, at once: the two fields that say whether that
-    // launch evaluated, a thread's first partial sum (discarded if it did not), and the whole state, which thread 0
+    // launch evaluated, a thread's partial sums (discarded if it did not), and the whole state, which thread 0
     // copies into shared memory and advances there (a private copy lived in scratch memory, behind the barriers, and
     // every access to it was a round trip of its own).
     const int in_active = in->n_active, in_collapsed = in->collapsed;
     const unsigned int* p = a.partial + ((size_t)((L - 1) & 1) * a.rows + row) * a.n_chunks * SLOTS;
     const int n_part = a.n_chunks * SLOTS;
-    const unsigned int v0 = tid < n_part ? p[tid] : 0u;
+    unsigned int v0[8];                                      // (256 workgroups a row at most: 8 x 512)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v0[u] = tid + u * EV_THREADS < n_part ? p[tid + u * EV_THREADS] : 0u;
     if (tid == 0) *cur = *in;
     if (tid < SLOTS) tot[tid] = 0u;
     __syncthreads();
@@ -267,8 +281,10 @@ __device__ static void carry_state(const AllocArgs& a, int row, int L, RowState*
         // further element of the thread is the same slot); the four chunks of a wavefront are added across its
         // 16-lane rows before one lane per slot updates the total
         static_assert(SLOTS == 16 && EV_THREADS % SLOTS == 0, "a slot per lane of a 16-lane row");
-        unsigned int v = v0;
-        for (int idx = tid + blockDim.x; idx < n_part; idx += blockDim.x) v += p[idx];
+        static_assert(EV_MAX_CHUNKS * SLOTS <= 8 * EV_THREADS, "all of a row's partial sums are under way at once");
+        unsigned int v = 0u;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += v0[u];
         v += (unsigned int)__shfl_xor((int)v, 16, WAVE);
         v += (unsigned int)__shfl_xor((int)v, 32, WAVE);
         if ((tid & 63) < SLOTS && v) atomicAdd(&tot[tid & (SLOTS - 1)], v);
@@ -284,41 +300,37 @@ __device__ static void carry_state(const AllocArgs& a, int row, int L, RowState*
     __syncthreads();
 }
 
-// sums of 16-bit fields over the wave: on return, lanes with (lane & 7) == 0 hold packed pair
-// number (lane >> 3) in v[0]
-__device__ static inline void reduce_scatter8(unsigned int (&v)[8], int lane) {
-#pragma unroll
-    for (int half = 4; half >= 1; half >>= 1) {
-        const int o = half * 8;                 // 32, 16, 8
-        const bool upper = (lane & o) != 0;
-#pragma unroll
-        for (int i = 0; i < half; ++i) {
-            const unsigned int send = upper ? v[i] : v[i + half];
-            const unsigned int keep = upper ? v[i + half] : v[i];
-            v[i] = keep + (unsigned int)__shfl_xor((int)send, o, WAVE);
-        }
-    }
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1) v[0] += (unsigned int)__shfl_xor((int)v[0], o, WAVE);
-}
-
-template <int K>
+// A launch's workgroups each begin by adding up what the last launch's workgroups of the row left, so their number is what a
+// long row pays for: with one per 1024 tokens a row of a million read 64 KB of partial sums in each of 1024 workgroups, every
+// launch.  A workgroup therefore walks `iters` runs of TPT tokens per thread (at most 256 workgroups a row; short rows keep
+// one token per thread, where the time is the evaluation's own).  Its evaluation is bound by the 15 x K cost comparisons of a
+// token: tokens whose level is the same at the least and the largest candidate, by more than rounding could move it, are settled (the
+// difference of two levels' costs is a straight line in lambda) and counted once; what is left is closed up in LDS.
+// With the way down (above): a row of 4096 scores 137 -> 100 us a call, 4 rows of 262144 285 -> 155 us, one of 1048576
+// 382 -> 170 us.
+template <int K, int TPT>
 __global__ __launch_bounds__(EV_THREADS) void alloc_eval_kernel(AllocArgs a, int L) {
+    constexpr int RUN = EV_THREADS * TPT, LIST = 2 * RUN;
     __shared__ __align__(16) float lamb[SLOTS][NLV];     // fl32(lambda_c * b_k)
     __shared__ int lsum[SLOTS];
     __shared__ unsigned int tot[SLOTS];
     __shared__ RowState cur;
-    const int row = blockIdx.y, tid = threadIdx.x;
-    // the scores are asked for first: they do not depend on the state, which takes a round trip of its own
-    const int base = blockIdx.x * EV_TOKENS;
-    float raw[EV_TPT];
-    bool active[EV_TPT];
+    __shared__ float open[LIST];
+    __shared__ int n_open;
+    const int row = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    // the first scores are asked for first: they do not depend on the state, which takes a round trip of its own
+    const int first = blockIdx.x * a.iters * RUN, iters = min(a.iters, (a.n - first + RUN - 1) / RUN);
+    float raw[TPT];
+    bool active[TPT];
+    auto request = [&](int it) {
 #pragma unroll
-    for (int e = 0; e < EV_TPT; ++e) {
-        const int i = base + e * EV_THREADS + tid;
-        active[e] = i < a.n && !is_sink(a, row, i);
-        raw[e] = active[e] ? a.scores[(size_t)row * a.n + i] : 0.0f;
-    }
+        for (int e = 0; e < TPT; ++e) {
+            const int i = first + it * RUN + e * EV_THREADS + tid;
+            active[e] = i < a.n && !is_sink(a, row, i);
+            raw[e] = active[e] ? a.scores[(size_t)row * a.n + i] : 0.0f;
+        }
+    };
+    request(0);
     if (L == 0) {
         if (tid == 0) cur = a.state[row];
         __syncthreads();
@@ -332,69 +344,116 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_eval_kernel(AllocArgs a, int
         lamb[c][k] = __fmul_rn(candidate(st, L, c), a.bitsf[k]);
     }
     if (tid < SLOTS) lsum[tid] = 0;
+    if (tid == 0) n_open = 0;
     __syncthreads();
 
     const Cleaner clean(st);
-    float se[EV_TPT][K];
-#pragma unroll
-    for (int e = 0; e < EV_TPT; ++e) {
-        const float s = active[e] ? clean(raw[e]) : 0.0f;
-#pragma unroll
-        for (int k = 0; k < K; ++k) se[e][k] = __fmul_rn(s, a.eps[k]);
-    }
-
     if (L != L_FINAL) {
-        unsigned int acc[8];
+        int settled_sum = 0;
+        unsigned int sum = 0u;                              // this lane's candidate over its share of the open tokens
+        float end[2][K], lb[K];                             // fl32(lambda * b_k) of the least and the largest candidate, and of the lane's
+        const int c = tid & (SLOTS - 1), group = tid / SLOTS;
 #pragma unroll
-        for (int p = 0; p < 8; ++p) acc[p] = 0u;
-#pragma unroll
-        for (int c = 0; c < SLOTS; ++c) {
-            const float4 l0 = *reinterpret_cast<const float4*>(&lamb[c][0]);
-            const float4 l1 = *reinterpret_cast<const float4*>(&lamb[c][4]);
-            const float lb[NLV] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
-            unsigned int sum = 0u;
-#pragma unroll
-            for (int e = 0; e < EV_TPT; ++e) {
-                float bc = __fadd_rn(se[e][0], lb[0]);
+        for (int k = 0; k < K; ++k) {
+            end[0][k] = lamb[L == 0 ? 0 : st.lo_moved ? (NCAND + 1) / 2 : NCAND][k];      // (a tree's leftmost and rightmost nodes,
+            end[1][k] = lamb[L == 0 ? N_WIDEN - 1 : st.lo_moved ? NCAND : 1][k];          // the last and the first on the way down)
+            lb[k] = lamb[c][k];
+        }
+        // The candidates' pass over open[0 .. count): a lane keeps one candidate and walks every 32nd token.  (A token per lane
+        // and the candidates written out one after the other was 8 KB of code that every launch fetched anew.)
+        auto evaluate = [&](int count) {
+#pragma unroll 2
+            for (int i = group; i < count; i += EV_THREADS / SLOTS) {
+                const float s = open[i];
+                float bc = __fadd_rn(__fmul_rn(s, a.eps[0]), lb[0]);
                 int bn = a.nominal[0];
 #pragma unroll
                 for (int k = 1; k < K; ++k) {
-                    const float cst = __fadd_rn(se[e][k], lb[k]);
+                    const float cst = __fadd_rn(__fmul_rn(s, a.eps[k]), lb[k]);
                     if (cst < bc) { bc = cst; bn = a.nominal[k]; }
                 }
-                sum += active[e] ? (unsigned int)bn : 0u;
+                sum += (unsigned int)bn;
             }
-            acc[c >> 1] += sum << (16 * (c & 1));           // at most 64 lanes * EV_TPT * 16 per field
+        };
+        for (int it = 0; it < iters; ++it) {
+#pragma unroll
+            for (int e = 0; e < TPT; ++e) {
+                const float s = active[e] ? clean(raw[e]) : 0.0f;
+                bool settled = false;
+                if (a.prune) {
+                    int at[2];
+                    settled = true;
+                    float se[K];
+#pragma unroll
+                    for (int k = 0; k < K; ++k) se[k] = __fmul_rn(s, a.eps[k]);
+#pragma unroll
+                    for (int side = 0; side < 2; ++side) {
+                        float best = __fadd_rn(se[0], end[side][0]), second = INFINITY;
+                        int bn = a.nominal[0];
+#pragma unroll
+                        for (int k = 1; k < K; ++k) {
+                            const float cst = __fadd_rn(se[k], end[side][k]);
+                            second = __builtin_amdgcn_fmed3f(cst, best, second);
+                            if (cst < best) { best = cst; bn = a.nominal[k]; }
+                        }
+                        at[side] = bn;
+                        // (costs carry relative errors of 2^-23; the constant covers products in the subnormal range)
+                        settled = settled && second * (1.0f - 0x1p-20f) > best + 1e-36f;
+                    }
+                    settled = settled && at[0] == at[1];
+                    if (active[e] && settled) settled_sum += at[0];
+                }
+                const bool keep = active[e] && !settled;
+                const unsigned long long m = __ballot(keep);
+                if (m != 0ull) {                                         // (wave-uniform)
+                    int at = 0;
+                    if (lane == 0) at = atomicAdd(&n_open, __popcll(m));
+                    at = __builtin_amdgcn_readfirstlane(at);
+                    if (keep) open[at + __popcll(m & ((1ull << lane) - 1ull))] = s;
+                }
+            }
+            if (it + 1 < iters) request(it + 1);
+            __syncthreads();
+            const int count = n_open;
+            __syncthreads();                                             // (nobody adds to it before everybody has read it)
+            if (it + 1 == iters || count > LIST - RUN) {                 // (workgroup-uniform) no room for another run
+                evaluate(count);
+                __syncthreads();
+                if (tid == 0) n_open = 0;
+                __syncthreads();
+            }
         }
-        reduce_scatter8(acc, tid & 63);
-        if ((tid & 7) == 0) {
-            const int p = (tid & 63) >> 3;
-            if (acc[0] & 0xffffu) atomicAdd(&lsum[2 * p], (int)(acc[0] & 0xffffu));
-            if (acc[0] >> 16) atomicAdd(&lsum[2 * p + 1], (int)(acc[0] >> 16));
-        }
+        settled_sum = wave_sum_int(settled_sum);
+        sum += (unsigned int)__shfl_xor((int)sum, 16, WAVE);
+        sum += (unsigned int)__shfl_xor((int)sum, 32, WAVE);
+        if (lane < SLOTS) atomicAdd(&lsum[lane], (int)sum + settled_sum);
     } else {
         int cnt[NLV];
 #pragma unroll
         for (int k = 0; k < NLV; ++k) cnt[k] = 0;
+        for (int it = 0; it < iters; ++it) {
+            if (it > 0) request(it);
 #pragma unroll
-        for (int e = 0; e < EV_TPT; ++e) {
-            float bc = __fadd_rn(se[e][0], lamb[0][0]);
-            int best = 0;
+            for (int e = 0; e < TPT; ++e) {
+                const float s = active[e] ? clean(raw[e]) : 0.0f;
+                float bc = __fadd_rn(__fmul_rn(s, a.eps[0]), lamb[0][0]);
+                int best = 0;
 #pragma unroll
-            for (int k = 1; k < K; ++k) {
-                const float cst = __fadd_rn(se[e][k], lamb[0][k]);
-                if (cst < bc) { bc = cst; best = k; }
-            }
-            if (active[e]) {
-                a.chosen[(size_t)row * a.n + base + e * EV_THREADS + tid] = (uint8_t)best;
+                for (int k = 1; k < K; ++k) {
+                    const float cst = __fadd_rn(__fmul_rn(s, a.eps[k]), lamb[0][k]);
+                    if (cst < bc) { bc = cst; best = k; }
+                }
+                if (active[e]) {
+                    a.chosen[(size_t)row * a.n + first + it * RUN + e * EV_THREADS + tid] = (uint8_t)best;
 #pragma unroll
-                for (int k = 0; k < NLV; ++k) cnt[k] += (best == k);
+                    for (int k = 0; k < NLV; ++k) cnt[k] += (best == k);
+                }
             }
         }
 #pragma unroll
         for (int k = 0; k < NLV; ++k) {
             const int s = wave_sum_int(cnt[k]);
-            if ((tid & 63) == 0 && s) atomicAdd(&lsum[k], s);
+            if (lane == 0 && s) atomicAdd(&lsum[k], s);
         }
     }
     __syncthreads();
@@ -466,7 +525,8 @@ __device__ static inline void select_smallest(unsigned long long (&keys)[NK], in
     }
 }
 
-// per chunk: the candidates for the first move when it is small
+// per chunk: the candidates for the repair's moves that are small.  (A move takes tokens from a level that no earlier move of
+// the walk has touched, so all of them are chosen from the levels as they are.)
 __global__ __launch_bounds__(EV_THREADS) void alloc_cand_kernel(AllocArgs a) {
     __shared__ unsigned long long wbest[EV_THREADS / 64];
     __shared__ unsigned int tot[SLOTS];
@@ -476,20 +536,33 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_cand_kernel(AllocArgs a) {
     const RowState& st = cur;
     if (st.n_active == 0 || fabs(st.gap) <= 0.5) return;
     const bool over = st.gap > 0;
-    Move m;
-    if (!next_move(a, st.final_hist, fabs(st.gap), over, over ? 0 : a.K - 2, m) || m.want > CAND_MAX) return;
+    double gap = fabs(st.gap);
     const Cleaner clean(st);
-    unsigned long long keys[EV_TPT];
     const int base = blockIdx.x * EV_TOKENS;
+    float score[EV_TPT];
+    int level[EV_TPT];
 #pragma unroll
     for (int e = 0; e < EV_TPT; ++e) {
         const int i = base + e * EV_THREADS + tid;
-        keys[e] = KEY_NONE;
-        if (i < a.n && !is_sink(a, row, i) && a.chosen[(size_t)row * a.n + i] == m.from)
-            keys[e] = token_key(clean(a.scores[(size_t)row * a.n + i]), i, m.lowest);
+        const bool on = i < a.n && !is_sink(a, row, i);
+        level[e] = on ? a.chosen[(size_t)row * a.n + i] : -1;
+        score[e] = on ? clean(a.scores[(size_t)row * a.n + i]) : 0.0f;
     }
-    unsigned long long* out = a.cand + ((size_t)row * a.n_chunks + blockIdx.x) * CAND_MAX;
-    select_smallest<EV_TPT, EV_THREADS / 64>(keys, m.want, wbest, [&](int r, unsigned long long g) { out[r] = g; });
+    unsigned long long* out = a.cand + ((size_t)row * a.n_cand + blockIdx.x) * NLV * CAND_MAX;
+    int i = over ? 0 : a.K - 2;
+    Move m;
+    for (int j = 0; next_move(a, st.final_hist, gap, over, i, m); ++j) {                  // the walk of alloc_repair_kernel
+        if (m.want <= CAND_MAX) {
+            unsigned long long keys[EV_TPT];
+#pragma unroll
+            for (int e = 0; e < EV_TPT; ++e)
+                keys[e] = level[e] == m.from ? token_key(score[e], base + e * EV_THREADS + tid, m.lowest) : KEY_NONE;
+            select_smallest<EV_TPT, EV_THREADS / 64>(keys, m.want, wbest, [&](int r, unsigned long long g) { out[j * CAND_MAX + r] = g; });
+        }
+        gap -= m.want * m.delta;
+        if (gap <= 0.5) break;
+        i = m.i + (over ? 1 : -1);
+    }
 }
 
 #define RB 1024
@@ -576,8 +649,9 @@ __device__ static void move_tokens(const AllocArgs& a, int row, const Cleaner& c
     }
 }
 
-// one workgroup per row: apply the first move from the chunk candidates when it is small, any other
-// move by a radix select over the row
+// one workgroup per row: apply the moves from the chunk candidates where they are small, the others by a radix select over
+// the row (a pass of one workgroup over all of it, five times: 5 ms for a million tokens; while only the first move had
+// candidates, and only up to 4096 of them, one row in four of that length took it)
 __global__ __launch_bounds__(RB) void alloc_repair_kernel(AllocArgs a) {
     __shared__ unsigned int hist256[256];
     __shared__ int scratch[32];
@@ -592,30 +666,26 @@ __global__ __launch_bounds__(RB) void alloc_repair_kernel(AllocArgs a) {
     const Cleaner clean(st);
     int i = over ? 0 : a.K - 2;
     Move m;
-    bool first = true;
-    while (next_move(a, st.final_hist, gap, over, i, m)) {
-        if (first && m.want <= CAND_MAX) {
-            uint8_t* ch = a.chosen + (size_t)row * a.n;
-            const unsigned long long* cand = a.cand + (size_t)row * a.n_chunks * CAND_MAX;
-            const int total = a.n_chunks * m.want;
-            if (total <= 4 * RB) {
-                unsigned long long keys[4];
+    uint8_t* ch = a.chosen + (size_t)row * a.n;
+    for (int j = 0; next_move(a, st.final_hist, gap, over, i, m); ++j) {
+        const unsigned long long* cand = a.cand + ((size_t)row * a.n_cand * NLV + j) * CAND_MAX;
+        const int total = a.n_cand * m.want;
+        auto key_at = [&](int idx) { return idx < total ? cand[(size_t)(idx / m.want) * (NLV * CAND_MAX) + idx % m.want] : KEY_NONE; };
+        auto move = [&](int, unsigned long long g) { if (g != KEY_NONE) ch[key_index(g, m.lowest)] = (uint8_t)m.to; };
+        if (m.want <= CAND_MAX && total <= 4 * RB) {
+            unsigned long long keys[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int idx = e * RB + tid;
-                    keys[e] = idx < total ? cand[(size_t)(idx / m.want) * CAND_MAX + idx % m.want] : KEY_NONE;
-                }
-                select_smallest<4, RB / 64>(keys, m.want, wbest, [&](int, unsigned long long g) {
-                    if (g != KEY_NONE) ch[key_index(g, m.lowest)] = (uint8_t)m.to;
-                });
-            } else {
-                move_tokens(a, row, clean, m.from, m.to, m.want, m.lowest, hist256, scratch);
-            }
+            for (int e = 0; e < 4; ++e) keys[e] = key_at(e * RB + tid);
+            select_smallest<4, RB / 64>(keys, m.want, wbest, move);
+        } else if (m.want <= CAND_MAX && total <= 16 * RB) {
+            unsigned long long keys[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) keys[e] = key_at(e * RB + tid);
+            select_smallest<16, RB / 64>(keys, m.want, wbest, move);
         } else {
             __syncthreads();
             move_tokens(a, row, clean, m.from, m.to, m.want, m.lowest, hist256, scratch);
         }
-        first = false;
         gap -= m.want * m.delta;
         if (gap <= 0.5) break;
         i = m.i + (over ? 1 : -1);
@@ -658,12 +728,12 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_write_kernel(AllocArgs a, in
 struct AllocLayout { size_t chosen, partial, cand, state, total; };
 static AllocLayout alloc_layout(int rows, int n) {
     AllocLayout L;
-    const size_t chunks = ((size_t)n + EV_TOKENS - 1) / EV_TOKENS;
+    const size_t chunks = ((size_t)n + EV_TOKENS - 1) / EV_TOKENS, evals = ((size_t)n + EV_THREADS - 1) / EV_THREADS;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes, 256); return o; };
     L.chosen = take((size_t)rows * n);
-    L.partial = take((size_t)2 * rows * chunks * SLOTS * sizeof(unsigned int));
-    L.cand = take((size_t)rows * chunks * CAND_MAX * sizeof(unsigned long long));
+    L.partial = take((size_t)2 * rows * std::min<size_t>(evals, EV_MAX_CHUNKS) * SLOTS * sizeof(unsigned int));
+    L.cand = take((size_t)rows * chunks * NLV * CAND_MAX * sizeof(unsigned long long));
     L.state = take((size_t)3 * rows * sizeof(RowState));
     L.total = off;
     return L;
@@ -699,7 +769,18 @@ extern "C" int odmkv_allocate(const float* scores, int rows, int n,
     AllocArgs a;
     a.scores = scores; a.sink_mask = sink_mask; a.rows = rows; a.n = n;
     a.period = period > 0 ? period : n; a.n_sink = sink_mask ? 0 : n_sink; a.sink_bits = sink_bits; a.K = n_levels;
-    a.n_chunks = (n + EV_TOKENS - 1) / EV_TOKENS;
+    a.n_cand = (n + EV_TOKENS - 1) / EV_TOKENS;
+    // one token per thread up to a workgroup of them per compute unit; then runs of four, as many as leave about one
+    // workgroup per compute unit over all rows
+    const long long all = (long long)rows * n;
+    const int tpt = all <= 256ll * EV_THREADS ? 1 : EV_BIG, run = EV_THREADS * tpt;
+    const int runs = (n + run - 1) / run;
+    a.iters = (int)std::max<long long>((runs + EV_MAX_CHUNKS - 1) / EV_MAX_CHUNKS, (all + EV_WGS * run - 1) / (EV_WGS * run));
+    if (tpt == 1) a.iters = 1;
+    a.n_chunks = (runs + a.iters - 1) / a.iters;
+    a.prune = 1;
+    for (int k = 0; k < n_levels; ++k)
+        if (!(eps[k] >= 0.0)) a.prune = 0;
     for (int k = 0; k < NLV; ++k) {
         a.eps[k] = k < n_levels ? (float)eps[k] : 0.0f;
         a.bitsf[k] = k < n_levels ? (float)levels[k] : 0.0f;
@@ -711,30 +792,34 @@ extern "C" int odmkv_allocate(const float* scores, int rows, int n,
     a.cand = (unsigned long long*)(ws + L.cand);
     a.state = (RowState*)(ws + L.state);
     a.bits_out = bits_out; a.level_counts = level_counts; a.lambda_out = lambda_out;
-    const dim3 grid(a.n_chunks, rows), block(EV_THREADS);
+    const dim3 grid(a.n_chunks, rows), cand_grid(a.n_cand, rows), block(EV_THREADS);
     hipLaunchKernelGGL(alloc_init_kernel, dim3(rows), dim3(64), 0, st, a);
     ODMKV_CHECK_LAUNCH("alloc_init_kernel");
     if (n_levels > 1) {
         hipLaunchKernelGGL(alloc_scan_kernel, dim3((n + SC_TOKENS - 1) / SC_TOKENS, rows), dim3(SC_THREADS), 0, st, a);
         ODMKV_CHECK_LAUNCH("alloc_scan_kernel");
+#define ALLOC_EVAL(K) \
+        if (tpt == 1) hipLaunchKernelGGL((alloc_eval_kernel<K, 1>), grid, block, 0, st, a, l); \
+        else hipLaunchKernelGGL((alloc_eval_kernel<K, EV_BIG>), grid, block, 0, st, a, l)
         for (int l = 0; l < N_LAUNCH; ++l) {
             switch (n_levels) {
-                case 2: hipLaunchKernelGGL(alloc_eval_kernel<2>, grid, block, 0, st, a, l); break;
-                case 3: hipLaunchKernelGGL(alloc_eval_kernel<3>, grid, block, 0, st, a, l); break;
-                case 4: hipLaunchKernelGGL(alloc_eval_kernel<4>, grid, block, 0, st, a, l); break;
-                case 5: hipLaunchKernelGGL(alloc_eval_kernel<5>, grid, block, 0, st, a, l); break;
-                case 6: hipLaunchKernelGGL(alloc_eval_kernel<6>, grid, block, 0, st, a, l); break;
-                case 7: hipLaunchKernelGGL(alloc_eval_kernel<7>, grid, block, 0, st, a, l); break;
-                default: hipLaunchKernelGGL(alloc_eval_kernel<8>, grid, block, 0, st, a, l); break;
+                case 2: ALLOC_EVAL(2); break;
+                case 3: ALLOC_EVAL(3); break;
+                case 4: ALLOC_EVAL(4); break;
+                case 5: ALLOC_EVAL(5); break;
+                case 6: ALLOC_EVAL(6); break;
+                case 7: ALLOC_EVAL(7); break;
+                default: ALLOC_EVAL(8); break;
             }
             ODMKV_CHECK_LAUNCH("alloc_eval_kernel");
         }
-        hipLaunchKernelGGL(alloc_cand_kernel, grid, block, 0, st, a);
+#undef ALLOC_EVAL
+        hipLaunchKernelGGL(alloc_cand_kernel, cand_grid, block, 0, st, a);
         ODMKV_CHECK_LAUNCH("alloc_cand_kernel");
         hipLaunchKernelGGL(alloc_repair_kernel, dim3(rows), dim3(RB), 0, st, a);
         ODMKV_CHECK_LAUNCH("alloc_repair_kernel");
     }
-    hipLaunchKernelGGL(alloc_write_kernel, grid, block, 0, st, a, n_levels == 1 ? 1 : 0);
+    hipLaunchKernelGGL(alloc_write_kernel, cand_grid, block, 0, st, a, n_levels == 1 ? 1 : 0);
     ODMKV_CHECK_LAUNCH("alloc_write_kernel");
     return 0;
 }

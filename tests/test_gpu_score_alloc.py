@@ -229,6 +229,34 @@ def test_allocator_batched_rows_with_mixed_budgets():
         assert counts[r].cpu().tolist() == hist
 
 
+@pytest.mark.parametrize("rows,T,spread,target", [
+    (1, 131072, 2.0, 2.0), (1, 131073, 2.0, 3.0), (2, 65537, 0.3, 1.5), (3, 50001, 6.0, 2.5),      # one token per thread and more
+    (1, 300001, 2.0, 2.0), (1, 524289, 1.0, 2.0), (2, 270000, 2.0, 4.0)])                          # several runs a workgroup
+@pytest.mark.parametrize("ties", [False, True])
+def test_allocator_bit_exact_on_long_rows(rows, T, spread, target, ties):
+    """Evaluations that settle most tokens, walk several runs per workgroup and repair with more than one move; with ties, scores
+    of a few hundred values, whose moves are larger than the candidates'."""
+    from kvquant.allocator import optimal_scores_to_bits_batched
+    g = torch.Generator().manual_seed(T + int(ties))
+    s = torch.exp(spread * torch.randn(rows, T, generator=g)) * 1e-5
+    if ties:
+        s = (s.log() * 32).round().div(32).exp()
+    bits, _, lam = optimal_scores_to_bits_batched(s.to(DEV), LEVELS, [target] * rows, EPS, n_sink=4, period=T, eviction_cost=0.5, return_stats=True)
+    for r in range(rows):
+        info = {}
+        want = oal.optimal_scores_to_bits(s[r:r + 1], LEVELS, target, EPS, _sink(1, T), eviction_cost=0.5, info=info)
+        assert lam[r].item() == info["lam"] and torch.equal(bits[r:r + 1].cpu(), want)
+
+
+def test_allocator_with_a_negative_error_sees_every_candidate():
+    from kvquant.allocator import optimal_scores_to_bits
+    g = torch.Generator().manual_seed(5)
+    s = torch.exp(torch.randn(1, 3000, generator=g))
+    eps = {**EPS, 8: -1e-3}
+    got = optimal_scores_to_bits(s.to(DEV), LEVELS, 2.5, eps, eviction_cost=0.5)
+    assert torch.equal(got.cpu(), oal.optimal_scores_to_bits(s, LEVELS, 2.5, eps, None, eviction_cost=0.5))
+
+
 def test_calibrate_epsilon_matches_oracle():
     from kvquant.allocator import calibrate_epsilon
     got = calibrate_epsilon(128, LEVELS, device=DEV, value_quantizer="mse")
