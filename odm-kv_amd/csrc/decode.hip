@@ -856,7 +856,8 @@ template <bool BF>
 __device__ static inline void exact_query(const DecodeArgs& a, int bq_first, int lane, uint4* qraw) {
     const int n = lane & 15, j = lane >> 4, h = n >> 1, lo = n & 1;
     const bool on = h < a.G && (BF || !lo);
-    if (a.q_dt == (BF ? ODMKV_BF16 : ODMKV_F16)) {
+    bool convert = a.q_dt != (BF ? ODMKV_BF16 : ODMKV_F16);
+    if (!convert) {
         typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
         u16x2 worst = (u16x2){0, 0};
 #pragma unroll
@@ -864,36 +865,34 @@ __device__ static inline void exact_query(const DecodeArgs& a, int bq_first, int
             qraw[kb] = make_uint4(0u, 0u, 0u, 0u);
             if (on) qraw[kb] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(a.q) + (size_t)(bq_first + h) * HD + 32 * j + 8 * kb);
         }
-        if constexpr (!BF) return;
+        if constexpr (BF) {
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            const uint32_t w[4] = {qraw[kb].x, qraw[kb].y, qraw[kb].z, qraw[kb].w};
+            for (int kb = 0; kb < 4; ++kb) {
+                const uint32_t w[4] = {qraw[kb].x, qraw[kb].y, qraw[kb].z, qraw[kb].w};
 #pragma unroll
-            for (int e = 0; e < 4; ++e)      // magnitude bits above those of 2^-14, the least normal fp16
-                worst = __builtin_elementwise_max(worst, __builtin_bit_cast(u16x2, w[e] & 0x7fff7fffu) - (u16x2){0x3880, 0x3880});
-        }
-        const bool plain = worst.x < 0x4780 - 0x3880 && worst.y < 0x4780 - 0x3880;      // (65536 = 0x4780)
-        if (__builtin_amdgcn_ballot_w64(on && !plain) == 0) {
-            if (lo) {
-#pragma unroll
-                for (int kb = 0; kb < 4; ++kb) qraw[kb] = make_uint4(0u, 0u, 0u, 0u);
+                for (int e = 0; e < 4; ++e)      // magnitude bits above those of 2^-14, the least normal fp16
+                    worst = __builtin_elementwise_max(worst, __builtin_bit_cast(u16x2, w[e] & 0x7fff7fffu) - (u16x2){0x3880, 0x3880});
+                if (lo) qraw[kb] = make_uint4(0u, 0u, 0u, 0u);
             }
-            return;
+            const bool plain = worst.x < 0x4780 - 0x3880 && worst.y < 0x4780 - 0x3880;      // (65536 = 0x4780)
+            convert = __builtin_amdgcn_ballot_w64(on && !plain) != 0;
         }
     }
+    if (convert) {
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
-        if (on) {
-            float qv[8];
-            load_q8(a.q, a.q_dt, (size_t)(bq_first + h) * HD + 32 * j + 8 * kb, qv);
+        for (int kb = 0; kb < 4; ++kb) {
+            uint32_t w[4] = {0u, 0u, 0u, 0u};
+            if (on) {
+                float qv[8];
+                load_q8(a.q, a.q_dt, (size_t)(bq_first + h) * HD + 32 * j + 8 * kb, qv);
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) {
-                if constexpr (BF) w[e >> 1] = lo ? bf16_pair(bf16_rest(qv[e]), bf16_rest(qv[e + 1])) : bf16_pair(qv[e], qv[e + 1]);
-                else w[e >> 1] = pack_h2(qv[e], qv[e + 1]);
+                for (int e = 0; e < 8; e += 2) {
+                    if constexpr (BF) w[e >> 1] = lo ? bf16_pair(bf16_rest(qv[e]), bf16_rest(qv[e + 1])) : bf16_pair(qv[e], qv[e + 1]);
+                    else w[e >> 1] = pack_h2(qv[e], qv[e + 1]);
+                }
             }
+            qraw[kb] = make_uint4(w[0], w[1], w[2], w[3]);
         }
-        qraw[kb] = make_uint4(w[0], w[1], w[2], w[3]);
     }
 }
 
@@ -1134,15 +1133,17 @@ __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(Deco
 #define NO_ROW (~(size_t)0)
 
 // where query head bq (head g of its group) of this launch's pass stands in out and lse
+// (BLOCK: a kernel of its own for blocks of query tokens; deciding it at run time cost the decode step's merge 0.15 of 4 us)
+template <bool BLOCK>
 __device__ static inline size_t out_row(const DecodeArgs& a, int bq, int bh, int g) {
-    if (a.block_len == 0) return bq;
+    if constexpr (!BLOCK) return bq;
     const int l = (a.pass0 + (int)blockIdx.y) * a.block_per + g / a.block_g;
     return l < a.block_len ? ((size_t)bh * a.block_g + g % a.block_g) * a.block_len + l : NO_ROW;
 }
 
 // MERGE_SPLIT: workgroups per query head (4 when there are few heads, so that the launch still covers the device;
 // 1 for large batches, where every further workgroup only repeats the reading)
-template <int GP, int MERGE_SPLIT>
+template <int GP, int MERGE_SPLIT, bool BLOCK>
 __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs a) {
     __shared__ float part[2][MERGE_SLICES][HD];      // [rotated | exact][slice][dim]
     constexpr int QD = HD / MERGE_SPLIT;                 // output dims of this workgroup
@@ -1157,9 +1158,9 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
     const int slice = __builtin_amdgcn_readfirstlane(tid >> 7);
     const int b = bq / a.Hq, hq = bq % a.Hq;
     const int bh = b * a.s.Hkv + hq / a.G, g = hq % a.G;
-    const size_t row = out_row(a, bq, bh, g);              // of out and lse
+    const size_t row = out_row<BLOCK>(a, bq, bh, g);       // of out and lse
     if (row == NO_ROW) return;                             // (workgroup-uniform: padding of a block's last pass)
-    const float* partial = a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE;
+    const float* partial = BLOCK ? a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE : a.partial;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
     if (a.k_new && g == 0 && quarter == 0 && tid == 0) a.s.seg_count[4][bh] += 1;      // the step's token is stored
     // this thread's share of the value rotation: requested first, it does not depend on the items
@@ -1239,7 +1240,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
 // the 64 KB of Pi_v are pulled into a compute unit once per group, not once per query head (2048 heads: 134 MB of reads
 // out of the L2s for 1 MB of results).  The four 128-thread slices take a head each (two each for groups of five to
 // eight); a slice walks its head's items in rounds of MERGE_CHUNK with a running maximum, as above.
-template <int GP>
+template <int GP, bool BLOCK>
 __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(DecodeArgs a) {
     constexpr int HPS = GP / MERGE_SLICES;                // heads per slice
     static_assert(HPS >= 1, "a slice takes whole heads");
@@ -1252,7 +1253,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
     const int tid = threadIdx.x, lane = tid & 63, j = tid & (HD - 1);
     const int slice = __builtin_amdgcn_readfirstlane(tid >> 7);
     const int b = bh / a.s.Hkv, hq0 = (bh % a.s.Hkv) * a.G;
-    const float* partial = a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE;
+    const float* partial = BLOCK ? a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE : a.partial;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
     if (a.k_new && tid == 0) a.s.seg_count[4][bh] += 1;   // the step's token is stored
     float pv[IN];
@@ -1325,7 +1326,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
         for (int r = 0; r < RS; ++r) tot += part2[g][r][j];
         const float L = headL[g];
         const float o32 = L > 0.0f ? tot / L : 0.0f;
-        const size_t row = out_row(a, b * a.Hq + hq0 + g, bh, g);
+        const size_t row = out_row<BLOCK>(a, b * a.Hq + hq0 + g, bh, g);
         if (row == NO_ROW) continue;
         const size_t oi = row * HD + j;
         if (a.out_dt == ODMKV_F32) reinterpret_cast<float*>(a.out)[oi] = o32;
@@ -1476,19 +1477,14 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
         // from 512 query heads on, a workgroup per (sequence, kv-head) merges all heads of the group (64 x 2048 tokens, 2048
         // heads: the merge 10.8 -> 4.8 us; 512 heads: 3.5 -> 3.2 us); ODMKV_MERGE_GROUP_FROM moves the limit, for measurements
         static const int group_from = [] { const char* e = getenv("ODMKV_MERGE_GROUP_FROM"); return e ? atoi(e) : 512; }();
-        if (heads >= group_from) {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_group_kernel<4>), dim3(B * store->Hkv, passes), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_group_kernel<8>), dim3(B * store->Hkv, passes), dim3(MERGE_THREADS), 0, st, a);
-        } else if (heads >= 256) {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 1>), dim3(B * Hq, passes), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_kernel<8, 1>), dim3(B * Hq, passes), dim3(MERGE_THREADS), 0, st, a);
-        } else if (heads >= 128) {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 2>), dim3(B * Hq * 2, passes), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_kernel<8, 2>), dim3(B * Hq * 2, passes), dim3(MERGE_THREADS), 0, st, a);
-        } else {
-            if (GP == 4) hipLaunchKernelGGL((decode_merge_kernel<4, 4>), dim3(B * Hq * 4, passes), dim3(MERGE_THREADS), 0, st, a);
-            else hipLaunchKernelGGL((decode_merge_kernel<8, 4>), dim3(B * Hq * 4, passes), dim3(MERGE_THREADS), 0, st, a);
-        }
+        const auto launch = [&](auto kernel, int wgs) { hipLaunchKernelGGL(kernel, dim3(wgs, passes), dim3(MERGE_THREADS), 0, st, a); };
+#define ODMKV_MERGE(BLOCK)                                                                                                        \
+        if (heads >= group_from) launch(GP == 4 ? decode_merge_group_kernel<4, BLOCK> : decode_merge_group_kernel<8, BLOCK>, B * store->Hkv);   \
+        else if (heads >= 256) launch(GP == 4 ? decode_merge_kernel<4, 1, BLOCK> : decode_merge_kernel<8, 1, BLOCK>, B * Hq);      \
+        else if (heads >= 128) launch(GP == 4 ? decode_merge_kernel<4, 2, BLOCK> : decode_merge_kernel<8, 2, BLOCK>, B * Hq * 2);  \
+        else launch(GP == 4 ? decode_merge_kernel<4, 4, BLOCK> : decode_merge_kernel<8, 4, BLOCK>, B * Hq * 4)
+        if (a.block_len) { ODMKV_MERGE(true); } else { ODMKV_MERGE(false); }
+#undef ODMKV_MERGE
         ODMKV_CHECK_LAUNCH("decode_merge_kernel");
     }
     return 0;
