@@ -113,8 +113,6 @@ __host__ __device__ static inline long long row_offset(const RowsJob& j, long lo
 __host__ __device__ static inline int container_bytes(int bits) { return bits == 2 ? HD / 4 : bits <= 4 ? HD / 2 : HD; }
 // a tile of 64 rows that the matrix-core quantiser leaves to the exact one carries this in place of its first norm
 #define ROWS_HANDED_OVER 0x7fc0beefu
-// the exact quantiser (rows.hip); flagged: only tiles that carry the mark
-int launch_quantize_rows_exact(const RowsJob& j, int dtype, bool flagged, hipStream_t st);
 // the matrix-core quantiser for 16-bit rows of 2, 3 and 4 bits, and the matrix-core dequantiser from byte codes into
 // 16-bit rows (pack.hip), one or two jobs a launch
 int launch_quantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st);
