@@ -92,16 +92,25 @@ __global__ __launch_bounds__(MN_THREADS) void mean_final_kernel(MeanArgs a) {
     }
 }
 
-static int mean_chunk(int batch, int rows, int cols, int per_thread) {
+// row runs that put two workgroups on every compute unit
+static int mean_runs(int batch, int cols, int per_thread) {
     const long long blocks = ((cols + MN_THREADS * per_thread - 1) / (MN_THREADS * per_thread)) * (long long)batch;
-    const long long chunks = std::max<long long>(1, 512 / blocks);
-    return (int)std::min<long long>(256, std::max<long long>(16, (rows + chunks - 1) / chunks));
+    return (int)std::max<long long>(1, 512 / blocks);
+}
+#define MN_CHUNK_MIN 16
+#define MN_CHUNK_MAX 256
+static int mean_chunk(int batch, int rows, int cols, int per_thread) {
+    const int runs = mean_runs(batch, cols, per_thread);
+    return std::min(MN_CHUNK_MAX, std::max(MN_CHUNK_MIN, (int)(((long long)rows + runs - 1) / runs)));
 }
 
+// Room for the partial sums of any call with at most `rows` rows.  (The parts of one call, ceil(rows / chunk), are no monotone
+// function of its rows: 8193 rows in runs of 33 make 249, 8189 in runs of 32 make 256.)
 extern "C" size_t odmkv_token_mean_workspace_bytes(int batch, int rows, int cols) {
     if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-    const int chunk = std::min(mean_chunk(batch, rows, cols, 8), mean_chunk(batch, rows, cols, 4));
-    return (size_t)batch * ((rows + chunk - 1) / chunk) * cols * sizeof(float);
+    const long long runs = std::max(mean_runs(batch, cols, 8), mean_runs(batch, cols, 4));
+    const long long shortest = ((long long)rows + MN_CHUNK_MIN - 1) / MN_CHUNK_MIN, longest = ((long long)rows + MN_CHUNK_MAX - 1) / MN_CHUNK_MAX;
+    return (size_t)batch * std::min(shortest, std::max(runs, longest)) * cols * sizeof(float);
 }
 
 extern "C" int odmkv_token_mean(const void* x, int dtype, int batch, int rows, int cols, int64_t stride_b, int64_t stride_t,

@@ -57,3 +57,8 @@ def test_scores_of_all_sequences(B, Hq, Hkv, T, dtype, gap, rope):
             assert torch.equal(got[b][:, :4], got[b][:, 4:].max().expand(Hkv, 4))   # the sinks take their own sequence's largest
         module.q_norm = nn.Identity()
         assert scorer.score_prompt(k, v, 0, module=module, hidden_states=h) is None
+
+
+@pytest.mark.parametrize("T", [8193, 8196, 8197])
+def test_prompts_whose_mean_is_cut_otherwise_without_the_sinks(T):
+    test_scores_of_all_sequences(2, 4, 2, T, torch.float16, 0, True)
