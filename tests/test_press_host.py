@@ -200,3 +200,32 @@ def test_release_dense_cache_needs_decode_quant():
         TurboQuantPerTokenBackendPress(scorer=_scorer(), bit_levels=(0, 2, 4, 16), key_quantizer="mse",
                                        value_quantizer="mse", target_avg_bits=2.0, decode_quant=False,
                                        release_dense_cache=True)
+
+
+class _CountingScorer:
+    """Scores a prompt in one call, on any device: every score is the scorer's own number."""
+    def __init__(self, number):
+        self.number, self.calls = number, 0
+
+    def score_prefill(self, keys, values, layer_idx, *, module=None, hidden_states=None):
+        raise AssertionError("the one-call form covers this prompt")
+
+    def score_decode(self, key, value, layer_idx, *, module=None, hidden_states=None):
+        return torch.ones(key.shape[0])
+
+    def score_prompt(self, keys, values, layer_idx, *, module, hidden_states, out=None, rope_tables=None):
+        self.calls += 1
+        return torch.full(keys.shape[:3], self.number)
+
+
+def test_a_scorer_assigned_after_construction_scores_the_next_prompt():
+    from kvquant import TurboQuantPerTokenPress
+    first, second = _CountingScorer(1.0), _CountingScorer(2.0)
+    press = TurboQuantPerTokenPress(scorer=first, bit_levels=(0, 2, 4, 16), value_quantizer="mse", layerwise=True, target_avg_bits=2.0)
+    press._finalize_prefill = lambda cache: None
+    keys = torch.zeros(2, 3, 10, 128)
+    press._prefill_hook(torch.nn.Module(), None, torch.zeros(2, 10, 64), 0, keys, keys)
+    press.scorer = second
+    press._prefill_hook(torch.nn.Module(), None, torch.zeros(2, 10, 64), 1, keys, keys)
+    assert (first.calls, second.calls) == (1, 1)
+    assert (press._prefill_scores[0] == 1.0).all() and (press._prefill_scores[1] == 2.0).all()
