@@ -296,7 +296,8 @@ class RiskScorer(ExpectedAttentionScorer):
         n_q = weight.shape[0] // D
         if (D != _lib.HEAD_DIM or kt is None or T <= self.n_sink or hidden_states.shape[:2] != (B, T) or weight.shape[1] != hidden
                 or hidden % 8 or weight.shape[0] != n_q * D or n_q % H or n_q // H > 8 or values.dtype != keys.dtype
-                or values.stride() != keys.stride() or not values.is_cuda or weight.device != keys.device != hidden_states.device
+                or values.stride() != keys.stride() or not keys.is_cuda
+                or any(x.device != keys.device for x in (values, hidden_states, weight) + (() if bias is None else (bias,)))
                 or not 0 <= self.n_sink <= 64):
             return None
         from .attention_utils import _head_geometry

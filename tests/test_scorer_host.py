@@ -21,3 +21,54 @@ def test_the_mean_workspace_holds_every_run_of_rows(batch, cols):
         for rows in (1, 15, 16, 17, 4095, 4097, 8189, 8193, 65537, 131073, 131072 * 2 + 1):
             chunk = min(256, max(16, -(-rows // runs)))
             assert _lib.lib.odmkv_token_mean_workspace_bytes(batch, rows, cols) >= batch * -(-rows // chunk) * cols * 4
+
+
+class _Fake:
+    """The face of a GPU tensor: what the covering checks of RiskScorer.score_prompt look at."""
+    is_cuda = True
+
+    def __init__(self, shape, dtype, device):
+        import torch
+        self.shape, self.dtype, self.device = torch.Size(shape), dtype, torch.device(device)
+
+    def dim(self):
+        return len(self.shape)
+
+    def stride(self, i=None):
+        s = [1]
+        for n in reversed(self.shape[1:]):
+            s.insert(0, s[0] * n)
+        return tuple(s) if i is None else s[i]
+
+    def data_ptr(self):
+        return 4096
+
+
+@pytest.mark.parametrize("away", ["keys", "values", "hidden", "weight", "bias", None])
+def test_a_prompt_spread_over_devices_is_left_to_the_general_path(away, monkeypatch):
+    import torch
+    from types import SimpleNamespace
+    from kvquant import RiskScorer, scorer as sc
+
+    class Reached(Exception):
+        pass
+
+    def reached(*args, **kw):
+        raise Reached
+
+    where = {n: "cuda:1" if n == away else "cuda:0" for n in ("keys", "values", "hidden", "weight", "bias")}
+    f16, B, H, T, hidden, n_q = torch.float16, 2, 2, 40, 64, 4
+    keys, values = (_Fake((B, H, T, 128), f16, where[n]) for n in ("keys", "values"))
+    h = _Fake((B, T, hidden), f16, where["hidden"])
+    w, b = _Fake((n_q * 128, hidden), f16, where["weight"]), _Fake((n_q * 128,), f16, where["bias"])
+    monkeypatch.setattr(sc, "_plain_projection", lambda module: (w, b))
+    monkeypatch.setattr(sc, "lib", SimpleNamespace(odmkv_prompt_scores_workspace_bytes=reached, odmkv_prompt_scores=reached))
+    module = SimpleNamespace(config=SimpleNamespace(num_attention_heads=n_q, head_dim=128))
+    scorer = RiskScorer(n_future_positions=8, n_sink=4, epsilon=1e-2)
+    scorer.normalize_grain = "global"
+    call = lambda: scorer.score_prompt(keys, values, 0, module=module, hidden_states=h, out=object())
+    if away is None:
+        with pytest.raises(Reached):                       # the same call on one device is the library's
+            call()
+    else:
+        assert call() is None
