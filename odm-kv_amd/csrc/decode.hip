@@ -1141,6 +1141,13 @@ __device__ static inline size_t out_row(const DecodeArgs& a, int bq, int bh, int
     return l < a.block_len ? ((size_t)bh * a.block_g + g % a.block_g) * a.block_len + l : NO_ROW;
 }
 
+// The step's token is stored.  In a full segment no workgroup owned a place for it (the host sized the segment too small):
+// the count stays, as in append_exact_kernel, since the kernels take the tiles up to it for the segment's own.
+__device__ static inline void count_new_token(const odmkv_packed_t& s, int bh) {
+    const int count = s.seg_count[4][bh];
+    if (count < (s.seg_tile[4][bh + 1] - s.seg_tile[4][bh]) * TILE) s.seg_count[4][bh] = count + 1;
+}
+
 // MERGE_SPLIT: workgroups per query head (4 when there are few heads, so that the launch still covers the device;
 // 1 for large batches, where every further workgroup only repeats the reading)
 template <int GP, int MERGE_SPLIT, bool BLOCK>
@@ -1162,7 +1169,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
     if (row == NO_ROW) return;                             // (workgroup-uniform: padding of a block's last pass)
     const float* partial = BLOCK ? a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE : a.partial;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
-    if (a.k_new && g == 0 && quarter == 0 && tid == 0) a.s.seg_count[4][bh] += 1;      // the step's token is stored
+    if (a.k_new && g == 0 && quarter == 0 && tid == 0) count_new_token(a.s, bh);
     // this thread's share of the value rotation: requested first, it does not depend on the items
     const int jj = tid % QD, rs = tid / QD;
     float pv[IN];
@@ -1255,7 +1262,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
     const int b = bh / a.s.Hkv, hq0 = (bh % a.s.Hkv) * a.G;
     const float* partial = BLOCK ? a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE : a.partial;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
-    if (a.k_new && tid == 0) a.s.seg_count[4][bh] += 1;   // the step's token is stored
+    if (a.k_new && tid == 0) count_new_token(a.s, bh);
     float pv[IN];
 #pragma unroll
     for (int ii = 0; ii < IN; ++ii) pv[ii] = a.pi_v[(size_t)(slice * IN + ii) * HD + j];

@@ -67,3 +67,28 @@ def test_a_blocks_own_tokens_merged_with_the_stores_part(L, G, masked, qt, kt):
     want = (both[..., :1] * out_s.double().cpu() + both[..., 1:] @ vr).transpose(1, 2)
     tol = {torch.float32: 2e-5, torch.float16: 1e-3, torch.bfloat16: 8e-3}[qt]
     assert ((out.double().cpu() - want).norm(dim=-1) <= tol * (want.norm(dim=-1) + 1e-3)).all()
+
+
+@pytest.mark.parametrize("B,H,G", [(1, 2, 4), (2, 1, 7), (64, 2, 4)])             # (the last: the merge by groups of heads)
+def test_a_step_into_full_exact_segments_leaves_their_counts(B, H, G):
+    import ctypes as C
+    from kvquant import _lib
+    from kvquant.tq_adaptive_backend import TurboQuantAdaptiveKVCacheState
+    g = torch.Generator(device="cuda").manual_seed(B)
+    k, v = (torch.randn(B, H, 128, 128, generator=g, device="cuda").half() for _ in range(2))
+    bits = torch.full((B, H, 128), 16, dtype=torch.int32, device="cuda")
+    bits[:, :, 64:] = 3                                        # 64 exact tokens a pair: one tile, and no room beside them
+    st = TurboQuantAdaptiveKVCacheState(128, LEVELS, device="cuda", dtype=k.dtype, key_quantizer="mse", value_quantizer="mse", exact_slack=0)
+    st.prefill(k, v, bits)
+    q = torch.randn(B, H * G, 128, generator=g, device="cuda").half()
+    want = st.decode_attention(q)
+    ws = torch.empty(_lib.lib.odmkv_decode_workspace_bytes(B, H * G, st._items[2]), dtype=torch.uint8, device="cuda")
+    step = _lib.Step(C.pointer(st._packed), C.pointer(st._worklist), st._pi_k_ops.data_ptr(), st.pi_v.data_ptr(), st._decode_cb.data_ptr(),
+                     st._decode_cb_host, st._decode_inv, ws.data_ptr(), ws.numel(), B, H * G, _lib.F16, _lib.F32, 128 ** -0.5)
+    token = torch.full((B, H, 128), 9.0, dtype=torch.float16, device="cuda")
+    out = torch.empty_like(want)
+    for _ in range(2):
+        _lib.check(_lib.lib.odmkv_decode_step(C.byref(step), q.data_ptr(), token.data_ptr(), token.data_ptr(), token.stride(0), token.stride(1),
+                                              128, out.data_ptr(), None, _lib.stream_ptr(out.device)))
+        assert torch.equal(out, want) and (st._bufs["seg_count"][4] == 64).all()
+    assert torch.equal(st.materialize()[0][:, :, :64], k[:, :, :64])
