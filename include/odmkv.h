@@ -228,7 +228,7 @@ typedef struct odmkv_packed {
  * (The per-level mask / nonzero of tq_adaptive_backend.py:355-361.) */
 int odmkv_level_counts(const int32_t* bits, int B, int Hkv, int T, int32_t* counts, void* stream);
 
-/* A layer's levels between the allocation and the store, in one pass over bits (device int32 [rows, T], 16-byte aligned;
+/* A layer's levels between the allocation and the store, in one pass over bits (device int32 [rows, T];
  * rows = B*Hkv): the tokens from tail_begin on are set to 16 bits (in bits too), the levels are written down as bytes
  * (device uint8 [rows, stride], T levels followed by 16s: what the store's level map reads behind the last token), and
  * they are counted: counts int32 [rows, odmkv_finish_levels_chunks(stride), 2, 6], device memory or page-locked host

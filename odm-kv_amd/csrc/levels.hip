@@ -18,6 +18,7 @@ struct LevelsArgs {
     int32_t* counts;                     // [rows, chunks, 2, 6]: tokens in [lo, hi) as allocated, and all of them as stored
     long long stride;
     int T, lo, hi, tail, chunks;
+    int vec;                             // every row of bits starts on a multiple of 16 bytes
 };
 
 // Bound by latency: 1 MB in, 0.26 MB out for a 32k-token layer of 8 heads.  One launch stands for the torch operations it
@@ -31,14 +32,13 @@ __global__ __launch_bounds__(LV_THREADS) void finish_levels_kernel(LevelsArgs a)
     int32_t* src = a.bits + (size_t)row * a.T;
     uint8_t* dst = a.levels + (size_t)row * a.stride;
     unsigned long long bulk = 0ull, all = 0ull;
-    const bool vec = (a.T & 3) == 0;                                  // rows keep the alignment of the first (checked on the host)
     const int end = min((long long)(chunk + 1) * LV_CHUNK, a.stride);
 #pragma unroll
     for (int u = 0; u < LV_CHUNK / (4 * LV_THREADS); ++u) {
         const int t = chunk * LV_CHUNK + (u * LV_THREADS + tid) * 4;
         if (t >= end) continue;
         int b[4] = {16, 16, 16, 16};
-        if (vec && t + 3 < a.T) {
+        if (a.vec && t + 3 < a.T) {
             const int4 v = *reinterpret_cast<const int4*>(src + t);
             b[0] = v.x; b[1] = v.y; b[2] = v.z; b[3] = v.w;
         } else {
@@ -74,9 +74,10 @@ extern "C" int odmkv_finish_levels(int32_t* bits, int rows, int T, int count_beg
                                    uint8_t* levels, int64_t stride, int32_t* counts, void* stream) {
     ODMKV_CHECK_ARG(bits && levels && counts, "finish_levels: null pointer");
     ODMKV_CHECK_ARG(rows > 0 && rows <= 65535 && T > 0, "finish_levels: bad shape rows=%d T=%d", rows, T);
-    ODMKV_CHECK_ARG(stride >= T && stride % 4 == 0 && stride < (1ll << 31) && ((uintptr_t)levels & 3) == 0 && ((uintptr_t)bits & 15) == 0,
+    ODMKV_CHECK_ARG(stride >= T && stride % 4 == 0 && stride < (1ll << 31) && ((uintptr_t)levels & 3) == 0 && ((uintptr_t)bits & 3) == 0,
                     "finish_levels: level rows must hold T tokens and start on multiples of four");
-    LevelsArgs a = {bits, levels, counts, (long long)stride, T, count_begin, count_end, tail_begin, level_chunks(stride)};
+    LevelsArgs a = {bits, levels, counts, (long long)stride, T, count_begin, count_end, tail_begin, level_chunks(stride),
+                    (T & 3) == 0 && ((uintptr_t)bits & 15) == 0};
     hipLaunchKernelGGL(finish_levels_kernel, dim3(a.chunks, rows), dim3(LV_THREADS), 0, (hipStream_t)stream, a);
     ODMKV_CHECK_LAUNCH("finish_levels_kernel");
     return 0;

@@ -37,3 +37,44 @@ def test_levels_counted_overridden_and_written_down(B, H, T, tail):
         _lib.check(_lib.lib.odmkv_evicted_indices(levels.data_ptr(), B, H, T, room, n, out.data_ptr(), ws.data_ptr(), ws.numel(),
                                                   _lib.stream_ptr(dev.device)))
         assert all(torch.equal(a.cpu(), b) for a, b in zip(out, want))
+
+
+@pytest.mark.parametrize("T,skip", [(4, 1), (4096, 2), (4097, 2), (8200, 3), (8200, 4)])
+def test_levels_that_start_anywhere(T, skip):
+    # (a group of layers inside one allocation: its first row starts where the layers before it end)
+    from kvquant import _lib
+    g = torch.Generator().manual_seed(T + skip)
+    bits = LEVELS[torch.randint(0, 6, (3, T), generator=g)].to(torch.int32)
+    dev = torch.zeros(skip + 3 * T, dtype=torch.int32, device="cuda")
+    dev[skip:] = bits.reshape(-1).cuda()
+    room = (T + 3) & ~3
+    levels = torch.empty((3, room), dtype=torch.uint8, device="cuda")
+    counts = torch.full((3, _lib.lib.odmkv_finish_levels_chunks(room), 2, 6), -1, dtype=torch.int32, pin_memory=True)
+    _lib.check(_lib.lib.odmkv_finish_levels(dev.data_ptr() + 4 * skip, 3, T, 1, T, T - 3, levels.data_ptr(), room, counts.data_ptr(),
+                                            _lib.stream_ptr(dev.device)))
+    torch.cuda.synchronize()
+    bulk = torch.stack([(bits[:, 1:] == b).sum(-1) for b in LEVELS.tolist()], dim=-1)
+    bits[:, T - 3:] = 16
+    assert torch.equal(dev[skip:].cpu(), bits.reshape(-1)) and (dev[:skip] == 0).all() and torch.equal(levels[:, :T].cpu().int(), bits)
+    assert torch.equal(counts.sum(dim=1)[:, 0].long(), bulk)
+    assert torch.equal(counts.sum(dim=1)[:, 1].long(), torch.stack([(bits == b).sum(-1) for b in LEVELS.tolist()], dim=-1))
+
+
+def test_a_prompt_whose_first_layer_stays_in_fp16_has_groups_that_start_anywhere():
+    # two kv-heads of 333 tokens: the second layer's levels start 8 bytes off a multiple of 16
+    from types import SimpleNamespace
+    from kvquant import RiskScorer, TurboQuantPerTokenBackendPress
+    scorer = RiskScorer(n_future_positions=16, n_sink=4, epsilon=1e-2)
+    scorer.normalize_grain = "global"
+    press = TurboQuantPerTokenBackendPress(scorer=scorer, bit_levels=(0, 2, 3, 4, 8, 16), target_avg_bits=2.0, eviction_cost=0.5,
+                                           key_quantizer="mse", value_quantizer="mse", sink_tokens=4, layerwise=True, buffer_size=128,
+                                           initial_layers_fp16=1)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    k, v = (torch.randn(1, 2, 333, 128, generator=g, device="cuda").half() for _ in range(2))
+    cache = SimpleNamespace(layers=[SimpleNamespace(keys=k.clone(), values=v.clone()) for _ in range(2)])
+    press._head_dim = 128
+    press._prefill_scores = {i: torch.rand(1, 2, 333, generator=g, device="cuda") for i in range(2)}
+    press._finalize_prefill(cache)
+    assert press._states[0].level_counts()[16] == 2 * 333
+    counts = press._states[1].level_counts()
+    assert sum(counts.values()) == 2 * 333 and counts[16] < 2 * 333 and not press._states[1].masked_key_indices() is None
