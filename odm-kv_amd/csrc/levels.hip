@@ -5,6 +5,7 @@
 
 #define LV_THREADS 256
 #define LV_CHUNK 4096           // tokens per workgroup: sixteen per thread
+#define LV_MAX_ROWS 65532       // rows of a launch (its y index): the largest multiple of four, so that each starts as aligned as the first
 
 // 6-bit counters of the six levels in one 64-bit word; a value that is no level adds nothing (as in pack.hip)
 __device__ static inline unsigned long long count_of(int bits) {
@@ -73,13 +74,17 @@ extern "C" int odmkv_finish_levels_chunks(int64_t stride) { return stride > 0 ? 
 extern "C" int odmkv_finish_levels(int32_t* bits, int rows, int T, int count_begin, int count_end, int tail_begin,
                                    uint8_t* levels, int64_t stride, int32_t* counts, void* stream) {
     ODMKV_CHECK_ARG(bits && levels && counts, "finish_levels: null pointer");
-    ODMKV_CHECK_ARG(rows > 0 && rows <= 65535 && T > 0, "finish_levels: bad shape rows=%d T=%d", rows, T);
+    ODMKV_CHECK_ARG(rows > 0 && T > 0, "finish_levels: bad shape rows=%d T=%d", rows, T);
     ODMKV_CHECK_ARG(stride >= T && stride % 4 == 0 && stride < (1ll << 31) && ((uintptr_t)levels & 3) == 0 && ((uintptr_t)bits & 3) == 0,
                     "finish_levels: level rows must hold T tokens and start on multiples of four");
     LevelsArgs a = {bits, levels, counts, (long long)stride, T, count_begin, count_end, tail_begin, level_chunks(stride),
                     (T & 3) == 0 && ((uintptr_t)bits & 15) == 0};
-    hipLaunchKernelGGL(finish_levels_kernel, dim3(a.chunks, rows), dim3(LV_THREADS), 0, (hipStream_t)stream, a);
-    ODMKV_CHECK_LAUNCH("finish_levels_kernel");
+    for (int r0 = 0; r0 < rows; r0 += LV_MAX_ROWS) {                  // (32 layers x 256 sequences x 8 heads are 65536 rows)
+        const int n = std::min(rows - r0, LV_MAX_ROWS);
+        hipLaunchKernelGGL(finish_levels_kernel, dim3(a.chunks, n), dim3(LV_THREADS), 0, (hipStream_t)stream, a);
+        ODMKV_CHECK_LAUNCH("finish_levels_kernel");
+        a.bits += (size_t)n * T; a.levels += (size_t)n * stride; a.counts += (size_t)n * a.chunks * 12;
+    }
     return 0;
 }
 

@@ -78,3 +78,20 @@ def test_a_prompt_whose_first_layer_stays_in_fp16_has_groups_that_start_anywhere
     assert press._states[0].level_counts()[16] == 2 * 333
     counts = press._states[1].level_counts()
     assert sum(counts.values()) == 2 * 333 and counts[16] < 2 * 333 and not press._states[1].masked_key_indices() is None
+
+
+@pytest.mark.parametrize("rows,T", [(65532, 4), (65533, 3), (65536, 4), (131073, 1)])
+def test_more_rows_than_a_launch_takes(rows, T):
+    from kvquant import _lib
+    g = torch.Generator().manual_seed(rows)
+    bits = LEVELS[torch.randint(0, 6, (rows, T), generator=g)].to(torch.int32)
+    dev = bits.cuda()
+    levels = torch.empty((rows, 8), dtype=torch.uint8, device="cuda")
+    counts = torch.full((rows, 1, 2, 6), -1, dtype=torch.int32, pin_memory=True)
+    _lib.check(_lib.lib.odmkv_finish_levels(dev.data_ptr(), rows, T, 0, T, T - 1, levels.data_ptr(), 8, counts.data_ptr(),
+                                            _lib.stream_ptr(dev.device)))
+    torch.cuda.synchronize()
+    assert torch.equal(counts[:, 0, 0].long(), torch.stack([(bits == b).sum(-1) for b in LEVELS.tolist()], dim=-1))
+    bits[:, T - 1:] = 16
+    assert torch.equal(dev.cpu(), bits) and torch.equal(levels[:, :T].cpu().int(), bits) and (levels[:, T:] == 16).all()
+    assert torch.equal(counts[:, 0, 1].long(), torch.stack([(bits == b).sum(-1) for b in LEVELS.tolist()], dim=-1))
