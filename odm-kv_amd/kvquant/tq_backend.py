@@ -223,13 +223,19 @@ class TurboQuantMSE:
         return MSEQuantized(indices=indices, norms=norms, bits=self.bits)
 
     def dequantize(self, q: MSEQuantized) -> torch.Tensor:
+        if q.bits not in SUPPORTED_WIDTHS:
+            raise ValueError(f"bit width {q.bits} is not one of {SUPPORTED_WIDTHS}")
+        _lib.require_gpu(q.indices, "indices")
+        _lib.require_gpu(q.norms, "norms")
         row_bytes = self.dim // _container(q.bits)[0]
-        if q.bits not in SUPPORTED_WIDTHS or q.indices.shape[-1] != row_bytes:
+        if q.indices.shape[-1] < row_bytes or (q.bits == 8 and q.indices.shape[-1] != row_bytes):
             raise ValueError(f"indices of shape {tuple(q.indices.shape)} do not hold {self.dim} codes of {q.bits} bits")
-        flat = q.indices.reshape(-1, row_bytes).contiguous()
+        # (container bytes in a wider type count as bytes, padding behind a row's codes is left out: as in _unpack_indices)
+        indices = q.indices[..., :row_bytes].to(torch.uint8)
+        flat = indices.reshape(-1, row_bytes).contiguous()
         norms = q.norms.float().reshape(-1).contiguous()
         out = torch.empty(flat.shape[0], self.dim, dtype=torch.float32, device=flat.device)
         _lib.check(lib.odmkv_dequantize_rows_packed(
             flat.data_ptr(), norms.data_ptr(), flat.shape[0], q.bits, self.pi.data_ptr(),
             self.centroids.data_ptr(), out.data_ptr(), _lib.stream_ptr(flat.device)))
-        return out.reshape(*q.indices.shape[:-1], self.dim)
+        return out.reshape(*indices.shape[:-1], self.dim)

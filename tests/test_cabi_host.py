@@ -226,3 +226,13 @@ def test_store_finish_staged_sizes_the_store_without_a_gpu(lib):
     rc = f(chunks.ctypes.data, n_chunks, B, H, T, slack, 0, 0, None, 0, C.byref(staging), counts.ctypes.data,
            seg_tile.ctypes.data, off, size, marks, C.byref(store), C.byref(need), None)
     assert rc == -1 and b"must take values" in lib.odmkv_last_error()
+
+
+def test_rows_on_the_cpu_are_refused():
+    import torch
+    from kvquant.tq_backend import MSEQuantized, TurboQuantMSE
+    q = TurboQuantMSE(128, 2, device="cpu", dtype=torch.float16)
+    with pytest.raises(RuntimeError, match="must live on the GPU"):
+        q.quantize(torch.zeros(3, 128, dtype=torch.float16))
+    with pytest.raises(RuntimeError, match="must live on the GPU"):
+        q.dequantize(MSEQuantized(torch.zeros(3, 32, dtype=torch.uint8), torch.ones(3), 2))

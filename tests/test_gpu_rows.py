@@ -51,3 +51,19 @@ def test_round_trip_in_place(B, H, T, lo, hi, bits, dtype):
     for got, y in zip((got_k, got_v), want):
         assert torch.equal(got[:, :, :lo], y[:, :, :lo]) and torch.equal(got[:, :, hi:], y[:, :, hi:])
         assert ((got.float() - y.float()).abs() <= step * y.float().abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("kind", [torch.uint8, torch.int16, torch.int32, torch.int64])
+@pytest.mark.parametrize("bits,pad", [(2, 0), (3, 0), (4, 5), (8, 0), (2, 3)])
+def test_indices_in_wider_types_and_padded_rows(bits, pad, kind):
+    from kvquant.tq_backend import MSEQuantized, TurboQuantMSE, _unpack_indices
+    x = _rows(70, torch.float16, bits)
+    x[5, 7], x[6, 9] = 1.0, 2.0
+    q = TurboQuantMSE(128, bits, device="cuda", dtype=x.dtype, seed=7)
+    got = q.quantize(x.view(2, 35, 128))
+    want = q.dequantize(got)
+    indices = torch.cat([got.indices.to(kind), torch.full((2, 35, pad), 85, dtype=kind, device="cuda")], dim=-1)
+    assert torch.equal(_unpack_indices(indices, bits, 128), _unpack_indices(got.indices, bits, 128))
+    assert torch.equal(q.dequantize(MSEQuantized(indices, got.norms, bits)), want)
+    with pytest.raises(ValueError):
+        q.dequantize(MSEQuantized(got.indices[..., :-1], got.norms, bits))
