@@ -408,7 +408,8 @@ class WindowRiskScorer(RiskScorer):
             return self._fallback.score_prefill(keys, values, layer_idx)
         p = _launch_window_attention(keys, queries, self.n_sink, T - w, D ** -0.5)
         core = _launch_score(keys[:, self.n_sink:], values[:, self.n_sink:], None, p, H, 0, self.epsilon)
-        if self.normalize_grain in ("layer", "global"):
+        plain = type(self)._maybe_normalize is BaseScorer._maybe_normalize and "_maybe_normalize" not in self.__dict__
+        if plain and self.normalize_grain in ("layer", "global"):
             return _scale_on_device(core, self.n_sink, self.normalize_grain == "layer")
         top = core.max().reshape(1, 1).expand(H, self.n_sink)
         return self._maybe_normalize(torch.cat([top, core], dim=1))

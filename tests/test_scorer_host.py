@@ -72,3 +72,32 @@ def test_a_prompt_spread_over_devices_is_left_to_the_general_path(away, monkeypa
             call()
     else:
         assert call() is None
+
+
+@pytest.mark.parametrize("where", ["class", "instance", "nowhere"])
+@pytest.mark.parametrize("grain", ["layer", "global", "head"])
+def test_a_window_scorers_own_normalisation_is_asked(grain, where, monkeypatch):
+    import torch
+    from types import SimpleNamespace
+    from kvquant import WindowRiskScorer, scorer as sc
+    core = torch.arange(12.0).reshape(2, 6)
+
+    class Halved(WindowRiskScorer):
+        def _maybe_normalize(self, raw):
+            return raw / 2
+
+    scorer = (Halved if where == "class" else WindowRiskScorer)(window=4, n_future_positions=8, n_sink=2, epsilon=1e-2)
+    if where == "instance":
+        scorer._maybe_normalize = lambda raw: raw / 2
+    scorer.normalize_grain = grain
+    monkeypatch.setattr(sc, "_launch_window_attention", lambda *a: None)
+    monkeypatch.setattr(sc, "_launch_score", lambda *a: core)
+    monkeypatch.setattr(sc, "_scale_on_device", lambda scores, pad, scale: "on the device")
+    monkeypatch.setattr(scorer, "_window_queries", lambda module, h, w: None)
+    keys = torch.zeros(2, 8, 128)
+    got = scorer.score_prefill(keys, keys, 0, module=SimpleNamespace(), hidden_states=torch.zeros(1, 8, 64))
+    padded = torch.cat([torch.full((2, 2), 11.0), core], dim=1)
+    if where == "nowhere":
+        assert got == "on the device" if grain != "head" else torch.equal(got, sc._normalize_scores(padded, grain=grain))
+    else:
+        assert torch.equal(got, padded / 2)
