@@ -6,6 +6,7 @@
 // (1 KB contiguous for a dense cache) per load instruction.  All reductions run in a fixed
 // order (shuffle butterflies, then ordered sums over chunk partials): results do not depend
 // on scheduling.
+#include <algorithm>
 #include "common.h"
 
 #define ROWS_PER_WG 256     // rows of one kv-head handled by a 256-thread workgroup
@@ -1071,8 +1072,42 @@ static PromptLayout prompt_layout(int B, int T, int hidden, int Hq, int Hkv) {
     return L;
 }
 
+// Sequences of one turn: as many as keep the workspace (mostly logits and partial sums, 34 MB for a sequence of 131072 tokens
+// and 32 query heads) within this, one at least.  Where that splits a batch its sequences are long, and what a turn repeats
+// (a pass over the weight and the RoPE tables, 14 us) is small beside them.
+#define PROMPT_WORKSPACE (64u << 20)
+static int prompt_turn(int B, int T, int hidden, int Hq, int Hkv) {
+    const size_t one = prompt_layout(1, T, hidden, Hq, Hkv).total;
+    return (int)std::max<size_t>(1, std::min<size_t>({(size_t)B, PROMPT_WORKSPACE / one, 65535u / (unsigned)Hkv}));
+}
+
 extern "C" size_t odmkv_prompt_scores_workspace_bytes(int B, int T, int hidden, int Hq, int Hkv) {
-    return B > 0 && T > 0 && hidden > 0 && Hq > 0 && Hkv > 0 ? prompt_layout(B, T, hidden, Hq, Hkv).total : 0;
+    if (B <= 0 || T <= 0 || hidden <= 0 || Hq <= 0 || Hkv <= 0) return 0;
+    return prompt_layout(prompt_turn(B, T, hidden, Hq, Hkv), T, hidden, Hq, Hkv).total;
+}
+
+// B sequences of *p, the first of them sequence b0
+static int prompt_scores(const odmkv_prompt_t* p, int b0, int B, void* stream) {
+    const PromptLayout L = prompt_layout(B, p->T, p->hidden, p->Hq, p->Hkv);
+    char* ws = (char*)p->workspace;
+    const char* h0 = (const char*)p->hidden_states + ((long long)b0 * p->h_stride_b + (long long)p->n_sink * p->h_stride_t) * 2;
+    if (int rc = odmkv_token_mean(h0, p->dtype, B, p->T - p->n_sink, p->hidden, p->h_stride_b, p->h_stride_t, ws + L.mean,
+                                  ws + L.mean_ws, L.q - L.mean_ws, stream)) return rc;
+    float* mu = (float*)(ws + L.mu);
+    if (int rc = odmkv_project_rows(p->weight, p->ld_weight, p->bias, ws + L.mean, p->dtype, B, p->Hq * HD, p->hidden,
+                                    p->cosine ? (void*)(ws + L.q) : (void*)mu, p->cosine ? p->dtype : ODMKV_F32, stream)) return rc;
+    if (p->cosine)
+        if (int rc = odmkv_average_rope(ws + L.q, p->cosine, p->sine, p->dtype, B * p->Hq, p->positions, mu, stream)) return rc;
+    const size_t elem = p->kv_dtype == ODMKV_F32 ? 4 : 2;
+    const bool together = B == 1 || p->stride_b == p->Hkv * p->stride_h;
+    for (int b = 0; b < B; b += together ? B : 1) {
+        const int n = together ? B : 1;
+        const long long at = (long long)(b0 + b) * p->stride_b * (long long)elem;
+        if (int rc = score_heads((const char*)p->K + at, (const char*)p->V + at, p->kv_dtype, n * p->Hkv, p->Hkv, p->T, p->stride_h, p->stride_t,
+                                 mu + (size_t)b * p->Hq * HD, n * p->Hq, nullptr, p->n_sink, p->eps, p->round_dtype,
+                                 p->scores + (size_t)(b0 + b) * p->Hkv * p->T, ws + L.score, p->workspace_bytes - L.score, stream)) return rc;
+    }
+    return 0;
 }
 
 extern "C" int odmkv_prompt_scores(const odmkv_prompt_t* p, void* stream) {
@@ -1083,26 +1118,9 @@ extern "C" int odmkv_prompt_scores(const odmkv_prompt_t* p, void* stream) {
     ODMKV_CHECK_ARG(p->B > 0 && p->T > p->n_sink && p->n_sink >= 0 && p->hidden > 0 && p->Hkv > 0 && p->Hq > 0 && p->Hq % p->Hkv == 0
                     && (!p->cosine || p->positions > 0), "prompt_scores: bad shape");
     ODMKV_CHECK_ARG(p->workspace_bytes >= odmkv_prompt_scores_workspace_bytes(p->B, p->T, p->hidden, p->Hq, p->Hkv), "prompt_scores: workspace too small");
-    const PromptLayout L = prompt_layout(p->B, p->T, p->hidden, p->Hq, p->Hkv);
-    char* ws = (char*)p->workspace;
-    const char* h0 = (const char*)p->hidden_states + (size_t)p->n_sink * p->h_stride_t * 2;
-    if (int rc = odmkv_token_mean(h0, p->dtype, p->B, p->T - p->n_sink, p->hidden, p->h_stride_b, p->h_stride_t, ws + L.mean,
-                                  ws + L.mean_ws, L.q - L.mean_ws, stream)) return rc;
-    float* mu = (float*)(ws + L.mu);
-    if (int rc = odmkv_project_rows(p->weight, p->ld_weight, p->bias, ws + L.mean, p->dtype, p->B, p->Hq * HD, p->hidden,
-                                    p->cosine ? (void*)(ws + L.q) : (void*)mu, p->cosine ? p->dtype : ODMKV_F32, stream)) return rc;
-    if (p->cosine)
-        if (int rc = odmkv_average_rope(ws + L.q, p->cosine, p->sine, p->dtype, p->B * p->Hq, p->positions, mu, stream)) return rc;
-    if (p->B == 1 || p->stride_b == p->Hkv * p->stride_h)
-        return score_heads(p->K, p->V, p->kv_dtype, p->B * p->Hkv, p->Hkv, p->T, p->stride_h, p->stride_t, mu, p->B * p->Hq, nullptr,
-                           p->n_sink, p->eps, p->round_dtype, p->scores, ws + L.score, p->workspace_bytes - L.score, stream);
-    const size_t elem = p->kv_dtype == ODMKV_F32 ? 4 : 2;
-    for (int b = 0; b < p->B; ++b) {
-        const size_t at = (size_t)b * p->stride_b * elem;
-        if (int rc = score_heads((const char*)p->K + at, (const char*)p->V + at, p->kv_dtype, p->Hkv, p->Hkv, p->T, p->stride_h, p->stride_t,
-                                 mu + (size_t)b * p->Hq * HD, p->Hq, nullptr, p->n_sink, p->eps, p->round_dtype,
-                                 p->scores + (size_t)b * p->Hkv * p->T, ws + L.score, p->workspace_bytes - L.score, stream)) return rc;
-    }
+    const int turn = prompt_turn(p->B, p->T, p->hidden, p->Hq, p->Hkv);
+    for (int b = 0; b < p->B; b += turn)
+        if (int rc = prompt_scores(p, b, std::min(turn, p->B - b), stream)) return rc;
     return 0;
 }
 

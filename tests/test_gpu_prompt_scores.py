@@ -62,3 +62,11 @@ def test_scores_of_all_sequences(B, Hq, Hkv, T, dtype, gap, rope):
 @pytest.mark.parametrize("T", [8193, 8196, 8197])
 def test_prompts_whose_mean_is_cut_otherwise_without_the_sinks(T):
     test_scores_of_all_sequences(2, 4, 2, T, torch.float16, 0, True)
+
+
+@pytest.mark.parametrize("gap", [0, 1])
+def test_a_batch_scored_in_turns(gap):
+    # 4.2 MB of workspace a sequence, 15 sequences a turn (64 MB)
+    from kvquant import _lib
+    assert _lib.lib.odmkv_prompt_scores_workspace_bytes(17, 100001, 256, 8, 1) < 17 * _lib.lib.odmkv_prompt_scores_workspace_bytes(1, 100001, 256, 8, 1) / 1.1
+    test_scores_of_all_sequences(17, 8, 1, 100001, torch.float16, gap, True)

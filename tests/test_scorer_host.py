@@ -101,3 +101,14 @@ def test_a_window_scorers_own_normalisation_is_asked(grain, where, monkeypatch):
         assert got == "on the device" if grain != "head" else torch.equal(got, sc._normalize_scores(padded, grain=grain))
     else:
         assert torch.equal(got, padded / 2)
+
+
+def test_a_batch_of_long_prompts_does_not_grow_the_workspace():
+    from kvquant import _lib
+    need = _lib.lib.odmkv_prompt_scores_workspace_bytes
+    for T, hidden, n_q, n_kv in ((131072, 4096, 32, 8), (32768, 3584, 28, 4), (4096, 2048, 16, 2), (100, 1024, 8, 8)):
+        one = need(1, T, hidden, n_q, n_kv)
+        assert one > T * (n_q + n_kv) * 4
+        for B in (2, 3, 16, 64, 300, 9000):
+            assert need(B, T, hidden, n_q, n_kv) <= max(one, 64 << 20)
+    assert need(2, 8192, 4096, 32, 8) > need(1, 8192, 4096, 32, 8)          # (short ones are still scored together)
