@@ -223,10 +223,13 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
         arrived = {}
         groups = []                 # layers whose bits lie one behind the other share a launch: [device, T, tail, bits of each]
         order = []
+        # the window is written into the levels below: into a copy where they may be somebody else's as well
+        ours = (type(self)._allocate_bits_for_prefill is TurboQuantPerTokenPress._allocate_bits_for_prefill
+                and "_allocate_bits_for_prefill" not in self.__dict__)
         for layer_idx, bits in self._allocate_bits_for_prefill().items():
             keys, _ = self._get_cache_tensors(cache, layer_idx)
             dev, T = keys.device, bits.shape[2]
-            bits = bits.to(dtype=torch.int32, device=dev).contiguous()
+            bits = bits.to(dtype=torch.int32, device=dev, copy=not ours).contiguous()
             tail = 0 if layer_idx < self.initial_layers_fp16 else T - min(max(self.buffer_size, 0), T)
             last = groups[-1] if groups else None
             if not (last and last[:3] == [dev, T, tail] and last[3][0].shape == bits.shape

@@ -95,3 +95,25 @@ def test_more_rows_than_a_launch_takes(rows, T):
     bits[:, T - 1:] = 16
     assert torch.equal(dev.cpu(), bits) and torch.equal(levels[:, :T].cpu().int(), bits) and (levels[:, T:] == 16).all()
     assert torch.equal(counts[:, 0, 1].long(), torch.stack([(bits == b).sum(-1) for b in LEVELS.tolist()], dim=-1))
+
+
+def test_levels_that_a_subclass_keeps_are_left_as_they_were():
+    from types import SimpleNamespace
+    from kvquant import RiskScorer, TurboQuantPerTokenBackendPress
+
+    class Keeping(TurboQuantPerTokenBackendPress):
+        def _allocate_bits_for_prefill(self):
+            self.kept = super()._allocate_bits_for_prefill()
+            self.copies = {i: b.clone() for i, b in self.kept.items()}
+            return self.kept
+
+    press = Keeping(scorer=RiskScorer(n_future_positions=16, n_sink=4, epsilon=1e-2), bit_levels=(0, 2, 3, 4, 8, 16), target_avg_bits=2.0,
+                    eviction_cost=0.5, key_quantizer="mse", value_quantizer="mse", sink_tokens=4, layerwise=True, buffer_size=128)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    k, v = (torch.randn(1, 2, 400, 128, generator=g, device="cuda").half() for _ in range(2))
+    cache = SimpleNamespace(layers=[SimpleNamespace(keys=k.clone(), values=v.clone()) for _ in range(2)])
+    press._head_dim = 128
+    press._prefill_scores = {i: torch.rand(1, 2, 400, generator=g, device="cuda") for i in range(2)}
+    press._finalize_prefill(cache)
+    assert all(torch.equal(press.kept[i], press.copies[i]) for i in range(2)) and (press.kept[0][..., -128:] != 16).any()
+    assert press._states[0].level_counts()[16] >= 2 * 128
