@@ -224,8 +224,7 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
         groups = []                 # layers whose bits lie one behind the other share a launch: [device, T, tail, bits of each]
         order = []
         # the window is written into the levels below: into a copy where they may be somebody else's as well
-        ours = (type(self)._allocate_bits_for_prefill is TurboQuantPerTokenPress._allocate_bits_for_prefill
-                and "_allocate_bits_for_prefill" not in self.__dict__)
+        ours = self._own_allocation()
         for layer_idx, bits in self._allocate_bits_for_prefill().items():
             keys, _ = self._get_cache_tensors(cache, layer_idx)
             dev, T = keys.device, bits.shape[2]

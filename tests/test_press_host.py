@@ -229,3 +229,18 @@ def test_a_scorer_assigned_after_construction_scores_the_next_prompt():
     press._prefill_hook(torch.nn.Module(), None, torch.zeros(2, 10, 64), 1, keys, keys)
     assert (first.calls, second.calls) == (1, 1)
     assert (press._prefill_scores[0] == 1.0).all() and (press._prefill_scores[1] == 2.0).all()
+
+
+def test_an_overridden_allocation_finds_the_sink_masks():
+    from kvquant import TurboQuantPerTokenPress
+    seen = {}
+
+    class Own(TurboQuantPerTokenPress):
+        def _allocate_bits_for_prefill(self):
+            seen.update(self._prefill_sink_masks)
+            return {}
+
+    press = Own(scorer=_CountingScorer(1.0), bit_levels=(0, 2, 4, 16), value_quantizer="mse", layerwise=True, target_avg_bits=2.0, sink_tokens=4)
+    keys = torch.zeros(1, 3, 10, 128)
+    press._prefill_hook(torch.nn.Module(), None, torch.zeros(1, 10, 64), 0, keys, keys)
+    assert torch.equal(seen[0], torch.arange(10).expand(3, 10) < 4)
