@@ -67,3 +67,29 @@ def test_indices_in_wider_types_and_padded_rows(bits, pad, kind):
     assert torch.equal(q.dequantize(MSEQuantized(indices, got.norms, bits)), want)
     with pytest.raises(ValueError):
         q.dequantize(MSEQuantized(got.indices[..., :-1], got.norms, bits))
+
+
+def test_rows_that_are_shared_or_recorded_are_refused_as_by_torch():
+    from kvquant import TurboQuantBackendPress
+    press = TurboQuantBackendPress(key_bits=3, value_bits=2, value_quantizer="mse")
+    make = lambda heads=2, **kw: torch.randn(1, heads, 40, 128, device="cuda", dtype=torch.float16, **kw)
+    for k, v in ((make(1).expand(1, 2, 40, 128), make(1).expand(1, 2, 40, 128)),              # one row for two heads
+                 (make(requires_grad=True), make()), (make(), make(requires_grad=True))):     # leaves of a graph
+        before = k.detach().clone()
+        with pytest.raises(RuntimeError):
+            press._quantise_span(0, k, v, 0, 30)
+            torch.cuda.synchronize()
+        assert not k.requires_grad or torch.equal(k.detach(), before)
+    # and what a gradient is recorded for is recorded: the quantised rows pass none on
+    k, leaf = make(), make(requires_grad=True)
+    values = leaf * 1.0
+    press._quantise_span(0, k, values, 0, 30)
+    values.float().sum().backward()
+    assert (leaf.grad[:, :, :30] == 0).all() and (leaf.grad[:, :, 30:] == 1).all()
+    # [B, T, H, D] in memory, as a projection leaves it
+    k = torch.randn(1, 40, 2, 128, device="cuda", dtype=torch.float16).transpose(1, 2)
+    a, b = k.contiguous(), k.contiguous()
+    press._quantise_span(0, a, b, 0, 30)
+    v = k.contiguous().transpose(1, 2).contiguous().transpose(1, 2)
+    press._quantise_span(0, k, v, 0, 30)
+    assert torch.equal(k, a) and torch.equal(v, b)

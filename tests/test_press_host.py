@@ -244,3 +244,19 @@ def test_an_overridden_allocation_finds_the_sink_masks():
     keys = torch.zeros(1, 3, 10, 128)
     press._prefill_hook(torch.nn.Module(), None, torch.zeros(1, 10, 64), 0, keys, keys)
     assert torch.equal(seen[0], torch.arange(10).expand(3, 10) < 4)
+
+
+def test_the_uniform_press_refuses_cpu_tensors(monkeypatch):
+    from types import SimpleNamespace
+    from kvquant import TurboQuantBackendPress, backend_press
+
+    def launched(*args):
+        raise AssertionError("addresses of host memory handed to a kernel")
+
+    monkeypatch.setattr(backend_press, "_lib", SimpleNamespace(
+        lib=SimpleNamespace(odmkv_round_trip_workspace_bytes=lambda n: 1, odmkv_round_trip_rows=launched),
+        workspace=lambda *a: torch.empty(1), stream_ptr=lambda d: 0, check=lambda rc: None, dtype_code=lambda t: 0))
+    press = TurboQuantBackendPress(key_bits=3, value_bits=2, value_quantizer="mse")
+    k, v = torch.zeros(1, 2, 20, 128, dtype=torch.float16), torch.zeros(1, 2, 20, 128, dtype=torch.float16)
+    with pytest.raises(RuntimeError, match="must live on the GPU"):
+        press._quantise_span(0, k, v, 0, 10)
