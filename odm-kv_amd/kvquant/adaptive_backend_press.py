@@ -286,7 +286,8 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
         # the usual decode step: the attention call has stored the token natively, the buffer grows by one
         layer_idx = getattr(module, "layer_idx", None)
         state = self._states.get(layer_idx)
-        if state is not None and state._fast is not None and state.exact_decode_append and module.__dict__.get("_odmkv_state") is state:
+        if (state is not None and state._fast is not None and state.exact_decode_append and module.__dict__.get("_odmkv_state") is state
+                and self.decode_quant and layer_idx >= self.initial_layers_fp16):
             cache, hidden_states = kwargs.get("past_key_values"), kwargs.get("hidden_states")
             if cache is not None and hidden_states is not None and hidden_states.shape[1] == 1:
                 layers = getattr(cache, "layers", None)

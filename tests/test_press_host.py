@@ -260,3 +260,21 @@ def test_the_uniform_press_refuses_cpu_tensors(monkeypatch):
     k, v = torch.zeros(1, 2, 20, 128, dtype=torch.float16), torch.zeros(1, 2, 20, 128, dtype=torch.float16)
     with pytest.raises(RuntimeError, match="must live on the GPU"):
         press._quantise_span(0, k, v, 0, 10)
+
+
+@pytest.mark.parametrize("decode_quant,fp16_layers,counted", [(True, 0, True), (False, 0, False), (True, 1, False)])
+def test_the_short_way_through_the_hook_counts_what_the_long_way_counts(decode_quant, fp16_layers, counted):
+    from types import SimpleNamespace
+    from kvquant import TurboQuantPerTokenBackendPress
+    press = TurboQuantPerTokenBackendPress(scorer=_scorer(), bit_levels=(0, 2, 4, 16), key_quantizer="mse", value_quantizer="mse",
+                                           target_avg_bits=2.0, initial_layers_fp16=fp16_layers)
+    press.decode_quant = decode_quant
+    for fast in (object(), None):                             # a store with the native step armed, and one without
+        state = SimpleNamespace(_fast=fast, exact_decode_append=True, seq_len=41)
+        press._states, press._buffer_counts, press._buffer_start_seqs = {0: state}, {}, {0: 40}
+        module = torch.nn.Module()
+        module.layer_idx, module._odmkv_state = 0, state
+        keys = torch.zeros(1, 2, 41, 8)
+        cache = SimpleNamespace(layers=[SimpleNamespace(keys=keys, values=keys, _tq_backend_state=state)])
+        press._forward_hook(module, (), {"past_key_values": cache, "hidden_states": torch.zeros(1, 1, 16)}, None)
+        assert press._buffer_counts.get(0, 0) == int(counted)
