@@ -237,26 +237,29 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
             groups[-1][3].append(bits)
             order.append(layer_idx)
         evicted = []                # per group: level maps of its layers
-        for dev, T, tail, members in groups:
-            # one pass over the levels: bulk shares counted, the window (or the whole layer) set to 16, the level map
-            # written; the counts go straight to page-locked memory, and all layers share the one wait below
-            n, (B, H, _) = len(members), members[0].shape
-            room = (T + 2 * self.buffer_size + 255) & ~255
-            levels = torch.empty((n, B, H, room), dtype=torch.uint8, device=dev)
-            chunks = _lib.lib.odmkv_finish_levels_chunks(room)
-            counts = torch.empty((n, B * H, chunks, 2, 6), dtype=torch.int32, pin_memory=True)
-            start, end = self._bulk(T)
-            with torch.cuda.device(dev):
-                _lib.check(_lib.lib.odmkv_finish_levels(members[0].data_ptr(), n * B * H, T, start, end, tail, levels.data_ptr(), room,
-                                                        counts.data_ptr(), _lib.stream_ptr(dev)))
-                ev = arrived.setdefault(dev, torch.cuda.Event())
-                ev.record(torch.cuda.current_stream(dev))
-            plan.extend(zip(order[len(plan):], members, levels, counts))
-            evicted.append((levels, T))
-        for layer_idx, *_ in plan:                                # (the host's part while the counts are on their way)
-            self._get_or_create_state(layer_idx, self._get_cache_tensors(cache, layer_idx)[0])
-        for ev in arrived.values():
-            ev.synchronize()
+        try:
+            for dev, T, tail, members in groups:
+                # one pass over the levels: bulk shares counted, the window (or the whole layer) set to 16, the level map
+                # written; the counts go straight to page-locked memory, and all layers share the one wait below
+                n, (B, H, _) = len(members), members[0].shape
+                room = (T + 2 * self.buffer_size + 255) & ~255
+                levels = torch.empty((n, B, H, room), dtype=torch.uint8, device=dev)
+                chunks = _lib.lib.odmkv_finish_levels_chunks(room)
+                counts = torch.empty((n, B * H, chunks, 2, 6), dtype=torch.int32, pin_memory=True)
+                start, end = self._bulk(T)
+                with torch.cuda.device(dev):
+                    _lib.check(_lib.lib.odmkv_finish_levels(members[0].data_ptr(), n * B * H, T, start, end, tail, levels.data_ptr(), room,
+                                                            counts.data_ptr(), _lib.stream_ptr(dev)))
+                    ev = arrived.setdefault(dev, torch.cuda.Event())
+                    ev.record(torch.cuda.current_stream(dev))
+                plan.extend(zip(order[len(plan):], members, levels, counts))
+                evicted.append((levels, T))
+            for layer_idx, *_ in plan:                            # (the host's part while the counts are on their way)
+                self._get_or_create_state(layer_idx, self._get_cache_tensors(cache, layer_idx)[0])
+        finally:
+            # (also where a store cannot be made: the kernels write into page-locked memory that is given back on the way out)
+            for ev in arrived.values():
+                ev.synchronize()
         masked, at = [], 0
         totals = [counts.numpy().sum(axis=1).swapaxes(0, 1) for *_, counts in plan]      # (bulk, stored) of every layer
         for levels, T in evicted:

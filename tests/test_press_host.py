@@ -278,3 +278,30 @@ def test_the_short_way_through_the_hook_counts_what_the_long_way_counts(decode_q
         cache = SimpleNamespace(layers=[SimpleNamespace(keys=keys, values=keys, _tq_backend_state=state)])
         press._forward_hook(module, (), {"past_key_values": cache, "hidden_states": torch.zeros(1, 1, 16)}, None)
         assert press._buffer_counts.get(0, 0) == int(counted)
+
+
+def test_a_prefill_that_fails_waits_for_the_counts_it_asked_for(monkeypatch):
+    from types import SimpleNamespace
+    from kvquant import TurboQuantPerTokenBackendPress, _lib, adaptive_backend_press as abp
+    calls = []
+    monkeypatch.setattr(abp, "_lib", SimpleNamespace(
+        lib=SimpleNamespace(odmkv_finish_levels_chunks=lambda n: 1, odmkv_finish_levels=lambda *a: calls.append("launched") or 0),
+        check=_lib.check, stream_ptr=lambda d: 0, LEVEL_ORDER=_lib.LEVEL_ORDER))
+
+    class Event:
+        def record(self, stream): calls.append("recorded")
+        def synchronize(self): calls.append("waited")
+
+    empty = torch.empty
+    monkeypatch.setattr(abp.torch, "empty", lambda *a, pin_memory=False, **kw: empty(*a, **kw))
+    monkeypatch.setattr(abp.torch.cuda, "Event", Event)
+    monkeypatch.setattr(abp.torch.cuda, "current_stream", lambda d=None: None)
+    monkeypatch.setattr(abp.torch.cuda, "device", lambda d: __import__("contextlib").nullcontext())
+    press = TurboQuantPerTokenBackendPress(scorer=_scorer(), bit_levels=(0, 2, 4, 16), key_quantizer="mse", value_quantizer="mse",
+                                           target_avg_bits=2.0, layerwise=True)
+    press._allocate_bits_for_prefill = lambda: {0: torch.full((1, 2, 200), 2, dtype=torch.int32)}
+    keys = torch.zeros(1, 2, 200, 128)
+    cache = SimpleNamespace(layers=[SimpleNamespace(keys=keys, values=keys)])
+    with pytest.raises(RuntimeError, match="no CPU path"):        # the store lives on the GPU
+        press._finalize_prefill(cache)
+    assert calls == ["launched", "recorded", "waited"]
