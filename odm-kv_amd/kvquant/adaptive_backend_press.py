@@ -242,7 +242,7 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
                 # one pass over the levels: bulk shares counted, the window (or the whole layer) set to 16, the level map
                 # written; the counts go straight to page-locked memory, and all layers share the one wait below
                 n, (B, H, _) = len(members), members[0].shape
-                room = (T + 2 * self.buffer_size + 255) & ~255
+                room = (T + 2 * max(self.buffer_size, 0) + 255) & ~255
                 levels = torch.empty((n, B, H, room), dtype=torch.uint8, device=dev)
                 chunks = _lib.lib.odmkv_finish_levels_chunks(room)
                 counts = torch.empty((n, B * H, chunks, 2, 6), dtype=torch.int32, pin_memory=True)

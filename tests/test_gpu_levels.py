@@ -117,3 +117,18 @@ def test_levels_that_a_subclass_keeps_are_left_as_they_were():
     press._finalize_prefill(cache)
     assert all(torch.equal(press.kept[i], press.copies[i]) for i in range(2)) and (press.kept[0][..., -128:] != 16).any()
     assert press._states[0].level_counts()[16] >= 2 * 128
+
+
+@pytest.mark.parametrize("buffer_size", [-200, 0])
+def test_a_prompt_without_a_decode_buffer(buffer_size):
+    from types import SimpleNamespace
+    from kvquant import RiskScorer, TurboQuantPerTokenBackendPress
+    press = TurboQuantPerTokenBackendPress(scorer=RiskScorer(n_future_positions=16, n_sink=4, epsilon=1e-2), bit_levels=(0, 2, 3, 4, 8, 16),
+                                           target_avg_bits=2.0, key_quantizer="mse", value_quantizer="mse", sink_tokens=4, layerwise=True,
+                                           buffer_size=buffer_size)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    k, v = (torch.randn(1, 2, 300, 128, generator=g, device="cuda").half() for _ in range(2))
+    press._head_dim = 128
+    press._prefill_scores = {0: torch.rand(1, 2, 300, generator=g, device="cuda")}
+    press._finalize_prefill(SimpleNamespace(layers=[SimpleNamespace(keys=k, values=v)]))
+    assert sum(press._states[0].level_counts().values()) == 600
