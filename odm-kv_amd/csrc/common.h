@@ -43,6 +43,11 @@ void odmkv_set_error(const char* fmt, ...);
         }                                                                            \
     } while (0)
 
+// More than 64 KB of LDS for a kernel.  The attribute belongs to the function on the current device, so it is set before every
+// launch: layers of one model may live on several devices.
+#define ODMKV_ALLOW_LDS(kernel, bytes) \
+    ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(bytes)))
+
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // pack.hip: byte offset, inside the pack workspace, of the list of tiles the fp16 quantiser hands to the exact one
 size_t pack_redo_offset(int nseg, int T);

@@ -1551,12 +1551,7 @@ extern "C" size_t odmkv_pack_workspace_bytes(int B, int Hkv, int T) {
 template <int DT>
 static int launch_quant_f16(const QuantArgs& qa, hipStream_t st) {
     const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QP_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave) + (QF_MAX_RUNS + 1) * sizeof(int);
-    static bool attr_set = false;
-    if (!attr_set) {
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_pack_f16_kernel<DT>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
+    ODMKV_ALLOW_LDS((quant_pack_f16_kernel<DT>), lds);
     const int total = qa.tile_base[ODMKV_NQ];
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -1574,12 +1569,7 @@ static int launch_quant(const QuantArgs& qa, hipStream_t st) {
     // fp32 rows take 128 registers on top of the 128 accumulators: one wave per SIMD then
     constexpr int NW = (DT == ODMKV_F32) ? 4 : 8;
     const size_t lds = QP_PI_BYTES + (size_t)NW * QP_STAGE + QP_THR_FLOATS * sizeof(float);
-    static bool attr_set = false;
-    if (!attr_set) {
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_pack_kernel<DT, NW>),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
+    ODMKV_ALLOW_LDS((quant_pack_kernel<DT, NW>), lds);
     const int total = qa.tile_base[ODMKV_NQ];
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -2109,11 +2099,7 @@ static int compute_units() {
 
 template <int DT>
 static int launch_dequant(const DequantArgs& da, hipStream_t st) {
-    static bool attr_set = false;
-    if (!attr_set) {
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(dequant_kernel<DT>), hipFuncAttributeMaxDynamicSharedMemorySize, DQ_LDS));
-        attr_set = true;
-    }
+    ODMKV_ALLOW_LDS((dequant_kernel<DT>), DQ_LDS);
     // one persistent workgroup per compute unit, keys on the even and values on the odd ones; never
     // more workgroups than there are tiles for their waves
     const int need = (da.tile_base[ODMKV_NQ] + DQ_NW - 1) / DQ_NW, pairs = std::max(1, std::min(compute_units() / 2, need));
@@ -2334,12 +2320,8 @@ static dim3 rows_grid(const RowsJob* jobs, int n_jobs, int waves) {
 
 int launch_quantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
     const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QP_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave);
-    static bool attr_set = false;
-    if (!attr_set) {
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_f16_kernel<ODMKV_F16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&quant_rows_f16_kernel<ODMKV_BF16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
+    if (dtype == ODMKV_F16) ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_F16>, lds);
+    else ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_BF16>, lds);
     RowsArgs a;
     for (int i = 0; i < 2; ++i) a.job[i] = jobs[i < n_jobs ? i : 0];
     a.n_jobs = n_jobs;
@@ -2351,12 +2333,8 @@ int launch_quantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStre
 }
 
 int launch_dequantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
-    static bool attr_set = false;
-    if (!attr_set) {
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dequant_rows_f16_kernel<ODMKV_F16>), hipFuncAttributeMaxDynamicSharedMemorySize, DQ_LDS));
-        ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dequant_rows_f16_kernel<ODMKV_BF16>), hipFuncAttributeMaxDynamicSharedMemorySize, DQ_LDS));
-        attr_set = true;
-    }
+    if (dtype == ODMKV_F16) ODMKV_ALLOW_LDS(dequant_rows_f16_kernel<ODMKV_F16>, DQ_LDS);
+    else ODMKV_ALLOW_LDS(dequant_rows_f16_kernel<ODMKV_BF16>, DQ_LDS);
     RowsArgs a;
     for (int i = 0; i < 2; ++i) a.job[i] = jobs[i < n_jobs ? i : 0];
     a.n_jobs = n_jobs;
