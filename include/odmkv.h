@@ -24,6 +24,7 @@ extern "C" {
 #define ODMKV_EINVAL   (-1)   /* bad argument: shape, level set, null pointer, unsupported head_dim */
 #define ODMKV_ENOSPACE (-2)   /* workspace too small */
 #define ODMKV_EHIP     (-3)   /* a HIP runtime call failed */
+#define ODMKV_ENOMEM   (-4)   /* out of host memory */
 
 /* element types of K/V/Q tensors */
 #define ODMKV_F16  0
@@ -504,7 +505,8 @@ typedef struct odmkv_worklist {
  * of a pair's levels where the runs alone are many more than those places.  chains, pairs: -1 by these rules, 0 never,
  * 1 always; waves: 0 by the items' length and widths, or 8, 12, 16.
  * table (host int32, `capacity` integers) receives the items, the ranges at shape->range_at and, where shape->ordered, the
- * dispatch order at shape->order_at; too small a table gives ODMKV_ENOSPACE with shape->need set.  No counterpart in the
+ * dispatch order at shape->order_at; too small a table gives ODMKV_ENOSPACE with shape->need set, a list that does not
+ * fit host memory ODMKV_ENOMEM.  No counterpart in the
  * reference. */
 typedef struct odmkv_worklist_choice {
     double multiple;                 /* items (or workgroups) per compute unit of the winning cut */

@@ -8,6 +8,7 @@
 #include <math.h>
 #include <string.h>
 #include <algorithm>
+#include <exception>
 #include <functional>
 #include <queue>
 #include <vector>
@@ -179,9 +180,9 @@ struct Cutter {
 
 }  // namespace
 
-extern "C" int odmkv_worklist_cut(const int64_t* counts, const int64_t* seg_tile, int nseg, int n_cu, int64_t target_items,
-                                  int64_t min_item_bytes, int chains, int pairs, int waves, odmkv_worklist_choice_t* choice,
-                                  int32_t* table, uint64_t capacity, odmkv_worklist_shape_t* shape) {
+static int worklist_cut(const int64_t* counts, const int64_t* seg_tile, int nseg, int n_cu, int64_t target_items,
+                        int64_t min_item_bytes, int chains, int pairs, int waves, odmkv_worklist_choice_t* choice,
+                        int32_t* table, uint64_t capacity, odmkv_worklist_shape_t* shape) {
     ODMKV_CHECK_ARG(counts && seg_tile && choice && shape && (table || !capacity), "odmkv_worklist_cut: null pointer");
     ODMKV_CHECK_ARG(nseg > 0 && n_cu > 0 && min_item_bytes >= 0, "odmkv_worklist_cut: bad sizes (segments %d, compute units %d)", nseg, n_cu);
     Cutter k;
@@ -200,6 +201,7 @@ extern "C" int odmkv_worklist_cut(const int64_t* counts, const int64_t* seg_tile
             // exact segments grow between rebuilds: their whole capacity
             const int64_t nt = li == 4 ? seg_tile[(size_t)li * (nseg + 1) + s + 1] - t0 : (c + TILE - 1) / TILE;
             if (nt <= 0) continue;
+            ODMKV_CHECK_ARG(nt < (1 << 30), "odmkv_worklist_cut: %lld tiles of level %d in segment %d", (long long)nt, li, s);
             k.total += nt * kTileCost[li]; k.total_bytes += nt * kTileBytes[li];
             k.runs.push_back({s, li, nt, t0, c});
             if (li == 4) { n_exact += 1; continue; }
@@ -325,4 +327,15 @@ extern "C" int odmkv_worklist_cut(const int64_t* counts, const int64_t* seg_tile
         for (int i = 0; i < n_heads; ++i) table[at_order + i] = head[by[i]];
     }
     return 0;
+}
+
+extern "C" int odmkv_worklist_cut(const int64_t* counts, const int64_t* seg_tile, int nseg, int n_cu, int64_t target_items,
+                                  int64_t min_item_bytes, int chains, int pairs, int waves, odmkv_worklist_choice_t* choice,
+                                  int32_t* table, uint64_t capacity, odmkv_worklist_shape_t* shape) {
+    try {                                                     // (callers are C: nothing is thrown through them)
+        return worklist_cut(counts, seg_tile, nseg, n_cu, target_items, min_item_bytes, chains, pairs, waves, choice, table, capacity, shape);
+    } catch (const std::exception& e) {
+        odmkv_set_error("odmkv_worklist_cut: %s", e.what());
+        return ODMKV_ENOMEM;
+    }
 }

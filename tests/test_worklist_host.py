@@ -132,3 +132,33 @@ def test_explicit_targets_and_ragged_stores(target, monkeypatch):
         st._build_items(target, 1)
         items, heads = _check(st)
         assert (items[:, 0] != 2).all()
+
+
+def test_a_list_that_does_not_fit_host_memory_is_an_error_not_an_abort():
+    # 2^24 items in a process that may take 300 MB more: nothing is thrown through the C entry
+    import os
+    import subprocess
+    import sys
+    code = """
+import ctypes as C, resource
+import numpy as np
+from kvquant import _lib
+pages = int(open("/proc/self/statm").read().split()[0])
+resource.setrlimit(resource.RLIMIT_AS, (pages * resource.getpagesize() + (300 << 20),) * 2)
+counts = np.zeros((5, 1), np.int64); counts[0] = 64 << 24
+tiles = np.zeros((5, 2), np.int64); tiles[0, 1] = 1 << 24
+choice, shape = _lib.WorklistChoice(), _lib.WorklistShape()
+rc = _lib.lib.odmkv_worklist_cut(counts.ctypes.data, tiles.ctypes.data, 1, 256, 1 << 24, 0, -1, -1, 0, C.byref(choice), None, 0, C.byref(shape))
+assert rc == -4, rc
+try:
+    _lib.check(rc)
+except RuntimeError as e:
+    assert "worklist_cut" in str(e)
+counts[0] = 64 << 30
+assert _lib.lib.odmkv_worklist_cut(counts.ctypes.data, tiles.ctypes.data, 1, 256, 0, 0, -1, -1, 0, C.byref(choice), None, 0, C.byref(shape)) == -1
+print("ended")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=root,
+                       env=dict(os.environ, PYTHONPATH=os.path.join(root, "odm-kv_amd"), HIP_VISIBLE_DEVICES="-1"))
+    assert r.returncode == 0 and "ended" in r.stdout, (r.returncode, r.stderr[-800:])
