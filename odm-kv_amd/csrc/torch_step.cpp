@@ -188,6 +188,21 @@ PyMemberDef step_members[] = {
 
 PyTypeObject StepType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+PyObject* alias_both(const at::Tensor& keys, const at::Tensor& values, long long length) {
+    const at::Tensor* both[2] = {&keys, &values};
+    for (const at::Tensor* t : both)
+        if (t->dim() != 4 || t->size(2) < 1) return PyErr_Format(PyExc_ValueError, "alias: [B, H, n, D] tensors with a token at least");
+    at::Tensor view[2];
+    for (int i = 0; i < 2; ++i) {
+        const auto z = both[i]->sizes(); const auto r = both[i]->strides();
+        view[i] = both[i]->as_strided({z[0], z[1], length, z[3]}, {r[0], r[1], 0, r[3]}, both[i]->storage_offset() + (z[2] - 1) * r[2]);
+    }
+    PyObject* out = PyTuple_New(2);
+    if (out)
+        for (int i = 0; i < 2; ++i) PyTuple_SET_ITEM(out, i, THPVariable_Wrap(std::move(view[i])));
+    return out;
+}
+
 // alias(keys, values, length): [B, H, n, D] each -> stride-0 views [B, H, length, D] of the last token
 PyObject* native_alias(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (n != 3 || !THPVariable_Check(a[0]) || !THPVariable_Check(a[1])) {
@@ -197,14 +212,7 @@ PyObject* native_alias(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const long long length = PyLong_AsLongLong(a[2]);
     if (PyErr_Occurred()) return nullptr;
     GUARDED(
-        PyObject* both = PyTuple_New(2);
-        for (int i = 0; i < 2; ++i) {
-            const at::Tensor& t = THPVariable_Unpack(a[i]);
-            const auto z = t.sizes(); const auto r = t.strides();
-            PyTuple_SET_ITEM(both, i, THPVariable_Wrap(t.as_strided({z[0], z[1], length, z[3]}, {r[0], r[1], 0, r[3]},
-                                                                    t.storage_offset() + (z[2] - 1) * r[2])));
-        }
-        return both;
+        return alias_both(THPVariable_Unpack(a[0]), THPVariable_Unpack(a[1]), length);
     )
 }
 

@@ -305,3 +305,15 @@ def test_a_prefill_that_fails_waits_for_the_counts_it_asked_for(monkeypatch):
     with pytest.raises(RuntimeError, match="no CPU path"):        # the store lives on the GPU
         press._finalize_prefill(cache)
     assert calls == ["launched", "recorded", "waited"]
+
+
+def test_aliases_of_what_is_no_cache_layer_are_refused():
+    from kvquant import _lib
+    k = torch.arange(24.0).reshape(1, 2, 3, 4)
+    a, b = _lib._native.alias(k, k + 1, 7)
+    assert a.shape == b.shape == (1, 2, 7, 4) and torch.equal(a, k[:, :, -1:].expand(1, 2, 7, 4)) and torch.equal(b, a + 1)
+    for bad in (k[0], k[:, :, :0], torch.zeros(3)):
+        with pytest.raises(ValueError, match="alias"):
+            _lib._native.alias(k, bad, 7)
+    with pytest.raises(RuntimeError):
+        _lib._native.alias(k, k, -1)
