@@ -51,15 +51,20 @@ def fused_decode_enabled() -> bool:
 _causal_checked: dict = {}
 
 
-def _store_part_is_open(attention_mask: torch.Tensor, store_len: int) -> bool:
+def _store_part_is_open(attention_mask: torch.Tensor, store_len: int, layer=None) -> bool:
     """True when the boolean / additive mask of a multi-token step lets every query see every stored token (what a
-    causal mask without padding does).  The same mask object goes to every layer of a forward: checked once."""
+    causal mask without padding does).  The look waits for the device, and the same mask goes to every layer of a forward:
+    the answer serves the layers above the one that asked.  A mask may be written to between forwards: its version, where
+    torch counts one (not for inference tensors), and a layer index that does not ascend ask again."""
+    version = None if attention_mask.is_inference() else attention_mask._version
     hit = _causal_checked.get("last")
-    if hit is not None and hit[0] is attention_mask and hit[1] == store_len:      # (the entry keeps the tensor alive)
-        return hit[2]
-    part = attention_mask[..., :store_len]
-    ok = bool(part.all()) if attention_mask.dtype == torch.bool else bool((part == 0).all())
-    _causal_checked["last"] = (attention_mask, store_len, ok)
+    if (hit is not None and hit[0] is attention_mask and hit[1:3] == (store_len, version)      # (the entry keeps the tensor alive)
+            and layer is not None and hit[3] is not None and layer > hit[3]):
+        ok = hit[4]
+    else:
+        part = attention_mask[..., :store_len]
+        ok = bool(part.all()) if attention_mask.dtype == torch.bool else bool((part == 0).all())
+    _causal_checked["last"] = (attention_mask, store_len, version, layer, ok)
     return ok
 
 
@@ -83,7 +88,7 @@ def _fused_decode(module, query, key, value, attention_mask, dropout, kwargs):
     if scaling is None:
         scaling = D ** -0.5
     if L > 1:
-        return _fused_block(state, query, key, value, attention_mask, scaling, k_len)
+        return _fused_block(state, query, key, value, attention_mask, scaling, k_len, getattr(module, "layer_idx", None))
     if state.seq_len not in (k_len - 1, k_len):
         return None
     if state.seq_len == k_len - 1 and getattr(state, "exact_decode_append", False):
@@ -107,7 +112,7 @@ def _fused_decode(module, query, key, value, attention_mask, dropout, kwargs):
     return out.to(query.dtype).view(B, 1, Hq, D)
 
 
-def _fused_block(state, query, key, value, attention_mask, scaling, k_len):
+def _fused_block(state, query, key, value, attention_mask, scaling, k_len, layer=None):
     """A block of L new tokens after the prefill (the reference runner feeds every question this way,
     benchmark/core/pipeline.py:170-185; the reference's wrapper treats any q_len != k_len alike,
     attention_patch.py:38-48): every new token sees the whole store, through the fused kernel, and the new tokens at or
@@ -120,7 +125,7 @@ def _fused_block(state, query, key, value, attention_mask, scaling, k_len):
     if attention_mask is not None:
         if attention_mask.dim() != 4 or attention_mask.shape[-2] != L or attention_mask.shape[-1] != k_len:
             return None
-        if not _store_part_is_open(attention_mask, k_len - L):
+        if not _store_part_is_open(attention_mask, k_len - L, layer):
             return None
     out_s, lse_s = state.decode_attention_block(query, scaling=scaling)          # [B, Hq, L, D], [B, Hq, L]
     k, v = key[:, :, -L:, :], value[:, :, -L:, :]

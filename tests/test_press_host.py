@@ -317,3 +317,23 @@ def test_aliases_of_what_is_no_cache_layer_are_refused():
             _lib._native.alias(k, bad, 7)
     with pytest.raises(RuntimeError):
         _lib._native.alias(k, k, -1)
+
+
+@pytest.mark.parametrize("inference", [False, True])
+@pytest.mark.parametrize("additive", [False, True])
+def test_a_mask_written_to_between_forwards_is_looked_at_again(inference, additive, monkeypatch):
+    from kvquant import attention_patch as ap
+    looks = []
+    monkeypatch.setattr(ap, "bool", lambda x: looks.append(1) or x.item(), raising=False)
+    with torch.inference_mode(inference):
+        mask = torch.zeros(1, 1, 3, 13) if additive else torch.ones(1, 1, 3, 13, dtype=torch.bool)
+        assert [ap._store_part_is_open(mask, 10, layer) for layer in (0, 1, 5)] == [True] * 3
+        assert len(looks) == 1                                # the layers of one forward share the look
+        mask[0, 0, 1, 4] = float("-inf") if additive else False
+        assert [ap._store_part_is_open(mask, 10, layer) for layer in (0, 1, 5)] == [False] * 3      # the question after a rewind
+        assert len(looks) == 2 and ap._store_part_is_open(mask, 4, 6) and len(looks) == 3
+        assert ap._store_part_is_open(mask, 4) and ap._store_part_is_open(mask, 4) and len(looks) == 5   # (no layer index)
+    if not inference:
+        assert ap._store_part_is_open(mask, 4, 7) and len(looks) == 6
+        mask[0, 0, 1, 2] = float("-inf") if additive else False
+        assert not ap._store_part_is_open(mask, 4, 8)
