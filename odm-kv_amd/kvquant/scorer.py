@@ -123,7 +123,7 @@ def _query_covariance(module: nn.Module, q: torch.Tensor, q_len: int, n_future: 
     rotary_emb = getattr(module, "rotary_emb", None)
     if rotary_emb is not None and n_future > 0:
         pos = torch.arange(q_len, q_len + n_future, device=q.device).unsqueeze(0)
-        cos, sin = _aligned_rotary_outputs(rotary_emb, q.new_empty(1, dtype=torch.float32), pos)
+        cos, sin = _aligned_rotary_outputs(rotary_emb, q.new_empty((1, n_q, D), dtype=torch.float32), pos)   # (like the mean queries)
         if cos.shape != (1, n_future, D) or sin.shape != cos.shape:
             return None
         cos, sin = cos.contiguous(), sin.contiguous()
@@ -316,7 +316,7 @@ class RiskScorer(ExpectedAttentionScorer):
             hit = None if rope_tables is None else rope_tables.get(key)
             if hit is None:
                 pos = torch.arange(T, T + n_future, device=dev).unsqueeze(0)
-                cos, sin = _aligned_rotary_outputs(rotary_emb, hidden_states.new_empty(1), pos)
+                cos, sin = _aligned_rotary_outputs(rotary_emb, hidden_states.new_empty((1, n_q, D)), pos)       # (like the mean queries)
                 if cos.shape != (1, n_future, D) or sin.shape != cos.shape:
                     return None
                 hit = (cos.contiguous(), sin.contiguous(), rotary_emb)

@@ -87,3 +87,29 @@ def test_scores_normalised_on_the_device(rows, cols, pad):
         assert torch.allclose(_scale_on_device(y.cuda(), pad, True).cpu(), _normalize_scores(padded), rtol=1e-6, atol=1e-7)
     x[0, cols // 2] = float("nan")
     assert _scale_on_device(x.cuda(), pad, True).isnan().all()
+
+
+def test_rotary_modules_see_mean_queries():
+    # a rotary module may read the dimension, the heads or the type off the tensor it is handed
+    from types import SimpleNamespace
+    from kvquant import ExpectedAttentionScorer, RiskScorer
+    seen = []
+
+    def rotary(x, pos):
+        seen.append((tuple(x.shape), x.dtype))
+        a = pos[..., None].float() * (500000.0 ** (-torch.arange(0, x.shape[-1], 2, device=x.device).float() / x.shape[-1]))
+        a = torch.cat((a, a), dim=-1)
+        return a.cos().to(x.dtype), a.sin().to(x.dtype)
+    module = torch.nn.Module()
+    module.config = SimpleNamespace(num_attention_heads=4, head_dim=128)
+    module.q_proj = torch.nn.Linear(64, 512, bias=False, device="cuda", dtype=torch.float16)
+    module.rotary_emb = rotary
+    k = torch.randn(1, 2, 60, 128, device="cuda", dtype=torch.float16)
+    h = torch.randn(1, 60, 64, device="cuda", dtype=torch.float16)
+    risk = RiskScorer(n_future_positions=16, n_sink=4, epsilon=1e-2)
+    risk.normalize_grain = "global"
+    with torch.inference_mode():
+        assert risk.score_prompt(k, k, 0, module=module, hidden_states=h) is not None
+        risk.score_prefill(k[0], k[0], 0, module=module, hidden_states=h)
+        ExpectedAttentionScorer(n_future_positions=16, n_sink=4).score_prefill(k[0], k[0], 0, module=module, hidden_states=h)
+    assert seen == [((1, 4, 128), torch.float16)] * 2 + [((1, 4, 128), torch.float32)]
