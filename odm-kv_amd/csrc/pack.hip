@@ -1855,8 +1855,9 @@ struct DequantArgs {
 
 // x_hat[token][j] = |x| * sum_i c[code_i] * Pi[i][j] on the fp16 matrix cores (v_mfma_f32_16x16x32_f16): operand
 // A = Pi^T (rows = outputs j, steps = i), B = the centroids of 16 tokens' codes, both as fp16 high + low terms
-// (three products: hi*hi, lo*hi, hi*lo; the fourth is below 2^-22), accumulated in fp32.  The result differs from
-// the fp32 sum by about 1e-6 of the row's norm: less than the rounding of a 16-bit cache by two orders of magnitude.
+// (three products: hi*hi, lo*hi, hi*lo; the fourth is below 2^-22), accumulated in fp32.  Against fp64 the rows are off by
+// 2.8e-7 (2 bits) to 3.2e-7 of their norm, fp32 sums by 2.05e-7: less than the rounding of a 16-bit cache by three orders of
+// magnitude, and what a store has always written into a model's cache (rows outside the store: dequant_rows_f16_kernel).
 // Persistent workgroups of DQ_NW waves keep Pi^T in LDS in operand order (even workgroups keys, odd ones values) and
 // walk the tiles of all levels, a wave per tile.
 #define DQ_NW 8
@@ -1868,6 +1869,8 @@ struct DequantArgs {
 // Pi^T as the A operands of dq_tile, hi then lo: lane 16 q + r of block (jb, ch) holds Pi[32 ch + 8 q .. + 7][j] of the
 // output j = 32 (jb >> 1) + 8 (r >> 2) + 4 (jb & 1) + (r & 3): a lane's accumulators of two neighbouring blocks are then
 // eight consecutive outputs.
+// UP: times 2^UP (see dequant_rows_f16_kernel).
+template <int UP>
 __device__ static inline void dq_load_rotation(const float* pi, uint16_t* pih, int tid) {
     const float4* __restrict__ src = reinterpret_cast<const float4*>(pi);
     constexpr int PER_THREAD = HD * HD / 4 / (DQ_NW * 64);
@@ -1884,13 +1887,16 @@ __device__ static inline void dq_load_rotation(const float* pi, uint16_t* pih, i
         for (int t = 0; t < 4; ++t) {
             const int j = j0 + t, jb = 2 * (j >> 5) + ((j >> 2) & 1), r = 4 * ((j >> 3) & 3) + (j & 3);
             const int dst = (((jb * 4 + ch) * 64) + 16 * q + r) * 8 + e;
-            const uint16_t h = Elem<ODMKV_F16>::from_f32(pv[t]);
+            const float x = pv[t] * (float)(1 << UP);
+            const uint16_t h = Elem<ODMKV_F16>::from_f32(x);
             pih[dst] = h;
-            pih[HD * HD + dst] = Elem<ODMKV_F16>::from_f32(pv[t] - Elem<ODMKV_F16>::to_f32(h));
+            pih[HD * HD + dst] = Elem<ODMKV_F16>::from_f32(x - Elem<ODMKV_F16>::to_f32(h));
         }
     }
 }
+template <int UP>
 __device__ static inline uint32_t dq_centroid(float c) {
+    c *= (float)(1 << UP);
     const uint16_t h = Elem<ODMKV_F16>::from_f32(c);
     return (uint32_t)h | ((uint32_t)Elem<ODMKV_F16>::from_f32(c - Elem<ODMKV_F16>::to_f32(h)) << 16);
 }
@@ -1900,7 +1906,7 @@ __device__ static inline uint32_t dq_centroid(float c) {
 // Every operand of Pi^T is read once for all four token blocks (64 KB of LDS reads per tile; with a read per block, 256 KB,
 // the LDS pipe and the latency of its reads set the time), whose four accumulators are chains of their own; a lane stores 16
 // bytes of a row at a time, a token's four lanes 64.  A 2-bit layer of 32k tokens and 8 heads (both tensors): 81 -> 39 us.
-template <int DT>
+template <int DT, int UP>
 __device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* codes, const uint32_t* cb, const float* norms,
                                                const long long* offs, void* out, int lane) {
     const int r16 = lane & 15, q = lane >> 4;
@@ -1946,7 +1952,7 @@ __device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* 
             if (off >= 0) {                                   // outputs 32 jp + 8 q .. + 7 of the token
                 float r[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) r[e] = acc[e >> 2][tb][e & 3] * nrm;
+                for (int e = 0; e < 8; ++e) r[e] = acc[e >> 2][tb][e & 3] * (1.0f / (1 << UP) / (1 << UP)) * nrm;      // (an exact power of two)
                 store8<DT>(out, (size_t)off + 32 * jp + 8 * q, r);
             }
         }
@@ -2001,8 +2007,8 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
     if (table)
         for (int e = tid; e < DQ_MAX_RUNS; e += DQ_NW * 64)
             wbase[e + 1] = e < n_runs ? (a.s.seg_count[e / a.nseg][e % a.nseg] + TILE - 1) / TILE : 0;
-    dq_load_rotation(is_v ? a.pi_v : a.pi_k, reinterpret_cast<uint16_t*>(smem), tid);
-    for (int i = tid; i < DQ_CB_WORDS; i += DQ_NW * 64) cb[i] = dq_centroid(a.cb[i]);
+    dq_load_rotation<0>(is_v ? a.pi_v : a.pi_k, reinterpret_cast<uint16_t*>(smem), tid);
+    for (int i = tid; i < DQ_CB_WORDS; i += DQ_NW * 64) cb[i] = dq_centroid<0>(a.cb[i]);
     __syncthreads();
     if (table && wave == 0) {                                  // 16 entries per lane, a scan over the lanes' totals
         int mine[DQ_MAX_RUNS / 64], tot = 0;
@@ -2061,7 +2067,7 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
             default: dq_unpack<8>(src, is_v, codes, lane); break;
         }
         wave_lds_fence();
-        dq_tile<DT>(piA, codes, cb + codebook_offset(li), norms, offs, out, lane);
+        dq_tile<DT, 0>(piA, codes, cb + codebook_offset(li), norms, offs, out, lane);
         wave_lds_fence();                                        // offs / norms / codes free for the next tile
     }
 }
@@ -2280,6 +2286,12 @@ __global__ __launch_bounds__(QF_NW * 64) void quant_rows_f16_kernel(RowsArgs a) 
     }
 }
 
+// Rotation and centroids of unit vectors are about 0.09: the low parts of their fp16 pairs lie below fp16's least normal value
+// and keep a few bits only.  Times 2^8 both keep all eleven, and the result comes no further from fp64 than with fp32 sums
+// rounded once, which these rows had before the matrix cores did them.  Elements that are not the nearest 16-bit value to
+// the fp64 result, Gaussian rows: fp32 sums 1.05e-3 of all (fp16) and 1.6e-4 (bf16), plain pairs 2.3e-3 and 3.6e-4, these
+// 0.90e-3 and 1.3e-4; 67.5 us for an 8k-token pass with either.
+#define DQ_UP 8
 template <int DT>
 __global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
@@ -2290,8 +2302,8 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a
     uint32_t* cb = reinterpret_cast<uint32_t*>(smem + QP_PI_BYTES + DQ_NW * QP_STAGE);
     float* norms = reinterpret_cast<float*>(cb + DQ_CB_WORDS) + wave * TILE;
     long long* offs = reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + wave * TILE;
-    dq_load_rotation(j.pi, reinterpret_cast<uint16_t*>(smem), tid);
-    for (int i = tid; i < (1 << j.bits); i += DQ_NW * 64) cb[i] = dq_centroid(j.cb[i]);
+    dq_load_rotation<DQ_UP>(j.pi, reinterpret_cast<uint16_t*>(smem), tid);
+    for (int i = tid; i < (1 << j.bits); i += DQ_NW * 64) cb[i] = dq_centroid<DQ_UP>(j.cb[i]);
     __syncthreads();
     const long long tiles = (j.n + TILE - 1) / TILE, stride = (long long)(gridDim.x / a.n_jobs) * DQ_NW;
     for (long long tile = (long long)(blockIdx.x / a.n_jobs) * DQ_NW + wave; tile < tiles; tile += stride) {
@@ -2307,7 +2319,7 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a
             *reinterpret_cast<uint4*>(codes + token * CODE_ROW + 16 * piece) = v;
         }
         wave_lds_fence();
-        dq_tile<DT>(reinterpret_cast<const uint4*>(smem), codes, cb, norms, offs, j.out, lane);
+        dq_tile<DT, DQ_UP>(reinterpret_cast<const uint4*>(smem), codes, cb, norms, offs, j.out, lane);
         wave_lds_fence();
     }
 }
