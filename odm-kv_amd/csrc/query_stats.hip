@@ -298,8 +298,13 @@ extern "C" int odmkv_average_rope(const void* mu, const void* cosine, const void
 //   mu = sum_t q_t / n,  C = sum_t (q_t - mu) (q_t - mu)^T / n,  mu' = R mu,  C' = R C R^T,  R = diag(c) + diag(s) (half rotation)
 // The queries are taken relative to a pivot near their mean (the mean of 64 of them, the same for every workgroup of a head),
 // x = q - pivot in fp32, and x as three bf16 pieces whose sum it is: six products of pieces on the matrix cores (what they
-// leave out is below 2^-24), fp32 sums over at most 512 tokens at a time, fp64 behind that, where the rest of the mean is
-// subtracted.  (Products of the 16-bit queries as they are would be exact and a sixth of the work, but with a mean several
+// leave out, second times third piece twice and third times third, is up to 2^-21 of the product, always with its sign, where x
+// has all of fp32's bits), fp32 sums over at most 512 tokens at a time, fp64 behind that, where the rest of the mean is
+// subtracted.  The pivot is rounded to the queries' type: q - pivot and its running sum then mostly are exact, and the third
+// piece is mostly empty.  (With all of fp32's bits in the pivot every addition to a running sum was off by the same share of
+// its last place.)  Off fp64 over 600 to 32768 tokens, relative: means through the RoPE 0.3e-7 to 0.5e-7 (with such a pivot
+// 1.0e-7 to 5.1e-7; tensor operations in fp32 0.6e-7 to 1.2e-7), covariances 0.7e-7 to 1.7e-7 (1.2e-7 to 4.5e-7; 3.9e-7 to 2.7e-6).
+// (Products of the 16-bit queries as they are would be exact and a sixth of the work, but with a mean several
 // times the deviation their fp32 sums keep less of the covariance than sums of centred queries do.)
 // v_mfma_f32_32x32x16_bf16: D[32x32] += A[32x16] B[16x32], lane l supplies A[l % 32][8 (l / 32) + e] and the same of B^T:
 // both operands are the queries with the dims along the lanes and eight tokens in a lane.  A lane loads four dims
@@ -360,7 +365,7 @@ __global__ __launch_bounds__(CV_WAVES * 64) void cov_part_kernel(CovArgs a) {
         for (int i = 0; i < CV_SAMPLE / 4; ++i) s += Elem<DT>::to_f32(v[i]);
         sums[tid >> 7][tid & 127] = s;
         __syncthreads();
-        if (tid < HD) pivot[tid] = (sums[0][tid] + sums[1][tid] + sums[2][tid] + sums[3][tid]) / (float)CV_SAMPLE;
+        if (tid < HD) pivot[tid] = Elem<DT>::to_f32(Elem<DT>::from_f32((sums[0][tid] + sums[1][tid] + sums[2][tid] + sums[3][tid]) / (float)CV_SAMPLE));
         __syncthreads();
     }
     const float4 c4 = *reinterpret_cast<const float4*>(pivot + 4 * p);
@@ -444,18 +449,18 @@ __global__ __launch_bounds__(CV_WAVES * 64) void cov_part_kernel(CovArgs a) {
 
 // means of cos and sin over the positions (a workgroup per sixteen columns)
 __global__ __launch_bounds__(MN_THREADS) void rope_mean_kernel(CovArgs a) {
-    __shared__ float red[2][16][17];
+    __shared__ double red[2][16][17];
     const int c = threadIdx.x & 15, g = threadIdx.x >> 4, col = blockIdx.x * 16 + c;
-    float sc = 0.0f, ss = 0.0f;
+    double sc = 0.0, ss = 0.0;                                        // (cos and sin cancel over the positions)
 #pragma unroll 8
     for (int x = g; x < a.positions; x += 16) { sc += a.cosine[(size_t)x * HD + col]; ss += a.sine[(size_t)x * HD + col]; }
     red[0][g][c] = sc; red[1][g][c] = ss;
     __syncthreads();
     if (g < 2) {
-        float t = 0.0f;
+        double t = 0.0;
 #pragma unroll
         for (int k = 0; k < 16; ++k) t += red[g][k][c];
-        a.rope[g * HD + col] = t / (float)a.positions;
+        a.rope[g * HD + col] = (float)(t / a.positions);
     }
 }
 
@@ -500,8 +505,8 @@ __global__ __launch_bounds__(256) void cov_final_kernel(CovArgs a) {
     }
     if (blockIdx.x == 0 && tid < HD) {
         const float* pivot = part + CV_BLOCKS * 1024 + HD;
-        const float m = (float)(mean[tid] + pivot[tid]), o = (float)(mean[tid ^ 64] + pivot[tid ^ 64]);
-        a.mu[(size_t)h * HD + tid] = cs[0][tid] * m + cs[1][tid] * (tid < 64 ? -o : o);
+        const double m = mean[tid] + pivot[tid], o = mean[tid ^ 64] + pivot[tid ^ 64];
+        a.mu[(size_t)h * HD + tid] = (float)(cs[0][tid] * m + cs[1][tid] * (tid < 64 ? -o : o));
     }
 }
 
