@@ -1460,7 +1460,9 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
         // compute units); groups of up to four heads in the shared-lane form
         const bool pair = work->two_per_cu != 0 && (GP == 8 || g4_forced != 0);
         // a block of query tokens: several passes' workgroups in one launch run in rounds whatever the list, so they share
-        // compute units too (an order is not needed: the passes even the rounds out)
+        // compute units too (an order is not needed: the passes even the rounds out).  Whole calls in the list's own form / in
+        // pairs: 32k tokens, 32 heads over 8, bf16: 5 query tokens 41 / 33 us, 29: 165 / 122, 256: 1272 / 863; 28 over 4 at three
+        // bits: 29: 250 / 179; 2000 tokens: 9: 23 / 20, 29: 48 / 39; 131072 tokens: 29: 324 / 278; 700 tokens, 8 over 8: 17.5 / 17.8
         if (passes > 1 && !pair && !a.order) rc = GP == 4 ? launch_main<4, false, 8, true, false, true>(a, grid, e0, e1, st)
                                                           : launch_main<8, false, 8, false, false, true>(a, grid, e0, e1, st);
         else if (pair && GP == 4) rc = chain ? launch_main<4, true, 8, true, true, true>(a, grid, e0, e1, st)
@@ -1554,7 +1556,9 @@ __global__ __launch_bounds__(256) void block_queries_kernel(BlockQueryArgs a) {
     reinterpret_cast<uint4*>(a.out)[(size_t)row * PIECES + piece] = v;
 }
 
-#define BLOCK_WORKSPACE (64u << 20)      // a longer block goes in several launches
+// A longer block goes in several launches (32k tokens, 32 heads over 8: 118 query tokens fill it).  256 tokens there with 16, 64
+// and 256 MB: 985, 863, 840 us; 600 tokens on 2000: 554, 447, 427 us; 29 tokens on 32k at 28 heads over 4: 184, 179, 179 us.
+#define BLOCK_WORKSPACE (64u << 20)
 static int block_passes(int B, int G, int L, int n_items, int Hkv, int* per) {
     *per = std::max(1, ODMKV_MAX_GROUP / G);
     const int passes = (L + *per - 1) / *per;

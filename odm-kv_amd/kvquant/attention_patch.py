@@ -23,8 +23,11 @@ from transformers.modeling_utils import ALL_ATTENTION_FUNCTIONS
 from kvquant import _lib
 from kvquant._lib import stream_ptr
 
-# tokens of a block whose own part the library computes (every pair on the vector ALU); longer blocks are matrix products
-_NATIVE_BLOCK = 256
+# Pairs of query rows and new tokens (sequences x query heads x tokens^2) up to which the library computes a block's own part,
+# every pair on the vector ALU; larger blocks are matrix products, some twenty tensor operations of 230 to 260 us of host time.
+# Measured (library / tensor operations): one sequence of 32 heads, 29 tokens 14 / 244 us, 256 tokens 103 / 235, 384 tokens 213 /
+# 240, 512 tokens 367 / 231; eight sequences, 64 tokens 67 / 259, 128 tokens 295 / 259; 8 heads over 8, 512 tokens 150 / 253.
+_NATIVE_PAIRS = 3 << 20
 _PATCH_ATTR = "_kvtoken_quant_attention_patched"
 # how many decode calls took the fused kernel / the wrapped attention function (diagnostics)
 call_counts = {"fused": 0, "dense": 0}
@@ -130,7 +133,7 @@ def _fused_block(state, query, key, value, attention_mask, scaling, k_len, layer
     out_s, lse_s = state.decode_attention_block(query, scaling=scaling)          # [B, Hq, L, D], [B, Hq, L]
     k, v = key[:, :, -L:, :], value[:, :, -L:, :]
     mask = attention_mask
-    if (L <= _NATIVE_BLOCK and query.dtype in _lib._DT and k.dtype == v.dtype and k.dtype in _lib._DT and query.stride(3) == 1
+    if (B * Hq * L * L <= _NATIVE_PAIRS and query.dtype in _lib._DT and k.dtype == v.dtype and k.dtype in _lib._DT and query.stride(3) == 1
             and k.stride(3) == 1 and v.stride(3) == 1 and k.data_ptr() % 16 == 0 and not any(x % 8 for x in k.stride()[:3]) and (mask is None or (mask.dtype == torch.bool and mask.shape[1] == 1
                                                            and mask.shape[0] in (1, B) and mask.stride(3) == 1 and mask.is_cuda))):
         out = torch.empty(B, L, Hq, D, dtype=query.dtype, device=query.device)

@@ -92,3 +92,22 @@ def test_a_step_into_full_exact_segments_leaves_their_counts(B, H, G):
                                               128, out.data_ptr(), None, _lib.stream_ptr(out.device)))
         assert torch.equal(out, want) and (st._bufs["seg_count"][4] == 64).all()
     assert torch.equal(st.materialize()[0][:, :, :64], k[:, :, :64])
+
+
+@pytest.mark.parametrize("B,Hq,H,L", [(1, 8, 8, 627), (1, 8, 8, 628), (3, 28, 4, 193), (3, 28, 4, 194), (2, 4, 2, 2)])
+def test_blocks_on_either_side_of_the_native_limit(B, Hq, H, L):
+    # 3 << 20 pairs: 627 tokens of 8 heads, 193 tokens of 3 x 28
+    from types import SimpleNamespace
+    from kvquant import attention_patch as ap
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q = torch.randn(B, L, Hq, 128, generator=g, device="cuda").half().transpose(1, 2)
+    k, v = (torch.randn(B, L, H, 128, generator=g, device="cuda").half().transpose(1, 2) for _ in range(2))
+    out_s, lse_s = torch.randn(B, Hq, L, 128, generator=g, device="cuda"), torch.randn(B, Hq, L, generator=g, device="cuda")
+    state = SimpleNamespace(seq_len=50, decode_attention_block=lambda query, scaling: (out_s, lse_s))
+    with torch.inference_mode():
+        got = ap._fused_block(state, q, k, v, None, 0.08, 50 + L)
+        logits = (q.float() @ k.float().repeat_interleave(Hq // H, 1).transpose(-1, -2).contiguous()) * 0.08
+        keep = torch.ones(L, L, dtype=torch.bool, device="cuda").tril()
+        both = torch.cat([lse_s.unsqueeze(-1), logits.masked_fill(~keep, float("-inf"))], -1).softmax(-1)
+        want = both[..., :1] * out_s + both[..., 1:] @ v.float().repeat_interleave(Hq // H, 1)
+    assert got.shape == (B, L, Hq, 128) and (got.float() - want.transpose(1, 2)).norm() <= 1e-3 * want.norm()
