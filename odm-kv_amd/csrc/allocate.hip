@@ -41,8 +41,8 @@
 #define EV_TPT 2                              // tokens per thread of the candidates' and the last pass
 #endif
 #define EV_TOKENS (EV_THREADS * EV_TPT)
-#define EV_WGS 512ll                          // workgroups an evaluation is cut for over all rows (256: 305 us for 4 x 262144, 1024: 280, 512: 268)
-#define EV_BIG 2                              // tokens per thread and run where there are more than one per thread
+#define EV_WGS 512ll                          // workgroups an evaluation is cut for over all rows (a call with 4 x 262144 scores: 256 164 us, 512 149, 1024 165)
+#define EV_BIG 2                              // tokens per thread and run of a call with more than 256 x EV_THREADS of them
 #define EV_MAX_CHUNKS 256                     // workgroups of a row in an evaluation
 #define CAND_MAX 16                           // repair moves of at most this many tokens take the short path
 
@@ -770,8 +770,8 @@ extern "C" int odmkv_allocate(const float* scores, int rows, int n,
     a.scores = scores; a.sink_mask = sink_mask; a.rows = rows; a.n = n;
     a.period = period > 0 ? period : n; a.n_sink = sink_mask ? 0 : n_sink; a.sink_bits = sink_bits; a.K = n_levels;
     a.n_cand = (n + EV_TOKENS - 1) / EV_TOKENS;
-    // one token per thread up to a workgroup of them per compute unit; then runs of four, as many as leave about one
-    // workgroup per compute unit over all rows
+    // one token per thread up to a workgroup of them per compute unit; then EV_BIG tokens per thread and run, as many runs as
+    // leave EV_WGS workgroups over all rows, two per compute unit
     const long long all = (long long)rows * n;
     const int tpt = all <= 256ll * EV_THREADS ? 1 : EV_BIG, run = EV_THREADS * tpt;
     const int runs = (n + run - 1) / run;

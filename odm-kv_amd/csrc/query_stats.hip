@@ -43,7 +43,9 @@ __device__ static inline void add16(const uint4& v, float* acc) {
 // workgroup's rows with four requests in flight.  Two workgroups per compute unit with long runs of rows each, and loads that
 // leave nothing in the caches, read at 6.4 TB/s (32k x 4096: 42 us; 131k: 159 us, where runs of 256 rows do best); two
 // thousand workgroups of 32 rows with plain loads reached 4 TB/s (66 us; 220 us).  The torch form (conversion to fp32, mean)
-// moved five times the bytes: 250 us.
+// moved five times the bytes: 250 us.  The sums are formed in another order than torch's; rounded to 16 bits, 0 to 3 columns in
+// 10000 are not the nearest value to the fp64 mean (300 to 131072 tokens; torch's fp32 mean 0 to 5), so that a mean query may land
+// one step of its type apart from torch's.
 template <int DT>
 __global__ __launch_bounds__(MN_THREADS) void mean_part_kernel(MeanArgs a) {
     constexpr int N = Vec16<DT>::N, U = 4;

@@ -281,7 +281,7 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
                 self._buffer_start_seqs[layer_idx] = int(keys.shape[2])
                 self._buffer_counts[layer_idx] = 0
             if self._last_hooked_layer_idx is None or layer_idx == self._last_hooked_layer_idx:
-                release_staging(keys.device)             # the prompt is stored: the worst-case staging store can go
+                release_staging(keys.device)             # the prompt is stored: worst-case stores that direct fills left can go
         self._reset_prefill_state()
 
     # ------------------------------------------------------------------ hook

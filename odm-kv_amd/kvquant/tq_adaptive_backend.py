@@ -148,7 +148,8 @@ def reserve_state_memory(device, n_states: int) -> None:
 
 def release_staging(device=None) -> None:
     """Hand the staging stores (of one device, or of all) back to the allocator: a press does so when the last layer
-    of a prefill is stored, so that the decode steps which follow do not hold a worst-case store they never use.
+    of a prefill is stored, so that the decode steps which follow do not hold a worst-case store they never use (a fill whose
+    counts the press knows takes none; one that went through `prefill` or `append` directly may have left one).
     (Work already queued on the staging store's stream keeps its memory until it has run: the allocator returns a
     block to the stream it was requested on.)"""
     for key in [k for k in _STAGING if device is None or k[0] == _dev_key(device)]:
