@@ -77,7 +77,7 @@ int odmkv_score_model_dtype(const void* K, const void* V, int dtype, int Hkv, in
 
 /* The mean query (kvquant/scorer.py:204-227, kvquant/attention_utils.py:57-115), around the layer's own projection:
  * odmkv_token_mean: out [batch, cols] = mean over the tokens of x [batch, rows, cols] (`dtype`, element strides; rows of whole
- * 16-byte pieces), summed in fp32 and rounded to dtype; workspace odmkv_token_mean_workspace_bytes.
+ * 16-byte pieces), summed in fp32 and rounded to dtype; workspace odmkv_token_mean_workspace_bytes (room for any call with at most that many rows).
  * odmkv_average_rope: out fp32 [heads, 128] = c * mu + s * rotate_half(mu) with c, s the means over the positions of cosine,
  * sine [positions, 128]; mu [heads, 128], all contiguous and of `dtype`; every product, sum and mean is rounded to dtype. */
 size_t odmkv_token_mean_workspace_bytes(int batch, int rows, int cols);
@@ -94,7 +94,8 @@ int odmkv_project_rows(const void* weight, int64_t ld, const void* bias, const v
 /* A prompt's risk scores from its hidden states (kvquant/scorer.py:285-325, 385-416), all sequences of the batch in one call:
  * token mean behind the sinks, projection, averaged RoPE, odmkv_score_model_dtype.  hidden_states [B, T, hidden], weight
  * [Hq * 128, hidden] and bias of `dtype` (float16 / bfloat16); cosine, sine [positions, 128] of dtype, or both NULL; K, V of
- * kv_dtype with element strides; scores fp32 [B, Hkv, T]. */
+ * kv_dtype with element strides; scores fp32 [B, Hkv, T].  Long batches go in turns: the workspace stays within 64 MB, or what one
+ * sequence takes. */
 typedef struct odmkv_prompt {
     const void* hidden_states; int64_t h_stride_b, h_stride_t;
     const void* weight; int64_t ld_weight;
@@ -537,7 +538,7 @@ int odmkv_decode_attn(const void* q, int q_dtype, int B, int Hq, float scaling,
 
 /* One decode step of a layer in one call, for a serving loop whose host time per layer matters: the step's new token
  * of every (sequence, kv-head) is stored exact behind the others (odmkv_append_exact: k_new, v_new, strides, pos as
- * there; both NULL = the store already holds it), then odmkv_decode_attn runs for the step's query over the store, the
+ * there, a full segment's count stays; both NULL = the store already holds it), then odmkv_decode_attn runs for the step's query over the store, the
  * new token included.  Stands where the reference's forward hook appends the token to its state and the model then
  * attends over the re-materialised cache (kvquant/adaptive_backend_press.py:221-262; append_all_exact,
  * kvquant/tq_adaptive_backend.py:412-440).  What does not change from step to step sits in a block the caller fills

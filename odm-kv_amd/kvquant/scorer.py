@@ -98,11 +98,12 @@ class _NormFallback(BaseScorer):
 
 
 def _plain_projection(module: nn.Module):
-    """(weight, bias) of a query projection that is a 16-bit nn.Linear and nothing more (no q_norm behind it, no hooks, no
-    replaced forward), or (None, None)."""
+    """(weight, bias) of a query projection that is a 16-bit nn.Linear and nothing more (no q_norm behind it, no hooks of its own
+    or on all modules, no replaced forward, no autocast), or (None, None)."""
     proj = getattr(module, "q_proj", None)
     if (type(proj) is not nn.Linear or proj._forward_hooks or proj._forward_pre_hooks or "forward" in proj.__dict__
-            or hasattr(module, "qkv_proj") or hasattr(module, "q_norm")):
+            or hasattr(module, "qkv_proj") or hasattr(module, "q_norm") or torch.is_autocast_enabled("cuda")
+            or nn.modules.module._has_any_global_hook()):
         return None, None
     w, b = proj.weight, proj.bias
     if (type(w) is not nn.Parameter or w.dtype not in (torch.float16, torch.bfloat16) or not w.is_cuda or w.stride(1) != 1

@@ -70,3 +70,28 @@ def test_a_batch_scored_in_turns(gap):
     from kvquant import _lib
     assert _lib.lib.odmkv_prompt_scores_workspace_bytes(17, 100001, 256, 8, 1) < 17 * _lib.lib.odmkv_prompt_scores_workspace_bytes(1, 100001, 256, 8, 1) / 1.1
     test_scores_of_all_sequences(17, 8, 1, 100001, torch.float16, gap, True)
+
+
+def test_a_projection_that_is_watched_or_cast_is_called():
+    from kvquant import RiskScorer
+    module = nn.Module()
+    module.config = SimpleNamespace(num_attention_heads=2, head_dim=128)
+    module.q_proj = nn.Linear(64, 256, bias=False, device="cuda", dtype=torch.float16)
+    k = torch.randn(1, 2, 40, 128, device="cuda", dtype=torch.float16)
+    h = torch.randn(1, 40, 64, device="cuda", dtype=torch.float16)
+    scorer = RiskScorer(n_future_positions=8, n_sink=4, epsilon=1e-2)
+    scorer.normalize_grain = "global"
+    call = lambda: scorer.score_prompt(k, k, 0, module=module, hidden_states=h)
+    with torch.inference_mode():
+        assert call() is not None
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert call() is None
+        handle = nn.modules.module.register_module_forward_hook(lambda m, i, o: None)
+        try:
+            assert call() is None
+        finally:
+            handle.remove()
+        handle = module.q_proj.register_forward_hook(lambda m, i, o: None)
+        assert call() is None
+        handle.remove()
+        assert call() is not None
