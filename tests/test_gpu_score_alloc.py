@@ -257,6 +257,62 @@ def test_allocator_with_a_negative_error_sees_every_candidate():
     assert torch.equal(got.cpu(), oal.optimal_scores_to_bits(s, LEVELS, 2.5, eps, None, eviction_cost=0.5))
 
 
+def _awkward_scores(kind, rows, n, g):
+    if kind == "within a few thousand floats":                 # nothing settles until the bracket is a few floats wide
+        return 0.3 + 1e-4 * torch.rand(rows, n, generator=g)
+    if kind == "16-bit values":                                # many equal scores, at many values
+        return torch.rand(rows, n, generator=g).bfloat16().float()
+    s = torch.exp(2.0 * torch.randn(rows, n, generator=g)) * 1e-5
+    if kind == "half zeros":
+        s[torch.rand(rows, n, generator=g) < 0.5] = 0.0
+    elif kind == "two far groups":                             # a gap of thirty octaves in the middle of the histogram
+        s[:, n // 3:] *= 2.0 ** -30
+    elif kind == "tiny":                                       # few halvings are left behind the way down; subnormal products
+        s *= 1e-33
+    return s
+
+
+@pytest.mark.parametrize("kind", ["within a few thousand floats", "16-bit values", "half zeros", "two far groups", "tiny", "log-normal"])
+@pytest.mark.parametrize("rows,n", [(1, 513), (2, 8192 + 1), (33, 20000), (1, 150000)])
+def test_allocator_bit_exact_where_the_histogram_says_little(kind, rows, n):
+    """The search's guess only saves time: rows it misses, rows whose open list does not fit LDS, rows of equal scores.  33 rows
+    of 20000 are cut into few, long chunks; a wave's ragged ends are at 513 and 8193."""
+    from kvquant.allocator import optimal_scores_to_bits_batched
+    g = torch.Generator().manual_seed(n + rows)
+    s = _awkward_scores(kind, rows, n, g)
+    targets = [(1.5, 2.0, 3.0)[r % 3] for r in range(rows)]
+    bits, counts, lam = optimal_scores_to_bits_batched(s.to(DEV), LEVELS, targets, EPS, n_sink=3, period=n, eviction_cost=0.5, return_stats=True)
+    for r in sorted({0, 1 % rows, rows - 1}):
+        info = {}
+        want = oal.optimal_scores_to_bits(s[r:r + 1], LEVELS, targets[r], EPS, (torch.arange(n) < 3)[None], eviction_cost=0.5, info=info)
+        assert lam[r].item() == info["lam"] and torch.equal(bits[r:r + 1].cpu(), want)
+        assert counts[r].tolist() == [(want[:, 3:] == b).sum().item() for b in LEVELS]
+
+
+@pytest.mark.parametrize("eps", [{0: 1.0, 2: 0.1, 3: 0.1, 4: 0.1, 8: 0.0, 16: 0.0},                  # equal errors: levels nobody needs
+                                 {0: 0.2, 2: 0.3, 3: 0.05, 4: 0.06, 8: 0.001, 16: 0.002},             # errors that grow with the width
+                                 {0: 1.0, 2: 0.5, 3: 0.25, 4: 0.0, 8: -1e-3, 16: -2e-3}])             # negative ones
+@pytest.mark.parametrize("n", [700, 20011])
+def test_allocator_bit_exact_with_odd_error_tables(eps, n):
+    s = torch.exp(torch.randn(1, n, generator=torch.Generator().manual_seed(n)))
+    _check_alloc_eps(s, 2.5, eps)
+
+
+def _check_alloc_eps(scores, target, eps):
+    from kvquant.allocator import optimal_scores_to_bits
+    got = optimal_scores_to_bits(scores.to(DEV), LEVELS, target, eps, eviction_cost=0.5)
+    assert torch.equal(got.cpu(), oal.optimal_scores_to_bits(scores, LEVELS, target, eps, None, eviction_cost=0.5))
+
+
+@pytest.mark.parametrize("rows", [2048, 2049])
+def test_allocator_takes_many_rows_in_turns(rows):
+    from kvquant.allocator import optimal_scores_to_bits_batched
+    s = torch.exp(torch.randn(rows, 40, generator=torch.Generator().manual_seed(rows)))
+    bits = optimal_scores_to_bits_batched(s.to(DEV), LEVELS, 2.0, EPS, eviction_cost=0.5).cpu()
+    for r in (0, 1, 1023, 2047, rows - 1):
+        assert torch.equal(bits[r:r + 1], oal.optimal_scores_to_bits(s[r:r + 1], LEVELS, 2.0, EPS, None, eviction_cost=0.5))
+
+
 def test_calibrate_epsilon_matches_oracle():
     from kvquant.allocator import calibrate_epsilon
     got = calibrate_epsilon(128, LEVELS, device=DEV, value_quantizer="mse")
