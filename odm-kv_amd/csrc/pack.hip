@@ -467,6 +467,8 @@ __device__ static __forceinline__ void stage_codes_v(const f32x32& acc, int g, c
     }
 }
 
+struct AsStaged { __device__ uint32_t operator()(uint32_t w) const { return w; } };       // the staged words are codes already
+
 // ---- direct packing (widths 2, 4, 8; tiles that start empty) -----------------------------------------
 // The four outputs a lane holds for a token are neighbours in the token's code stream, and the four
 // tokens it holds for a value dim are neighbours in the dim's stream: 4*W bits that go to the staging
@@ -497,15 +499,15 @@ __device__ static __forceinline__ void stage_direct_k(const f32x32& a0, const f3
 }
 
 // lane (n, j) gathers dims 32j..32j+31 of its four slots key_slot(n, 0..3) from the staged token streams
-template <int W>
-__device__ static __forceinline__ void store_direct_k(const uint8_t* stage, uint8_t* kcodes, int tile, int lane) {
+template <int W, typename F>
+__device__ static __forceinline__ void store_direct_k(const uint8_t* stage, uint8_t* kcodes, int tile, int lane, F decode) {
     const int n = lane & 15, j = lane >> 4;
     uint32_t words[4 * W];
 #pragma unroll
     for (int b = 0; b < 4; ++b)
 #pragma unroll
         for (int i = 0; i < W; ++i)
-            words[b * W + i] = *reinterpret_cast<const uint32_t*>(stage + key_slot(n, b) * Direct<W>::ROW_K + 4 * W * j + 4 * i);
+            words[b * W + i] = decode(*reinterpret_cast<const uint32_t*>(stage + key_slot(n, b) * Direct<W>::ROW_K + 4 * W * j + 4 * i));
     uint8_t* dst = kcodes + (size_t)tile * (TILE * 16 * W);
 #pragma unroll
     for (int ch = 0; ch < W; ++ch)
@@ -526,8 +528,8 @@ __device__ static __forceinline__ void stage_direct_v(const f32x32& acc, int g, 
 
 // lane (n, j) gathers slots 32k+8j..+7 (k = 0, 1) of dims 16m+n (m = 0..7) from the staged dim streams:
 // W bytes per (k, m)
-template <int W>
-__device__ static __forceinline__ void store_direct_v(const uint8_t* stage, uint8_t* vcodes, int tile, int lane) {
+template <int W, typename F>
+__device__ static __forceinline__ void store_direct_v(const uint8_t* stage, uint8_t* vcodes, int tile, int lane, F decode) {
     const int n = lane & 15, j = lane >> 4;
     uint32_t words[4 * W];
 #pragma unroll
@@ -546,7 +548,7 @@ __device__ static __forceinline__ void store_direct_v(const uint8_t* stage, uint
 #pragma unroll
     for (int ch = 0; ch < W; ++ch)
         *reinterpret_cast<uint4*>(dst + ((size_t)ch * TILE + lane) * 16) =
-            make_uint4(words[4 * ch], words[4 * ch + 1], words[4 * ch + 2], words[4 * ch + 3]);
+            make_uint4(decode(words[4 * ch]), decode(words[4 * ch + 1]), decode(words[4 * ch + 2]), decode(words[4 * ch + 3]));
 }
 
 // Generic stores (any width; tiles that already hold `lo` tokens keep them: KEEP).  Slots at and behind
@@ -810,9 +812,9 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
             wave_lds_fence();
             if (direct) {
                 switch (li) {
-                    case 0: store_direct_k<2>(stage, a.s.kcodes[0], tile, ln); break;
-                    case 2: store_direct_k<4>(stage, a.s.kcodes[2], tile, ln); break;
-                    default: store_direct_k<8>(stage, a.s.kcodes[3], tile, ln); break;
+                    case 0: store_direct_k<2>(stage, a.s.kcodes[0], tile, ln, AsStaged()); break;
+                    case 2: store_direct_k<4>(stage, a.s.kcodes[2], tile, ln, AsStaged()); break;
+                    default: store_direct_k<8>(stage, a.s.kcodes[3], tile, ln, AsStaged()); break;
                 }
             } else if (lo > 0) {
                 switch (li) {
@@ -842,9 +844,9 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
                 }
                 wave_lds_fence();
                 switch (li) {
-                    case 0: store_direct_v<2>(stage, a.s.vcodes[0], tile, ln); break;
-                    case 2: store_direct_v<4>(stage, a.s.vcodes[2], tile, ln); break;
-                    default: store_direct_v<8>(stage, a.s.vcodes[3], tile, ln); break;
+                    case 0: store_direct_v<2>(stage, a.s.vcodes[0], tile, ln, AsStaged()); break;
+                    case 2: store_direct_v<4>(stage, a.s.vcodes[2], tile, ln, AsStaged()); break;
+                    default: store_direct_v<8>(stage, a.s.vcodes[3], tile, ln, AsStaged()); break;
                 }
             } else {
                 switch (li) {
@@ -896,7 +898,7 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
 // the chain itself, one lane per value, and replaces their codes in the packed tiles it has already
 // written.  Rows of zeros are exact either way.
 // Tiles the scheme does not cover go to the exact kernel through a list: 8-bit tiles (a tenth of
-// their values lie inside the band), tiles with a row whose squared norm is not finite, and tiles
+// their values lie inside the band), tiles of a width whose table does not mirror around its middle, tiles with a row whose squared norm is not finite, and tiles
 // with more listed values than the list has room for.
 //
 // Operands: for keys D = Pi (rows) x tokens (columns), so a lane ends with four consecutive outputs
@@ -924,87 +926,136 @@ __device__ static __forceinline__ qf_f4 qf_mfma(const uint4& a, const uint4& b, 
 }
 #define QF_LIST 256                     // listed values a wave can hold (it works them off 64 at a time)
 #define QF_GT_BITS 19                   // tile numbers in a list entry
-#define QF_NW 8
+#define QF_NW 8                         // two wavefronts a SIMD
+#define QF_STAGE 5120                   // Direct<4>: 64 tokens of 80 bytes, 128 dims of 40
 #define QF_PI_BYTES (2 * HD * HD * 2)   // Pi as fp16 hi and lo, in matrix-operand order
 #define QF_THR_BYTES 1152               // QP_THR_FLOATS floats, padded to a multiple of 16
 
 struct QfWave {                          // per-wave scratch in LDS
-    unsigned long long off[TILE];        // element offset of the token's row (~0: no row, zeros)
-    float den[TILE], rinv[TILE], band[TILE];
+    unsigned long long off[TILE];        // element offset of the token's row
+    float den[TILE], rinv[TILE];
     uint32_t list[QF_LIST];              // slot in the tile | output << 6 | tile number << 13
     int count, pad[3];
 };
 
-template <int W> struct GuardCoder {
-    static constexpr int K = 1 << W;
-    float t[(W <= 3) ? K - 1 : 1];
-    const float* thr;
-    __device__ inline GuardCoder(const float* thr_li) : thr(thr_li) {
-        if constexpr (W <= 3) {
+// A table that mirrors around its middle threshold (Lloyd-Max tables of a symmetric density do, to the last bit or two): the code of y is that of
+// |y - middle| among half as many thresholds, with all bits turned where y lies below.  A comparison then is a subtraction whose sign
+// bit is the answer and whose size is the distance the band is held against, and a bit moves into the word by one funnel
+// shift: 7 / 11 / 17 instructions a value of 2 / 3 / 4 bits, where the search through the whole table takes 11 / 18 and, at 4 bits, four reads of LDS.
+// What push() collects are sign bits; decode() turns fields of them into codes, four or more at a time.
+#define QF_MIRROR 1.0e-6f                // how far a mirrored threshold may be from its place (the band grows by as much)
+template <int W> struct MirrorCoder {
+    static constexpr int H = (1 << (W - 1)) - 1;            // thresholds on one side of the middle
+    float mid, u[H];
+    __device__ inline MirrorCoder(const float* thr_li) : mid(-thr_li[H]) {
 #pragma unroll
-            for (int k = 0; k < K - 1; ++k) t[k] = thr_li[k];
-        }
+        for (int k = 0; k < H; ++k) u[k] = 0.5f * (thr_li[H + 1 + k] - thr_li[H - 1 - k]);
     }
-    // r * 2^W + code(y), and m = distance from y to the nearest threshold: the binary search meets
-    // both neighbours of y on its way, so the minimum over the thresholds it compares with is exact
-    __device__ __forceinline__ uint32_t push(uint32_t r, float y, float& m) const {
+    __device__ __forceinline__ uint32_t push(uint32_t r, float x, float scale, float& m) const {
+        const float z = __fmaf_rn(x, scale, mid), a = fabsf(z);
+        r = __builtin_amdgcn_alignbit(r, __float_as_uint(z), 31);
         if constexpr (W == 2) {
-            const bool b1 = y >= t[1];
-            r = r + r + (b1 ? 1u : 0u);
-            const float ts = b1 ? t[2] : t[0];
-            const bool b0 = y >= ts;
-            m = fminf(fabsf(y - t[1]), fabsf(y - ts));
-            return r + r + (b0 ? 1u : 0u);
+            const float e = a - u[0];
+            r = __builtin_amdgcn_alignbit(r, __float_as_uint(e), 31);
+            m = fminf(a, fabsf(e));
         } else if constexpr (W == 3) {
-            const bool b2 = y >= t[3];
-            r = r + r + (b2 ? 1u : 0u);
-            const float ta = b2 ? t[5] : t[1];
-            const bool b1 = y >= ta;
-            r = r + r + (b1 ? 1u : 0u);
-            const float lo_pair = b1 ? t[2] : t[0], hi_pair = b1 ? t[6] : t[4];
-            const float tb = b2 ? hi_pair : lo_pair;
-            const bool b0 = y >= tb;
-            m = fminf(fminf(fabsf(y - t[3]), fabsf(y - ta)), fabsf(y - tb));
-            return r + r + (b0 ? 1u : 0u);
+            const float e1 = a - u[1], e2 = a - (e1 < 0.0f ? u[0] : u[2]);
+            r = __builtin_amdgcn_alignbit(r, __float_as_uint(e1), 31);
+            r = __builtin_amdgcn_alignbit(r, __float_as_uint(e2), 31);
+            m = fminf(fminf(a, fabsf(e1)), fabsf(e2));
         } else {
-            int pos = 0;
-            m = INFINITY;
-#pragma unroll
-            for (int s = K / 2; s >= 1; s >>= 1) {
-                const float tv = thr[pos + s - 1];
-                m = fminf(m, fabsf(y - tv));
-                if (y >= tv) pos += s;
-            }
-            return (r << W) | (uint32_t)pos;
+            const float e1 = a - u[3], e2 = a - (e1 < 0.0f ? u[1] : u[5]);
+            const float lo = e2 < 0.0f ? u[0] : u[2], hi = e2 < 0.0f ? u[4] : u[6], e3 = a - (e1 < 0.0f ? lo : hi);
+            r = __builtin_amdgcn_alignbit(r, __float_as_uint(e1), 31);
+            r = __builtin_amdgcn_alignbit(r, __float_as_uint(e2), 31);
+            r = __builtin_amdgcn_alignbit(r, __float_as_uint(e3), 31);
+            m = fminf(fminf(a, fabsf(e1)), fminf(fabsf(e2), fabsf(e3)));
         }
+        return r;
+    }
+    // fields whose top bits are `top`: code = not (signs, the lower ones turned where the first is set)
+    __device__ static __forceinline__ uint32_t decode(uint32_t r, uint32_t top) {
+        const uint32_t t = r & top;
+        return ~(r ^ (t - (t >> (W - 1))));
     }
 };
+// a staged word of W-bit codes in fields of S bits (2 or 4) -> codes
+template <int W, int S>
+__device__ static __forceinline__ uint32_t qf_decode(uint32_t x) {
+    constexpr uint32_t ONES = S == 2 ? 0x55555555u : 0x11111111u;
+    return MirrorCoder<W>::decode(x, ONES << (W - 1)) & (ONES * ((1u << W) - 1u));
+}
 
-// rotation estimate -> codes into the staging area; values inside the band -> the wave's list
+// does the width's table mirror?  (a lane per pair of thresholds, all lanes get the answer)
+template <int W>
+__device__ static inline bool qf_mirrors(const float* thr, int lane) {
+    constexpr int H = (1 << (W - 1)) - 1;
+    const int k = lane < H ? lane : 0;
+    const float up = thr[H + 1 + k] - thr[H], down = thr[H] - thr[H - 1 - k];
+    return !__any(!(fabsf(up - down) <= QF_MIRROR));
+}
+
+// sixteen tokens' rows in matrix-operand order: lane 16q + r holds elements 32 ch + 8 q .. + 7 of token 16 tb + r in x[tb][ch]
+typedef uint4 QfRows[4][4];
+
+// Sums of squares in the definition's order, a token per lane (lane = token), out of the operand registers: the four registers of a word
+// (one per token block) and the four rows of 16 lanes (one per 8 elements) change places in four swaps, and a lane holds 32 consecutive
+// elements of its own token.  (The rows used to be read twice, once with a token per lane and once in operand order.)
+template <int DT>
+__device__ static __forceinline__ float qf_sum_squares(const QfRows& x, uint32_t& any) {
+    float ss = 0.0f;
+    any = 0u;
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) {
+        uint32_t w[4][4];                                    // [8 elements][word]
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            uint32_t r[4];
+#pragma unroll
+            for (int tb = 0; tb < 4; ++tb) r[tb] = c == 0 ? x[tb][ch].x : c == 1 ? x[tb][ch].y : c == 2 ? x[tb][ch].z : x[tb][ch].w;
+            const auto a = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false);
+            const auto b = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+            const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+            const auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+            w[0][c] = lo[0]; w[1][c] = lo[1]; w[2][c] = hi[0]; w[3][c] = hi[1];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float x0 = Elem<DT>::to_f32((uint16_t)(w[q][c] & 0xffffu)), x1 = Elem<DT>::to_f32((uint16_t)(w[q][c] >> 16));
+                ss = __fmaf_rn(x0, x0, ss);
+                ss = __fmaf_rn(x1, x1, ss);
+                if constexpr (DT != ODMKV_F16) any |= w[q][c];
+            }
+        __builtin_amdgcn_sched_barrier(0);                   // (the copies of one chunk at a time: sixteen registers, not 64)
+    }
+    return ss;
+}
+
+// Rotation estimate -> codes into the staging area: fields of W bits side by side (DIRECT), or of 4 bits where they have to be moved
+// one by one when they are stored (3 bits; tiles that hold tokens already), as sign bits, decoded then; values inside the band -> the wave's list, of the tokens of `listed` alone (rows of zeros: the estimate is the exact 0)
 template <int DT, int W, bool IS_V, bool DIRECT>
-__device__ static __forceinline__ void qf_code_tile(const void* base, const uint4* piA, const float* thr, QfWave& w,
-                                                    uint8_t* stage, int lane, int gt) {
+__device__ static __forceinline__ void qf_code_tile(const QfRows& xb, const uint4* piA, const float* thr, QfWave& w,
+                                                    uint8_t* stage, int lane, int gt, unsigned long long listed) {
     const int r16 = lane & 15, q = lane >> 4;
-    const GuardCoder<W> code(thr);
+    const MirrorCoder<W> code(thr);
+    constexpr float BAND = (DT == ODMKV_F16 ? QF_BAND : QF_BAND_BF16) + QF_MIRROR;
     constexpr int NT = IS_V ? 16 : 4;
-    float rinv[NT], band[NT];
-    uint4 xb[4][4];
+    float rinv[NT];
+    uint32_t may = 0u;                                          // band flags that count, in f's order (below)
 #pragma unroll
     for (int tb = 0; tb < 4; ++tb) {
         if constexpr (IS_V) {
             const float4 ri = *reinterpret_cast<const float4*>(&w.rinv[16 * tb + 4 * q]);
-            const float4 bd = *reinterpret_cast<const float4*>(&w.band[16 * tb + 4 * q]);
             rinv[4 * tb] = ri.x; rinv[4 * tb + 1] = ri.y; rinv[4 * tb + 2] = ri.z; rinv[4 * tb + 3] = ri.w;
-            band[4 * tb] = bd.x; band[4 * tb + 1] = bd.y; band[4 * tb + 2] = bd.z; band[4 * tb + 3] = bd.w;
+            may |= ((uint32_t)(listed >> (16 * tb + 4 * q)) & 15u) << (28 - 4 * tb);
         } else {
             rinv[tb] = w.rinv[16 * tb + r16];
-            band[tb] = w.band[16 * tb + r16];
+            may |= ((listed >> (16 * tb + r16)) & 1ull) ? 15u << (28 - 4 * tb) : 0u;
         }
-        const unsigned long long o = w.off[16 * tb + r16];
-        const uint4* row = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(base) + (o == ~0ull ? 0ull : o)) + q;
-#pragma unroll
-        for (int ch = 0; ch < 4; ++ch) xb[tb][ch] = (o == ~0ull) ? make_uint4(0u, 0u, 0u, 0u) : row[4 * ch];
     }
+    may |= may >> 16;
 #pragma unroll 1
     for (int k = 0; k < 4; ++k) {
         uint32_t f = 0u;                                        // band flags of this pair of output blocks, first value on top
@@ -1018,40 +1069,28 @@ __device__ static __forceinline__ void qf_code_tile(const void* base, const uint
             for (int ch = 0; ch < 4; ++ch) {
                 const uint4 ah = piA[(ob * 4 + ch) * 64 + lane];
                 const uint4 al = piA[HD * HD / 8 + (ob * 4 + ch) * 64 + lane];
+                // (the four blocks' chains in turn: an accumulator's next product waits for its last)
 #pragma unroll
-                for (int tb = 0; tb < 4; ++tb) {
-                    if constexpr (IS_V) {
-                        acc[tb] = qf_mfma<DT>(xb[tb][ch], ah, acc[tb]);
-                        acc[tb] = qf_mfma<DT>(xb[tb][ch], al, acc[tb]);
-                    } else {
-                        acc[tb] = qf_mfma<DT>(ah, xb[tb][ch], acc[tb]);
-                        acc[tb] = qf_mfma<DT>(al, xb[tb][ch], acc[tb]);
-                    }
-                }
+                for (int tb = 0; tb < 4; ++tb) acc[tb] = IS_V ? qf_mfma<DT>(xb[tb][ch], ah, acc[tb]) : qf_mfma<DT>(ah, xb[tb][ch], acc[tb]);
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[tb] = IS_V ? qf_mfma<DT>(xb[tb][ch], al, acc[tb]) : qf_mfma<DT>(al, xb[tb][ch], acc[tb]);
             }
 #pragma unroll
             for (int tb = 0; tb < 4; ++tb) {
                 uint32_t g = 0u;
 #pragma unroll
                 for (int r = 3; r >= 0; --r) {
-                    const float y = acc[tb][r] * (IS_V ? rinv[4 * tb + r] : rinv[tb]);
+                    const float scale = IS_V ? rinv[4 * tb + r] : rinv[tb];
                     float m;
-                    if constexpr (DIRECT) g = code.push(g, y, m);
-                    else g = (g << 8) | code.push(0u, y, m);
-                    const bool near = m < (IS_V ? band[4 * tb + r] : band[tb]);
-                    f = f + f + (near ? 1u : 0u);
+                    g = code.push(DIRECT ? g : g << (4 - W), acc[tb][r], scale, m);
+                    f = __builtin_amdgcn_alignbit(f, __float_as_uint(m - BAND), 31);
                 }
-                if constexpr (!IS_V) {
-                    const int token = 16 * tb + r16, grp = 4 * ob + q;
-                    if constexpr (DIRECT) put_group<W>(stage + token * Direct<W>::ROW_K + grp * Direct<W>::GROUP_BYTES, g);
-                    else *reinterpret_cast<uint32_t*>(stage + token * CODE_ROW + 4 * grp) = g;
-                } else {
-                    const int dim = 16 * ob + r16, tg = 4 * tb + q;
-                    if constexpr (DIRECT) put_group<W>(stage + dim * Direct<W>::ROW_V + tg * Direct<W>::GROUP_BYTES, g);
-                    else *reinterpret_cast<uint32_t*>(stage + dim * CODE_ROW_T + 4 * tg) = g;
-                }
+                constexpr int S = DIRECT ? W : 4;               // bits a code takes in the staging area
+                if constexpr (!IS_V) put_group<S>(stage + (16 * tb + r16) * Direct<S>::ROW_K + (4 * ob + q) * Direct<S>::GROUP_BYTES, g);
+                else put_group<S>(stage + (16 * ob + r16) * Direct<S>::ROW_V + (4 * tb + q) * Direct<S>::GROUP_BYTES, g);
             }
         }
+        f &= may;
         while (f) {                                             // rare: a few values per lane and tile
             const int b = 31 - __clz(f);
             f &= ~(1u << b);
@@ -1111,8 +1150,9 @@ __device__ static __forceinline__ float qf_chain(const RowRegs<DT>& x, const flo
 // Entries first .. first + n - 1 of the wave's list (n <= 64), a lane each: the value by the definition's
 // own chain, its code, and that code in place of the estimate's in the packed tile.  The tile's codes,
 // positions and norms were written by this wave: the caller has waited for those stores.
+// An entry of the tile at hand (gt_now) finds its row and its norm in the wave's scratch, one of an earlier tile looks them up.
 template <int DT, bool IS_V>
-__device__ static void qf_fix_listed(const QuantArgs& a, const float* thrs, const QfWave& w, int lane, int first, int n) {
+__device__ static void qf_fix_listed(const QuantArgs& a, const float* thrs, const QfWave& w, int lane, int first, int n, int gt_now) {
     const bool on = lane < n;
     const uint32_t e = w.list[first + (on ? lane : 0)];
     const int token = e & 63, out = (e >> 6) & 127, gt = (int)(e >> 13);
@@ -1120,12 +1160,15 @@ __device__ static void qf_fix_listed(const QuantArgs& a, const float* thrs, cons
 #pragma unroll
     for (int k = 1; k < ODMKV_NQ; ++k) li += (gt >= a.tile_base[k]);
     const int tile = gt - a.tile_base[li];
-    const int bh = find_segment(a.s.seg_tile[li], a.nseg, tile);
-    const size_t slot = (size_t)tile * TILE + token;
-    const size_t off = (size_t)(bh / a.Hkv) * a.sB + (size_t)(bh % a.Hkv) * a.sH +
-                       (size_t)(a.s.pos[li][slot] - a.pos_offset) * a.sT;
-    // written by this wave a moment ago: read past the vector cache
-    const float den = __hip_atomic_load((IS_V ? a.s.vnorm[li] : a.s.knorm[li]) + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1e-10f;
+    size_t off = w.off[token];
+    float den = w.den[token];
+    if (gt != gt_now) {
+        const int bh = find_segment(a.s.seg_tile[li], a.nseg, tile);
+        const size_t slot = (size_t)tile * TILE + token;
+        off = (size_t)(bh / a.Hkv) * a.sB + (size_t)(bh % a.Hkv) * a.sH + (size_t)(a.s.pos[li][slot] - a.pos_offset) * a.sT;
+        // written by this wave a moment ago: read past the vector cache
+        den = __hip_atomic_load((IS_V ? a.s.vnorm[li] : a.s.knorm[li]) + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1e-10f;
+    }
     RowRegs<DT> x;
     x.load(IS_V ? a.V : a.K, off);
     const float4* __restrict__ prow = reinterpret_cast<const float4*>((IS_V ? a.pi_v : a.pi_k) + out * HD);
@@ -1166,35 +1209,114 @@ __device__ static void qf_fix_listed(const QuantArgs& a, const float* thrs, cons
     }
 }
 
+// codes staged in 4 bits each, packed one by one; tiles that already hold `lo` tokens keep them (KEEP)
+template <int W, bool KEEP>
+__device__ static __forceinline__ void qf_pack_k(const uint8_t* stage, uint8_t* kcodes, int tile, int lane, int lo) {
+    const int n = lane & 15, j = lane >> 4;
+    uint8_t* dst = kcodes + (size_t)tile * (TILE * 16 * W);
+    uint32_t words[4 * W];
+#pragma unroll
+    for (int k = 0; k < 4 * W; ++k) words[k] = 0u;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const uint4 v = *reinterpret_cast<const uint4*>(stage + key_slot(n, b) * Direct<4>::ROW_K + 16 * j);
+        const uint32_t w[4] = {qf_decode<W, 4>(v.x), qf_decode<W, 4>(v.y), qf_decode<W, 4>(v.z), qf_decode<W, 4>(v.w)};
+#pragma unroll
+        for (int e = 0; e < 32; ++e) put_code<W>(words, 32 * b + e, (w[e >> 3] >> (4 * (e & 7))) & 15u);
+        __builtin_amdgcn_sched_barrier(0);                   // (a block's 32 codes at a time: all 128 unpacked ahead do not fit the registers)
+    }
+    if constexpr (KEEP) {
+        // a slot's codes are W whole words of the lane's stream
+#pragma unroll
+        for (int c = 0; c < W; ++c) {
+            const uint4 old = *reinterpret_cast<const uint4*>(dst + ((size_t)c * TILE + lane) * 16);
+            const uint32_t o[4] = {old.x, old.y, old.z, old.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (key_slot(n, (4 * c + i) / W) < lo) words[4 * c + i] = o[i];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < W; ++c)
+        *reinterpret_cast<uint4*>(dst + ((size_t)c * TILE + lane) * 16) = make_uint4(words[4 * c], words[4 * c + 1], words[4 * c + 2], words[4 * c + 3]);
+}
+
+template <int W, bool KEEP>
+__device__ static __forceinline__ void qf_pack_v(const uint8_t* stage, uint8_t* vcodes, int tile, int lane, int lo) {
+    const int n = lane & 15, j = lane >> 4;
+    uint8_t* dst = vcodes + (size_t)tile * (TILE * 16 * W);
+    uint32_t old[4 * W], words[4 * W];
+    if constexpr (KEEP) {
+#pragma unroll
+        for (int c = 0; c < W; ++c) {
+            const uint4 o = *reinterpret_cast<const uint4*>(dst + ((size_t)c * TILE + lane) * 16);
+            old[4 * c] = o.x; old[4 * c + 1] = o.y; old[4 * c + 2] = o.z; old[4 * c + 3] = o.w;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4 * W; ++k) words[k] = 0u;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const uint32_t v = qf_decode<W, 4>(*reinterpret_cast<const uint32_t*>(stage + (16 * m + n) * Direct<4>::ROW_V + 16 * k + 4 * j));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int ci = 64 * k + 8 * m + e;
+                uint32_t c = (v >> (4 * e)) & 15u;
+                if constexpr (KEEP) c = (32 * k + 8 * j + e < lo) ? get_code<W>(old, ci) : c;     // stored earlier: keep
+                put_code<W>(words, ci, c);
+            }
+            if (m % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+    for (int c = 0; c < W; ++c)
+        *reinterpret_cast<uint4*>(dst + ((size_t)c * TILE + lane) * 16) = make_uint4(words[4 * c], words[4 * c + 1], words[4 * c + 2], words[4 * c + 3]);
+}
+
 // the staged codes packed into the store
 template <int W, bool IS_V, bool DIRECT>
 __device__ static __forceinline__ void qf_store_tile(const QuantArgs& a, const uint8_t* stage, int lane, int li, int tile, int lo) {
     uint8_t* codes = IS_V ? a.s.vcodes[li] : a.s.kcodes[li];
     if constexpr (!IS_V) {
-        if constexpr (DIRECT) store_direct_k<W>(stage, codes, tile, lane);
-        else if (lo > 0) pack_store_k<W, true>(stage, codes, tile, lane, lo);
-        else pack_store_k<W, false>(stage, codes, tile, lane, 0);
+        if constexpr (DIRECT) store_direct_k<W>(stage, codes, tile, lane, [](uint32_t x) { return qf_decode<W, W>(x); });
+        else if (lo > 0) qf_pack_k<W, true>(stage, codes, tile, lane, lo);
+        else qf_pack_k<W, false>(stage, codes, tile, lane, 0);
     } else {
-        if constexpr (DIRECT) store_direct_v<W>(stage, codes, tile, lane);
-        else if (lo > 0) pack_store_v<W, true>(stage, codes, tile, lane, lo);
-        else pack_store_v<W, false>(stage, codes, tile, lane, 0);
+        if constexpr (DIRECT) store_direct_v<W>(stage, codes, tile, lane, [](uint32_t x) { return qf_decode<W, W>(x); });
+        else if (lo > 0) qf_pack_v<W, true>(stage, codes, tile, lane, lo);
+        else qf_pack_v<W, false>(stage, codes, tile, lane, 0);
     }
 }
 
-struct QfTile { int wi, gt, li, tile, bh, lo, hi; };
+struct QfTile { int wi, gt, li, tile, bh, lo, hi; };        // (all of it in scalar registers)
 #define QF_MAX_RUNS 1024                // (level, segment) pairs whose tile counts fit the walk table
 
-// Per wave: the next tile and the positions of its tokens are looked up while the current tile's rows are on
-// their way.  (Requesting the next tile's rows a whole tile ahead was measured: no faster, and its 64 registers
-// per lane are the ones the kernel does not have.)
-template <int DT, bool IS_V>
+// The last of n_runs (<= 1024) ascending entries that is at most wi, by the wavefront: every 16th entry, then the sixteen behind it.  (Halving
+// steps were ten dependent reads of LDS, and left everything that follows from the answer in vector registers.)
+__device__ static __forceinline__ int find_run(const int* base, int n_runs, int wi, int lane) {
+    const int c = 16 * lane;
+    const int block = 16 * (__popcll(__ballot(c < n_runs && base[c < n_runs ? c : 0] <= wi)) - 1);
+    const int e = block + (lane & 15);
+    return block + __popcll(__ballot(lane < 16 && e < n_runs && base[e < n_runs ? e : 0] <= wi)) - 1;
+}
+__device__ static __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// What bounds it: two wavefronts a SIMD that wait for memory two fifths of their time (256 matrix instructions and 1900 vector ones a
+// tile, 22 % and 43 % of their pipes).  us a layer with its rows cold: 32k tokens of 8 heads, 2 bits, fp16 95 -> 75; 131k tokens of bf16 at 2 to 4
+// bits, 40 % evicted, 241 -> 202; two sequences of 777 tokens, a tile a wavefront, 33 -> 24.5.  The registers are full: three wavefronts a
+// SIMD (168 a lane), or the next rows requested ahead of the coding, leave 90 to 210 of them in scratch memory, whose
+// reads wait behind the rows: 96 to 104 us.
+// Per wave: a tile's positions are looked up a tile ahead and its rows requested as soon as the registers are free.  ready() is
+// called once, behind the first tile's requests: it lays out the rotation and the thresholds and ends with the workgroup's barrier.
+template <int DT, bool IS_V, typename F>
 __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float* thrs, QfWave& w, uint8_t* stage,
-                               int lane, int wave, const int* wbase) {
+                               int lane, int wave, const int* wbase, F ready) {
     // wbase (LDS, or null): running count, over the (level, segment) pairs, of the tiles that receive tokens in this
     // call.  The waves then share out those tiles alone; a store laid out for the worst case, or one that already
     // holds a long context, has many times more tiles than that.  Without the table every tile is looked at.
     const int n_runs = ODMKV_NQ * a.nseg;
-    const int total_tiles = wbase ? wbase[n_runs] : a.tile_base[ODMKV_NQ];
+    const int total_tiles = wbase ? uniform(wbase[n_runs]) : a.tile_base[ODMKV_NQ];
     const int stride = (gridDim.x >> 1) * QF_NW;
     int32_t* redo_count = a.redo + (IS_V ? 1 : 0);
     int32_t* redo_list = a.redo + 2 + (IS_V ? a.redo_cap : 0);
@@ -1210,25 +1332,23 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
         for (; wi < total_tiles; wi += stride) {
             int li, bh, tile, lo, hi;
             if (wbase) {
-                int e = 0;                                       // the largest pair with wbase[e] <= wi
-                for (int step = QF_MAX_RUNS / 2; step >= 1; step >>= 1)
-                    if (e + step < n_runs && wbase[e + step] <= wi) e += step;
+                const int e = find_run(wbase, n_runs, wi, lane);
                 li = e / a.nseg; bh = e - li * a.nseg;
-                const int old = a.old_count[e];
-                const int local = old / TILE + (wi - wbase[e]);
-                tile = a.s.seg_tile[li][bh] + local;
+                const int old = uniform(a.old_count[e]), first = uniform(a.s.seg_tile[li][bh]), count = uniform(a.s.seg_count[li][bh]);
+                const int local = old / TILE + (wi - uniform(wbase[e]));
+                tile = first + local;
                 lo = max(old - local * TILE, 0);
-                hi = min(a.s.seg_count[li][bh] - local * TILE, TILE);
+                hi = min(count - local * TILE, TILE);
             } else {
                 li = 0;
 #pragma unroll
                 for (int k = 1; k < ODMKV_NQ; ++k) li += (wi >= a.tile_base[k]);
                 tile = wi - a.tile_base[li];
                 const int32_t* seg_tile = a.s.seg_tile[li];
-                bh = find_segment(seg_tile, a.nseg, tile);
-                const int ts = (tile - seg_tile[bh]) * TILE;
-                lo = max(a.old_count[li * a.nseg + bh] - ts, 0);
-                hi = min(a.s.seg_count[li][bh] - ts, TILE);
+                bh = uniform(find_segment(seg_tile, a.nseg, tile));
+                const int ts = (tile - uniform(seg_tile[bh])) * TILE;
+                lo = max(uniform(a.old_count[li * a.nseg + bh]) - ts, 0);
+                hi = min(uniform(a.s.seg_count[li][bh]) - ts, TILE);
                 if (lo >= hi) continue;                         // nothing new in this tile (wave-uniform)
             }
             const int gt = a.tile_base[li] + tile;
@@ -1241,46 +1361,54 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
     const auto row_offset = [&](const QfTile& d, int pos) {
         return (size_t)(d.bh / a.Hkv) * a.sB + (size_t)(d.bh % a.Hkv) * a.sH + (size_t)(pos - a.pos_offset) * a.sT;
     };
+    const auto positions = [&](const QfTile& d) {
+        return lane >= d.lo && lane < d.hi ? a.s.pos[d.li][(size_t)d.tile * TILE + lane] : a.pos_offset;
+    };
+    const auto request = [&](const QfTile& d, int pos, QfRows& x) {
+        const int r16 = lane & 15, q = lane >> 4;
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) {
+            const int token = 16 * tb + r16;
+            const size_t off = row_offset(d, __shfl(pos, token, WAVE));
+            const uint4* row = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(base) + off) + q;
+            const bool on = token >= d.lo && token < d.hi;
+#pragma unroll
+            for (int ch = 0; ch < 4; ++ch) x[tb][ch] = on ? row[4 * ch] : make_uint4(0u, 0u, 0u, 0u);
+        }
+    };
 
     QfTile cur;
-    bool more = next_tile((blockIdx.x >> 1) * QF_NW + wave, cur);
+    QfRows xb;
+    bool more = next_tile(wave * (gridDim.x >> 1) + (blockIdx.x >> 1), cur);      // (a round of tiles goes over the workgroups first)
+    int pos = 0;
+    if (more) {
+        pos = positions(cur);
+        request(cur, pos, xb);
+    }
+    ready();
     if (!more) return;
+    const int mirrors = (qf_mirrors<2>(thrs, lane) ? 1 : 0) | (qf_mirrors<3>(thrs + thr_offset(1), lane) ? 2 : 0) | (qf_mirrors<4>(thrs + thr_offset(2), lane) ? 4 : 0);
     int n_listed = 0;                                           // == w.count between tiles
     if (lane == 0) w.count = 0;
-    int pos = 0;
-    if (lane >= cur.lo && lane < cur.hi) pos = a.s.pos[cur.li][(size_t)cur.tile * TILE + lane];
     while (true) {
+        // the lane index as a tile's phases see it: opaque, so that their addresses are computed there and not carried (spilled) round the loop
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
         const bool valid = lane >= cur.lo && lane < cur.hi;
-        size_t off = 0;
-        RowRegs<DT> x;
-        if (valid) {
-            off = row_offset(cur, pos);
-            x.load(base, off);
-        } else {
-            x.zero();
-        }
+        const size_t off = row_offset(cur, pos);
         // the next tile and its positions are found while this tile's rows are on their way
         QfTile nxt;
         more = next_tile(cur.wi + stride, nxt);
-        if (more && lane >= nxt.lo && lane < nxt.hi) pos = a.s.pos[nxt.li][(size_t)nxt.tile * TILE + lane];
+        if (more) pos = positions(nxt);
 
         // a token per lane: the norm in the definition's order, and what the matrix layout needs per token
-        float ss = 0.0f;
-#pragma unroll
-        for (int j = 0; j < HD; ++j) {
-            const float xj = x.get(j);
-            ss = __fmaf_rn(xj, xj, ss);
-        }
+        uint32_t any;
+        const float ss = qf_sum_squares<DT>(xb, any);
         const float norm = sqrtf(ss);
         bool odd = !(ss <= 3.4028234663852886e38f);              // a row with an infinite or NaN norm: exact kernel
-        if constexpr (DT != ODMKV_F16) {
-            // bf16 reaches down to 1e-38: a row whose squares vanish or nearly do (but which is not all zeros) also goes there
-            uint32_t any = 0u;
-#pragma unroll
-            for (int i = 0; i < RowRegs<DT>::N; ++i) any |= x.w[i];
-            odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
-        }
-        const bool ok = !__any(odd);
+        // bf16 reaches down to 1e-38: a row whose squares vanish or nearly do (but which is not all zeros) also goes there
+        if constexpr (DT != ODMKV_F16) odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
+        const bool ok = !__any(odd) && ((mirrors >> cur.li) & 1);
         const float* thr = thrs + thr_offset(cur.li);
         const bool direct = cur.li != 1 && cur.lo == 0 && (!IS_V || cur.hi == TILE);
         const int variant = cur.li == 0 ? (direct ? 0 : 1) : cur.li == 1 ? 2 : (direct ? 3 : 4);
@@ -1288,28 +1416,28 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
         int n = 0;
         if (ok) {
             const float den = norm + 1e-10f;
-            w.off[lane] = valid ? (unsigned long long)off : ~0ull;
+            w.off[lane] = off;
             w.den[lane] = den;
             w.rinv[lane] = 1.0f / den;
-            w.band[lane] = (valid && ss > 0.0f) ? (DT == ODMKV_F16 ? QF_BAND : QF_BAND_BF16) : -1.0f;  // rows of zeros: the estimate is the exact 0
+            const unsigned long long listed = __ballot(valid && ss > 0.0f);
             wave_lds_fence();
             switch (variant) {
-                case 0: qf_code_tile<DT, 2, IS_V, true>(base, piA, thr, w, stage, lane, cur.gt); break;
-                case 1: qf_code_tile<DT, 2, IS_V, false>(base, piA, thr, w, stage, lane, cur.gt); break;
-                case 2: qf_code_tile<DT, 3, IS_V, false>(base, piA, thr, w, stage, lane, cur.gt); break;
-                case 3: qf_code_tile<DT, 4, IS_V, true>(base, piA, thr, w, stage, lane, cur.gt); break;
-                default: qf_code_tile<DT, 4, IS_V, false>(base, piA, thr, w, stage, lane, cur.gt); break;
+                case 0: qf_code_tile<DT, 2, IS_V, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                case 1: qf_code_tile<DT, 2, IS_V, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                case 2: qf_code_tile<DT, 3, IS_V, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                case 3: qf_code_tile<DT, 4, IS_V, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                default: qf_code_tile<DT, 4, IS_V, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
             }
             wave_lds_fence();
             n = w.count;
         }
         if (ok && n <= QF_LIST) {
             switch (variant) {
-                case 0: qf_store_tile<2, IS_V, true>(a, stage, lane, cur.li, cur.tile, cur.lo); break;
-                case 1: qf_store_tile<2, IS_V, false>(a, stage, lane, cur.li, cur.tile, cur.lo); break;
-                case 2: qf_store_tile<3, IS_V, false>(a, stage, lane, cur.li, cur.tile, cur.lo); break;
-                case 3: qf_store_tile<4, IS_V, true>(a, stage, lane, cur.li, cur.tile, cur.lo); break;
-                default: qf_store_tile<4, IS_V, false>(a, stage, lane, cur.li, cur.tile, cur.lo); break;
+                case 0: qf_store_tile<2, IS_V, true>(a, stage, ln, cur.li, cur.tile, cur.lo); break;
+                case 1: qf_store_tile<2, IS_V, false>(a, stage, ln, cur.li, cur.tile, cur.lo); break;
+                case 2: qf_store_tile<3, IS_V, false>(a, stage, ln, cur.li, cur.tile, cur.lo); break;
+                case 3: qf_store_tile<4, IS_V, true>(a, stage, ln, cur.li, cur.tile, cur.lo); break;
+                default: qf_store_tile<4, IS_V, false>(a, stage, ln, cur.li, cur.tile, cur.lo); break;
             }
             if (valid) (IS_V ? a.s.vnorm[cur.li] : a.s.knorm[cur.li])[(size_t)cur.tile * TILE + lane] = norm;
             n_listed = n;
@@ -1320,36 +1448,39 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
             n_listed = n_before;
             if (ok && lane == 0) w.count = n_before;
         }
-        wave_lds_fence();                                       // staging area and scratch free for the next tile
+        wave_lds_fence();                                       // staging area free for the next tile
         if (n_listed >= WAVE || (!more && n_listed > 0)) {
             __builtin_amdgcn_s_waitcnt(0);                      // this wave's codes, positions and norms are in memory
             while (n_listed >= WAVE) {
                 n_listed -= WAVE;
-                qf_fix_listed<DT, IS_V>(a, thrs, w, lane, n_listed, WAVE);
+                qf_fix_listed<DT, IS_V>(a, thrs, w, ln, n_listed, WAVE, cur.gt);
             }
-            if (!more && n_listed > 0) { qf_fix_listed<DT, IS_V>(a, thrs, w, lane, 0, n_listed); n_listed = 0; }
+            if (!more && n_listed > 0) { qf_fix_listed<DT, IS_V>(a, thrs, w, ln, 0, n_listed, cur.gt); n_listed = 0; }
             if (lane == 0) w.count = n_listed;
-            wave_lds_fence();
         }
+        wave_lds_fence();                                       // and the scratch
         if (!more) break;
+        request(nxt, pos, xb);
         cur = nxt;
     }
 }
 
-template <int DT>
-__device__ static inline void qf_load_rotation(const float* pi, uint16_t* pih, int tid) {
-    // Pi -> hi + lo in the rows' 16-bit type, in the order the matrix instruction reads a 16-output x 32-step block:
-    // lane 16q + r of block (ob, ch) holds Pi[16 ob + r][32 ch + 8 q .. + 7]
-    // (all of a thread's reads are asked for at once: eight round trips to memory would cost more
-    // than the tiles of a short call)
+// Pi -> hi + lo in the rows' 16-bit type, in the order the matrix instruction reads a 16-output x 32-step block:
+// lane 16q + r of block (ob, ch) holds Pi[16 ob + r][32 ch + 8 q .. + 7]
+// (all of a thread's reads are asked for at once, and ahead of the first tile's: eight round trips to memory would cost more
+// than the tiles of a short call)
+#define QF_PI_READS ((HD * HD / 4 + QF_NW * 64 - 1) / (QF_NW * 64))
+__device__ static __forceinline__ void qf_request_rotation(const float* pi, float4 (&p)[QF_PI_READS], int tid) {
     const float4* __restrict__ pi4 = reinterpret_cast<const float4*>(pi);
-    constexpr int PER_THREAD = HD * HD / 4 / (QF_NW * 64);
-    float4 p[PER_THREAD];
 #pragma unroll
-    for (int k = 0; k < PER_THREAD; ++k) p[k] = pi4[tid + k * (QF_NW * 64)];
+    for (int k = 0; k < QF_PI_READS; ++k) p[k] = pi4[min(tid + k * (QF_NW * 64), HD * HD / 4 - 1)];
+}
+template <int DT>
+__device__ static __forceinline__ void qf_lay_out_rotation(const float4 (&p)[QF_PI_READS], uint16_t* pih, int tid) {
 #pragma unroll
-    for (int k = 0; k < PER_THREAD; ++k) {
+    for (int k = 0; k < QF_PI_READS; ++k) {
         const int c = tid + k * (QF_NW * 64);               // four consecutive j of row i
+        if (c >= HD * HD / 4) break;
         const int i = c >> 5, j = (c & 31) * 4;
         const int ob = i >> 4, r = i & 15, ch = j >> 5, q = (j >> 3) & 3, e = j & 7;
         const int dst = (((ob * 4 + ch) * 64) + 16 * q + r) * 8 + e;
@@ -1369,12 +1500,12 @@ template <int DT>
 __global__ __launch_bounds__(QF_NW * 64) void quant_pack_f16_kernel(QuantArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
     uint16_t* pih = reinterpret_cast<uint16_t*>(smem);
-    float* thrs = reinterpret_cast<float*>(smem + QF_PI_BYTES + QF_NW * QP_STAGE);
+    float* thrs = reinterpret_cast<float*>(smem + QF_PI_BYTES + QF_NW * QF_STAGE);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    uint8_t* stage = smem + QF_PI_BYTES + wave * QP_STAGE;
-    QfWave& w = reinterpret_cast<QfWave*>(smem + QF_PI_BYTES + QF_NW * QP_STAGE + QF_THR_BYTES)[wave];
-    int* wbase = reinterpret_cast<int*>(smem + QF_PI_BYTES + QF_NW * QP_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave));
+    uint8_t* stage = smem + QF_PI_BYTES + wave * QF_STAGE;
+    QfWave& w = reinterpret_cast<QfWave*>(smem + QF_PI_BYTES + QF_NW * QF_STAGE + QF_THR_BYTES)[wave];
+    int* wbase = reinterpret_cast<int*>(smem + QF_PI_BYTES + QF_NW * QF_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave));
     const bool is_v = (blockIdx.x & 1) != 0;
     const int n_runs = ODMKV_NQ * a.nseg;
     const bool walk_table = n_runs <= QF_MAX_RUNS;
@@ -1389,14 +1520,11 @@ __global__ __launch_bounds__(QF_NW * 64) void quant_pack_f16_kernel(QuantArgs a)
             wbase[e + 1] = n;
         }
     }
-    {
-        qf_load_rotation<DT>(is_v ? a.pi_v : a.pi_k, pih, tid);
-        for (int i = tid; i < QP_THR_FLOATS; i += QF_NW * 64) {
-            const int li = i < 3 ? 0 : i < 10 ? 1 : i < 25 ? 2 : 3;
-            const int k = i - thr_offset(li);
-            thrs[i] = decision_threshold(a.cb[codebook_offset(li) + k], a.cb[codebook_offset(li) + k + 1]);
-        }
-    }
+    float4 rotation[QF_PI_READS];
+    qf_request_rotation(is_v ? a.pi_v : a.pi_k, rotation, tid);
+    const int t_li = tid < 3 ? 0 : tid < 10 ? 1 : tid < 25 ? 2 : 3, t_at = codebook_offset(t_li) + tid - thr_offset(t_li);
+    static_assert(QP_THR_FLOATS <= QF_NW * 64, "a threshold per thread");
+    const float c_lo = tid < QP_THR_FLOATS ? a.cb[t_at] : 0.0f, c_hi = tid < QP_THR_FLOATS ? a.cb[t_at + 1] : 0.0f;
     __syncthreads();
     if (walk_table && wave == 0) {
         // running sum by one wave: 16 entries per lane, a scan over the lanes' totals, the entries again
@@ -1416,8 +1544,13 @@ __global__ __launch_bounds__(QF_NW * 64) void quant_pack_f16_kernel(QuantArgs a)
     }
     __syncthreads();
     const uint4* piA = reinterpret_cast<const uint4*>(smem);
-    if (is_v) qf_walk<DT, true>(a, piA, thrs, w, stage, lane, wave, walk_table ? wbase : nullptr);
-    else qf_walk<DT, false>(a, piA, thrs, w, stage, lane, wave, walk_table ? wbase : nullptr);
+    const auto ready = [&] {
+        qf_lay_out_rotation<DT>(rotation, pih, tid);
+        if (tid < QP_THR_FLOATS) thrs[tid] = decision_threshold(c_lo, c_hi);
+        __syncthreads();
+    };
+    if (is_v) qf_walk<DT, true>(a, piA, thrs, w, stage, lane, wave, walk_table ? wbase : nullptr, ready);
+    else qf_walk<DT, false>(a, piA, thrs, w, stage, lane, wave, walk_table ? wbase : nullptr, ready);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1550,7 +1683,7 @@ extern "C" size_t odmkv_pack_workspace_bytes(int B, int Hkv, int T) {
 
 template <int DT>
 static int launch_quant_f16(const QuantArgs& qa, hipStream_t st) {
-    const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QP_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave) + (QF_MAX_RUNS + 1) * sizeof(int);
+    const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QF_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave) + (QF_MAX_RUNS + 1) * sizeof(int);
     ODMKV_ALLOW_LDS((quant_pack_f16_kernel<DT>), lds);
     const int total = qa.tile_base[ODMKV_NQ];
     int dev = 0, cus = 256;
@@ -2034,13 +2167,12 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
     for (int wi = wg * DQ_NW + wave; wi < total; wi += n_wg * DQ_NW) {
         int li, bh, tile, hi;
         if (table) {
-            int e = 0;                                           // the largest pair with wbase[e] <= wi
-            for (int step = DQ_MAX_RUNS / 2; step >= 1; step >>= 1)
-                if (e + step < n_runs && wbase[e + step] <= wi) e += step;
+            const int e = find_run(wbase, n_runs, wi, lane);
             li = e / a.nseg; bh = e - li * a.nseg;
-            const int local = wi - wbase[e];
-            tile = a.s.seg_tile[li][bh] + local;
-            hi = min(a.s.seg_count[li][bh] - local * TILE, TILE);
+            const int first = uniform(a.s.seg_tile[li][bh]), count = uniform(a.s.seg_count[li][bh]);
+            const int local = wi - uniform(wbase[e]);
+            tile = first + local;
+            hi = min(count - local * TILE, TILE);
         } else {
             li = 0;
 #pragma unroll
@@ -2164,28 +2296,53 @@ extern "C" int odmkv_dequant_from(const odmkv_packed_t* store, void* K, void* V,
 // rows outside the store on the matrix cores: the 16-bit quantiser's estimate with the codes as bytes or in the reference's
 // container, and the dequantiser from byte codes.  Workgroups of the even index take job 0, of the odd one job 1 (keys and
 // values of a layer in one launch), a wave a tile of 64 rows.  A row per lane without them took 150 us for 64512 rows (the
-// fused multiply-adds of the rotation on the vector ALU); here keys and values of 64512 rows each are quantised in 33 us and
+// fused multiply-adds of the rotation on the vector ALU); here keys and values of 64512 rows each are quantised in 29 us and
 // dequantised in 26 us.
 // ------------------------------------------------------------------------------------------------
 struct RowsArgs { RowsJob job[2]; int n_jobs; };
 
-template <int DT, int W>
+template <int DT, int W, typename F>
 __device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* thr, QfWave& w, uint8_t* stage, int lane, long long tile0,
-                               long long stride) {
+                               long long stride, F ready) {
     const long long tiles = (j.n + TILE - 1) / TILE;
     const int row_bytes = j.packed ? container_bytes(W) : HD;
     constexpr int EFF = W == 3 ? 4 : W;
     int n_listed = 0, it = 0;                                   // it: the tile's number in this wave's walk (what the list keeps)
+    // rows of a tile as matrix operands; off: the element offset of the lane's own row, found once and handed round
+    const auto request = [&](long long tile, long long& off, QfRows& x) {
+        const long long r = tile * TILE + lane;
+        const int rows = (int)min((long long)TILE, j.n - tile * TILE), r16 = lane & 15, q = lane >> 4;
+        off = r < j.n ? row_offset(j, r) : 0;
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) {
+            const int token = 16 * tb + r16;
+            const uint32_t lo = __shfl((uint32_t)off, token, WAVE), hi = __shfl((uint32_t)(off >> 32), token, WAVE);
+            const uint4* row = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(j.x) + (long long)(((unsigned long long)hi << 32) | lo)) + q;
+            const bool on = token < rows;
+#pragma unroll
+            for (int ch = 0; ch < 4; ++ch) x[tb][ch] = on ? row[4 * ch] : make_uint4(0u, 0u, 0u, 0u);
+        }
+    };
+    long long off = 0;
+    QfRows xb;
+    if (tile0 < tiles) request(tile0, off, xb);
+    ready();
+    const bool mirror = qf_mirrors<W>(thr, lane);
     if (lane == 0) w.count = 0;
     const auto fix = [&](int first, int n) {                    // n <= 64 listed values, a lane each, by the definition
         const bool on = lane < n;
         const uint32_t e = w.list[first + (on ? lane : 0)];
         const int out = (e >> 6) & 127;
         const long long r = (tile0 + (long long)(e >> 13) * stride) * TILE + (e & 63);
-        // written by this wave a moment ago: read past the vector cache
-        const float den = __hip_atomic_load(j.norms + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1e-10f;
+        size_t at = w.off[e & 63];
+        float den = w.den[e & 63];
+        if ((int)(e >> 13) != it) {                             // of an earlier tile
+            // written by this wave a moment ago: read past the vector cache
+            den = __hip_atomic_load(j.norms + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1e-10f;
+            at = (size_t)row_offset(j, r);
+        }
         RowRegs<DT> x;
-        x.load(j.x, (size_t)row_offset(j, r));
+        x.load(j.x, at);
         const float y = qf_chain<DT>(x, reinterpret_cast<const float4*>(j.pi + out * HD), den);
         int code = 0;
 #pragma unroll
@@ -2199,54 +2356,60 @@ __device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* 
         if (old != (uint32_t)code) atomicXor(word, (old ^ (uint32_t)code) << (bit & 31));
     };
     for (long long tile = tile0; tile < tiles; tile += stride, ++it) {
+        int ln = lane;                                          // opaque, as in qf_walk
+        asm volatile("" : "+v"(ln));
         const long long r = tile * TILE + lane;
         const bool valid = r < j.n;
-        const long long off = valid ? row_offset(j, r) : 0;
-        RowRegs<DT> x;
-        if (valid) x.load(j.x, (size_t)off);
-        else x.zero();
-        float ss = 0.0f;
-#pragma unroll
-        for (int e = 0; e < HD; ++e) {
-            const float xj = x.get(e);
-            ss = __fmaf_rn(xj, xj, ss);
-        }
+        uint32_t any;
+        const float ss = qf_sum_squares<DT>(xb, any);
         const float norm = sqrtf(ss);
         bool odd = !(ss <= 3.4028234663852886e38f);              // as in qf_walk
-        if constexpr (DT != ODMKV_F16) {
-            uint32_t any = 0u;
-#pragma unroll
-            for (int i = 0; i < RowRegs<DT>::N; ++i) any |= x.w[i];
-            odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
-        }
-        const bool ok = !__any(odd);
+        if constexpr (DT != ODMKV_F16) odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
+        const bool ok = !__any(odd) && mirror;
         const int n_before = n_listed;
         int n = 0;
         if (ok) {
             const float den = norm + 1e-10f;
-            w.off[lane] = valid ? (unsigned long long)off : ~0ull;
+            w.off[lane] = (unsigned long long)off;
+            w.den[lane] = den;
             w.rinv[lane] = 1.0f / den;
-            w.band[lane] = (valid && ss > 0.0f) ? (DT == ODMKV_F16 ? QF_BAND : QF_BAND_BF16) : -1.0f;
+            const unsigned long long listed = __ballot(valid && ss > 0.0f);
             wave_lds_fence();
-            qf_code_tile<DT, W, false, false>(j.x, piA, thr, w, stage, lane, it);
+            qf_code_tile<DT, W, false, false>(xb, piA, thr, w, stage, ln, it, listed);
             wave_lds_fence();
             n = w.count;
         }
         if (ok && n <= QF_LIST) {
             const int rows = (int)min((long long)TILE, j.n - tile * TILE);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {                       // sixteen codes of a row per lane and turn
-                const int token = 8 * i + (lane >> 3), piece = lane & 7;
-                const uint4 v = *reinterpret_cast<const uint4*>(stage + token * CODE_ROW + 16 * piece);
+            for (int i = 0; i < 4; ++i) {                       // 32 codes of a row per lane and turn
+                const int token = 16 * i + (ln >> 2), piece = ln & 3;
+                const uint4 v = *reinterpret_cast<const uint4*>(stage + token * Direct<4>::ROW_K + 16 * piece);
                 if (token >= rows) continue;
                 uint8_t* dst = j.codes + (size_t)(tile * TILE + token) * row_bytes;
-                if (!j.packed) { *reinterpret_cast<uint4*>(dst + 16 * piece) = v; continue; }
-                const uint32_t b[4] = {v.x, v.y, v.z, v.w};     // four codes each -> EFF bits apart
-                uint32_t g[4];
+                uint32_t g[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-                for (int k = 0; k < 4; ++k) g[k] = (b[k] & 0xffu) | ((b[k] >> (8 - EFF)) & (0xffu << EFF)) | ((b[k] >> (16 - 2 * EFF)) & (0xffu << (2 * EFF))) | ((b[k] >> (24 - 3 * EFF)) & (0xffu << (3 * EFF)));
-                if constexpr (EFF == 2) *reinterpret_cast<uint32_t*>(dst + 4 * piece) = (g[0] & 0xffu) | ((g[1] & 0xffu) << 8) | ((g[2] & 0xffu) << 16) | (g[3] << 24);
-                else *reinterpret_cast<uint2*>(dst + 8 * piece) = make_uint2((g[0] & 0xffffu) | (g[1] << 16), (g[2] & 0xffffu) | (g[3] << 16));
+                for (int k = 0; k < 4; ++k) g[k] = qf_decode<W, 4>(g[k]);
+                if (!j.packed) {
+                    uint32_t b[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const uint32_t h = g[k >> 1] >> (16 * (k & 1));      // four codes -> a byte each
+                        b[k] = (h & 0xfu) | ((h & 0xf0u) << 4) | ((h & 0xf00u) << 8) | ((h & 0xf000u) << 12);
+                    }
+                    *reinterpret_cast<uint4*>(dst + 32 * piece) = make_uint4(b[0], b[1], b[2], b[3]);
+                    *reinterpret_cast<uint4*>(dst + 32 * piece + 16) = make_uint4(b[4], b[5], b[6], b[7]);
+                } else if constexpr (EFF == 4) {
+                    *reinterpret_cast<uint4*>(dst + 16 * piece) = make_uint4(g[0], g[1], g[2], g[3]);
+                } else {
+                    uint32_t c[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {                // 2 bits of every four -> side by side
+                        const uint32_t h = (g[k] | (g[k] >> 2)) & 0x0f0f0f0fu, t = (h | (h >> 4)) & 0x00ff00ffu;
+                        c[k] = (t | (t >> 8)) & 0xffffu;
+                    }
+                    *reinterpret_cast<uint2*>(dst + 8 * piece) = make_uint2(c[0] | (c[1] << 16), c[2] | (c[3] << 16));
+                }
             }
             if (valid) j.norms[r] = norm;
             n_listed = n;
@@ -2262,8 +2425,9 @@ __device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* 
             while (n_listed >= WAVE) { n_listed -= WAVE; fix(n_listed, WAVE); }
             if (!more && n_listed > 0) { fix(0, n_listed); n_listed = 0; }
             if (lane == 0) w.count = n_listed;
-            wave_lds_fence();
         }
+        wave_lds_fence();
+        if (more) request(tile + stride, off, xb);
     }
 }
 
@@ -2273,18 +2437,24 @@ __global__ __launch_bounds__(QF_NW * 64) void quant_rows_f16_kernel(RowsArgs a) 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const RowsJob& j = a.job[a.n_jobs == 2 ? (blockIdx.x & 1) : 0];
-    float* thr = reinterpret_cast<float*>(smem + QF_PI_BYTES + QF_NW * QP_STAGE);
-    uint8_t* stage = smem + QF_PI_BYTES + wave * QP_STAGE;
-    QfWave& w = reinterpret_cast<QfWave*>(smem + QF_PI_BYTES + QF_NW * QP_STAGE + QF_THR_BYTES)[wave];
-    qf_load_rotation<DT>(j.pi, reinterpret_cast<uint16_t*>(smem), tid);
-    if (tid < (1 << j.bits) - 1) thr[tid] = decision_threshold(j.cb[tid], j.cb[tid + 1]);
-    __syncthreads();
+    float* thr = reinterpret_cast<float*>(smem + QF_PI_BYTES + QF_NW * QF_STAGE);
+    uint8_t* stage = smem + QF_PI_BYTES + wave * QF_STAGE;
+    QfWave& w = reinterpret_cast<QfWave*>(smem + QF_PI_BYTES + QF_NW * QF_STAGE + QF_THR_BYTES)[wave];
+    float4 rotation[QF_PI_READS];
+    qf_request_rotation(j.pi, rotation, tid);
+    const bool has_thr = tid < (1 << j.bits) - 1;
+    const float c_lo = has_thr ? j.cb[tid] : 0.0f, c_hi = has_thr ? j.cb[tid + 1] : 0.0f;
+    const auto ready = [&] {
+        qf_lay_out_rotation<DT>(rotation, reinterpret_cast<uint16_t*>(smem), tid);
+        if (has_thr) thr[tid] = decision_threshold(c_lo, c_hi);
+        __syncthreads();
+    };
     const uint4* piA = reinterpret_cast<const uint4*>(smem);
-    const long long first = (long long)(blockIdx.x / a.n_jobs) * QF_NW + wave, stride = (long long)(gridDim.x / a.n_jobs) * QF_NW;
+    const long long first = (long long)wave * (gridDim.x / a.n_jobs) + blockIdx.x / a.n_jobs, stride = (long long)(gridDim.x / a.n_jobs) * QF_NW;
     switch (j.bits) {
-        case 2: qr_walk<DT, 2>(j, piA, thr, w, stage, lane, first, stride); break;
-        case 3: qr_walk<DT, 3>(j, piA, thr, w, stage, lane, first, stride); break;
-        default: qr_walk<DT, 4>(j, piA, thr, w, stage, lane, first, stride); break;
+        case 2: qr_walk<DT, 2>(j, piA, thr, w, stage, lane, first, stride, ready); break;
+        case 3: qr_walk<DT, 3>(j, piA, thr, w, stage, lane, first, stride, ready); break;
+        default: qr_walk<DT, 4>(j, piA, thr, w, stage, lane, first, stride, ready); break;
     }
 }
 
@@ -2333,7 +2503,7 @@ static dim3 rows_grid(const RowsJob* jobs, int n_jobs, int waves) {
 }
 
 int launch_quantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
-    const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QP_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave);
+    const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QF_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave);
     if (dtype == ODMKV_F16) ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_F16>, lds);
     else ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_BF16>, lds);
     RowsArgs a;

@@ -378,6 +378,35 @@ def test_fp16_rows_next_to_thresholds_get_the_exact_codes(per_row, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shift,covered", [(0.0, True), (2e-7, True), (3e-3, False)])
+def test_fp16_tables_that_do_not_mirror_go_to_the_exact_kernel(shift, covered, dtype):
+    """The matrix-core quantiser codes |y - middle| against half the thresholds, which needs a table that is the same on both
+    sides to within 1e-6; the lowest centroid moved by 2e-7 still is, by 3e-3 is not.  Ragged tiles, and an append onto them."""
+    g = torch.Generator().manual_seed(3)
+    B, H, T = 1, 2, 700
+    k = torch.randn(B, H, T, 128, generator=g).to(dtype).to(DEV)
+    v = torch.randn(B, H, T, 128, generator=g).to(dtype).to(DEV)
+    bits = torch.tensor([2, 3, 4], dtype=torch.int32)[torch.randint(3, (B, H, T), generator=g)].to(DEV)
+    stores = []
+    for x, y in ((k, v), (k.float(), v.float())):
+        st = _state(dtype=dtype)
+        st.codebooks = st.codebooks.clone()
+        for at in (0, 4, 12):                                  # the lowest centroid of 2, 3 and 4 bits
+            st.codebooks[at] -= shift
+        st.prefill(x[:, :, :411], y[:, :, :411], bits[:, :, :411])
+        st.append(x[:, :, 411:], y[:, :, 411:], bits[:, :, 411:])
+        stores.append(st)
+    if covered:
+        assert _handed_over(stores[0], B, H, T - 411) == (0, 0)
+    for li, w in enumerate((2, 3, 4)):
+        first = stores[0]._seg_tile[li]
+        used = torch.cat([torch.arange(int(first[h]), int(first[h]) + -(-int((bits[0, h] == w).sum()) // 64)) for h in range(H)]).to(DEV)
+        for name, per_tile in (("kcodes", 1024 * w), ("vcodes", 1024 * w), ("knorm", 64), ("vnorm", 64)):
+            a, b = (st._bufs[name][li].view(-1, per_tile)[used] for st in stores)
+            assert torch.equal(a, b), (name, w)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_fp16_special_rows_and_ordinary_ones(dtype):
     g = torch.Generator().manual_seed(11)
     B, H, T = 2, 2, 1500
