@@ -2003,28 +2003,33 @@ struct DequantArgs {
 // output j = 32 (jb >> 1) + 8 (r >> 2) + 4 (jb & 1) + (r & 3): a lane's accumulators of two neighbouring blocks are then
 // eight consecutive outputs.
 // UP: times 2^UP (see dequant_rows_f16_kernel).
+// A thread reads eight rows of one column and writes an operand's 16 bytes at once; four neighbours of a row scattered two bytes
+// at a time met eight to a bank: 4 us of every launch.
+#define DQ_PI_GROUPS (HD * HD / 8 / (DQ_NW * 64))
+__device__ static __forceinline__ void dq_request_rotation(const float* __restrict__ pi, float (&p)[8 * DQ_PI_GROUPS], int tid) {
+#pragma unroll
+    for (int k = 0; k < DQ_PI_GROUPS; ++k) {
+        const int g = tid + k * (DQ_NW * 64), j = g & (HD - 1), i = 8 * (g / HD);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[8 * k + e] = pi[(i + e) * HD + j];
+    }
+}
 template <int UP>
-__device__ static inline void dq_load_rotation(const float* pi, uint16_t* pih, int tid) {
-    const float4* __restrict__ src = reinterpret_cast<const float4*>(pi);
-    constexpr int PER_THREAD = HD * HD / 4 / (DQ_NW * 64);
-    float4 p[PER_THREAD];
+__device__ static __forceinline__ void dq_lay_out_rotation(const float (&p)[8 * DQ_PI_GROUPS], uint4* pih, int tid) {
 #pragma unroll
-    for (int k = 0; k < PER_THREAD; ++k) p[k] = src[tid + k * (DQ_NW * 64)];
+    for (int k = 0; k < DQ_PI_GROUPS; ++k) {
+        const int g = tid + k * (DQ_NW * 64), j = g & (HD - 1), ib = g / HD;
+        const int ch = ib >> 2, q = ib & 3, jb = 2 * (j >> 5) + ((j >> 2) & 1), r = 4 * ((j >> 3) & 3) + (j & 3);
+        uint32_t h[4], l[4];
 #pragma unroll
-    for (int k = 0; k < PER_THREAD; ++k) {
-        const int c = tid + k * (DQ_NW * 64);                // four consecutive j of row i
-        const int i = c >> 5, j0 = (c & 31) * 4;
-        const int ch = i >> 5, q = (i >> 3) & 3, e = i & 7;
-        const float pv[4] = {p[k].x, p[k].y, p[k].z, p[k].w};
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int j = j0 + t, jb = 2 * (j >> 5) + ((j >> 2) & 1), r = 4 * ((j >> 3) & 3) + (j & 3);
-            const int dst = (((jb * 4 + ch) * 64) + 16 * q + r) * 8 + e;
-            const float x = pv[t] * (float)(1 << UP);
-            const uint16_t h = Elem<ODMKV_F16>::from_f32(x);
-            pih[dst] = h;
-            pih[HD * HD + dst] = Elem<ODMKV_F16>::from_f32(x - Elem<ODMKV_F16>::to_f32(h));
+        for (int e = 0; e < 4; ++e) {
+            const float x0 = p[8 * k + 2 * e] * (float)(1 << UP), x1 = p[8 * k + 2 * e + 1] * (float)(1 << UP);
+            const uint16_t h0 = Elem<ODMKV_F16>::from_f32(x0), h1 = Elem<ODMKV_F16>::from_f32(x1);
+            h[e] = h0 | ((uint32_t)h1 << 16);
+            l[e] = Elem<ODMKV_F16>::from_f32(x0 - Elem<ODMKV_F16>::to_f32(h0)) | ((uint32_t)Elem<ODMKV_F16>::from_f32(x1 - Elem<ODMKV_F16>::to_f32(h1)) << 16);
         }
+        pih[(jb * 4 + ch) * 64 + 16 * q + r] = make_uint4(h[0], h[1], h[2], h[3]);
+        pih[HD * HD / 8 + (jb * 4 + ch) * 64 + 16 * q + r] = make_uint4(l[0], l[1], l[2], l[3]);
     }
 }
 template <int UP>
@@ -2039,7 +2044,8 @@ __device__ static inline uint32_t dq_centroid(float c) {
 // Every operand of Pi^T is read once for all four token blocks (64 KB of LDS reads per tile; with a read per block, 256 KB,
 // the LDS pipe and the latency of its reads set the time), whose four accumulators are chains of their own; a lane stores 16
 // bytes of a row at a time, a token's four lanes 64.  A 2-bit layer of 32k tokens and 8 heads (both tensors): 81 -> 39 us
-// repeated on one layer, 66 us where the rows come from memory (the layers of a prefill, one after the other).
+// repeated on one layer, 66 us where the rows come from memory (the layers of a prefill, one after the other); 59 with a tile's codes
+// requested under the products of the tile before it (18 us instead of 24 for a tile a wavefront).
 template <int DT, int UP>
 __device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* codes, const uint32_t* cb, const float* norms,
                                                const long long* offs, void* out, int lane) {
@@ -2096,14 +2102,11 @@ __device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* 
 // the tile's codes of width W -> one byte each in LDS, [token][dim]: the matrix operand wants eight consecutive dims of a
 // token per lane, the tile keeps (4 tokens x 32 dims) of keys or (16 tokens x 8 dims) of values per lane
 template <int W>
-__device__ static __forceinline__ void dq_unpack(const uint8_t* src, bool is_v, uint8_t* codes, int lane) {
+__device__ static __forceinline__ void dq_unpack(const uint4 (&raw)[8], bool is_v, uint8_t* codes, int lane) {
     const int n = lane & 15, j = lane >> 4;
     uint32_t words[4 * W];
 #pragma unroll
-    for (int c = 0; c < W; ++c) {
-        const uint4 v = *reinterpret_cast<const uint4*>(src + ((size_t)c * TILE + lane) * 16);
-        words[4 * c] = v.x; words[4 * c + 1] = v.y; words[4 * c + 2] = v.z; words[4 * c + 3] = v.w;
-    }
+    for (int c = 0; c < W; ++c) { words[4 * c] = raw[c].x; words[4 * c + 1] = raw[c].y; words[4 * c + 2] = raw[c].z; words[4 * c + 3] = raw[c].w; }
     if (!is_v) {
 #pragma unroll
         for (int b = 0; b < 4; ++b)
@@ -2141,8 +2144,10 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
     if (table)
         for (int e = tid; e < DQ_MAX_RUNS; e += DQ_NW * 64)
             wbase[e + 1] = e < n_runs ? (a.s.seg_count[e / a.nseg][e % a.nseg] + TILE - 1) / TILE : 0;
-    dq_load_rotation<0>(is_v ? a.pi_v : a.pi_k, reinterpret_cast<uint16_t*>(smem), tid);
-    for (int i = tid; i < DQ_CB_WORDS; i += DQ_NW * 64) cb[i] = dq_centroid<0>(a.cb[i]);
+    float rotation[8 * DQ_PI_GROUPS];
+    dq_request_rotation(is_v ? a.pi_v : a.pi_k, rotation, tid);
+    static_assert(DQ_CB_WORDS <= DQ_NW * 64, "a centroid per thread");
+    const float centroid = tid < CODEBOOK_FLOATS ? a.cb[tid] : 0.0f;
     __syncthreads();
     if (table && wave == 0) {                                  // 16 entries per lane, a scan over the lanes' totals
         int mine[DQ_MAX_RUNS / 64], tot = 0;
@@ -2162,45 +2167,65 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
     __syncthreads();
     const uint4* piA = reinterpret_cast<const uint4*>(smem);
     void* out = is_v ? a.V : a.K;
-    const int wg = blockIdx.x >> 1, n_wg = gridDim.x >> 1;
-    const int total = table ? wbase[n_runs] : a.tile_base[ODMKV_NQ];
-    for (int wi = wg * DQ_NW + wave; wi < total; wi += n_wg * DQ_NW) {
-        int li, bh, tile, hi;
-        if (table) {
-            const int e = find_run(wbase, n_runs, wi, lane);
-            li = e / a.nseg; bh = e - li * a.nseg;
-            const int first = uniform(a.s.seg_tile[li][bh]), count = uniform(a.s.seg_count[li][bh]);
-            const int local = wi - uniform(wbase[e]);
-            tile = first + local;
-            hi = min(count - local * TILE, TILE);
-        } else {
-            li = 0;
+    const int total = table ? uniform(wbase[n_runs]) : a.tile_base[ODMKV_NQ];
+    const int n_wg = gridDim.x >> 1, stride = n_wg * DQ_NW;
+    // the tile at or behind wi that has tokens to write: its codes, norms and rows are asked for
+    int li = 0, hi = 0;
+    uint4 raw[8];
+    float norm = 0.0f;
+    long long off = -1ll;
+    const auto next_tile = [&](int wi) -> int {
+        for (; wi < total; wi += stride) {
+            int bh, tile;
+            if (table) {
+                const int e = find_run(wbase, n_runs, wi, lane);
+                li = e / a.nseg; bh = e - li * a.nseg;
+                const int first = uniform(a.s.seg_tile[li][bh]), count = uniform(a.s.seg_count[li][bh]);
+                const int local = wi - uniform(wbase[e]);
+                tile = first + local;
+                hi = min(count - local * TILE, TILE);
+            } else {
+                li = 0;
 #pragma unroll
-            for (int k = 1; k < ODMKV_NQ; ++k) li += (wi >= a.tile_base[k]);
-            tile = wi - a.tile_base[li];
-            bh = find_segment(a.s.seg_tile[li], a.nseg, tile);
-            hi = min(a.s.seg_count[li][bh] - (tile - a.s.seg_tile[li][bh]) * TILE, TILE);
-            if (hi <= 0) continue;                               // wave-uniform
-        }
-        // positions ascend inside a segment: a tile whose last token lies before t_min has nothing to write
-        const int32_t* pos = a.s.pos[li] + (size_t)tile * TILE;
-        if (a.t_min > 0 && pos[hi - 1] < a.t_min) continue;
-        const bool valid = lane < hi;
-        {
+                for (int k = 1; k < ODMKV_NQ; ++k) li += (wi >= a.tile_base[k]);
+                tile = wi - a.tile_base[li];
+                bh = uniform(find_segment(a.s.seg_tile[li], a.nseg, tile));
+                hi = uniform(min(a.s.seg_count[li][bh] - (tile - a.s.seg_tile[li][bh]) * TILE, TILE));
+                if (hi <= 0) continue;                           // wave-uniform
+            }
+            const int32_t* pos = a.s.pos[li] + (size_t)tile * TILE;
+            const bool valid = lane < hi;
             const int t = valid ? pos[lane] : -1;
+            // positions ascend inside a segment: a tile whose last token lies before t_min has nothing to write
+            if (a.t_min > 0 && __builtin_amdgcn_readlane(t, hi - 1) < a.t_min) continue;
+            const int W = width_of(li);
+            const uint4* src = reinterpret_cast<const uint4*>((is_v ? a.s.vcodes[li] : a.s.kcodes[li]) + (size_t)tile * (TILE * 16) * W) + lane;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) raw[c] = c < W ? src[c * TILE] : make_uint4(0u, 0u, 0u, 0u);
+            norm = valid ? (is_v ? a.s.vnorm[li] : a.s.knorm[li])[(size_t)tile * TILE + lane] : 0.0f;
             const bool write = valid && t >= a.t_min && t < a.T;
-            offs[lane] = write ? (long long)((size_t)(bh / a.s.Hkv) * a.sB + (size_t)(bh % a.s.Hkv) * a.sH + (size_t)t * a.sT) : -1ll;
-            norms[lane] = valid ? (is_v ? a.s.vnorm[li] : a.s.knorm[li])[(size_t)tile * TILE + lane] : 0.0f;
+            off = write ? (long long)((size_t)(bh / a.s.Hkv) * a.sB + (size_t)(bh % a.s.Hkv) * a.sH + (size_t)t * a.sT) : -1ll;
+            return wi;
         }
-        const uint8_t* src = (is_v ? a.s.vcodes[li] : a.s.kcodes[li]) + (size_t)tile * (TILE * 16) * width_of(li);
+        return total;
+    };
+    int wi = next_tile(wave * n_wg + (blockIdx.x >> 1));         // (a round of tiles goes over the workgroups first)
+    dq_lay_out_rotation<0>(rotation, reinterpret_cast<uint4*>(smem), tid);
+    if (tid < DQ_CB_WORDS) cb[tid] = dq_centroid<0>(centroid);
+    __syncthreads();
+    while (wi < total) {
+        offs[lane] = off;
+        norms[lane] = norm;
         switch (li) {
-            case 0: dq_unpack<2>(src, is_v, codes, lane); break;
-            case 1: dq_unpack<3>(src, is_v, codes, lane); break;
-            case 2: dq_unpack<4>(src, is_v, codes, lane); break;
-            default: dq_unpack<8>(src, is_v, codes, lane); break;
+            case 0: dq_unpack<2>(raw, is_v, codes, lane); break;
+            case 1: dq_unpack<3>(raw, is_v, codes, lane); break;
+            case 2: dq_unpack<4>(raw, is_v, codes, lane); break;
+            default: dq_unpack<8>(raw, is_v, codes, lane); break;
         }
         wave_lds_fence();
-        dq_tile<DT, 0>(piA, codes, cb + codebook_offset(li), norms, offs, out, lane);
+        const uint32_t* table_of = cb + codebook_offset(li);
+        wi = next_tile(wi + stride);                             // (under way while this one is multiplied)
+        dq_tile<DT, 0>(piA, codes, table_of, norms, offs, out, lane);
         wave_lds_fence();                                        // offs / norms / codes free for the next tile
     }
 }
@@ -2297,7 +2322,7 @@ extern "C" int odmkv_dequant_from(const odmkv_packed_t* store, void* K, void* V,
 // container, and the dequantiser from byte codes.  Workgroups of the even index take job 0, of the odd one job 1 (keys and
 // values of a layer in one launch), a wave a tile of 64 rows.  A row per lane without them took 150 us for 64512 rows (the
 // fused multiply-adds of the rotation on the vector ALU); here keys and values of 64512 rows each are quantised in 29 us and
-// dequantised in 26 us.
+// dequantised in 20 us.
 // ------------------------------------------------------------------------------------------------
 struct RowsArgs { RowsJob job[2]; int n_jobs; };
 
@@ -2462,7 +2487,7 @@ __global__ __launch_bounds__(QF_NW * 64) void quant_rows_f16_kernel(RowsArgs a) 
 // and keep a few bits only.  Times 2^8 both keep all eleven, and the result comes no further from fp64 than with fp32 sums
 // rounded once, which these rows had before the matrix cores did them.  Elements that are not the nearest 16-bit value to
 // the fp64 result, Gaussian rows: fp32 sums 1.05e-3 of all (fp16) and 1.6e-4 (bf16), plain pairs 2.3e-3 and 3.6e-4, these
-// 0.90e-3 and 1.3e-4; 67.5 us for an 8k-token pass with either.
+// 0.90e-3 and 1.3e-4; the time is the same with either.
 #define DQ_UP 8
 template <int DT>
 __global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a) {
@@ -2474,23 +2499,37 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a
     uint32_t* cb = reinterpret_cast<uint32_t*>(smem + QP_PI_BYTES + DQ_NW * QP_STAGE);
     float* norms = reinterpret_cast<float*>(cb + DQ_CB_WORDS) + wave * TILE;
     long long* offs = reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + wave * TILE;
-    dq_load_rotation<DQ_UP>(j.pi, reinterpret_cast<uint16_t*>(smem), tid);
-    for (int i = tid; i < (1 << j.bits); i += DQ_NW * 64) cb[i] = dq_centroid<DQ_UP>(j.cb[i]);
-    __syncthreads();
-    const long long tiles = (j.n + TILE - 1) / TILE, stride = (long long)(gridDim.x / a.n_jobs) * DQ_NW;
-    for (long long tile = (long long)(blockIdx.x / a.n_jobs) * DQ_NW + wave; tile < tiles; tile += stride) {
+    float rotation[8 * DQ_PI_GROUPS];
+    dq_request_rotation(j.pi, rotation, tid);
+    const float centroid = tid < (1 << j.bits) ? j.cb[tid] : 0.0f;                 // (16 at most: the launch takes 2, 3 and 4 bits)
+    const long long tiles = (j.n + TILE - 1) / TILE, n_wg = gridDim.x / a.n_jobs, stride = n_wg * DQ_NW;
+    uint4 raw[8];
+    float norm = 0.0f;
+    long long off = -1ll;
+    const auto request = [&](long long tile) {                   // eight codes' rows a turn, 16 codes a lane
         const long long r = tile * TILE + lane;
-        const bool valid = r < j.n;
-        offs[lane] = valid ? row_offset(j, r) : -1ll;
-        norms[lane] = valid ? j.norms[r] : 0.0f;
         const int rows = (int)min((long long)TILE, j.n - tile * TILE);
+        off = r < j.n ? row_offset(j, r) : -1ll;
+        norm = r < j.n ? j.norms[r] : 0.0f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int token = 8 * i + (lane >> 3), piece = lane & 7;
-            const uint4 v = token < rows ? *reinterpret_cast<const uint4*>(j.codes + (size_t)(tile * TILE + token) * HD + 16 * piece) : make_uint4(0u, 0u, 0u, 0u);
-            *reinterpret_cast<uint4*>(codes + token * CODE_ROW + 16 * piece) = v;
+            raw[i] = token < rows ? *reinterpret_cast<const uint4*>(j.codes + (size_t)(tile * TILE + token) * HD + 16 * piece) : make_uint4(0u, 0u, 0u, 0u);
         }
+    };
+    long long tile = (long long)wave * n_wg + blockIdx.x / a.n_jobs;
+    if (tile < tiles) request(tile);
+    dq_lay_out_rotation<DQ_UP>(rotation, reinterpret_cast<uint4*>(smem), tid);
+    if (tid < (1 << j.bits)) cb[tid] = dq_centroid<DQ_UP>(centroid);
+    __syncthreads();
+    while (tile < tiles) {
+        offs[lane] = off;
+        norms[lane] = norm;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<uint4*>(codes + (8 * i + (lane >> 3)) * CODE_ROW + 16 * (lane & 7)) = raw[i];
         wave_lds_fence();
+        tile += stride;
+        if (tile < tiles) request(tile);                         // (under way while this one is multiplied)
         dq_tile<DT, DQ_UP>(reinterpret_cast<const uint4*>(smem), codes, cb, norms, offs, j.out, lane);
         wave_lds_fence();
     }
