@@ -14,9 +14,14 @@
 // The same two operand fragments serve both passes; only their roles (A or B) swap.  The queries of a
 // kv-head (up to 256 at a time) sit in LDS, a wave holds its 64 tokens in registers (each lane the half row it
 // contracts) and every 16-byte LDS read of a query fragment feeds two matrix instructions.
+// What bounds it: 67 million exponentials a pass at a quarter of the vector rate (8 us), the products (7 us) and the vector work around
+// them (5 us), which only other wavefronts overlap.  The queries' 70 KB leave room for two workgroups a compute unit, so a workgroup has eight
+// wavefronts of at most 128 registers: four a SIMD.  32k tokens of 8 heads, 64 queries, us: four wavefronts a workgroup 43 + 48, eight 38 + 36.
 #include "common.h"
 
-#define WIN_CHUNK 256        // tokens per workgroup (4 waves x 64)
+#define WIN_WAVES 8
+#define WIN_THREADS (WIN_WAVES * 64)
+#define WIN_CHUNK (WIN_WAVES * 64)       // tokens per workgroup
 #define WIN_ROWS 256         // queries staged in LDS at a time
 #define WIN_QROW 136         // 16-bit entries per LDS row: 128 + 8, 16-byte reads of consecutive rows on distinct banks
 
@@ -55,9 +60,9 @@ __device__ static inline void ms2_merge(float& m, float& s, float m2, float s2) 
 __device__ static inline int acc_row(int r, int half) { return 8 * (r >> 2) + 4 * half + (r & 3); }
 
 template <int DT, int PASS>
-__global__ __launch_bounds__(256) void window_kernel(WinArgs a) {
+__global__ __launch_bounds__(WIN_THREADS, 4) void window_kernel(WinArgs a) {
     extern __shared__ __align__(16) uint16_t q_s[];                 // [WIN_ROWS][WIN_QROW]
-    __shared__ float ml_s[WIN_ROWS];
+    __shared__ __align__(16) float ml_s[WIN_ROWS];
     const int chunk = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int t0 = chunk * WIN_CHUNK + wave * 64;                    // first of this wave's 64 core tokens
@@ -83,30 +88,30 @@ __global__ __launch_bounds__(256) void window_kernel(WinArgs a) {
     for (int rg = 0; rg < a.R; rg += WIN_ROWS) {
         const int nr = min(WIN_ROWS, a.R - rg), nrb = (nr + 31) >> 5;
         __syncthreads();                                            // the previous group's reads are done
-        {
-            // all of a thread's 16-byte pieces are requested before the first is stored (one round trip to
-            // the caches instead of sixteen)
-            uint4 stage[WIN_ROWS * 16 / 256];
+        // a thread's 16-byte pieces are requested four at a time before the first is stored (a round trip each would be eight)
+#pragma unroll 1
+        for (int i0 = 0; i0 < WIN_ROWS * 16; i0 += 4 * WIN_THREADS) {
+            uint4 stage[4];
 #pragma unroll
-            for (int i = 0; i < WIN_ROWS * 16 / 256; ++i) {
-                const int e = tid + 256 * i, row = e >> 4, pc = e & 15;
+            for (int i = 0; i < 4; ++i) {
+                const int e = i0 + tid + WIN_THREADS * i, row = e >> 4, pc = e & 15;
                 stage[i] = row < nr ? qsrc[(size_t)(rg + row) * 16 + pc] : make_uint4(0u, 0u, 0u, 0u);
             }
 #pragma unroll
-            for (int i = 0; i < WIN_ROWS * 16 / 256; ++i) {
-                const int e = tid + 256 * i, row = e >> 4, pc = e & 15;
+            for (int i = 0; i < 4; ++i) {
+                const int e = i0 + tid + WIN_THREADS * i, row = e >> 4, pc = e & 15;
                 if (row < nrb * 32) *reinterpret_cast<uint4*>(q_s + (size_t)row * WIN_QROW + pc * 8) = stage[i];
             }
         }
         if (PASS == 2) {
             // queries beyond the last take weight 0: exp2(0 - inf)
-            for (int e = tid; e < nrb * 32; e += 256) ml_s[e] = e < nr ? a.mz[(size_t)h * a.R + rg + e] : INFINITY;
+            for (int e = tid; e < nrb * 32; e += WIN_THREADS) ml_s[e] = e < nr ? a.mz[(size_t)h * a.R + rg + e] : INFINITY;
         }
         __syncthreads();
         if (!active) {
             if (PASS == 1) {                                        // neutral entries for the merge
                 for (int e = lane; e < nr; e += 64) {
-                    float* st = a.stats + (((size_t)h * a.R + rg + e) * a.nstat + chunk * 4 + wave) * 2;
+                    float* st = a.stats + (((size_t)h * a.R + rg + e) * a.nstat + chunk * WIN_WAVES + wave) * 2;
                     st[0] = -INFINITY; st[1] = 0.0f;
                 }
             }
@@ -120,6 +125,7 @@ __global__ __launch_bounds__(256) void window_kernel(WinArgs a) {
             const uint16_t* qrow = q_s + (size_t)(rb * 32 + col) * WIN_QROW + 64 * half;
 #pragma unroll
             for (int st = 0; st < 8; ++st) {
+                if (st % 4 == 0) __builtin_amdgcn_sched_barrier(0);     // (four fragments under way: all eight leave the accumulators no room)
                 const uint4 qv = *reinterpret_cast<const uint4*>(qrow + 8 * st);
                 const uint4 ka = k0[st], kb = k1[st];
                 if (PASS == 1) { acc0 = win_mfma<DT>(ka, qv, acc0); acc1 = win_mfma<DT>(kb, qv, acc1); }
@@ -128,7 +134,6 @@ __global__ __launch_bounds__(256) void window_kernel(WinArgs a) {
             if (PASS == 1) {
                 // this lane's query: row rho of the kv-head; its position decides which of the last keys it sees
                 const int rho = rg + rb * 32 + col;
-                const int qpos = a.qpos0 + rho % a.W;
                 float mx = -INFINITY, z = 0.0f;
                 if (!need_mask && !tail) {
                     // every token of the wave is a key every query sees: the maximum is taken on the raw
@@ -141,34 +146,40 @@ __global__ __launch_bounds__(256) void window_kernel(WinArgs a) {
                     for (int r = 0; r < 16; ++r)
                         z += __builtin_amdgcn_exp2f(__fmaf_rn(acc0[r], a.c, -mx)) + __builtin_amdgcn_exp2f(__fmaf_rn(acc1[r], a.c, -mx));
                 } else {
-                    float s0[16], s1[16];
+                    const int qpos = a.qpos0 + rho % a.W;
+                    int first = t0 + 4 * half;                      // opaque: 32 positions worked out ahead of the loop take 32 registers
+                    asm volatile("" : "+v"(first));
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        const int ta = t0 + acc_row(r, half), tb = ta + 32;
+                        const int ta = first + acc_row(r, 0), tb = ta + 32;
                         const bool va = ta < a.Tc && a.n_sink + ta <= qpos;
                         const bool vb = tb < a.Tc && a.n_sink + tb <= qpos;
-                        s0[r] = va ? acc0[r] * a.c : -INFINITY;
-                        s1[r] = vb ? acc1[r] * a.c : -INFINITY;
-                        mx = fmaxf(mx, fmaxf(s0[r], s1[r]));
+                        acc0[r] = va ? acc0[r] * a.c : -INFINITY;
+                        acc1[r] = vb ? acc1[r] * a.c : -INFINITY;
+                        mx = fmaxf(mx, fmaxf(acc0[r], acc1[r]));
                     }
                     if (mx > -INFINITY) {
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(s0[r] - mx) + __builtin_amdgcn_exp2f(s1[r] - mx);
+                        for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(acc0[r] - mx) + __builtin_amdgcn_exp2f(acc1[r] - mx);
                     }
                 }
                 // the other half of the wave holds the same query's other tokens
                 const float m2 = __shfl_xor(mx, 32, WAVE), z2 = __shfl_xor(z, 32, WAVE);
                 ms2_merge(mx, z, m2, z2);
                 if (half == 0 && rho < a.R) {
-                    float* st = a.stats + (((size_t)h * a.R + rho) * a.nstat + chunk * 4 + wave) * 2;
+                    float* st = a.stats + (((size_t)h * a.R + rho) * a.nstat + chunk * WIN_WAVES + wave) * 2;
                     st[0] = mx; st[1] = z;
                 }
             } else {
                 const int ta = t0 + col, tb = ta + 32;               // this lane's tokens
+                const int row0 = rb * 32 + 4 * half;
+                float4 ml4;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int row = rb * 32 + acc_row(r, half);
-                    const float ml = ml_s[row];                     // M + log2 Z: exp2(s - ml) = exp2(s - M) / Z
+                    const int row = row0 + acc_row(r, 0);
+                    if (r % 4 == 0) ml4 = *reinterpret_cast<const float4*>(&ml_s[row]);
+                    // M + log2 Z: exp2(s - ml) = exp2(s - M) / Z
+                    const float ml = r % 4 == 0 ? ml4.x : r % 4 == 1 ? ml4.y : r % 4 == 2 ? ml4.z : ml4.w;
                     float ea = __builtin_amdgcn_exp2f(__fmaf_rn(acc0[r], a.c, -ml));
                     float eb = __builtin_amdgcn_exp2f(__fmaf_rn(acc1[r], a.c, -ml));
                     if (need_mask) {
@@ -211,7 +222,7 @@ static inline int win_chunks(int Tc) { return (Tc + WIN_CHUNK - 1) / WIN_CHUNK; 
 
 extern "C" size_t odmkv_window_attention_workspace_bytes(int Hkv, int Hq, int W, int T) {
     if (Hkv <= 0 || Hq <= 0 || W <= 0 || T <= 0) return 0;
-    const size_t rows = (size_t)Hq * W, nstat = (size_t)win_chunks(T) * 4;
+    const size_t rows = (size_t)Hq * W, nstat = (size_t)win_chunks(T) * WIN_WAVES;
     return align_up(rows * nstat * 8, 256) + align_up(rows * 8, 256);
 }
 
@@ -222,7 +233,7 @@ static int run_window(WinArgs& a, hipStream_t st) {
                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&window_kernel<DT, 2>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    dim3 grid(a.nchunks, a.Hkv), block(256);
+    dim3 grid(a.nchunks, a.Hkv), block(WIN_THREADS);
     hipLaunchKernelGGL((window_kernel<DT, 1>), grid, block, lds, st, a);
     ODMKV_CHECK_LAUNCH("window_kernel<1>");
     hipLaunchKernelGGL(window_stats_kernel, dim3(a.Hkv * a.R), dim3(64), 0, st, a);
@@ -248,11 +259,11 @@ extern "C" int odmkv_window_attention(const void* K, int dtype, int Hkv, int T, 
     WinArgs a;
     a.K = K; a.Q = Q; a.sH = stride_h; a.sT = stride_t;
     a.Hkv = Hkv; a.G = Hq / Hkv; a.W = W; a.R = a.G * W; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
-    a.nchunks = win_chunks(a.Tc); a.nstat = a.nchunks * 4; a.qpos0 = q_pos0;
+    a.nchunks = win_chunks(a.Tc); a.nstat = a.nchunks * WIN_WAVES; a.qpos0 = q_pos0;
     a.c = scaling * 1.4426950408889634f;
     const size_t rows = (size_t)Hq * W;
     a.stats = (float*)workspace;                          // the workspace is sized for the chunks of all T tokens
-    a.mz = (float*)((char*)workspace + align_up(rows * (size_t)win_chunks(T) * 4 * 8, 256));
+    a.mz = (float*)((char*)workspace + align_up(rows * (size_t)win_chunks(T) * WIN_WAVES * 8, 256));
     a.p = p;
     hipStream_t st = (hipStream_t)stream;
     if (dtype == ODMKV_F16) return run_window<ODMKV_F16>(a, st);

@@ -421,6 +421,19 @@ def test_window_attention_kernel_matches_oracle(hkv, hq, T, W, dtype):
     np.testing.assert_allclose(got.sum(-1).cpu().numpy(), 1.0, rtol=1e-4)
 
 
+@pytest.mark.parametrize("T,W,n_sink", [(512, 8, 0), (515, 64, 4), (516, 64, 4), (517, 1, 4), (1024 + 64, 64, 0), (1025, 65, 1)])
+def test_window_attention_at_the_edges_of_its_workgroups(T, W, n_sink):
+    """512 tokens behind the sinks a workgroup, 64 a wavefront: whole ones, one token more and less, wavefronts without any; 260 queries
+    a kv-head (W = 65) do not fit one group of 256."""
+    from kvquant.scorer import _launch_window_attention
+    g = torch.Generator().manual_seed(T + W)
+    k = torch.randn(2, T, 128, generator=g).half()
+    q = (torch.randn(8, W, 128, generator=g) * 1.5).half()
+    want = osc.window_attention(k.double(), q.double(), n_sink, T - W)[0]
+    got = _launch_window_attention(k.to(DEV), q.to(DEV), n_sink, T - W, 128 ** -0.5)
+    np.testing.assert_allclose(got.cpu().numpy(), want.numpy(), rtol=SCORE_RTOL, atol=1e-12)
+
+
 def test_window_attention_rejects_fp32_keys():
     from kvquant.scorer import _launch_window_attention
     k = torch.randn(1, 64, 128, device=DEV)
