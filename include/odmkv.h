@@ -472,10 +472,8 @@ int odmkv_flush_rank(const float* scores, const float* minmax, int B, int H, int
  * dispatch_order: NULL (workgroup k takes item k), or device int32 [n_items], a permutation of the
  * items in the order the workgroups should take them (longest first, when there are more items than
  * compute units).
- * wavefronts: wavefronts of the workgroup that runs an item: 8 (0 means 8), 12 or 16.  Eight start and finish
- * faster and suit items of fewer than sixteen tiles; sixteen stream long 2- and 3-bit items about 1.1 times
- * faster; twelve (three units in flight per wavefront) are 5 % ahead where 4- and 8-bit tokens carry the bytes, and
- * 2 % ahead of eight on items of 6 to 15 tiles of 3 bits and wider.
+ * wavefronts: wavefronts of the workgroup that runs an item: 8 (0 means 8), 12, or 16 (runs as 12).  Eight start and finish
+ * faster and suit short items of 3 bits and wider; twelve stream long items, and short ones of 2 bits, 2 to 12 % faster.
  * Two launches per call (main kernel, merge); the workspace holds the per-item partial results.
  */
 typedef struct odmkv_worklist {

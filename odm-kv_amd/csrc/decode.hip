@@ -19,7 +19,7 @@
 // A separate query-preparation launch was measured too: the same time per call, one launch more.)
 //
 // Two forms of the quantised levels: the general one (compute_unit: up to 8 heads of a group in one pass), and one for
-// groups of up to four heads at four wavefronts per SIMD (sixteen wavefronts, or two workgroups of eight;
+// groups of up to four heads in the shared-lane form (twelve wavefronts, or two workgroups of eight;
 // compute_unit_g4: the lanes are shared out between a unit's two token blocks, the softmax step runs once per unit).
 //
 // Main kernel, per wavefront and unit of 32 tokens (half a tile), on v_mfma_f32_16x16x32_f16 (D[16x16] += A[16x32]
@@ -478,7 +478,7 @@ __device__ static inline void compute_unit(const Unit<W>& t, int nvalid, int lan
     wave_lds_fence();                                      // the p buffer is free for the next unit
 }
 
-// ---- groups of up to four query heads on sixteen wavefronts (decode_main_kernel<4, ., 16, true>) ------------------
+// ---- groups of up to four query heads on twelve wavefronts, or in pairs of workgroups (decode_main_kernel<4, ., ., true>) ----
 // Four heads need 8 of the 16 matrix rows.  The general form leaves rows 8..15 empty and every lane of wave rows 2, 3
 // (lanes 32..63) then runs the softmax step on heads that do not exist.  Here rows 8..15 repeat rows 0..7
 // (load_queries_g4) and the two token blocks of a unit share the lanes out between them: after the key products lane
@@ -781,7 +781,7 @@ __device__ static inline void run_quant_level(const DecodeArgs& a, int li, int b
     }
 }
 
-// The same walk for groups of up to four heads with compute_unit_g4 (sixteen wavefronts, two unit buffers; an
+// The same walk for groups of up to four heads with compute_unit_g4 (two unit buffers; an
 // eight-wavefront ring of five buffers, every unit of a short item requested at once, measured no faster).
 template <int W, int NW>
 __device__ static inline void run_quant_level_g4(const DecodeArgs& a, int li, int bq_first, int tile0, int ntiles, int ntok,
@@ -982,7 +982,7 @@ __device__ static inline void run_exact_level(const DecodeArgs& a, int bh, int b
 // ------------------------------------------------------------------------------------------------
 // main kernel
 // ------------------------------------------------------------------------------------------------
-// G4: the quantised levels run compute_unit_g4 (GP = 4 and sixteen wavefronts only)
+// G4: the quantised levels run compute_unit_g4 (GP = 4; twelve wavefronts, or PAIR: eight alone lose 2 % by it)
 // CHAIN: a workgroup may take several consecutive items, the quantised levels of one (sequence, kv-head) one after the
 // other (item word 6 = how many follow): the queries are rotated once, the accumulators run through, the table is rebuilt
 // between the levels, one result is written at the first item's place and empty results at the others'.
@@ -991,7 +991,7 @@ __device__ static inline void run_exact_level(const DecodeArgs& a, int bh, int b
 // compute units, whose workgroups would otherwise run one after the other, each paying its start and its end alone.
 template <int GP, bool ORDERED, int NW, bool G4 = false, bool CHAIN = false, bool PAIR = false>
 __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(DecodeArgs a) {
-    static_assert(!G4 || (GP == 4 && (NW == 16 || PAIR)), "the shared-lane form is built for four heads and four wavefronts per SIMD");
+    static_assert(!G4 || (GP == 4 && (NW == 12 || PAIR)), "the shared-lane form is built for four heads");
     static_assert(!PAIR || (NW == 8 && 2 * Lds<NW>::TOTAL <= 160 * 1024), "two workgroups of eight wavefronts share a compute unit");
     static_assert(!CHAIN || ORDERED, "chains come with a dispatch order (fewer workgroups than items)");
     // one static LDS block: the table sits at LDS address 0 and that is known when the kernel is compiled, so a
@@ -1445,15 +1445,17 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
         // when measuring, the events are attached to the dispatch itself: they carry the kernel's own
         // start and end timestamps, not those of separate marker packets
         hipEvent_t e0 = (hipEvent_t)ev_start, e1 = (hipEvent_t)ev_stop;
-        const int nw = work->wavefronts == 0 ? 8 : work->wavefronts;
+        const int nw = work->wavefronts >= 12 ? 12 : 8;
         int rc;
 #define ODMKV_LAUNCH_MAIN(GPV, ORD, CH) \
-        (nw == 16 ? launch_main<GPV, ORD, 16, false, CH>(a, grid, e0, e1, st) : nw == 12 ? launch_main<GPV, ORD, 12, false, CH>(a, grid, e0, e1, st) \
-                                                                               : launch_main<GPV, ORD, 8, false, CH>(a, grid, e0, e1, st))
-        // groups of up to four heads on sixteen wavefronts: the form that shares the lanes out between a unit's two token
+        (nw == 12 ? launch_main<GPV, ORD, 12, false, CH>(a, grid, e0, e1, st) : launch_main<GPV, ORD, 8, false, CH>(a, grid, e0, e1, st))
+        // Twelve wavefronts run what used to take sixteen: with 170 registers instead of 128 and the shared-lane form they are as fast
+        // or faster on every shape (us a layer, 16 / 12: 32k tokens 32 heads over 8 14.50 / 14.20, 3 bits 16.70 / 16.25; 131k tokens
+        // 23.6 / 23.6; 28 over 4 20.4 / 19.4; 4- and 8-bit levels at 131k in the general form of 12 24.6, in this one 24.4).
+        // groups of up to four heads on twelve wavefronts: the form that shares the lanes out between a unit's two token
         // blocks (its softmax step costs half the instructions); ODMKV_DECODE_G4=0 selects the general form, for measurements
         static const int g4_forced = [] { const char* e = getenv("ODMKV_DECODE_G4"); return e ? atoi(e) : -1; }();
-        const bool g4 = GP == 4 && nw == 16 && g4_forced != 0;
+        const bool g4 = GP == 4 && nw == 12 && g4_forced != 0;
         const bool chain = work->n_workgroups > 0 && work->n_workgroups != n_items;      // workgroups that take several items
         const dim3 grid(chain ? work->n_workgroups : n_items, passes);
         // two eight-wavefront workgroups per compute unit (always with a dispatch order: the list has more items than
@@ -1469,11 +1471,11 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
                                                           : launch_main<4, true, 8, true, false, true>(a, grid, e0, e1, st);
         else if (pair) rc = chain ? launch_main<8, true, 8, false, true, true>(a, grid, e0, e1, st)
                                   : launch_main<8, true, 8, false, false, true>(a, grid, e0, e1, st);
-        else if (chain && g4) rc = launch_main<4, true, 16, true, true>(a, grid, e0, e1, st);
+        else if (chain && g4) rc = launch_main<4, true, 12, true, true>(a, grid, e0, e1, st);
         else if (chain && GP == 4) rc = ODMKV_LAUNCH_MAIN(4, true, true);
         else if (chain) rc = ODMKV_LAUNCH_MAIN(8, true, true);
-        else if (g4 && !a.order) rc = launch_main<4, false, 16, true>(a, grid, e0, e1, st);
-        else if (g4) rc = launch_main<4, true, 16, true>(a, grid, e0, e1, st);
+        else if (g4 && !a.order) rc = launch_main<4, false, 12, true>(a, grid, e0, e1, st);
+        else if (g4) rc = launch_main<4, true, 12, true>(a, grid, e0, e1, st);
         else if (GP == 4 && !a.order) rc = ODMKV_LAUNCH_MAIN(4, false, false);
         else if (GP == 4) rc = ODMKV_LAUNCH_MAIN(4, true, false);
         else if (!a.order) rc = ODMKV_LAUNCH_MAIN(8, false, false);
