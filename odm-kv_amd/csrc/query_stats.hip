@@ -313,7 +313,7 @@ extern "C" int odmkv_average_rope(const void* mu, const void* cosine, const void
 // (4 p .. 4 p + 3, p = l % 32) of eight tokens and pairs the tokens up by byte permutes: block b = the dims 4 p + b.  Ten of the
 // sixteen 32x32 blocks (the others mirror them).
 // Floors for 32 heads of 32k tokens: 268 MB once, 129 GFLOP of bf16 products.  As tensor operations (conversion, mean,
-// subtraction, fp32 product) 1050 us, here 139 + 25 (bound by the matrix cores: 0.93 PFLOP/s).
+// subtraction, fp32 product) 1050 us, here 139 + 15 (bound by the matrix cores: 0.93 PFLOP/s).
 // ------------------------------------------------------------------------------------------------
 #define CV_WAVES 8
 #define CV_BLOCKS 10                 // (0,0) (0,1) (0,2) (0,3) (1,1) (1,2) (1,3) (2,2) (2,3) (3,3)
@@ -482,19 +482,42 @@ __global__ __launch_bounds__(256) void cov_final_kernel(CovArgs a) {
     __shared__ float cs[2][HD];
     const int h = blockIdx.y, tid = threadIdx.x;
     const float* part = a.part + (size_t)h * a.slices * CV_PART;
+    // A thread's four entries and its share of the means, eight slices of each asked for at once (one after the other they were a chain
+    // of forty round trips: 26 us a call of 32 heads of 32k tokens, 15 now); added up in the slices' order
+    double s[4] = {0.0, 0.0, 0.0, 0.0}, sm = 0.0;
+    int at[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int e = tid + 256 * u, r = e >> 7;
+        at[u] = cov_at(blockIdx.x * 4 + (r & 3) + 64 * (r >> 2), e & 127);
+    }
+    for (int k0 = 0; k0 < a.slices; k0 += 8) {
+        float v[4][8], vm[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float* slice = part + (size_t)min(k0 + k, a.slices - 1) * CV_PART;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u][k] = slice[at[u]];
+            vm[k] = slice[CV_BLOCKS * 1024 + (tid & (HD - 1))];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (k0 + k >= a.slices) break;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s[u] += (double)v[u][k];
+            sm += (double)vm[k];
+        }
+    }
     if (tid < HD) {
-        double s = 0.0;
-        for (int k = 0; k < a.slices; ++k) s += (double)part[(size_t)k * CV_PART + CV_BLOCKS * 1024 + tid];
-        mean[tid] = s / a.tokens;                            // relative to the pivot
+        mean[tid] = sm / a.tokens;                           // relative to the pivot
         cs[0][tid] = a.cosine ? a.rope[tid] : 1.0f;
         cs[1][tid] = a.cosine ? a.rope[HD + tid] : 0.0f;
     }
     __syncthreads();
-    for (int e = tid; e < 8 * HD; e += 256) {
-        const int r = e >> 7, i = blockIdx.x * 4 + (r & 3) + 64 * (r >> 2), j = e & 127, at = cov_at(i, j);
-        double s = 0.0;
-        for (int k = 0; k < a.slices; ++k) s += (double)part[(size_t)k * CV_PART + at];
-        c[r][j] = (float)(s / a.tokens - mean[i] * mean[j]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int e = tid + 256 * u, r = e >> 7, i = blockIdx.x * 4 + (r & 3) + 64 * (r >> 2), j = e & 127;
+        c[r][j] = (float)(s[u] / a.tokens - mean[i] * mean[j]);
     }
     __syncthreads();
     for (int e = tid; e < 8 * HD; e += 256) {
