@@ -25,6 +25,7 @@ struct ScoreArgs {
     int round_dt;         // -1, or ODMKV_F16 / ODMKV_BF16: round logits, softmax and group mean like a model of that dtype
     int use_vnorm;        // expected-attention score: multiply (p + eps) by |v|
     int ea_cpw;           // expected-attention score: 256-token chunks a workgroup walks
+    int kn2_given;        // kn2 is filled in already (attention weights given: nothing is left for the logits pass)
     int nstat;            // softmax statistics entries per query head (one per chunk, or one per wave and chunk)
     float* scores;        // [Hkv, T]
     float* logits;        // [Hq, Tc]
@@ -978,7 +979,8 @@ extern "C" size_t odmkv_score_workspace_bytes(int Hkv, int Hq, int T) {
 template <int DT>
 static int run_score(ScoreArgs& a, hipStream_t st) {
     dim3 grid(a.nchunks, a.Hkv), block(256);
-    if constexpr (DT != ODMKV_F32) {
+    if (a.kn2_given) {
+    } else if constexpr (DT != ODMKV_F32) {
         // 16-bit keys feed the matrix cores as they lie in memory; the mode that rounds like a 16-bit model and
         // the call that brings its own attention weights keep the kernel that forms every product in fp32
         if (a.round_dt < 0 && a.Gl > 0) {
@@ -1014,7 +1016,7 @@ extern "C" int odmkv_score(const void* K, const void* V, int dtype, int Hkv, int
 // Hkv kv-heads (of Hkv / Hlayer sequences that lie one behind the other), scored together
 static int score_heads(const void* K, const void* V, int dtype, int Hkv, int Hlayer, int T, int64_t stride_h, int64_t stride_t,
                        const float* mu, int Hq, const float* attn, int n_sink, float eps, int round_dtype, float* scores,
-                       void* workspace, size_t workspace_bytes, void* stream) {
+                       void* workspace, size_t workspace_bytes, void* stream, bool kn2_given = false) {
     ODMKV_CHECK_ARG(K && V && scores && workspace, "score: null pointer");
     ODMKV_CHECK_ARG(round_dtype == -1 || round_dtype == ODMKV_F16 || round_dtype == ODMKV_BF16,
                     "score: rounding dtype %d (-1, fp16 or bf16)", round_dtype);
@@ -1036,7 +1038,7 @@ static int score_heads(const void* K, const void* V, int dtype, int Hkv, int Hla
     a.K = K; a.V = V; a.sH = stride_h; a.sT = stride_t;
     a.Hlayer = Hlayer; a.Hkv = Hkv; a.Hq = Hq; a.G = Hq / Hkv; a.Gl = attn ? 0 : Hq / Hkv; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
     a.nchunks = n_chunks(a.Tc); a.eps = eps; a.mu = mu; a.attn = attn; a.scores = scores;
-    a.cov = nullptr; a.use_vnorm = 0; a.ea_cpw = 1; a.nstat = a.nchunks; a.round_dt = round_dtype;
+    a.cov = nullptr; a.use_vnorm = 0; a.ea_cpw = 1; a.nstat = a.nchunks; a.round_dt = round_dtype; a.kn2_given = kn2_given;
     a.logits = (float*)(ws + L.logits); a.kn2 = (float*)(ws + L.kn2); a.p = (float*)(ws + L.p);
     a.stats = (float*)(ws + L.stats); a.mz = (float*)(ws + L.mz); a.opart = (float*)(ws + L.opart);
     a.psum = (float*)(ws + L.psum); a.obar = (float*)(ws + L.obar);
@@ -1044,6 +1046,14 @@ static int score_heads(const void* K, const void* V, int dtype, int Hkv, int Hla
     if (dtype == ODMKV_F16) return run_score<ODMKV_F16>(a, st);
     if (dtype == ODMKV_BF16) return run_score<ODMKV_BF16>(a, st);
     return run_score<ODMKV_F32>(a, st);
+}
+
+// The scores given attention weights and |k|^2 (window.hip): where a call of that workspace keeps |k|^2 [Hkv, T], and the rest of it
+float* score_kn2(void* workspace, int Hkv, int Hq, int T) { return (float*)((char*)workspace + score_layout(Hkv, Hq, T).kn2); }
+int score_given_kn2(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t, const float* attn,
+                    float eps, float* scores, void* workspace, size_t workspace_bytes, void* stream) {
+    return score_heads(K, V, dtype, Hkv, Hkv, T, stride_h, stride_t, nullptr, Hkv, attn, 0, eps, -1, scores, workspace, workspace_bytes,
+                       stream, true);
 }
 
 extern "C" int odmkv_score_model_dtype(const void* K, const void* V, int dtype, int Hkv, int T,
@@ -1197,7 +1207,7 @@ extern "C" int odmkv_score_expected(const void* K, const void* V, int dtype, int
     ScoreArgs a;
     a.K = K; a.V = V; a.sH = stride_h; a.sT = stride_t;
     a.Hlayer = Hkv; a.Hkv = Hkv; a.Hq = Hq; a.G = Hq / Hkv; a.Gl = a.G; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
-    a.nchunks = n_chunks(a.Tc); a.eps = eps; a.mu = mu; a.attn = nullptr; a.scores = scores;
+    a.nchunks = n_chunks(a.Tc); a.eps = eps; a.mu = mu; a.attn = nullptr; a.scores = scores; a.kn2_given = 0;
     a.cov = cov; a.use_vnorm = use_vnorm ? 1 : 0; a.ea_cpw = 1; a.nstat = a.nchunks; a.round_dt = -1;
     a.logits = (float*)(ws + L.logits); a.kn2 = (float*)(ws + L.kn2); a.p = (float*)(ws + L.p);
     a.stats = (float*)(ws + L.stats); a.mz = (float*)(ws + L.mz); a.opart = (float*)(ws + L.opart);

@@ -38,7 +38,25 @@ struct WinArgs {
     float* stats;         // [Hkv R][nstat][2]
     float* mz;            // [Hkv R]: maximum + log2(sum), both in base-2 units
     float* p;             // [Hkv][Tc]
+    float* kn2;           // [Hkv][Tc]: |k|^2, or null (pass 1 holds every key anyway)
 };
+
+// sum of squares of 64 elements: eight running sums, then a tree
+template <int DT>
+__device__ static inline float half_row_squares(const uint4 (&k)[8]) {
+    float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const uint32_t w[4] = {k[i].x, k[i].y, k[i].z, k[i].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x0 = Elem<DT>::to_f32((uint16_t)(w[e] & 0xffffu)), x1 = Elem<DT>::to_f32((uint16_t)(w[e] >> 16));
+            s[2 * e] = __fmaf_rn(x0, x0, s[2 * e]);
+            s[2 * e + 1] = __fmaf_rn(x1, x1, s[2 * e + 1]);
+        }
+    }
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
 
 template <int DT>
 __device__ static inline f32x16 win_mfma(uint4 a, uint4 b, f32x16 c) {
@@ -82,6 +100,13 @@ __global__ __launch_bounds__(WIN_THREADS, 4) void window_kernel(WinArgs a) {
                                                           (size_t)(a.n_sink + min(t0 + 32 + col, a.Tc - 1)) * a.sT + 64 * half);
 #pragma unroll
         for (int i = 0; i < 8; ++i) { k0[i] = p0[i]; k1[i] = p1[i]; }
+    }
+    if (PASS == 1 && a.kn2 != nullptr && active) {
+        float s0 = half_row_squares<DT>(k0), s1 = half_row_squares<DT>(k1);
+        s0 += __shfl_xor(s0, 32, WAVE);
+        s1 += __shfl_xor(s1, 32, WAVE);
+        const int t = t0 + 32 * half + col;                         // the upper half stores the second block
+        if (t < a.Tc) a.kn2[(size_t)h * a.Tc + t] = half ? s1 : s0;
     }
     float pacc0 = 0.0f, pacc1 = 0.0f;
     const uint4* qsrc = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(a.Q) + (size_t)h * a.R * HD);
@@ -243,9 +268,9 @@ static int run_window(WinArgs& a, hipStream_t st) {
     return 0;
 }
 
-extern "C" int odmkv_window_attention(const void* K, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
-                                      const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling,
-                                      float* p, void* workspace, size_t workspace_bytes, void* stream) {
+static int window_attention(const void* K, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
+                            const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling,
+                            float* p, float* kn2, void* workspace, size_t workspace_bytes, void* stream) {
     ODMKV_CHECK_ARG(K && Q && p && workspace, "window_attention: null pointer");
     ODMKV_CHECK_ARG(dtype == ODMKV_F16 || dtype == ODMKV_BF16,
                     "window_attention: keys and queries must be float16 or bfloat16 (dtype %d)", dtype);
@@ -264,8 +289,41 @@ extern "C" int odmkv_window_attention(const void* K, int dtype, int Hkv, int T, 
     const size_t rows = (size_t)Hq * W;
     a.stats = (float*)workspace;                          // the workspace is sized for the chunks of all T tokens
     a.mz = (float*)((char*)workspace + align_up(rows * (size_t)win_chunks(T) * WIN_WAVES * 8, 256));
-    a.p = p;
+    a.p = p; a.kn2 = kn2;
     hipStream_t st = (hipStream_t)stream;
     if (dtype == ODMKV_F16) return run_window<ODMKV_F16>(a, st);
     return run_window<ODMKV_BF16>(a, st);
+}
+
+extern "C" int odmkv_window_attention(const void* K, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
+                                      const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling,
+                                      float* p, void* workspace, size_t workspace_bytes, void* stream) {
+    return window_attention(K, dtype, Hkv, T, stride_h, stride_t, Q, Hq, W, q_pos0, n_sink, scaling, p, nullptr, workspace, workspace_bytes, stream);
+}
+
+// attention mass | its workspace | the score's
+extern "C" size_t odmkv_window_score_workspace_bytes(int Hkv, int Hq, int W, int T) {
+    if (Hkv <= 0 || Hq <= 0 || W <= 0 || T <= 0) return 0;
+    return align_up((size_t)Hkv * T * 4, 256) + odmkv_window_attention_workspace_bytes(Hkv, Hq, W, T) + odmkv_score_workspace_bytes(Hkv, Hkv, T);
+}
+
+// The window's attention mass and the risk scores with it: the first pass over the keys leaves |k|^2 too, and the score is spared a pass
+// of its own over them for that (12 us of 165 for 32k tokens of 8 heads).
+extern "C" int odmkv_window_score(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
+                                  const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling, float eps,
+                                  float* scores, void* workspace, size_t workspace_bytes, void* stream) {
+    ODMKV_CHECK_ARG(K && V && scores && workspace, "window_score: null pointer");
+    ODMKV_CHECK_ARG(Hkv > 0 && Hq > 0 && W >= 1 && n_sink >= 0 && T > n_sink, "window_score: bad shape Hkv=%d Hq=%d W=%d T=%d n_sink=%d", Hkv, Hq, W, T, n_sink);
+    ODMKV_CHECK_ARG(workspace_bytes >= odmkv_window_score_workspace_bytes(Hkv, Hq, W, T), "window_score: workspace too small");
+    const int Tc = T - n_sink;
+    char* ws = (char*)workspace;
+    float* p = (float*)ws;
+    ws += align_up((size_t)Hkv * T * 4, 256);
+    const size_t attn_bytes = odmkv_window_attention_workspace_bytes(Hkv, Hq, W, T), score_bytes = odmkv_score_workspace_bytes(Hkv, Hkv, T);
+    char* score_ws = ws + attn_bytes;
+    if (int rc = window_attention(K, dtype, Hkv, T, stride_h, stride_t, Q, Hq, W, q_pos0, n_sink, scaling, p,
+                                  score_kn2(score_ws, Hkv, Hkv, Tc), ws, attn_bytes, stream)) return rc;
+    const size_t behind = (size_t)n_sink * stride_t * 2;                             // (16-bit rows)
+    return score_given_kn2((const char*)K + behind, (const char*)V + behind, dtype, Hkv, Tc, stride_h, stride_t, p, eps, scores, score_ws,
+                           score_bytes, stream);
 }

@@ -340,15 +340,37 @@ class RiskScorer(ExpectedAttentionScorer):
         return _launch_score(keys, values, None, attn_weights, H, 0, self.epsilon)
 
 
-def _launch_window_attention(keys: torch.Tensor, queries: torch.Tensor, n_sink: int, q_pos0: int,
-                             scaling: float) -> torch.Tensor:
-    """p fp32 [Hkv, T - n_sink]: attention mass of the window queries [Hq, W, d] (rotated to positions
-    q_pos0 .. q_pos0 + W - 1) over the core keys, per-query causal softmax, mean over queries and group."""
+def _check_window_keys(keys: torch.Tensor) -> None:
     _lib.require_gpu(keys, "keys")
     if keys.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError(f"window attention runs on the 16-bit matrix cores: keys must be float16 or bfloat16, got {keys.dtype}")
     if keys.shape[-1] != _lib.HEAD_DIM:
         raise ValueError(f"the HIP kernels are written for head_dim {_lib.HEAD_DIM}, got {keys.shape[-1]}")
+
+
+def _launch_window_score(keys: torch.Tensor, values: torch.Tensor, queries: torch.Tensor, n_sink: int, q_pos0: int,
+                         scaling: float, eps: float) -> torch.Tensor:
+    """Risk scores fp32 [Hkv, T - n_sink] of the core tokens with the window's attention mass (below), in one call."""
+    _check_window_keys(keys)
+    keys, values = _kv_operands(keys, values)
+    H, T, D = keys.shape
+    Hq, W, _ = queries.shape
+    q = queries.to(keys.dtype).contiguous()
+    dev = keys.device
+    scores = torch.empty(H, T - n_sink, dtype=torch.float32, device=dev)
+    ws_bytes = lib.odmkv_window_score_workspace_bytes(H, Hq, W, T)
+    ws = _lib.workspace(dev, ws_bytes, "window")
+    _lib.check(lib.odmkv_window_score(
+        keys.data_ptr(), values.data_ptr(), _lib.dtype_code(keys), H, T, keys.stride(0), keys.stride(1), q.data_ptr(), Hq, W,
+        int(q_pos0), int(n_sink), float(scaling), float(eps), scores.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev)))
+    return scores
+
+
+def _launch_window_attention(keys: torch.Tensor, queries: torch.Tensor, n_sink: int, q_pos0: int,
+                             scaling: float) -> torch.Tensor:
+    """p fp32 [Hkv, T - n_sink]: attention mass of the window queries [Hq, W, d] (rotated to positions
+    q_pos0 .. q_pos0 + W - 1) over the core keys, per-query causal softmax, mean over queries and group."""
+    _check_window_keys(keys)
     if keys.stride(-1) != 1 or keys.stride(0) % 8 or keys.stride(1) % 8 or keys.data_ptr() % 16:
         keys = keys.contiguous()
     H, T, D = keys.shape
@@ -407,8 +429,7 @@ class WindowRiskScorer(RiskScorer):
             queries = self._window_queries(module, hidden_states, w)
         except (AttributeError, NotImplementedError):
             return self._fallback.score_prefill(keys, values, layer_idx)
-        p = _launch_window_attention(keys, queries, self.n_sink, T - w, D ** -0.5)
-        core = _launch_score(keys[:, self.n_sink:], values[:, self.n_sink:], None, p, H, 0, self.epsilon)
+        core = _launch_window_score(keys, values, queries, self.n_sink, T - w, D ** -0.5, self.epsilon)
         plain = type(self)._maybe_normalize is BaseScorer._maybe_normalize and "_maybe_normalize" not in self.__dict__
         if plain and self.normalize_grain in ("layer", "global"):
             return _scale_on_device(core, self.n_sink, self.normalize_grain == "layer")
