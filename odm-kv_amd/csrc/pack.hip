@@ -275,13 +275,21 @@ __global__ __launch_bounds__(CP_THREADS) void compact_kernel(CompactArgs a) {
     __shared__ int cap[5];
     __shared__ int wave_tot[5][CP_THREADS / 64];
     const int bh = blockIdx.y, chunk = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int sl[CP_TPT];
+    const int t0 = chunk * CP_TOKENS + tid * CP_TPT;
+    load_slots(a, bh, t0, sl);
     if (tid < 5) {
         const int32_t* cc = a.chunk_count + (size_t)bh * a.n_chunks * 5 + tid;
         int before = 0, total = 0;
-        for (int c = 0; c < a.n_chunks; ++c) {
-            const int v = cc[(size_t)c * 5];
-            total += v;
-            before += (c < chunk) ? v : 0;
+        for (int c0 = 0; c0 < a.n_chunks; c0 += 16) {        // sixteen counts under way
+            int v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = c0 + u < a.n_chunks ? cc[(size_t)(c0 + u) * 5] : 0;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                total += v[u];
+                before += c0 + u < chunk ? v[u] : 0;
+            }
         }
         const int old = a.old_count[tid * a.nseg + bh];
         const int room = (a.seg_tile[tid][bh + 1] - a.seg_tile[tid][bh]) * TILE;
@@ -289,9 +297,6 @@ __global__ __launch_bounds__(CP_THREADS) void compact_kernel(CompactArgs a) {
         cap[tid] = room;
         if (chunk == 0) a.seg_count[tid][bh] = min(old + total, room);
     }
-    int sl[CP_TPT];
-    const int t0 = chunk * CP_TOKENS + tid * CP_TPT;
-    load_slots(a, bh, t0, sl);
     int mine[5], incl[5];
 #pragma unroll
     for (int L = 0; L < 5; ++L) {
@@ -691,7 +696,9 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
     __syncthreads();
 
     const int wg = blockIdx.x >> 1, n_wg = gridDim.x >> 1;
-    for (int wi = wg * NW + wave; wi < n_work; wi += n_wg * NW) {
+    // (a round of tiles goes over the workgroups first: a handed-over list shorter than the wavefronts then has a SIMD's matrix cores to a
+    // tile instead of half, and most compute units instead of the first few)
+    for (int wi = wave * n_wg + wg; wi < n_work; wi += n_wg * NW) {
         const int gt = tile_list ? tile_list[wi] : wi;
         int li = 0;
 #pragma unroll
