@@ -162,3 +162,14 @@ print("ended")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=root,
                        env=dict(os.environ, PYTHONPATH=os.path.join(root, "odm-kv_amd"), HIP_VISIBLE_DEVICES="-1"))
     assert r.returncode == 0 and "ended" in r.stdout, (r.returncode, r.stderr[-800:])
+
+
+@pytest.mark.parametrize("share3,waves", [(0.0, 12), (0.05, 12), (0.10, 8), (0.25, 8)])   # share of 3-bit tokens; 0.05: 7.3 % of the bytes, 0.10: 14 %
+def test_short_items_of_two_bits_take_twelve_wavefronts(share3, waves):
+    counts = np.zeros((5, 8), np.int64)
+    n3 = int(8192 * share3) // TILE * TILE
+    counts[0], counts[1], counts[4] = 8192 - n3, n3, 132
+    st = _state(counts)
+    st._build_items()
+    _check(st)
+    assert st._items[2] <= 256 and st._worklist.wavefronts == waves and not st._worklist.two_per_cu
