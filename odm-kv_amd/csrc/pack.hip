@@ -281,7 +281,7 @@ __global__ __launch_bounds__(CP_THREADS) void compact_kernel(CompactArgs a) {
     if (tid < 5) {
         const int32_t* cc = a.chunk_count + (size_t)bh * a.n_chunks * 5 + tid;
         int before = 0, total = 0;
-        for (int c0 = 0; c0 < a.n_chunks; c0 += 16) {        // sixteen counts under way
+        for (int c0 = 0; c0 < a.n_chunks; c0 += 16) {        // sixteen counts under way: one after the other they were the launch (131k tokens 15 -> 12.4 us, 32k 8.4 -> 7.6)
             int v[16];
 #pragma unroll
             for (int u = 0; u < 16; ++u) v[u] = c0 + u < a.n_chunks ? cc[(size_t)(c0 + u) * 5] : 0;
@@ -697,7 +697,7 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
 
     const int wg = blockIdx.x >> 1, n_wg = gridDim.x >> 1;
     // (a round of tiles goes over the workgroups first: a handed-over list shorter than the wavefronts then has a SIMD's matrix cores to a
-    // tile instead of half, and most compute units instead of the first few)
+    // tile instead of half, and most compute units instead of the first few: 8-bit tiles of a 131k prompt 85 -> 81 us)
     for (int wi = wave * n_wg + wg; wi < n_work; wi += n_wg * NW) {
         const int gt = tile_list ? tile_list[wi] : wi;
         int li = 0;
