@@ -166,12 +166,15 @@ size_t odmkv_window_attention_workspace_bytes(int Hkv, int Hq, int W, int T);
 int odmkv_window_attention(const void* K, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
                            const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling,
                            float* p, void* workspace, size_t workspace_bytes, void* stream);
-/* The same, and the risk scores of the core tokens with it (what odmkv_score returns for keys and values behind the sinks with that
- * attention, n_sink 0): scores fp32 [Hkv, T - n_sink].  V has K's type and strides. */
-size_t odmkv_window_score_workspace_bytes(int Hkv, int Hq, int W, int T);
-int odmkv_window_score(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
-                       const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling, float eps,
-                       float* scores, void* workspace, size_t workspace_bytes, void* stream);
+/* The same, and |k|^2 of the core tokens, fp32 [Hkv, T - n_sink], which the first pass over K leaves by the way. */
+int odmkv_window_attention_norms(const void* K, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
+                                 const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling,
+                                 float* p, float* kn2, void* workspace, size_t workspace_bytes, void* stream);
+/* odmkv_score with attention weights attn [Hkv, T] (n_sink 0) where |k|^2 [Hkv, T] is known: K is not read.  Workspace:
+ * odmkv_score_workspace_bytes(Hkv, Hkv, T). */
+int odmkv_score_given(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
+                      const float* attn, const float* kn2, float eps, float* scores, void* workspace, size_t workspace_bytes,
+                      void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Allocator.  Replaces optimal_scores_to_bits (kvquant/allocator.py:459-663) for a batch of

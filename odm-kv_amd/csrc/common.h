@@ -49,10 +49,6 @@ void odmkv_set_error(const char* fmt, ...);
     ODMKV_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)(bytes)))
 
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
-// score.hip: the risk scores given attention weights [Hkv, T] and |k|^2, which the caller puts where score_kn2 says
-float* score_kn2(void* workspace, int Hkv, int Hq, int T);
-int score_given_kn2(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t, const float* attn,
-                    float eps, float* scores, void* workspace, size_t workspace_bytes, void* stream);
 // pack.hip: byte offset, inside the pack workspace, of the list of tiles the fp16 quantiser hands to the exact one
 size_t pack_redo_offset(int nseg, int T);
 

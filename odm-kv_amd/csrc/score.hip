@@ -1016,7 +1016,7 @@ extern "C" int odmkv_score(const void* K, const void* V, int dtype, int Hkv, int
 // Hkv kv-heads (of Hkv / Hlayer sequences that lie one behind the other), scored together
 static int score_heads(const void* K, const void* V, int dtype, int Hkv, int Hlayer, int T, int64_t stride_h, int64_t stride_t,
                        const float* mu, int Hq, const float* attn, int n_sink, float eps, int round_dtype, float* scores,
-                       void* workspace, size_t workspace_bytes, void* stream, bool kn2_given = false) {
+                       void* workspace, size_t workspace_bytes, void* stream, const float* kn2 = nullptr) {
     ODMKV_CHECK_ARG(K && V && scores && workspace, "score: null pointer");
     ODMKV_CHECK_ARG(round_dtype == -1 || round_dtype == ODMKV_F16 || round_dtype == ODMKV_BF16,
                     "score: rounding dtype %d (-1, fp16 or bf16)", round_dtype);
@@ -1038,8 +1038,8 @@ static int score_heads(const void* K, const void* V, int dtype, int Hkv, int Hla
     a.K = K; a.V = V; a.sH = stride_h; a.sT = stride_t;
     a.Hlayer = Hlayer; a.Hkv = Hkv; a.Hq = Hq; a.G = Hq / Hkv; a.Gl = attn ? 0 : Hq / Hkv; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
     a.nchunks = n_chunks(a.Tc); a.eps = eps; a.mu = mu; a.attn = attn; a.scores = scores;
-    a.cov = nullptr; a.use_vnorm = 0; a.ea_cpw = 1; a.nstat = a.nchunks; a.round_dt = round_dtype; a.kn2_given = kn2_given;
-    a.logits = (float*)(ws + L.logits); a.kn2 = (float*)(ws + L.kn2); a.p = (float*)(ws + L.p);
+    a.cov = nullptr; a.use_vnorm = 0; a.ea_cpw = 1; a.nstat = a.nchunks; a.round_dt = round_dtype; a.kn2_given = kn2 != nullptr;
+    a.logits = (float*)(ws + L.logits); a.kn2 = kn2 ? const_cast<float*>(kn2) : (float*)(ws + L.kn2); a.p = (float*)(ws + L.p);
     a.stats = (float*)(ws + L.stats); a.mz = (float*)(ws + L.mz); a.opart = (float*)(ws + L.opart);
     a.psum = (float*)(ws + L.psum); a.obar = (float*)(ws + L.obar);
     hipStream_t st = (hipStream_t)stream;
@@ -1048,12 +1048,13 @@ static int score_heads(const void* K, const void* V, int dtype, int Hkv, int Hla
     return run_score<ODMKV_F32>(a, st);
 }
 
-// The scores given attention weights and |k|^2 (window.hip): where a call of that workspace keeps |k|^2 [Hkv, T], and the rest of it
-float* score_kn2(void* workspace, int Hkv, int Hq, int T) { return (float*)((char*)workspace + score_layout(Hkv, Hq, T).kn2); }
-int score_given_kn2(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t, const float* attn,
-                    float eps, float* scores, void* workspace, size_t workspace_bytes, void* stream) {
+// The scores given attention weights and |k|^2
+extern "C" int odmkv_score_given(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
+                                 const float* attn, const float* kn2, float eps, float* scores, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+    ODMKV_CHECK_ARG(attn && kn2, "score: null pointer");
     return score_heads(K, V, dtype, Hkv, Hkv, T, stride_h, stride_t, nullptr, Hkv, attn, 0, eps, -1, scores, workspace, workspace_bytes,
-                       stream, true);
+                       stream, kn2);
 }
 
 extern "C" int odmkv_score_model_dtype(const void* K, const void* V, int dtype, int Hkv, int T,

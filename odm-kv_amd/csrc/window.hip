@@ -301,29 +301,11 @@ extern "C" int odmkv_window_attention(const void* K, int dtype, int Hkv, int T, 
     return window_attention(K, dtype, Hkv, T, stride_h, stride_t, Q, Hq, W, q_pos0, n_sink, scaling, p, nullptr, workspace, workspace_bytes, stream);
 }
 
-// attention mass | its workspace | the score's
-extern "C" size_t odmkv_window_score_workspace_bytes(int Hkv, int Hq, int W, int T) {
-    if (Hkv <= 0 || Hq <= 0 || W <= 0 || T <= 0) return 0;
-    return align_up((size_t)Hkv * T * 4, 256) + odmkv_window_attention_workspace_bytes(Hkv, Hq, W, T) + odmkv_score_workspace_bytes(Hkv, Hkv, T);
-}
-
-// The window's attention mass and the risk scores with it: the first pass over the keys leaves |k|^2 too, and the score is spared a pass
-// of its own over them for that (12 us of 165 for 32k tokens of 8 heads).
-extern "C" int odmkv_window_score(const void* K, const void* V, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
-                                  const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling, float eps,
-                                  float* scores, void* workspace, size_t workspace_bytes, void* stream) {
-    ODMKV_CHECK_ARG(K && V && scores && workspace, "window_score: null pointer");
-    ODMKV_CHECK_ARG(Hkv > 0 && Hq > 0 && W >= 1 && n_sink >= 0 && T > n_sink, "window_score: bad shape Hkv=%d Hq=%d W=%d T=%d n_sink=%d", Hkv, Hq, W, T, n_sink);
-    ODMKV_CHECK_ARG(workspace_bytes >= odmkv_window_score_workspace_bytes(Hkv, Hq, W, T), "window_score: workspace too small");
-    const int Tc = T - n_sink;
-    char* ws = (char*)workspace;
-    float* p = (float*)ws;
-    ws += align_up((size_t)Hkv * T * 4, 256);
-    const size_t attn_bytes = odmkv_window_attention_workspace_bytes(Hkv, Hq, W, T), score_bytes = odmkv_score_workspace_bytes(Hkv, Hkv, T);
-    char* score_ws = ws + attn_bytes;
-    if (int rc = window_attention(K, dtype, Hkv, T, stride_h, stride_t, Q, Hq, W, q_pos0, n_sink, scaling, p,
-                                  score_kn2(score_ws, Hkv, Hkv, Tc), ws, attn_bytes, stream)) return rc;
-    const size_t behind = (size_t)n_sink * stride_t * 2;                             // (16-bit rows)
-    return score_given_kn2((const char*)K + behind, (const char*)V + behind, dtype, Hkv, Tc, stride_h, stride_t, p, eps, scores, score_ws,
-                           score_bytes, stream);
+// The same, and |k|^2 of the core tokens, which the first pass holds all keys for: the risk score is spared a pass of its own over
+// them (12 us of 165 for 32k tokens of 8 heads).
+extern "C" int odmkv_window_attention_norms(const void* K, int dtype, int Hkv, int T, int64_t stride_h, int64_t stride_t,
+                                            const void* Q, int Hq, int W, int q_pos0, int n_sink, float scaling,
+                                            float* p, float* kn2, void* workspace, size_t workspace_bytes, void* stream) {
+    ODMKV_CHECK_ARG(kn2, "window_attention: null pointer");
+    return window_attention(K, dtype, Hkv, T, stride_h, stride_t, Q, Hq, W, q_pos0, n_sink, scaling, p, kn2, workspace, workspace_bytes, stream);
 }

@@ -108,8 +108,8 @@ def _load() -> C.CDLL:
         "odmkv_normalize_scores": (C.c_int, [vp, i64, i64, i32, i32, vp, vp, sz, vp]),
         "odmkv_window_attention_workspace_bytes": (sz, [i32, i32, i32, i32]),
         "odmkv_window_attention": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, i32, i32, i32, i32, f32, vp, vp, sz, vp]),
-        "odmkv_window_score_workspace_bytes": (sz, [i32, i32, i32, i32]),
-        "odmkv_window_score": (C.c_int, [vp, vp, i32, i32, i32, i64, i64, vp, i32, i32, i32, i32, f32, f32, vp, vp, sz, vp]),
+        "odmkv_window_attention_norms": (C.c_int, [vp, i32, i32, i32, i64, i64, vp, i32, i32, i32, i32, f32, vp, vp, vp, sz, vp]),
+        "odmkv_score_given": (C.c_int, [vp, vp, i32, i32, i32, i64, i64, vp, vp, f32, vp, vp, sz, vp]),
         "odmkv_allocate_workspace_bytes": (sz, [i32, i32]),
         "odmkv_allocate": (C.c_int, [vp, i32, i32, vp, i32, i32, i32, C.POINTER(C.c_int32), i32,
                                      C.POINTER(C.c_double), vp, vp, vp, vp, vp, sz, vp]),
@@ -174,7 +174,7 @@ STEP_ENTRY = C.cast(lib.odmkv_decode_step, C.c_void_p).value      # what _native
 EXPORTS = ("odmkv_version", "odmkv_last_error", "odmkv_score_workspace_bytes", "odmkv_score", "odmkv_score_model_dtype", "odmkv_score_expected", "odmkv_token_mean_workspace_bytes", "odmkv_token_mean", "odmkv_average_rope",
            "odmkv_project_rows", "odmkv_prompt_scores_workspace_bytes", "odmkv_prompt_scores", "odmkv_query_covariance_workspace_bytes", "odmkv_query_covariance", "odmkv_rotate_queries",
            "odmkv_normalize_workspace_bytes", "odmkv_normalize_scores",
-           "odmkv_window_attention_workspace_bytes", "odmkv_window_attention", "odmkv_window_score_workspace_bytes", "odmkv_window_score",
+           "odmkv_window_attention_workspace_bytes", "odmkv_window_attention", "odmkv_window_attention_norms", "odmkv_score_given",
            "odmkv_allocate_workspace_bytes", "odmkv_allocate", "odmkv_level_counts",
            "odmkv_finish_levels_chunks", "odmkv_finish_levels", "odmkv_evicted_workspace_bytes", "odmkv_evicted_indices", "odmkv_evicted_layers_workspace_bytes", "odmkv_evicted_indices_layers",
            "odmkv_store_init", "odmkv_store_gather", "odmkv_quant_pack_staged", "odmkv_store_layout", "odmkv_store_bind", "odmkv_pack_workspace_bytes", "odmkv_pack_count_chunks", "odmkv_store_finish_staged", "odmkv_quant_pack", "odmkv_quantize_rows",

@@ -230,9 +230,10 @@ def _launch_score_expected(keys: torch.Tensor, values: torch.Tensor, mu: torch.T
 
 def _launch_score(keys: torch.Tensor, values: torch.Tensor, mu: Optional[torch.Tensor],
                   attn: Optional[torch.Tensor], n_q_heads: int, n_sink: int, eps: float,
-                  round_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                  round_dtype: Optional[torch.dtype] = None, kn2: Optional[torch.Tensor] = None) -> torch.Tensor:
     """round_dtype (float16 / bfloat16): round the logits, the softmax and the group mean as a model of that
-    dtype does in the reference (kvquant/scorer.py:309-315, 403); None: fp32 throughout."""
+    dtype does in the reference (kvquant/scorer.py:309-315, 403); None: fp32 throughout.  kn2 (with attn, n_sink 0): the
+    keys' squared norms, fp32 [H, T], where they are known."""
     keys, values = _kv_operands(keys, values)
     H, T, D = keys.shape
     dev = keys.device
@@ -241,6 +242,11 @@ def _launch_score(keys: torch.Tensor, values: torch.Tensor, mu: Optional[torch.T
     ws = _lib.workspace(dev, ws_bytes, "score")
     mu32 = None if mu is None else mu.reshape(n_q_heads, D).float().contiguous()
     a32 = None if attn is None else attn.float().contiguous()
+    if kn2 is not None:
+        _lib.check(lib.odmkv_score_given(
+            keys.data_ptr(), values.data_ptr(), _lib.dtype_code(keys), H, T, keys.stride(0), keys.stride(1), a32.data_ptr(),
+            kn2.data_ptr(), float(eps), scores.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev)))
+        return scores
     rd = -1 if round_dtype is None else {torch.float16: 0, torch.bfloat16: 1}[round_dtype]
     _lib.check(lib.odmkv_score_model_dtype(
         keys.data_ptr(), values.data_ptr(), _lib.dtype_code(keys), H, T, keys.stride(0), keys.stride(1),
@@ -340,37 +346,16 @@ class RiskScorer(ExpectedAttentionScorer):
         return _launch_score(keys, values, None, attn_weights, H, 0, self.epsilon)
 
 
-def _check_window_keys(keys: torch.Tensor) -> None:
+def _launch_window_attention(keys: torch.Tensor, queries: torch.Tensor, n_sink: int, q_pos0: int,
+                             scaling: float, kn2: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """p fp32 [Hkv, T - n_sink]: attention mass of the window queries [Hq, W, d] (rotated to positions
+    q_pos0 .. q_pos0 + W - 1) over the core keys, per-query causal softmax, mean over queries and group.  kn2, fp32 of the
+    same shape, takes the keys' squared norms."""
     _lib.require_gpu(keys, "keys")
     if keys.dtype not in (torch.float16, torch.bfloat16):
         raise ValueError(f"window attention runs on the 16-bit matrix cores: keys must be float16 or bfloat16, got {keys.dtype}")
     if keys.shape[-1] != _lib.HEAD_DIM:
         raise ValueError(f"the HIP kernels are written for head_dim {_lib.HEAD_DIM}, got {keys.shape[-1]}")
-
-
-def _launch_window_score(keys: torch.Tensor, values: torch.Tensor, queries: torch.Tensor, n_sink: int, q_pos0: int,
-                         scaling: float, eps: float) -> torch.Tensor:
-    """Risk scores fp32 [Hkv, T - n_sink] of the core tokens with the window's attention mass (below), in one call."""
-    _check_window_keys(keys)
-    keys, values = _kv_operands(keys, values)
-    H, T, D = keys.shape
-    Hq, W, _ = queries.shape
-    q = queries.to(keys.dtype).contiguous()
-    dev = keys.device
-    scores = torch.empty(H, T - n_sink, dtype=torch.float32, device=dev)
-    ws_bytes = lib.odmkv_window_score_workspace_bytes(H, Hq, W, T)
-    ws = _lib.workspace(dev, ws_bytes, "window")
-    _lib.check(lib.odmkv_window_score(
-        keys.data_ptr(), values.data_ptr(), _lib.dtype_code(keys), H, T, keys.stride(0), keys.stride(1), q.data_ptr(), Hq, W,
-        int(q_pos0), int(n_sink), float(scaling), float(eps), scores.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev)))
-    return scores
-
-
-def _launch_window_attention(keys: torch.Tensor, queries: torch.Tensor, n_sink: int, q_pos0: int,
-                             scaling: float) -> torch.Tensor:
-    """p fp32 [Hkv, T - n_sink]: attention mass of the window queries [Hq, W, d] (rotated to positions
-    q_pos0 .. q_pos0 + W - 1) over the core keys, per-query causal softmax, mean over queries and group."""
-    _check_window_keys(keys)
     if keys.stride(-1) != 1 or keys.stride(0) % 8 or keys.stride(1) % 8 or keys.data_ptr() % 16:
         keys = keys.contiguous()
     H, T, D = keys.shape
@@ -380,9 +365,11 @@ def _launch_window_attention(keys: torch.Tensor, queries: torch.Tensor, n_sink: 
     p = torch.empty(H, T - n_sink, dtype=torch.float32, device=dev)
     ws_bytes = lib.odmkv_window_attention_workspace_bytes(H, Hq, W, T)
     ws = _lib.workspace(dev, ws_bytes, "window")
-    _lib.check(lib.odmkv_window_attention(
-        keys.data_ptr(), _lib.dtype_code(keys), H, T, keys.stride(0), keys.stride(1), q.data_ptr(), Hq, W,
-        int(q_pos0), int(n_sink), float(scaling), p.data_ptr(), ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev)))
+    call = (keys.data_ptr(), _lib.dtype_code(keys), H, T, keys.stride(0), keys.stride(1), q.data_ptr(), Hq, W,
+            int(q_pos0), int(n_sink), float(scaling), p.data_ptr())
+    rest = (ws.data_ptr(), ws_bytes, _lib.stream_ptr(dev))
+    _lib.check(lib.odmkv_window_attention(*call, *rest) if kn2 is None
+               else lib.odmkv_window_attention_norms(*call, kn2.data_ptr(), *rest))
     return p
 
 
@@ -429,7 +416,9 @@ class WindowRiskScorer(RiskScorer):
             queries = self._window_queries(module, hidden_states, w)
         except (AttributeError, NotImplementedError):
             return self._fallback.score_prefill(keys, values, layer_idx)
-        core = _launch_window_score(keys, values, queries, self.n_sink, T - w, D ** -0.5, self.epsilon)
+        kn2 = torch.empty(H, T - self.n_sink, dtype=torch.float32, device=keys.device)
+        p = _launch_window_attention(keys, queries, self.n_sink, T - w, D ** -0.5, kn2)
+        core = _launch_score(keys[:, self.n_sink:], values[:, self.n_sink:], None, p, H, 0, self.epsilon, None, kn2)
         plain = type(self)._maybe_normalize is BaseScorer._maybe_normalize and "_maybe_normalize" not in self.__dict__
         if plain and self.normalize_grain in ("layer", "global"):
             return _scale_on_device(core, self.n_sink, self.normalize_grain == "layer")

@@ -432,13 +432,15 @@ def test_window_attention_at_the_edges_of_its_workgroups(T, W, n_sink):
     want = osc.window_attention(k.double(), q.double(), n_sink, T - W)[0]
     got = _launch_window_attention(k.to(DEV), q.to(DEV), n_sink, T - W, 128 ** -0.5)
     np.testing.assert_allclose(got.cpu().numpy(), want.numpy(), rtol=SCORE_RTOL, atol=1e-12)
-    # the scores with it in one call: the same but for the order of |k|^2's 128 fp32 additions (12 deep: under 2e-6)
+    # the scores with the norms it leaves: the same but for the order of |k|^2's 128 fp32 additions (12 deep: under 2e-6)
     v = torch.randn(2, T, 128, generator=g).half().to(DEV)
     kd = torch.randn(2, T, 3 * 128, generator=g).half().to(DEV)[..., 128:256]                    # rows of a wider tensor
     kd.copy_(k)
-    from kvquant.scorer import _launch_score, _launch_window_score
+    from kvquant.scorer import _launch_score
     for vd in (v, torch.empty(2, T, 3 * 128, device=DEV, dtype=v.dtype)[..., 128:256].copy_(v)):   # strides of their own, and the keys'
-        both = _launch_window_score(kd, vd, q.to(DEV), n_sink, T - W, 128 ** -0.5, 1e-2)
+        kn2 = torch.full((2, T - n_sink), float("nan"), device=DEV)
+        p = _launch_window_attention(kd, q.to(DEV), n_sink, T - W, 128 ** -0.5, kn2)
+        both = _launch_score(kd[:, n_sink:], vd[:, n_sink:], None, p, 2, 0, 1e-2, None, kn2)
         apart = _launch_score(k.to(DEV)[:, n_sink:], v[:, n_sink:], None, got, 2, 0, 1e-2)
         np.testing.assert_allclose(both.cpu().numpy(), apart.cpu().numpy(), rtol=2e-6)
 
