@@ -2,7 +2,7 @@
 // tokens is handed over as further heads of their kv-head).
 //
 // Two launches per call:
-//   1. main:  one workgroup (8, 12 or 16 wavefronts) per work item = a run of 64-token tiles of one (sequence,
+//   1. main:  one workgroup (8 or 12 wavefronts) per work item = a run of 64-token tiles of one (sequence,
 //             kv-head, level).  It rounds the group's queries to fp16 (what a model in fp16/bf16 hands over
 //             anyway), rotates them into the basis of the quantised keys on the matrix cores (q' = Pi_k q16 from a
 //             precomputed fp16 high + low operand table, kept as fp16 high + low rows), and streams the item's packed
