@@ -36,8 +36,12 @@
 // corners it therefore beats it, as computed, throughout the box.  And a level with fewer bits that loses by
 // that much at some lambda loses at every smaller one (its difference falls with lambda), one with more bits at every larger
 // one: a sum that is above the budget with every token that is nearly tied counted at its least is above it for all smaller
-// multipliers.  An error that is negative or not finite breaks the first part: such calls keep the window open, and the
-// replay asks all tokens every time.
+// multipliers.  A cost with a negative error is a difference of two products, whose sizes add up to no more than the cost and twice the
+// negative one: there the margin grows by 2^-18 of the score times the largest negative error, which is linear in (s, lambda) as well
+// (eight of the roundings above, 3 x 2^-24, each side, and two where the second best is below zero).  Infinite errors are constant in lambda (and 0 * inf, a NaN, meets
+// zero scores alone, which take the first level in any case); NaN, and -inf behind another, are given the infinity that every token
+// treats alike (odmkv_allocate).  Without a window for such tables the replay asked all tokens, in one workgroup a row.
+// Us a call, one row of 262144: with a negative error 3900 -> 62, an infinite one 3900 -> 59, eviction at an infinite cost 2640 -> 61.
 #include <algorithm>
 #include <cmath>
 #include "common.h"
@@ -56,7 +60,7 @@
 #define HB_BINS 1024                          // bin 0: zeros; the last: infinities and NaN; between them equal steps of the bit pattern
 #define MAX_TURN 2048                         // rows of a turn: what the histograms' workspace is cut for
 #define LAMBDA_CAP 100000008.0f               // the fp32 number behind the largest multiplier that is asked for, 1e8
-#define KEEP (1.0f - 0x1p-20f)                // one cost beats another by more than rounding: other * KEEP > best + TINY
+#define KEEP (1.0f - 0x1p-20f)                // one cost beats another by more than rounding: other * KEEP > best + slack()
 #define TINY 1e-36f
 
 struct RowState {
@@ -77,12 +81,11 @@ struct AllocArgs {
     int n_chunks, iters;           // workgroups of a row in a pass, and how many runs of tokens each of them walks
     int chunk_tokens;
     int n_cand;                    // workgroups of a row in the assignment
-    int n_pass;                    // the narrowing pass, if any, and the collecting one
     int n_scan;                    // workgroups of a row in the range and the histogram
     // the levels on the lower hull of (bits, error): beyond a ratio score / lambda of step_at[i] a token takes step_bits[i] more than before
     int n_steps, first_bits;
     float step_at[NLV], step_bits[NLV];
-    int prune;                     // every error is finite and not negative: the window may be narrowed
+    float slack_s;                 // 2^-18 of the largest negative error's size
     float eps[NLV];
     float bitsf[NLV];
     int nominal[NLV];
@@ -103,6 +106,9 @@ __device__ static inline bool is_sink(const AllocArgs& a, int row, int i) {
     if (a.sink_mask) return a.sink_mask[(size_t)row * a.n + i] != 0;
     return a.n_sink > 0 && (i % a.period) < a.n_sink;
 }
+
+// what a cost of a token must be beaten by, beside the factor KEEP
+__device__ static inline float slack(const AllocArgs& a, float s) { return __fmaf_rn(s, a.slack_s, TINY); }
 
 // torch's clamp(min=0) / non-finite patch / nan_to_num, in that order
 __device__ static inline float clean_score(float v, bool patch, float top) {
@@ -283,7 +289,7 @@ __global__ __launch_bounds__(SE_THREADS) void alloc_search_kernel(AllocArgs a) {
     const float budget = (float)(target * (double)total);
     // (Scores that are not finite count as beyond everything.)
     float l0 = SE_LEAST, l1 = LAMBDA_CAP, guess = 1.0f;
-    if (a.prune && total != 0u) {
+    if (total != 0u) {
 #pragma unroll 1
         for (int round = 0; round < 3; ++round) {
             const float span = log2f(l1 / l0) * (1.0f / (float)(SE_THREADS - 1)), base = l0;
@@ -361,14 +367,14 @@ __device__ static inline double replay(float lb, F above) {
     return (lo + hi) * 0.5;
 }
 
-// Start of pass j: the state before it in `cur` (shared memory) for the whole workgroup.  The collecting pass narrows the window by what the
+// Start of a pass: the state before it in `cur` (shared memory) for the whole workgroup.  The collecting pass narrows the window by what the
 // narrowing one found, and the row's first workgroup writes the new state to third 1.  Ends with a barrier.
 template <bool COLLECT>
-__device__ static void carry_state(const AllocArgs& a, int row, int j, RowState* cur, unsigned int* tot) {
+__device__ static void carry_state(const AllocArgs& a, int row, RowState* cur, unsigned int* tot) {
     const int tid = threadIdx.x;
     // everything the launch needs of the last one is asked for at once: a thread's partial sums and the whole state
     unsigned int v0[8];                                      // (256 workgroups a row at most: 8 x 512)
-    const int n_part = COLLECT && j > 0 ? a.n_chunks * SLOTS : 0;
+    const int n_part = COLLECT ? a.n_chunks * SLOTS : 0;
     const unsigned int* p = a.partial + (size_t)row * a.n_chunks * SLOTS;
 #pragma unroll
     for (int u = 0; u < 8; ++u) v0[u] = tid + u * EV_THREADS < n_part ? p[tid + u * EV_THREADS] : 0u;
@@ -389,7 +395,7 @@ __device__ static void carry_state(const AllocArgs& a, int row, int j, RowState*
         if ((tid & 63) < SLOTS && v) atomicAdd(&tot[tid & (SLOTS - 1)], v);
         __syncthreads();
         if (tid == 0) {
-            if (j > 0 && cur->n_active != 0) {
+            if (cur->n_active != 0) {
                 for (int i = 0; i < NGRID; ++i) {            // sums up to 2^24: exact in fp32
                     const float sum = (float)tot[i], off = (float)tot[NGRID + i];
                     shrink(*cur, cur->grid[i], fmaxf(sum - off, 0.0f), sum + off);
@@ -421,7 +427,7 @@ __device__ static void carry_state(const AllocArgs& a, int row, int j, RowState*
 // long row pays for: a workgroup walks `iters` runs of TPT tokens per thread (at most 256 workgroups a row; short rows keep
 // one token per thread).
 template <int K, int TPT, bool COLLECT>
-__global__ __launch_bounds__(EV_THREADS) void alloc_pass_kernel(AllocArgs a, int j) {
+__global__ __launch_bounds__(EV_THREADS) void alloc_pass_kernel(AllocArgs a) {
     constexpr int RUN = EV_THREADS * TPT, LIST = 2 * RUN;
     __shared__ unsigned int lsum[SLOTS];
     __shared__ unsigned int tot[SLOTS];
@@ -444,7 +450,7 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_pass_kernel(AllocArgs a, int
     request(0);
     if (tid < SLOTS) lsum[tid] = 0u;
     if (tid == 0) n_open = 0;
-    carry_state<COLLECT>(a, row, j, &cur, tot);
+    carry_state<COLLECT>(a, row, &cur, tot);
     const RowState& st = cur;
     if (st.n_active == 0) return;                            // (the finish looks at no partial sum of such a row)
     const Cleaner clean(st);
@@ -473,11 +479,12 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_pass_kernel(AllocArgs a, int
                 if (cst < best) { best = cst; bn = a.nominal[k]; }
             }
             sum += (unsigned int)bn;
-            if (!(second * KEEP > best + TINY)) {            // nearly tied: by how much the level may be another at this multiplier's neighbours
+            const float margin = best + slack(a, s);
+            if (!(second * KEEP > margin)) {                 // nearly tied: by how much the level may be another at this multiplier's neighbours
                 int lo = bn, hi = bn;
 #pragma unroll 1
                 for (int k = 0; k < K; ++k)
-                    if (__fadd_rn(__fmul_rn(s, a.eps[k]), __fmul_rn(st.grid[c], a.bitsf[k])) * KEEP <= best + TINY) { lo = min(lo, a.nominal[k]); hi = max(hi, a.nominal[k]); }
+                    if (__fadd_rn(__fmul_rn(s, a.eps[k]), __fmul_rn(st.grid[c], a.bitsf[k])) * KEEP <= margin) { lo = min(lo, a.nominal[k]); hi = max(hi, a.nominal[k]); }
                 ties += (unsigned int)max(bn - lo, hi - bn);
             }
         }
@@ -488,31 +495,28 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_pass_kernel(AllocArgs a, int
 #pragma unroll
         for (int e = 0; e < TPT; ++e) {
             const float s = active[e] ? clean(raw[e]) : 0.0f;
-            bool settled = false;
-            if (a.prune) {
-                int at[2];
-                settled = true;
-                float se[K];
+            int at[2];
+            bool settled = true;
+            float se[K];
 #pragma unroll
-                for (int k = 0; k < K; ++k) se[k] = __fmul_rn(s, a.eps[k]);
+            for (int k = 0; k < K; ++k) se[k] = __fmul_rn(s, a.eps[k]);
 #pragma unroll
-                for (int side = 0; side < 2; ++side) {
-                    float best = __fadd_rn(se[0], end[side][0]), second = INFINITY;
-                    int bn = 0;
+            for (int side = 0; side < 2; ++side) {
+                float best = __fadd_rn(se[0], end[side][0]), second = INFINITY;
+                int bn = 0;
 #pragma unroll
-                    for (int k = 1; k < K; ++k) {
-                        const float cst = __fadd_rn(se[k], end[side][k]);
-                        second = __builtin_amdgcn_fmed3f(cst, best, second);
-                        if (cst < best) { best = cst; bn = k; }
-                    }
-                    at[side] = bn;
-                    settled = settled && second * KEEP > best + TINY;
+                for (int k = 1; k < K; ++k) {
+                    const float cst = __fadd_rn(se[k], end[side][k]);
+                    second = __builtin_amdgcn_fmed3f(cst, best, second);
+                    if (cst < best) { best = cst; bn = k; }
                 }
-                settled = settled && at[0] == at[1];
-                if (active[e] && settled) {
+                at[side] = bn;
+                settled = settled && second * KEEP > best + slack(a, s);
+            }
+            settled = (settled && at[0] == at[1]) || s == 0.0f;        // (a zero takes the first level: every cost is lambda's part alone, or a NaN)
+            if (active[e] && settled) {
 #pragma unroll
-                    for (int k = 0; k < K; ++k) cnt[k] += at[0] == k;
-                }
+                for (int k = 0; k < K; ++k) cnt[k] += at[0] == k;
             }
             bool keep = active[e] && !settled;
             unsigned long long m = __ballot(keep);
@@ -720,7 +724,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
                     if (v0 < p0) { p0 = v0; b0 = k; }
                     if (v1 < p1) { p1 = v1; b1 = k; }
                 }
-                const bool is_settled = b0 == b1 && q0 * KEEP > p0 + TINY && q1 * KEEP > p1 + TINY;
+                const bool is_settled = b0 == b1 && q0 * KEEP > p0 + slack(a, s) && q1 * KEEP > p1 + slack(a, s);
 #pragma unroll
                 for (int k = 0; k < K; ++k) cnt[k] += is_settled && b0 == k ? tokens : 0;
                 const bool keep = on && !is_settled;
@@ -751,7 +755,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
         for (int k = 0; k < K; ++k) settled_sum += settled[k] * a.nominal[k];
         __syncthreads();
     };
-    const bool may_close = a.prune && cur.wa == la && cur.wb == lb;      // (else the final multiplier may lie beside the window)
+    const bool may_close = cur.wa == la && cur.wb == lb;     // (else the final multiplier may lie beside the window)
     const double lam = replay(lb, [&](float lambda) {            // (every thread runs it: the answers are the workgroup's)
         if (lambda <= la || lambda == known_above) return true;
         if (lambda >= lb || lambda == known_within) return false;
@@ -1150,17 +1154,12 @@ static int launch_search(const AllocArgs& a, int tpt, hipStream_t st) {
     const dim3 grid(a.n_chunks, a.rows), block(EV_THREADS);
     hipLaunchKernelGGL(alloc_search_kernel, dim3(a.rows), dim3(SE_THREADS), 0, st, a);
     ODMKV_CHECK_LAUNCH("alloc_search_kernel");
-    for (int j = 0; j < a.n_pass; ++j) {
-        const bool collect = j == a.n_pass - 1;
-        if (tpt == 1) {
-            if (collect) hipLaunchKernelGGL((alloc_pass_kernel<K, 1, true>), grid, block, 0, st, a, j);
-            else hipLaunchKernelGGL((alloc_pass_kernel<K, 1, false>), grid, block, 0, st, a, j);
-        } else {
-            if (collect) hipLaunchKernelGGL((alloc_pass_kernel<K, EV_BIG, true>), grid, block, 0, st, a, j);
-            else hipLaunchKernelGGL((alloc_pass_kernel<K, EV_BIG, false>), grid, block, 0, st, a, j);
-        }
-        ODMKV_CHECK_LAUNCH("alloc_pass_kernel");
-    }
+    if (tpt == 1) hipLaunchKernelGGL((alloc_pass_kernel<K, 1, false>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((alloc_pass_kernel<K, EV_BIG, false>), grid, block, 0, st, a);
+    ODMKV_CHECK_LAUNCH("alloc_pass_kernel (narrow)");
+    if (tpt == 1) hipLaunchKernelGGL((alloc_pass_kernel<K, 1, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((alloc_pass_kernel<K, EV_BIG, true>), grid, block, 0, st, a);
+    ODMKV_CHECK_LAUNCH("alloc_pass_kernel (collect)");
     hipLaunchKernelGGL((alloc_finish_kernel<K>), dim3(a.rows), dim3(FN_THREADS), 0, st, a);
     ODMKV_CHECK_LAUNCH("alloc_finish_kernel");
     hipLaunchKernelGGL((alloc_assign_kernel<K>), dim3(a.n_cand, a.rows), block, 0, st, a);
@@ -1196,24 +1195,32 @@ extern "C" int odmkv_allocate(const float* scores, int rows, int n,
     a.n = n;
     a.period = period > 0 ? period : n; a.n_sink = sink_mask ? 0 : n_sink; a.sink_bits = sink_bits; a.K = n_levels;
     a.n_cand = (n + EV_TOKENS - 1) / EV_TOKENS;
-    a.prune = 1;
-    for (int k = 0; k < n_levels; ++k)
-        if (!(eps[k] >= 0.0) || !std::isfinite((float)eps[k])) a.prune = 0;
     for (int k = 0; k < NLV; ++k) {
         a.eps[k] = k < n_levels ? (float)eps[k] : 0.0f;
         a.bitsf[k] = k < n_levels ? (float)levels[k] : 0.0f;
         a.nominal[k] = k < n_levels ? levels[k] : 0;
     }
-    a.n_pass = a.prune ? 2 : 1;
+    // A NaN or infinite error means the same for every positive score at every multiplier, and a zero score takes the first level whatever
+    // the table says (its product is a NaN, or it costs least): the first level's NaN, which keeps every token, is -inf; another's, never
+    // below anything, and -inf behind -inf, never below that, are +inf.
+    bool seen_lowest = false;
+    float negative = 0.0f;
+    for (int k = 0; k < n_levels; ++k) {
+        if (std::isnan(a.eps[k])) a.eps[k] = k == 0 ? -INFINITY : INFINITY;
+        if (a.eps[k] == -INFINITY && seen_lowest) a.eps[k] = INFINITY;
+        seen_lowest = seen_lowest || a.eps[k] == -INFINITY;
+        if (std::isfinite(a.eps[k])) negative = std::max(negative, -a.eps[k]);
+    }
+    a.slack_s = 0x1p-18f * negative;
     a.n_steps = 0;
     a.first_bits = levels[0];
-    for (int at = 0; a.prune && at < n_levels - 1;) {
+    for (int at = 0; at < n_levels - 1;) {
         int next = -1;
         double ratio = INFINITY;                                         // score / lambda from which `next` is better than `at`
         for (int k = at + 1; k < n_levels; ++k) {
             const double gain = (double)a.eps[at] - (double)a.eps[k];
             const double r = gain > 0.0 ? (levels[k] - levels[at]) / gain : INFINITY;
-            if (r <= ratio && r < 1e30) { ratio = r; next = k; }
+            if ((r < ratio || (r == ratio && r > 0.0)) && r < 1e30) { ratio = r; next = k; }      // (out of an infinite error: the narrowest finite one)
         }
         if (next < 0) break;
         a.step_at[a.n_steps] = (float)ratio;
