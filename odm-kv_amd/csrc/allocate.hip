@@ -262,9 +262,15 @@ __global__ __launch_bounds__(SE_THREADS) void alloc_search_kernel(AllocArgs a) {
     __shared__ int last_above, first_within, last_over;
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     static_assert(HB_BINS == SE_THREADS, "a bin per thread");
-    const unsigned int mine = a.hist[(size_t)row * HB_BINS + tid];
+    unsigned int mine = a.hist[(size_t)row * HB_BINS + tid];
+    const unsigned int zeros = a.hist[(size_t)row * HB_BINS], odd = a.hist[(size_t)row * HB_BINS + HB_BINS - 1];
     double target = a.target[row];                           // clamp the budget into the level range
     const Bins bins = row_bins(a, row);
+    const bool has_finite = bins.top != 0u || zeros != 0u;
+    if (has_finite) {                                        // infinities and NaN are taken for the largest finite score
+        if (tid == HB_BINS - 1) mine = 0u;
+        if (tid == (bins.top == 0u ? 0 : 1 + (int)((bins.top - bins.base) >> bins.shift))) mine += odd;
+    }
     unsigned int incl = mine;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -283,11 +289,10 @@ __global__ __launch_bounds__(SE_THREADS) void alloc_search_kernel(AllocArgs a) {
     from[tid] = total - before;
     if (tid == 0) from[HB_BINS] = 0u;
     __syncthreads();
-    const unsigned int finite = total - from[HB_BINS - 1];
     target = fmin(target, (double)a.nominal[a.K - 1]);
     target = fmax(target, (double)a.nominal[0]);
     const float budget = (float)(target * (double)total);
-    // (Scores that are not finite count as beyond everything.)
+    // (Without a finite score, those that are not count as beyond everything.)
     float l0 = SE_LEAST, l1 = LAMBDA_CAP, guess = 1.0f;
     if (total != 0u) {
 #pragma unroll 1
@@ -335,8 +340,8 @@ __global__ __launch_bounds__(SE_THREADS) void alloc_search_kernel(AllocArgs a) {
                                  guess * (1.0f + w2), guess * (1.0f + w1), guess * (1.0f + w), hi};
         for (int i = 0; i < NGRID; ++i) st.grid[i] = fminf(fmaxf(at[i], lo), hi);
         st.n_active = (int)total;
-        st.has_finite = finite != 0u;
-        st.has_nonfinite = finite != total;
+        st.has_finite = has_finite;
+        st.has_nonfinite = odd != 0u;
         st.max_finite = bins.top;
         for (int k = 0; k < NLV; ++k) st.final_hist[k] = 0;
     }

@@ -267,12 +267,15 @@ def _awkward_scores(kind, rows, n, g):
         s[torch.rand(rows, n, generator=g) < 0.5] = 0.0
     elif kind == "two far groups":                             # a gap of thirty octaves in the middle of the histogram
         s[:, n // 3:] *= 2.0 ** -30
+    elif kind == "a third not finite":
+        s[torch.rand(rows, n, generator=g) < 0.3] = float("inf")
+        s[torch.rand(rows, n, generator=g) < 0.05] = float("nan")
     elif kind == "tiny":                                       # few halvings are left behind the way down; subnormal products
         s *= 1e-33
     return s
 
 
-@pytest.mark.parametrize("kind", ["within a few thousand floats", "16-bit values", "half zeros", "two far groups", "tiny", "log-normal"])
+@pytest.mark.parametrize("kind", ["within a few thousand floats", "16-bit values", "half zeros", "two far groups", "a third not finite", "tiny", "log-normal"])
 @pytest.mark.parametrize("rows,n", [(1, 513), (2, 8192 + 1), (33, 20000), (1, 150000)])
 def test_allocator_bit_exact_where_the_histogram_says_little(kind, rows, n):
     """The search's guess only saves time: rows it misses, rows whose open list does not fit LDS, rows of equal scores.  33 rows
@@ -331,25 +334,36 @@ def test_allocator_treats_an_error_that_is_not_a_number_as_never_below_another()
     assert torch.equal(*(optimal_scores_to_bits(s, LEVELS, 2.0, e, eviction_cost=0.5) for e in (first, lowest)))
 
 
+def _least_time(s, eps):
+    from kvquant.allocator import optimal_scores_to_bits
+    best = INF
+    for _ in range(6):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        optimal_scores_to_bits(s, LEVELS, 2.0, eps, eviction_cost=0.5)
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
 @pytest.mark.parametrize("errors", ["eviction forbidden", "infinite", "negative", "all negative"])
 def test_allocator_narrows_its_search_whatever_the_errors(errors):
     """A search that asks every score of a long row at every multiplier in one workgroup takes 35 to 60 times an ordinary call
     (measured, 262144 scores); with the few undecided ones alone it takes about as long as one: a factor of 8 lies between."""
-    from kvquant.allocator import optimal_scores_to_bits
     s = (torch.exp(2.0 * torch.randn(1, 262144, generator=torch.Generator().manual_seed(8))) * 1e-5).to(DEV)
+    assert _least_time(s, {**EPS, **ODD_ERRORS[errors]}) < 8.0 * _least_time(s, EPS)
 
-    def least(eps):
-        best = INF
-        for _ in range(6):
-            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            a.record()
-            optimal_scores_to_bits(s, LEVELS, 2.0, eps, eviction_cost=0.5)
-            b.record()
-            b.synchronize()
-            best = min(best, a.elapsed_time(b))
-        return best
 
-    assert least({**EPS, **ODD_ERRORS[errors]}) < 8.0 * least(EPS)
+def test_allocator_narrows_its_search_where_scores_are_not_finite():
+    """They stand for the largest finite score, and the search's guess has to count them there (measured: 22 times an ordinary call
+    where it took them for more than that)."""
+    g = torch.Generator().manual_seed(9)
+    s = torch.rand(1, 262144, generator=g)
+    odd = s.clone()
+    odd[torch.rand(1, 262144, generator=g) < 0.3] = INF
+    odd[torch.rand(1, 262144, generator=g) < 0.05] = float("nan")
+    assert _least_time(odd.to(DEV), EPS) < 8.0 * _least_time(s.to(DEV), EPS)
 
 
 @pytest.mark.parametrize("rows", [2048, 2049])
