@@ -60,13 +60,14 @@
 #define HB_BINS 1024                          // bin 0: zeros; the last: infinities and NaN; between them equal steps of the bit pattern
 #define MAX_TURN 2048                         // rows of a turn: what the histograms' workspace is cut for
 #define LAMBDA_CAP 100000008.0f               // the fp32 number behind the largest multiplier that is asked for, 1e8
+#define LAMBDA_LEAST 0x1p-66f                 // no multiplier that is asked for or returned is less: 64 halvings of 1 and the middle of what is left
 #define KEEP (1.0f - 0x1p-20f)                // one cost beats another by more than rounding: other * KEEP > best + slack()
 #define TINY 1e-36f
 
 struct RowState {
     double target, gap, lam;
     float la, lb;            // the window: the mean is above the budget at lambda <= la, within it at lambda >= lb
-    float wa, wb;            // [la, lb], stretched to any final multiplier outside it: what "open" is decided over
+    float wa, wb;            // [la, lb] above LAMBDA_LEAST, stretched to any final multiplier outside it: what "open" is decided over
     float grid[NGRID];       // the narrowing pass' multipliers, ascending
     int n_active;
     unsigned int max_finite; // bit pattern
@@ -407,7 +408,7 @@ __device__ static void carry_state(const AllocArgs& a, int row, RowState* cur, u
                 }
             }
             const float la = cur->la, lb = cur->lb;
-            cur->wa = la; cur->wb = lb;
+            cur->wa = fmaxf(la, LAMBDA_LEAST); cur->wb = lb; // (at 0 itself scores whose products are all below TINY would stay open)
             // After 27 halvings behind the first that moved the lower end the bracket is narrower than the gap of two fp32 numbers, and
             // the final multiplier lies in the window.  With fewer of them, or where no bracket reaches a mean within the budget, it
             // may lie beside it: between the two that the sequence ends at if the mean inside the window is above the budget
@@ -704,7 +705,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
     // A list that does not fit LDS (scores within a thousandth of each other, all different): after every third sum, an eighth of the bracket
     // later, the tokens that are settled by now are counted and the others closed up, chunk by chunk where they lie, until it fits.
     auto close_up = [&] {
-        const float from = fmaxf(la, known_above), to = known_within < 0.0f ? lb : fminf(lb, known_within);
+        const float from = fmaxf(cur.wa, known_above), to = known_within < 0.0f ? lb : fminf(lb, known_within);
         float c0[K], c1[K];
         int cnt[K];
 #pragma unroll
@@ -760,7 +761,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
         for (int k = 0; k < K; ++k) settled_sum += settled[k] * a.nominal[k];
         __syncthreads();
     };
-    const bool may_close = cur.wa == la && cur.wb == lb;     // (else the final multiplier may lie beside the window)
+    const bool may_close = cur.wa == fmaxf(la, LAMBDA_LEAST) && cur.wb == lb;     // (else the final multiplier may lie beside the window)
     const double lam = replay(lb, [&](float lambda) {            // (every thread runs it: the answers are the workgroup's)
         if (lambda <= la || lambda == known_above) return true;
         if (lambda >= lb || lambda == known_within) return false;

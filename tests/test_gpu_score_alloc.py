@@ -318,6 +318,7 @@ def test_allocator_bit_exact_with_infinite_and_negative_errors(errors, n, target
     g = torch.Generator().manual_seed(n)
     s = torch.exp(2.0 * torch.randn(1, n, generator=g)) * 1e-5
     _check_alloc_eps(s, target, {**EPS, **ODD_ERRORS[errors]})
+    _check_alloc_eps(s * 1e-32, target, {**EPS, **ODD_ERRORS[errors]})               # down to the subnormal numbers
     if errors == "eviction forbidden":                         # 0 * inf: a zero score takes the first level
         s[torch.rand(1, n, generator=g) < 0.3] = 0.0
         _check_alloc_eps(s, target, {**EPS, **ODD_ERRORS[errors]})
