@@ -278,7 +278,7 @@ def _awkward_scores(kind, rows, n, g):
 @pytest.mark.parametrize("kind", ["within a few thousand floats", "16-bit values", "half zeros", "two far groups", "a third not finite", "tiny", "log-normal"])
 @pytest.mark.parametrize("rows,n", [(1, 513), (2, 8192 + 1), (33, 20000), (1, 150000)])
 def test_allocator_bit_exact_where_the_histogram_says_little(kind, rows, n):
-    """The search's guess only saves time: rows it misses, rows whose open list does not fit LDS, rows of equal scores.  33 rows
+    """The search's guess only saves time: rows it misses, rows whose final multiplier lies beside the window (tiny), rows of equal scores.  33 rows
     of 20000 are cut into few, long chunks; a wave's ragged ends are at 513 and 8193."""
     from kvquant.allocator import optimal_scores_to_bits_batched
     g = torch.Generator().manual_seed(n + rows)
@@ -305,6 +305,42 @@ def _check_alloc_eps(scores, target, eps):
     from kvquant.allocator import optimal_scores_to_bits
     got = optimal_scores_to_bits(scores.to(DEV), LEVELS, target, eps, eviction_cost=0.5)
     assert torch.equal(got.cpu(), oal.optimal_scores_to_bits(scores, LEVELS, target, eps, None, eviction_cost=0.5))
+
+
+def _least_open_entries(s, lam):
+    """No fewer scores of a row than this stay undecided in the search's window, whatever the window is.  It holds the final multiplier, and
+    no two of the multipliers that may bound it are closer than 2 x 2^-18 of the guess (csrc/allocate.hip, the narrowing pass): 0.9 of that,
+    for their rounding.  The windows of that width around lam are covered by sixteen, each holding a stretch common to its neighbours; a
+    score that is undecided over such a stretch is undecided over all that hold it.  Equal scores of 64 neighbours may be one entry."""
+    eps = np.array([EPS[b] * (0.5 if b == 0 else 1.0) for b in LEVELS], np.float32)
+    bits = np.array(LEVELS, np.float32)
+    width, least = 0.9 * 2.0 ** -17, None
+    place = np.arange(s.size) // 64
+    for i in range(16):
+        ends, level, tied = (lam * (1 - width * i / 16), lam * (1 + width * (1 - (i + 1) / 16))), [], np.zeros(s.size, bool)
+        for end in ends:
+            cost = np.sort(s[None] * eps[:, None] + (np.float32(end) * bits)[:, None], axis=0)
+            level.append((s[None] * eps[:, None] + (np.float32(end) * bits)[:, None]).argmin(axis=0))
+            tied |= ~(cost[1] * np.float32(1 - 2.0 ** -20) > cost[0] + np.float32(1e-36))
+        open_ = tied | (level[0] != level[1])
+        n = len(set(zip(place[open_].tolist(), s[open_].tolist())))
+        least = n if least is None else min(least, n)
+    return least
+
+
+@pytest.mark.parametrize("n,target", [(600001, 2.0), (1048576, 3.0), (1048576, 1.5)])
+def test_allocator_closes_up_a_list_that_does_not_fit_lds(n, target):
+    """Scores within 1e-4 of each other: the list of undecided ones is longer than the 16384 that the replay keeps in LDS, and is closed up in
+    memory two or three times while the bracket narrows, over 196 chunks and over the most there are."""
+    from kvquant.allocator import optimal_scores_to_bits_batched
+    s = 0.3 + 3e-5 * torch.rand(1, n, generator=torch.Generator().manual_seed(n))
+    bits, counts, lam = optimal_scores_to_bits_batched(s.to(DEV), LEVELS, [target], EPS, eviction_cost=0.5, return_stats=True)
+    info = {}
+    want = oal.optimal_scores_to_bits(s, LEVELS, target, EPS, None, eviction_cost=0.5, info=info)
+    assert lam[0].item() == info["lam"] and torch.equal(bits.cpu(), want)
+    assert counts[0].tolist() == [(want == b).sum().item() for b in LEVELS]
+    assert 2.0 ** -36 < info["lam"] < 1e8                        # the final multiplier lies inside the window: the list may be closed up
+    assert _least_open_entries(s[0].numpy(), info["lam"]) > 16384
 
 
 INF = float("inf")
