@@ -97,7 +97,7 @@ struct AllocArgs {
     float* open;                   // [rows, n]: the open tokens' scores, a region per chunk
     uint8_t* open_n;               // [rows, n]: how many tokens an entry stands for
     unsigned long long* cand;      // [rows, n_cand, NLV, CAND_MAX]: per move of the repair
-    RowState* state;               // [3][rows]: the search and the finish leave third 2, the collecting pass third 1
+    RowState* state;               // [2][rows]: the search and the finish leave half 1, the collecting pass half 0
     int32_t* bits_out;
     int32_t* level_counts;
     double* lambda_out;
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(SE_THREADS) void alloc_search_kernel(AllocArgs a) {
         }
     }
     if (tid == 0) {
-        RowState& st = a.state[(size_t)2 * a.rows + row];
+        RowState& st = a.state[(size_t)a.rows + row];
         st.target = target; st.gap = 0.0; st.lam = 1.0;
         st.la = 0.0f; st.lb = LAMBDA_CAP;                    // nothing is known yet
         // the ends a little outside the bins' bounds, and three pairs around the guess: as far off as a bin is wide, an eighth and a 64th of it
@@ -374,7 +374,7 @@ __device__ static inline double replay(float lb, F above) {
 }
 
 // Start of a pass: the state before it in `cur` (shared memory) for the whole workgroup.  The collecting pass narrows the window by what the
-// narrowing one found, and the row's first workgroup writes the new state to third 1.  Ends with a barrier.
+// narrowing one found, and the row's first workgroup writes the new state to half 0.  Ends with a barrier.
 template <bool COLLECT>
 __device__ static void carry_state(const AllocArgs& a, int row, RowState* cur, unsigned int* tot) {
     const int tid = threadIdx.x;
@@ -384,7 +384,7 @@ __device__ static void carry_state(const AllocArgs& a, int row, RowState* cur, u
     const unsigned int* p = a.partial + (size_t)row * a.n_chunks * SLOTS;
 #pragma unroll
     for (int u = 0; u < 8; ++u) v0[u] = tid + u * EV_THREADS < n_part ? p[tid + u * EV_THREADS] : 0u;
-    if (tid == 0) *cur = a.state[(size_t)2 * a.rows + row];
+    if (tid == 0) *cur = a.state[(size_t)a.rows + row];
     if (tid < SLOTS) tot[tid] = 0u;
     __syncthreads();
     if constexpr (COLLECT) {
@@ -422,7 +422,7 @@ __device__ static void carry_state(const AllocArgs& a, int row, RowState* cur, u
             }
         }
         __syncthreads();
-        if (tid == 0 && blockIdx.x == 0) a.state[(size_t)a.rows + row] = *cur;
+        if (tid == 0 && blockIdx.x == 0) a.state[row] = *cur;
     }
 }
 
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
     __shared__ int settled[NLV], hist[NLV];
     __shared__ int red[2][FN_WAVES];
     const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const RowState* in = a.state + (size_t)a.rows + row;
+    const RowState* in = a.state + row;
     const unsigned int* part = a.partial + ((size_t)a.rows + row) * a.n_chunks * SLOTS;
     unsigned int v[EV_MAX_CHUNKS * SLOTS / FN_THREADS];
     const int n_part = a.n_chunks * SLOTS;
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
     if (tid <= EV_MAX_CHUNKS) at[tid] = 0;
     __syncthreads();
     if (cur.n_active == 0) {
-        if (tid == 0) a.state[(size_t)2 * a.rows + row] = cur;
+        if (tid == 0) a.state[(size_t)a.rows + row] = cur;
         return;
     }
 #pragma unroll
@@ -818,7 +818,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
         const double avg = (double)((float)S / nf);
         cur.gap = (avg - target) * (double)cur.n_active;
         cur.lam = lam;
-        a.state[(size_t)2 * a.rows + row] = cur;
+        a.state[(size_t)a.rows + row] = cur;
         if (a.lambda_out) a.lambda_out[row] = lam;
     }
 }
@@ -903,7 +903,7 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_assign_kernel(AllocArgs a) {
         on[e] = i < a.n && !is_sink(a, row, i);
         score[e] = on[e] ? a.scores[(size_t)row * a.n + i] : 0.0f;
     }
-    if (tid == 0) cur = a.state[(size_t)2 * a.rows + row];
+    if (tid == 0) cur = a.state[(size_t)a.rows + row];
     __syncthreads();
     const RowState& st = cur;
     const Cleaner clean(st);
@@ -1073,7 +1073,7 @@ __global__ __launch_bounds__(RB) void alloc_repair_kernel(AllocArgs a) {
     __shared__ int scratch[32];
     __shared__ unsigned long long wbest[RB / 64];
     const int row = blockIdx.x, tid = threadIdx.x;
-    const RowState& st = a.state[(size_t)2 * a.rows + row];
+    const RowState& st = a.state[(size_t)a.rows + row];
     if (st.n_active == 0) return;                            // (its counts are the cleared ones)
     if (a.level_counts && tid < a.K) a.level_counts[row * a.K + tid] = st.final_hist[tid];
     double gap = st.gap;
@@ -1145,7 +1145,7 @@ static AllocLayout alloc_layout(int rows, int n) {
     L.open = take((size_t)rows * n * sizeof(float));
     L.open_n = take((size_t)rows * n);
     L.cand = take((size_t)rows * chunks * NLV * CAND_MAX * sizeof(unsigned long long));
-    L.state = take((size_t)3 * rows * sizeof(RowState));
+    L.state = take((size_t)2 * rows * sizeof(RowState));
     L.total = off;
     return L;
 }

@@ -56,8 +56,8 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 #define PBUF (8 * PROW)     // one p buffer: 8 head rows
 
 // LDS of the main kernel: [table, later the combine area] [rotated query rows]
-// [p buffers] [per-wave scalars].  NW = wavefronts of the workgroup: 8 (short items: less set-up and a lighter combine),
-// 16 (long items: four wavefronts per SIMD keep its issue slots full) or 12 (three units in flight per wavefront).
+// [p buffers] [per-wave scalars].  NW = wavefronts of the workgroup: 8 (short items: less set-up and a lighter combine)
+// or 12 (three 2-bit units in flight per wavefront; the rule is worklist.cpp's).
 // One p buffer per wavefront (bf16 exact rows need a second one for the weights' low pieces: it lies in the table's
 // space, which an exact item does not use), so that eight wavefronts stay under half a compute unit's 160 KB.
 #define QROW_LDS 272                             // bytes of a query row in LDS: 128 x 16 bit + 16 (bank spread)
@@ -68,7 +68,7 @@ struct Lds {
     static constexpr int SCALARS = LDS_PBUFS + NW * PBUF;
     static constexpr int TOTAL = SCALARS + NW * 4 * 8 * 4 + 8 * 4;
     static_assert(NW * ODMKV_MAX_GROUP * HD * 4 <= LUT_BYTES, "combine area must fit the table's space");
-    static_assert(NW >= 8 && NW <= 16, "wave count (the first eight rotate the queries)");
+    static_assert(NW == 8 || NW == 12, "wave count (the first eight rotate the queries)");
     static_assert(TOTAL <= 160 * 1024, "LDS of one workgroup");
 };
 
@@ -992,6 +992,7 @@ __device__ static inline void run_exact_level(const DecodeArgs& a, int bh, int b
 template <int GP, bool ORDERED, int NW, bool G4 = false, bool CHAIN = false, bool PAIR = false>
 __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(DecodeArgs a) {
     static_assert(!G4 || (GP == 4 && (NW == 12 || PAIR)), "the shared-lane form is built for four heads");
+    static_assert(NW == 8 || G4 == (GP == 4), "twelve wavefronts take four heads in the shared-lane form");
     static_assert(!PAIR || (NW == 8 && 2 * Lds<NW>::TOTAL <= 160 * 1024), "two workgroups of eight wavefronts share a compute unit");
     static_assert(!CHAIN || ORDERED, "chains come with a dispatch order (fewer workgroups than items)");
     // one static LDS block: the table sits at LDS address 0 and that is known when the kernel is compiled, so a
@@ -1447,20 +1448,18 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
         hipEvent_t e0 = (hipEvent_t)ev_start, e1 = (hipEvent_t)ev_stop;
         const int nw = work->wavefronts >= 12 ? 12 : 8;
         int rc;
+        // (twelve wavefronts: groups of up to four heads run the form that shares the lanes out between a unit's two token blocks, whose
+        // softmax step costs half the instructions; larger groups fill the lanes as they are)
 #define ODMKV_LAUNCH_MAIN(GPV, ORD, CH) \
-        (nw == 12 ? launch_main<GPV, ORD, 12, false, CH>(a, grid, e0, e1, st) : launch_main<GPV, ORD, 8, false, CH>(a, grid, e0, e1, st))
+        (nw == 12 ? launch_main<GPV, ORD, 12, GPV == 4, CH>(a, grid, e0, e1, st) : launch_main<GPV, ORD, 8, false, CH>(a, grid, e0, e1, st))
         // Twelve wavefronts run what used to take sixteen: with 170 registers instead of 128 and the shared-lane form they are as fast
         // or faster on every shape (us a layer, 16 / 12: 32k tokens 32 heads over 8 14.50 / 14.20, 3 bits 16.70 / 16.25; 131k tokens
         // 23.6 / 23.6; 28 over 4 20.4 / 19.4; 4- and 8-bit levels at 131k in the general form of 12 24.6, in this one 24.4).
-        // groups of up to four heads on twelve wavefronts: the form that shares the lanes out between a unit's two token
-        // blocks (its softmax step costs half the instructions); ODMKV_DECODE_G4=0 selects the general form, for measurements
-        static const int g4_forced = [] { const char* e = getenv("ODMKV_DECODE_G4"); return e ? atoi(e) : -1; }();
-        const bool g4 = GP == 4 && nw == 12 && g4_forced != 0;
         const bool chain = work->n_workgroups > 0 && work->n_workgroups != n_items;      // workgroups that take several items
         const dim3 grid(chain ? work->n_workgroups : n_items, passes);
         // two eight-wavefront workgroups per compute unit (always with a dispatch order: the list has more items than
         // compute units); groups of up to four heads in the shared-lane form
-        const bool pair = work->two_per_cu != 0 && (GP == 8 || g4_forced != 0);
+        const bool pair = work->two_per_cu != 0;
         // a block of query tokens: several passes' workgroups in one launch run in rounds whatever the list, so they share
         // compute units too (an order is not needed: the passes even the rounds out).  Whole calls in the list's own form / in
         // pairs: 32k tokens, 32 heads over 8, bf16: 5 query tokens 41 / 33 us, 29: 165 / 122, 256: 1272 / 863; 28 over 4 at three
@@ -1471,11 +1470,8 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
                                                           : launch_main<4, true, 8, true, false, true>(a, grid, e0, e1, st);
         else if (pair) rc = chain ? launch_main<8, true, 8, false, true, true>(a, grid, e0, e1, st)
                                   : launch_main<8, true, 8, false, false, true>(a, grid, e0, e1, st);
-        else if (chain && g4) rc = launch_main<4, true, 12, true, true>(a, grid, e0, e1, st);
         else if (chain && GP == 4) rc = ODMKV_LAUNCH_MAIN(4, true, true);
         else if (chain) rc = ODMKV_LAUNCH_MAIN(8, true, true);
-        else if (g4 && !a.order) rc = launch_main<4, false, 12, true>(a, grid, e0, e1, st);
-        else if (g4) rc = launch_main<4, true, 12, true>(a, grid, e0, e1, st);
         else if (GP == 4 && !a.order) rc = ODMKV_LAUNCH_MAIN(4, false, false);
         else if (GP == 4) rc = ODMKV_LAUNCH_MAIN(4, true, false);
         else if (!a.order) rc = ODMKV_LAUNCH_MAIN(8, false, false);

@@ -278,8 +278,9 @@ static int worklist_cut(const int64_t* counts, const int64_t* seg_tile, int nseg
     shape->n_items = n; shape->ordered = ordered;
     shape->n_workgroups = chained ? n_heads : 0;
     shape->two_per_cu = paired;
-    // Wavefronts per item: eight for short items (less set-up, a lighter combine), twelve (16 says the same: long and narrow) for long
-    // ones.  Items of 6 to 15 tiles that are mostly 3 bits and wider: twelve as well, 2-3 % ahead of eight (measured on a 28-head, 3-bit
+    // Wavefronts per item: eight for short items (less set-up, a lighter combine), twelve for long ones (reported as 16 where they are
+    // narrow: callers of the cutter have read that number since sixteen ran; the kernel takes both for twelve).
+    // Items of 6 to 15 tiles that are mostly 3 bits and wider: twelve as well, 2-3 % ahead of eight (measured on a 28-head, 3-bit
     // store of 32k tokens: their loops wait on memory, and a third unit in flight pays).  Short items whose quantised tokens are
     // nearly all of 2 bits: twelve too, us a layer with eight / twelve: 600 tokens 10.83 / 10.64, 8192 11.60 / 11.35, 28 heads over 4
     // 11.77 / 11.59; with a quarter of 3 bits among them (8192 tokens at 2.25 bits) 12.02 / 12.24, at 3 bits 12.07 / 12.37.
