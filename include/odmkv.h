@@ -189,6 +189,8 @@ int odmkv_score_given(const void* K, const void* V, int dtype, int Hkv, int T, i
  * bits_out: device int32 [rows, n].
  * level_counts: device int32 [rows, n_levels] count of non-sink tokens per level, or NULL.
  * lambda_out: device fp64 [rows] the multiplier found, or NULL.
+ * The workspace is about 6 bytes a score (5 of them the list of undecided scores, 1 the repair's candidates) and 4 KB a row, for
+ * the first 2048 rows at most: a call of more rows runs in turns.
  */
 size_t odmkv_allocate_workspace_bytes(int rows, int n);
 int odmkv_allocate(const float* scores, int rows, int n,

@@ -20,7 +20,7 @@
 //   repair    (one workgroup a row) the moves.
 // What was 24 launches, ten of which walked all scores with fifteen multipliers each, is eight, and eight multipliers once.
 // us a call: 4096 scores 107 -> 53, 2 rows of 12432 107 -> 55, 4 of 262144 158 -> 69, one of 1048576 183 -> 80.
-// Every workgroup writes its partial sums with plain stores and is done.  The next launch begins,
+// Every workgroup writes its partial sums with plain stores and is done (the scan's alone add to the row's histogram by atomics).  The next launch begins,
 // in every workgroup, by adding up the row's partial sums of the launch before (a few hundred
 // numbers); the row's first workgroup also writes the new state down for the launch after.  Nothing waits on another workgroup
 // and the host is never consulted.  All sums are integers, so the result does not depend on the order
