@@ -6,6 +6,7 @@
 // the definition; the tile's own layout (what the decode kernel's matrix operands want, quant.h) is
 // produced and consumed by a re-layout through LDS.
 #include <algorithm>
+#include <type_traits>
 #include "quant.h"
 
 // ------------------------------------------------------------------------------------------------
@@ -905,7 +906,7 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
 // the chain itself, one lane per value, and replaces their codes in the packed tiles it has already
 // written.  Rows of zeros are exact either way.
 // Tiles the scheme does not cover go to the exact kernel through a list: 8-bit tiles (a tenth of
-// their values lie inside the band), tiles of a width whose table does not mirror around its middle, tiles with a row whose squared norm is not finite, and tiles
+// their values lie inside the band), tiles with a row whose squared norm is not finite, and tiles
 // with more listed values than the list has room for.
 //
 // Operands: for keys D = Pi (rows) x tokens (columns), so a lane ends with four consecutive outputs
@@ -985,6 +986,55 @@ template <int W> struct MirrorCoder {
         const uint32_t t = r & top;
         return ~(r ^ (t - (t >> (W - 1))));
     }
+    __device__ static __forceinline__ uint32_t finish(uint32_t r) { return r; }
+};
+// Any other table: a binary search, which meets both neighbours of y on its way, so the minimum over the thresholds it compares with is
+// the distance to the nearest.  finish() turns four codes, in fields of 4 bits, into the sign bits that the mirrored search would have collected.
+// us with the lowest centroid moved by 3e-3, by the exact kernel / by this search (the package's tables): prefill of 131k tokens of 8 heads, fp16,
+// 2 bits 1170 / 380 (345), 3 bits 1180 / 430 (400), 4 bits 1225 / 535 (450); 516096 rows outside a store, which the exact kernel takes in few
+// workgroups, 6400 / 90 (78), 6500 / 104 (96), 6600 / 115 (105).
+template <int W> struct SearchCoder {
+    static constexpr int K = 1 << W;
+    static constexpr uint32_t LOWEST = 0x1111u;
+    static constexpr int T = W == 4 ? 3 : K - 1;             // the thresholds of the first two steps (W = 4), or all of them
+    float t[T];
+    const float* thr;
+    __device__ inline SearchCoder(const float* thr_li) : thr(thr_li) {
+#pragma unroll
+        for (int k = 0; k < T; ++k) t[k] = thr_li[W == 4 ? 4 * k + 3 : k];
+    }
+    __device__ __forceinline__ uint32_t push(uint32_t r, float x, float scale, float& m) const {
+        const float y = x * scale;
+        if constexpr (W == 2) {
+            const bool b1 = y >= t[1];
+            const float ts = b1 ? t[2] : t[0];
+            m = fminf(fabsf(y - t[1]), fabsf(y - ts));
+            return (r << 2) | (b1 ? 2u : 0u) | (y >= ts ? 1u : 0u);
+        } else if constexpr (W == 3) {
+            const bool b2 = y >= t[3];
+            const float ta = b2 ? t[5] : t[1];
+            const bool b1 = y >= ta;
+            const float lo_pair = b1 ? t[2] : t[0], hi_pair = b1 ? t[6] : t[4];
+            const float tb = b2 ? hi_pair : lo_pair;
+            m = fminf(fminf(fabsf(y - t[3]), fabsf(y - ta)), fabsf(y - tb));
+            return (r << 3) | (b2 ? 4u : 0u) | (b1 ? 2u : 0u) | (y >= tb ? 1u : 0u);
+        } else {
+            const bool b3 = y >= t[1];
+            const float ta = b3 ? t[2] : t[0];
+            const bool b2 = y >= ta;
+            int pos = (b3 ? 8 : 0) + (b2 ? 4 : 0);
+            const float tb = thr[pos + 1];
+            pos += y >= tb ? 2 : 0;
+            const float tc = thr[pos];
+            pos += y >= tc ? 1 : 0;
+            m = fminf(fminf(fabsf(y - t[1]), fabsf(y - ta)), fminf(fabsf(y - tb), fabsf(y - tc)));
+            return (r << W) | (uint32_t)pos;
+        }
+    }
+    __device__ static __forceinline__ uint32_t finish(uint32_t g) {
+        const uint32_t t = ~g & (LOWEST << (W - 1));
+        return ~g ^ (t - (t >> (W - 1)));
+    }
 };
 // a staged word of W-bit codes in fields of S bits (2 or 4) -> codes
 template <int W, int S>
@@ -993,7 +1043,7 @@ __device__ static __forceinline__ uint32_t qf_decode(uint32_t x) {
     return MirrorCoder<W>::decode(x, ONES << (W - 1)) & (ONES * ((1u << W) - 1u));
 }
 
-// does the width's table mirror?  (a lane per pair of thresholds, all lanes get the answer)
+// does the width's table mirror?  (a lane per pair of thresholds, all lanes get the answer; the package's own tables do)
 template <int W>
 __device__ static inline bool qf_mirrors(const float* thr, int lane) {
     constexpr int H = (1 << (W - 1)) - 1;
@@ -1042,12 +1092,14 @@ __device__ static __forceinline__ float qf_sum_squares(const QfRows& x, uint32_t
 
 // Rotation estimate -> codes into the staging area: fields of W bits side by side (DIRECT), or of 4 bits where they have to be moved
 // one by one when they are stored (3 bits; tiles that hold tokens already), as sign bits, decoded then; values inside the band -> the wave's list, of the tokens of `listed` alone (rows of zeros: the estimate is the exact 0)
-template <int DT, int W, bool IS_V, bool DIRECT>
+template <int DT, int W, bool IS_V, bool DIRECT, bool MIRROR>
 __device__ static __forceinline__ void qf_code_tile(const QfRows& xb, const uint4* piA, const float* thr, QfWave& w,
                                                     uint8_t* stage, int lane, int gt, unsigned long long listed) {
     const int r16 = lane & 15, q = lane >> 4;
-    const MirrorCoder<W> code(thr);
-    constexpr float BAND = (DT == ODMKV_F16 ? QF_BAND : QF_BAND_BF16) + QF_MIRROR;
+    constexpr int S = DIRECT ? W : 4;                           // bits a code takes in the staging area
+    static_assert(MIRROR || !DIRECT, "the search leaves fields of 4 bits");
+    const std::conditional_t<MIRROR, MirrorCoder<W>, SearchCoder<W>> code(thr);
+    constexpr float BAND = (DT == ODMKV_F16 ? QF_BAND : QF_BAND_BF16) + (MIRROR ? QF_MIRROR : 0.0f);
     constexpr int NT = IS_V ? 16 : 4;
     float rinv[NT];
     uint32_t may = 0u;                                          // band flags that count, in f's order (below)
@@ -1092,7 +1144,7 @@ __device__ static __forceinline__ void qf_code_tile(const QfRows& xb, const uint
                     g = code.push(DIRECT ? g : g << (4 - W), acc[tb][r], scale, m);
                     f = __builtin_amdgcn_alignbit(f, __float_as_uint(m - BAND), 31);
                 }
-                constexpr int S = DIRECT ? W : 4;               // bits a code takes in the staging area
+                g = code.finish(g);
                 if constexpr (!IS_V) put_group<S>(stage + (16 * tb + r16) * Direct<S>::ROW_K + (4 * ob + q) * Direct<S>::GROUP_BYTES, g);
                 else put_group<S>(stage + (16 * ob + r16) * Direct<S>::ROW_V + (4 * tb + q) * Direct<S>::GROUP_BYTES, g);
             }
@@ -1372,7 +1424,9 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
         return lane >= d.lo && lane < d.hi ? a.s.pos[d.li][(size_t)d.tile * TILE + lane] : a.pos_offset;
     };
     const auto request = [&](const QfTile& d, int pos, QfRows& x) {
-        const int r16 = lane & 15, q = lane >> 4;
+        int ln = lane;                                          // opaque, as below
+        asm volatile("" : "+v"(ln));
+        const int r16 = ln & 15, q = ln >> 4;
 #pragma unroll
         for (int tb = 0; tb < 4; ++tb) {
             const int token = 16 * tb + r16;
@@ -1394,7 +1448,7 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
     }
     ready();
     if (!more) return;
-    const int mirrors = (qf_mirrors<2>(thrs, lane) ? 1 : 0) | (qf_mirrors<3>(thrs + thr_offset(1), lane) ? 2 : 0) | (qf_mirrors<4>(thrs + thr_offset(2), lane) ? 4 : 0);
+    const int mirrors = uniform((qf_mirrors<2>(thrs, lane) ? 1 : 0) | (qf_mirrors<3>(thrs + thr_offset(1), lane) ? 2 : 0) | (qf_mirrors<4>(thrs + thr_offset(2), lane) ? 4 : 0));
     int n_listed = 0;                                           // == w.count between tiles
     if (lane == 0) w.count = 0;
     while (true) {
@@ -1415,25 +1469,34 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
         bool odd = !(ss <= 3.4028234663852886e38f);              // a row with an infinite or NaN norm: exact kernel
         // bf16 reaches down to 1e-38: a row whose squares vanish or nearly do (but which is not all zeros) also goes there
         if constexpr (DT != ODMKV_F16) odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
-        const bool ok = !__any(odd) && ((mirrors >> cur.li) & 1);
+        const bool ok = !__any(odd);
         const float* thr = thrs + thr_offset(cur.li);
-        const bool direct = cur.li != 1 && cur.lo == 0 && (!IS_V || cur.hi == TILE);
+        const bool mirror = (mirrors >> cur.li) & 1;             // (another table's codes are staged in 4 bits each: three more coders instead of five)
+        const bool direct = mirror && cur.li != 1 && cur.lo == 0 && (!IS_V || cur.hi == TILE);
         const int variant = cur.li == 0 ? (direct ? 0 : 1) : cur.li == 1 ? 2 : (direct ? 3 : 4);
         const int n_before = n_listed;
         int n = 0;
         if (ok) {
             const float den = norm + 1e-10f;
-            w.off[lane] = off;
-            w.den[lane] = den;
-            w.rinv[lane] = 1.0f / den;
+            w.off[ln] = off;
+            w.den[ln] = den;
+            w.rinv[ln] = 1.0f / den;
             const unsigned long long listed = __ballot(valid && ss > 0.0f);
             wave_lds_fence();
-            switch (variant) {
-                case 0: qf_code_tile<DT, 2, IS_V, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
-                case 1: qf_code_tile<DT, 2, IS_V, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
-                case 2: qf_code_tile<DT, 3, IS_V, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
-                case 3: qf_code_tile<DT, 4, IS_V, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
-                default: qf_code_tile<DT, 4, IS_V, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+            if (__builtin_expect(!mirror, 0)) {
+                switch (cur.li) {
+                    case 0: qf_code_tile<DT, 2, IS_V, false, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                    case 1: qf_code_tile<DT, 3, IS_V, false, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                    default: qf_code_tile<DT, 4, IS_V, false, false>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                }
+            } else {
+                switch (variant) {
+                    case 0: qf_code_tile<DT, 2, IS_V, true, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                    case 1: qf_code_tile<DT, 2, IS_V, false, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                    case 2: qf_code_tile<DT, 3, IS_V, false, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                    case 3: qf_code_tile<DT, 4, IS_V, true, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                    default: qf_code_tile<DT, 4, IS_V, false, true>(xb, piA, thr, w, stage, ln, cur.gt, listed); break;
+                }
             }
             wave_lds_fence();
             n = w.count;
@@ -2397,7 +2460,7 @@ __device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* 
         const float norm = sqrtf(ss);
         bool odd = !(ss <= 3.4028234663852886e38f);              // as in qf_walk
         if constexpr (DT != ODMKV_F16) odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
-        const bool ok = !__any(odd) && mirror;
+        const bool ok = !__any(odd);
         const int n_before = n_listed;
         int n = 0;
         if (ok) {
@@ -2407,7 +2470,8 @@ __device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* 
             w.rinv[lane] = 1.0f / den;
             const unsigned long long listed = __ballot(valid && ss > 0.0f);
             wave_lds_fence();
-            qf_code_tile<DT, W, false, false>(xb, piA, thr, w, stage, ln, it, listed);
+            if (mirror) qf_code_tile<DT, W, false, false, true>(xb, piA, thr, w, stage, ln, it, listed);
+            else qf_code_tile<DT, W, false, false, false>(xb, piA, thr, w, stage, ln, it, listed);
             wave_lds_fence();
             n = w.count;
         }

@@ -377,27 +377,42 @@ def test_fp16_rows_next_to_thresholds_get_the_exact_codes(per_row, dtype):
     _check_store_against_oracle(st, ref)
 
 
+def _move_centroids(table, kind):
+    """A table of `kind`: the lowest centroid moved (a threshold moves by half), or the upper half drawn out."""
+    table = table.clone()
+    if kind == "upper half drawn out":
+        table[table > 0.02] *= 1.25
+    else:
+        table[0] -= kind
+    return table
+
+
+# thresholds up to 1e-6 from where their mirror images would have them are taken for mirrored: moves either side of that
+TABLES = [0.0, 2e-7, 1.6e-6, 3e-6, 3e-3, "upper half drawn out"]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("shift,covered", [(0.0, True), (2e-7, True), (3e-3, False)])
-def test_fp16_tables_that_do_not_mirror_go_to_the_exact_kernel(shift, covered, dtype):
-    """The matrix-core quantiser codes |y - middle| against half the thresholds, which needs a table that is the same on both
-    sides to within 1e-6; the lowest centroid moved by 2e-7 still is, by 3e-3 is not.  Ragged tiles, and an append onto them."""
+@pytest.mark.parametrize("kind", TABLES)
+def test_fp16_tables_that_mirror_and_tables_that_do_not(kind, dtype):
+    """The matrix-core quantiser codes |y - middle| against half the thresholds of a table that is the same on both
+    sides to within 1e-6, and searches any other; either way no tile goes to the exact kernel.  Ragged tiles, and an append onto them."""
     g = torch.Generator().manual_seed(3)
     B, H, T = 1, 2, 700
     k = torch.randn(B, H, T, 128, generator=g).to(dtype).to(DEV)
     v = torch.randn(B, H, T, 128, generator=g).to(dtype).to(DEV)
     bits = torch.tensor([2, 3, 4], dtype=torch.int32)[torch.randint(3, (B, H, T), generator=g)].to(DEV)
-    stores = []
+    stores, handed = [], []
     for x, y in ((k, v), (k.float(), v.float())):
         st = _state(dtype=dtype)
         st.codebooks = st.codebooks.clone()
-        for at in (0, 4, 12):                                  # the lowest centroid of 2, 3 and 4 bits
-            st.codebooks[at] -= shift
+        for first, n in ((0, 4), (4, 8), (12, 16)):            # the tables of 2, 3 and 4 bits
+            st.codebooks[first:first + n] = _move_centroids(st.codebooks[first:first + n], kind)
         st.prefill(x[:, :, :411], y[:, :, :411], bits[:, :, :411])
+        handed.append(_handed_over(st, B, H, 411))
         st.append(x[:, :, 411:], y[:, :, 411:], bits[:, :, 411:])
+        handed.append(_handed_over(st, B, H, T - 411))
         stores.append(st)
-    if covered:
-        assert _handed_over(stores[0], B, H, T - 411) == (0, 0)
+    assert handed[:2] == [(0, 0), (0, 0)]
     for li, w in enumerate((2, 3, 4)):
         first = stores[0]._seg_tile[li]
         used = torch.cat([torch.arange(int(first[h]), int(first[h]) + -(-int((bits[0, h] == w).sum()) // 64)) for h in range(H)]).to(DEV)

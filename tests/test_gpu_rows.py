@@ -33,6 +33,21 @@ def test_codes_of_16_bit_rows(n, bits, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("move", [2e-7, 1.6e-6, 3e-6, 3e-3, -0.1])
+def test_codes_of_16_bit_rows_by_tables_that_do_not_mirror(move, bits, dtype):
+    """Either side of the 1e-6 by which a threshold (it moves by half as much as a centroid) may be off its mirror image, and far."""
+    from kvquant.tq_backend import TurboQuantMSE, _pack_indices
+    x = _rows(33000, dtype, bits)
+    q = TurboQuantMSE(128, bits, device="cuda", dtype=dtype, seed=7)
+    q.centroids = q.centroids.clone()
+    q.centroids[0 if move < 0 else -1] += move
+    codes, _ = q.quantize_codes(x)
+    exact, _ = q.quantize_codes(x.float())
+    assert torch.equal(codes, exact) and torch.equal(q.quantize(x).indices, _pack_indices(exact, bits))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,H,T,lo,hi,bits", [(1, 1, 1, 0, 1, (3, 2)), (2, 3, 90, 17, 81, (2, 4)), (1, 8, 1300, 0, 1172, (3, 2)), (2, 2, 70, 0, 70, (8, 3))])
 def test_round_trip_in_place(B, H, T, lo, hi, bits, dtype):
     from kvquant import TurboQuantBackendPress
