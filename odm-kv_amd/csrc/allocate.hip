@@ -595,11 +595,15 @@ __global__ __launch_bounds__(EV_THREADS) void alloc_pass_kernel(AllocArgs a) {
 }
 
 // ---- the replay ----
-#define FN_THREADS 512                        // (two wavefronts a SIMD: sixteen got in the way of the replay's scalar steps)
-#define FN_WAVES (FN_THREADS / 64)
-#define FN_OPEN 16384                         // entries of the list kept in LDS; a longer one is read from memory every time
-template <int K>
+// FN_OPEN entries of the list are kept in LDS; a longer one is read from memory every time.  Up to a row a compute unit, a workgroup has eight
+// wavefronts (two a SIMD: sixteen got in the way of the replay's scalar steps) and room for 16384; 84 KB and 143 registers leave
+// a compute unit to one row at a time, so that a call of more rows takes four wavefronts and room for 4096 (23 KB), four rows and more at a time.  us a call,
+// eight wavefronts and 16384 / these: 300 rows of 128 scores 88 / 73, 1024 160 / 110, 4096 561 / 360 (two wavefronts and 2048: 324), 2048 of
+// 20000 692 / 598; lists beyond the room (512 rows of 20000 scores that are nearly equal) 851 / 837 (two and 2048: 880).
+#define FN_ROWS 256
+template <int K, int FN_THREADS, int FN_OPEN>
 __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
+    constexpr int FN_WAVES = FN_THREADS / 64;
     __shared__ RowState cur;
     __shared__ float open[FN_OPEN];
     __shared__ uint8_t open_n[FN_OPEN];
@@ -616,7 +620,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
     for (int u = 0; u < EV_MAX_CHUNKS * SLOTS / FN_THREADS; ++u) v[u] = tid + u * FN_THREADS < n_part ? part[tid + u * FN_THREADS] : 0u;
     if (tid == 0) cur = *in;
     if (tid < NLV) { settled[tid] = 0; hist[tid] = 0; }
-    if (tid <= EV_MAX_CHUNKS) at[tid] = 0;
+    for (int i = tid; i <= EV_MAX_CHUNKS; i += FN_THREADS) at[i] = 0;
     __syncthreads();
     if (cur.n_active == 0) {
         if (tid == 0) a.state[(size_t)a.rows + row] = cur;
@@ -750,7 +754,7 @@ __global__ __launch_bounds__(FN_THREADS) void alloc_finish_kernel(AllocArgs a) {
             if (lane == 0 && s) atomicAdd(&settled[k], s);
         }
         __syncthreads();                                     // everybody has read where its chunks began
-        if (tid < EV_MAX_CHUNKS) at[tid + 1] = tid < a.n_chunks ? left[tid] : 0;     // (the old sums behind the last chunk must not be summed again)
+        for (int i = tid; i < EV_MAX_CHUNKS; i += FN_THREADS) at[i + 1] = i < a.n_chunks ? left[i] : 0;     // (the old sums behind the last chunk must not be summed again)
         __syncthreads();
         running_sum();
         __syncthreads();
@@ -1166,7 +1170,8 @@ static int launch_search(const AllocArgs& a, int tpt, hipStream_t st) {
     if (tpt == 1) hipLaunchKernelGGL((alloc_pass_kernel<K, 1, true>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((alloc_pass_kernel<K, EV_BIG, true>), grid, block, 0, st, a);
     ODMKV_CHECK_LAUNCH("alloc_pass_kernel (collect)");
-    hipLaunchKernelGGL((alloc_finish_kernel<K>), dim3(a.rows), dim3(FN_THREADS), 0, st, a);
+    if (a.rows <= FN_ROWS) hipLaunchKernelGGL((alloc_finish_kernel<K, 512, 16384>), dim3(a.rows), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((alloc_finish_kernel<K, 256, 4096>), dim3(a.rows), dim3(256), 0, st, a);
     ODMKV_CHECK_LAUNCH("alloc_finish_kernel");
     hipLaunchKernelGGL((alloc_assign_kernel<K>), dim3(a.n_cand, a.rows), block, 0, st, a);
     ODMKV_CHECK_LAUNCH("alloc_assign_kernel");
