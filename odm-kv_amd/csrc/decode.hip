@@ -57,7 +57,7 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 
 // LDS of the main kernel: [table, later the combine area] [rotated query rows]
 // [p buffers] [per-wave scalars].  NW = wavefronts of the workgroup: 8 (short items: less set-up and a lighter combine)
-// or 12 (three 2-bit units in flight per wavefront; the rule is worklist.cpp's).
+// or 12 (the rule is worklist.cpp's).
 // One p buffer per wavefront (bf16 exact rows need a second one for the weights' low pieces: it lies in the table's
 // space, which an exact item does not use), so that eight wavefronts stay under half a compute unit's 160 KB.
 #define QROW_LDS 272                             // bytes of a query row in LDS: 128 x 16 bit + 16 (bank spread)
@@ -703,8 +703,8 @@ __device__ static inline void run_quant_level(const DecodeArgs& a, int li, int b
     // microsecond later).  Loads return in issue order: the (small) query goes first.
     RotQuery rq;
     if (first) request_rot_query(rq, a, bq_first, tid);
-    // DEPTH units of this wavefront are under way at any time: two (one for the widest rows: registers); twelve
-    // wavefronts have the registers for a third 2-bit unit.  (Six units in flight with eight wavefronts were measured:
+    // DEPTH units of this wavefront are under way at any time: two (one for the widest rows: registers); groups of
+    // five to eight heads on twelve wavefronts have the registers for a third 2-bit unit.  (Six units in flight with eight wavefronts were measured:
     // no gain, the eight are bound by their arithmetic.)
     constexpr int DEPTH = W == 8 ? 1 : (NW == 12 && W == 2) ? 3 : 2;
     if constexpr (DEPTH <= 2) {

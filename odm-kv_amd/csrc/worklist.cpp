@@ -278,10 +278,9 @@ static int worklist_cut(const int64_t* counts, const int64_t* seg_tile, int nseg
     shape->n_items = n; shape->ordered = ordered;
     shape->n_workgroups = chained ? n_heads : 0;
     shape->two_per_cu = paired;
-    // Wavefronts per item: eight for short items (less set-up, a lighter combine), twelve for long ones (reported as 16 where they are
-    // narrow: callers of the cutter have read that number since sixteen ran; the kernel takes both for twelve).
+    // Wavefronts per item: eight for short items (less set-up, a lighter combine), twelve for long ones.
     // Items of 6 to 15 tiles that are mostly 3 bits and wider: twelve as well, 2-3 % ahead of eight (measured on a 28-head, 3-bit
-    // store of 32k tokens: their loops wait on memory, and a third unit in flight pays).  Short items whose quantised tokens are
+    // store of 32k tokens: their loops wait on memory, and a third wavefront a SIMD pays).  Short items whose quantised tokens are
     // nearly all of 2 bits: twelve too, us a layer with eight / twelve: 600 tokens 10.83 / 10.64, 8192 11.60 / 11.35, 28 heads over 4
     // 11.77 / 11.59; with a quarter of 3 bits among them (8192 tokens at 2.25 bits) 12.02 / 12.24, at 3 bits 12.07 / 12.37.
     double q_tiles = 0.0;
@@ -297,10 +296,9 @@ static int worklist_cut(const int64_t* counts, const int64_t* seg_tile, int nseg
     const double mean = q_groups ? q_tiles / (double)q_groups : 0.0;
     const int64_t q_all = q_bytes[0] + q_bytes[1] + q_bytes[2] + q_bytes[3];
     const double q_floor = (double)std::max<int64_t>(q_all, 1);
-    const bool wide = (double)(q_bytes[2] + q_bytes[3]) >= 0.4 * q_floor;
-    const bool medium = q_groups && mean >= 6 && mean < 16 && (double)(q_all - q_bytes[0]) >= 0.5 * q_floor;
-    const bool narrow = q_groups && (double)q_bytes[0] >= 0.9 * q_floor;
-    const int automatic = !(q_groups && mean >= 16) ? (medium || narrow ? 12 : 8) : wide ? 12 : 16;
+    const bool medium = mean >= 6 && (double)(q_all - q_bytes[0]) >= 0.5 * q_floor;
+    const bool narrow = (double)q_bytes[0] >= 0.9 * q_floor;
+    const int automatic = q_groups && (mean >= 16 || medium || narrow) ? 12 : 8;
     shape->wavefronts = paired ? 8 : waves > 0 ? waves : automatic;
     if (capacity < shape->need) {
         odmkv_set_error("odmkv_worklist_cut: the table needs %llu integers, %llu given", (unsigned long long)shape->need, (unsigned long long)capacity);

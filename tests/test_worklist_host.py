@@ -76,7 +76,7 @@ def test_one_long_sequence_gets_an_item_per_compute_unit():
     st._build_items()
     items, heads = _check(st)
     w = st._worklist
-    assert 200 <= len(items) <= 256 and w.two_per_cu == 0 and w.n_workgroups == 0 and w.wavefronts == 16
+    assert 200 <= len(items) <= 256 and w.two_per_cu == 0 and w.n_workgroups == 0 and w.wavefronts == 12
 
 
 def test_a_batch_with_two_levels_a_pair_runs_two_workgroups_per_compute_unit():
