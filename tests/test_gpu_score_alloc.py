@@ -580,6 +580,30 @@ def test_window_attention_at_the_edges_of_its_workgroups(T, W, n_sink):
         np.testing.assert_allclose(both.cpu().numpy(), apart.cpu().numpy(), rtol=2e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hkv,hq,T,W,data", [
+    (2, 2, 300, 20, "plain"), (2, 2, 131, 48, "plain"), (2, 4, 389, 50, "plain"),      # 1, 2 and 4 blocks of 32 queries: 8, 4 and 2 shares of the tokens
+    (1, 5, 260, 60, "plain"),                                                           # 300 queries: a second turn of the wavefronts over the same tokens
+    (1, 5, 98400, 60, "plain"),                                                         # the same over a tile of 256 tokens
+    (8, 8, 8448, 33, "plain"), (8, 24, 8321, 64, "rising"),                              # two tiles of 128 a workgroup, the last one short
+    (2, 8, 1030, 64, "rising"), (2, 8, 1030, 64, "negative")])
+def test_window_attention_over_its_ways_of_sharing_the_work(hkv, hq, T, W, data, dtype):
+    """Rising: every token's logits lie above those before it, so that the statistics' reference point moves again and again; negative:
+    no logit is positive.  Sums of at most 2^17 terms in fp32, exponents to 2^-22: 1e-5."""
+    from kvquant.scorer import _launch_window_attention
+    g = torch.Generator().manual_seed(T + W)
+    k = torch.randn(hkv, T, 128, generator=g)
+    q = torch.randn(hq, W, 128, generator=g) * 1.5
+    if data != "plain":
+        k = k * 0.1 + torch.ones(128) * (torch.linspace(0.0, 3.0, T)[:, None] if data == "rising" else -2.0)
+        q = q * 0.1 + 1.0
+    k, q = k.to(dtype), q.to(dtype)
+    want = osc.window_attention(k.double(), q.double(), 4, T - W)[0]
+    got = _launch_window_attention(k.to(DEV), q.to(DEV), 4, T - W, 128 ** -0.5)
+    err = (got.cpu().double() - want).norm() / want.norm()
+    assert err < 1e-5, float(err)
+
+
 def test_window_attention_rejects_fp32_keys():
     from kvquant.scorer import _launch_window_attention
     k = torch.randn(1, 64, 128, device=DEV)
