@@ -1164,7 +1164,8 @@ __device__ static __forceinline__ void qf_code_tile(const QfRows& xb, const uint
 }
 
 // the definition's own value: the row's quotients times Pi's row, one fused multiply-add after the other
-template <int DT>
+// (HALVES: Pi's row in two halves, where the registers of a whole one are needed for something else)
+template <int DT, bool HALVES = false>
 __device__ static __forceinline__ float qf_chain(const RowRegs<DT>& x, const float4* __restrict__ prow, float den) {
     float y = 0.0f;
     bool row_plain = !(den >= 9.094947017729282e-13f && den <= 1.152921504606847e18f);
@@ -1183,6 +1184,7 @@ __device__ static __forceinline__ float qf_chain(const RowRegs<DT>& x, const flo
         const float nden = -den;
 #pragma unroll
         for (int c = 0; c < HD / 4; ++c) {
+            if (HALVES && c % 8 == 0) __builtin_amdgcn_sched_barrier(0);
             const float4 p = prow[c];
             const float pv[4] = {p.x, p.y, p.z, p.w};
 #pragma unroll
@@ -1197,6 +1199,7 @@ __device__ static __forceinline__ float qf_chain(const RowRegs<DT>& x, const flo
     } else {
 #pragma unroll
         for (int c = 0; c < HD / 4; ++c) {
+            if (HALVES && c % 4 == 0) __builtin_amdgcn_sched_barrier(0);
             const float4 p = prow[c];
             const float pv[4] = {p.x, p.y, p.z, p.w};
 #pragma unroll
@@ -2389,10 +2392,9 @@ extern "C" int odmkv_dequant_from(const odmkv_packed_t* store, void* K, void* V,
 
 // ------------------------------------------------------------------------------------------------
 // rows outside the store on the matrix cores: the 16-bit quantiser's estimate with the codes as bytes or in the reference's
-// container, and the dequantiser from byte codes.  Workgroups of the even index take job 0, of the odd one job 1 (keys and
-// values of a layer in one launch), a wave a tile of 64 rows.  A row per lane without them took 150 us for 64512 rows (the
-// fused multiply-adds of the rotation on the vector ALU); here keys and values of 64512 rows each are quantised in 29 us and
-// dequantised in 20 us.
+// container, the dequantiser from byte codes, and both in one pass.  Where there are two jobs (keys and values of a layer in one launch), workgroups of
+// the even index take job 0, of the odd one job 1; a wave takes a tile of 64 rows.  A row per lane without them took 150 us for 64512 rows (the
+// fused multiply-adds of the rotation on the vector ALU).
 // ------------------------------------------------------------------------------------------------
 struct RowsArgs { RowsJob job[2]; int n_jobs; };
 
@@ -2528,11 +2530,10 @@ __device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* 
 }
 
 template <int DT>
-__global__ __launch_bounds__(QF_NW * 64) void quant_rows_f16_kernel(RowsArgs a) {
+__global__ __launch_bounds__(QF_NW * 64) void quant_rows_f16_kernel(RowsJob j) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const RowsJob& j = a.job[a.n_jobs == 2 ? (blockIdx.x & 1) : 0];
     float* thr = reinterpret_cast<float*>(smem + QF_PI_BYTES + QF_NW * QF_STAGE);
     uint8_t* stage = smem + QF_PI_BYTES + wave * QF_STAGE;
     QfWave& w = reinterpret_cast<QfWave*>(smem + QF_PI_BYTES + QF_NW * QF_STAGE + QF_THR_BYTES)[wave];
@@ -2546,7 +2547,7 @@ __global__ __launch_bounds__(QF_NW * 64) void quant_rows_f16_kernel(RowsArgs a) 
         __syncthreads();
     };
     const uint4* piA = reinterpret_cast<const uint4*>(smem);
-    const long long first = (long long)wave * (gridDim.x / a.n_jobs) + blockIdx.x / a.n_jobs, stride = (long long)(gridDim.x / a.n_jobs) * QF_NW;
+    const long long first = (long long)wave * gridDim.x + blockIdx.x, stride = (long long)gridDim.x * QF_NW;
     switch (j.bits) {
         case 2: qr_walk<DT, 2>(j, piA, thr, w, stage, lane, first, stride, ready); break;
         case 3: qr_walk<DT, 3>(j, piA, thr, w, stage, lane, first, stride, ready); break;
@@ -2572,7 +2573,7 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a
     long long* offs = reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + wave * TILE;
     float rotation[8 * DQ_PI_GROUPS];
     dq_request_rotation(j.pi, rotation, tid);
-    const float centroid = tid < (1 << j.bits) ? j.cb[tid] : 0.0f;                 // (16 at most: the launch takes 2, 3 and 4 bits)
+    const float centroid = tid < (1 << j.bits) ? j.cb[tid] : 0.0f;                 // (256 at most)
     const long long tiles = (j.n + TILE - 1) / TILE, n_wg = gridDim.x / a.n_jobs, stride = n_wg * DQ_NW;
     uint4 raw[8];
     float norm = 0.0f;
@@ -2612,16 +2613,344 @@ static dim3 rows_grid(const RowsJob* jobs, int n_jobs, int waves) {
     return dim3((unsigned)(n_jobs * std::max<long long>(1, std::min<long long>(most, compute_units() / n_jobs))));
 }
 
-int launch_quantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
-    const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QF_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave);
-    if (dtype == ODMKV_F16) ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_F16>, lds);
-    else ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_BF16>, lds);
+// ------------------------------------------------------------------------------------------------
+// rows quantised and dequantised where they lie: the quantiser's estimate and the dequantiser's products one behind the other, the codes in registers.
+// The estimate leaves lane 16 q + r with outputs 16 ob + 4 q .. + 3 of token 16 tb + r, and what a matrix instruction contracts over may come in any
+// order that both operands share: the outputs of two blocks are the eight steps that the lane supplies to the second product, whose other operand is
+// Pi^T laid out in that order.  A pair of codes is looked up at a time, in the form the comparisons leave it (their sign bits).
+// What bounds it: a tile a wavefront for 8k tokens of 8 heads, so that the rows' way from memory, 256 + 384 matrix instructions and the chain of the listed
+// values between them come one behind the other.  us for keys and values of
+// 8064 tokens of 8 heads: 27.6 + 4.6 (the look for tiles left over) + 20.9 -> 40.7, of it 9 until the rows are there, 8 the estimate, 5 the listed values, 7 the
+// second product (the matrix cores' own 6.5); 600 tokens 35 -> 22 a call, 16384 of 24 heads 180 -> 146; rows of infinities, which the exact quantiser
+// took in few workgroups, 6500 -> 740.
+// ------------------------------------------------------------------------------------------------
+#define RT_NW 8
+// a barrier for LDS alone (__syncthreads waits for every load under way)
+__device__ static inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+struct RtWave {                          // per-wave scratch in LDS
+    long long off[TILE];                 // element offset of the token's row
+    float den[TILE], rinv[TILE], norm[TILE];
+    uint32_t list[QF_LIST];              // slot in the tile | output << 6
+    int count, pad[3];
+};
+// LDS: Pi in the estimate's order (hi, lo) | Pi^T in the second product's (hi, lo) | pairs of centroids | thresholds | per-wave scratch
+#define RT_PAIRS 256
+#define RT_THR_BYTES 64
+#define RT_LDS (2 * QF_PI_BYTES + RT_PAIRS * 8 + RT_THR_BYTES + RT_NW * sizeof(RtWave))
+typedef uint32_t RtCodes[4][4];          // [tb][s]: the codes of outputs 32 s + 4 q .. + 3 in the lower half, of 32 s + 16 + 4 q .. + 3 in the upper, W bits each
+
+// a code in the form that the comparisons leave (MirrorCoder: their sign bits)
+template <int W>
+__device__ static inline uint32_t rt_raw(uint32_t code, bool mirror) {
+    constexpr uint32_t M = (1u << W) - 1u, TOP = 1u << (W - 1);
+    const uint32_t n = ~code & M, t = n & TOP;
+    return mirror ? n ^ (t - (t >> (W - 1))) : code;
+}
+
+// Pi^T as A operands, hi then lo, times 2^DQ_UP: lane 16 q + r of block (jb, s) holds Pi[i][j] of i = 32 s + 4 q + e (e < 4) and 32 s + 16 + 4 q + e - 4, of
+// the output j = 32 (jb >> 1) + 8 (r >> 2) + 4 (jb & 1) + (r & 3) (dq_lay_out_rotation)
+__device__ static __forceinline__ void rt_request_rotation(const float* __restrict__ pi, float (&p)[8 * DQ_PI_GROUPS], int tid) {
+#pragma unroll
+    for (int k = 0; k < DQ_PI_GROUPS; ++k) {
+        const int g = tid + k * (RT_NW * 64), j = g & (HD - 1), sq = g / HD, i = 32 * (sq >> 2) + 4 * (sq & 3);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[8 * k + e] = pi[(i + (e & 3) + 16 * (e >> 2)) * HD + j];
+    }
+}
+
+// the estimate's codes of a tile; values inside the band -> the wave's list (qf_code_tile)
+template <int DT, int W, bool MIRROR>
+__device__ static __forceinline__ void rt_code_tile(const QfRows& xb, const uint4* piA, const float* thr, RtWave& w, int lane, unsigned long long listed, RtCodes& g) {
+    const int r16 = lane & 15, q = lane >> 4;
+    const std::conditional_t<MIRROR, MirrorCoder<W>, SearchCoder<W>> code(thr);
+    constexpr float BAND = (DT == ODMKV_F16 ? QF_BAND : QF_BAND_BF16) + (MIRROR ? QF_MIRROR : 0.0f);
+    float rinv[4];
+    uint32_t may = 0u;                                          // band flags that count, in f's order (below)
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        rinv[tb] = w.rinv[16 * tb + r16];
+        may |= ((listed >> (16 * tb + r16)) & 1ull) ? 15u << (28 - 4 * tb) : 0u;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) g[tb][s] = 0u;
+    }
+    may |= may >> 16;
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+        uint32_t f = 0u;                                        // band flags of this pair of output blocks, first value on top
+#pragma unroll
+        for (int o2 = 0; o2 < 2; ++o2) {
+            const int ob = 2 * k + o2;
+            qf_f4 acc[4];
+#pragma unroll
+            for (int tb = 0; tb < 4; ++tb) acc[tb] = (qf_f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int ch = 0; ch < 4; ++ch) {
+                const uint4 ah = piA[(ob * 4 + ch) * 64 + lane];
+                const uint4 al = piA[HD * HD / 8 + (ob * 4 + ch) * 64 + lane];
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[tb] = qf_mfma<DT>(ah, xb[tb][ch], acc[tb]);
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[tb] = qf_mfma<DT>(al, xb[tb][ch], acc[tb]);
+            }
+#pragma unroll
+            for (int tb = 0; tb < 4; ++tb) {
+                uint32_t c = 0u;
+#pragma unroll
+                for (int r = 3; r >= 0; --r) {
+                    float m;
+                    c = code.push(c, acc[tb][r], rinv[tb], m);
+                    f = __builtin_amdgcn_alignbit(f, __float_as_uint(m - BAND), 31);
+                }
+#pragma unroll
+                for (int s = 0; s < 4; ++s) g[tb][s] |= s == k ? c << (16 * o2) : 0u;       // (k is in a scalar register)
+            }
+        }
+        f &= may;
+        while (f) {                                             // rare: a few values per lane and tile
+            const int b = 31 - __clz(f);
+            f &= ~(1u << b);
+            const int v = 31 - b;                               // v = o2*16 + tb*4 + (3 - r)
+            const int idx = atomicAdd(&w.count, 1);
+            if (idx < QF_LIST) w.list[idx] = (uint32_t)(16 * ((v >> 2) & 3) + r16) | ((uint32_t)(16 * (2 * k + (v >> 4)) + 4 * q + 3 - (v & 3)) << 6);
+        }
+    }
+}
+
+// the definition's own code of (token, out) of the tile at hand
+template <int DT, int W>
+__device__ static __forceinline__ uint32_t rt_chain_code(const RowsJob& j, const float* thr, const RtWave& w, int token, int out) {
+    RowRegs<DT> x;
+    x.load(j.x, (size_t)w.off[token]);
+    const float y = qf_chain<DT, true>(x, reinterpret_cast<const float4*>(j.pi + out * HD), w.den[token]);
+    int code = 0;
+#pragma unroll
+    for (int st = (1 << W) / 2; st >= 1; st >>= 1)
+        if (y >= thr[code + st - 1]) code += st;
+    return (uint32_t)code;
+}
+
+// a tile's rows as matrix operands; off: the element offset of the lane's own row, found once and handed round
+__device__ static __forceinline__ void rt_request(const RowsJob& j, long long tile, long long& off, QfRows& x) {
+    int lane = threadIdx.x & 63;                                // opaque, as in rt_walk
+    asm volatile("" : "+v"(lane));
+    const int r16 = lane & 15, q = lane >> 4;
+    const long long r = tile * TILE + lane;
+    const int rows = (int)min((long long)TILE, j.n - tile * TILE);
+    off = r < j.n ? row_offset(j, r) : 0;
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+        const int token = 16 * tb + r16;
+        const uint32_t lo = __shfl((uint32_t)off, token, WAVE), hi = __shfl((uint32_t)(off >> 32), token, WAVE);
+        const uint4* row = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(j.x) + (long long)(((unsigned long long)hi << 32) | lo)) + q;
+        const bool on = token < rows;
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch) x[tb][ch] = on ? row[4 * ch] : make_uint4(0u, 0u, 0u, 0u);
+    }
+}
+
+template <int DT, int W, typename F>
+__device__ static __forceinline__ void rt_walk(const RowsJob& j, const uint4* piA, const uint4* piB, const uint2* pairs, const float* thr, RtWave& w, int lane0,
+                               long long tile0, long long stride, const uint32_t (&touched)[2], F ready) {
+    const long long tiles = (j.n + TILE - 1) / TILE;
+    const bool mirror = ready(qf_mirrors<W>(thr, lane0));
+#pragma unroll 1
+    for (long long tile = tile0; tile < tiles; tile += stride) {
+        long long off;
+        QfRows xb;
+        rt_request(j, tile, off, xb);
+        asm volatile("" ::"v"(touched[0]), "v"(touched[1]));      // (their registers are theirs until they have come)
+        int lane = lane0;                                       // opaque: what follows from it is worked out in a tile's phases, not carried round the loop
+        asm volatile("" : "+v"(lane));
+        const int r16 = lane & 15, q = lane >> 4;
+        const int rows = (int)min((long long)TILE, j.n - tile * TILE);
+        uint32_t any;
+        const float ss = qf_sum_squares<DT>(xb, any);
+        const float norm = sqrtf(ss), den = norm + 1e-10f;
+        bool odd = !(ss <= 3.4028234663852886e38f);              // as in qf_walk
+        if constexpr (DT != ODMKV_F16) odd = odd || ((any & 0x7fff7fffu) != 0u && ss < 1e-30f);
+        const bool ok = !__any(odd);
+        w.off[lane] = off;
+        w.den[lane] = den;
+        w.rinv[lane] = 1.0f / den;
+        w.norm[lane] = norm;
+        if (lane == 0) w.count = 0;
+        const unsigned long long listed = __ballot(lane < rows && ss > 0.0f);
+        wave_lds_fence();
+        RtCodes g;
+        int n = QF_LIST + 1;
+        if (ok) {
+            if (mirror) rt_code_tile<DT, W, true>(xb, piA, thr, w, lane, listed, g);
+            else rt_code_tile<DT, W, false>(xb, piA, thr, w, lane, listed, g);
+            wave_lds_fence();
+            n = uniform(w.count);
+        }
+        if (n <= QF_LIST) {
+#pragma unroll 1
+            for (int first = 0; first < n; first += WAVE) {     // 64 listed values at a time, a lane each, by the definition
+                const bool on = first + lane < n;
+                const uint32_t e = w.list[on ? first + lane : first];
+                const int token = e & 63, out = (e >> 6) & 127;
+                const uint32_t raw = rt_raw<W>(rt_chain_code<DT, W>(j, thr, w, token, out), mirror);
+                // the estimate's, out of the register of the lane that holds it
+                const int owner = 16 * ((out >> 2) & 3) + (token & 15), at = 4 * (token >> 4) + (out >> 5), sh = 16 * ((out >> 4) & 1) + W * (out & 3);
+                uint32_t word = 0u;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const uint32_t v = __shfl(g[i >> 2][i & 3], owner, WAVE);
+                    word = i == at ? v : word;
+                }
+                const uint32_t diff = ((word >> sh) & ((1u << W) - 1u)) ^ raw;
+                unsigned long long off_by = __ballot(on && diff != 0u);
+                while (off_by) {                                // (a value in millions)
+                    const int l = __builtin_ctzll(off_by);
+                    off_by &= off_by - 1ull;
+                    const int to = __builtin_amdgcn_readlane(owner, l), which = __builtin_amdgcn_readlane(at, l);
+                    const uint32_t flip = (uint32_t)__builtin_amdgcn_readlane((int)(diff << sh), l);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) g[i >> 2][i & 3] ^= i == which && lane == to ? flip : 0u;
+                }
+            }
+        } else {
+            // A row the estimate does not cover, or more listed values than there is room for: every value of the tile by the definition, a token
+            // a lane, one output after the other.
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) g[tb][s] = 0u;
+#pragma unroll 1
+                for (int o = 0; o < 32; ++o) {
+                    const int out = 32 * s + o;
+                    const uint32_t raw = rt_raw<W>(rt_chain_code<DT, W>(j, thr, w, lane, out), mirror) << (16 * (o >> 4) + W * (o & 3));
+#pragma unroll
+                    for (int tb = 0; tb < 4; ++tb) {
+                        const uint32_t v = __shfl(raw, 16 * tb + r16, WAVE);
+                        g[tb][s] |= q == ((o >> 2) & 3) ? v : 0u;
+                    }
+                }
+            }
+        }
+        // the second product (dq_tile)
+        __builtin_amdgcn_sched_barrier(0);
+        uint4 bh[4][4], bl[4][4];
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const uint32_t v = g[tb][s];
+                constexpr uint32_t M = (1u << (2 * W)) - 1u;
+                const uint2 c0 = pairs[v & M], c1 = pairs[(v >> (2 * W)) & M], c2 = pairs[(v >> 16) & M], c3 = pairs[(v >> (16 + 2 * W)) & M];
+                bh[tb][s] = make_uint4(c0.x, c1.x, c2.x, c3.x);
+                bl[tb][s] = make_uint4(c0.y, c1.y, c2.y, c3.y);
+            }
+#pragma unroll 1
+        for (int jp = 0; jp < 4; ++jp) {                         // outputs 32 jp .. + 31
+            qf_f4 acc[2][4];
+#pragma unroll
+            for (int o2 = 0; o2 < 2; ++o2)
+#pragma unroll
+                for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = (qf_f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int o2 = 0; o2 < 2; ++o2)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const uint4 ah = piB[((2 * jp + o2) * 4 + s) * 64 + lane];
+                    const uint4 al = piB[HD * HD / 8 + ((2 * jp + o2) * 4 + s) * 64 + lane];
+#pragma unroll
+                    for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = qf_mfma<ODMKV_F16>(ah, bh[tb][s], acc[o2][tb]);
+#pragma unroll
+                    for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = qf_mfma<ODMKV_F16>(al, bh[tb][s], acc[o2][tb]);
+#pragma unroll
+                    for (int tb = 0; tb < 4; ++tb) acc[o2][tb] = qf_mfma<ODMKV_F16>(ah, bl[tb][s], acc[o2][tb]);
+                }
+#pragma unroll
+            for (int tb = 0; tb < 4; ++tb) {
+                const int token = 16 * tb + r16;
+                const float nrm = w.norm[token];
+                if (token < rows) {                              // outputs 32 jp + 8 q .. + 7 of the token
+                    float r[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) r[e] = acc[e >> 2][tb][e & 3] * (1.0f / (1 << DQ_UP) / (1 << DQ_UP)) * nrm;      // (an exact power of two)
+                    store8<DT>(j.out, (size_t)w.off[token] + 32 * jp + 8 * q, r);
+                }
+            }
+        }
+        wave_lds_fence();                                        // the scratch is free for the next tile
+    }
+}
+
+template <int DT>
+__global__ __launch_bounds__(RT_NW * 64) void round_trip_rows_kernel(RowsArgs a) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    static_assert(RT_NW == QF_NW && RT_NW == DQ_NW, "the rotations are laid out by as many threads");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const RowsJob& j = a.job[a.n_jobs == 2 ? (blockIdx.x & 1) : 0];
+    uint2* pairs = reinterpret_cast<uint2*>(smem + 2 * QF_PI_BYTES);
+    float* thr = reinterpret_cast<float*>(smem + 2 * QF_PI_BYTES + RT_PAIRS * 8);
+    RtWave& w = reinterpret_cast<RtWave*>(smem + 2 * QF_PI_BYTES + RT_PAIRS * 8 + RT_THR_BYTES)[wave];
+    float4 rotation[QF_PI_READS];
+    float back[8 * DQ_PI_GROUPS];
+    qf_request_rotation(j.pi, rotation, tid);
+    rt_request_rotation(j.pi, back, tid);
+    const int n_cb = 1 << j.bits, mask = n_cb - 1;
+    const bool has_thr = tid < n_cb - 1;
+    const float c_lo = has_thr ? j.cb[tid] : 0.0f, c_hi = has_thr ? j.cb[tid + 1] : 0.0f;
+    // a thread's pair of codes, as codes and as the mirrored comparisons leave them
+    const auto code_of = [&](uint32_t raw) { const uint32_t t = raw & (n_cb >> 1); return ~(raw ^ (t - (t >> (j.bits - 1)))) & mask; };
+    const bool has_pair = tid < n_cb * n_cb;
+    const int e0 = has_pair ? tid & mask : 0, e1 = has_pair ? tid >> j.bits : 0;
+    const float p0 = j.cb[e0], p1 = j.cb[e1], m0 = j.cb[code_of(e0)], m1 = j.cb[code_of(e1)];
+    const long long first = (long long)wave * (gridDim.x / a.n_jobs) + blockIdx.x / a.n_jobs, stride = (long long)(gridDim.x / a.n_jobs) * RT_NW;
+    // The first tile's cache lines on their way while the rotations are laid out (two words a lane; all of the rows in registers beside the two
+    // rotations made the compiler spill what arrived).
+    uint32_t touched[2] = {0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const long long r = first * TILE + 32 * i + (lane >> 1);
+        if (r < j.n) touched[i] = reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(j.x) + row_offset(j, r))[32 * (lane & 1)];
+    }
+    qf_lay_out_rotation<DT>(rotation, reinterpret_cast<uint16_t*>(smem), tid);
+    dq_lay_out_rotation<DQ_UP>(back, reinterpret_cast<uint4*>(smem + QF_PI_BYTES), tid);
+    if (has_thr) thr[tid] = decision_threshold(c_lo, c_hi);
+    lds_barrier();                                               // (the rows may still be on their way)
+    const auto ready = [&](bool mirror) __attribute__((always_inline)) {
+        if (has_pair) {
+            const uint32_t lo = dq_centroid<DQ_UP>(mirror ? m0 : p0), hi = dq_centroid<DQ_UP>(mirror ? m1 : p1);
+            pairs[tid] = make_uint2((lo & 0xffffu) | (hi << 16), (lo >> 16) | (hi & 0xffff0000u));
+        }
+        lds_barrier();
+        return mirror;
+    };
+    const uint4* piA = reinterpret_cast<const uint4*>(smem);
+    const uint4* piB = reinterpret_cast<const uint4*>(smem + QF_PI_BYTES);
+    switch (j.bits) {
+        case 2: rt_walk<DT, 2>(j, piA, piB, pairs, thr, w, lane, first, stride, touched, ready); break;
+        case 3: rt_walk<DT, 3>(j, piA, piB, pairs, thr, w, lane, first, stride, touched, ready); break;
+        default: rt_walk<DT, 4>(j, piA, piB, pairs, thr, w, lane, first, stride, touched, ready); break;
+    }
+}
+
+// 16-bit rows of 2, 3 and 4 bits, one or two jobs a launch.  A workgroup a tile as long as there are compute units: fewer wavefronts share a SIMD.
+int launch_round_trip_rows(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
+    if (dtype == ODMKV_F16) ODMKV_ALLOW_LDS(round_trip_rows_kernel<ODMKV_F16>, RT_LDS);
+    else ODMKV_ALLOW_LDS(round_trip_rows_kernel<ODMKV_BF16>, RT_LDS);
     RowsArgs a;
     for (int i = 0; i < 2; ++i) a.job[i] = jobs[i < n_jobs ? i : 0];
     a.n_jobs = n_jobs;
-    const dim3 grid = rows_grid(jobs, n_jobs, QF_NW);
-    if (dtype == ODMKV_F16) hipLaunchKernelGGL(quant_rows_f16_kernel<ODMKV_F16>, grid, dim3(QF_NW * 64), lds, st, a);
-    else hipLaunchKernelGGL(quant_rows_f16_kernel<ODMKV_BF16>, grid, dim3(QF_NW * 64), lds, st, a);
+    const dim3 grid = rows_grid(jobs, n_jobs, 1);
+    if (dtype == ODMKV_F16) hipLaunchKernelGGL(round_trip_rows_kernel<ODMKV_F16>, grid, dim3(RT_NW * 64), RT_LDS, st, a);
+    else hipLaunchKernelGGL(round_trip_rows_kernel<ODMKV_BF16>, grid, dim3(RT_NW * 64), RT_LDS, st, a);
+    ODMKV_CHECK_LAUNCH("round_trip_rows_kernel");
+    return 0;
+}
+
+int launch_quantize_rows_f16(const RowsJob& job, int dtype, hipStream_t st) {
+    const size_t lds = QF_PI_BYTES + (size_t)QF_NW * QF_STAGE + QF_THR_BYTES + QF_NW * sizeof(QfWave);
+    if (dtype == ODMKV_F16) ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_F16>, lds);
+    else ODMKV_ALLOW_LDS(quant_rows_f16_kernel<ODMKV_BF16>, lds);
+    const dim3 grid = rows_grid(&job, 1, QF_NW);
+    if (dtype == ODMKV_F16) hipLaunchKernelGGL(quant_rows_f16_kernel<ODMKV_F16>, grid, dim3(QF_NW * 64), lds, st, job);
+    else hipLaunchKernelGGL(quant_rows_f16_kernel<ODMKV_BF16>, grid, dim3(QF_NW * 64), lds, st, job);
     ODMKV_CHECK_LAUNCH("quant_rows_f16_kernel");
     return 0;
 }

@@ -58,14 +58,11 @@ __global__ __launch_bounds__(64) void quantize_rows_kernel(RowsJob job) {
     quantize_rows_tile<W, DT>(job, blockIdx.x, cb);
 }
 
-// The tiles that the matrix-core quantiser has marked, of both tensors (rows with infinities or many values next to a
-// threshold; usually none: the launch's own time counts).  A workgroup looks 64 tiles over, a lane each, and does the marked
-// ones.  With a workgroup per tile and a launch per tensor a pass over 8k tokens of 8 heads took 69.3 us, with this one 67.2.
-struct FlaggedArgs { RowsJob job[2]; };
+// The tiles that the matrix-core quantiser has marked (rows with infinities or many values next to a threshold; usually none: the launch's own
+// time counts).  A workgroup looks 64 tiles over, a lane each, and does the marked ones.
 template <int DT>
-__global__ __launch_bounds__(64) void quantize_flagged_rows_kernel(FlaggedArgs a) {
+__global__ __launch_bounds__(64) void quantize_flagged_rows_kernel(RowsJob job) {
     __shared__ float cb[16];
-    const RowsJob& job = a.job[blockIdx.y];
     const int64_t tile0 = (int64_t)blockIdx.x * WAVE, at = (tile0 + threadIdx.x) * WAVE;
     unsigned long long marked = __ballot(at < job.n && __float_as_uint(job.norms[at]) == ROWS_HANDED_OVER);
     while (marked) {                                           // (wave-uniform; a wavefront is the workgroup)
@@ -159,27 +156,13 @@ static int check_rows(const char* who, const void* x, const float* pi, const flo
 }
 
 // 16-bit rows of 2, 3 and 4 bits take the matrix cores first and the exact quantiser for what they leave
-static int quantize(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st) {
-    RowsJob fast[2];
-    int n_fast = 0;
-    for (int i = 0; i < n_jobs; ++i)
-        if (dtype != ODMKV_F32 && jobs[i].bits < 8) fast[n_fast++] = jobs[i];
-    if (n_fast) {
-        if (int rc = launch_quantize_rows_f16(fast, n_fast, dtype, st)) return rc;
-        FlaggedArgs a;
-        long long most = 0;
-        for (int i = 0; i < 2; ++i) {
-            a.job[i] = fast[i < n_fast ? i : 0];
-            most = std::max(most, a.job[i].n);
-        }
-        const dim3 grid((unsigned)((most + WAVE * WAVE - 1) / (WAVE * WAVE)), n_fast), block(WAVE);
-        if (dtype == ODMKV_F16) hipLaunchKernelGGL(quantize_flagged_rows_kernel<ODMKV_F16>, grid, block, 0, st, a);
-        else hipLaunchKernelGGL(quantize_flagged_rows_kernel<ODMKV_BF16>, grid, block, 0, st, a);
-        ODMKV_CHECK_LAUNCH("quantize_flagged_rows_kernel");
-    }
-    for (int i = 0; i < n_jobs; ++i)
-        if (dtype == ODMKV_F32 || jobs[i].bits == 8)
-            if (int rc = launch_quantize_rows_exact(jobs[i], dtype, st)) return rc;
+static int quantize(const RowsJob& job, int dtype, hipStream_t st) {
+    if (dtype == ODMKV_F32 || job.bits == 8) return launch_quantize_rows_exact(job, dtype, st);
+    if (int rc = launch_quantize_rows_f16(job, dtype, st)) return rc;
+    const dim3 grid((unsigned)((job.n + WAVE * WAVE - 1) / (WAVE * WAVE))), block(WAVE);
+    if (dtype == ODMKV_F16) hipLaunchKernelGGL(quantize_flagged_rows_kernel<ODMKV_F16>, grid, block, 0, st, job);
+    else hipLaunchKernelGGL(quantize_flagged_rows_kernel<ODMKV_BF16>, grid, block, 0, st, job);
+    ODMKV_CHECK_LAUNCH("quantize_flagged_rows_kernel");
     return 0;
 }
 
@@ -188,7 +171,7 @@ static int quantize_rows(const char* who, const void* x, int dtype, int64_t N, i
     if (int rc = check_rows(who, x, pi, cb, codes, norms, dtype, N, stride_n, bits)) return rc;
     if (N == 0) return 0;
     const RowsJob j = {x, 0, (long long)stride_n, (long long)N, (long long)N, bits, packed, pi, cb, codes, norms, nullptr};
-    return quantize(&j, 1, dtype, (hipStream_t)stream);
+    return quantize(j, dtype, (hipStream_t)stream);
 }
 
 extern "C" int odmkv_quantize_rows(const void* x, int dtype, int64_t N, int64_t stride_n, int bits,
@@ -254,6 +237,14 @@ extern "C" int odmkv_round_trip_rows(void* K, void* V, int dtype, int64_t groups
         if (int rc = check_rows("round_trip_rows", x, j[i].pi, j[i].cb, codes, norms, dtype, n, stride_row, j[i].bits)) return rc;
         ODMKV_CHECK_ARG(stride_group % 8 == 0, "round_trip_rows: rows must be 16-byte aligned");
     }
-    if (int rc = quantize(j, 2, dtype, (hipStream_t)stream)) return rc;
-    return launch_dequantize_rows_f16(j, 2, dtype, (hipStream_t)stream);
+    // 2, 3 and 4 bits in one pass, 8 bits by the exact quantiser and the dequantiser
+    RowsJob narrow[2], wide[2];
+    int n_narrow = 0, n_wide = 0;
+    for (int i = 0; i < 2; ++i) (j[i].bits < 8 ? narrow[n_narrow++] : wide[n_wide++]) = j[i];
+    if (n_narrow)
+        if (int rc = launch_round_trip_rows(narrow, n_narrow, dtype, (hipStream_t)stream)) return rc;
+    if (n_wide == 0) return 0;
+    for (int i = 0; i < n_wide; ++i)
+        if (int rc = quantize(wide[i], dtype, (hipStream_t)stream)) return rc;
+    return launch_dequantize_rows_f16(wide, n_wide, dtype, (hipStream_t)stream);
 }

@@ -70,6 +70,36 @@ def test_round_trip_in_place(B, H, T, lo, hi, bits, dtype):
         assert ((got.float() - y.float()).abs() <= step * y.float().abs() + 1e-5).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bits", [2, 3, 4])
+@pytest.mark.parametrize("n,shift", [(1, 0.0), (64, 0.0), (65, 0.0), (40000, 0.0), (130, 3e-3)])
+def test_round_trip_takes_the_quantiser_s_codes(n, shift, bits, dtype):
+    """In one pass over the rows, every code is the one that the quantiser gives: ordinary rows, rows of zeros, one element, tiny and large ones, tiles with
+    more values next to a threshold than the list holds, and infinities; tables that mirror and one that does not; whole tiles, one row and one
+    row more, several tiles a wavefront."""
+    from kvquant import TurboQuantBackendPress
+    x = _rows(n, dtype, bits)
+    press = TurboQuantBackendPress(key_bits=bits, value_bits=bits, value_quantizer="mse")
+    kq, vq = press._q(bits, 42, x), press._q(bits, 2042, x)
+    kq.centroids = kq.centroids.clone()
+    kq.centroids[0] -= shift
+    if n >= 130:                                                 # (the first tile holds rows without a norm already)
+        mid = float((kq.centroids[0] + kq.centroids[1]) / 2)     # on the first threshold after the rotation: 128 listed values a row
+        x[70:78] = (torch.full((8, 128), mid, device="cuda") @ kq.pi).to(dtype)
+        x[79] = 0.0
+    k, v = x.view(1, 1, n, 128).clone(), x.view(1, 1, n, 128).clone()
+    press._quantise_span(0, k, v, 0, n)
+    step = 2 ** -10 if dtype == torch.float16 else 2 ** -7
+    for got, q in ((k, kq), (v, vq)):
+        codes, norms = q.quantize_codes(x.float())
+        want = (q.centroids.double()[codes.long()] @ q.pi.double()) * norms.double()[:, None]
+        finite = torch.isfinite(want).all(dim=-1)
+        assert finite.sum() >= n - 2 and not torch.isfinite(got.view(n, 128)[~finite]).any()
+        # a code more or less moves the row by a centroid's distance, some tenths of a percent of its norm at the least
+        scale = norms.double()[finite, None].abs()
+        assert ((got.view(n, 128)[finite].double() - want[finite]).abs() <= step * want[finite].abs() + 1e-6 * scale + 1e-7).all()
+
+
 @pytest.mark.parametrize("kind", [torch.uint8, torch.int16, torch.int32, torch.int64])
 @pytest.mark.parametrize("bits,pad", [(2, 0), (3, 0), (4, 5), (8, 0), (2, 3)])
 def test_indices_in_wider_types_and_padded_rows(bits, pad, kind):
