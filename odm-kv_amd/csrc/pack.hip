@@ -898,14 +898,21 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
 // kernel above spends its time on, yet the chain's last bits matter only when y lies next to a
 // threshold.  So y is first computed fast: the fp16 row as it is, against Pi split into two fp16
 // terms (hi + lo, 22 bits), on v_mfma_f32_16x16x32_f16, then scaled by 1 / (|x| + 1e-10).  That
-// estimate differs from the chain's result by rounding alone: at most about 2.5e-5 on the scale
-// |y| <= 1 under the most pessimistic model of the matrix unit's adder (every one of the 128 terms
-// truncated at the scale of the largest partial sum); measured, a band of 1e-7 already leaves no code
-// different over 1e8 values.  Values farther than QF_BAND (twice that bound) from every threshold therefore have the chain's code already; the few within the band
-// (two to eight in a thousand) are listed, and whenever a wave has 64 of them it recomputes them by
+// estimate differs from the chain's result by rounding alone.  On the scale |y| <= 1, in which no partial sum exceeds 1 (Cauchy-Schwarz):
+//   the chain        128 roundings to nearest of numbers below 1                                          3.8e-6
+//   the estimate     8 instructions, each off by at most 5.5 units in the last place of its largest term  5.2e-6
+//                    (measured on the instruction: next to a term of 1 a product counts down to 2^-26 and
+//                    is dropped below, so 32 of them lose at most 4 units of 2^-23; 1.6 million random
+//                    sums of either type, 32 products and an addend, were off by 5.3 at the most)
+//   Pi's two terms (2^-25 an element at the least), 1 / |x| and the product with it                       0.6e-6
+// together 9.6e-6.  Measured, a band of 1e-7 already leaves no code
+// different over 1e8 values.  Values farther than QF_BAND from every threshold therefore have the chain's code already; the few within the band
+// (a half to two in a thousand) are listed, and whenever a wave has 64 of them it recomputes them by
 // the chain itself, one lane per value, and replaces their codes in the packed tiles it has already
 // written.  Rows of zeros are exact either way.
-// Tiles the scheme does not cover go to the exact kernel through a list: 8-bit tiles (a tenth of
+// (With a band of 5e-5, for an instruction that cuts every one of its terms at its largest one's last place, four times as many were listed, and
+// the chains, whose lanes read rows apart from each other's, took 56 of the 217 us of 131k tokens of bf16 and 11 of the 82 of 32k of fp16.)
+// Tiles the scheme does not cover go to the exact kernel through a list: 8-bit tiles (a fiftieth of
 // their values lie inside the band), tiles with a row whose squared norm is not finite, and tiles
 // with more listed values than the list has room for.
 //
@@ -919,10 +926,10 @@ typedef __bf16 qf_b8 __attribute__((ext_vector_type(8)));
 typedef float qf_f4 __attribute__((ext_vector_type(4)));
 
 #ifndef QF_BAND
-#define QF_BAND 5.0e-5f
+#define QF_BAND 1.2e-5f
 #endif
 // bf16 rows meet Pi as two bf16 terms (16 bits: up to 7.6e-6 more on the estimate, by Cauchy-Schwarz over the row)
-#define QF_BAND_BF16 7.0e-5f
+#define QF_BAND_BF16 2.0e-5f
 
 // D += A x B on the matrix cores of the rows' own 16-bit type (operands as they sit in four 32-bit registers)
 template <int DT>
