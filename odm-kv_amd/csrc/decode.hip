@@ -1121,7 +1121,7 @@ __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(Deco
 #pragma unroll
         for (int w = 0; w < NW; ++w) L += wl[w * 8 + g];
         dst[g * PSTRIDE + HD] = wM[g];
-        dst[g * PSTRIDE + HD + 1] = L;
+        dst[g * PSTRIDE + HD + 1] = li == 4 ? -L : L;          // (the sign tells the merge that the item is one of exact rows)
     }
 }
 
@@ -1132,6 +1132,21 @@ __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(Deco
 #define MERGE_SLICES (MERGE_THREADS / HD)
 #define MERGE_CHUNK 64            // items merged per round: one per lane of a wavefront
 #define NO_ROW (~(size_t)0)
+
+// sum and maximum over a wavefront without LDS (six reads one behind the other of a shuffle's)
+template <typename F>
+__device__ static inline float wave_fold_dpp(float v, F f) {
+    v = f(v, dpp<0xB1>(v));                               // lane ^ 1
+    v = f(v, dpp<0x4E>(v));                               // lane ^ 2
+    v = f(v, dpp<0x141>(v));                              // the other four of eight
+    v = f(v, dpp<0x140>(v));                              // the other eight of sixteen
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ static inline float wave_max_dpp(float v) { return wave_fold_dpp(v, [](float x, float y) { return fmaxf(x, y); }); }
+__device__ static inline float wave_sum_dpp(float v) { return wave_fold_dpp(v, [](float x, float y) { return x + y; }); }
 
 // where query head bq (head g of its group) of this launch's pass stands in out and lse
 // (BLOCK: a kernel of its own for blocks of query tokens; deciding it at run time cost the decode step's merge 0.15 of 4 us)
@@ -1153,11 +1168,12 @@ __device__ static inline void count_new_token(const odmkv_packed_t& s, int bh) {
 // 1 for large batches, where every further workgroup only repeats the reading)
 template <int GP, int MERGE_SPLIT, bool BLOCK>
 __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs a) {
-    __shared__ float part[2][MERGE_SLICES][HD];      // [rotated | exact][slice][dim]
+    __shared__ __align__(16) float part[2][MERGE_SLICES][HD];      // [rotated | exact][slice][dim]
     constexpr int QD = HD / MERGE_SPLIT;                 // output dims of this workgroup
     constexpr int RS = MERGE_THREADS / QD;                // row slices of the rotation
     constexpr int IN = HD / RS;                           // rows per slice
-    __shared__ float part2[RS * QD];
+    constexpr int RW = RS > MERGE_THREADS / WAVE ? MERGE_THREADS / WAVE : RS;      // sums of the slices: one a wavefront where it holds two
+    __shared__ float part2[RW * QD];
     // MERGE_SPLIT workgroups per query head: each merges the head's partial results in full (they are small and
     // shared through the caches) and rotates back its share of the output dims, so that no workgroup has to pull
     // the whole 64 KB rotation through one compute unit
@@ -1184,11 +1200,9 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
     for (int c0 = 0; c0 < n; c0 += MERGE_CHUNK) {
         const int nc = min(n - c0, MERGE_CHUNK);
         float m_i = -INFINITY, l_i = 0.0f;
-        int level = 0;
         if (lane < nc) {
-            const float* p = partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE;
-            m_i = p[HD]; l_i = p[HD + 1];
-            level = a.items[8 * (i0 + c0 + lane) + 1];
+            const float2 ml = *reinterpret_cast<const float2*>(partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE + HD);
+            m_i = ml.x; l_i = ml.y;
         }
         float vals[MERGE_CHUNK / MERGE_SLICES];
 #pragma unroll
@@ -1196,12 +1210,12 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
             const int it = slice + k * MERGE_SLICES;
             vals[k] = it < nc ? partial[((size_t)(i0 + c0 + it) * GP + g) * PSTRIDE + j] : 0.0f;
         }
-        const float Mc = fmaxf(M, wave_max(m_i));
+        const float Mc = fmaxf(M, wave_max_dpp(m_i));
         const float f_old = M > -INFINITY ? __builtin_amdgcn_exp2f(M - Mc) : 0.0f;
         const float w = m_i > -INFINITY ? __builtin_amdgcn_exp2f(m_i - Mc) : 0.0f;
-        L = __fmaf_rn(L, f_old, wave_sum(l_i * w));
+        L = __fmaf_rn(L, f_old, wave_sum_dpp(fabsf(l_i) * w));
         arot *= f_old; aex *= f_old;
-        const int wsgn = __float_as_int(level == 4 ? -w : w);          // the sign bit marks exact items
+        const int wsgn = __float_as_int(copysignf(w, l_i));            // the sign bit marks exact items
 #pragma unroll
         for (int k = 0; k < MERGE_CHUNK / MERGE_SLICES; ++k) {
             const int it = slice + k * MERGE_SLICES;                     // wave-uniform
@@ -1219,20 +1233,25 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
     // rotate the quantised part back: out_j = sum_i rot_i Pi_v[i][j] for this workgroup's dims; the slices split the i range
     float o = 0.0f;
 #pragma unroll
-    for (int ii = 0; ii < IN; ++ii) {
-        const int i = rs * IN + ii;
-        float r = part[0][0][i];
+    for (int ii = 0; ii < IN; ii += 4) {
+        f4 r = *reinterpret_cast<const f4*>(&part[0][0][rs * IN + ii]);
 #pragma unroll
-        for (int sl = 1; sl < MERGE_SLICES; ++sl) r += part[0][sl][i];
-        o = __fmaf_rn(r, pv[ii], o);
+        for (int sl = 1; sl < MERGE_SLICES; ++sl) r += *reinterpret_cast<const f4*>(&part[0][sl][rs * IN + ii]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o = __fmaf_rn(r[e], pv[ii + e], o);
     }
-    part2[rs * QD + jj] = o;
+    if constexpr (RW < RS) {                               // two slices a wavefront: its halves
+        static_assert(QD == 32, "a slice a half");
+        const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(o), __float_as_uint(o), false, false);
+        o = __uint_as_float(both[0]) + __uint_as_float(both[1]);
+        if (lane < QD) part2[(tid / WAVE) * QD + lane] = o;
+    } else part2[rs * QD + jj] = o;
     __syncthreads();
     if (tid < QD) {
         const int dim = quarter * QD + tid;
         float tot = 0.0f;
 #pragma unroll
-        for (int r = 0; r < RS; ++r) tot += part2[r * QD + tid];
+        for (int r = 0; r < RW; ++r) tot += part2[r * QD + tid];
 #pragma unroll
         for (int sl = 0; sl < MERGE_SLICES; ++sl) tot += part[1][sl][dim];
         const float o32 = L > 0.0f ? tot / L : 0.0f;
@@ -1275,18 +1294,16 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
             for (int c0 = 0; c0 < n; c0 += MERGE_CHUNK) {
                 const int nc = min(n - c0, MERGE_CHUNK);
                 float m_i = -INFINITY, l_i = 0.0f;
-                int level = 0;
                 if (lane < nc) {
-                    const float* p = partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE;
-                    m_i = p[HD]; l_i = p[HD + 1];
-                    level = a.items[8 * (i0 + c0 + lane) + 1];
+                    const float2 ml = *reinterpret_cast<const float2*>(partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE + HD);
+                    m_i = ml.x; l_i = ml.y;
                 }
-                const float Mc = fmaxf(M, wave_max(m_i));
+                const float Mc = fmaxf(M, wave_max_dpp(m_i));
                 const float f_old = M > -INFINITY ? __builtin_amdgcn_exp2f(M - Mc) : 0.0f;
                 const float w = m_i > -INFINITY ? __builtin_amdgcn_exp2f(m_i - Mc) : 0.0f;
-                L = __fmaf_rn(L, f_old, wave_sum(l_i * w));
+                L = __fmaf_rn(L, f_old, wave_sum_dpp(fabsf(l_i) * w));
                 arot *= f_old; aex *= f_old;
-                const int wsgn = __float_as_int(level == 4 ? -w : w);      // the sign bit marks exact items
+                const int wsgn = __float_as_int(copysignf(w, l_i));        // the sign bit marks exact items
                 for (int it0 = 0; it0 < nc; it0 += 4) {                    // four items' values under way at a time
                     float vals[4];
 #pragma unroll
