@@ -1014,7 +1014,7 @@ __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(Deco
     const int bh = d0.x;
     int li = d0.y, tile0 = d0.z, ntiles = d0.w, ntok = d1.x;
     const int pass = blockIdx.y;                               // (0 but for blocks of query tokens)
-    const int bq_first = (pass * a.B + bh / a.s.Hkv) * a.Hq + (bh % a.s.Hkv) * a.G;      // first query head of the group
+    const int bq_first = pass * a.B * a.Hq + bh * a.G;          // first query head of the group
 
     float* dst = a.partial + ((size_t)pass * a.n_items + item) * GP * PSTRIDE;      // where this item's result goes
 
@@ -1177,12 +1177,10 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
     // MERGE_SPLIT workgroups per query head: each merges the head's partial results in full (they are small and
     // shared through the caches) and rotates back its share of the output dims, so that no workgroup has to pull
     // the whole 64 KB rotation through one compute unit
-    const int bq = blockIdx.x / MERGE_SPLIT, quarter = blockIdx.x % MERGE_SPLIT;
+    const int g = blockIdx.x / MERGE_SPLIT, quarter = blockIdx.x % MERGE_SPLIT, bh = blockIdx.z;      // (a grid without divisions)
     const int tid = threadIdx.x, lane = tid & 63, j = tid & (HD - 1);
     const int slice = __builtin_amdgcn_readfirstlane(tid >> 7);
-    const int b = bq / a.Hq, hq = bq % a.Hq;
-    const int bh = b * a.s.Hkv + hq / a.G, g = hq % a.G;
-    const size_t row = out_row<BLOCK>(a, bq, bh, g);       // of out and lse
+    const size_t row = out_row<BLOCK>(a, bh * a.G + g, bh, g);       // of out and lse
     if (row == NO_ROW) return;                             // (workgroup-uniform: padding of a block's last pass)
     const float* partial = BLOCK ? a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE : a.partial;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
@@ -1215,14 +1213,16 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
         const float w = m_i > -INFINITY ? __builtin_amdgcn_exp2f(m_i - Mc) : 0.0f;
         L = __fmaf_rn(L, f_old, wave_sum_dpp(fabsf(l_i) * w));
         arot *= f_old; aex *= f_old;
-        const int wsgn = __float_as_int(copysignf(w, l_i));            // the sign bit marks exact items
+        const int exact = __float_as_int(l_i) >> 31;                   // (the sign marks exact items)
 #pragma unroll
         for (int k = 0; k < MERGE_CHUNK / MERGE_SLICES; ++k) {
             const int it = slice + k * MERGE_SLICES;                     // wave-uniform
             if (it < nc) {
-                const float ww = __int_as_float(__builtin_amdgcn_readlane(wsgn, it));
-                if (__float_as_uint(ww) >> 31) aex = __fmaf_rn(vals[k], -ww, aex);
-                else arot = __fmaf_rn(vals[k], ww, arot);
+                // (a branch an item cost 0.15 us of the call; the value, not the weight, is what becomes zero: it may be infinite)
+                const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), it));
+                const int ex = __builtin_amdgcn_readlane(exact, it);
+                aex = __fmaf_rn(__int_as_float(__float_as_int(vals[k]) & ex), wi, aex);
+                arot = __fmaf_rn(__int_as_float(__float_as_int(vals[k]) & ~ex), wi, arot);
             }
         }
         M = Mc;
@@ -1279,7 +1279,6 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
     const int bh = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, j = tid & (HD - 1);
     const int slice = __builtin_amdgcn_readfirstlane(tid >> 7);
-    const int b = bh / a.s.Hkv, hq0 = (bh % a.s.Hkv) * a.G;
     const float* partial = BLOCK ? a.partial + (size_t)blockIdx.y * a.n_items * GP * PSTRIDE : a.partial;
     const int i0 = a.item_range[bh], n = a.item_range[bh + 1] - i0;
     if (a.k_new && tid == 0) count_new_token(a.s, bh);
@@ -1351,7 +1350,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
         for (int r = 0; r < RS; ++r) tot += part2[g][r][j];
         const float L = headL[g];
         const float o32 = L > 0.0f ? tot / L : 0.0f;
-        const size_t row = out_row<BLOCK>(a, b * a.Hq + hq0 + g, bh, g);
+        const size_t row = out_row<BLOCK>(a, bh * a.G + g, bh, g);
         if (row == NO_ROW) continue;
         const size_t oi = row * HD + j;
         if (a.out_dt == ODMKV_F32) reinterpret_cast<float*>(a.out)[oi] = o32;
@@ -1501,12 +1500,13 @@ int odmkv_decode_launch(const void* q, int q_dtype, int B, int Hq, float scaling
         // from 512 query heads on, a workgroup per (sequence, kv-head) merges all heads of the group (64 x 2048 tokens, 2048
         // heads: the merge 10.8 -> 4.8 us; 512 heads: 3.5 -> 3.2 us); ODMKV_MERGE_GROUP_FROM moves the limit, for measurements
         static const int group_from = [] { const char* e = getenv("ODMKV_MERGE_GROUP_FROM"); return e ? atoi(e) : 512; }();
-        const auto launch = [&](auto kernel, int wgs) { hipLaunchKernelGGL(kernel, dim3(wgs, passes), dim3(MERGE_THREADS), 0, st, a); };
+        const auto launch = [&](auto kernel, int wgs, int pairs) { hipLaunchKernelGGL(kernel, dim3(wgs, passes, pairs), dim3(MERGE_THREADS), 0, st, a); };
+        const int pairs = B * store->Hkv;                   // (fewer than 512 where they are the grid's third axis)
 #define ODMKV_MERGE(BLOCK)                                                                                                        \
-        if (heads >= group_from) launch(GP == 4 ? decode_merge_group_kernel<4, BLOCK> : decode_merge_group_kernel<8, BLOCK>, B * store->Hkv);   \
-        else if (heads >= 256) launch(GP == 4 ? decode_merge_kernel<4, 1, BLOCK> : decode_merge_kernel<8, 1, BLOCK>, B * Hq);      \
-        else if (heads >= 128) launch(GP == 4 ? decode_merge_kernel<4, 2, BLOCK> : decode_merge_kernel<8, 2, BLOCK>, B * Hq * 2);  \
-        else launch(GP == 4 ? decode_merge_kernel<4, 4, BLOCK> : decode_merge_kernel<8, 4, BLOCK>, B * Hq * 4)
+        if (heads >= group_from) launch(GP == 4 ? decode_merge_group_kernel<4, BLOCK> : decode_merge_group_kernel<8, BLOCK>, pairs, 1);   \
+        else if (heads >= 256) launch(GP == 4 ? decode_merge_kernel<4, 1, BLOCK> : decode_merge_kernel<8, 1, BLOCK>, G, pairs);      \
+        else if (heads >= 128) launch(GP == 4 ? decode_merge_kernel<4, 2, BLOCK> : decode_merge_kernel<8, 2, BLOCK>, G * 2, pairs);  \
+        else launch(GP == 4 ? decode_merge_kernel<4, 4, BLOCK> : decode_merge_kernel<8, 4, BLOCK>, G * 4, pairs)
         if (a.block_len) { ODMKV_MERGE(true); } else { ODMKV_MERGE(false); }
 #undef ODMKV_MERGE
         ODMKV_CHECK_LAUNCH("decode_merge_kernel");
