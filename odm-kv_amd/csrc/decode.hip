@@ -1297,23 +1297,29 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
                     const float2 ml = *reinterpret_cast<const float2*>(partial + ((size_t)(i0 + c0 + lane) * GP + g) * PSTRIDE + HD);
                     m_i = ml.x; l_i = ml.y;
                 }
+                // eight items' values under way at a time, the first eight beside the (m, l) of all
+                float vals[8];
+                const auto request = [&](int it0) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k)
+                        vals[k] = it0 + k < nc ? partial[((size_t)(i0 + c0 + it0 + k) * GP + g) * PSTRIDE + j] : 0.0f;
+                };
+                request(0);
                 const float Mc = fmaxf(M, wave_max_dpp(m_i));
                 const float f_old = M > -INFINITY ? __builtin_amdgcn_exp2f(M - Mc) : 0.0f;
                 const float w = m_i > -INFINITY ? __builtin_amdgcn_exp2f(m_i - Mc) : 0.0f;
                 L = __fmaf_rn(L, f_old, wave_sum_dpp(fabsf(l_i) * w));
                 arot *= f_old; aex *= f_old;
-                const int wsgn = __float_as_int(copysignf(w, l_i));        // the sign bit marks exact items
-                for (int it0 = 0; it0 < nc; it0 += 4) {                    // four items' values under way at a time
-                    float vals[4];
+                const int exact = __float_as_int(l_i) >> 31;               // (the sign marks exact items)
+                for (int it0 = 0; it0 < nc; it0 += 8) {
+                    if (it0 > 0) request(it0);
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        vals[k] = it0 + k < nc ? partial[((size_t)(i0 + c0 + it0 + k) * GP + g) * PSTRIDE + j] : 0.0f;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
+                    for (int k = 0; k < 8; ++k) {
                         if (it0 + k < nc) {
-                            const float ww = __int_as_float(__builtin_amdgcn_readlane(wsgn, it0 + k));
-                            if (__float_as_uint(ww) >> 31) aex = __fmaf_rn(vals[k], -ww, aex);
-                            else arot = __fmaf_rn(vals[k], ww, arot);
+                            const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), it0 + k));
+                            const int ex = __builtin_amdgcn_readlane(exact, it0 + k);
+                            aex = __fmaf_rn(__int_as_float(__float_as_int(vals[k]) & ex), wi, aex);
+                            arot = __fmaf_rn(__int_as_float(__float_as_int(vals[k]) & ~ex), wi, arot);
                         }
                     }
                 }
