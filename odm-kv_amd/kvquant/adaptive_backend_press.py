@@ -260,17 +260,19 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
             # (also where a store cannot be made: the kernels write into page-locked memory that is given back on the way out)
             for ev in arrived.values():
                 ev.synchronize()
-        masked, at = [], 0
         totals = [counts.numpy().sum(axis=1).swapaxes(0, 1) for *_, counts in plan]      # (bulk, stored) of every layer
+        # The GPU has run dry while the counts were on their way: the quantisers first, what only the host needs behind everything that is launched
+        states = []
+        for (layer_idx, bits, levels, _), (_, stored) in zip(plan, totals):
+            keys, values = self._get_cache_tensors(cache, layer_idx)
+            states.append(self._get_or_create_state(layer_idx, keys))
+            states[-1].prefill(keys, values, bits, _known_counts=stored, _levels=levels)
+        masked, at = [], 0
         for levels, T in evicted:
             masked += evicted_indices(levels, T, [int(stored[:, 0].sum()) for _, stored in totals[at:at + len(levels)]])
             at += len(levels)
-        for (layer_idx, bits, levels, counts), (bulk, stored), gone in zip(plan, totals, masked):
-            keys, values = self._get_cache_tensors(cache, layer_idx)
-            wanted = sorted(set(int(b) for b in self.bit_levels) | {16})
-            self._store_observed_ratios(layer_idx, bits.shape[1], wanted, bulk[:, [_lib.LEVEL_ORDER.index(b) for b in wanted]])
-            state = self._get_or_create_state(layer_idx, keys)
-            state.prefill(keys, values, bits, _known_counts=stored, _levels=levels)
+        for (layer_idx, *_), state, gone in zip(plan, states, masked):
+            keys, _ = self._get_cache_tensors(cache, layer_idx)
             state.adopt_masked(gone)
             module = self._layer_modules.get(layer_idx)
             if module is not None:
@@ -282,6 +284,10 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
                 self._buffer_counts[layer_idx] = 0
             if self._last_hooked_layer_idx is None or layer_idx == self._last_hooked_layer_idx:
                 release_staging(keys.device)             # the prompt is stored: worst-case stores that direct fills left can go
+        wanted = sorted(set(int(b) for b in self.bit_levels) | {16})
+        columns = [_lib.LEVEL_ORDER.index(b) for b in wanted]
+        for (layer_idx, bits, *_), (bulk, _) in zip(plan, totals):
+            self._store_observed_ratios(layer_idx, bits.shape[1], wanted, bulk[:, columns])
         self._reset_prefill_state()
 
     # ------------------------------------------------------------------ hook
