@@ -89,14 +89,22 @@ template <> struct Elem<ODMKV_F32> {
     __device__ static inline float from_f32(float f) { return f; }
 };
 
-// wave-wide reductions (64 lanes) through cross-lane shuffles
-__device__ static inline float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+// Wave-wide reductions (64 lanes, all of them active; every lane ends with the result) by DPP moves and lane swaps: a shuffle is a read of LDS, six of them
+// one behind the other.
+template <int CTRL>
+__device__ static inline float wave_dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
-__device__ static inline float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-    return v;
+template <typename F>
+__device__ static inline float wave_fold(float v, F f) {
+    v = f(v, wave_dpp<0xB1>(v));                          // lane ^ 1
+    v = f(v, wave_dpp<0x4E>(v));                          // lane ^ 2
+    v = f(v, wave_dpp<0x141>(v));                         // the other four of eight
+    v = f(v, wave_dpp<0x140>(v));                         // the other eight of sixteen
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
+__device__ static inline float wave_sum(float v) { return wave_fold(v, [](float x, float y) { return x + y; }); }
+__device__ static inline float wave_max(float v) { return wave_fold(v, [](float x, float y) { return fmaxf(x, y); }); }

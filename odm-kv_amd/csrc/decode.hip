@@ -1133,21 +1133,6 @@ __global__ __launch_bounds__(NW * 64, PAIR ? 4 : 1) void decode_main_kernel(Deco
 #define MERGE_CHUNK 64            // items merged per round: one per lane of a wavefront
 #define NO_ROW (~(size_t)0)
 
-// sum and maximum over a wavefront without LDS (six reads one behind the other of a shuffle's)
-template <typename F>
-__device__ static inline float wave_fold_dpp(float v, F f) {
-    v = f(v, dpp<0xB1>(v));                               // lane ^ 1
-    v = f(v, dpp<0x4E>(v));                               // lane ^ 2
-    v = f(v, dpp<0x141>(v));                              // the other four of eight
-    v = f(v, dpp<0x140>(v));                              // the other eight of sixteen
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ static inline float wave_max_dpp(float v) { return wave_fold_dpp(v, [](float x, float y) { return fmaxf(x, y); }); }
-__device__ static inline float wave_sum_dpp(float v) { return wave_fold_dpp(v, [](float x, float y) { return x + y; }); }
-
 // where query head bq (head g of its group) of this launch's pass stands in out and lse
 // (BLOCK: a kernel of its own for blocks of query tokens; deciding it at run time cost the decode step's merge 0.15 of 4 us)
 template <bool BLOCK>
@@ -1208,10 +1193,10 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
             const int it = slice + k * MERGE_SLICES;
             vals[k] = it < nc ? partial[((size_t)(i0 + c0 + it) * GP + g) * PSTRIDE + j] : 0.0f;
         }
-        const float Mc = fmaxf(M, wave_max_dpp(m_i));
+        const float Mc = fmaxf(M, wave_max(m_i));
         const float f_old = M > -INFINITY ? __builtin_amdgcn_exp2f(M - Mc) : 0.0f;
         const float w = m_i > -INFINITY ? __builtin_amdgcn_exp2f(m_i - Mc) : 0.0f;
-        L = __fmaf_rn(L, f_old, wave_sum_dpp(fabsf(l_i) * w));
+        L = __fmaf_rn(L, f_old, wave_sum(fabsf(l_i) * w));
         arot *= f_old; aex *= f_old;
         const int exact = __float_as_int(l_i) >> 31;                   // (the sign marks exact items)
 #pragma unroll
@@ -1305,10 +1290,10 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_group_kernel(Decod
                         vals[k] = it0 + k < nc ? partial[((size_t)(i0 + c0 + it0 + k) * GP + g) * PSTRIDE + j] : 0.0f;
                 };
                 request(0);
-                const float Mc = fmaxf(M, wave_max_dpp(m_i));
+                const float Mc = fmaxf(M, wave_max(m_i));
                 const float f_old = M > -INFINITY ? __builtin_amdgcn_exp2f(M - Mc) : 0.0f;
                 const float w = m_i > -INFINITY ? __builtin_amdgcn_exp2f(m_i - Mc) : 0.0f;
-                L = __fmaf_rn(L, f_old, wave_sum_dpp(fabsf(l_i) * w));
+                L = __fmaf_rn(L, f_old, wave_sum(fabsf(l_i) * w));
                 arot *= f_old; aex *= f_old;
                 const int exact = __float_as_int(l_i) >> 31;               // (the sign marks exact items)
                 for (int it0 = 0; it0 < nc; it0 += 8) {
