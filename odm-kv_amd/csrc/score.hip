@@ -220,11 +220,16 @@ __global__ __launch_bounds__(256) void score_logits_kernel(ScoreArgs a) {
 // ---- pass 1 over 16-bit K on the matrix cores ----
 // v_mfma_f32_16x16x32_{f16,bf16}: D[16x16] += A[16x32] . B[32x16]; lane (n = lane % 16, j = lane / 16) supplies
 // A[n][8j+e] and B[8j+e][n] and holds D[4j+r][n].  B = 16 tokens x 32 dims of K exactly as they lie in memory (a
-// lane's 16 bytes), A = the mean queries of four heads, head (row % 4) in every row, as 16-bit pieces whose sum
-// is the fp32 value (fp16: high + low of the vector scaled by a power of two into fp16's range; bf16: three
-// pieces).  A wave takes 64 tokens as four groups of 16; after the products lane (j, n) keeps group j's
-// accumulator: the logits of four heads for token 16j + n.  |k|^2 is the diagonal of K_g . K_g^T, the same
-// registers as both operands.  All of a workgroup's rows are requested before anything is computed.
+// lane's 16 bytes), A = the mean queries of four heads as 16-bit pieces whose sum is the fp32 value (fp16: high +
+// low of the vector scaled by a power of two into fp16's range, twice over; bf16: three pieces and an unused row):
+// row 4 * piece + head, so that one product holds every piece, and the pieces are added in fp32 behind it.  A wave
+// takes 64 tokens as four groups of 16; lane (j, n) holds piece j of four heads for token n of each group, and the
+// swaps that add the pieces leave it with the logits of token 16j + n.  |k|^2 is the diagonal of K_g . K_g^T, the
+// same registers as both operands.  All of a workgroup's rows are requested before anything is computed.
+// Memory bounds it (behind a cache just written, 131072 tokens of 8 KV heads also push the last-level cache's dirty
+// lines out).  One product a piece into one sum, and a branch around each lane's pick, had cost 48 products instead
+// of 16 and 0.5-1.5 us a layer: 32768 tokens fp16 17.0 -> 16.2 us, 131072 tokens bf16 76.3 -> 74.7 us.  The logits'
+// mean error against 64 bits, of the sum of the terms' magnitudes: bf16 1.1e-8 -> 0.7e-8, fp16 1.4e-8 -> 1.3e-8.
 typedef _Float16 sc_h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 sc_b8 __attribute__((ext_vector_type(8)));
 typedef float sc_f4 __attribute__((ext_vector_type(4)));
@@ -236,13 +241,45 @@ __device__ static __forceinline__ sc_f4 sc_mfma(const uint4& a, const uint4& b, 
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(sc_b8, a), __builtin_bit_cast(sc_b8, b), c, 0, 0, 0);
 }
 
+// a ? x : y of two computed values, never a branch around them
+__device__ static __forceinline__ float sc_pick(int a, float x, float y) {
+    const uint32_t k = a ? 0xffffffffu : 0u;
+    return __uint_as_float((__float_as_uint(x) & k) | (__float_as_uint(y) & ~k));
+}
+__device__ static __forceinline__ void sc_swap16(float& x, float& y) {        // rows of 16 lanes: x = (x0, y0, x2, y2), y = (x1, y1, x3, y3)
+    const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(w[0]); y = __uint_as_float(w[1]);
+}
+__device__ static __forceinline__ void sc_swap32(float& x, float& y) {        // x = (x0, x1, y0, y1), y = (x2, x3, y2, y3)
+    const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(w[0]); y = __uint_as_float(w[1]);
+}
+// Lane (j, n) is left with the sum of v[j] over the rows of 16 lanes of column n: all four rows, the first three (the
+// fourth's values are not looked at), and the first two, which the other two repeat.
+__device__ static __forceinline__ float sc_scatter(float (&v)[4]) {
+    sc_swap32(v[0], v[2]); sc_swap32(v[1], v[3]);
+    float x = v[0] + v[2], y = v[1] + v[3];
+    sc_swap16(x, y);
+    return x + y;
+}
+__device__ static __forceinline__ float sc_scatter3(float (&v)[4], int lane) {
+    sc_swap32(v[0], v[2]); sc_swap32(v[1], v[3]);
+    float x = v[0] + sc_pick(lane & 16, 0.0f, v[2]), y = v[1] + sc_pick(lane & 16, 0.0f, v[3]);
+    sc_swap16(x, y);
+    return x + y;
+}
+__device__ static __forceinline__ float sc_scatter2(float (&v)[4], int lane) {
+    sc_swap16(v[0], v[1]); sc_swap16(v[2], v[3]);
+    return sc_pick(lane & 32, v[2] + v[3], v[0] + v[1]);
+}
+
 template <int DT, int GMAX>
 __global__ __launch_bounds__(256) void score_logits16_kernel(ScoreArgs a) {
     static_assert(DT == ODMKV_F16 || DT == ODMKV_BF16, "16-bit keys");
     static_assert(ROWS_PER_WG == 256, "four waves of 64 tokens");
     constexpr int NP = DT == ODMKV_F16 ? 2 : 3;     // 16-bit pieces of a mean query
     constexpr int HB = GMAX / 4;                    // blocks of four heads
-    __shared__ uint4 mu_op[HB][4][NP][16];          // [head block][32-dim block][piece][4 j + head % 4]: 8 elements
+    __shared__ uint4 mu_op[HB][4][WAVE];            // [head block][32-dim block][16 j + 4 piece + head % 4]: 8 elements
     __shared__ float unscale[GMAX];                 // 2^exponent / sqrt(d) per head
     __shared__ float red_m[4][GMAX], red_s[4][GMAX];
     const int chunk = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
@@ -296,46 +333,60 @@ __global__ __launch_bounds__(256) void score_logits16_kernel(ScoreArgs a) {
                 x[e] -= Elem<DT>::to_f32(b0); x[e + 1] -= Elem<DT>::to_f32(b1);       // exact: what the piece left over
                 w[e >> 1] = (uint32_t)b0 | ((uint32_t)b1 << 16);
             }
-            mu_op[hb][i][pc][tid & 15] = make_uint4(w[0], w[1], w[2], w[3]);
+            mu_op[hb][i][16 * sjj + 4 * pc + (tid & 3)] = make_uint4(w[0], w[1], w[2], w[3]);
+            if (NP == 2) mu_op[hb][i][16 * sjj + 4 * (pc + 2) + (tid & 3)] = make_uint4(w[0], w[1], w[2], w[3]);
         }
+        if (NP == 3) mu_op[hb][i][16 * sjj + 12 + (tid & 3)] = make_uint4(0u, 0u, 0u, 0u);
     }
     lds_barrier();
-    // |k|^2: lane (n / 4, n) holds the diagonal element of token n in component n % 4
+    uint4 mu8[HB][4];
+#pragma unroll
+    for (int hb = 0; hb < HB; ++hb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mu8[hb][i] = mu_op[hb][i][lane];
+    // a group's products as its keys arrive: |k|^2 (lane (n / 4, n) holds the diagonal element of token n in component
+    // n % 4) and the heads' pieces (lane (j, n): piece j of four heads)
+    float kn[4];
+    sc_f4 acc[HB][4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         sc_f4 gr = (sc_f4){0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) gr = sc_mfma<DT>(kx[q][i], kx[q][i], gr);
-        const int r = n & 3, t = t0 + 16 * q + n;
-        const float kn = r == 0 ? gr[0] : r == 1 ? gr[1] : r == 2 ? gr[2] : gr[3];
-        if (j == (n >> 2) && t < a.Tc) a.kn2[(size_t)h * a.Tc + t] = kn;
+        for (int hb = 0; hb < HB; ++hb) acc[hb][q] = (sc_f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            gr = sc_mfma<DT>(kx[q][i], kx[q][i], gr);
+#pragma unroll
+            for (int hb = 0; hb < HB; ++hb) acc[hb][q] = sc_mfma<DT>(mu8[hb][i], kx[q][i], acc[hb][q]);
+        }
+        const float lo = sc_pick(n & 1, gr[1], gr[0]), hi = sc_pick(n & 1, gr[3], gr[2]);
+        kn[q] = j == (n >> 2) ? sc_pick(n & 2, hi, lo) : 0.0f;
     }
     const int t = t0 + lane;                      // this lane's token: group j, column n
+    const bool in = t < a.Tc;
+    {
+        const float v = sc_scatter(kn);
+        if (in) a.kn2[(size_t)h * a.Tc + t] = v;
+    }
 #pragma unroll
     for (int hb = 0; hb < HB; ++hb) {
-        if (4 * hb >= a.Gl) break;
-        sc_f4 acc[4];
+        float d[4], m[4], e[4];                   // (heads past the group's last are computed and not stored: the four chains run side by side)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[q] = (sc_f4){0.0f, 0.0f, 0.0f, 0.0f};
+        for (int r = 0; r < 4; ++r) {
+            float v[4] = {acc[hb][0][r], acc[hb][1][r], acc[hb][2][r], acc[hb][3][r]};
+            const float x = (NP == 2 ? sc_scatter2(v, lane) : sc_scatter3(v, lane)) * unscale[4 * hb + r];    // every lane takes part
+            d[r] = in ? x : -INFINITY;
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int r = 0; r < 4; ++r) m[r] = wave_max(d[r]);
 #pragma unroll
-            for (int pc = NP - 1; pc >= 0; --pc) {           // small pieces first
-                const uint4 mu8 = mu_op[hb][i][pc][4 * j + (n & 3)];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc[q] = sc_mfma<DT>(mu8, kx[q][i], acc[q]);
-            }
-        const sc_f4 mine = j == 0 ? acc[0] : j == 1 ? acc[1] : j == 2 ? acc[2] : acc[3];
+        for (int r = 0; r < 4; ++r) e[r] = wave_sum(d[r] == -INFINITY ? 0.0f : __expf(d[r] - m[r]));
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int g = 4 * hb + r;
-            if (g < a.Gl) {
-                const float d = t < a.Tc ? mine[r] * unscale[g] : -INFINITY;
-                if (t < a.Tc) a.logits[((size_t)h * a.G + g) * a.Tc + t] = d;
-                const float m = wave_max(d);
-                const float s = wave_sum(d == -INFINITY ? 0.0f : __expf(d - m));
-                if (lane == 0) { red_m[wave][g] = m; red_s[wave][g] = s; }
-            }
+            if (g >= a.Gl) break;
+            if (in) a.logits[((size_t)h * a.G + g) * a.Tc + t] = d[r];
+            if (lane == 0) { red_m[wave][g] = m[r]; red_s[wave][g] = e[r]; }
         }
     }
     __syncthreads();
@@ -371,7 +422,7 @@ template <int DT> struct VTrip { static constexpr int ROWS = DT == ODMKV_F32 ? 8
 // Memory bounds the passes; what stood beside it was the merge of the block statistics: four entries a lane asked
 // for ahead of V (a longer prompt's rest came behind V's rows) and a chain of twelve shuffles and exponentials.
 // With eight entries, the largest taken first and the reduction in registers, a layer of 8 KV heads in bf16:
-// 131072 tokens 62.6 -> 56.7 us, 32768 tokens 14.0 -> 13.4 us (and the logits pass 79.2 -> 76.7, 17.5 -> 16.5 us).
+// 131072 tokens 62.6 -> 56.7 us, 32768 tokens 14.0 -> 13.4 us.
 
 // lane `src` of this lane's group of 16 (a row of the data-parallel-primitive network)
 __device__ static inline float group16_bcast(float v, int src) {
