@@ -1176,7 +1176,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void decode_merge_kernel(DecodeArgs 
 #pragma unroll
     for (int ii = 0; ii < IN; ++ii) pv[ii] = a.pi_v[(size_t)(rs * IN + ii) * HD + quarter * QD + jj];
     // The items are merged MERGE_CHUNK at a time with a running maximum, like an online softmax.  Inside a round
-    // nothing crosses wavefronts: lane i of every wavefront holds item i's (m, l, level), the maximum and the
+    // nothing crosses wavefronts: lane i of every wavefront holds item i's (m, l; l < 0: exact rows), the maximum and the
     // normaliser come from wave reductions, and the weight of the item a wavefront is adding (the same item for the
     // whole wavefront) is read from its lane.  Every wavefront thus repeats the few scalars and no barrier is needed.
     float M = -INFINITY, L = 0.0f, arot = 0.0f, aex = 0.0f;

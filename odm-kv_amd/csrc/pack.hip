@@ -1372,8 +1372,8 @@ __device__ static __forceinline__ int find_run(const int* base, int n_runs, int 
 __device__ static __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // What bounds it: two wavefronts a SIMD that wait for memory two fifths of their time (256 matrix instructions and 1900 vector ones a
-// tile, 22 % and 43 % of their pipes).  us a layer with its rows cold: 32k tokens of 8 heads, 2 bits, fp16 95 -> 75; 131k tokens of bf16 at 2 to 4
-// bits, 40 % evicted, 241 -> 202; two sequences of 777 tokens, a tile a wavefront, 33 -> 24.5.  The registers are full: three wavefronts a
+// tile, 22 % and 43 % of their pipes).  us a layer with its rows cold: 32k tokens of 8 heads, 2 bits, fp16 95 -> 75, 72 with the
+// guard band of today; 131k tokens of bf16 at 2 to 4 bits, 40 % evicted, 241 -> 202, 167 with that band (a quarter of the listed values); two sequences of 777 tokens, a tile a wavefront, 33 -> 24.5.  The registers are full: three wavefronts a
 // SIMD (168 a lane), or the next rows requested ahead of the coding, leave 90 to 210 of them in scratch memory, whose
 // reads wait behind the rows: 96 to 104 us.
 // Per wave: a tile's positions are looked up a tile ahead and its rows requested as soon as the registers are free.  ready() is

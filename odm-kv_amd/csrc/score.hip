@@ -4,7 +4,7 @@
 // |v - obar|^2, which is computed directly rather than expanded, to avoid cancellation).
 // A row of 128 elements is handled by 16 lanes x 8 elements, so a wavefront reads four rows
 // (1 KB contiguous for a dense cache) per load instruction.  All reductions run in a fixed
-// order (shuffle butterflies, then ordered sums over chunk partials): results do not depend
+// order (butterflies inside a wavefront, then ordered sums over chunk partials): results do not depend
 // on scheduling.
 #include <algorithm>
 #include "common.h"
