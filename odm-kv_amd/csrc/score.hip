@@ -274,7 +274,7 @@ __device__ static __forceinline__ float sc_scatter2(float (&v)[4], int lane) {
 }
 
 template <int DT, int GMAX>
-__global__ __launch_bounds__(256) void score_logits16_kernel(ScoreArgs a) {
+__global__ __launch_bounds__(256, 4) void score_logits16_kernel(ScoreArgs a) {
     static_assert(DT == ODMKV_F16 || DT == ODMKV_BF16, "16-bit keys");
     static_assert(ROWS_PER_WG == 256, "four waves of 64 tokens");
     constexpr int NP = DT == ODMKV_F16 ? 2 : 3;     // 16-bit pieces of a mean query
