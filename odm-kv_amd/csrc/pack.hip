@@ -2077,7 +2077,9 @@ struct DequantArgs {
 #define DQ_CB_WORDS CODEBOOK_FLOATS
 #define DQ_MAX_RUNS 1024                 // (level, segment) pairs whose tile counts fit the walk table
 // LDS: Pi^T (hi, lo) | per-wave codes | centroids (fp16 hi | lo << 16) | norms | row offsets | walk table
-#define DQ_LDS (QP_PI_BYTES + DQ_NW * QP_STAGE + DQ_CB_WORDS * 4 + DQ_NW * TILE * (4 + 8) + (DQ_MAX_RUNS + 1) * 4)
+#define DQ_PAIRS (16 + 64 + 256)         // pairs of codes of 2, 3 and 4 bits
+#define DQ_PAIR_ROW 80                   // LDS bytes of a token's 64 pairs (16-byte pieces; 16 rows' pieces fall on different banks)
+#define DQ_LDS (QP_PI_BYTES + DQ_NW * QP_STAGE + DQ_CB_WORDS * 4 + DQ_NW * TILE * (4 + 8) + DQ_PAIRS * 8 + (DQ_MAX_RUNS + 1) * 4)
 
 // Pi^T as the A operands of dq_tile, hi then lo: lane 16 q + r of block (jb, ch) holds Pi[32 ch + 8 q .. + 7][j] of the
 // output j = 32 (jb >> 1) + 8 (r >> 2) + 4 (jb & 1) + (r & 3): a lane's accumulators of two neighbouring blocks are then
@@ -2119,18 +2121,10 @@ __device__ static inline uint32_t dq_centroid(float c) {
     return (uint32_t)h | ((uint32_t)Elem<ODMKV_F16>::from_f32(c - Elem<ODMKV_F16>::to_f32(h)) << 16);
 }
 
-// One tile of 64 tokens: codes one byte each [token][dim] in LDS (rows of CODE_ROW), cb the width's centroids, offs the
-// element offset of every token's row in `out` (-1: none).
-// Every operand of Pi^T is read once for all four token blocks (64 KB of LDS reads per tile; with a read per block, 256 KB,
-// the LDS pipe and the latency of its reads set the time), whose four accumulators are chains of their own; a lane stores 16
-// bytes of a row at a time, a token's four lanes 64.  A 2-bit layer of 32k tokens and 8 heads (both tensors): 81 -> 39 us
-// repeated on one layer, 66 us where the rows come from memory (the layers of a prefill, one after the other); 59 with a tile's codes
-// requested under the products of the tile before it (18 us instead of 24 for a tile a wavefront).
-template <int DT, int UP>
-__device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* codes, const uint32_t* cb, const float* norms,
-                                               const long long* offs, void* out, int lane) {
+// The centroids of a tile's 64 tokens as B operands: lane (r16, q) holds those of codes 32 ch + 8 q .. + 7 of token 16 tb + r16,
+// high terms in bh, low ones in bl.  Codes one byte each [token][dim] in LDS (rows of CODE_ROW), cb the width's centroids ...
+__device__ static __forceinline__ void dq_centroids(const uint8_t* codes, const uint32_t* cb, uint4 (&bh)[4][4], uint4 (&bl)[4][4], int lane) {
     const int r16 = lane & 15, q = lane >> 4;
-    uint4 bh[4][4], bl[4][4];                                 // B: the centroids of the token's codes 32 ch + 8 q .. + 7
 #pragma unroll
     for (int tb = 0; tb < 4; ++tb)
 #pragma unroll
@@ -2145,6 +2139,33 @@ __device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* 
             bl[tb][ch] = make_uint4(__builtin_amdgcn_perm(t[1], t[0], 0x07060302u), __builtin_amdgcn_perm(t[3], t[2], 0x07060302u),
                                     __builtin_amdgcn_perm(t[5], t[4], 0x07060302u), __builtin_amdgcn_perm(t[7], t[6], 0x07060302u));
         }
+}
+// ... or (2 to 4 bits) a byte for two codes (rows of DQ_PAIR_ROW), looked up in a table of pairs: half the look-ups and nothing
+// to put together.  With a byte a code, 128 look-ups, 128 permutations and (values) 128 single-byte writes a lane, a 2-bit layer of 32k
+// tokens and 8 heads took 59.3 us, so 57.8; the results are the same to the bit.
+__device__ static __forceinline__ void dq_centroid_pairs(const uint8_t* codes, const uint2* pairs, uint4 (&bh)[4][4], uint4 (&bl)[4][4], int lane) {
+    const int r16 = lane & 15, q = lane >> 4;
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch) {
+            const uint32_t v = *reinterpret_cast<const uint32_t*>(&codes[(16 * tb + r16) * DQ_PAIR_ROW + 16 * ch + 4 * q]);
+            const uint2 c0 = pairs[v & 0xffu], c1 = pairs[(v >> 8) & 0xffu], c2 = pairs[(v >> 16) & 0xffu], c3 = pairs[v >> 24];
+            bh[tb][ch] = make_uint4(c0.x, c1.x, c2.x, c3.x);
+            bl[tb][ch] = make_uint4(c0.y, c1.y, c2.y, c3.y);
+        }
+}
+
+// One tile of 64 tokens from its operands, offs the element offset of every token's row in `out` (-1: none).
+// Every operand of Pi^T is read once for all four token blocks (64 KB of LDS reads per tile; with a read per block, 256 KB,
+// the LDS pipe and the latency of its reads set the time), whose four accumulators are chains of their own; a lane stores 16
+// bytes of a row at a time, a token's four lanes 64.  A 2-bit layer of 32k tokens and 8 heads (both tensors): 81 -> 39 us
+// repeated on one layer, 66 us where the rows come from memory (the layers of a prefill, one after the other); 59 with a tile's codes
+// requested under the products of the tile before it (18 us instead of 24 for a tile a wavefront).
+template <int DT, int UP>
+__device__ static __forceinline__ void dq_tile(const uint4* piA, const uint4 (&bh)[4][4], const uint4 (&bl)[4][4], const float* norms,
+                                               const long long* offs, void* out, int lane) {
+    const int r16 = lane & 15, q = lane >> 4;
 #pragma unroll 1
     for (int jp = 0; jp < 4; ++jp) {                          // outputs 32 jp .. + 31
         qf_f4 acc[2][4];
@@ -2179,23 +2200,18 @@ __device__ static __forceinline__ void dq_tile(const uint4* piA, const uint8_t* 
     }
 }
 
-// the tile's codes of width W -> one byte each in LDS, [token][dim]: the matrix operand wants eight consecutive dims of a
+// the tile's 8-bit codes -> one byte each in LDS, [token][dim]: the matrix operand wants eight consecutive dims of a
 // token per lane, the tile keeps (4 tokens x 32 dims) of keys or (16 tokens x 8 dims) of values per lane
-template <int W>
-__device__ static __forceinline__ void dq_unpack(const uint4 (&raw)[8], bool is_v, uint8_t* codes, int lane) {
+__device__ static __forceinline__ void dq_unpack_bytes(const uint4 (&raw)[8], bool is_v, uint8_t* codes, int lane) {
     const int n = lane & 15, j = lane >> 4;
-    uint32_t words[4 * W];
+    uint32_t words[32];
 #pragma unroll
-    for (int c = 0; c < W; ++c) { words[4 * c] = raw[c].x; words[4 * c + 1] = raw[c].y; words[4 * c + 2] = raw[c].z; words[4 * c + 3] = raw[c].w; }
+    for (int c = 0; c < 8; ++c) { words[4 * c] = raw[c].x; words[4 * c + 1] = raw[c].y; words[4 * c + 2] = raw[c].z; words[4 * c + 3] = raw[c].w; }
     if (!is_v) {
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
-            for (int i = 0; i < 32; i += 4) {
-                const uint32_t w4 = get_code<W>(words, 32 * b + i) | (get_code<W>(words, 32 * b + i + 1) << 8) |
-                                    (get_code<W>(words, 32 * b + i + 2) << 16) | (get_code<W>(words, 32 * b + i + 3) << 24);
-                *reinterpret_cast<uint32_t*>(&codes[key_slot(n, b) * CODE_ROW + 32 * j + i]) = w4;
-            }
+            for (int i = 0; i < 32; i += 4) *reinterpret_cast<uint32_t*>(&codes[key_slot(n, b) * CODE_ROW + 32 * j + i]) = words[8 * b + i / 4];
     } else {
 #pragma unroll
         for (int k = 0; k < 2; ++k)
@@ -2203,7 +2219,64 @@ __device__ static __forceinline__ void dq_unpack(const uint4 (&raw)[8], bool is_
             for (int m = 0; m < 8; ++m)
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    codes[(32 * k + 8 * j + e) * CODE_ROW + 16 * m + n] = (uint8_t)get_code<W>(words, 64 * k + 8 * m + e);
+                    codes[(32 * k + 8 * j + e) * CODE_ROW + 16 * m + n] = (uint8_t)get_code<8>(words, 64 * k + 8 * m + e);
+    }
+}
+
+// the tile's codes of width W -> a byte for the codes of dims 2 i and 2 i + 1, [token][i]: keys hold a token's 32 dims a lane; of values, lane n
+// holds eight tokens of dim n, so neighbours exchange words, the even one making the bytes of the first four tokens, the odd one those of the others
+template <int W>
+__device__ static __forceinline__ void dq_unpack_pairs(const uint4 (&raw)[8], bool is_v, uint8_t* codes, int lane) {
+    static_assert(W <= 4, "two codes a byte");
+    const int n = lane & 15, j = lane >> 4;
+    uint32_t words[4 * W + 1];
+#pragma unroll
+    for (int c = 0; c < W; ++c) { words[4 * c] = raw[c].x; words[4 * c + 1] = raw[c].y; words[4 * c + 2] = raw[c].z; words[4 * c + 3] = raw[c].w; }
+    words[4 * W] = 0u;
+    constexpr uint32_t M2 = (1u << (2 * W)) - 1u, M1 = (1u << W) - 1u;
+    if (!is_v) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            uint32_t o[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {                      // eight codes: 8 W bits
+                const int at = (32 * b + 8 * k) * W;
+                if constexpr (W == 4) {
+                    o[k] = words[at >> 5];
+                } else {
+                    const uint32_t x = __builtin_amdgcn_alignbit(words[(at >> 5) + 1], words[at >> 5], at & 31);
+                    o[k] = (x & M2) | ((x & (M2 << (2 * W))) << (8 - 2 * W)) | ((x & (M2 << (4 * W))) << (16 - 4 * W)) | ((x & (M2 << (6 * W))) << (24 - 6 * W));
+                }
+            }
+            *reinterpret_cast<uint4*>(&codes[key_slot(n, b) * DQ_PAIR_ROW + 16 * j]) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+    } else {
+        const bool odd = (n & 1) != 0;
+        uint32_t even[4 * W + 1], other[4 * W + 1];            // the even dim's words and the odd one's
+#pragma unroll
+        for (int c = 0; c < 4 * W; ++c) {
+            const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)words[c], 0xB1, 0xf, 0xf, false);       // lane ^ 1
+            even[c] = odd ? y : words[c]; other[c] = odd ? words[c] : y;
+        }
+        even[4 * W] = other[4 * W] = 0u;
+        const uint32_t shift = odd ? 4 * W : 0;                // (the four tokens' codes to the front)
+#pragma unroll
+        for (int c = 0; c < 4 * W; ++c) {
+            even[c] = __builtin_amdgcn_alignbit(even[c + 1], even[c], shift);
+            other[c] = __builtin_amdgcn_alignbit(other[c + 1], other[c], shift);
+        }
+        uint8_t* to = codes + (8 * j + (odd ? 4 : 0)) * DQ_PAIR_ROW + (n >> 1);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int m = 0; m < 8; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int at = (64 * k + 8 * m + e) * W, c = at >> 5, r = at & 31;
+                    const uint32_t x = r + W > 32 ? __builtin_amdgcn_alignbit(even[c + 1], even[c], r) : even[c] >> r;
+                    const uint32_t y = r + W > 32 ? __builtin_amdgcn_alignbit(other[c + 1], other[c], r) : other[c] >> r;
+                    to[(32 * k + e) * DQ_PAIR_ROW + 8 * m] = (uint8_t)((x & M1) | ((y & M1) << W));
+                }
     }
 }
 
@@ -2216,7 +2289,8 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
     uint32_t* cb = reinterpret_cast<uint32_t*>(smem + QP_PI_BYTES + DQ_NW * QP_STAGE);
     float* norms = reinterpret_cast<float*>(cb + DQ_CB_WORDS) + wave * TILE;      // [DQ_NW][64] norm of the wave's tokens
     long long* offs = reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + wave * TILE;   // element offset of the row, -1: none
-    int* wbase = reinterpret_cast<int*>(reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + DQ_NW * TILE);
+    uint2* pairs = reinterpret_cast<uint2*>(reinterpret_cast<long long*>(cb + DQ_CB_WORDS + DQ_NW * TILE) + DQ_NW * TILE);      // 2, 3, 4 bits
+    int* wbase = reinterpret_cast<int*>(pairs + DQ_PAIRS);
     const bool is_v = (blockIdx.x & 1) != 0;
     // running count of the tiles that hold tokens over the (level, segment) pairs, so that the waves share out those alone
     const int n_runs = ODMKV_NQ * a.nseg;
@@ -2228,6 +2302,10 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
     dq_request_rotation(is_v ? a.pi_v : a.pi_k, rotation, tid);
     static_assert(DQ_CB_WORDS <= DQ_NW * 64, "a centroid per thread");
     const float centroid = tid < CODEBOOK_FLOATS ? a.cb[tid] : 0.0f;
+    static_assert(DQ_PAIRS <= DQ_NW * 64, "a pair per thread");
+    const int pw = tid < 16 ? 2 : tid < 80 ? 3 : 4, pe = tid < 16 ? tid : tid < 80 ? tid - 16 : tid < DQ_PAIRS ? tid - 80 : 0;
+    const float* pc = a.cb + (pw == 2 ? 0 : pw == 3 ? 4 : 12);
+    const float pair0 = pc[pe & ((1 << pw) - 1)], pair1 = pc[pe >> pw];
     __syncthreads();
     if (table && wave == 0) {                                  // 16 entries per lane, a scan over the lanes' totals
         int mine[DQ_MAX_RUNS / 64], tot = 0;
@@ -2292,20 +2370,27 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_kernel(DequantArgs a) {
     int wi = next_tile(wave * n_wg + (blockIdx.x >> 1));         // (a round of tiles goes over the workgroups first)
     dq_lay_out_rotation<0>(rotation, reinterpret_cast<uint4*>(smem), tid);
     if (tid < DQ_CB_WORDS) cb[tid] = dq_centroid<0>(centroid);
+    if (tid < DQ_PAIRS) {
+        const uint32_t p0 = dq_centroid<0>(pair0), p1 = dq_centroid<0>(pair1);
+        pairs[tid] = make_uint2((p0 & 0xffffu) | (p1 << 16), (p0 >> 16) | (p1 & 0xffff0000u));
+    }
     __syncthreads();
     while (wi < total) {
         offs[lane] = off;
         norms[lane] = norm;
         switch (li) {
-            case 0: dq_unpack<2>(raw, is_v, codes, lane); break;
-            case 1: dq_unpack<3>(raw, is_v, codes, lane); break;
-            case 2: dq_unpack<4>(raw, is_v, codes, lane); break;
-            default: dq_unpack<8>(raw, is_v, codes, lane); break;
+            case 0: dq_unpack_pairs<2>(raw, is_v, codes, lane); break;
+            case 1: dq_unpack_pairs<3>(raw, is_v, codes, lane); break;
+            case 2: dq_unpack_pairs<4>(raw, is_v, codes, lane); break;
+            default: dq_unpack_bytes(raw, is_v, codes, lane); break;
         }
         wave_lds_fence();
-        const uint32_t* table_of = cb + codebook_offset(li);
+        const int level = li;
         wi = next_tile(wi + stride);                             // (under way while this one is multiplied)
-        dq_tile<DT, 0>(piA, codes, table_of, norms, offs, out, lane);
+        uint4 bh[4][4], bl[4][4];
+        if (level == 3) dq_centroids(codes, cb + codebook_offset(3), bh, bl, lane);
+        else dq_centroid_pairs(codes, pairs + (level == 0 ? 0 : level == 1 ? 16 : 80), bh, bl, lane);
+        dq_tile<DT, 0>(piA, bh, bl, norms, offs, out, lane);
         wave_lds_fence();                                        // offs / norms / codes free for the next tile
     }
 }
@@ -2609,7 +2694,9 @@ __global__ __launch_bounds__(DQ_NW * 64) void dequant_rows_f16_kernel(RowsArgs a
         wave_lds_fence();
         tile += stride;
         if (tile < tiles) request(tile);                         // (under way while this one is multiplied)
-        dq_tile<DT, DQ_UP>(reinterpret_cast<const uint4*>(smem), codes, cb, norms, offs, j.out, lane);
+        uint4 bh[4][4], bl[4][4];
+        dq_centroids(codes, cb, bh, bl, lane);
+        dq_tile<DT, DQ_UP>(reinterpret_cast<const uint4*>(smem), bh, bl, norms, offs, j.out, lane);
         wave_lds_fence();
     }
 }

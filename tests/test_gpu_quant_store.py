@@ -107,6 +107,29 @@ def _ulp_close_fp16(a: torch.Tensor, b: torch.Tensor, max_ulp=1, max_frac=0.02, 
     assert float((d > 0).float().mean()) <= max_frac
 
 
+@pytest.mark.parametrize("width", [2, 3, 4, 8])
+@pytest.mark.parametrize("B,H,T", [(1, 1, 1), (1, 2, 64), (2, 1, 65), (1, 3, 197), (70, 8, 33)])
+def test_materialize_of_one_width_against_fp64(width, B, H, T):
+    """Against fp64 rows from the codes and norms that the store holds.  The fp16 pairs are whole to 2^-25 (centroids) and 2^-25
+    (rotation), each next to factors whose magnitudes add up to at most sqrt(128): 3.4e-7 of the norm either; lo * lo is left out,
+    2^-22; the fp32 sums stay below 1e-7: less than 1.1e-6 together.  (70 x 8 pairs: more runs than the walk's table holds.)"""
+    from packed_layout import decode_level
+    from kvquant.tq_backend import _load_or_compute_codebook
+    g = torch.Generator().manual_seed(T * 10 + width)
+    k = torch.randn(B, H, T, 128, generator=g).half(); v = (torch.randn(B, H, T, 128, generator=g) * 3).half()
+    state = _state()
+    state.prefill(k.to(DEV), v.to(DEV), torch.full((B, H, T), width, device=DEV))
+    got = decode_level(state, (2, 3, 4, 8).index(width))
+    c = _load_or_compute_codebook(width, 128, "cpu", torch.float32).double()
+    at = (torch.as_tensor(got["bh"]).long(), torch.as_tensor(got["pos"]).long())
+    for out, codes, norm, pi in zip(state.materialize(torch.float32), (got["kcodes"], got["vcodes"]), (got["knorm"], got["vnorm"]),
+                                    (state.pi_k, state.pi_v)):
+        n = torch.as_tensor(np.asarray(norm)).double()[:, None]
+        want = c[torch.as_tensor(np.asarray(codes)).long()] @ pi.cpu().double() * n
+        err = (out.cpu().double().view(B * H, T, 128)[at] - want).abs() / n
+        assert len(n) == B * H * T and float(err.max()) < 1.1e-6
+
+
 @pytest.mark.parametrize("B,H,T", [(1, 2, 300), (2, 3, 129), (1, 8, 1000)])
 def test_prefill_codes_positions_and_materialize(B, H, T):
     g = torch.Generator().manual_seed(B * 1000 + T)
