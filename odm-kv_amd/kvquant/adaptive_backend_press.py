@@ -236,7 +236,7 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
                 groups.append([dev, T, tail, []])
             groups[-1][3].append(bits)
             order.append(layer_idx)
-        evicted = []                # per group: level maps of its layers
+        evicted = []                # per group: level maps of its layers, tokens, where it begins in the plan
         try:
             for dev, T, tail, members in groups:
                 # one pass over the levels: bulk shares counted, the window (or the whole layer) set to 16, the level map
@@ -252,8 +252,8 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
                                                             counts.data_ptr(), _lib.stream_ptr(dev)))
                     ev = arrived.setdefault(dev, torch.cuda.Event())
                     ev.record(torch.cuda.current_stream(dev))
+                evicted.append((levels, T, len(plan)))
                 plan.extend(zip(order[len(plan):], members, levels, counts))
-                evicted.append((levels, T))
             for layer_idx, *_ in plan:                            # (the host's part while the counts are on their way)
                 self._get_or_create_state(layer_idx, self._get_cache_tensors(cache, layer_idx)[0])
         finally:
@@ -261,33 +261,32 @@ class TurboQuantPerTokenBackendPress(TurboQuantPerTokenPress):
             for ev in arrived.values():
                 ev.synchronize()
         totals = [counts.numpy().sum(axis=1).swapaxes(0, 1) for *_, counts in plan]      # (bulk, stored) of every layer
-        # The GPU has run dry while the counts were on their way: the quantisers first, what only the host needs behind everything that is launched
-        states = []
-        for (layer_idx, bits, levels, _), (_, stored) in zip(plan, totals):
-            keys, values = self._get_cache_tensors(cache, layer_idx)
-            states.append(self._get_or_create_state(layer_idx, keys))
-            states[-1].prefill(keys, values, bits, _known_counts=stored, _levels=levels)
-        masked, at = [], 0
-        for levels, T in evicted:
-            masked += evicted_indices(levels, T, [int(stored[:, 0].sum()) for _, stored in totals[at:at + len(levels)]])
-            at += len(levels)
-        for (layer_idx, *_), state, gone in zip(plan, states, masked):
-            keys, _ = self._get_cache_tensors(cache, layer_idx)
-            state.adopt_masked(gone)
-            module = self._layer_modules.get(layer_idx)
-            if module is not None:
-                if self.release_dense_cache and layer_idx >= self.initial_layers_fp16:
-                    self._release_dense(cache, layer_idx, state)
-                self._sync_cache_from_state(cache, layer_idx, module, state, prefill_fast=True)
-            if self.buffer_size > 0:
-                self._buffer_start_seqs[layer_idx] = int(keys.shape[2])
-                self._buffer_counts[layer_idx] = 0
-            if self._last_hooked_layer_idx is None or layer_idx == self._last_hooked_layer_idx:
-                release_staging(keys.device)             # the prompt is stored: worst-case stores that direct fills left can go
         wanted = sorted(set(int(b) for b in self.bit_levels) | {16})
         columns = [_lib.LEVEL_ORDER.index(b) for b in wanted]
-        for (layer_idx, bits, *_), (bulk, _) in zip(plan, totals):
-            self._store_observed_ratios(layer_idx, bits.shape[1], wanted, bulk[:, columns])
+        # One layer is finished before the next is stored: with the dense copy released its memory is the next store's, and what
+        # cannot be stored leaves the layers before it whole.  (The GPU has run dry while the counts were on their way: a layer's
+        # quantiser goes first, the lists of evicted positions and the shares of the levels, which only the host needs, behind it.)
+        for levels, T, first in evicted:
+            masked = None
+            members = zip(plan[first:first + len(levels)], totals[first:first + len(levels)])
+            for i, ((layer_idx, bits, level_map, _), (bulk, stored)) in enumerate(members):
+                keys, values = self._get_cache_tensors(cache, layer_idx)
+                state = self._get_or_create_state(layer_idx, keys)
+                state.prefill(keys, values, bits, _known_counts=stored, _levels=level_map)
+                if masked is None:
+                    masked = evicted_indices(levels, T, [int(s[:, 0].sum()) for _, s in totals[first:first + len(levels)]])
+                state.adopt_masked(masked[i])
+                module = self._layer_modules.get(layer_idx)
+                if module is not None:
+                    if self.release_dense_cache and layer_idx >= self.initial_layers_fp16:
+                        self._release_dense(cache, layer_idx, state)
+                    self._sync_cache_from_state(cache, layer_idx, module, state, prefill_fast=True)
+                if self.buffer_size > 0:
+                    self._buffer_start_seqs[layer_idx] = int(keys.shape[2])
+                    self._buffer_counts[layer_idx] = 0
+                self._store_observed_ratios(layer_idx, bits.shape[1], wanted, bulk[:, columns])
+                if self._last_hooked_layer_idx is None or layer_idx == self._last_hooked_layer_idx:
+                    release_staging(keys.device)         # the prompt is stored: worst-case stores that direct fills left can go
         self._reset_prefill_state()
 
     # ------------------------------------------------------------------ hook

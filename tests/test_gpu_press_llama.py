@@ -520,3 +520,50 @@ def test_question_block_takes_the_fused_path(release):
     assert fused.shape == (n_q, 1000)
     assert (fused - dense).abs().max().item() < LOGIT_ATOL
     assert (fused_next - dense_next).abs().max().item() < LOGIT_ATOL
+
+
+@torch.inference_mode()
+@pytest.mark.parametrize("release", [False, True])
+@pytest.mark.parametrize("failing", [None, 2])
+def test_a_prompt_stored_in_one_go_finishes_every_layer_before_the_next(monkeypatch, release, failing):
+    """layerwise=False: all layers are stored behind the last one's hook.  Each is attached, given its evicted positions and
+    (released) rid of its dense copy before the next one's store is made: the memory in use falls by what a layer's packed
+    store is smaller than its dense tensors, and a layer that cannot be stored leaves those before it whole."""
+    from transformers import DynamicCache
+    from kvquant.tq_adaptive_backend import TurboQuantAdaptiveKVCacheState
+    model, ids, T = _model(9, layers=3), _ids(2048, 61), 2048
+    attn = [block.self_attn for block in model.model.layers]
+    press, cache = _press(target=1.7, release_dense_cache=release), DynamicCache()
+    press.layerwise = False
+    dense, seen = 2 * 2 * T * 128 * 2, []
+    store = TurboQuantAdaptiveKVCacheState.prefill
+
+    def spy(state, *args, **kw):
+        layer = len(seen)
+        seen.append((state, torch.cuda.memory_allocated()))
+        for l, (earlier, _) in enumerate(seen[:-1]):
+            assert attn[l].__dict__["_odmkv_state"] is earlier and cache.layers[l]._tq_backend_state is earlier
+            assert type(cache.layers[l]).__name__ == ("PackedCacheLayer" if release else "DynamicLayer")
+            assert press._buffer_start_seqs[l] == T and press._buffer_counts[l] == 0
+            gone = int((earlier._level_map == 0).sum())
+            assert gone > 0 and len(attn[l].masked_key_indices) == 3 and attn[l].masked_key_indices[0].numel() == gone
+            assert all((l, h) in press._observed_ratios for h in range(2))
+        if layer == failing:
+            raise MemoryError("no room for this layer's store")
+        return store(state, *args, **kw)
+
+    monkeypatch.setattr(TurboQuantAdaptiveKVCacheState, "prefill", spy)
+    model.model(input_ids=ids, past_key_values=DynamicCache())            # (the library's own workspaces)
+    with press(model):
+        if failing is None:
+            model.model(input_ids=ids, past_key_values=cache)
+        else:
+            with pytest.raises(MemoryError):
+                model.model(input_ids=ids, past_key_values=cache)
+            assert attn[failing].__dict__.get("_odmkv_state") is None and type(cache.layers[failing]).__name__ == "DynamicLayer"
+    assert len(seen) == 3
+    if release:
+        # what a layer keeps beside its arena: the newest token's rows, the evicted positions (24 bytes each), blocks of 512 bytes
+        for (state, before), (_, after) in zip(seen, seen[1:]):
+            kept = state._arena.numel() + 24 * int((state._level_map == 0).sum()) + (64 << 10)
+            assert after <= before - dense + kept, (before, after, dense, kept)
