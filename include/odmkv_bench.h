@@ -44,6 +44,11 @@ int odmkv_bench_probe_read(const void* buf, size_t bytes, int grid, void* sink, 
  * its list holds).  counts: host int32[2].  Waits for the stream. */
 int odmkv_bench_pack_handed_over(const void* workspace, int B, int Hkv, int T, int32_t* counts, void* stream);
 
+/* What the quantiser's guard band rests on: n instructions v_mfma_f32_16x16x32_{f16,bf16}, each D[16][16] = C[16][16] plus the
+ * products of A's rows [16][32] and B's rows [16][32] (16-bit, contiguous, 16-byte aligned; C and D fp32).  dtype: ODMKV_F16 or
+ * ODMKV_BF16. */
+int odmkv_bench_probe_products(int dtype, const void* A, const void* B, const float* C, float* D, int64_t n, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

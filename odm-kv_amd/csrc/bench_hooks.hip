@@ -87,3 +87,34 @@ extern "C" int odmkv_bench_pack_handed_over(const void* workspace, int B, int Hk
     ODMKV_CHECK_HIP(hipStreamSynchronize((hipStream_t)stream));
     return 0;
 }
+
+// one matrix instruction a workgroup (a wavefront): D = A . B^T + C over 32 terms
+typedef _Float16 probe_h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 probe_b8 __attribute__((ext_vector_type(8)));
+typedef float probe_f4 __attribute__((ext_vector_type(4)));
+template <int DT>
+__global__ __launch_bounds__(64) void probe_products_kernel(const uint16_t* A, const uint16_t* B, const float* C, float* D) {
+    const int n = threadIdx.x & 15, j = threadIdx.x >> 4;
+    const size_t at = (size_t)blockIdx.x * 16;
+    const uint4 a = *reinterpret_cast<const uint4*>(A + (at + n) * 32 + 8 * j);
+    const uint4 b = *reinterpret_cast<const uint4*>(B + (at + n) * 32 + 8 * j);
+    probe_f4 d;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) d[r] = C[(at + 4 * j + r) * 16 + n];
+    if constexpr (DT == ODMKV_F16)
+        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(probe_h8, a), __builtin_bit_cast(probe_h8, b), d, 0, 0, 0);
+    else
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(probe_b8, a), __builtin_bit_cast(probe_b8, b), d, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) D[(at + 4 * j + r) * 16 + n] = d[r];
+}
+
+extern "C" int odmkv_bench_probe_products(int dtype, const void* A, const void* B, const float* C, float* D, int64_t n, void* stream) {
+    ODMKV_CHECK_ARG(A && B && C && D && n > 0 && n < (1ll << 31), "probe_products: bad arguments");
+    ODMKV_CHECK_ARG(dtype == ODMKV_F16 || dtype == ODMKV_BF16, "probe_products: 16-bit operands only");
+    ODMKV_CHECK_ARG(((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0, "probe_products: operands must be 16-byte aligned");
+    const auto kernel = dtype == ODMKV_F16 ? probe_products_kernel<ODMKV_F16> : probe_products_kernel<ODMKV_BF16>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(64), 0, (hipStream_t)stream, (const uint16_t*)A, (const uint16_t*)B, C, D);
+    ODMKV_CHECK_LAUNCH("probe_products_kernel");
+    return 0;
+}

@@ -899,13 +899,13 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
 // threshold.  So y is first computed fast: the fp16 row as it is, against Pi split into two fp16
 // terms (hi + lo, 22 bits), on v_mfma_f32_16x16x32_f16, then scaled by 1 / (|x| + 1e-10).  That
 // estimate differs from the chain's result by rounding alone.  On the scale |y| <= 1, in which no partial sum exceeds 1 (Cauchy-Schwarz):
-//   the chain        128 roundings to nearest of numbers below 1                                          3.8e-6
-//   the estimate     8 instructions, each off by at most 5.5 units in the last place of its largest term  5.2e-6
-//                    (measured on the instruction: next to a term of 1 a product counts down to 2^-26 and
-//                    is dropped below, so 32 of them lose at most 4 units of 2^-23; 1.6 million random
-//                    sums of either type, 32 products and an addend, were off by 5.3 at the most)
-//   Pi's two terms (2^-25 an element at the least), 1 / |x| and the product with it                       0.6e-6
-// together 9.6e-6.  Measured, a band of 1e-7 already leaves no code
+//   the chain        128 roundings to nearest of numbers below 1                                                                3.8e-6
+//   the estimate     The instruction adds eight products after eight to the sum, and each time the nine terms lose at most 2^-24 of
+//                    the largest product or 2^-26 of the sum and the new sum is rounded to nearest (measured, and held by a test of
+//                    the instruction alone).  32 times, of a sum of at most 1: 32 (9 * 2^-26 + 2^-24)                           6.2e-6
+//                    and of the largest products, which add up to at most 1: 9 * 2^-24                                         0.5e-6
+//   Pi's two terms (2^-25 an element at the least), 1 / |x|, the product with it and the chain's quotients                       0.6e-6
+// together 11.1e-6.  Measured, a band of 1e-7 already leaves no code
 // different over 1e8 values.  Values farther than QF_BAND from every threshold therefore have the chain's code already; the few within the band
 // (a half to two in a thousand) are listed, and whenever a wave has 64 of them it recomputes them by
 // the chain itself, one lane per value, and replaces their codes in the packed tiles it has already

@@ -499,3 +499,75 @@ def test_lloyd_max_on_the_device_gives_the_reference_tables(golden, bits):
     out = torch.empty(512, dtype=torch.float64, device=DEV)
     assert _lib.lib.odmkv_lloyd_max(512, 128, 500, 1e-10, 5.0, out.data_ptr(), None, None) == -1
     assert _lib.lib.odmkv_lloyd_max(4, 64, 500, 1e-10, 5.0, out.data_ptr(), None, None) == -1
+
+
+def _products(A, B, C):
+    """n instructions: C + A . B^T, [n, 16, 32] and [n, 16, 32] of a 16-bit type, [n, 16, 16] fp32."""
+    import ctypes
+    import os
+    from kvquant import _lib
+    blib = ctypes.CDLL(os.path.join(os.path.dirname(_lib.__file__), "..", "lib", "libodmkv_bench.so"))
+    A, B, C = (t.contiguous() for t in (A, B, C))
+    n = A.shape[0]
+    assert A.shape == B.shape == (n, 16, 32) and C.shape == (n, 16, 16) and C.dtype == torch.float32 and A.dtype == B.dtype
+    out = torch.empty_like(C)
+    vp = ctypes.c_void_p
+    blib.odmkv_bench_probe_products.argtypes = [ctypes.c_int, vp, vp, vp, vp, ctypes.c_int64, vp]
+    rc = blib.odmkv_bench_probe_products(_lib.dtype_code(A), A.data_ptr(), B.data_ptr(), C.data_ptr(), out.data_ptr(), n, _lib.stream_ptr(A.device))
+    assert rc == 0
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kind", ["beside one product", "beside the sum", "of one sign", "of many sizes", "cancelling", "below the normal numbers"])
+def test_the_matrix_instruction_rounds_as_the_guard_band_assumes(kind, dtype):
+    """What pack.hip's guard band is derived from.  v_mfma_f32_16x16x32_{f16,bf16} adds eight products after eight to the sum; each time
+    the nine terms lose at most 2^-24 of the largest product or 2^-26 of the sum, and the new sum is rounded to nearest:
+    9 (2^-24 P + 2^-26 |sum|) + 2^-24 |new sum|, an operand below the type's normal numbers counting as the smallest of them in P."""
+    g = torch.Generator(device=DEV).manual_seed(len(kind))
+    bits, least = (10, 2.0 ** -14) if dtype == torch.float16 else (7, 2.0 ** -126)
+    n = 256
+
+    def ints(lo, hi, *shape):
+        return torch.randint(lo, hi, shape, generator=g, device=DEV).float()
+
+    def mantissas(largest):                                       # (the largest lose most where they are cut)
+        return torch.full((n, 16, 32), 2 - 2.0 ** -bits, device=DEV) if largest else 1 + ints(0, 2 ** bits, n, 16, 32) / 2 ** bits
+
+    worst = 0.0
+    for turn in range(96):
+        A, B, C = mantissas(turn % 3 == 0), mantissas(turn % 6 == 0), torch.zeros(n, 16, 16, device=DEV)
+        if kind in ("beside one product", "beside the sum", "of one sign"):
+            e = ints(20, 30, n, 1, 32) if turn % 2 else ints(22, 29, n, 1, 1).expand(n, 1, 32)
+            if kind == "of one sign":                             # under 2^-24 in the large product's eight, under 2^-26 behind it
+                e = torch.where(torch.arange(32, device=DEV) // 8 == turn % 4, 25.0, 27.0).expand(n, 1, 32)
+            A, B = A * 2.0 ** -(e / 2).floor(), B * 2.0 ** -(e - (e / 2).floor())
+            if kind == "beside the sum":
+                C += 1.0 + (torch.rand(C.shape, generator=g, device=DEV) if turn % 4 > 1 else 0.0)
+            else:
+                at = (8 * (turn % 4) + turn // 4) % 32
+                A[:, :, at] = B[:, :, at] = 1.0
+            if kind != "of one sign" and turn % 5 == 1:
+                A *= 2 * ints(0, 2, n, 16, 32) - 1
+            if turn % 5 == 2:
+                C = -C
+        elif kind == "cancelling":
+            A, B = A * 2.0 ** -ints(0, 3, n, 16, 32) * (2 * ints(0, 2, n, 16, 32) - 1), B * 2.0 ** -ints(0, 3, n, 16, 32)
+            C = -(A @ B.transpose(-1, -2))
+        else:
+            A = torch.randn(A.shape, generator=g, device=DEV) * 2.0 ** -ints(0, 13, n, 16, 32)
+            B = torch.randn(B.shape, generator=g, device=DEV) * 2.0 ** -ints(0, 13, n, 16, 32)
+            C = torch.randn(C.shape, generator=g, device=DEV) * 2.0 ** -ints(0, 30, n, 16, 16)
+            if kind == "below the normal numbers":
+                A, C = A * least, C * least
+        A, B = A.to(dtype), B.to(dtype)
+        got, total, bound = _products(A, B, C).double(), C.double(), torch.zeros(n, 16, 16, device=DEV, dtype=torch.float64)
+        for s in range(0, 32, 8):
+            a, b = A[:, :, None, s:s + 8].double(), B[:, None, :, s:s + 8].double()
+            largest = (a.abs().clamp_min(least) * b.abs().clamp_min(least)).amax(-1)
+            bound += 9 * (2.0 ** -24 * largest + 2.0 ** -26 * total.abs())
+            total = total + (a * b).sum(-1)
+            bound += 2.0 ** -24 * total.abs()
+        # fp32's own smallest numbers: sums below 2^-126 may vanish
+        worst = max(worst, float(((got - total).abs() / (bound + 2.0 ** -126)).max()))
+    assert worst <= 1.0, worst
