@@ -905,7 +905,8 @@ __global__ __launch_bounds__(NW * 64) void quant_pack_kernel(QuantArgs a) {
 //                    the instruction alone).  32 times, of a sum of at most 1: 32 (9 * 2^-26 + 2^-24)                           6.2e-6
 //                    and of the largest products, which add up to at most 1: 9 * 2^-24                                         0.5e-6
 //   Pi's two terms (2^-25 an element at the least), 1 / |x|, the product with it and the chain's quotients                       0.6e-6
-// together 11.1e-6.  Measured, a band of 1e-7 already leaves no code
+//   rows of tiny numbers (qf_raise_tiny)                                                                                         0.3e-6
+// together 11.4e-6.  Measured, a band of 1e-7 already leaves no code
 // different over 1e8 values.  Values farther than QF_BAND from every threshold therefore have the chain's code already; the few within the band
 // (a half to two in a thousand) are listed, and whenever a wave has 64 of them it recomputes them by
 // the chain itself, one lane per value, and replaces their codes in the packed tiles it has already
@@ -1095,6 +1096,29 @@ __device__ static __forceinline__ float qf_sum_squares(const QfRows& x, uint32_t
         __builtin_amdgcn_sched_barrier(0);                   // (the copies of one chunk at a time: sixteen registers, not 64)
     }
     return ss;
+}
+
+// fp16 rows of tiny numbers: the matrix instruction takes an operand below 2^-14 for one of 2^-14 when it lines up products, and cuts them up to
+// 36 * 2^-38 from the sum: 2.7e-7 of a norm of 2^-11, but 1.9e-5 seen for elements of 2^-24, more than the guard band.  A row whose norm is below
+// 2^-11 is therefore multiplied by 2^13 in its registers, which is exact, and its estimate's scale by 2^-13.  Returns the scale.
+template <int DT>
+__device__ static __forceinline__ float qf_raise_tiny(QfRows& x, float ss, float rinv, int lane) {
+    if constexpr (DT == ODMKV_F16) {
+        const unsigned long long rows = __ballot(ss > 0.0f && ss < 2.384185791015625e-07f);
+        if (__builtin_expect(rows != 0ull, 0)) {
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+            const auto raise = [](uint32_t w, _Float16 by) { return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w) * by); };
+#pragma unroll
+            for (int tb = 0; tb < 4; ++tb) {
+                const _Float16 by = ((rows >> (16 * tb + (lane & 15))) & 1ull) ? (_Float16)8192.0f : (_Float16)1.0f;
+#pragma unroll
+                for (int ch = 0; ch < 4; ++ch)
+                    x[tb][ch] = make_uint4(raise(x[tb][ch].x, by), raise(x[tb][ch].y, by), raise(x[tb][ch].z, by), raise(x[tb][ch].w, by));
+            }
+            rinv *= ((rows >> lane) & 1ull) ? 1.0f / 8192.0f : 1.0f;
+        }
+    }
+    return rinv;
 }
 
 // Rotation estimate -> codes into the staging area: fields of W bits side by side (DIRECT), or of 4 bits where they have to be moved
@@ -1490,7 +1514,7 @@ __device__ static void qf_walk(const QuantArgs& a, const uint4* piA, const float
             const float den = norm + 1e-10f;
             w.off[ln] = off;
             w.den[ln] = den;
-            w.rinv[ln] = 1.0f / den;
+            w.rinv[ln] = qf_raise_tiny<DT>(xb, ss, 1.0f / den, ln);
             const unsigned long long listed = __ballot(valid && ss > 0.0f);
             wave_lds_fence();
             if (__builtin_expect(!mirror, 0)) {
@@ -2561,7 +2585,7 @@ __device__ static void qr_walk(const RowsJob& j, const uint4* piA, const float* 
             const float den = norm + 1e-10f;
             w.off[lane] = (unsigned long long)off;
             w.den[lane] = den;
-            w.rinv[lane] = 1.0f / den;
+            w.rinv[lane] = qf_raise_tiny<DT>(xb, ss, 1.0f / den, lane);
             const unsigned long long listed = __ballot(valid && ss > 0.0f);
             wave_lds_fence();
             if (mirror) qf_code_tile<DT, W, false, false, true>(xb, piA, thr, w, stage, ln, it, listed);
@@ -2865,7 +2889,7 @@ __device__ static __forceinline__ void rt_walk(const RowsJob& j, const uint4* pi
         const bool ok = !__any(odd);
         w.off[lane] = off;
         w.den[lane] = den;
-        w.rinv[lane] = 1.0f / den;
+        w.rinv[lane] = qf_raise_tiny<DT>(xb, ss, 1.0f / den, lane);
         w.norm[lane] = norm;
         if (lane == 0) w.count = 0;
         const unsigned long long listed = __ballot(lane < rows && ss > 0.0f);

@@ -501,6 +501,24 @@ def test_lloyd_max_on_the_device_gives_the_reference_tables(golden, bits):
     assert _lib.lib.odmkv_lloyd_max(4, 64, 500, 1e-10, 5.0, out.data_ptr(), None, None) == -1
 
 
+def _small_rows(n, seed):
+    """fp16 rows of a few units of 2^-24 an element up to norms of 1e-3: numbers below fp16's normal range (2^-14), whose products the matrix
+    instruction aligns as if they were 2^-14."""
+    g = torch.Generator().manual_seed(seed)
+    scale = torch.logspace(-24, -14, n, base=2.0)[torch.randperm(n, generator=g)]
+    x = torch.randn(n, 128, generator=g) * scale[:, None]
+    x[::5, 8:] = 0.0                                             # few elements: one group of eight holds them
+    return x.half()
+
+
+@pytest.mark.parametrize("width", [2, 3, 4])
+def test_fp16_rows_below_the_normal_numbers(width):
+    """Every code of a row of tiny numbers is the definition's, and the exact kernel is not asked for."""
+    k, v = (_small_rows(2 * 8192, seed).view(1, 2, 8192, 128).to(DEV) for seed in (width, 50 + width))
+    handed = _same_bytes_in_both_types(k, v, torch.full((1, 2, 8192), width, dtype=torch.int32, device=DEV))
+    assert handed == (0, 0)
+
+
 def _products(A, B, C):
     """n instructions: C + A . B^T, [n, 16, 32] and [n, 16, 32] of a 16-bit type, [n, 16, 16] fp32."""
     import ctypes
@@ -571,3 +589,43 @@ def test_the_matrix_instruction_rounds_as_the_guard_band_assumes(kind, dtype):
         # fp32's own smallest numbers: sums below 2^-126 may vanish
         worst = max(worst, float(((got - total).abs() / (bound + 2.0 ** -126)).max()))
     assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_codes_where_the_instruction_cuts_tiny_elements(bits):
+    """Elements of 2^-24 count as 2^-14 where the instruction lines products up: the plain sum over Pi's two fp16 terms is off by up to 2e-5 of
+    such a row's norm.  Thresholds put between a value and that sum, for the values where the two are farthest apart."""
+    from kvquant.tq_backend import TurboQuantMSE
+    steps, tried = torch.arange(1 << bits, dtype=torch.float32) - (1 << bits) / 2 + 0.5, 0
+    for seed in range(42, 58):
+        q = TurboQuantMSE(128, bits, device=DEV, dtype=torch.float16, seed=seed)
+        high = q.pi.half()
+        low = (q.pi - high.float()).half()
+
+        def off(x):
+            """(the plain sum less the value, the value) over the row's norm, [row, output]"""
+            n, sums = x.shape[0] // 16, []
+            for block in range(0, 128, 16):
+                total = torch.zeros(n, 16, 16, device=DEV)
+                for step in range(0, 128, 32):
+                    for term in (high, low):
+                        total = _products(term[block:block + 16, step:step + 32].expand(n, 16, 32), x.view(n, 16, 128)[:, :, step:step + 32], total)
+                sums.append(total.transpose(-1, -2))
+            norm = x.double().norm(dim=-1, keepdim=True) + 1e-10
+            y = x.double() @ q.pi.double().T / norm
+            return torch.cat(sums, dim=-1).reshape(-1, 128).double() / norm - y, y
+
+        one, _ = off((torch.eye(128, device=DEV) * 2.0 ** -24).half())              # of one element [element, output]
+        most = one.abs().topk(8, dim=0).indices
+        for n in range(1, 9):                                                      # the elements that lose most of an output, all the same way
+            x = torch.zeros(128, 128, device=DEV)
+            x.scatter_(1, most[:n].T, one.gather(0, most[:n]).sign().T.float() * 2.0 ** -24)
+            x = x.half()
+            err, y = off(x)
+            for row, at in (err.abs() > 1.25e-5).nonzero().tolist():
+                e, v = float(err[row, at]), float(y[row, at])     # (the band is 1.2e-5; 1e-6 more for a table that mirrors, which this one does not)
+                q.centroids = (v + 0.02 * e + 0.1 * steps).to(DEV)
+                q.centroids[0] -= 0.01
+                assert torch.equal(q.quantize_codes(x)[0], q.quantize_codes(x.float())[0]), (seed, n, row, at, e, v)
+                tried += 1
+    assert tried >= 4

@@ -165,3 +165,24 @@ def test_the_round_trip_is_no_further_from_fp64_than_fp32_sums(bits, heavy, dtyp
         wrong += int((got.view(-1, 128) != exact).sum())
         wrong32 += int((q.dequantize(q.quantize(x.view(-1, 128))).to(dtype) != exact).sum())
     assert wrong <= 1.25 * wrong32
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4])
+def test_codes_of_fp16_rows_below_the_normal_numbers(bits):
+    """Rows of a few units of 2^-24 an element up to norms of 1e-3, outside a store and in the round trip: the definition's codes."""
+    from kvquant import TurboQuantBackendPress
+    n, g = 16384, torch.Generator().manual_seed(bits)
+    x = torch.randn(n, 128, generator=g) * torch.logspace(-24, -14, n, base=2.0)[torch.randperm(n, generator=g)][:, None]
+    x[::5, 8:] = 0.0
+    x = x.half().cuda()
+    press = TurboQuantBackendPress(key_bits=bits, value_bits=bits, value_quantizer="mse")
+    kq, vq = press._q(bits, 42, x), press._q(bits, 2042, x)
+    assert torch.equal(kq.quantize_codes(x)[0], kq.quantize_codes(x.float())[0])
+    k, v = x.view(1, 1, n, 128).clone(), x.view(1, 1, n, 128).clone()
+    press._quantise_span(0, k, v, 0, n)
+    for got, q in ((k, kq), (v, vq)):
+        codes, norms = q.quantize_codes(x.float())
+        want = (q.centroids.double()[codes.long()] @ q.pi.double()) * norms.double()[:, None]
+        # half a unit of fp16's smallest numbers, or a step; another code moves the row by some tenths of a percent of its norm at the least
+        err = (got.view(n, 128).double() - want).abs()
+        assert (err <= 2.0 ** -25 + 2.0 ** -10 * want.abs() + 1e-6 * norms.double()[:, None]).all()
