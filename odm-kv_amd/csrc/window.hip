@@ -58,10 +58,10 @@ __device__ static inline f32x16 win_mfma(uint4 a, uint4 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// merge two (max, sum) pairs kept in base-2 units
+// merge two (max, sum) pairs kept in base-2 units (a maximum of -inf: nothing seen yet, the sum is 0, or NaN where a logit was)
 __device__ static inline void ms2_merge(float& m, float& s, float m2, float s2) {
     const float mn = fmaxf(m, m2);
-    if (mn == -INFINITY) { m = mn; s = 0.0f; return; }
+    if (mn == -INFINITY) { m = mn; s += s2; return; }
     s = s * __builtin_amdgcn_exp2f(m - mn) + s2 * __builtin_amdgcn_exp2f(m2 - mn);
     m = mn;
 }
@@ -90,6 +90,7 @@ __device__ static inline float squares8(const uint4& k) {
 
 // A query's statistics over the tokens that a lane has seen: the sum of exp2(s - ref).  The reference point is the largest s or up to 4 below it (an
 // exponent of that size is still rounded to 2^-22): sixteen tokens whose sum is at most 16 need no maximum, which most have not but the first.
+// A logit that is NaN makes the sum NaN, wherever it comes, and the query then votes for nothing.
 struct QueryStat { float ref, sum; };
 #define WIN_RISE 16.0f
 
@@ -107,10 +108,10 @@ __device__ static inline void fold_products(const f32x16& p, float c, QueryStat&
 #pragma unroll
         for (int r = 0; r < 16; ++r) ref = fmaxf(ref, p[r] * c);
         z = 0.0f;
+        const float by = ref > -INFINITY ? ref : 0.0f;              // (nothing but -inf and NaN: sums to 0 or NaN)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(__fmaf_rn(p[r], c, -ref));
-        if (!(ref > -INFINITY)) z = 0.0f;
-        q.sum = q.ref > -INFINITY ? q.sum * __builtin_amdgcn_exp2f(q.ref - ref) : 0.0f;
+        for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(__fmaf_rn(p[r], c, -by));
+        q.sum *= q.ref > -INFINITY ? __builtin_amdgcn_exp2f(q.ref - ref) : 1.0f;
         q.ref = ref;
     }
     q.sum += z;
@@ -120,11 +121,11 @@ __device__ static inline void fold_masked(const f32x16& s, QueryStat& q) {
     float ref = q.ref;
 #pragma unroll
     for (int r = 0; r < 16; ++r) ref = fmaxf(ref, s[r]);
+    const float by = ref > -INFINITY ? ref : 0.0f;
     float z = 0.0f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(s[r] - ref);
-    if (!(ref > -INFINITY)) z = 0.0f;
-    q.sum = (q.ref > -INFINITY ? q.sum * __builtin_amdgcn_exp2f(q.ref - ref) : 0.0f) + z;
+    for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(s[r] - by);
+    q.sum = __fmaf_rn(q.sum, q.ref > -INFINITY ? __builtin_amdgcn_exp2f(q.ref - ref) : 1.0f, z);
     q.ref = ref;
 }
 

@@ -604,6 +604,31 @@ def test_window_attention_over_its_ways_of_sharing_the_work(hkv, hq, T, W, data,
     assert err < 1e-5, float(err)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lo,hi", [(4, 36), (4, 132), (4, 1030), (300, 301), (640, 800), (966, 1030), (1000, 1003), (1029, 1030)])
+def test_window_attention_over_keys_that_are_not_numbers(lo, hi, dtype):
+    """A query that sees such a key votes for no other token, wherever the key lies: in a lane's first tokens, whole blocks and tiles of them, one, inside
+    the window (the queries ahead of it vote as ever); the other head is untouched."""
+    from kvquant.scorer import _launch_window_attention
+    g = torch.Generator().manual_seed(lo + hi)
+    T, W, n_sink = 1030, 64, 4
+    k = torch.randn(2, T, 128, generator=g).to(dtype)
+    q = (torch.randn(8, W, 128, generator=g) * 1.5).to(dtype)
+    k[0, lo:hi] = float("nan")
+    got = _launch_window_attention(k.to(DEV), q.to(DEV), n_sink, T - W, 128 ** -0.5).cpu().double()
+    nan = torch.zeros(T, dtype=torch.bool)
+    nan[lo:hi] = True
+    logits = (q[:4].double() @ k[0].double().nan_to_num().T * 128 ** -0.5)[..., n_sink:]        # [4, W, T - n_sink]
+    seen = torch.arange(n_sink, T) <= torch.arange(T - W, T)[:, None]
+    a = torch.softmax(logits.masked_fill(~seen, float("-inf")), dim=-1)
+    a[:, (seen & nan[n_sink:]).any(dim=-1)] = 0.0                 # what a query votes that sees one of them
+    want = a.reshape(4 * W, -1).sum(dim=0) / (4 * W)
+    assert torch.isnan(got[0][nan[n_sink:]]).all()
+    np.testing.assert_allclose(got[0][~nan[n_sink:]].numpy(), want[~nan[n_sink:]].numpy(), rtol=SCORE_RTOL, atol=1e-12)
+    other = osc.window_attention(k[1:].double(), q[4:].double(), n_sink, T - W)[0]
+    np.testing.assert_allclose(got[1:].numpy(), other.numpy(), rtol=SCORE_RTOL, atol=1e-12)
+
+
 def test_window_attention_rejects_fp32_keys():
     from kvquant.scorer import _launch_window_attention
     k = torch.randn(1, 64, 128, device=DEV)
