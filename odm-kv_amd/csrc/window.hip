@@ -131,7 +131,7 @@ __device__ static inline void fold_masked(const f32x16& s, QueryStat& q) {
 
 // a tile of keys on its way from memory into LDS without passing through registers: 16 bytes a lane, a wavefront's 1024 bytes one behind the other from `to` on
 __device__ static inline void request_to_lds(const uint16_t* from, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "{m0}"(to) : "memory");      // (m0 is the place in LDS)
 }
 
 template <int DT, int PASS>
