@@ -89,6 +89,13 @@ template <> struct Elem<ODMKV_F32> {
     __device__ static inline float from_f32(float f) { return f; }
 };
 
+// of the current device, and what they all have if it does not say
+static inline int compute_units() {
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) return v;
+    return 256;
+}
+
 // Wave-wide reductions (64 lanes, all of them active; every lane ends with the result) by DPP moves and lane swaps: a shuffle is a read of LDS, six of them
 // one behind the other.
 template <int CTRL>

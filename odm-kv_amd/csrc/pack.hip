@@ -2444,12 +2444,6 @@ __global__ __launch_bounds__(64) void exact_scatter_kernel(odmkv_packed_t s, voi
     }
 }
 
-static int compute_units() {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) return v;
-    return 256;
-}
-
 template <int DT>
 static int launch_dequant(const DequantArgs& da, hipStream_t st) {
     ODMKV_ALLOW_LDS((dequant_kernel<DT>), DQ_LDS);

@@ -1197,11 +1197,7 @@ static int run_expected(ScoreArgs& a, hipStream_t st) {
     if (a.cov) {
         // A workgroup prepares its head's covariance (64 KB) once: give it as many chunks as still leaves
         // `per_cu` workgroups for every compute unit.
-        int dev = 0, cus = 256;
-        if (hipGetDevice(&dev) == hipSuccess) {
-            int v = 0;
-            if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) cus = v;
-        }
+        const int cus = compute_units();
         auto pick = [&](int cpi, int max_cpw, int per_cu) {
             int cpw = max_cpw;
             while (cpw > 1 && (long)((a.nchunks + cpi * cpw - 1) / (cpi * cpw)) * a.Hq < (long)per_cu * cus) cpw >>= 1;

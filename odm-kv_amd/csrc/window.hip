@@ -279,7 +279,7 @@ __global__ __launch_bounds__(WIN_THREADS, 4) void window_kernel(WinArgs a) {
     }
 }
 
-// merge a query's statistics, one of every share of 256 tokens, into M + log2 Z: 64 queries a workgroup, a lane each, the entries shared out over its wavefronts
+// merge a query's statistics, one of every share of a workgroup's tokens, into M + log2 Z: 64 queries a workgroup, a lane each, the entries shared out over its wavefronts
 #define WIN_STAT_WAVES 16
 __global__ __launch_bounds__(WIN_STAT_WAVES * 64) void window_stats_kernel(WinArgs a) {
     __shared__ float ms[WIN_STAT_WAVES][64], ss[WIN_STAT_WAVES][64];
@@ -314,9 +314,9 @@ static inline int win_slots(int R) { return R > 128 ? 8 : R > 64 ? 4 : R > 32 ? 
 // 26.8 / 34.7, 20k 51.0 / 53.8, 32k 64.8 / 58.8, 131k 217 / 178; before 59, 64, 68 and 195).
 static inline bool win_turns(int R) { return R > 32 * WIN_WAVES; }
 static inline int64_t win_all_tiles(int Hkv, int Tc) { return (int64_t)Hkv * ((Tc + WIN_TILE - 1) / WIN_TILE); }
-static inline int win_tile(int Hkv, int R, int Tc) { return win_turns(R) && win_all_tiles(Hkv, Tc) > 3 * 256 ? 2 * WIN_TILE : WIN_TILE; }
-static inline int win_tiles(int Hkv, int R, int Tc) {
-    return win_turns(R) ? 1 : (int)std::max<int64_t>(1, (win_all_tiles(Hkv, Tc) + 2 * 256 - 1) / (2 * 256));
+static inline int win_tile(int Hkv, int R, int Tc, int cus) { return win_turns(R) && win_all_tiles(Hkv, Tc) > 3 * cus ? 2 * WIN_TILE : WIN_TILE; }
+static inline int win_tiles(int Hkv, int R, int Tc, int cus) {
+    return win_turns(R) ? 1 : (int)std::max<int64_t>(1, (win_all_tiles(Hkv, Tc) + 2 * cus - 1) / (2 * cus));
 }
 static inline int win_chunks(int tile, int tiles, int Tc) { return (Tc + tiles * tile - 1) / (tiles * tile); }
 
@@ -356,7 +356,8 @@ static int window_attention(const void* K, int dtype, int Hkv, int T, int64_t st
     WinArgs a;
     a.K = K; a.Q = Q; a.sH = stride_h; a.sT = stride_t;
     a.Hkv = Hkv; a.G = Hq / Hkv; a.W = W; a.R = a.G * W; a.T = T; a.Tc = T - n_sink; a.n_sink = n_sink;
-    a.tile = win_tile(Hkv, a.R, a.Tc); a.tiles = win_tiles(Hkv, a.R, a.Tc); a.nchunks = win_chunks(a.tile, a.tiles, a.Tc); a.qpos0 = q_pos0;
+    const int cus = compute_units();
+    a.tile = win_tile(Hkv, a.R, a.Tc, cus); a.tiles = win_tiles(Hkv, a.R, a.Tc, cus); a.nchunks = win_chunks(a.tile, a.tiles, a.Tc); a.qpos0 = q_pos0;
     a.qblocks = (a.R + 31) / 32; a.slots = win_slots(a.R);
     a.inv_w = 1.0f / (float)W;
     a.c = scaling * 1.4426950408889634f;
