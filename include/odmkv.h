@@ -378,7 +378,8 @@ int odmkv_dequantize_rows_packed(const uint8_t* indices, const float* norms, int
 
 /* Rows of K and V quantised and dequantised in place (float16 / bfloat16): groups x group_rows rows each, row (g, t) at
  * element g * stride_group + t * stride_row of both (what the uniform-width press does to the model's cache,
- * kvquant/backend_press.py:94-148).  workspace: odmkv_round_trip_workspace_bytes(groups * group_rows). */
+ * kvquant/backend_press.py:94-148).  workspace: odmkv_round_trip_workspace_bytes(groups * group_rows) where bits_k or bits_v
+ * is 8; the narrower widths need none (workspace may be NULL).  No two rows may share memory. */
 size_t odmkv_round_trip_workspace_bytes(int64_t n);
 int odmkv_round_trip_rows(void* K, void* V, int dtype, int64_t groups, int64_t group_rows, int64_t stride_group,
                           int64_t stride_row, int bits_k, int bits_v, const float* pi_k, const float* pi_v,

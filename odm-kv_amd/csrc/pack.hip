@@ -2502,7 +2502,7 @@ extern "C" int odmkv_dequant_from(const odmkv_packed_t* store, void* K, void* V,
 
 // ------------------------------------------------------------------------------------------------
 // rows outside the store on the matrix cores: the 16-bit quantiser's estimate with the codes as bytes or in the reference's
-// container, the dequantiser from byte codes, and both in one pass.  Where there are two jobs (keys and values of a layer in one launch), workgroups of
+// container, the dequantiser from byte codes (8 bits), and both in one pass (2 to 4 bits).  Where there are two jobs (keys and values of a layer in one launch), workgroups of
 // the even index take job 0, of the odd one job 1; a wave takes a tile of 64 rows.  A row per lane without them took 150 us for 64512 rows (the
 // fused multiply-adds of the rotation on the vector ALU).
 // ------------------------------------------------------------------------------------------------

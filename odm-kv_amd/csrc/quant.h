@@ -114,7 +114,8 @@ __host__ __device__ static inline int container_bytes(int bits) { return bits ==
 // a tile of 64 rows that the matrix-core quantiser leaves to the exact one carries this in place of its first norm
 #define ROWS_HANDED_OVER 0x7fc0beefu
 // on the matrix cores (pack.hip): the quantiser for 16-bit rows of 2, 3 and 4 bits; the dequantiser from byte codes into 16-bit rows, one or two jobs a
-// launch; both in one pass over 16-bit rows of 2, 3 and 4 bits, into `out` (which may be x), one or two jobs a launch
+// launch (8-bit codes: the narrower ones go the next way); both in one pass over 16-bit rows of 2, 3 and 4 bits, into `out` (which may be x), one or
+// two jobs a launch
 int launch_quantize_rows_f16(const RowsJob& job, int dtype, hipStream_t st);
 int launch_dequantize_rows_f16(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st);
 int launch_round_trip_rows(const RowsJob* jobs, int n_jobs, int dtype, hipStream_t st);

@@ -143,15 +143,13 @@ static int launch_quantize_rows_exact(const RowsJob& j, int dtype, hipStream_t s
     return 0;
 }
 
-static int check_rows(const char* who, const void* x, const float* pi, const float* cb, const void* codes, const float* norms, int dtype,
-                      int64_t N, int64_t stride_n, int bits) {
-    ODMKV_CHECK_ARG(x && pi && cb && codes && norms, "%s: null pointer", who);
+static int check_rows(const char* who, const void* x, const float* pi, const float* cb, int dtype, int64_t N, int64_t stride_n, int bits) {
+    ODMKV_CHECK_ARG(x && pi && cb, "%s: null pointer", who);
     ODMKV_CHECK_ARG(dtype == ODMKV_F16 || dtype == ODMKV_BF16 || dtype == ODMKV_F32, "%s: bad dtype %d", who, dtype);
     ODMKV_CHECK_ARG(bits == 2 || bits == 3 || bits == 4 || bits == 8, "%s: width %d not in {2,3,4,8}", who, bits);
     ODMKV_CHECK_ARG(N >= 0 && N < ((int64_t)1 << 37), "%s: bad row count", who);
     const int align = dtype == ODMKV_F32 ? 4 : 8;
-    ODMKV_CHECK_ARG(stride_n % align == 0 && stride_n >= HD && ((uintptr_t)x & 15) == 0 && ((uintptr_t)codes & 15) == 0,
-                    "%s: rows must be 16-byte aligned", who);
+    ODMKV_CHECK_ARG(stride_n % align == 0 && stride_n >= HD && ((uintptr_t)x & 15) == 0, "%s: rows must be 16-byte aligned", who);
     return 0;
 }
 
@@ -168,7 +166,9 @@ static int quantize(const RowsJob& job, int dtype, hipStream_t st) {
 
 static int quantize_rows(const char* who, const void* x, int dtype, int64_t N, int64_t stride_n, int bits, const float* pi, const float* cb,
                          uint8_t* codes, float* norms, int packed, void* stream) {
-    if (int rc = check_rows(who, x, pi, cb, codes, norms, dtype, N, stride_n, bits)) return rc;
+    ODMKV_CHECK_ARG(codes && norms, "%s: null pointer", who);
+    if (int rc = check_rows(who, x, pi, cb, dtype, N, stride_n, bits)) return rc;
+    ODMKV_CHECK_ARG(((uintptr_t)codes & 15) == 0, "%s: rows must be 16-byte aligned", who);
     if (N == 0) return 0;
     const RowsJob j = {x, 0, (long long)stride_n, (long long)N, (long long)N, bits, packed, pi, cb, codes, norms, nullptr};
     return quantize(j, dtype, (hipStream_t)stream);
@@ -224,18 +224,20 @@ extern "C" int odmkv_round_trip_rows(void* K, void* V, int dtype, int64_t groups
     const int64_t n = groups * group_rows;
     ODMKV_CHECK_ARG(groups > 0 && group_rows > 0, "round_trip_rows: bad shape");
     ODMKV_CHECK_ARG(dtype == ODMKV_F16 || dtype == ODMKV_BF16, "round_trip_rows: 16-bit rows only");
-    ODMKV_CHECK_ARG(workspace && workspace_bytes >= odmkv_round_trip_workspace_bytes(n), "round_trip_rows: workspace too small");
+    ODMKV_CHECK_ARG((bits_k != 8 && bits_v != 8) || (workspace && ((uintptr_t)workspace & 15) == 0 && workspace_bytes >= odmkv_round_trip_workspace_bytes(n)),
+                    "round_trip_rows: workspace too small");
     RowsJob j[2];
-    char* ws = (char*)workspace;
+    char* ws = (char*)workspace;                               // (8 bits: codes and norms between the two steps)
     for (int i = 0; i < 2; ++i) {
-        uint8_t* codes = (uint8_t*)ws;
-        float* norms = (float*)(ws + align_up((size_t)n * HD, 256));
-        ws += align_up((size_t)n * HD, 256) + align_up((size_t)n * sizeof(float), 256);
         void* x = i ? V : K;
         j[i] = {x, (long long)stride_group, (long long)stride_row, (long long)group_rows, (long long)n, i ? bits_v : bits_k, 0,
-                i ? pi_v : pi_k, i ? cb_v : cb_k, codes, norms, x};
-        if (int rc = check_rows("round_trip_rows", x, j[i].pi, j[i].cb, codes, norms, dtype, n, stride_row, j[i].bits)) return rc;
+                i ? pi_v : pi_k, i ? cb_v : cb_k, nullptr, nullptr, x};
+        if (int rc = check_rows("round_trip_rows", x, j[i].pi, j[i].cb, dtype, n, stride_row, j[i].bits)) return rc;
         ODMKV_CHECK_ARG(stride_group % 8 == 0, "round_trip_rows: rows must be 16-byte aligned");
+        if (j[i].bits != 8) continue;
+        j[i].codes = (uint8_t*)ws;
+        j[i].norms = (float*)(ws + align_up((size_t)n * HD, 256));
+        ws += align_up((size_t)n * HD, 256) + align_up((size_t)n * sizeof(float), 256);
     }
     // 2, 3 and 4 bits in one pass, 8 bits by the exact quantiser and the dequantiser
     RowsJob narrow[2], wide[2];

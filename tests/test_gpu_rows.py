@@ -186,3 +186,25 @@ def test_codes_of_fp16_rows_below_the_normal_numbers(bits):
         # half a unit of fp16's smallest numbers, or a step; another code moves the row by some tenths of a percent of its norm at the least
         err = (got.view(n, 128).double() - want).abs()
         assert (err <= 2.0 ** -25 + 2.0 ** -10 * want.abs() + 1e-6 * norms.double()[:, None]).all()
+
+
+@pytest.mark.parametrize("bits", [(2, 2), (4, 3), (8, 3), (2, 8), (8, 8)])
+def test_the_round_trip_takes_a_workspace_for_8_bits_alone(bits, monkeypatch):
+    from kvquant import TurboQuantBackendPress, _lib
+    asked, workspace = [], _lib.workspace
+    monkeypatch.setattr(_lib, "workspace", lambda device, size, name, *a: (asked.append(size) if name == "round_trip" else None) or workspace(device, size, name, *a))
+    k, v = (torch.randn(1, 2, 300, 128, generator=torch.Generator().manual_seed(s)).half().cuda() for s in (1, 2))
+    press = TurboQuantBackendPress(key_bits=bits[0], value_bits=bits[1], value_quantizer="mse")
+    got_k, got_v = k.clone(), v.clone()
+    press._quantise_span(0, got_k, got_v, 0, 300)
+    assert asked == ([_lib.lib.odmkv_round_trip_workspace_bytes(600)] if 8 in bits else [])
+    for got, x, b, seed in ((got_k, k, bits[0], 42), (got_v, v, bits[1], 2042)):
+        q = press._q(b, seed, x)
+        want = q.dequantize(q.quantize(x.view(-1, 128))).view(x.shape)
+        assert ((got.float() - want).abs() <= 2 ** -10 * want.abs() + 1e-5).all()       # (as in test_round_trip_in_place)
+    kq, vq = press._q(bits[0], 42, k), press._q(bits[1], 2042, v)
+    rc = _lib.lib.odmkv_round_trip_rows(k.data_ptr(), v.data_ptr(), _lib.dtype_code(k), 2, 300, 300 * 128, 128, kq.bits, vq.bits, kq.pi.data_ptr(),
+                                        vq.pi.data_ptr(), kq.centroids.data_ptr(), vq.centroids.data_ptr(), None, 0, _lib.stream_ptr(k.device))
+    torch.cuda.synchronize()
+    assert rc == (-1 if 8 in bits else 0)
+    assert 8 in bits or (torch.equal(k, got_k) and torch.equal(v, got_v))
