@@ -337,3 +337,30 @@ def test_a_mask_written_to_between_forwards_is_looked_at_again(inference, additi
         assert ap._store_part_is_open(mask, 4, 7) and len(looks) == 6
         mask[0, 0, 1, 2] = float("-inf") if additive else False
         assert not ap._store_part_is_open(mask, 4, 8)
+
+
+def test_rows_that_share_memory_do_not_take_the_one_pass_kernel():
+    """The kernel rewrites a row while others are still to be read.  Layouts of caches pass; expanded tensors, overlapping windows of one
+    sequence, and keys that are the values or begin inside them do not.  Against a count of every element's address."""
+    from kvquant.backend_press import _rows_apart
+    base = torch.zeros(1 << 16, dtype=torch.float16)
+
+    def view(at, B, H, n, strides):
+        return base.as_strided((B, H, n, 8), (*strides, 1), at)
+
+    def apart(k, v):
+        index = torch.arange(base.numel())
+        return torch.cat([index.as_strided(t.shape, t.stride(), t.storage_offset()).flatten() for t in (k, v)]).bincount().max() == 1
+
+    some = []
+    for B, H, n, strides in [(1, 4, 6, (192, 48, 8)), (2, 4, 6, (192, 48, 8)), (1, 4, 6, (192, 8, 32)), (2, 3, 6, (480, 160, 16)), (1, 4, 6, (384, 16, 64)),
+                             (1, 4, 6, (0, 0, 8)), (1, 4, 6, (32, 8, 8)), (1, 4, 6, (96, 24, 8)), (1, 1, 6, (8, 8, 8)), (2, 1, 6, (24, 24, 8)), (1, 1, 1, (8, 8, 8))]:
+        k = view(0, B, H, n, strides)
+        for off in (0, 4, 8, 16, 32, 184, 192, 4096):
+            v = view(off, B, H, n, strides)
+            for a, b in ((k, v), (v, k)):
+                assert apart(a, b) or not _rows_apart(a, b), (strides, off)
+            some.append((_rows_apart(k, v), bool(apart(k, v)), strides, off))
+    assert (True, True, (192, 48, 8), 4096) in some and (True, True, (192, 8, 32), 192) in some       # one behind the other
+    assert (True, True, (384, 16, 64), 8) in some                                                     # keys and values of a token side by side
+    assert not any(fast for fast, _, strides, _ in some if strides in ((0, 0, 8), (32, 8, 8), (96, 24, 8)))
