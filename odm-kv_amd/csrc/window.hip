@@ -58,11 +58,11 @@ __device__ static inline f32x16 win_mfma(uint4 a, uint4 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// merge two (max, sum) pairs kept in base-2 units (a maximum of -inf: nothing seen yet, the sum is 0, or NaN where a logit was)
+// merge two (max, sum) pairs kept in base-2 units (a maximum of -inf: nothing seen yet, the sum is 0, or NaN where a logit was; either stays
+// so times exp2(-inf).  A branch for it kept the statistics kernel from asking for eight entries at once: 0.9 us a call)
 __device__ static inline void ms2_merge(float& m, float& s, float m2, float s2) {
-    const float mn = fmaxf(m, m2);
-    if (mn == -INFINITY) { m = mn; s += s2; return; }
-    s = s * __builtin_amdgcn_exp2f(m - mn) + s2 * __builtin_amdgcn_exp2f(m2 - mn);
+    const float mn = fmaxf(m, m2), by = mn > -INFINITY ? mn : 0.0f;
+    s = s * __builtin_amdgcn_exp2f(m - by) + s2 * __builtin_amdgcn_exp2f(m2 - by);
     m = mn;
 }
 
@@ -111,7 +111,7 @@ __device__ static inline void fold_products(const f32x16& p, float c, QueryStat&
         const float by = ref > -INFINITY ? ref : 0.0f;              // (nothing but -inf and NaN: sums to 0 or NaN)
 #pragma unroll
         for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(__fmaf_rn(p[r], c, -by));
-        q.sum *= q.ref > -INFINITY ? __builtin_amdgcn_exp2f(q.ref - ref) : 1.0f;
+        q.sum *= __builtin_amdgcn_exp2f(q.ref - by);
         q.ref = ref;
     }
     q.sum += z;
@@ -125,7 +125,7 @@ __device__ static inline void fold_masked(const f32x16& s, QueryStat& q) {
     float z = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) z += __builtin_amdgcn_exp2f(s[r] - by);
-    q.sum = __fmaf_rn(q.sum, q.ref > -INFINITY ? __builtin_amdgcn_exp2f(q.ref - ref) : 1.0f, z);
+    q.sum = __fmaf_rn(q.sum, __builtin_amdgcn_exp2f(q.ref - by), z);
     q.ref = ref;
 }
 
