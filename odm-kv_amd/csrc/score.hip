@@ -454,7 +454,8 @@ __global__ __launch_bounds__(256) void score_pv_kernel(ScoreArgs a) {
         for (int g = 0; g < GMAX; ++g)
             if (g < a.G) lg[g] = a.logits[((size_t)h * a.G + g) * a.Tc + t];
     }
-    constexpr int NPRE = 8;                        // statistics entries per lane and head requested ahead (512 blocks, 131072 tokens: behind V they would arrive with it)
+    constexpr int NPRE = 8;                        // statistics entries per lane and head requested ahead: 512 blocks of 256 tokens.  A longer prompt's rest is asked
+                                                   // for behind V and arrives with it; 16 entries take 152 registers for eight heads (126), and a wavefront a SIMD less
     float2 pre[GMAX / 4][NPRE];
 #pragma unroll
     for (int gi = 0; gi < GMAX / 4; ++gi)

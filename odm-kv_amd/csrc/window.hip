@@ -18,7 +18,7 @@
 // What bounds it: 67 MB of keys a pass (12 us at the rate these reads reach, the first tile of 64 KB a compute unit 5 to 9 us after the start) and
 // 13 us of products and vector work (67 million exponentials at half the vector rate, a subtraction and an addition each), of which a tile's part
 // runs under the next tile's way.  32k tokens of 8 heads, 64 queries, bf16, us a pass: 41.5 + 33.8 -> 29.3 + 28.1; whole calls of 32
-// heads over 8, us: 600 tokens 33.5 -> 19.3, 8k 40 -> 27.4, 131k 226 -> 179.  Before, 64 tokens lay in a
+// heads over 8, us: 600 tokens 32 -> 18, 8k 40.7 -> 27.1, 32k 75 -> 61, 131k 234 -> 183 (fp16 239 -> 188).  Before, 64 tokens lay in a
 // wavefront's registers and 256 queries in LDS: all keys were asked for before the first product, every wavefront closed 256 queries' statistics
 // for its 64 tokens, and the tokens inside the window divided by W at every logit, in wavefronts that ran 10 us longer than the others.
 // Tried, no faster: 16 wavefronts and four tiles under way (33 + 29), 256 tokens in one tile (33.5 + 28.7), wave priorities, the next products
